@@ -193,6 +193,17 @@ int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_t* ids, int
                           void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip, void* stream);
 
 /*
+ * The same with a workspace (16-byte aligned), which lets a call with few queries spread the slots of a query over
+ * several workgroups: dsa_sparse_mla_fwd_workspace_bytes is what the call can use (0: it would not spread them).
+ * With less, every query's slots stay in one workgroup.
+ */
+size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int K);
+int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv,
+                          int K, int q_start, float sm_scale, int d_v, void* out, float* lse,
+                          void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Sparse MQA-MLA attention backward: dQ and dKV of dsa_sparse_mla_fwd given dO, the saved out and
  * natural-log lse.  P and dS enter the matrix products as bf16 (as in the reference's kernel); the
  * contribution of one (query, key) pair to dKV - a row of 576 values, summed over all heads in

@@ -1,18 +1,29 @@
 // Sparse MQA-MLA attention forward for gfx950.
 //
-// One 256-thread workgroup (4 waves) per query; wave w owns heads [32w, 32w+32).  The query's
-// selected latent rows are gathered 32 at a time straight from global memory into LDS
-// (global_load_lds, 16 B per lane, STAGES tiles in flight) in a layout of nine 128-byte groups per
-// key row with an XOR swizzle on the 16-byte slot, so both MFMA operand reads below are spread
-// over the LDS banks:
+// The selected latent rows are gathered 32 at a time straight from global memory into LDS
+// (global_load_lds, 16 B per lane) in a layout of nine 128-byte groups per key row with an XOR
+// swizzle on the 16-byte slot, so both MFMA operand reads below are spread over the LDS banks:
 //   S^T[key, head] = KV_tile . Q^T      36 x v_mfma_f32_32x32x16_bf16, A = KV rows from LDS
-//                                         (ds_read_b128), B = this wave's Q slice held in registers
+//                                         (ds_read_b128), B = the wave's Q slice held in registers
 //   O^T[dv, head] += V_tile^T . P^T     32 x MFMA, A = LDS transpose reads (ds_read_b64_tr_b16),
 //                                         B = the softmaxed S^T accumulators re-used in place
 // With S^T a lane owns one head (column), so the online-softmax statistics are per lane and need
 // one cross-lane exchange per tile; the accumulator layout of S^T is, up to a fixed permutation
 // of the keys inside a tile, the B-operand layout of the second product, so P never touches LDS.
 // MFMA-bound: 2*H*(576+512) flop per (query, key) pair against 1152 gathered bytes.
+//
+// A 256-thread workgroup has four waves of up to 512 registers, one per SIMD.  How they share a
+// query's heads and slots is the MODE:
+//   0  128 heads, one tile at a time: wave w owns heads [32w, 32w + 32).
+//   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
+//      of every other tile; the two streams' sums are merged through LDS at the end.
+//   2  32 heads, two tiles at a time: waves (stream, b) compute S^T of the same heads and own half
+//      of the value columns.
+// With fewer than 128 heads mode 0 leaves waves without work, at the same time per tile; modes 1
+// and 2 spend 68 / 52 matrix instructions per wave on two tiles instead of one and are then bound
+// by the gather.  A query's heads may also be spread over several workgroups, and its slots over
+// `ksplit` of them (few queries: one workgroup per query would leave most of the 256 compute units
+// idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
 #include "mla_tile.h"
 
 namespace {
@@ -36,44 +47,140 @@ __device__ __forceinline__ void mfma_chain_done(f32x16& acc) {
   asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc));
 }
 
-// The softmax of a head is taken relative to a reference point fixed before the first P.V
-// product, so the O^T accumulators are never rescaled.  The fast pass (EXACT = false) uses the
-// maximum of the first tile; a query in which a later tile exceeds that by more than 2^64 is
-// marked (NaN with a payload in lse) and redone by the EXACT = true pass, which first finds the
-// true row maximum with an extra sweep of S^T over all tiles.
-constexpr unsigned LSE_REDO_MARK = 0x7fc0d5a0u;
+struct FwdArgs {
+  const __bf16* q; const __bf16* kv; const int* ids;
+  __bf16* out; float* lse; void* p_out;
+  int S, H, Skv, K, q_start;
+  float sm_scale;
+  const float* sink;
+  int p_skip;
+  int n_hg, ksplit, k_loc;                   // head groups per query, slot ranges per query, slots of a range
+  f32x4* part_o; float* part_ml;             // ksplit > 1: sums [S][ksplit][H/32][16][4][64] x 4, (m, l) [S][ksplit][H][2]
+};
 
-// One query, by the 256 threads of a workgroup.
-template <int STAGES, int POUT, bool EXACT>   // POUT: 0 none, 1 bf16, 2 f32
-__device__ __forceinline__ void fwd_query(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
-    __bf16* __restrict__ out, float* __restrict__ lse, void* __restrict__ p_out,
-    int S, int H, int Skv, int K, int q_start, float sm_scale, const float* __restrict__ sink, int p_skip, int qi) {
+// The softmax of a head is taken relative to a reference point, the maximum of the first tile, so the
+// O^T accumulators are never rescaled (a rescaling branch in the loop, even one never taken, costs the
+// register allocator hundreds of spills).  Where a later tile exceeds it by more than 2^64 (exp2 then nears
+// the end of fp32) the wave marks its heads - a NaN with a payload in lse, or in the statistics of its
+// slot range - and the kernel that follows does them again relative to the true row maximum.
+constexpr float REDO_ABOVE = 64.0f;
+constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
+__device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
+
+struct Final { float o_scale; float inv; float lse; };
+// Denominator, output factor and natural-log lse of a head from its reference point m (base 2) and sum l.
+// A sink logit is one more term exp(sink) in the denominator with no value row; the reference moves to
+// max(m, sink) so that neither term can overflow.  A query without any valid slot gets lse = sink (+inf
+// without a sink) and a zero output row.
+__device__ __forceinline__ Final finish_head(float m, float l, const float* sink) {
+  float o_scale = 1.0f;
+  if (sink) {
+    const float sk2 = *sink * LOG2E;
+    const float nm = fmaxf(m, sk2);
+    o_scale = exp2f(m - nm);
+    l = l * o_scale + exp2f(sk2 - nm);
+    m = nm;
+  }
+  Final f;
+  f.o_scale = o_scale;
+  f.inv = l > 0.f ? o_scale / l : 0.f;
+  f.lse = l > 0.f ? (m + log2f(l)) * 0.6931471805599453f : INFINITY;
+  return f;
+}
+
+__device__ __forceinline__ i16x4 read_tr(const unsigned char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p));
+}
+__device__ __forceinline__ bf16x8 value_operand(const i16x4& lo, const i16x4& hi) {
+  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// maximum of a tile's logits for the lane's head (both half-waves)
+__device__ __forceinline__ float tile_max(const f32x16& sacc) {
+  float mx = sacc[0];
+#pragma unroll
+  for (int e = 1; e < 16; e++) mx = fmaxf(mx, sacc[e]);
+  return fmaxf(mx, __shfl_xor(mx, 32, 64));
+}
+// P of a tile relative to `ref` (base 2) as the B operand of the second product; l gains the lane's share of the sum
+__device__ __forceinline__ void softmax_numerators(const f32x16& sacc, float c2, float ref, float& l, bf16x8 (&pb)[2]) {
+  float psum = 0.f;
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float pe = __builtin_amdgcn_exp2f(fmaf(sacc[8 * s + e], c2, -ref));
+      psum += pe;
+      pb[s][e] = (__bf16)pe;
+    }
+  l += psum;
+}
+// one 32 x 32 block of O^T (lane = head): to the workspace as it lies, or normalised to the lane's output row
+__device__ __forceinline__ void store_partial(const f32x16& t, f32x4* p) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const f32x4 v = {t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]};
+    p[j * 64] = v;
+  }
+}
+__device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned short* p) {   // all lanes of the wave
+  uint4 o[2];
+  acc_row_to_16B(t, scale, o);
+  *(uint4*)p = o[0];
+  *(uint4*)(p + 16) = o[1];
+}
+
+template <int MODE, int STAGES, bool SPLIT, int POUT>   // SPLIT: ksplit > 1; POUT: 0 none, 1 bf16, 2 f32
+__global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
+  constexpr int STREAMS = MODE == 0 ? 1 : 2;
+  constexpr int NDT = MODE == 2 ? DTILES / 2 : DTILES;      // value column tiles of a wave
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, g = lane >> 5;
-  const int qpos = q_start + qi;
-  const int NT = K / BI;
+  const int stream = STREAMS == 2 ? wave >> 1 : 0, sub = wave & 1;
+  const int S = a.S, H = a.H, K = a.K, p_skip = a.p_skip;
 
-  int* idx_s = (int*)(smem + STAGES * TILE_BYTES);
-  unsigned* tmask = (unsigned*)(idx_s + K);
+  // Workgroup -> (query, head group, slot range).  The head groups of one slot range gather the same rows:
+  // they sit eight workgroups apart, i.e. on the same XCD and its L2.  Longest prefixes first.
+  int qi, hg = 0, sp = 0;
+  if (MODE == 0 && !SPLIT) {
+    qi = S - 1 - (int)blockIdx.x;
+  } else {
+    const int i = (int)blockIdx.x >> 3;
+    hg = i % a.n_hg;
+    const int u = (i / a.n_hg) * 8 + ((int)blockIdx.x & 7);
+    if (u >= S * (SPLIT ? a.ksplit : 1)) return;
+    qi = S - 1 - (SPLIT ? u / a.ksplit : u);
+    sp = SPLIT ? u % a.ksplit : 0;
+  }
+  const int qpos = a.q_start + qi;
+  const int k0 = sp * a.k_loc;
+  const int KL = min(a.k_loc, K - k0), NT = KL / BI;         // slots and tiles of this range
+  const int tile0 = k0 / BI;
+  const int hb = MODE == 0 ? wave : (MODE == 1 ? 2 * hg + sub : hg);   // 32-head block of the wave
+
+  constexpr int RING = STREAMS * STAGES * TILE_BYTES;
+  int* idx_s = (int*)(smem + RING);
+  unsigned* tmask = (unsigned*)(idx_s + KL);
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
 
   // ---- this wave's Q slice as the B operand of S^T = KV . Q^T, requested before the ids are staged
   // so that both come back in one round trip to memory ---------------------------------------------
-  const int h = wave * 32 + r;
+  const int h = hb * 32 + r;
   const bool head_ok = h < H;
   bf16x8 qreg[KSTEPS];
   {
-    const bf16x8* qp = (const bf16x8*)(q + ((size_t)qi * H + (head_ok ? h : 0)) * DQK) + g;
+    const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : 0)) * DQK) + g;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
   }
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- stage the ids, mark valid slots, list the tiles that have any ---------------------
-  const int ntiles = stage_ids(ids, qi, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
+  const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, qpos, idx_s, tmask, tlist, ntile_s);
+  const int nsteps = (ntiles + STREAMS - 1) / STREAMS;
   // the slice must have landed before the gather pipeline starts: the loop below counts
   // outstanding vector-memory operations by hand
   DSA_WAIT_VMCNT(0);
@@ -83,63 +190,71 @@ __device__ __forceinline__ void fwd_query(
   // slots of tiles that are never visited still need their -inf in p_out
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
   if (POUT != 0 && head_ok && ntiles < NT) {
-    for (int t = p_skip / BI; t < NT; t++) {
-      if (tmask[t] != 0u) continue;
-      const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(t * BI - p_skip) + 16 * g;
+    for (int t = 0; t < NT; t++) {
+      if (tmask[t] != 0u || (tile0 + t) * BI < p_skip || (STREAMS == 2 && (t & 1) != stream)) continue;
+      const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + t) * BI - p_skip) + 16 * g;
       if (POUT == 2) {
         const f32x4 ninf = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-        for (int j = 0; j < 4; j++) *(f32x4*)((float*)p_out + pbase + 4 * j) = ninf;
+        for (int j = 0; j < 4; j++) *(f32x4*)((float*)a.p_out + pbase + 4 * j) = ninf;
       } else {
         const uint4 ninf = make_uint4(0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u);
 #pragma unroll
-        for (int j = 0; j < 2; j++) *(uint4*)((unsigned short*)p_out + pbase + 8 * j) = ninf;
+        for (int j = 0; j < 2; j++) *(uint4*)((unsigned short*)a.p_out + pbase + 8 * j) = ninf;
       }
     }
   }
 
-  // ---- gather of tile n of the list into ring slot n % STAGES; lane-dependent LDS offsets ----
+  // ---- gather of tile n of the list into ring slot n % (STREAMS * STAGES); lane-dependent LDS offsets ----
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  auto issue = [&](int n) { gather_tile(kv, idx_s, tlist[n], lds0 + (unsigned)((n % STAGES) * TILE_BYTES)); };
-  // The same gather in nine steps (one 128-byte group of the key rows each), issued between MFMAs:
-  // nine transfers in a row hold the wave until the memory pipeline has taken them all (about 520
-  // clocks per tile of 4200).
-  unsigned g_goff = 0, g_lb = 0;
-  auto gather_prepare = [&](int n) {
-    const int gkey = tid >> 3, gsub = tid & 7;
-    int kid = idx_s[tlist[n] * BI + gkey];
-    kid = kid < 0 ? 0 : kid;
-    g_goff = (unsigned)kid * (DQK * 2) + (unsigned)((gsub ^ swz(gkey)) * 16);
-    g_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + wave * 1024));
+  auto issue = [&](int n) {
+    gather_tile(a.kv, idx_s, tlist[min(n, ntiles - 1)], lds0 + (unsigned)((n % (STREAMS * STAGES)) * TILE_BYTES));
   };
-  auto gather_step = [&](int grp) { dma16(g_lb + grp * GRP_BYTES, g_goff + grp * 128, kv); };
+  // The same gather in single steps (one 128-byte group of the key rows of a tile each), issued between
+  // MFMAs: nine transfers in a row hold the wave until the memory pipeline has taken them all (about 520
+  // clocks per tile of 4200).
+  // (Two streams and an odd tile count: the last tile is gathered twice and masked out in the second stream.)
+  unsigned g_goff[STREAMS], g_lb[STREAMS];
+  auto gather_prepare = [&](int n0) {
+#pragma unroll
+    for (int s = 0; s < STREAMS; s++) {
+      const int n = n0 + s;
+      const int gkey = tid >> 3, gsub = tid & 7;
+      int kid = idx_s[tlist[min(n, ntiles - 1)] * BI + gkey];
+      kid = kid < 0 ? 0 : kid;
+      g_goff[s] = (unsigned)kid * (DQK * 2) + (unsigned)((gsub ^ swz(gkey)) * 16);
+      g_lb[s] = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % (STREAMS * STAGES)) * TILE_BYTES + wave * 1024));
+    }
+  };
+  auto gather_step = [&](int s, int grp) {
+    dma16(g_lb[s] + grp * GRP_BYTES, g_goff[s] + grp * 128, a.kv);
+  };
   const LaneOffsets lo = lane_offsets();
   const unsigned (&qk_off)[4] = lo.row_off;          // A operand of S^T: row r, 16-byte chunk 2*ks + g
   const unsigned (&pv_off)[2][2][2] = lo.tr_off;     // A operand of O^T: transpose reads, [s][t][dt & 1]
 
-  const float c2 = sm_scale * LOG2E;
+  const float c2 = a.sm_scale * LOG2E;
   float m_ref = -1e30f, l_run = 0.f;
-  bool overflow = false;
-  f32x16 oacc[DTILES];
-#pragma unroll
-  for (int dt = 0; dt < DTILES; dt++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) oacc[dt][e] = 0.f;
+  f32x16 oacc[NDT];
 
   // S^T of the tile in stage buffer tb.  Operand reads run four k-steps ahead of the MFMAs; the
   // scheduling fences keep that order (and with it the register budget: Q slice 144 + O^T
   // accumulators 256 of 512 per lane).
   auto qk_tile = [&](const unsigned char* tb, unsigned mask, f32x16& sacc, bool gather) {
-    bf16x8 a[4];
+    bf16x8 f[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) a[ks] = *(const bf16x8*)(tb + (ks >> 2) * GRP_BYTES + qk_off[ks & 3]);
+    for (int ks = 0; ks < 4; ks++) f[ks] = *(const bf16x8*)(tb + (ks >> 2) * GRP_BYTES + qk_off[ks & 3]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
-      if (ks == 0) mfma_first(sacc, a[0], qreg[0]);
-      else mfma_next(sacc, a[ks & 3], qreg[ks]);
-      if (ks + 4 < KSTEPS) a[ks & 3] = *(const bf16x8*)(tb + ((ks + 4) >> 2) * GRP_BYTES + qk_off[ks & 3]);
-      if (ks % 7 == 3 && gather) gather_step(ks / 7);          // groups 0 .. 4
+      if (ks == 0) mfma_first(sacc, f[0], qreg[0]);
+      else mfma_next(sacc, f[ks & 3], qreg[ks]);
+      if (ks + 4 < KSTEPS) f[ks & 3] = *(const bf16x8*)(tb + ((ks + 4) >> 2) * GRP_BYTES + qk_off[ks & 3]);
+      if (STREAMS == 1) {
+        if (ks % 7 == 3 && gather) gather_step(0, ks / 7);                // groups 0 .. 4
+      } else {
+        if (ks % 2 == 1 && gather) gather_step((ks / 2) / 9, (ks / 2) % 9);   // all 18 of the next two tiles
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     mfma_chain_done(sacc);
@@ -151,89 +266,76 @@ __device__ __forceinline__ void fwd_query(
         if (!((mg >> (8 * (e >> 2) + (e & 3))) & 1u)) sacc[e] = -INFINITY;
     }
   };
-  auto tile_max = [&](const f32x16& sacc) {
-    float mx = sacc[0];
-#pragma unroll
-    for (int e = 1; e < 16; e++) mx = fmaxf(mx, sacc[e]);
-    return fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
-  };
-  auto wait_tile = [&](int n) {
-    const int ahead = min(STAGES - 2, ntiles - 1 - n);   // tiles allowed to stay in flight
-    if (ahead >= 2) { DSA_WAIT_VMCNT(18); }
-    else if (ahead == 1) { DSA_WAIT_VMCNT(9); }
-    else { DSA_WAIT_VMCNT(0); }
-    __syncthreads();
+
+  auto issue_first = [&]() {
+    for (int n = 0; n < STREAMS * (STAGES - 1) && n < STREAMS * nsteps; n++) issue(n);
   };
 
-  if (EXACT) {   // extra sweep: true maximum of every head over all valid slots
-    for (int n = 0; n < STAGES - 1 && n < ntiles; n++) issue(n);
-    for (int n = 0; n < ntiles; n++) {
-      wait_tile(n);
-      if (n + STAGES - 1 < ntiles) issue(n + STAGES - 1);
-      f32x16 sacc;
-      qk_tile(smem + (n % STAGES) * TILE_BYTES, tmask[tlist[n]], sacc, false);
-      m_ref = fmaxf(m_ref, tile_max(sacc));
+#pragma unroll
+  for (int dt = 0; dt < NDT; dt++) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) oacc[dt][e] = 0.f;
+  }
+  issue_first();
+  bool overflow = false;
+  int stores_after = 0;                      // p_out stores a wave issued after the transfers it waits for (two streams)
+  for (int step = 0; step < nsteps; step++) {
+    if (STREAMS == 1) {
+      const int ahead = min(STAGES - 2, ntiles - 1 - step);   // tiles allowed to stay in flight
+      if (ahead >= 2) { DSA_WAIT_VMCNT(18); }
+      else if (ahead == 1) { DSA_WAIT_VMCNT(9); }
+      else { DSA_WAIT_VMCNT(0); }
+    } else {
+      static_assert(STREAMS == 1 || STAGES == 2, "one step of transfers in flight");
+      if (POUT != 0 && stores_after == 4) { DSA_WAIT_VMCNT(4); }
+      else if (POUT != 0 && stores_after == 2) { DSA_WAIT_VMCNT(2); }
+      else { DSA_WAIT_VMCNT(0); }
     }
     __syncthreads();
-  }
-
-  for (int n = 0; n < STAGES - 1 && n < ntiles; n++) issue(n);
-
-  for (int n = 0; n < ntiles; n++) {
-    wait_tile(n);
-    const bool more = n + STAGES - 1 < ntiles;
-    if (more) gather_prepare(n + STAGES - 1);
-
-    const int tile = tlist[n];
-    const unsigned mask = tmask[tile];
-    const unsigned char* tb = smem + (n % STAGES) * TILE_BYTES;
+    const int next0 = STREAMS == 1 ? step + STAGES - 1 : STREAMS * (step + STAGES - 1);
+    const bool more = next0 < ntiles;
+    if (more) gather_prepare(next0);
+    const int n = STREAMS * step + stream;
+    const bool real = STREAMS == 1 || n < ntiles;
+    const int tile = tlist[real ? n : ntiles - 1];
+    const unsigned mask = real ? tmask[tile] : 0u;
+    const unsigned char* tb = smem + (n % (STREAMS * STAGES)) * TILE_BYTES;
 
     f32x16 sacc;
     qk_tile(tb, mask, sacc, more);
-    if (POUT != 0 && head_ok && tile * BI >= p_skip) {
-      const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(tile * BI - p_skip);
+    if (STREAMS == 2) stores_after = 0;
+    if (POUT != 0 && head_ok && real && (tile0 + tile) * BI >= p_skip) {
+      const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + tile) * BI - p_skip);
       if (POUT == 2) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           f32x4 v = {sacc[4 * j], sacc[4 * j + 1], sacc[4 * j + 2], sacc[4 * j + 3]};
-          *(f32x4*)((float*)p_out + prow + 4 * g + 8 * j) = v;
+          if (MODE != 2 || (j >> 1) == sub) *(f32x4*)((float*)a.p_out + prow + 4 * g + 8 * j) = v;
         }
       } else {
         // A lane holds keys 8j + 4g .. +3 of its head (j = 0..3): 8-byte pieces.  The two half-waves
         // trade pieces so that each lane ends up with 8 consecutive keys, twice: 16-byte stores.
         uint4 o[2];
         acc_row_to_16B(sacc, 1.0f, o);
-        *(uint4*)((unsigned short*)p_out + prow + 8 * g) = o[0];
-        *(uint4*)((unsigned short*)p_out + prow + 16 + 8 * g) = o[1];
+        if (MODE != 2 || sub == 0) *(uint4*)((unsigned short*)a.p_out + prow + 8 * g) = o[0];
+        if (MODE != 2 || sub == 1) *(uint4*)((unsigned short*)a.p_out + prow + 16 + 8 * g) = o[1];
       }
+      if (STREAMS == 2) stores_after = POUT == 2 ? (MODE == 2 ? 2 : 4) : (MODE == 2 ? 0 : 2);
     }
 
     // ---- softmax numerators (base 2), one head per lane -----------------------------------
     {
-      const float mx = tile_max(sacc);
-      if (!EXACT) {
-        if (n == 0) m_ref = mx;
-        overflow |= (mx > m_ref + 64.0f);
-      }
+      const float mx = tile_max(sacc) * c2;
+      if (step == 0) m_ref = STREAMS == 1 ? mx : fmaxf(mx, -1e30f);       // (a masked-out tile has the maximum -inf)
+      overflow |= (mx > m_ref + REDO_ABOVE);
     }
     bf16x8 pb[2];
-    {
-      float psum = 0.f;
-#pragma unroll
-      for (int s = 0; s < 2; s++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const float pe = __builtin_amdgcn_exp2f(fmaf(sacc[8 * s + e], c2, -m_ref));
-          psum += pe;
-          pb[s][e] = (__bf16)pe;
-        }
-      l_run += psum;
-    }
+    softmax_numerators(sacc, c2, m_ref, l_run, pb);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- O^T += V^T . P^T -----------------------------------------------------------------
     {
-      typedef short i16x8 __attribute__((ext_vector_type(8)));
+      const unsigned char* vb = tb + (MODE == 2 ? sub * (NDT / 2) * GRP_BYTES : 0);     // the wave's value columns
       i16x4 v[2][2][2];   // [ring][s][t]
 #pragma unroll
       for (int dt = 0; dt < 2; dt++)
@@ -241,118 +343,309 @@ __device__ __forceinline__ void fwd_query(
         for (int s = 0; s < 2; s++)
 #pragma unroll
           for (int t = 0; t < 2; t++)
-            v[dt][s][t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                LDS_PTR(i16x4, tb + (dt >> 1) * GRP_BYTES + pv_off[s][t][dt & 1]));
+            v[dt][s][t] = read_tr(vb + (dt >> 1) * GRP_BYTES + pv_off[s][t][dt & 1]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int dt = 0; dt < DTILES; dt++) {
+      for (int dt = 0; dt < NDT; dt++) {
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-          i16x8 av = __builtin_shufflevector(v[dt & 1][s][0], v[dt & 1][s][1], 0, 1, 2, 3, 4, 5, 6, 7);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), pb[s], oacc[dt], 0, 0, 0);
-        }
-        if (dt + 2 < DTILES) {
+        for (int s = 0; s < 2; s++)
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value_operand(v[dt & 1][s][0], v[dt & 1][s][1]), pb[s], oacc[dt], 0, 0, 0);
+        if (dt + 2 < NDT) {
 #pragma unroll
           for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int t = 0; t < 2; t++)
-              v[dt & 1][s][t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                  LDS_PTR(i16x4, tb + ((dt + 2) >> 1) * GRP_BYTES + pv_off[s][t][dt & 1]));
+              v[dt & 1][s][t] = read_tr(vb + ((dt + 2) >> 1) * GRP_BYTES + pv_off[s][t][dt & 1]);
         }
-        if (dt % 4 == 1 && more) gather_step(5 + dt / 4);        // groups 5 .. 8
+        if (STREAMS == 1 && dt % 4 == 1 && more) gather_step(0, 5 + dt / 4);        // groups 5 .. 8
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
 
-  // ---- epilogue: normalise, write out[i,h,:] and lse[i,h] ---------------------------------
   float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-  if (!EXACT && __ballot(overflow) != 0ull) {
-    // leave the query to the exact pass (it rewrites out, lse and p_out of all heads)
-    if (lane == 0 && wave * 32 < H) ((unsigned*)lse)[(size_t)qi * H + wave * 32] = LSE_REDO_MARK;
+  bool again = __ballot(overflow) != 0ull;   // the same for all lanes of a wave
+
+  f32x4* box = (f32x4*)(smem + (size_t)sub * NDT * 4096) + lane;
+  float mine = 1.0f;
+  // ---- two streams: the second one's sums reach the first through the (now free) tile ring, scaled to the
+  // common reference point; the first one's waves finish --------------------------------------------------
+  if (STREAMS == 2) {
+    __syncthreads();                         // the last tiles and the id arrays have been read
+    static_assert(STREAMS == 1 || 2 * NDT * 4096 + 1024 <= RING, "the hand-over fits the tile ring");
+    float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the two waves' boxes
+    if (g == 0) {
+      ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
+      ml[((stream * 2 + sub) * 32 + r) * 2 + 1] = l_tot;
+    }
+    __syncthreads();
+    const float m_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2], l_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2 + 1];
+    again |= is_marked(m_o);
+    const float nm = fmaxf(m_ref, m_o);
+    const float f = __builtin_amdgcn_exp2f(m_ref - nm);
+    l_tot = l_tot * f + l_o * __builtin_amdgcn_exp2f(m_o - nm);
+    m_ref = nm;
+    if (stream == 1) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = oacc[dt][4 * j + e] * f;
+          box[(dt * 4 + j) * 64] = v;
+        }
+    }
+    __syncthreads();
+    if (stream == 1) return;
+    mine = f;
+  }
+  auto merged = [&](int dt) {                // column tile dt of the wave's heads, both streams
+    if (STREAMS == 1) return oacc[dt];
+    f32x16 t;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const f32x4 v = box[(dt * 4 + j) * 64];
+#pragma unroll
+      for (int e = 0; e < 4; e++) t[4 * j + e] = fmaf(oacc[dt][4 * j + e], mine, v[e]);
+    }
+    return t;
+  };
+  if (!head_ok) return;                      // the same for all lanes of a wave
+  const bool stats = g == 0 && (MODE != 2 || sub == 0);
+  float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
+  if (again) {
+    if (stats) {
+      if (SPLIT) part_ml[0] = __builtin_bit_cast(float, REDO_MARK);
+      else a.lse[(size_t)qi * H + h] = __builtin_bit_cast(float, REDO_MARK);
+    }
     return;
   }
-  float o_scale = 1.0f;
-  if (sink) {
-    // per-head sink logit: one more term exp(sink) in the denominator, with no value row.  The
-    // reference point moves to max(reference, sink) so that neither term can overflow; a query
-    // without any valid slot ends with lse = sink and a zero output row.
-    const float sk2 = sink[head_ok ? h : 0] * LOG2E;
-    const float nm = fmaxf(m_ref, sk2);
-    o_scale = exp2f(m_ref - nm);
-    l_tot = l_tot * o_scale + exp2f(sk2 - nm);
-    m_ref = nm;
-  }
-  const float inv = l_tot > 0.f ? o_scale / l_tot : 0.f;
-  if (head_ok) {
-    if (g == 0) lse[(size_t)qi * H + h] = l_tot > 0.f ? (m_ref + log2f(l_tot)) * 0.6931471805599453f : INFINITY;
-    unsigned short* op = (unsigned short*)out + ((size_t)qi * H + h) * DV + 8 * g;
+
+  // ---- epilogue: the wave's column tiles, normalised to out[i,h,:] with lse[i,h], or as they are to the workspace ----
+  const int dt0 = MODE == 2 ? sub * NDT : 0;
+  if (SPLIT) {
+    if (stats) { part_ml[0] = m_ref; part_ml[1] = l_tot; }
+    f32x4* po = a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt0) * 256 + lane;
 #pragma unroll
-    for (int dt = 0; dt < DTILES; dt++) {
-      uint4 o[2];
-      acc_row_to_16B(oacc[dt], inv, o);       // head_ok is the same for all lanes of a wave
-      *(uint4*)(op + 32 * dt) = o[0];
-      *(uint4*)(op + 32 * dt + 16) = o[1];
+    for (int dt = 0; dt < NDT; dt++) {
+      store_partial(merged(dt), po + dt * 256);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return;
+  }
+  const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
+  if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
+  unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
+#pragma unroll
+  for (int dt = 0; dt < NDT; dt++) {
+    store_out(merged(dt), fin.inv, op + 32 * dt);
+    if (STREAMS == 2) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// One 32-head block of a query relative to the true maximum of every head, all slots, one tile at a time: every
+// wave computes S^T of the block and sums its own value column tile dt.  For the marked blocks only: simple, and
+// light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.
+__device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int dt, f32x16& acc, float& m, float& l) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int NT = a.K / BI;
+  int* idx_s = (int*)(smem + TILE_BYTES);
+  unsigned* tmask = (unsigned*)(idx_s + a.K);
+  int* tlist = (int*)(tmask + NT);
+  __syncthreads();
+  const int ntiles = stage_ids(a.ids, qi, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  const LaneOffsets lo = lane_offsets();
+  const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * a.H + hb * 32 + r) * DQK) + g;
+  const float c2 = a.sm_scale * LOG2E;
+  unsigned v_off[2][2];                      // the wave's value columns: lo.tr_off[s][t][dt & 1]
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      v_off[s][t] = (unsigned)((dt >> 1) * GRP_BYTES) + lo.tr_off[s][t][0] + (unsigned)(dt & 1) * (lo.tr_off[s][t][1] - lo.tr_off[s][t][0]);
+  m = -1e30f;
+  l = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll 1
+  for (int step = 0; step < 2 * ntiles; step++) {            // first sweep: the maximum; second: the sums
+    const int tile = tlist[step < ntiles ? step : step - ntiles];
+    __syncthreads();
+    gather_tile(a.kv, idx_s, tile, (unsigned)(uintptr_t)smem);
+    DSA_WAIT_VMCNT(0);
+    __syncthreads();
+    f32x16 sacc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) sacc[e] = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < KSTEPS / 4; c++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(smem + c * GRP_BYTES + lo.row_off[j]),
+                                                       qp[2 * (4 * c + j)], sacc, 0, 0, 0);
+    const unsigned mg = tmask[tile] >> (4 * g);
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+      if (!((mg >> (8 * (e >> 2) + (e & 3))) & 1u)) sacc[e] = -INFINITY;
+    if (step < ntiles) {
+      m = fmaxf(m, tile_max(sacc) * c2);
+    } else {
+      bf16x8 pb[2];
+      softmax_numerators(sacc, c2, m, l, pb);
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            value_operand(read_tr(smem + v_off[s][0]), read_tr(smem + v_off[s][1])), pb[s], acc, 0, 0, 0);
+    }
+  }
+  l += __shfl_xor(l, 32, 64);
+}
+
+__device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, int dt, const f32x16& acc, float m, float l) {
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int h = hb * 32 + r;
+  const Final fin = finish_head(m, l, a.sink ? a.sink + h : nullptr);
+  if (dt == 0 && g == 0) a.lse[(size_t)qi * a.H + h] = fin.lse;
+  store_out(acc, fin.inv, (unsigned short*)a.out + ((size_t)qi * a.H + h) * DV + 32 * dt + 8 * g);
+}
+
+// ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
+// redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
+__global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
+  const int wave = threadIdx.x >> 6;
+  const int qc = (int)blockIdx.x * 32 + (int)(threadIdx.x & 31);
+  for (int hb = 0; hb < a.H / 32; hb++) {
+    unsigned todo = (unsigned)__ballot(qc < a.S && is_marked(a.lse[(size_t)(qc < a.S ? qc : 0) * a.H + hb * 32]));
+    __syncthreads();                         // every wave reads the same marks before any of them is rewritten
+    while (todo) {
+      const int qi = (int)blockIdx.x * 32 + __builtin_ctz(todo);
+      todo &= todo - 1;
+      for (int dt = wave; dt < DTILES; dt += 4) {
+        f32x16 acc;
+        float m, l;
+        redo_block(a, qi, hb, dt, acc, m, l);
+        write_block(a, qi, hb, dt, acc, m, l);
+      }
     }
   }
 }
 
-// Fast pass: workgroup b takes query S - 1 - b (longest prefixes first).  Exact pass: workgroup b
-// looks at the marks of queries 32b .. 32b + 31 with one load per lane and redoes the marked ones,
-// so that a launch in which nothing is marked costs a few microseconds, not a full-size workgroup
-// per query.
-template <int STAGES, int POUT, bool EXACT>
-__global__ __launch_bounds__(256, 1) void mla_fwd_kernel(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
-    __bf16* __restrict__ out, float* __restrict__ lse, void* __restrict__ p_out,
-    int S, int H, int Skv, int K, int q_start, float sm_scale, const float* __restrict__ sink, int p_skip) {
-  if (!EXACT) {
-    fwd_query<STAGES, POUT, false>(q, kv, ids, out, lse, p_out, S, H, Skv, K, q_start, sm_scale, sink, p_skip,
-                                   S - 1 - (int)blockIdx.x);
-    return;
+// Sum of the ksplit partial results of a query: one wave per (query, 32-head block, value column tile), reading
+// the accumulator layout in which they were stored (1 KB per instruction).  HBM / L2-bound: ksplit * H * 2 KB per query.
+__global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31;
+  const int HB = a.H / 32;
+  const int dt = ((int)blockIdx.x & 3) * 4 + wave;
+  const int hb = ((int)blockIdx.x >> 2) % HB, qi = ((int)blockIdx.x >> 2) / HB;
+  const int ns = a.ksplit;
+  const float* ml = a.part_ml + ((size_t)qi * ns * a.H + hb * 32 + r) * 2;
+  const f32x4* po = a.part_o + (((size_t)qi * ns * HB + hb) * DTILES + dt) * 256 + lane;
+  const size_t o_step = (size_t)HB * DTILES * 256;
+  float m = -1e30f;
+  bool again = false;                        // the same for all threads of the workgroup
+#pragma unroll 8
+  for (int s = 0; s < ns; s++) {
+    const float ms = ml[(size_t)s * a.H * 2];
+    again |= is_marked(ms);
+    m = fmaxf(m, ms);
   }
-  const int qc = (int)blockIdx.x * 32 + (int)(threadIdx.x & 31);
-  bool redo = false;
-  if (qc < S) {
-    const unsigned* lw = (const unsigned*)lse + (size_t)qc * H;
-    for (int w = 0; w * 32 < H; w++) redo |= (lw[w * 32] == LSE_REDO_MARK);
+  float l = 0.f;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.f;
+  if (__ballot(again) != 0ull) {
+    redo_block(a, qi, hb, dt, acc, m, l);
+  } else {
+#pragma unroll 4
+    for (int s = 0; s < ns; s++) {
+      const float f = __builtin_amdgcn_exp2f(ml[(size_t)s * a.H * 2] - m);
+      l = fmaf(ml[(size_t)s * a.H * 2 + 1], f, l);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const f32x4 v = po[s * o_step + j * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[4 * j + e] = fmaf(v[e], f, acc[4 * j + e]);
+      }
+    }
   }
-  unsigned todo = (unsigned)__ballot(redo);      // every wave reads the same 32 marks before any of them is rewritten
-  while (todo) {
-    const int b = __builtin_ctz(todo);
-    todo &= todo - 1;
-    fwd_query<STAGES, POUT, true>(q, kv, ids, out, lse, p_out, S, H, Skv, K, q_start, sm_scale, sink, p_skip,
-                                  (int)blockIdx.x * 32 + b);
-    __syncthreads();
-  }
+  write_block(a, qi, hb, dt, acc, m, l);
 }
 
-template <int STAGES>
-int launch_fwd(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K, int q_start,
-               float sm_scale, void* out, float* lse, void* p_out, int p_out_f32, const float* sink, int p_skip, hipStream_t st) {
-  const size_t smem = (size_t)STAGES * TILE_BYTES + (size_t)K * 4 + (size_t)(K / BI) * 8 + 16;   // ids, tile masks, tile list, counters
+// ---------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------
+struct FwdPlan { int mode, n_hg, ksplit, k_loc; };
+
+int max_slots(int mode, int stages) {        // slots of a range whose id arrays fit LDS beside the tile ring
+  const int ring = (mode == 0 ? stages : 2 * stages) * TILE_BYTES;
+  return (160 * 1024 - ring - 16) * 16 / 68 / 64 * 64;                  // 4 B per slot + 8 B per tile of 32
+}
+
+FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
+
+// The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
+// units, each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel that follows.
+// The constants are measured times in us (random rows; a pair of tiles on an idle chip and on a full one: the gathers
+// of 256 workgroups share the fabric): at 2048 slots and 128 heads one query takes 104 us in mode 0 and 17 us as
+// 32 workgroups of mode 2, 48 queries 104 and 45 us (mode 1 in two ranges), 200 queries of 64 heads 114 and 67 us
+// (mode 1), 4096 of 32 heads 1840 and 980 us (mode 2); 1500 queries of 128 heads stay in mode 0 (810 against 905 us).
+// A query with one pair of tiles has nothing to share out: mode 0.
+FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
+  if (K <= 2 * BI) return one_workgroup_per_query(K);
+  constexpr float FIXED = 6.0f, REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, COMBINE_BYTES_PER_US = 6e6f;
+  constexpr float PAIR_IDLE[3] = {2.95f, 1.6f, 1.3f}, PAIR_FULL[3] = {4.1f, 2.15f, 1.65f};
+  const int heads[3] = {128, 64, 32};
+  const int pairs = K / (2 * BI);
+  FwdPlan best = one_workgroup_per_query(K);
+  float best_t = 1e30f;
+  for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 3; mode++) {
+    const int n_hg = (H + heads[mode] - 1) / heads[mode];
+    for (int want = 1; want <= (may_split ? 32 : 1) && want <= pairs; want++) {
+      const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
+      if (ksplit != want || 64 * per > max_slots(mode, mode == 0 ? 3 : 2)) continue;
+      const long wgs = (long)S * n_hg * ksplit;
+      const float full = wgs < 256 ? (float)wgs / 256.0f : 1.0f;
+      float t = (float)((wgs + 255) / 256) * (FIXED + per * (PAIR_IDLE[mode] + full * (PAIR_FULL[mode] - PAIR_IDLE[mode])));
+      t += ksplit == 1 ? REDO : COMBINE + COMBINE_RANGE * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
+      if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
+      if (wgs >= 4096) break;                // more ranges only add rounds
+    }
+  }
+  return best;
+}
+
+size_t part_bytes(const FwdPlan& p, int S, int H) {
+  return p.ksplit > 1 ? (size_t)S * p.ksplit * H * (DV * 4 + 8) + 256 : 0;
+}
+
+template <int MODE, int STAGES, bool SPLIT>
+int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
+  const size_t smem = (size_t)(MODE == 0 ? STAGES : 2 * STAGES) * TILE_BYTES + ids_lds_bytes(a.k_loc);
   if (smem > 160 * 1024) return -1;
-  dim3 grid(S), block(256);
+  const int units = a.S * a.ksplit;
+  const dim3 grid(MODE == 0 && !SPLIT ? a.S : 8 * ((units + 7) / 8) * a.n_hg), block(256);
 #define DSA_FWD_LAUNCH(P) do { \
-    auto kern = mla_fwd_kernel<STAGES, P, false>; \
-    auto kern2 = mla_fwd_kernel<STAGES, P, true>; \
+    auto kern = mla_fwd_kernel<MODE, STAGES, SPLIT, P>; \
     if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return -2; \
-    if (dsa_reserve_lds((const void*)kern2, smem) != hipSuccess) return -2; \
-    kern<<<grid, block, smem, st>>>((const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, sink, p_skip); \
-    kern2<<<dim3((S + 31) / 32), block, smem, st>>>((const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, sink, p_skip); \
+    kern<<<grid, block, smem, st>>>(a); \
   } while (0)
-  if (!p_out) DSA_FWD_LAUNCH(0);
+  if (!a.p_out) DSA_FWD_LAUNCH(0);
   else if (!p_out_f32) DSA_FWD_LAUNCH(1);
   else DSA_FWD_LAUNCH(2);
 #undef DSA_FWD_LAUNCH
+  const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
+  if (dsa_reserve_lds(SPLIT ? (const void*)mla_fwd_combine_kernel : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess)
+    return -2;
+  if (SPLIT) mla_fwd_combine_kernel<<<dim3(a.S * (a.H / 32) * 4), block, tail, st>>>(a);
+  else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), block, tail, st>>>(a);
   return 0;
 }
 
-}  // namespace
-
-extern "C" int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
-                                     int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
-                                     int p_out_f32, const float* attn_sink, int p_out_skip, void* stream) {
+int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K, int q_start, float sm_scale,
+             int d_v, void* out, float* lse, void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
+             void* workspace, size_t workspace_bytes, void* stream) {
   DSA_REQUIRE(d_v == DV, "dsa_sparse_mla_fwd: only d_v = 512 (d_qk = 576) is supported, got d_v = %d", d_v);
   DSA_REQUIRE(S >= 0 && Skv > 0, "dsa_sparse_mla_fwd: bad sequence sizes S=%d Skv=%d", S, Skv);
   DSA_REQUIRE(H > 0 && H <= 128 && H % 32 == 0, "dsa_sparse_mla_fwd: head count must be 32, 64, 96 or 128, got %d", H);
@@ -361,21 +654,53 @@ extern "C" int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_
               "dsa_sparse_mla_fwd: p_out_skip must be a multiple of %d in [0, top-k), got %d", BI, p_out_skip);
   DSA_REQUIRE((size_t)Skv * DQK * 2 <= 0xffffffffull, "dsa_sparse_mla_fwd: kv larger than 4 GiB is not supported");
   DSA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)kv % 16) == 0 && ((uintptr_t)out % 8) == 0 &&
-              ((uintptr_t)p_out % 16) == 0 && ((uintptr_t)attn_sink % 4) == 0, "dsa_sparse_mla_fwd: misaligned pointer");
+              ((uintptr_t)p_out % 16) == 0 && ((uintptr_t)attn_sink % 4) == 0 && ((uintptr_t)workspace % 16) == 0,
+              "dsa_sparse_mla_fwd: misaligned pointer");
+  DSA_REQUIRE(K <= 8192, "dsa_sparse_mla_fwd: top-k %d exceeds the supported maximum 8192", K);
   if (S == 0) return DSA_OK;
   hipStream_t st = (hipStream_t)stream;
+  FwdPlan p = plan_fwd(S, H, K, true);
+  if (part_bytes(p, S, H) > workspace_bytes || (p.ksplit > 1 && workspace == nullptr)) p = plan_fwd(S, H, K, false);
+  FwdArgs a{(const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, attn_sink,
+            p_out ? p_out_skip : 0, p.n_hg, p.ksplit, p.k_loc, (f32x4*)workspace,
+            (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4)};
   int rc;
-  if (K <= 2048) rc = launch_fwd<4>(q, kv, ids, S, H, Skv, K, q_start, sm_scale, out, lse, p_out, p_out_f32, attn_sink, p_out ? p_out_skip : 0, st);
-  else if (K <= 8192) rc = launch_fwd<3>(q, kv, ids, S, H, Skv, K, q_start, sm_scale, out, lse, p_out, p_out_f32, attn_sink, p_out ? p_out_skip : 0, st);
-  else rc = -1;
-  DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d exceeds the supported maximum 8192", K);
+  const bool split = p.ksplit > 1;
+  if (p.mode == 1) rc = split ? launch_fwd<1, 2, true>(a, p_out_f32, st) : launch_fwd<1, 2, false>(a, p_out_f32, st);
+  else if (p.mode == 2) rc = split ? launch_fwd<2, 2, true>(a, p_out_f32, st) : launch_fwd<2, 2, false>(a, p_out_f32, st);
+  else if (p.k_loc > 2048) rc = split ? launch_fwd<0, 3, true>(a, p_out_f32, st) : launch_fwd<0, 3, false>(a, p_out_f32, st);
+  else rc = split ? launch_fwd<0, 4, true>(a, p_out_f32, st) : launch_fwd<0, 4, false>(a, p_out_f32, st);
+  DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d does not fit LDS", K);
   if (rc == -2) DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_fwd: cannot reserve LDS");
   DSA_CHECK_LAUNCH("dsa_sparse_mla_fwd");
   return DSA_OK;
 }
 
+}  // namespace
+
+extern "C" size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int K) {
+  (void)Skv;
+  if (S <= 0 || H <= 0 || H % 32 || K <= 0 || K % 64) return 0;
+  return part_bytes(plan_fwd(S, H, K, true), S, H);
+}
+
+extern "C" int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
+                                     int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
+                                     int p_out_f32, const float* attn_sink, int p_out_skip, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
+                  workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
+                                     int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
+                                     int p_out_f32, const float* attn_sink, int p_out_skip, void* stream) {
+  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
+                  nullptr, 0, stream);
+}
+
 extern "C" int dsa_sparse_mla_fwd(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
                                   int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
                                   int p_out_f32, void* stream) {
-  return dsa_sparse_mla_fwd_ex(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, nullptr, 0, stream);
+  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, nullptr, 0, nullptr, 0, stream);
 }

@@ -416,11 +416,13 @@ def _mla_fwd_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, q_start: i
                             device=q.device)
     lib = _lib.load()
     with torch.cuda.device(q.device):
-        _lib.check(lib.dsa_sparse_mla_fwd_ex(q.data_ptr(), kv.data_ptr(), ids.data_ptr(), S, H, kv.shape[0], K,
+        nbytes = lib.dsa_sparse_mla_fwd_workspace_bytes(S, H, kv.shape[0], K)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+        _lib.check(lib.dsa_sparse_mla_fwd_ws(q.data_ptr(), kv.data_ptr(), ids.data_ptr(), S, H, kv.shape[0], K,
                                              int(q_start), float(sm_scale), int(d_v), out.data_ptr(), lse.data_ptr(),
                                              p_out.data_ptr() if p_out_mode else None, int(p_out_mode == 2),
                                              attn_sink.data_ptr() if attn_sink is not None else None,
-                                             int(p_out_skip), _stream(q)),
+                                             int(p_out_skip), ws.data_ptr() if nbytes else None, nbytes, _stream(q)),
                    "dsa_sparse_mla_fwd")
     return out, lse, p_out
 

@@ -112,6 +112,49 @@ def test_forward_survives_a_late_dominant_key(gpu):
     assert (lse.cpu() - rl).abs().max().item() < 2e-2 * rl.abs().max().item() * 1e-2 + 1e-2
 
 
+@pytest.mark.parametrize("S,H,K,q_start,skv", [
+    (1, 128, 512, 900, None),         # one query: 32-head workgroups, a range per pair of tiles
+    (3, 64, 320, 500, 700),           # five pairs of tiles per query
+    (5, 96, 192, 300, None),          # the last 64-head workgroup holds 32 heads
+    (2, 32, 128, 400, None),
+    (300, 64, 192, 0, None),          # two tiles at a time without ranges, odd tile counts in the early rows
+    (300, 32, 256, 0, None),
+    (2, 128, 4096, 5000, None),       # ranges that fit the two-tile ring though the whole list does not
+])
+def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
+    """Few queries or few heads: heads and slots of a query are spread over workgroups and streams.  Slot lists with
+    holes, ranges without a valid slot, an empty row, sinks, logits, and a key that moves the softmax reference late."""
+    from loongforge_amd import ops
+
+    inp = O.make_mla_inputs(S, H, K, seed=S + H, skv=skv, q_start=q_start)
+    g = torch.Generator().manual_seed(K)
+    idx = inp.idx.clone()
+    idx[torch.rand(idx.shape, generator=g) < 0.3] = -1
+    idx[0, : K // 2] = -1
+    if S > 2:
+        idx[1] = -1
+        idx[2, 33:] = -1
+    sink = torch.linspace(-2, 2, H)
+    for name, sk in (("plain", None), ("sink", sink)):
+        if name == "sink" and (idx[0] >= 0).any():      # the last tile of a query beats those before it by far more than 2^64
+            last = int((idx[0] >= 0).nonzero()[-1])
+            kv = inp.kv.clone()
+            kv[idx[0, last].long()] = (inp.q[0, H - 1].float() * 40.0).to(torch.bfloat16)
+            inp.kv = kv
+        ro, rl, rp = O.sparse_mla_fwd(inp.q, inp.kv, idx, q_start, inp.sm_scale, 512, attn_sink=sk)
+        for dt in (None, torch.bfloat16, torch.float32):
+            out, lse, p = ops.sparse_mla_fwd(inp.q.to(gpu), inp.kv.to(gpu), idx.to(gpu), q_start, inp.sm_scale, 512, dt is not None,
+                                             dt or torch.bfloat16, attn_sink=None if sk is None else sk.to(gpu))
+            assert_close(out, ro, name + " out", atol=4e-2 if sk is not None else 2e-2)
+            fin = torch.isfinite(rl)
+            assert torch.equal(torch.isfinite(lse.cpu()), fin)
+            assert ((lse.cpu() - rl)[fin].abs() / rl[fin].abs().clamp_min(1)).max().item() < 1e-3
+            if dt is not None:
+                assert torch.equal(torch.isfinite(p.float().cpu()), torch.isfinite(rp))
+            if dt == torch.float32:
+                assert ((p.cpu() - rp)[torch.isfinite(rp)].abs() / rp[torch.isfinite(rp)].abs().clamp_min(1)).max().item() < 1e-3
+
+
 def test_forward_slot_permutation_invariance(gpu):
     inp = O.make_mla_inputs(100, 128, 128, seed=7)
     out1, lse1, _ = _run_fwd(inp, gpu)
