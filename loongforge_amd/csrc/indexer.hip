@@ -58,29 +58,112 @@ __device__ __forceinline__ float add_halves(float x) {
   return a + b;
 }
 
+// 32 heads x 32 keys of fp8 products into the weighted ReLU-sum of a lane's key
+__device__ __forceinline__ float head_sum(const i32x8 (&aq)[2], const i32x8 (&bk)[2], const float (&wq)[16], float sum) {
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.f;
+  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[0], bk[0], acc, 0, 0, 0, 127, 0, 127);
+  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[1], bk[1], acc, 0, 0, 0, 127, 0, 127);
+#pragma unroll
+  for (int e = 0; e < 16; e++) sum = fmaf(wq[e], relu1(acc[e]), sum);
+  return sum;
+}
+
+// a query's fp8 rows as the A operand, and the weights of the 16 heads a lane sees per head group
+template <int NHT>
+__device__ __forceinline__ void load_query(const unsigned char* __restrict__ q8, const float* __restrict__ q_w, int i, int r, int g,
+                                           i32x8 (&aq)[NHT][2], float (&wq)[NHT][16]) {
+#pragma unroll
+  for (int t = 0; t < NHT; t++) {
+    const unsigned char* row = q8 + ((size_t)i * NHT * 32 + 32 * t + r) * D + 32 * g;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const i32x4 lo = *(const i32x4*)(row + 64 * s);
+      const i32x4 hi = *(const i32x4*)(row + 64 * s + 16);
+      aq[t][s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+    const float* wrow = q_w + (size_t)i * NHT * 32 + 32 * t + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const f32x4 w4 = *(const f32x4*)(wrow + 8 * j);
+#pragma unroll
+      for (int e = 0; e < 4; e++) wq[t][4 * j + e] = w4[e];
+    }
+  }
+}
+
 template <int NHT>   // groups of 32 heads
-__global__ __launch_bounds__(64 * QB, 4) void indexer_logits_kernel(
+__global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kernel(
     const unsigned char* __restrict__ q8, const float* __restrict__ q_w, const unsigned char* __restrict__ k8,
     const float* __restrict__ k_scale, const int* __restrict__ ks, const int* __restrict__ ke,
-    int S, int Sk, float* __restrict__ logits, long ld, int relative, int q_begin, int q_count) {
+    int S, int Sk, float* __restrict__ logits, long ld, int relative, int q_begin, int q_count, int parts) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * TILE_BYTES + 2 * BK * 4];
-  constexpr int HI = NHT * 32;
   constexpr int NWAVE = QB;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: window tests below become scalar branches
   const int r = lane & 31, g = lane >> 5;
   const int nblk = (q_count + QB - 1) / QB;
-  const int blk = nblk - 1 - (int)blockIdx.x;            // longest windows first
+  const int blk = nblk - 1 - (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;            // longest windows first
   const int qb0 = q_begin + blk * QB;
   const int q_end = q_begin + q_count;
 
   // window union of the block
-  int jlo = 0x7fffffff, jhi = 0;
+  int jlo = 0x7fffffff, jhi = 0, total = 0;
   for (int t = 0; t < QB; t++) {
     const int i = qb0 + t;
-    if (i < q_end) { jlo = min(jlo, ks[i]); jhi = max(jhi, min(ke[i], Sk)); }
+    if (i < q_end) {
+      const int lo = max(ks[i], 0), hi = min(ke[i], Sk);
+      jlo = min(jlo, ks[i]);
+      jhi = max(jhi, hi);
+      total += (max(hi - lo, 0) + 31) / 32;
+    }
   }
   jlo = max(jlo, 0);
+
+  if (2 * total < 3 * ((jhi - jlo + 31) / 32)) {
+    // Unrelated windows (the sequences of a batch, or a single query): a key tile in LDS would serve one wave.  The
+    // block's 32-key sub-tiles are numbered through and every wave of its workgroups takes an equal run of them,
+    // whatever the lengths of the windows, with the key operand straight from global memory one sub-tile ahead.
+    const int my = part * NWAVE + wave;
+    const int a = (int)((long)total * my / (parts * NWAVE)), b = (int)((long)total * (my + 1) / (parts * NWAVE));
+    int before = 0;
+#pragma unroll 1
+    for (int i = qb0; i < min(qb0 + QB, q_end); i++) {
+      const int w_lo = max(ks[i], 0), w_hi = min(ke[i], Sk), n = (max(w_hi - w_lo, 0) + 31) / 32;
+      const int u_lo = max(a - before, 0), u_hi = min(b - before, n);
+      before += n;
+      if (u_lo >= u_hi) continue;
+      auto load_keys = [&](int u, i32x4 (&kk)[4], float& sc) {
+        const size_t j = (size_t)min(w_lo + 32 * u + r, Sk - 1);
+#pragma unroll
+        for (int x = 0; x < 4; x++) kk[x] = *(const i32x4*)(k8 + j * D + 32 * g + 64 * (x >> 1) + 16 * (x & 1));
+        sc = k_scale[j];
+      };
+      i32x4 kn[4];
+      float scn;
+      load_keys(u_lo, kn, scn);
+      i32x8 aq[NHT][2];
+      float wq[NHT][16];
+      load_query(q8, q_w, i, r, g, aq, wq);
+      float* lrow = logits + (size_t)(i - q_begin) * ld - (relative ? w_lo : 0);
+#pragma unroll 1
+      for (int u = u_lo; u < u_hi; u++) {
+        i32x8 bk[2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) bk[s] = __builtin_shufflevector(kn[2 * s], kn[2 * s + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+        const float ksc = scn;
+        if (u + 1 < u_hi) load_keys(u + 1, kn, scn);
+        float sum = 0.f;
+#pragma unroll
+        for (int h = 0; h < NHT; h++) sum = head_sum(aq[h], bk, wq[h], sum);
+        sum = add_halves(sum) * ksc;
+        const int j = w_lo + 32 * u + r;
+        if (g == 0 && j < w_hi) lrow[j] = sum;
+      }
+    }
+    return;
+  }
 
   // this wave's query
   const int i_q = qb0 + wave;
@@ -91,33 +174,16 @@ __global__ __launch_bounds__(64 * QB, 4) void indexer_logits_kernel(
   const int wlo = live ? qks : 0x7fffffff, whi = live ? qke : 0;     // the wave's window
   i32x8 aq[NHT][2];
   float wq[NHT][16];
-  {
-    const int is = live ? i_q : qb0;
-#pragma unroll
-    for (int t = 0; t < NHT; t++) {
-      const unsigned char* row = q8 + ((size_t)is * HI + 32 * t + r) * D + 32 * g;
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        const i32x4 lo = *(const i32x4*)(row + 64 * s);
-        const i32x4 hi = *(const i32x4*)(row + 64 * s + 16);
-        aq[t][s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
-      const float* wrow = q_w + (size_t)is * HI + 32 * t + 4 * g;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const f32x4 w4 = *(const f32x4*)(wrow + 8 * j);
-#pragma unroll
-        for (int e = 0; e < 4; e++) wq[t][4 * j + e] = w4[e];
-      }
-    }
-  }
+  load_query(q8, q_w, live ? i_q : qb0, r, g, aq, wq);
   DSA_WAIT_VMCNT(0);
 #pragma unroll
   for (int t = 0; t < NHT; t++)
 #pragma unroll
     for (int s = 0; s < 2; s++) asm volatile("" : "+v"(aq[t][s]));
 
-  const int t_lo = jlo / BK, t_hi = (jhi + BK - 1) / BK;      // key tiles [t_lo, t_hi)
+  // this part's share of the window union's key tiles: [t_lo, t_hi)
+  const int t_first = jlo / BK, t_all = max((jhi + BK - 1) / BK - t_first, 0);
+  const int t_lo = t_first + (int)((long)t_all * part / parts), t_hi = t_first + (int)((long)t_all * (part + 1) / parts);
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   const int gkey = tid >> 3, gsub = tid & 7;                  // 8 NWAVE key rows per DMA instruction
   auto issue = [&](int t) {
@@ -161,21 +227,13 @@ __global__ __launch_bounds__(64 * QB, 4) void indexer_logits_kernel(
         bk[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       }
       const float ksc = ksc_s[c * 32 + r];
-      float part = 0.f;
+      float sum = 0.f;
 #pragma unroll
-      for (int tt = 0; tt < NHT; tt++) {
-        f32x16 acc;
-#pragma unroll
-        for (int e = 0; e < 16; e++) acc[e] = 0.f;
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[tt][0], bk[0], acc, 0, 0, 0, 127, 0, 127);
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[tt][1], bk[1], acc, 0, 0, 0, 127, 0, 127);
-#pragma unroll
-        for (int e = 0; e < 16; e++) part = fmaf(wq[tt][e], relu1(acc[e]), part);
-      }
-      part = add_halves(part) * ksc;
+      for (int tt = 0; tt < NHT; tt++) sum = head_sum(aq[tt], bk, wq[tt], sum);
+      sum = add_halves(sum) * ksc;
       if (g == 0 && j >= qks && j < qke) {
         const int col = relative ? j - qks : j;
-        logits[(size_t)(qi - q_begin) * ld + col] = part;
+        logits[(size_t)(qi - q_begin) * ld + col] = sum;
       }
     }
   }
@@ -199,9 +257,17 @@ int dsa_indexer_logits_block(const void* q8, const float* q_w, const void* k8, c
     fill_neg_inf_kernel<<<dim3(2048), dim3(256), 0, st>>>(logits, q_count, (long)ld, width);
     DSA_CHECK_LAUNCH("dsa_indexer_logits(fill)");
   }
-  dim3 grid((q_count + QB - 1) / QB), block(64 * QB);
+  // Two workgroups of 128 registers fit a compute unit.  With too few blocks of queries to fill them their windows are
+  // cut into parts, for one round of workgroups where that leaves none over (under 128 blocks) and about one and a half
+  // of shorter ones beyond (us before -> after, 64 heads: one query x 4096 keys 52 -> 5, 61 x 20000 292 -> 18, 48
+  // unrelated windows of 7000 keys 807 -> 15, 500 x 8000 129 -> 39, 1500 x 7500 131 -> 89, 3000 x 7500 200 -> 166).
+  const int nblk = (q_count + QB - 1) / QB;
+  int parts = (nblk < 128 ? 512 : 768) / nblk;
+  if (parts > (Sk + BK - 1) / BK) parts = (Sk + BK - 1) / BK;
+  if (parts < 1) parts = 1;
+  dim3 grid(nblk * parts), block(64 * QB);
 #define DSA_IDX_LAUNCH(N) indexer_logits_kernel<N><<<grid, block, 0, st>>>( \
-    (const unsigned char*)q8, q_w, (const unsigned char*)k8, k_scale, ks, ke, S, Sk, logits, (long)ld, relative, q_begin, q_count)
+    (const unsigned char*)q8, q_w, (const unsigned char*)k8, k_scale, ks, ke, S, Sk, logits, (long)ld, relative, q_begin, q_count, parts)
   if (Hi == 32) DSA_IDX_LAUNCH(1);
   else DSA_IDX_LAUNCH(2);
 #undef DSA_IDX_LAUNCH

@@ -275,3 +275,28 @@ def test_indexer_kernel_with_fused_rotation_matches_rotating_first(gpu):
     for a, b in ((q1.grad, q2.grad), (k1.grad, k2.grad), (w1.grad, w2.grad)):
         scale = b.float().abs().max().item()
         assert (a.float() - b.float()).abs().max().item() <= 3e-2 * scale
+
+
+@pytest.mark.parametrize("Hi", [32, 64])
+def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
+    """Windows cut into parts over workgroups: shared ones (a chunk behind cached keys), unrelated ones (sequences of a
+    batch, some empty), a single query, window ends off every tile boundary."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(Hi)
+    for ks, ke, sk in (([0], [1], 5), ([3], [1999], 2000), ([0] * 9, list(range(700, 709)), 709),
+                       ([0, 40, 40, 171, 900, 901, 1500, 1500, 1777, 0], [40, 40, 171, 899, 901, 1500, 1777, 1501, 1999, 3], 2000)):
+        S = len(ks)
+        q = torch.randn(S, Hi, 128, generator=g).to(torch.float8_e4m3fn)
+        k = torch.randn(sk, 128, generator=g).to(torch.float8_e4m3fn)
+        w, sc = torch.randn(S, Hi, generator=g), torch.rand(sk, generator=g)
+        a, b = torch.tensor(ks, dtype=torch.int32), torch.tensor(ke, dtype=torch.int32)
+        ref = O.indexer_logits(q, w, k, sc, a, b)
+        for rel in (False, True):
+            got = ops.indexer_logits(q.to(gpu), w.to(gpu), k.to(gpu), sc.to(gpu), a.to(gpu), b.to(gpu), relative=rel).cpu()
+            for i in range(S):
+                n = max(ke[i] - ks[i], 0)
+                row = got[i, :n] if rel else got[i, ks[i]: ks[i] + n]
+                want = ref[i, ks[i]: ks[i] + n]
+                assert (row - want).abs().max().item() <= 1e-4 * max(want.abs().max().item(), 1.0) if n else True
+                assert int(torch.isfinite(got[i]).sum()) == n
