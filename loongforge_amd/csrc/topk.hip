@@ -14,9 +14,11 @@
 
 namespace {
 
-constexpr int BLOCK = 256;
-constexpr int NW = BLOCK / 64;
 constexpr int HBINS = 4096;
+// Every routine takes the workgroup size BL (256, or 1024 for few or long rows).  `scratch` holds three ints per wave for
+// reductions and four more for what they find.
+template <int BL> constexpr int NWAVES = BL / 64;
+template <int BL> constexpr int SCRATCH = 3 * (BL / 64) + 4;
 
 __device__ __forceinline__ unsigned f2key(float f) {       // larger float <-> larger unsigned
   unsigned u = __builtin_bit_cast(unsigned, f);
@@ -28,6 +30,7 @@ __device__ __forceinline__ float key2f(unsigned k) {
 }
 
 // exclusive prefix sum over the block (thread order), also returns the block total
+template <int BL>
 __device__ __forceinline__ int block_exscan(int v, int* scratch, int& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int inc = v;
@@ -41,22 +44,36 @@ __device__ __forceinline__ int block_exscan(int v, int* scratch, int& total) {
   __syncthreads();
   int base = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < NW; w++) { int s = scratch[w]; if (w < wave) base += s; tot += s; }
+  for (int w = 0; w < NWAVES<BL>; w++) { int s = scratch[w]; if (w < wave) base += s; tot += s; }
   total = tot;
   return base + inc - v;
+}
+
+// minimum, maximum and sum over the waves' entries (mn at 0, mx at NWAVES, count at 2 NWAVES)
+template <int BL>
+__device__ __forceinline__ void row_range(const int* scratch, float& mn, float& mx, int& count) {
+  const float* f = (const float*)scratch;
+  mn = f[0]; mx = f[NWAVES<BL>]; count = scratch[2 * NWAVES<BL>];
+#pragma unroll
+  for (int w = 1; w < NWAVES<BL>; w++) {
+    mn = fminf(mn, f[w]);
+    mx = fmaxf(mx, f[NWAVES<BL> + w]);
+    count += scratch[2 * NWAVES<BL> + w];
+  }
 }
 
 struct Pick { int bin; int above; };
 
 // Finds, scanning bins from the highest down, the bin in which the running count reaches `need`.
-// hist has nb bins (nb % BLOCK == 0).  Result: that bin and the number of keys in higher bins.
+// hist has nb bins (nb % BL == 0).  Result: that bin and the number of keys in higher bins.
+template <int BL>
 __device__ __forceinline__ Pick pick_bin(const int* hist, int nb, int need, int* scratch, int* res) {
-  const int per = nb / BLOCK;
+  const int per = nb / BL;
   const int hi = nb - 1 - (int)threadIdx.x * per;          // this thread owns bins hi, hi-1, ..., hi-per+1
   int local = 0;
   for (int b = 0; b < per; b++) local += hist[hi - b];
   int total;
-  int before = block_exscan(local, scratch, total);
+  int before = block_exscan<BL>(local, scratch, total);
   if (before < need && before + local >= need) {
     int run = before;
     for (int b = 0; b < per; b++) {
@@ -76,13 +93,13 @@ __device__ __forceinline__ bool comes_first(float a, int ia, float b, int ib) {
   return (a > b) || (a == b && (unsigned)ia < (unsigned)ib);
 }
 
-// Bitonic sort of Kp2 = EPT * BLOCK (score, id) pairs held in LDS.  A pair becomes one 64-bit
+// Bitonic sort of Kp2 = EPT * BL (score, id) pairs held in LDS.  A pair becomes one 64-bit
 // key whose unsigned order is the output order (descending score, then ascending id, id -1 last),
 // so a compare-exchange is one 64-bit compare and two selects.  Thread t keeps
 // elements [t*EPT, (t+1)*EPT) in registers: strides below EPT are register compare-exchanges,
 // strides inside a wave's span exchange through LDS without a workgroup barrier (LDS operations
 // of one wave complete in order), and only the strides that cross waves need barriers.  The
-// exchange buffer holds element j of thread t at j * BLOCK + t, so every LDS access of a wave is
+// exchange buffer holds element j of thread t at j * BL + t, so every LDS access of a wave is
 // bank-conflict free; the sorted elements go straight from registers to global memory.
 __device__ __forceinline__ unsigned long long sort_key(float score, int id) {
   const unsigned bits = __builtin_bit_cast(unsigned, score + 0.0f);          // -0 -> +0
@@ -94,7 +111,7 @@ __device__ __forceinline__ float sort_key_score(unsigned long long key) {
   return __builtin_bit_cast(float, asc ^ ((asc >> 31) ? 0x80000000u : 0xffffffffu));
 }
 
-template <int EPT>
+template <int BL, int EPT>
 __device__ __forceinline__ void bitonic_regs(float* outv, int* outi, unsigned long long* xbuf, int Kp2, float* sv, int* si, int K) {
   const int tid = threadIdx.x;
   const int base = tid * EPT;
@@ -108,11 +125,11 @@ __device__ __forceinline__ void bitonic_regs(float* outv, int* outi, unsigned lo
         const int pt = tid ^ (stride / EPT);
         const bool cross_wave = stride / EPT >= 64;
 #pragma unroll
-        for (int j = 0; j < EPT; j++) xbuf[j * BLOCK + tid] = key[j];
+        for (int j = 0; j < EPT; j++) xbuf[j * BL + tid] = key[j];
         if (cross_wave) __syncthreads(); else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         unsigned long long pk[EPT];
 #pragma unroll
-        for (int j = 0; j < EPT; j++) pk[j] = xbuf[j * BLOCK + pt];
+        for (int j = 0; j < EPT; j++) pk[j] = xbuf[j * BL + pt];
         if (cross_wave) __syncthreads(); else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         // this lane keeps the smaller key when it holds the lower element of an ascending pair or
         // the upper element of a descending one (size > stride >= EPT: the same for all j)
@@ -153,13 +170,16 @@ __device__ __forceinline__ void bitonic_regs(float* outv, int* outi, unsigned lo
 constexpr int LIN_SPARE = 960;               // extra buffer entries for the threshold bin's surplus
 constexpr int REG_ROW = 8192 + 4 * 256;      // longest row (plus alignment slack) the register variant holds
 constexpr int REG_ROW_BIG = 32768 + 4 * 256; // the same for the variant with twice the registers
+constexpr int WIDE_ROWS = 256;               // at most so many rows: the 1024-thread kernel
 constexpr int LIN_MAX_BIN = 256;             // largest segment ranked by pairwise counting
 
 // Threshold bin of a filled histogram (thread t owns bins [PER t, PER t + PER)), then the segment
 // starts written over the counts.  False when a bin is too crowded for the ranking step.
+template <int BL>
 __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff, int& tbin, int& above, int& c) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int PER = HBINS / BLOCK;
+  constexpr int PER = HBINS / BL;
+  int* found = scratch + 3 * NWAVES<BL>;
   int cnt[PER], local = 0;
 #pragma unroll
   for (int b4 = 0; b4 < PER; b4 += 4) {
@@ -169,17 +189,17 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
 #pragma unroll
   for (int b = 0; b < PER; b++) local += cnt[b];
   int total;
-  const int before = block_exscan(local, scratch, total);
+  const int before = block_exscan<BL>(local, scratch, total);
   if (before < keff && before + local >= keff) {
     int run = before;
 #pragma unroll
     for (int b = 0; b < PER; b++) {
-      if (run < keff && run + cnt[b] >= keff) { scratch[8] = tid * PER + b; scratch[9] = run; scratch[10] = cnt[b]; }
+      if (run < keff && run + cnt[b] >= keff) { found[0] = tid * PER + b; found[1] = run; found[2] = cnt[b]; }
       run += cnt[b];
     }
   }
   __syncthreads();
-  tbin = scratch[8]; above = scratch[9]; c = scratch[10];
+  tbin = found[0]; above = found[1]; c = found[2];
   int big = 0;
 #pragma unroll
   for (int b = 0; b < PER; b++) if (tid * PER + b < tbin) big = max(big, cnt[b]);
@@ -188,7 +208,9 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
   __syncthreads();
   if (lane == 0) scratch[wave] = big;
   __syncthreads();
-  big = max(max(scratch[0], scratch[1]), max(scratch[2], scratch[3]));
+  big = 0;
+#pragma unroll
+  for (int w = 0; w < NWAVES<BL>; w++) big = max(big, scratch[w]);
   if (big > LIN_MAX_BIN || c > LIN_SPARE) return false;
   {
     int run = before, st[PER];
@@ -202,11 +224,11 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
 }
 
 // Final position of every scattered element: hist[b] is the end of segment b by now.
-template <class BinOf>
+template <int BL, class BinOf>
 __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const int* hist, int filled, int keff, int K,
                                          int base_id, BinOf bin_of, float* sv, int* si) {
   const int tid = threadIdx.x;
-  for (int p = tid; p < filled; p += BLOCK) {
+  for (int p = tid; p < filled; p += BL) {
     const unsigned long long key = obuf[p];
     const float v = sort_key_score(key);
     const int b = bin_of(v);
@@ -216,74 +238,16 @@ __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const i
     const int pos = start + rank;
     if (pos < keff) { sv[pos] = v; si[pos] = base_id + (int)(unsigned)key; }
   }
-  for (int t = keff + tid; t < K; t += BLOCK) { sv[t] = -INFINITY; si[t] = -1; }
+  for (int t = keff + tid; t < K; t += BL) { sv[t] = -INFINITY; si[t] = -1; }
 }
 
-__device__ __forceinline__ bool linear_select_sort(const float* __restrict__ src, unsigned* keys, int n, int K, int base_id,
-                                                   int* hist, int* scratch, unsigned long long* obuf, float* sv, int* si) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // ---- stage the row as keys; range of the finite values ---------------------------------------
-  float mn = INFINITY, mx = -INFINITY;
-  int nfin = 0;
-  for (int e0 = tid; e0 < n; e0 += 8 * BLOCK) {   // eight loads in flight per thread
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = e0 + i * BLOCK < n ? src[e0 + i * BLOCK] : -INFINITY;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      if (e0 + i * BLOCK < n) keys[e0 + i * BLOCK] = f2key(v[i]);
-      if (fabsf(v[i]) < INFINITY) { mn = fminf(mn, v[i]); mx = fmaxf(mx, v[i]); nfin++; }
-      else if (!(v[i] < INFINITY)) mx = INFINITY;   // +inf or NaN: infinite span below, the general path takes the row
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    mn = fminf(mn, __shfl_xor(mn, o, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    nfin += __shfl_xor(nfin, o, 64);
-  }
-  __syncthreads();
-  if (lane == 0) { ((float*)scratch)[wave] = mn; ((float*)scratch)[4 + wave] = mx; scratch[8 + wave] = nfin; }
-  __syncthreads();
-  mn = fminf(fminf(((float*)scratch)[0], ((float*)scratch)[1]), fminf(((float*)scratch)[2], ((float*)scratch)[3]));
-  mx = fmaxf(fmaxf(((float*)scratch)[4], ((float*)scratch)[5]), fmaxf(((float*)scratch)[6], ((float*)scratch)[7]));
-  nfin = scratch[8] + scratch[9] + scratch[10] + scratch[11];
-  __syncthreads();
-  const float span = mx - mn;
-  if (!(span > 0.f) || !(span < INFINITY)) return false;
-  const int keff = min(K, nfin);
-  const float scale = ((float)HBINS - 0.5f) / span;
-  auto bin_of = [&](float v) { return min(HBINS - 1, (int)((mx - v) * scale)); };
-  // ---- histogram ------------------------------------------------------------------------------
-  for (int b = tid; b < HBINS; b += BLOCK) hist[b] = 0;
-  __syncthreads();
-  for (int e = tid; e < n; e += BLOCK) {
-    const float v = key2f(keys[e]);
-    if (fabsf(v) < INFINITY) atomicAdd(&hist[bin_of(v)], 1);
-  }
-  __syncthreads();
-  int tbin, above, c;
-  if (!lin_threshold(hist, scratch, keff, tbin, above, c)) return false;
-  // ---- scatter ------------------------------------------------------------------------------------
-  for (int e = tid; e < n; e += BLOCK) {
-    const float v = key2f(keys[e]);
-    if (fabsf(v) < INFINITY) {
-      const int b = bin_of(v);
-      if (b <= tbin) obuf[atomicAdd(&hist[b], 1)] = sort_key(v, e);
-    }
-  }
-  __syncthreads();
-  lin_rank(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
-  return true;
-}
-
-// The same for rows of at most 4 NV BLOCK elements, with the row held in registers instead of
-// LDS: thread t owns the 16-byte chunks t, t + BLOCK, ... of the row counted from the 16-byte
+// The same for rows of at most 4 NV BL elements, with the row held in registers instead of
+// LDS: thread t owns the 16-byte chunks t, t + BL, ... of the row counted from the 16-byte
 // boundary at or below its first element, so the whole row is fetched by NV vector loads issued
 // together and the workgroup needs only the histogram and the output buffer in LDS.  The row is
-// positions [off, m) of that layout; chunk i (positions [4 BLOCK i, 4 BLOCK (i + 1))) is touched only
+// positions [off, m) of that layout; chunk i (positions [4 BL i, 4 BL (i + 1))) is touched only
 // while it holds any of them.
-template <int NV>
+template <int BL, int NV>
 __device__ __forceinline__ void load_row_regs(const float* __restrict__ src, int n, float (&v)[NV][4], int& off, int& m) {
   const int tid = threadIdx.x;
   off = (int)(((uintptr_t)src >> 2) & 3);                  // elements between that boundary and src
@@ -291,7 +255,7 @@ __device__ __forceinline__ void load_row_regs(const float* __restrict__ src, int
   m = n + off;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    const int p = 4 * (tid + BLOCK * i);
+    const int p = 4 * (tid + BL * i);
     if (p >= off && p + 4 <= m) {
       const float4 x = *(const float4*)(base + p);
       v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
@@ -300,6 +264,30 @@ __device__ __forceinline__ void load_row_regs(const float* __restrict__ src, int
       for (int j = 0; j < 4; j++) v[i][j] = (p + j >= off && p + j < m) ? base[p + j] : -INFINITY;
     }
   }
+}
+
+// Rows of at most SHORT_ROW elements: one element per thread, ranked by counting the elements that precede it.  (The
+// first rows of a causal window: a row of one element has no spread, and the sorting network of the general path
+// would take 50 us over its 2048 output slots.)  False for rows that hold a NaN or +inf.
+constexpr int SHORT_ROW = 256;
+template <int BL>
+__device__ __forceinline__ bool rank_short_row(const float* __restrict__ src, int n, int K, int base_id, unsigned long long* buf,
+                                               float* sv, int* si) {
+  const int tid = threadIdx.x;
+  const float v = tid < n ? src[tid] : -INFINITY;
+  const bool live = v > -INFINITY;
+  const unsigned long long key = live ? sort_key(v, tid) : ~0ull;
+  if (tid < SHORT_ROW) buf[tid] = key;
+  if (__syncthreads_or(!(v < INFINITY))) return false;
+  const int nfin = __syncthreads_count(live);
+  if (tid < SHORT_ROW) {
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < n; j++) rank += buf[j] < key;
+    if (live && rank < K) { sv[rank] = v; si[rank] = base_id + tid; }
+  }
+  for (int t = min(K, nfin) + tid; t < K; t += BL) { sv[t] = -INFINITY; si[t] = -1; }
+  return true;
 }
 
 // min / max of three without the canonicalising v_max that fminf / fmaxf put in front of every operand
@@ -320,14 +308,14 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
 // x in [mn, mx]), and chunks wholly inside the row need no position tests.  Returns 1 when the row is
 // done, 0 when it is unsuitable (no spread, a crowded bin), -1 when it holds a non-finite value (the
 // caller then runs the tolerant form below on the same registers).
-template <int NV>
+template <int BL, int NV>
 __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int off, int m, int K, int base_id, int* hist,
                                                   int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int CH = 4 * BLOCK;
+  constexpr int CH = 4 * BL;
   const int nch = (m + CH - 1) / CH;                        // chunks that hold any of the row
   auto chunk_full = [&](int i) { return (i > 0 || off == 0) && CH * (i + 1) <= m; };   // the same for all threads
-  for (int b = tid; b < HBINS; b += BLOCK) hist[b] = 0;
+  for (int b = tid; b < HBINS; b += BL) hist[b] = 0;
   float mn = INFINITY, mx = -INFINITY;
   bool nan = false;
 #pragma unroll
@@ -338,7 +326,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
       mx = max3_raw(mx, v[i][0], v[i][1]); mx = max3_raw(mx, v[i][2], v[i][3]);
       nan |= __builtin_isunordered(v[i][0], v[i][1]) | __builtin_isunordered(v[i][2], v[i][3]);
     } else {
-      const int p = 4 * (tid + BLOCK * i);
+      const int p = 4 * (tid + BL * i);
 #pragma unroll
       for (int j = 0; j < 4; j++)
         if (p + j >= off && p + j < m) {
@@ -353,11 +341,10 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
     mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   }
   const bool wave_nan = __ballot(nan) != 0ull;
-  if (lane == 0) { ((float*)scratch)[wave] = mn; ((float*)scratch)[4 + wave] = mx; scratch[8 + wave] = wave_nan; }
+  if (lane == 0) { ((float*)scratch)[wave] = mn; ((float*)scratch)[NWAVES<BL> + wave] = mx; scratch[2 * NWAVES<BL> + wave] = wave_nan; }
   __syncthreads();
-  mn = fminf(fminf(((float*)scratch)[0], ((float*)scratch)[1]), fminf(((float*)scratch)[2], ((float*)scratch)[3]));
-  mx = fmaxf(fmaxf(((float*)scratch)[4], ((float*)scratch)[5]), fmaxf(((float*)scratch)[6], ((float*)scratch)[7]));
-  const bool any_nan = (scratch[8] | scratch[9] | scratch[10] | scratch[11]) != 0;
+  int any_nan;
+  row_range<BL>(scratch, mn, mx, any_nan);
   __syncthreads();
   if (any_nan || !(mn > -INFINITY) || !(mx < INFINITY)) return -1;
   const float span = mx - mn;
@@ -372,7 +359,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
 #pragma unroll
       for (int j = 0; j < 4; j++) atomicAdd(&hist[bin_of(v[i][j])], 1);
     } else {
-      const int p = 4 * (tid + BLOCK * i);
+      const int p = 4 * (tid + BL * i);
 #pragma unroll
       for (int j = 0; j < 4; j++)
         if (p + j >= off && p + j < m) atomicAdd(&hist[bin_of(v[i][j])], 1);
@@ -380,11 +367,11 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   }
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold(hist, scratch, keff, tbin, above, c)) return 0;
+  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return 0;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     if (i >= nch) continue;
-    const int p = 4 * (tid + BLOCK * i);
+    const int p = 4 * (tid + BL * i);
     const bool full = chunk_full(i);
 #pragma unroll
     for (int j = 0; j < 4; j++)
@@ -394,17 +381,17 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
       }
   }
   __syncthreads();
-  lin_rank(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
+  lin_rank<BL>(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
   return 1;
 }
 
 // The tolerant form: values that are not finite (-inf marks a column that cannot be selected) are skipped
 // one by one.
-template <int NV>
+template <int BL, int NV>
 __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], int off, int K, int base_id, int* hist,
                                                      int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int b = tid; b < HBINS; b += BLOCK) hist[b] = 0;
+  for (int b = tid; b < HBINS; b += BL) hist[b] = 0;
   float mn = INFINITY, mx = -INFINITY;
   int nfin = 0;
 #pragma unroll
@@ -419,11 +406,9 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
     mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     nfin += __shfl_xor(nfin, o, 64);
   }
-  if (lane == 0) { ((float*)scratch)[wave] = mn; ((float*)scratch)[4 + wave] = mx; scratch[8 + wave] = nfin; }
+  if (lane == 0) { ((float*)scratch)[wave] = mn; ((float*)scratch)[NWAVES<BL> + wave] = mx; scratch[2 * NWAVES<BL> + wave] = nfin; }
   __syncthreads();
-  mn = fminf(fminf(((float*)scratch)[0], ((float*)scratch)[1]), fminf(((float*)scratch)[2], ((float*)scratch)[3]));
-  mx = fmaxf(fmaxf(((float*)scratch)[4], ((float*)scratch)[5]), fmaxf(((float*)scratch)[6], ((float*)scratch)[7]));
-  nfin = scratch[8] + scratch[9] + scratch[10] + scratch[11];
+  row_range<BL>(scratch, mn, mx, nfin);
   __syncthreads();
   const float span = mx - mn;
   if (!(span > 0.f) || !(span < INFINITY)) return false;
@@ -437,48 +422,49 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
       if (fabsf(v[i][j]) < INFINITY) atomicAdd(&hist[bin_of(v[i][j])], 1);
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold(hist, scratch, keff, tbin, above, c)) return false;
+  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return false;
 #pragma unroll
   for (int i = 0; i < NV; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       if (fabsf(v[i][j]) < INFINITY) {
         const int b = bin_of(v[i][j]);
-        if (b <= tbin) obuf[atomicAdd(&hist[b], 1)] = sort_key(v[i][j], 4 * (tid + BLOCK * i) + j - off);
+        if (b <= tbin) obuf[atomicAdd(&hist[b], 1)] = sort_key(v[i][j], 4 * (tid + BL * i) + j - off);
       }
   __syncthreads();
-  lin_rank(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
+  lin_rank<BL>(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
   return true;
 }
 
-template <int NV>
+template <int BL, int NV>
 __device__ __forceinline__ bool linear_select_sort_regs(const float* __restrict__ src, int n, int K, int base_id,
                                                         int* hist, int* scratch, unsigned long long* obuf, float* sv, int* si) {
   float v[NV][4];
   int off, m;
-  load_row_regs<NV>(src, n, v, off, m);
-  const int r = select_regs_finite<NV>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
+  load_row_regs<BL, NV>(src, n, v, off, m);
+  const int r = select_regs_finite<BL, NV>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
   if (r >= 0) return r == 1;
   __syncthreads();
-  return select_regs_tolerant<NV>(v, off, K, base_id, hist, scratch, obuf, sv, si);
+  return select_regs_tolerant<BL, NV>(v, off, K, base_id, hist, scratch, obuf, sv, si);
 }
 
 // LEAN (sorted rows held in registers; implies !STAGED).  1: rows of up to REG_ROW elements, the kernel keeps to
 // 128 registers so that four workgroups share a compute unit.  2: rows of up to REG_ROW_BIG elements at up to 256
-// registers (two workgroups per compute unit).  A launch looks only at the rows whose length lies in
-// (n_above, n_upto] and leaves the others to the launch of the other variant; rows the single-sweep path turns
-// down take the general path on global memory and the plain LDS sorting network.  Rows are taken in ascending
+// registers (two workgroups per compute unit).  3: BL = 1024, rows of up to REG_ROW_BIG elements at 64 registers per
+// thread: one or two rows per compute unit, each four times as fast.  A launch looks only at the rows whose length
+// lies in (n_above, n_upto] and leaves the others to the launch of the other variant; rows the single-sweep path
+// turns down take the general path on global memory and the plain LDS sorting network.  Rows are taken in ascending
 // order (with causal windows the short ones first: 0.118 ms at 8192 x 8192 against 0.161 ms longest first and
 // 0.141 ms with short and long rows alternating).
-template <bool STAGED, int LEAN>
-__global__ __launch_bounds__(BLOCK, LEAN == 1 ? 4 : LEAN == 2 ? 2 : 1) void topk_kernel(
+template <int BL, bool STAGED, int LEAN>
+__global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 : 1) void topk_kernel(
     const float* __restrict__ logits, long ld, const int* __restrict__ row_begin, const int* __restrict__ row_end,
     int width, const int* __restrict__ id_base, int K, int Kp2, int sorted, float* __restrict__ scores,
     int* __restrict__ ids, int nmax, int n_above, int n_upto) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   int* hist = (int*)smem;                          // HBINS
-  int* scratch = hist + HBINS;                     // 16
-  float* outv = (float*)(scratch + 16);            // Kp2
+  int* scratch = hist + HBINS;                     // SCRATCH<BL>
+  float* outv = (float*)(scratch + SCRATCH<BL>);   // Kp2
   int* outi = (int*)(outv + Kp2);                  // Kp2
   unsigned* keys = (unsigned*)(outi + Kp2 + 2 * LIN_SPARE);   // nmax (STAGED only); the gap extends the (score, id) buffer
   const int tid = threadIdx.x;
@@ -495,76 +481,85 @@ __global__ __launch_bounds__(BLOCK, LEAN == 1 ? 4 : LEAN == 2 ? 2 : 1) void topk
 
   auto key_at = [&](int e) -> unsigned { return STAGED ? keys[e] : f2key(src[e]); };
 
-  if (sorted && n > 0) {   // single-sweep path, also for rows shorter than K
-    if (STAGED) {
-      if (linear_select_sort(src, keys, n, K, base_id, hist, scratch, (unsigned long long*)outv, sv, si)) return;
-      __syncthreads();
-    } else if (LEAN == 1 && n + 3 <= REG_ROW) {
+  if (sorted && n > 0 && n <= SHORT_ROW) {
+    if (rank_short_row<BL>(src, n, K, base_id, (unsigned long long*)outv, sv, si)) return;
+    __syncthreads();
+  } else if (sorted && n > 0) {   // single-sweep path, also for rows shorter than K
+    if (LEAN == 1 && n + 3 <= REG_ROW) {
       bool done;
       unsigned long long* obuf = (unsigned long long*)outv;
-      if (n + 3 <= 8 * BLOCK) done = linear_select_sort_regs<2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
-      else if (n + 3 <= 16 * BLOCK) done = linear_select_sort_regs<4>(src, n, K, base_id, hist, scratch, obuf, sv, si);
-      else done = linear_select_sort_regs<REG_ROW / (4 * BLOCK)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      if (n + 3 <= 8 * BL) done = linear_select_sort_regs<BL, 2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else if (n + 3 <= 16 * BL) done = linear_select_sort_regs<BL, 4>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else done = linear_select_sort_regs<BL, REG_ROW / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       if (done) return;
       __syncthreads();
     } else if (LEAN == 2 && n + 3 <= REG_ROW_BIG) {
       bool done;
       unsigned long long* obuf = (unsigned long long*)outv;
-      if (n + 3 <= 16 * 4 * BLOCK) done = linear_select_sort_regs<16>(src, n, K, base_id, hist, scratch, obuf, sv, si);
-      else if (n + 3 <= 24 * 4 * BLOCK) done = linear_select_sort_regs<24>(src, n, K, base_id, hist, scratch, obuf, sv, si);
-      else done = linear_select_sort_regs<REG_ROW_BIG / (4 * BLOCK)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      if (n + 3 <= 16 * 4 * BL) done = linear_select_sort_regs<BL, 16>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else if (n + 3 <= 24 * 4 * BL) done = linear_select_sort_regs<BL, 24>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else done = linear_select_sort_regs<BL, REG_ROW_BIG / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      if (done) return;
+      __syncthreads();
+    } else if (LEAN == 3 && n + 3 <= REG_ROW_BIG) {
+      bool done;
+      unsigned long long* obuf = (unsigned long long*)outv;
+      if (n + 3 <= 4 * BL) done = linear_select_sort_regs<BL, 1>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else if (n + 3 <= 2 * 4 * BL) done = linear_select_sort_regs<BL, 2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else if (n + 3 <= 4 * 4 * BL) done = linear_select_sort_regs<BL, 4>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else done = linear_select_sort_regs<BL, (REG_ROW_BIG + 4 * BL - 1) / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       if (done) return;
       __syncthreads();
     }
   }
   if (n <= K) {
-    for (int t = tid; t < Kp2; t += BLOCK) {
+    for (int t = tid; t < Kp2; t += BL) {
       float v = t < n ? src[t] : -INFINITY;
       outv[t] = v;
       outi[t] = (t < n && v != -INFINITY) ? base_id + t : -1;
     }
   } else {
     if (STAGED && !sorted) {
-      for (int e = tid; e < n; e += BLOCK) keys[e] = f2key(src[e]);
+      for (int e = tid; e < n; e += BL) keys[e] = f2key(src[e]);
     }
     // ---- pass 1: bits [31:20] ------------------------------------------------------------
-    for (int b = tid; b < HBINS; b += BLOCK) hist[b] = 0;
+    for (int b = tid; b < HBINS; b += BL) hist[b] = 0;
     __syncthreads();
-    for (int e = tid; e < n; e += BLOCK) atomicAdd(&hist[key_at(e) >> 20], 1);
+    for (int e = tid; e < n; e += BL) atomicAdd(&hist[key_at(e) >> 20], 1);
     __syncthreads();
-    Pick p1 = pick_bin(hist, 4096, K, scratch, scratch + 8);
+    Pick p1 = pick_bin<BL>(hist, 4096, K, scratch, scratch + 3 * NWAVES<BL>);
     int need = K - p1.above;
     // ---- pass 2: bits [19:10] among keys in bin p1 -----------------------------------------
-    for (int b = tid; b < 1024; b += BLOCK) hist[b] = 0;
+    for (int b = tid; b < 1024; b += BL) hist[b] = 0;
     __syncthreads();
-    for (int e = tid; e < n; e += BLOCK) {
+    for (int e = tid; e < n; e += BL) {
       unsigned k = key_at(e);
       if ((int)(k >> 20) == p1.bin) atomicAdd(&hist[(k >> 10) & 1023], 1);
     }
     __syncthreads();
-    Pick p2 = pick_bin(hist, 1024, need, scratch, scratch + 8);
+    Pick p2 = pick_bin<BL>(hist, 1024, need, scratch, scratch + 3 * NWAVES<BL>);
     need -= p2.above;
     // ---- pass 3: bits [9:0] ----------------------------------------------------------------
     const unsigned pre22 = ((unsigned)p1.bin << 10) | (unsigned)p2.bin;
-    for (int b = tid; b < 1024; b += BLOCK) hist[b] = 0;
+    for (int b = tid; b < 1024; b += BL) hist[b] = 0;
     __syncthreads();
-    for (int e = tid; e < n; e += BLOCK) {
+    for (int e = tid; e < n; e += BL) {
       unsigned k = key_at(e);
       if ((k >> 10) == pre22) atomicAdd(&hist[k & 1023], 1);
     }
     __syncthreads();
-    Pick p3 = pick_bin(hist, 1024, need, scratch, scratch + 8);
+    Pick p3 = pick_bin<BL>(hist, 1024, need, scratch, scratch + 3 * NWAVES<BL>);
     const unsigned thr = (pre22 << 10) | (unsigned)p3.bin;   // the K-th largest key
     const int ties = need - p3.above;                         // how many keys == thr to keep (>= 1)
     // ---- compaction in ascending column order ------------------------------------------------
-    const int cs = (n + BLOCK - 1) / BLOCK;
+    const int cs = (n + BL - 1) / BL;
     const int e0 = min(tid * cs, n), e1 = min(e0 + cs, n);
     int ngt = 0, neq = 0;
     for (int e = e0; e < e1; e++) { unsigned k = key_at(e); ngt += k > thr; neq += k == thr; }
     int tot;
-    const int eq_before = block_exscan(neq, scratch, tot);
+    const int eq_before = block_exscan<BL>(neq, scratch, tot);
     const int eq_take = max(0, min(neq, ties - eq_before));
-    int pos = block_exscan(ngt + eq_take, scratch, tot);
+    int pos = block_exscan<BL>(ngt + eq_take, scratch, tot);
     int eq_seen = 0;
     for (int e = e0; e < e1; e++) {
       unsigned k = key_at(e);
@@ -577,22 +572,22 @@ __global__ __launch_bounds__(BLOCK, LEAN == 1 ? 4 : LEAN == 2 ? 2 : 1) void topk
         pos++;
       }
     }
-    for (int t = K + tid; t < Kp2; t += BLOCK) { outv[t] = -INFINITY; outi[t] = -1; }
+    for (int t = K + tid; t < Kp2; t += BL) { outv[t] = -INFINITY; outi[t] = -1; }
   }
   __syncthreads();
 
   if (sorted) {   // bitonic sort, descending score, ascending id among equal scores
-    const int ept = LEAN != 0 ? 0 : Kp2 / BLOCK;
-    if (ept == 8) { bitonic_regs<8>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 4) { bitonic_regs<4>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 2) { bitonic_regs<2>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 1) { bitonic_regs<1>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 16) { bitonic_regs<16>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 32) { bitonic_regs<32>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    const int ept = LEAN != 0 ? 0 : Kp2 / BL;
+    if (ept == 8) { bitonic_regs<BL, 8>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    else if (ept == 4) { bitonic_regs<BL, 4>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    else if (ept == 2) { bitonic_regs<BL, 2>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    else if (ept == 1) { bitonic_regs<BL, 1>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    else if (ept == 16) { bitonic_regs<BL, 16>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
+    else if (ept == 32) { bitonic_regs<BL, 32>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
     else {
       for (int size = 2; size <= Kp2; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-          for (int t = tid; t < (Kp2 >> 1); t += BLOCK) {
+          for (int t = tid; t < (Kp2 >> 1); t += BL) {
             const int lo = 2 * t - (t & (stride - 1));
             const int hi = lo + stride;
             const bool desc = ((lo & size) == 0);
@@ -605,7 +600,7 @@ __global__ __launch_bounds__(BLOCK, LEAN == 1 ? 4 : LEAN == 2 ? 2 : 1) void topk
       }
     }
   }
-  for (int t = tid; t < K; t += BLOCK) { sv[t] = outv[t]; si[t] = outi[t]; }
+  for (int t = tid; t < K; t += BL) { sv[t] = outv[t]; si[t] = outi[t]; }
 }
 
 }  // namespace
@@ -618,34 +613,36 @@ int dsa_topk_launch(const float* logits, int S, int64_t ld, const int32_t* row_b
   if (S == 0) return DSA_OK;
   int Kp2 = 1;
   while (Kp2 < K) Kp2 <<= 1;
-  const size_t fixed = (size_t)HBINS * 4 + 64 + (size_t)Kp2 * 8 + (size_t)LIN_SPARE * 8;
+  const size_t buffers = (size_t)HBINS * 4 + (size_t)Kp2 * 8 + (size_t)LIN_SPARE * 8;
+  const size_t fixed = buffers + SCRATCH<256> * 4, wide = buffers + SCRATCH<1024> * 4;
   const size_t staged = fixed + (size_t)width * 4;
-  // sorted rows that fit a register variant need no staging buffer: rows of up to REG_ROW elements go to the
-  // 128-register kernel (four workgroups per compute unit), longer ones up to REG_ROW_BIG to its 256-register
-  // form in a second launch; each launch skips the other's rows
-  const bool lean = sorted && width + 3 <= REG_ROW_BIG;
-  const bool use_staged = !lean && staged <= 160 * 1024;
-  const size_t smem = use_staged ? staged : fixed;
-  const int none = 0x7fffffff;
-  if (lean) {
-    auto k1 = topk_kernel<false, 1>;
-    auto k2 = topk_kernel<false, 2>;
-    if (dsa_reserve_lds((const void*)k1, smem) != hipSuccess ||
-        dsa_reserve_lds((const void*)k2, smem) != hipSuccess)
-      DSA_FAIL(DSA_ERR_LAUNCH, "dsa_topk: cannot reserve %zu bytes of LDS", smem);
-    const int split = REG_ROW - 3;
-    k1<<<dim3(S), dim3(BLOCK), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, sorted, scores, ids,
-                                           width, -1, split);
-    if (width > split)
-      k2<<<dim3(S), dim3(BLOCK), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, sorted, scores,
-                                             ids, width, split, none);
+  // Sorted rows that fit a register variant need no staging buffer: rows of up to REG_ROW elements go to the
+  // 128-register kernel (four workgroups per compute unit), longer ones to a second launch; each launch skips the
+  // other's rows.  Only the device knows how long they are (a window of a wide key array may be short).  With no more rows
+  // than compute units the 1024-thread kernel takes them all and finishes a row sooner (us, top-k 2048: one row of 4096
+  // 11.5 -> 7.7, of 32768 29 -> 13.7, 48 windows of 7000 in a wide array 65 -> 10; 300 rows of 8000 16.5 against 17.6).
+  const int none = 0x7fffffff, split = REG_ROW - 3;
+  auto launch = [&](auto kern, int block, size_t smem, int n_above, int n_upto) {
+    if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return false;
+    kern<<<dim3(S), dim3(block), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, sorted, scores, ids,
+                                             width, n_above, n_upto);
+    return true;
+  };
+  bool ok;
+  if (sorted && S <= WIDE_ROWS) {
+    ok = launch(topk_kernel<1024, false, 3>, 1024, wide, -1, none);
+  } else if (sorted) {
+    ok = launch(topk_kernel<256, false, 1>, 256, fixed, -1, split);
+    if (ok && width > split) {
+      if (width + 3 <= REG_ROW_BIG) ok = launch(topk_kernel<256, false, 2>, 256, fixed, split, none);
+      else ok = launch(topk_kernel<1024, false, 3>, 1024, wide, split, none);
+    }
+  } else if (staged <= 160 * 1024) {
+    ok = launch(topk_kernel<256, true, 0>, 256, staged, -1, none);
   } else {
-    auto kern = use_staged ? topk_kernel<true, 0> : topk_kernel<false, 0>;
-    if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess)
-      DSA_FAIL(DSA_ERR_LAUNCH, "dsa_topk: cannot reserve %zu bytes of LDS", smem);
-    kern<<<dim3(S), dim3(BLOCK), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, sorted, scores, ids,
-                                             width, -1, none);
+    ok = launch(topk_kernel<256, false, 0>, 256, fixed, -1, none);
   }
+  if (!ok) DSA_FAIL(DSA_ERR_LAUNCH, "dsa_topk: cannot reserve LDS");
   DSA_CHECK_LAUNCH("dsa_topk");
   return DSA_OK;
 }

@@ -277,6 +277,33 @@ def test_indexer_kernel_with_fused_rotation_matches_rotating_first(gpu):
         assert (a.float() - b.float()).abs().max().item() <= 3e-2 * scale
 
 
+@pytest.mark.parametrize("copies", [1, 24])       # 13 rows: the 1024-thread kernel; 312 rows: the 256-thread ones
+@pytest.mark.parametrize("K", [64, 1000, 2048])
+def test_topk_row_lengths_at_the_edges_of_its_variants(gpu, copies, K):
+    """Rows whose lengths sit at the register variants' limits, in an array wider than any of them, plus rows of one
+    element, of equal values and of repeated values (ties by ascending column)."""
+    from loongforge_amd import ops
+
+    lengths = [1, 2, 255, 256, 257, 4093, 4094, 8190, 9213, 9214, 16382, 33789, 33790]
+    width = 34000
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(len(lengths), width, generator=g)
+    x[3] = 0.5
+    x[4] = torch.randint(0, 9, (width,), generator=g).float()
+    begin = torch.tensor([(7 * i) % 11 for i in range(len(lengths))], dtype=torch.int32)
+    end = begin + torch.tensor(lengths, dtype=torch.int32)
+    rep = lambda t: t.repeat(copies, *([1] * (t.ndim - 1))).to(gpu)                    # noqa: E731
+    sc, ids = ops.topk(rep(x), K, rep(begin), rep(end))
+    for i, n in enumerate(lengths):
+        row = x[i, int(begin[i]): int(end[i])]
+        v, order = torch.sort(row, descending=True, stable=True)
+        k = min(K, n)
+        for c in range(copies):
+            got_s, got_i = sc[c * len(lengths) + i].cpu(), ids[c * len(lengths) + i].cpu()
+            assert torch.equal(got_s[:k], v[:k]) and torch.equal(got_i[:k].long(), order[:k] + int(begin[i])), (n, c)
+            assert (got_i[k:] == -1).all() and torch.isinf(got_s[k:]).all(), (n, c)
+
+
 @pytest.mark.parametrize("Hi", [32, 64])
 def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
     """Windows cut into parts over workgroups: shared ones (a chunk behind cached keys), unrelated ones (sequences of a
