@@ -283,6 +283,17 @@ int dsa_mla_absorb(const void* a, int64_t a_tok, int64_t a_head, const void* w, 
                    int64_t c_head, int S, int H, int k_dim, int n_dim, void* stream);
 
 /*
+ * The whole query side at once: q_up [S, H, 192] (128 no-position and 64 rotary columns of a row, pairs adjacent) ->
+ * query [S, H, 576]: columns 0..511 as dsa_mla_absorb, columns 512..575 the rotated pe part as dsa_rope_rows writes it
+ * (multi_latent_attention.py:1177-1204 of the reference).  Strides in elements, multiples of 8; rows start on 16-byte
+ * boundaries; cos, sin [positions, 64] fp32 or bf16; position of token s: positions[s], or s / batch when NULL.
+ */
+int dsa_absorb_rope_query(const void* q_up, int64_t up_tok, int64_t up_head, const void* w, void* query,
+                          int64_t q_tok, int64_t q_head, const void* cos, const void* sin, int cos_sin_f32,
+                          const int32_t* positions, int batch, int S, int H, int out_pairing, void* stream);
+
+
+/*
  * Rotary position embedding of the MLA query / key rows, fused with the copies around it.  Per
  * (token, head) the call copies a "main" part of d_main bf16 elements between two strided tensors
  * (main_src NULL: no main part) and rotates a "pe" part of emb_dim bf16 elements, pair by pair:

@@ -39,6 +39,7 @@ SIGNATURES = {
     "dsa_attn_dist": (_i, [_vp, _i, _i, _i, _i, _i64, _i64, _f, _vp, _vp]),
     "dsa_attn_dist_qk": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]),
     "dsa_mla_absorb": (_i, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _i, _i, _i, _i, _vp]),
+    "dsa_absorb_rope_query": (_i, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp]),
     "dsa_rope_rows": (_i, [_vp, _i64, _i64, _vp, _i64, _i64, _i, _vp, _i64, _i64, _vp, _i64, _i64, _i, _vp, _vp, _i, _vp,
                            _i, _i, _i, _i, _i, _i, _vp]),
     "dsa_rope_headsum_inverse": (_i, [_vp, _i64, _i64, _vp, _i64, _i, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp]),

@@ -6,116 +6,248 @@
 // surrounds them:
 //   * query side   A = the no-position part of the up-projected query, [S, H, 128] inside [S, H, 192];
 //                  W = W_UK^T [H, 512, 128]; C = the latent part of the attention query,
-//                  [S, H, 512] inside [S, H, 576] (the rotary part is written by the rotary kernel)
+//                  [S, H, 512] inside [S, H, 576]; the rotary part of the same rows (64 elements of
+//                  a row, pairs adjacent in the source) can be rotated into place by the same kernel
 //   * output side  A = the attention output [S, H, 512]; W = W_UV [H, 128, 512];
 //                  C = [S, H * 128], the input of the output projection
-// HBM-bound (137 GFLOP against 1.3 GB at S = 8192, H = 128): one workgroup holds a head's 128 KB weight
-// matrix in LDS for many row blocks; a wave computes C^T[n, s] = W[n, :] . A[s, :]^T for 32 rows s at a
-// time, the weights as the MFMA A operand (LDS row reads), the activation rows as the B operand straight
-// from global memory (16 bytes per lane, next block requested before this block's MFMAs).  With C^T in
-// the accumulators a lane owns one output row, so the result leaves in 16-byte pieces.
+// HBM-bound at both ends: few rows read the weights (16.8 MB at 128 heads) once, many rows move their
+// own 1.3 KB per (token, head).
+//
+// Many rows (absorb_kernel): one workgroup holds a head's 128 KB weight matrix in LDS for many row
+// blocks; a wave computes C^T[n, s] = W[n, :] . A[s, :]^T for 32 rows s at a time, the weights as the
+// MFMA A operand (LDS row reads), the activation rows as the B operand straight from global memory (16
+// bytes per lane, next block requested before this block's MFMAs).  With C^T in the accumulators a lane
+// owns one output row; four column tiles go through an 8 KB strip per wave, so that a store instruction
+// writes four 256-byte row segments instead of 32 of 32 bytes.
+// Few rows (absorb_few_kernel): a wave per (head, 32 columns) reads its weight rows straight into
+// registers and walks the row blocks: 4x the waves, no trip of the weights through LDS.
 #include "mla_tile.h"
+#include "rope_quad.h"
 
 namespace {
 
-constexpr int ROWS = 128;                 // activation rows per workgroup step (32 per wave)
+constexpr int EMB = 64;                   // rotary elements of a row
 
-template <int K, int N>
-__global__ __launch_bounds__(256, 1) void absorb_kernel(
-    const __bf16* __restrict__ a, long a_tok, long a_head, const __bf16* __restrict__ w,
-    __bf16* __restrict__ c, long c_tok, long c_head, int S, int H, int splits) {
+struct AbsorbArgs {
+  const __bf16* a; long a_tok, a_head;
+  const __bf16* w;
+  __bf16* c; long c_tok, c_head;
+  int S, H;
+  // rotary part (pe_src == nullptr: none): same strides as a and c; position of a token: positions[s] or s / batch
+  const unsigned short* pe_src; unsigned short* pe_dst;
+  const void* cos; const void* sin; int cs_f32;
+  const int* positions; int batch; int out_pairing;
+};
+
+__device__ __forceinline__ long position_of(const AbsorbArgs& p, int s) { return p.positions ? p.positions[s] : s / p.batch; }
+__device__ __forceinline__ rope::QuadTables tables_of(const AbsorbArgs& p, long pos, int q) {
+  return p.out_pairing == rope::ADJ ? rope::load_tables<rope::ADJ>(p.cos, p.sin, p.cs_f32, pos, q, EMB)
+                                    : rope::load_tables<rope::SPLIT>(p.cos, p.sin, p.cs_f32, pos, q, EMB);
+}
+__device__ __forceinline__ void store_rotated(const AbsorbArgs& p, const rope::Quad& x, const rope::QuadTables& t, int s, int h, int q) {
+  unsigned short* dst = p.pe_dst + (size_t)s * p.c_tok + (size_t)h * p.c_head;
+  if (p.out_pairing == rope::ADJ) rope::store_quad<rope::ADJ>(rope::rotate<false>(x, t), dst, q, EMB);
+  else rope::store_quad<rope::SPLIT>(rope::rotate<false>(x, t), dst, q, EMB);
+}
+
+// WAVES * 32 rows per step.  ROPE: the rotary part of the same rows, read one step ahead like the rows themselves.
+template <int K, int N, int WAVES, bool ROPE>
+__global__ __launch_bounds__(64 * WAVES, 1) void absorb_kernel(AbsorbArgs p, int splits) {
   // W[h] in LDS as K / 64 column groups of [N rows][128 bytes]; inside a group the 16-byte chunk c of row n sits in slot
   // (c & 7) ^ swz(n): the layout of the attention kernels' key tiles, whose 128-bit row reads are bank-conflict free
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int KS = K / 16, NT = N / 32, CH = K / 8;                          // k-steps, output tiles, chunks per row
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, g = lane >> 5;
+  constexpr int ROWS = 32 * WAVES;
+  constexpr int ST = 16 / WAVES, SB = 64 * ST, SC = 4 * ST;                    // tiles, bytes and chunks of a strip row: 32 KB in all
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.x / splits, part = blockIdx.x % splits;
+  unsigned char* strip = smem + (size_t)N * K * 2 + wave * (32 * SB);          // [32 rows][SB], chunks XORed with the row
 
   // ---- the head's weights into LDS -------------------------------------------------------
   {
-    const uint4* src = (const uint4*)(w + (size_t)h * N * K);
-    for (int e = tid; e < N * CH; e += 256) {
+    const uint4* src = (const uint4*)(p.w + (size_t)h * N * K);
+#pragma unroll 8
+    for (int e = tid; e < N * CH; e += 64 * WAVES) {
       const int n = e / CH, ch = e % CH;
       *(uint4*)(smem + (size_t)(ch >> 3) * (N * 128) + n * 128 + (((ch & 7) ^ mla::swz(n & 31)) << 4)) = src[e];
     }
   }
   __syncthreads();
 
-  const int nblk = (S + ROWS - 1) / ROWS;
+  const int nblk = (p.S + ROWS - 1) / ROWS;
   const int b_lo = (int)((long)nblk * part / splits), b_hi = (int)((long)nblk * (part + 1) / splits);
   auto load_rows = [&](int blk, bf16x8 (&t)[KS]) {
-    const int s = min(blk * ROWS + wave * 32 + r, S - 1);
-    const bf16x8* p = (const bf16x8*)(a + (size_t)s * a_tok + (size_t)h * a_head) + g;
+    const int s = min(blk * ROWS + wave * 32 + r, p.S - 1);
+    const bf16x8* src = (const bf16x8*)(p.a + (size_t)s * p.a_tok + (size_t)h * p.a_head) + g;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) t[ks] = p[2 * ks];
+    for (int ks = 0; ks < KS; ks++) t[ks] = src[2 * ks];
+  };
+  // rotary quad of (row 8 i + lane / 8 of the wave's 32, quad lane % 8)
+  const int qd = lane & 7;
+  auto pe_row = [&](int blk, int i) { return min(blk * ROWS + wave * 32 + 8 * i + (lane >> 3), p.S - 1); };
+  auto load_pe = [&](int blk, uint4 (&t)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      t[i] = *(const uint4*)(p.pe_src + (size_t)pe_row(blk, i) * p.a_tok + (size_t)h * p.a_head + 8 * qd);
   };
   bf16x8 cur[KS], nxt[KS];
-  if (b_lo < b_hi) load_rows(b_lo, cur);
+  uint4 pe[4], pe_nxt[4];
+  if (b_lo < b_hi) {
+    load_rows(b_lo, cur);
+    if (ROPE) load_pe(b_lo, pe);
+  }
   for (int blk = b_lo; blk < b_hi; blk++) {
-    if (blk + 1 < b_hi) load_rows(blk + 1, nxt);
-    const int s = blk * ROWS + wave * 32 + r;
-    unsigned short* out = (unsigned short*)c + (size_t)min(s, S - 1) * c_tok + (size_t)h * c_head + 8 * g;
-#pragma unroll 2
-    for (int nt = 0; nt < NT; nt++) {
-      f32x16 acc;
+    const int s0 = blk * ROWS + wave * 32;
+    if (ROPE) {                              // the tables' rows first: they are waited for with the next rows still on their way
+      rope::QuadTables tb[4];
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[e] = 0.f;
-      const int n = 32 * nt + r;
-      const unsigned char* wrow = smem + n * 128;
-      const int sw = mla::swz(r);
+      for (int i = 0; i < 4; i++) tb[i] = tables_of(p, position_of(p, pe_row(blk, i)), qd);
+      if (blk + 1 < b_hi) { load_rows(blk + 1, nxt); load_pe(blk + 1, pe_nxt); }
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        const bf16x8 wv = *(const bf16x8*)(wrow + (ks >> 2) * (N * 128) + ((((2 * ks + g) & 7) ^ sw) << 4));
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, cur[ks], acc, 0, 0, 0);
+      for (int i = 0; i < 4; i++)
+        if (s0 + 8 * i + (lane >> 3) < p.S)
+          store_rotated(p, rope::adjacent_pairs(pe[i]), tb[i], s0 + 8 * i + (lane >> 3), h, qd);
+    } else if (blk + 1 < b_hi) {
+      load_rows(blk + 1, nxt);
+    }
+#pragma unroll 1
+    for (int nq = 0; nq < NT / ST; nq++) {
+#pragma unroll
+      for (int ni = 0; ni < ST; ni++) {
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[e] = 0.f;
+        const unsigned char* wrow = smem + (32 * (ST * nq + ni) + r) * 128;
+        const int sw = mla::swz(r);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          const bf16x8 wv = *(const bf16x8*)(wrow + (ks >> 2) * (N * 128) + ((((2 * ks + g) & 7) ^ sw) << 4));
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, cur[ks], acc, 0, 0, 0);
+        }
+        uint4 o[2];
+        acc_row_to_16B(acc, 1.0f, o);
+        *(uint4*)(strip + r * SB + (((4 * ni + g) ^ (r & (SC - 1))) << 4)) = o[0];
+        *(uint4*)(strip + r * SB + (((4 * ni + 2 + g) ^ (r & (SC - 1))) << 4)) = o[1];
       }
-      uint4 o[2];
-      acc_row_to_16B(acc, 1.0f, o);          // every lane takes part; rows past the end are not stored
-      if (s < S) {
-        *(uint4*)(out + 32 * nt) = o[0];
-        *(uint4*)(out + 32 * nt + 16) = o[1];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < SC / 2; i++) {
+        const int row = (64 / SC) * i + lane / SC, ch = lane % SC;
+        const uint4 v = *(const uint4*)(strip + row * SB + ((ch ^ (row & (SC - 1))) << 4));
+        if (s0 + row < p.S)
+          *(uint4*)((unsigned short*)p.c + (size_t)(s0 + row) * p.c_tok + (size_t)h * p.c_head + 32 * ST * nq + 8 * ch) = v;
       }
+      __builtin_amdgcn_wave_barrier();
     }
     if (blk + 1 < b_hi) {
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) cur[ks] = nxt[ks];
+      if (ROPE) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) pe[i] = pe_nxt[i];
+      }
     }
   }
 }
 
+// One wave per (head, 32 output columns) and FEW_STEP rows, plus one per head for their rotary part.
+constexpr int FEW_STEP = 32;
 template <int K, int N>
-int launch(const void* a, int64_t a_tok, int64_t a_head, const void* w, void* c, int64_t c_tok, int64_t c_head,
-           int S, int H, hipStream_t st) {
-  const int nblk = (S + ROWS - 1) / ROWS;
-  int splits = (512 + H - 1) / H;
-  if (splits > nblk) splits = nblk;
-  if (splits < 1) splits = 1;
-  const size_t smem = (size_t)K * N * 2;
-  auto kern = absorb_kernel<K, N>;
-  static bool configured = false;            // per template instance
-  if (!configured) {
-    if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return -2;
-    configured = true;
+__global__ __launch_bounds__(256, 2) void absorb_few_kernel(AbsorbArgs p) {
+  constexpr int KS = K / 16, NT = N / 32;
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int task = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int per = p.pe_src ? NT + 1 : NT;
+  const int h = task / per, nt = task % per;
+  if (h >= p.H) return;
+  const int s_lo = (int)blockIdx.y * FEW_STEP, s_hi = min(s_lo + FEW_STEP, p.S);
+  if (nt == NT) {
+    const int q = lane & 7;
+    for (int s = s_lo + (lane >> 3); s < s_hi; s += 8)
+      store_rotated(p, rope::load_quad<rope::ADJ>(p.pe_src + (size_t)s * p.a_tok + (size_t)h * p.a_head, q, EMB),
+                    tables_of(p, position_of(p, s), q), s, h, q);
+    return;
   }
-  kern<<<dim3((unsigned)(H * splits)), dim3(256), smem, st>>>((const __bf16*)a, (long)a_tok, (long)a_head, (const __bf16*)w,
-                                                               (__bf16*)c, (long)c_tok, (long)c_head, S, H, splits);
+  bf16x8 wv[KS];
+  const bf16x8* wp = (const bf16x8*)(p.w + ((size_t)h * N + 32 * nt + r) * K) + g;
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) wv[ks] = wp[2 * ks];
+  {
+    const int s = s_lo + r;
+    const bf16x8* ap = (const bf16x8*)(p.a + (size_t)min(s, p.S - 1) * p.a_tok + (size_t)h * p.a_head) + g;
+    bf16x8 av[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) av[ks] = ap[2 * ks];
+    __builtin_amdgcn_sched_barrier(0);       // all loads in flight before the first product
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[ks], av[ks], acc, 0, 0, 0);
+    uint4 o[2];
+    acc_row_to_16B(acc, 1.0f, o);            // every lane takes part; rows past the end are not stored
+    if (s < p.S) {
+      unsigned short* out = (unsigned short*)p.c + (size_t)s * p.c_tok + (size_t)h * p.c_head + 32 * nt + 8 * g;
+      *(uint4*)out = o[0];
+      *(uint4*)(out + 16) = o[1];
+    }
+  }
+}
+
+// Rows up to which the weights are better re-read per 32 rows (query side with rotary part, 128 heads: 1 row 5.4 against 12.7 us,
+// 48 rows 13.2 against 15.5, 100 rows 20.8 against 17.0).
+constexpr int FEW_ROWS = 64;
+
+template <int K, int N>
+int launch(const AbsorbArgs& p, hipStream_t st) {
+  if (p.S <= FEW_ROWS) {
+    const int tasks = p.H * (N / 32 + (p.pe_src ? 1 : 0));
+    absorb_few_kernel<K, N><<<dim3((tasks + 3) / 4, (p.S + FEW_STEP - 1) / FEW_STEP), dim3(256), 0, st>>>(p);
+    return 0;
+  }
+  constexpr int WAVES = K == 128 ? 8 : 4;    // rows of 1 KB in registers twice: four waves
+  const int nblk = (p.S + 32 * WAVES - 1) / (32 * WAVES);
+  int splits = (256 + p.H - 1) / p.H;        // one workgroup per compute unit: its LDS holds one weight matrix
+  if (splits > nblk) splits = nblk;
+  const size_t smem = (size_t)K * N * 2 + 32768;
+  auto kern = K == 128 && p.pe_src ? absorb_kernel<K, N, WAVES, K == 128> : absorb_kernel<K, N, WAVES, false>;
+  if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return -2;
+  kern<<<dim3((unsigned)(p.H * splits)), dim3(64 * WAVES), smem, st>>>(p, splits);
   return 0;
+}
+
+int absorb(const AbsorbArgs& p, int k_dim, int n_dim, const char* who, hipStream_t st) {
+  DSA_REQUIRE(p.S >= 0 && p.H > 0, "%s: bad sizes S=%d H=%d", who, p.S, p.H);
+  DSA_REQUIRE((k_dim == 128 && n_dim == 512) || (k_dim == 512 && n_dim == 128),
+              "%s: (k, n) must be (128, 512) (query side) or (512, 128) (output side), got (%d, %d)", who, k_dim, n_dim);
+  DSA_REQUIRE(p.a_tok % 8 == 0 && p.a_head % 8 == 0 && p.c_tok % 8 == 0 && p.c_head % 8 == 0,
+              "%s: row strides must be multiples of 8 elements", who);
+  DSA_REQUIRE(((uintptr_t)p.a % 16) == 0 && ((uintptr_t)p.w % 16) == 0 && ((uintptr_t)p.c % 16) == 0, "%s: misaligned pointer", who);
+  if (p.S == 0) return DSA_OK;
+  const int rc = k_dim == 128 ? launch<128, 512>(p, st) : launch<512, 128>(p, st);
+  if (rc == -2) DSA_FAIL(DSA_ERR_LAUNCH, "%s: cannot reserve LDS", who);
+  DSA_CHECK_LAUNCH(who);
+  return DSA_OK;
 }
 
 }  // namespace
 
 extern "C" int dsa_mla_absorb(const void* a, int64_t a_tok, int64_t a_head, const void* w, void* c, int64_t c_tok,
                               int64_t c_head, int S, int H, int k_dim, int n_dim, void* stream) {
-  DSA_REQUIRE(S >= 0 && H > 0, "dsa_mla_absorb: bad sizes S=%d H=%d", S, H);
-  DSA_REQUIRE((k_dim == 128 && n_dim == 512) || (k_dim == 512 && n_dim == 128),
-              "dsa_mla_absorb: (k, n) must be (128, 512) (query side) or (512, 128) (output side), got (%d, %d)", k_dim, n_dim);
-  DSA_REQUIRE(a_tok % 8 == 0 && a_head % 8 == 0 && c_tok % 8 == 0 && c_head % 8 == 0,
-              "dsa_mla_absorb: row strides must be multiples of 8 elements");
-  DSA_REQUIRE(((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)c % 16) == 0, "dsa_mla_absorb: misaligned pointer");
-  if (S == 0) return DSA_OK;
-  int rc;
-  if (k_dim == 128) rc = launch<128, 512>(a, a_tok, a_head, w, c, c_tok, c_head, S, H, (hipStream_t)stream);
-  else rc = launch<512, 128>(a, a_tok, a_head, w, c, c_tok, c_head, S, H, (hipStream_t)stream);
-  if (rc == -2) DSA_FAIL(DSA_ERR_LAUNCH, "dsa_mla_absorb: cannot reserve LDS");
-  DSA_CHECK_LAUNCH("dsa_mla_absorb");
-  return DSA_OK;
+  const AbsorbArgs p{(const __bf16*)a, (long)a_tok, (long)a_head, (const __bf16*)w, (__bf16*)c, (long)c_tok, (long)c_head, S, H,
+                     nullptr, nullptr, nullptr, nullptr, 0, nullptr, 1, 0};
+  return absorb(p, k_dim, n_dim, "dsa_mla_absorb", (hipStream_t)stream);
+}
+
+extern "C" int dsa_absorb_rope_query(const void* q_up, int64_t up_tok, int64_t up_head, const void* w, void* query,
+                                     int64_t q_tok, int64_t q_head, const void* cos, const void* sin, int cos_sin_f32,
+                                     const int32_t* positions, int batch, int S, int H, int out_pairing, void* stream) {
+  DSA_REQUIRE(q_up && query && cos && sin, "dsa_absorb_rope_query: null pointer");
+  DSA_REQUIRE(positions != nullptr || batch > 0, "dsa_absorb_rope_query: batch must be positive when no positions are given");
+  DSA_REQUIRE(out_pairing == 0 || out_pairing == 1, "dsa_absorb_rope_query: pairing must be 0 (adjacent) or 1 (split)");
+  DSA_REQUIRE(((uintptr_t)cos % 16) == 0 && ((uintptr_t)sin % 16) == 0, "dsa_absorb_rope_query: misaligned pointer");
+  const AbsorbArgs p{(const __bf16*)q_up, (long)up_tok, (long)up_head, (const __bf16*)w, (__bf16*)query, (long)q_tok, (long)q_head, S, H,
+                     (const unsigned short*)q_up + 128, (unsigned short*)query + 512, cos, sin, cos_sin_f32, positions, batch, out_pairing};
+  return absorb(p, 128, 512, "dsa_absorb_rope_query", (hipStream_t)stream);
 }

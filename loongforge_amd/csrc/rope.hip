@@ -12,11 +12,11 @@
 // (elements i, i + emb_dim/2); source and destination pairings are independent, and the cos / sin
 // rows are indexed with the pairing of the rotated side (destination in the forward direction,
 // source in the inverse one): c1_i = cos[2i], c2_i = cos[2i+1] or c1_i = cos[i], c2_i = cos[i + emb_dim/2].
-#include "dsa_common.h"
+#include "rope_quad.h"
 
 namespace {
 
-constexpr int ADJ = 0, SPLIT = 1;
+using namespace rope;
 
 struct RopeArgs {
   const unsigned short* main_src; long ms_tok, ms_head;     // strides in elements; nullptr: no main part
@@ -30,21 +30,8 @@ struct RopeArgs {
   int tokens, heads;
 };
 
-__device__ __forceinline__ void load4(const void* base, long idx, int f32, float (&o)[4]) {
-  if (f32) {
-    const f32x4 v = *(const f32x4*)((const float*)base + idx);
-    o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
-  } else {
-    const uint2 v = *(const uint2*)((const unsigned short*)base + idx);
-    o[0] = __builtin_bit_cast(float, v.x << 16); o[1] = __builtin_bit_cast(float, v.x & 0xffff0000u);
-    o[2] = __builtin_bit_cast(float, v.y << 16); o[3] = __builtin_bit_cast(float, v.y & 0xffff0000u);
-  }
-}
-
 template <int IN, int OUT, bool INVERSE>
 __global__ __launch_bounds__(256) void rope_rows_kernel(RopeArgs a) {
-#pragma clang fp contract(off)     // products and sums stay separate IEEE operations
-  const int half = a.emb >> 1;
   const int main_chunks = a.main_src ? a.d_main >> 3 : 0;
   const int quads = a.emb >> 3;                       // groups of four pairs
   const int per_head = main_chunks + quads;
@@ -61,56 +48,7 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RopeArgs a) {
       const int q = c - main_chunks;
       const unsigned short* src = a.pe_src + tok * a.ps_tok + head * a.ps_head;
       unsigned short* dst = a.pe_dst + tok * a.pd_tok + head * a.pd_head;
-      float x1[4], x2[4];
-      if (IN == ADJ) {
-        const uint4 v = *(const uint4*)(src + 8 * q);
-        const unsigned w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          x1[k] = __builtin_bit_cast(float, w[k] << 16);
-          x2[k] = __builtin_bit_cast(float, w[k] & 0xffff0000u);
-        }
-      } else {
-        load4(src, 4 * q, 0, x1);
-        load4(src, half + 4 * q, 0, x2);
-      }
-      constexpr int CS = INVERSE ? IN : OUT;           // pairing of the rotated side
-      float c1[4], c2[4], s1[4], s2[4];
-      const long crow = pos * a.emb;
-      if (CS == ADJ) {
-        float ca[4], cb[4], sa[4], sb[4];
-        load4(a.cos, crow + 8 * q, a.cs_f32, ca);
-        load4(a.cos, crow + 8 * q + 4, a.cs_f32, cb);
-        load4(a.sin, crow + 8 * q, a.cs_f32, sa);
-        load4(a.sin, crow + 8 * q + 4, a.cs_f32, sb);
-        c1[0] = ca[0]; c2[0] = ca[1]; c1[1] = ca[2]; c2[1] = ca[3]; c1[2] = cb[0]; c2[2] = cb[1]; c1[3] = cb[2]; c2[3] = cb[3];
-        s1[0] = sa[0]; s2[0] = sa[1]; s1[1] = sa[2]; s2[1] = sa[3]; s1[2] = sb[0]; s2[2] = sb[1]; s1[3] = sb[2]; s2[3] = sb[3];
-      } else {
-        load4(a.cos, crow + 4 * q, a.cs_f32, c1);
-        load4(a.cos, crow + half + 4 * q, a.cs_f32, c2);
-        load4(a.sin, crow + 4 * q, a.cs_f32, s1);
-        load4(a.sin, crow + half + 4 * q, a.cs_f32, s2);
-      }
-      float y1[4], y2[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        if (!INVERSE) {
-          y1[k] = x1[k] * c1[k] - x2[k] * s1[k];
-          y2[k] = x2[k] * c2[k] + x1[k] * s2[k];
-        } else {
-          y1[k] = x1[k] * c1[k] + x2[k] * s2[k];
-          y2[k] = (-x1[k]) * s1[k] + x2[k] * c2[k];
-        }
-      }
-      if (OUT == ADJ) {
-        uint4 o;
-        o.x = pack_bf16x2(y1[0], y2[0]); o.y = pack_bf16x2(y1[1], y2[1]);
-        o.z = pack_bf16x2(y1[2], y2[2]); o.w = pack_bf16x2(y1[3], y2[3]);
-        *(uint4*)(dst + 8 * q) = o;
-      } else {
-        *(uint2*)(dst + 4 * q) = make_uint2(pack_bf16x2(y1[0], y1[1]), pack_bf16x2(y1[2], y1[3]));
-        *(uint2*)(dst + half + 4 * q) = make_uint2(pack_bf16x2(y2[0], y2[1]), pack_bf16x2(y2[2], y2[3]));
-      }
+      rotate_quad<IN, OUT, INVERSE>(src, dst, q, a.emb, pos, a.cos, a.sin, a.cs_f32);
     }
   }
 }

@@ -593,8 +593,11 @@ class FusedAbsorbRopeQuery(torch.autograd.Function):
         query = q_up.new_empty(S, nheads, d_out + emb)
         positions = _token_positions(cu_seqlens_q, S, cp_rank, cp_size)
         out_pairing = ops.ROPE_ADJACENT if rotary_interleaved else ops.ROPE_SPLIT
-        ops.mla_absorb_into(q3[:, :, :d_nope], w_uk_t, query[:, :, :d_out])
-        ops.rope_rows(q3[:, :, d_nope:], query[:, :, d_out:], cos, sin, ops.ROPE_ADJACENT, out_pairing, False, positions, batch)
+        if emb == 64:
+            ops.absorb_rope_query_into(q3, w_uk_t, query, cos, sin, out_pairing, positions, batch)
+        else:
+            ops.mla_absorb_into(q3[:, :, :d_nope], w_uk_t, query[:, :, :d_out])
+            ops.rope_rows(q3[:, :, d_nope:], query[:, :, d_out:], cos, sin, ops.ROPE_ADJACENT, out_pairing, False, positions, batch)
         ctx.save_for_backward(q3, w_uk_t, cos, sin)
         ctx.args = (positions, batch, out_pairing, d_nope, d_out, emb, q_up.shape)
         return query.view(*lead, nheads, d_out + emb)

@@ -831,6 +831,33 @@ def mla_absorb_into(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor) -> None:
                                       c.stride(1), S, H, k, c.shape[2], _stream(a)), "dsa_mla_absorb")
 
 
+def absorb_rope_query_into(q_up: torch.Tensor, w: torch.Tensor, query: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                           out_pairing: int, positions: Optional[torch.Tensor] = None, batch: int = 1) -> None:
+    """``query[s, h, :512] = q_up[s, h, :128] @ w[h].T`` and ``query[s, h, 512:] = rope(q_up[s, h, 128:])`` (pairs adjacent
+    in ``q_up``), one kernel: :func:`mla_absorb_into` and :func:`rope_rows` over the rows of ``q_up [S, H, 192]`` and
+    ``query [S, H, 576]``.  No autograd."""
+    _need_gpu(q_up, w, query, cos, sin, positions)
+    if q_up.dtype != torch.bfloat16 or query.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise ValueError("mla_absorb expects bf16 tensors")
+    S, H = q_up.shape[:2]
+    if q_up.ndim != 3 or q_up.shape[2] != 192 or query.shape != (S, H, 576) or w.shape != (H, 512, 128):
+        raise ValueError("absorb_rope_query: shapes q_up %s, w %s, query %s do not fit" % (tuple(q_up.shape), tuple(w.shape), tuple(query.shape)))
+    if q_up.stride(2) != 1 or query.stride(2) != 1:
+        raise ValueError("mla_absorb: rows must be contiguous")
+    w = _c(w)
+    cos2, sin2 = _cos_sin(cos, sin, 64)
+    if positions is not None:
+        positions = _c(positions.int())
+        if positions.numel() != S:
+            raise ValueError("positions must hold one entry per token")
+    lib = _lib.load()
+    with torch.cuda.device(q_up.device):
+        _lib.check(lib.dsa_absorb_rope_query(q_up.data_ptr(), q_up.stride(0), q_up.stride(1), w.data_ptr(), query.data_ptr(),
+                                             query.stride(0), query.stride(1), cos2.data_ptr(), sin2.data_ptr(),
+                                             int(cos2.dtype == torch.float32), positions.data_ptr() if positions is not None else None,
+                                             int(batch), S, H, int(out_pairing), _stream(q_up)), "dsa_absorb_rope_query")
+
+
 class MlaAbsorb(torch.autograd.Function):
     """``out[s, h, :] = a[s, h, :] @ w[h].T`` through the HIP kernel, written into ``out`` (a view of a larger
     tensor, returned as is and marked dirty), with the two gradient products as plain library GEMMs."""

@@ -43,6 +43,25 @@ def test_absorb_kernel_in_place_views_and_gradients(gpu):
         ops.mla_absorb_into(a.detach(), w.detach()[:, :100], torch.empty(200, 8, 100, dtype=torch.bfloat16, device=gpu))
 
 
+@pytest.mark.parametrize("S,H", [(1, 3), (33, 16), (64, 2), (65, 5), (300, 128), (777, 1)])
+@pytest.mark.parametrize("pairing,dtype", [(0, torch.bfloat16), (1, torch.float32)])
+def test_absorb_and_rope_in_one_kernel(gpu, S, H, pairing, dtype):
+    """The query side in one kernel, for few and for many rows and ragged row blocks: bit-equal to the projection and the
+    rotary kernel run one after the other, with and without explicit positions."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(S)
+    q_up = torch.randn(S, H, 192, generator=g).to(torch.bfloat16).to(gpu)
+    w = (torch.randn(H, 512, 128, generator=g) * 128 ** -0.5).to(torch.bfloat16).to(gpu)
+    cos, sin = (torch.randn(S + 7, 64, generator=g).to(dtype).to(gpu) for _ in range(2))
+    for pos in (None, torch.randint(0, S + 7, (S,), generator=g, dtype=torch.int32).to(gpu)):
+        query, ref = (torch.zeros(S, H, 576, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+        ops.absorb_rope_query_into(q_up, w, query, cos, sin, pairing, pos, 2)
+        ops.mla_absorb_into(q_up[:, :, :128], w, ref[:, :, :512])
+        ops.rope_rows(q_up[:, :, 128:], ref[:, :, 512:], cos, sin, 0, pairing, False, pos, 2)
+        assert torch.equal(query, ref)
+
+
 class _Linear(torch.nn.Module):
     def __init__(self, n_in, n_out, **_):
         super().__init__()
