@@ -160,6 +160,18 @@ int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, const float*
                     void* stream);
 
 /*
+ * Windows of the causal queries [chunk_offset, chunk_offset + S) over packed sequences, cu[ncu] (i32, or i64 if cu_i64)
+ * their cumulative lengths (NULL: one sequence): ks[i] = start of the query's sequence, ke[i] = chunk_offset + i + 1;
+ * queries past the last sequence get ks = 0.  total (may be NULL; host-visible): the summed length of the sequences.
+ */
+int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, int chunk_offset, int32_t* ks, int32_t* ke,
+                       int32_t* total, void* stream);
+/*
+ * Position of packed token t + offset inside its own sequence, t in [0, tokens) (0 past the last sequence).
+ */
+int dsa_thd_positions(const void* cu, int cu_i64, int ncu, int tokens, int64_t offset, int32_t* positions, void* stream);
+
+/*
  * Sparse MQA-MLA attention forward.  Slot t of query i (global position q_start + i) is valid iff
  * ids[i,t] != -1, 0 <= ids[i,t] < Skv and ids[i,t] <= q_start + i.  Over the valid slots:
  *   s = q[i,h,:] . kv[ids[i,t],:]   P = softmax_t(s * sm_scale)   out[i,h,:] = sum_t P kv[ids[i,t], :d_v]

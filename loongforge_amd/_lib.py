@@ -28,6 +28,8 @@ SIGNATURES = {
     "dsa_indexer_topk_fwd_static": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "dsa_indexer_bwd_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "dsa_indexer_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "dsa_indexer_window": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
+    "dsa_thd_positions": (_i, [_vp, _i, _i, _i, _i64, _vp, _vp]),
     "dsa_sparse_mla_fwd": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp]),
     "dsa_sparse_mla_fwd_ex": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _i, _vp]),
     "dsa_sparse_mla_fwd_workspace_bytes": (_sz, [_i, _i, _i, _i]),
@@ -81,6 +83,16 @@ def load():
             fn.argtypes = args
         _lib = lib
         return _lib
+
+
+def load_host():
+    """The native host layer of :mod:`loongforge_amd.ops` (csrc/host), a torch extension over the same library."""
+    load()
+    try:
+        from . import _dsa_host
+    except ImportError as e:
+        raise DsaError("_dsa_host.so is missing or does not load; build it with `python -m loongforge_amd.csrc.build`") from e
+    return _dsa_host
 
 
 def load_bench():

@@ -3,6 +3,7 @@
     python -m loongforge_amd.csrc.build [--force]
 
 libdsa_hip.so    the C-ABI library of kernels (include/dsa_hip.h): every csrc/*.hip
+_dsa_host.so     the native host layer of loongforge_amd/ops.py (a torch extension): csrc/host/*.cpp
 libdsa_bench.so  measurement aids that only the benchmark loads (include/dsa_hip_bench.h):
                  csrc/bench/*.hip plus the error-state object
 
@@ -14,11 +15,13 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libdsa_hip.so")
 BENCH_LIB = os.path.join(PKG, "libdsa_bench.so")
+HOST_LIB = os.path.join(PKG, "_dsa_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -56,11 +59,41 @@ def _compile(src, force):
     return obj, log
 
 
+def _compile_host(force):
+    """csrc/host/host.cpp -> object file (host code only: g++)."""
+    src, obj = os.path.join(HERE, "host", "host.cpp"), os.path.join(OBJ_DIR, "host.o")
+    newest = max(os.path.getmtime(p) for p in [src, os.path.join(os.path.dirname(PKG), "include", "dsa_hip.h")])
+    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= newest:
+        return obj
+    from torch.utils.cpp_extension import include_paths
+
+    includes = include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"]]
+    res = subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+                          "-DUSE_ROCM", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_dsa_host"]
+                         + ["-I" + p for p in includes] + ["-c", src, "-o", obj], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("compiling host.cpp failed:\n" + res.stdout + res.stderr)
+    return obj
+
+
+def _link_host(obj):
+    from torch.utils.cpp_extension import library_paths
+
+    libs = ["-l" + n for n in ("dsa_hip", "c10", "c10_hip", "torch", "torch_cpu", "torch_python", "amdhip64")]
+    res = subprocess.run([os.environ.get("CXX", "g++"), "-shared", "-o", HOST_LIB, obj, "-L" + PKG]
+                         + ["-L" + p for p in library_paths()] + ["-L/opt/rocm/lib"] + libs + ["-Wl,-rpath,$ORIGIN"],
+                         capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
+
+
 def build(force=False, verbose=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs, bench_srcs = _sources(), _bench_sources()
     with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
+        host = ex.submit(_compile_host, force)
         results = list(ex.map(lambda s: _compile(s, force), srcs + bench_srcs))
+        host_obj = host.result()
     objs = [o for o, _ in results[:len(srcs)]]
     bench_objs = [o for o, _ in results[len(srcs):]] + [os.path.join(OBJ_DIR, "api.o")]
     for _, log in results:
@@ -73,6 +106,8 @@ def build(force=False, verbose=True):
             res = subprocess.run(cmd, capture_output=True, text=True)
             if res.returncode != 0:
                 raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
+    if force or not os.path.exists(HOST_LIB) or os.path.getmtime(HOST_LIB) < max(os.path.getmtime(host_obj), os.path.getmtime(LIB)):
+        _link_host(host_obj)
     return LIB
 
 

@@ -1,0 +1,505 @@
+// Native host layer of the tensor-level entry points (loongforge_amd/ops.py): argument checks, output and workspace
+// allocation and the call into the C-ABI library, one C++ call per operation.  In Python the same steps cost 13 - 20 us
+// per operation and the custom-op dispatcher another 8 - 10, more than most kernels of a decode step run; here 4 - 6 us
+// in all (one decode step, six operations: 150 us of host time before).
+//
+// Every function returns None, without having done anything, when a tensor is not a plain one (a subclass, a fake or
+// functional tensor, a traced or transformed call, or one whose gradient is being recorded): the caller then goes
+// through the registered custom op, whose implementation calls back here with force = true.
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <hip/hip_runtime_api.h>
+
+#include "../../../include/dsa_hip.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+namespace {
+
+// ---- plain tensors --------------------------------------------------------------------------------
+bool plain_call() {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+  constexpr c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::Tracer,
+                                     c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchVmapMode});
+  return !c10::impl::tls_local_dispatch_key_set().included_.has_any(odd);
+}
+bool plain_tensor(const Tensor& t, bool grad) {
+  constexpr c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchBatched,
+                                     c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
+  return !t.key_set().has_any(odd) && !(grad && t.requires_grad());
+}
+bool plain_tensor(const OptTensor& t, bool grad) { return !t || plain_tensor(*t, grad); }
+template <class... T>
+bool plain(const T&... t) {
+  if (!plain_call()) return false;
+  const bool grad = at::GradMode::is_enabled();
+  return (plain_tensor(t, grad) && ...);
+}
+#define PLAIN_OR_NONE(...) do { if (!force && !plain(__VA_ARGS__)) return py::none(); } while (0)
+
+// ---- checks ---------------------------------------------------------------------------------------
+void need_gpu(const Tensor& t) {
+  TORCH_CHECK(t.is_cuda(), "DSA kernels need tensors on a HIP device; got a ", c10::DeviceTypeName(t.device().type(), true), " tensor");
+}
+void need_gpu(const OptTensor& t) { if (t) need_gpu(*t); }
+template <class... T>
+void need_gpus(const T&... t) { (need_gpu(t), ...); }
+
+void check(int rc, const char* what) {
+  if (rc == 0) return;
+  const std::string msg = dsa_last_error();
+  if (rc == DSA_ERR_BAD_ARG) throw py::value_error(std::string(what) + ": " + msg);
+  PyErr_SetString(py::module_::import("loongforge_amd._lib").attr("DsaError").ptr(),
+                  (std::string(what) + " failed (status " + std::to_string(rc) + "): " + msg).c_str());
+  throw py::error_already_set();
+}
+// One call into the library, without the interpreter lock (a launch blocks while the queue is full).
+template <class F, class... A>
+void run(const char* what, F f, A... a) {
+  RECORD_FUNCTION(what, c10::ArrayRef<const c10::IValue>{});     // shows as a range in torch's profiler
+  int rc;
+  {
+    py::gil_scoped_release unlocked;
+    rc = f(a...);
+  }
+  check(rc, what);
+}
+#define REQUIRE(cond, ...) do { if (!(cond)) throw py::value_error(c10::str(__VA_ARGS__)); } while (0)
+
+// The device of a call: current for its duration, with its current stream.
+struct Call {
+  c10::DeviceGuard guard;
+  void* stream;
+  explicit Call(const Tensor& t) : guard(t.device()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+};
+
+Tensor f32(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
+Tensor i32(const Tensor& t) { return t.to(at::kInt).contiguous(); }
+Tensor make(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) { return at::empty(shape, like.options().dtype(type)); }
+at::ScalarType payload_type(bool raw) { return raw ? at::kByte : at::kFloat8_e4m3fn; }
+const void* ptr(const OptTensor& t) { return t && t->numel() ? t->const_data_ptr() : nullptr; }
+template <class P> P* out_ptr(const Tensor& t) { return t.numel() ? (P*)t.data_ptr() : nullptr; }
+
+Tensor as_u8(const Tensor& t) {
+  REQUIRE(t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte, "expected an fp8-e4m3 (or raw uint8) tensor, got ",
+          t.scalar_type());
+  return t.contiguous();
+}
+
+// ---- quantisers -------------------------------------------------------------------------------------
+py::object quant_rowwise(const Tensor& x_, double eps, bool pow2, bool force) {
+  PLAIN_OR_NONE(x_);
+  need_gpus(x_);
+  REQUIRE(x_.scalar_type() == at::kBFloat16, "quant_rowwise_e4m3 expects bf16 input, got ", x_.scalar_type());
+  const Tensor x = x_.contiguous();
+  const int64_t cols = x.size(-1), rows = x.numel() / std::max<int64_t>(cols, 1);
+  Call call(x);
+  Tensor x8 = make(x.sizes(), payload_type(force), x), scale_inv = make(x.sizes().slice(0, x.dim() - 1), at::kFloat, x);
+  run("dsa_quant_rowwise_e4m3", dsa_quant_rowwise_e4m3, x.const_data_ptr(), rows, (int)cols, x8.data_ptr(), (float*)scale_inv.data_ptr(), (float)eps, pow2, call.stream);
+  return py::make_tuple(x8, scale_inv);
+}
+
+py::object rotate_quant(const Tensor& x_, double eps, bool pow2, bool want_payload, bool want_rotated, bool force) {
+  PLAIN_OR_NONE(x_);
+  need_gpus(x_);
+  REQUIRE(x_.scalar_type() == at::kBFloat16, "rotate_quant_e4m3 expects bf16 input, got ", x_.scalar_type());
+  REQUIRE(x_.size(-1) == 128, "rotate_quant_e4m3 rotates rows of 128 elements, got ", x_.size(-1));
+  REQUIRE(want_payload || want_rotated, "rotate_quant_e4m3: no output requested");
+  const Tensor x = x_.contiguous();
+  Call call(x);
+  const auto lead = x.sizes().slice(0, x.dim() - 1);
+  Tensor x8 = want_payload ? make(x.sizes(), payload_type(force), x) : make({0}, payload_type(force), x);
+  Tensor scale_inv = want_payload ? make(lead, at::kFloat, x) : make({0}, at::kFloat, x);
+  Tensor y = want_rotated ? make(x.sizes(), at::kBFloat16, x) : make({0}, at::kBFloat16, x);
+  run("dsa_rotate_quant_e4m3", dsa_rotate_quant_e4m3, x.const_data_ptr(), x.numel() / 128, 128, want_payload ? x8.data_ptr() : nullptr, want_payload ? (float*)scale_inv.data_ptr() : nullptr, want_rotated ? y.data_ptr() : nullptr, (float)eps, pow2, call.stream);
+  return py::make_tuple(x8, scale_inv, y);
+}
+
+py::object quant_weights(const Tensor& x_, const Tensor& weights_, double factor, bool rotate, double eps, bool pow2, bool force) {
+  PLAIN_OR_NONE(x_, weights_);
+  need_gpus(x_, weights_);
+  REQUIRE(x_.scalar_type() == at::kBFloat16 && x_.size(-1) == 128, "quant_rowwise_e4m3_weights expects bf16 rows of 128 elements");
+  const auto lead = x_.sizes().slice(0, x_.dim() - 1);
+  REQUIRE(weights_.sizes() == lead, "quant_rowwise_e4m3_weights: one weight per row expected, got ", weights_.sizes(), " for rows ", lead);
+  const Tensor x = x_.contiguous(), weights = f32(weights_);
+  Call call(x);
+  Tensor x8 = make(x.sizes(), payload_type(force), x), scale_inv = make(lead, at::kFloat, x), scaled = make(lead, at::kFloat, x);
+  run("dsa_quant_rowwise_e4m3_weights", dsa_quant_rowwise_e4m3_weights, x.const_data_ptr(), x.numel() / 128, 128, x8.data_ptr(), (float*)scale_inv.data_ptr(), (float)eps, pow2, rotate, (const float*)weights.const_data_ptr(), (float)factor, (float*)scaled.data_ptr(), call.stream);
+  return py::make_tuple(x8, scale_inv, scaled);
+}
+
+py::object indexer_front(const Tensor& x_, int64_t rows_per_token, const OptTensor& ln_weight_, const OptTensor& ln_bias_, double ln_eps,
+                         const OptTensor& cos_, const OptTensor& sin_, int64_t pairing, const OptTensor& positions_, int64_t batch,
+                         bool rotate, const OptTensor& weights_, double factor, bool want_payload, bool want_rows, double eps, bool pow2,
+                         bool force) {
+  PLAIN_OR_NONE(x_, ln_weight_, ln_bias_, cos_, sin_, positions_, weights_);
+  need_gpus(x_);
+  REQUIRE(x_.scalar_type() == at::kBFloat16 && x_.size(-1) == 128, "indexer_front_e4m3 expects bf16 rows of 128 elements");
+  const Tensor x = x_.contiguous();
+  const int64_t rows = x.numel() / 128;
+  REQUIRE(rows_per_token > 0 && rows % rows_per_token == 0, "indexer_front_e4m3: ", rows, " rows are not a multiple of ", rows_per_token,
+          " rows per token");
+  REQUIRE(ln_weight_.has_value() == ln_bias_.has_value(), "indexer_front_e4m3: LayerNorm needs weight and bias");
+  const int64_t tokens = rows / rows_per_token;
+  int tables_f32 = 0;
+  OptTensor cos, sin, positions, ln_weight, ln_bias, weights;
+  if (pairing >= 0) {
+    REQUIRE(cos_ && sin_ && cos_->scalar_type() == sin_->scalar_type() &&
+            (cos_->scalar_type() == at::kFloat || cos_->scalar_type() == at::kBFloat16),
+            "indexer_front_e4m3: cos / sin must both be fp32 or bf16 tables");
+    REQUIRE(cos_->size(-1) == 64 && sin_->size(-1) == 64 && cos_->numel() == sin_->numel(),
+            "indexer_front_e4m3: cos / sin rows must have 64 entries");
+    cos = cos_->contiguous();
+    sin = sin_->contiguous();
+    tables_f32 = cos->scalar_type() == at::kFloat;
+    if (positions_) {
+      positions = i32(*positions_);
+      REQUIRE(positions->numel() == tokens, "indexer_front_e4m3: one position per token expected");
+    } else {
+      REQUIRE((tokens + batch - 1) / batch <= cos->numel() / 64, "indexer_front_e4m3: cos / sin tables are shorter than the sequence");
+    }
+  }
+  if (ln_weight_) {
+    ln_weight = f32(*ln_weight_);
+    ln_bias = f32(*ln_bias_);
+    REQUIRE(ln_weight->numel() == 128 && ln_bias->numel() == 128, "indexer_front_e4m3: LayerNorm weight and bias must have 128 entries");
+  }
+  if (weights_) {
+    REQUIRE(want_payload && weights_->numel() == rows, "indexer_front_e4m3: one weight per row expected, together with the payload");
+    weights = f32(*weights_);
+  }
+  Call call(x);
+  const auto lead = x.sizes().slice(0, x.dim() - 1);
+  Tensor x8 = want_payload ? make(x.sizes(), payload_type(force), x) : make({0}, payload_type(force), x);
+  Tensor scale_inv = want_payload ? make(lead, at::kFloat, x) : make({0}, at::kFloat, x);
+  Tensor y = want_rows ? make(x.sizes(), at::kBFloat16, x) : make({0}, at::kBFloat16, x);
+  Tensor scaled = weights ? make(lead, at::kFloat, x) : make({0}, at::kFloat, x);
+  run("dsa_indexer_front_e4m3", dsa_indexer_front_e4m3, x.const_data_ptr(), rows, 128, (int)rows_per_token, (const float*)ptr(ln_weight), (const float*)ptr(ln_bias), (float)ln_eps, ptr(cos), ptr(sin), tables_f32, (int)pairing, (const int32_t*)ptr(positions), (int)batch, rotate, out_ptr<void>(x8), out_ptr<float>(scale_inv), out_ptr<void>(y), (float)eps, pow2, (const float*)ptr(weights), (float)factor, out_ptr<float>(scaled), call.stream);
+  return py::make_tuple(x8, scale_inv, y, scaled);
+}
+
+// ---- indexer ----------------------------------------------------------------------------------------
+struct IndexerShape { int S, Hi, Sk; };
+IndexerShape indexer_shape(const Tensor& q8, const Tensor& q_w, const Tensor& k8, const Tensor& k_scale, const Tensor& ks, const Tensor& ke) {
+  need_gpus(q8, q_w, k8, k_scale, ks, ke);
+  REQUIRE(q8.dim() == 3 && k8.dim() == 2 && q_w.dim() == 2, "indexer expects q8 [S,H,128], k8 [Sk,128], q_w [S,H]");
+  REQUIRE(q8.size(2) == 128 && k8.size(1) == 128, "Only support dim with size 128.");
+  const int64_t S = q8.size(0), Hi = q8.size(1), Sk = k8.size(0);
+  REQUIRE(q_w.size(0) == S && q_w.size(1) == Hi && k_scale.dim() == 1 && k_scale.size(0) == Sk && ks.dim() == 1 && ks.size(0) == S &&
+          ke.dim() == 1 && ke.size(0) == S, "indexer: inconsistent shapes");
+  return {(int)S, (int)Hi, (int)Sk};
+}
+
+py::object indexer_topk(const Tensor& q8_, const Tensor& q_w_, const Tensor& k8_, const Tensor& k_scale_, const Tensor& ks_, const Tensor& ke_,
+                        int64_t K, bool sort, bool force) {
+  PLAIN_OR_NONE(q8_, q_w_, k8_, k_scale_, ks_, ke_);
+  const auto [S, Hi, Sk] = indexer_shape(q8_, q_w_, k8_, k_scale_, ks_, ke_);
+  const Tensor q8 = as_u8(q8_), k8 = as_u8(k8_), q_w = f32(q_w_), k_scale = f32(k_scale_), ks = i32(ks_), ke = i32(ke_);
+  Call call(q8);
+  Tensor scores = make({S, K}, at::kFloat, q8), ids = make({S, K}, at::kInt, q8);
+  const size_t nbytes = dsa_indexer_topk_workspace_bytes(S, Sk, (int)K);
+  Tensor ws = make({(int64_t)std::max<size_t>(nbytes, 1)}, at::kByte, q8);
+  run("dsa_indexer_topk_fwd", dsa_indexer_topk_fwd, q8.const_data_ptr(), (const float*)q_w.const_data_ptr(), k8.const_data_ptr(), (const float*)k_scale.const_data_ptr(), (const int32_t*)ks.const_data_ptr(), (const int32_t*)ke.const_data_ptr(), S, Hi, Sk, (int)K, sort, (float*)scores.data_ptr(), (int32_t*)ids.data_ptr(), ws.data_ptr(), nbytes, call.stream);
+  return py::make_tuple(scores, ids);
+}
+
+py::object topk(const Tensor& logits_, int64_t K, const OptTensor& row_begin, const OptTensor& row_end, const OptTensor& id_base, bool sort,
+                bool force) {
+  PLAIN_OR_NONE(logits_, row_begin, row_end, id_base);
+  need_gpus(logits_, row_begin, row_end, id_base);
+  REQUIRE(logits_.dim() == 2 && logits_.scalar_type() == at::kFloat, "topk expects a 2-D fp32 tensor");
+  const Tensor logits = logits_.stride(1) == 1 ? logits_ : logits_.contiguous();
+  const int64_t S = logits.size(0), width = logits.size(1);
+  OptTensor rb, re, ib;
+  if (row_begin) rb = i32(*row_begin);
+  if (row_end) re = i32(*row_end);
+  if (id_base) ib = i32(*id_base);
+  Call call(logits);
+  Tensor scores = make({S, K}, at::kFloat, logits), ids = make({S, K}, at::kInt, logits);
+  run("dsa_topk", dsa_topk, (const float*)logits.const_data_ptr(), (int)S, S > 0 ? logits.stride(0) : width, (const int32_t*)ptr(rb), (const int32_t*)ptr(re), (int)width, (const int32_t*)ptr(ib), (int)K, sort, (float*)scores.data_ptr(), (int32_t*)ids.data_ptr(), call.stream);
+  return py::make_tuple(scores, ids);
+}
+
+// ---- windows of packed sequences ------------------------------------------------------------------------
+// Whether the sequences cover the queries is only known on the device; the kernel leaves their length in pinned memory
+// and wait() looks at it, called after the kernels that use the window were launched: the device has work while the
+// host waits.  (Under graph capture nothing is checked.)
+struct WindowCheck {
+  Tensor total;
+  int64_t need = 0;
+  hipEvent_t done = nullptr;
+  WindowCheck() = default;
+  WindowCheck(const WindowCheck&) = delete;
+  ~WindowCheck() { if (done) { (void)hipEventSynchronize(done); (void)hipEventDestroy(done); } }
+  void wait() {
+    if (!done) return;
+    hipError_t rc;
+    {
+      py::gil_scoped_release unlocked;
+      rc = hipEventSynchronize(done);
+    }
+    TORCH_CHECK(rc == hipSuccess, "indexer window: ", hipGetErrorString(rc));
+    REQUIRE(*total.const_data_ptr<int>() >= need, "indexer: inconsistent shapes (the packed sequences hold ", *total.const_data_ptr<int>(),
+            " tokens, the queries end at ", need, ")");
+  }
+};
+
+Tensor seqlens(const Tensor& cu, const c10::Device& device) {
+  Tensor t = cu.to(device);
+  if (t.scalar_type() != at::kInt && t.scalar_type() != at::kLong) t = t.to(at::kLong);
+  return t.contiguous();
+}
+
+py::tuple indexer_window(const OptTensor& cu_, int64_t S, int64_t chunk_offset, const Tensor& like) {
+  need_gpus(like);
+  OptTensor cu;
+  if (cu_) cu = seqlens(*cu_, like.device());
+  Call call(like);
+  Tensor window = make({2, S}, at::kInt, like);
+  auto check = std::make_unique<WindowCheck>();
+  if (cu) {
+    hipStreamCaptureStatus capturing;
+    if (hipStreamIsCapturing((hipStream_t)call.stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
+      check->total = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+      check->need = chunk_offset + S;
+    }
+  }
+  run("dsa_indexer_window", dsa_indexer_window, cu ? ptr(cu) : nullptr, cu && cu->scalar_type() == at::kLong, cu ? (int)cu->numel() : 0, (int)S,
+      (int)chunk_offset, out_ptr<int32_t>(window), out_ptr<int32_t>(window) + S,
+      check->need ? (int32_t*)check->total.data_ptr() : nullptr, call.stream);
+  if (check->need && (hipEventCreateWithFlags(&check->done, hipEventDisableTiming) != hipSuccess ||
+                      hipEventRecord(check->done, (hipStream_t)call.stream) != hipSuccess))
+    throw std::runtime_error("indexer window: no event");
+  return py::make_tuple(window.select(0, 0), window.select(0, 1), std::move(check));
+}
+
+py::object thd_positions(const Tensor& cu_, int64_t tokens, int64_t offset) {
+  if (!cu_.is_cuda() || !plain(cu_) || cu_.numel() < 2) return py::none();
+  const Tensor cu = seqlens(cu_, cu_.device());
+  Call call(cu);
+  Tensor pos = make({tokens}, at::kInt, cu);
+  run("dsa_thd_positions", dsa_thd_positions, cu.const_data_ptr(), cu.scalar_type() == at::kLong, (int)cu.numel(), (int)tokens, offset,
+      out_ptr<int32_t>(pos), call.stream);
+  return py::cast(pos);
+}
+
+// ---- sparse MLA ---------------------------------------------------------------------------------------
+void mla_shape(const Tensor& q, const Tensor& kv, const Tensor& ids) {
+  need_gpus(q, kv, ids);
+  REQUIRE(q.dim() == 3 && kv.dim() == 2 && ids.dim() == 2, "sparse MLA expects q [S,H,576], kv [Skv,576], ids [S,K]");
+  REQUIRE(q.scalar_type() == at::kBFloat16 && kv.scalar_type() == at::kBFloat16, "sparse MLA expects bf16 q and kv");
+  REQUIRE(q.size(2) == 576 && kv.size(1) == 576, "you should assign dim otherwise: d_qk must be 576 (512 latent + 64 rope)");
+  REQUIRE(ids.size(0) == q.size(0), "ids and q disagree on the number of queries");
+  REQUIRE(ids.size(1) % 64 == 0, "top-k must be padded to a multiple of 64 (pad ids with -1)");
+}
+
+py::object mla_fwd(const Tensor& q_, const Tensor& kv_, const Tensor& ids_, int64_t q_start, double sm_scale, int64_t d_v, int64_t p_out_mode,
+                   const OptTensor& attn_sink, int64_t p_out_skip, bool force) {
+  PLAIN_OR_NONE(q_, kv_, ids_, attn_sink);
+  mla_shape(q_, kv_, ids_);
+  const Tensor q = q_.contiguous(), kv = kv_.contiguous(), ids = i32(ids_);
+  const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);
+  OptTensor sink;
+  if (attn_sink) {
+    need_gpus(attn_sink);
+    REQUIRE(attn_sink->numel() == H, "attn_sink must hold one logit per head (", H, "), got ", attn_sink->numel());
+    sink = f32(attn_sink->reshape({H}));
+  }
+  REQUIRE(p_out_mode == 0 || (p_out_skip >= 0 && p_out_skip < K && p_out_skip % 32 == 0),
+          "p_out_skip must be a multiple of 32 in [0, top-k), got ", p_out_skip);
+  Call call(q);
+  Tensor out = make({S, H, d_v}, at::kBFloat16, q), lse = make({S, H}, at::kFloat, q);
+  Tensor p_out = p_out_mode == 0 ? make({0}, at::kBFloat16, q)
+                                 : make({S, H, K - p_out_skip}, p_out_mode == 2 ? at::kFloat : at::kBFloat16, q);
+  const size_t nbytes = dsa_sparse_mla_fwd_workspace_bytes((int)S, (int)H, (int)Skv, (int)K);
+  Tensor ws;
+  if (nbytes) ws = make({(int64_t)nbytes}, at::kByte, q);
+  run("dsa_sparse_mla_fwd", dsa_sparse_mla_fwd_ws, q.const_data_ptr(), kv.const_data_ptr(), (const int32_t*)ids.const_data_ptr(), (int)S, (int)H, (int)Skv, (int)K, (int)q_start, (float)sm_scale, (int)d_v, out.data_ptr(), (float*)lse.data_ptr(), p_out_mode ? p_out.data_ptr() : nullptr, p_out_mode == 2, (const float*)ptr(sink), (int)p_out_skip, nbytes ? ws.data_ptr() : nullptr, nbytes, call.stream);
+  return py::make_tuple(out, lse, p_out);
+}
+
+py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, const Tensor& dout_, const Tensor& ids_, const Tensor& lse_,
+                   int64_t q_start, double sm_scale, int64_t d_v, const py::function& workspace, bool force) {
+  PLAIN_OR_NONE(q_, kv_, out_, dout_, ids_, lse_);
+  mla_shape(q_, kv_, ids_);
+  need_gpus(out_, dout_, lse_);
+  const Tensor q = q_.contiguous(), kv = kv_.contiguous(), ids = i32(ids_), out = out_.contiguous(), lse = f32(lse_);
+  const Tensor dout = dout_.to(at::kBFloat16).contiguous();
+  const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);
+  REQUIRE(out.sizes() == at::IntArrayRef({S, H, d_v}) && dout.sizes() == out.sizes() && lse.sizes() == at::IntArrayRef({S, H}),
+          "sparse_mla_bwd: out/dout must be [S,H,d_v] and lse [S,H]");
+  Tensor dq = at::empty_like(q), dkv = at::empty_like(kv);
+  const size_t full = dsa_sparse_mla_bwd_workspace_bytes((int)S, (int)H, (int)Skv, (int)K);
+  const auto [ws, nbytes] = py::cast<std::pair<Tensor, size_t>>(workspace(full, q.device()));
+  Call call(q);
+  run("dsa_sparse_mla_bwd", dsa_sparse_mla_bwd, q.const_data_ptr(), kv.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
+      (const int32_t*)ids.const_data_ptr(), (const float*)lse.const_data_ptr(), (int)S, (int)H, (int)Skv, (int)K, (int)q_start, (float)sm_scale,
+      (int)d_v, dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), nbytes, call.stream);
+  return py::make_tuple(dq, dkv);
+}
+
+py::object attn_dist(const Tensor& p_, double sm_scale, bool force) {
+  PLAIN_OR_NONE(p_);
+  need_gpus(p_);
+  REQUIRE(p_.dim() == 3 && (p_.scalar_type() == at::kBFloat16 || p_.scalar_type() == at::kFloat), "attn_dist expects p_out [S,H,K] in bf16 or fp32");
+  const Tensor p = p_.stride(2) == 1 ? p_ : p_.contiguous();
+  const int64_t S = p.size(0), H = p.size(1), K = p.size(2);
+  Call call(p);
+  Tensor target = make({S, K}, at::kFloat, p);
+  run("dsa_attn_dist", dsa_attn_dist, p.const_data_ptr(), p.scalar_type() == at::kFloat, (int)S, (int)H, (int)K, S > 0 ? p.stride(0) : H * K, p.stride(1), (float)sm_scale, (float*)target.data_ptr(), call.stream);
+  return py::cast(target);
+}
+
+py::object kl_loss(const Tensor& scores_, const Tensor& target_, double eps, bool force) {
+  PLAIN_OR_NONE(scores_, target_);
+  need_gpus(scores_, target_);
+  REQUIRE(scores_.dim() == 2 && target_.sizes() == scores_.sizes(), "indexer_kl_loss expects scores and target of one shape [S, K]");
+  const int64_t S = scores_.size(0), K = scores_.size(1);
+  Tensor scores = scores_.to(at::kFloat), target = target_.to(at::kFloat);
+  if (scores.stride(1) != 1) scores = scores.contiguous();
+  if (target.stride(1) != 1) target = target.contiguous();
+  Call call(scores);
+  Tensor row_loss = make({S}, at::kFloat, scores), grad = make({S, K}, at::kFloat, scores);
+  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, (const float*)target.const_data_ptr(), S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
+  return py::make_tuple(row_loss, grad);
+}
+
+// ---- absorption and rotary kernels (write into their arguments) ---------------------------------------
+void need_bf16(const Tensor& a, const Tensor& b, const Tensor& c) {
+  REQUIRE(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && c.scalar_type() == at::kBFloat16,
+          "mla_absorb expects bf16 tensors");
+}
+
+void absorb_into(const Tensor& a, const Tensor& w_, const Tensor& c) {
+  need_gpus(a, w_, c);
+  need_bf16(a, w_, c);
+  REQUIRE(a.dim() == 3 && c.dim() == 3 && w_.dim() == 3 && a.size(0) == c.size(0) && a.size(1) == c.size(1) && w_.size(0) == a.size(1) &&
+          w_.size(1) == c.size(2) && w_.size(2) == a.size(2),
+          "mla_absorb: shapes a ", a.sizes(), ", w ", w_.sizes(), ", c ", c.sizes(), " do not fit c[s,h,:] = a[s,h,:] @ w[h].T");
+  REQUIRE(a.stride(2) == 1 && c.stride(2) == 1, "mla_absorb: rows must be contiguous");
+  const Tensor w = w_.contiguous();
+  Call call(a);
+  run("dsa_mla_absorb", dsa_mla_absorb, a.const_data_ptr(), a.stride(0), a.stride(1), w.const_data_ptr(), c.data_ptr(), c.stride(0), c.stride(1), (int)a.size(0), (int)a.size(1), (int)a.size(2), (int)c.size(2), call.stream);
+}
+
+// cos / sin as contiguous [positions, emb] tables of one type
+std::pair<Tensor, Tensor> tables(const Tensor& cos_, const Tensor& sin_, int64_t emb) {
+  Tensor cos = cos_.reshape({-1, emb}), sin = sin_.reshape({-1, emb});
+  if (cos.scalar_type() != at::kFloat && cos.scalar_type() != at::kBFloat16) { cos = cos.to(at::kFloat); sin = sin.to(at::kFloat); }
+  if (sin.scalar_type() != cos.scalar_type()) sin = sin.to(cos.scalar_type());
+  return {cos.contiguous(), sin.contiguous()};
+}
+
+void absorb_rope_query_into(const Tensor& q_up, const Tensor& w_, const Tensor& query, const Tensor& cos_, const Tensor& sin_, int64_t out_pairing,
+                            const OptTensor& positions_, int64_t batch) {
+  need_gpus(q_up, w_, query, cos_, sin_, positions_);
+  need_bf16(q_up, w_, query);
+  const int64_t S = q_up.size(0), H = q_up.dim() > 1 ? q_up.size(1) : 0;
+  REQUIRE(q_up.dim() == 3 && q_up.size(2) == 192 && query.sizes() == at::IntArrayRef({S, H, 576}) && w_.sizes() == at::IntArrayRef({H, 512, 128}),
+          "absorb_rope_query: shapes q_up ", q_up.sizes(), ", w ", w_.sizes(), ", query ", query.sizes(), " do not fit");
+  REQUIRE(q_up.stride(2) == 1 && query.stride(2) == 1, "mla_absorb: rows must be contiguous");
+  const Tensor w = w_.contiguous();
+  const auto [cos, sin] = tables(cos_, sin_, 64);
+  OptTensor positions;
+  if (positions_) {
+    positions = i32(*positions_);
+    REQUIRE(positions->numel() == S, "positions must hold one entry per token");
+  }
+  Call call(q_up);
+  run("dsa_absorb_rope_query", dsa_absorb_rope_query, q_up.const_data_ptr(), q_up.stride(0), q_up.stride(1), w.const_data_ptr(), query.data_ptr(), query.stride(0), query.stride(1), cos.const_data_ptr(), sin.const_data_ptr(), cos.scalar_type() == at::kFloat, (const int32_t*)ptr(positions), (int)batch, (int)S, (int)H, (int)out_pairing, call.stream);
+}
+
+// The two projections around the attention without autograd: output allocation and kernel in one call.
+py::object absorbed_query(const Tensor& q_up, const Tensor& w, const Tensor& cos, const Tensor& sin, const OptTensor& positions,
+                          int64_t out_pairing) {
+  if (!plain(q_up, w, cos, sin, positions) || q_up.dim() < 3 || w.dim() != 3 || q_up.size(-1) != w.size(2) + 64) return py::none();
+  std::vector<int64_t> shape = q_up.sizes().vec();
+  const int64_t batch = q_up.dim() == 4 ? q_up.size(1) : 1;
+  const Tensor q3 = q_up.dim() == 3 ? q_up : q_up.reshape({-1, q_up.size(-2), q_up.size(-1)});
+  Tensor query = make({q3.size(0), q3.size(1), w.size(1) + 64}, q_up.scalar_type(), q_up);
+  absorb_rope_query_into(q3, w, query, cos, sin, out_pairing, positions, batch);
+  shape.back() = query.size(2);
+  return py::cast(q_up.dim() == 3 ? query : query.view(shape));
+}
+
+py::object absorb(const Tensor& a, const Tensor& w, bool flat) {
+  if (!plain(a, w) || a.dim() < 3 || w.dim() != 3) return py::none();
+  const Tensor a3 = a.dim() == 3 ? a : a.reshape({-1, a.size(-2), a.size(-1)});
+  Tensor out = make({a3.size(0), a3.size(1), w.size(1)}, a.scalar_type(), a);
+  absorb_into(a3, w, out);
+  if (!flat) return py::cast(out);
+  std::vector<int64_t> shape = a.sizes().slice(0, a.dim() - 1).vec();
+  shape.back() *= w.size(1);
+  return py::cast(out.view(shape));
+}
+
+struct Rows { void* p; int64_t tok, head; };
+Rows rows_view(const Tensor& t, const char* what) {
+  REQUIRE(t.scalar_type() == at::kBFloat16 && t.dim() == 3 && (t.size(2) <= 1 || t.stride(2) == 1), what,
+          " must be a bf16 [tokens, heads, width] view with unit inner stride");
+  return {t.data_ptr(), t.stride(0), t.stride(1)};
+}
+
+void rope_rows(const OptTensor& pe_src, const OptTensor& pe_dst, const OptTensor& cos_, const OptTensor& sin_, int64_t in_pairing,
+               int64_t out_pairing, bool inverse, const OptTensor& positions_, int64_t batch, const OptTensor& main_src, const OptTensor& main_dst) {
+  REQUIRE(pe_dst || main_dst, "rope_rows: nothing to do");
+  const Tensor& ref = pe_dst ? *pe_dst : *main_dst;
+  need_gpus(pe_src, pe_dst, cos_, sin_, positions_, main_src, main_dst);
+  const int64_t tokens = ref.size(0), heads = ref.size(1);
+  int64_t emb = 0, d_main = 0;
+  Rows ps{nullptr, 0, 0}, pd{nullptr, 0, 0}, ms{nullptr, 0, 0}, md{nullptr, 0, 0};
+  Tensor cos, sin;
+  OptTensor positions;
+  if (pe_dst) {
+    emb = pe_dst->size(2);
+    REQUIRE(pe_src && pe_src->sizes() == pe_dst->sizes(), "pe_src and pe_dst differ in shape: ", pe_src ? c10::str(pe_src->sizes()) : "none", " vs ",
+            pe_dst->sizes());
+    REQUIRE(cos_ && sin_, "rope_rows: rotary part without cos / sin");
+    ps = rows_view(*pe_src, "pe_src");
+    pd = rows_view(*pe_dst, "pe_dst");
+    std::tie(cos, sin) = tables(*cos_, *sin_, emb);
+    if (positions_) {
+      positions = i32(*positions_);
+      REQUIRE(positions->numel() == tokens, "positions must hold one entry per token");
+    }
+  }
+  if (main_dst) {
+    REQUIRE(main_src && main_src->sizes() == main_dst->sizes() && main_dst->size(0) == tokens && main_dst->size(1) == heads,
+            "main_src / main_dst shapes do not match the pe rows");
+    d_main = main_dst->size(2);
+    ms = rows_view(*main_src, "main_src");
+    md = rows_view(*main_dst, "main_dst");
+  }
+  Call call(ref);
+  run("dsa_rope_rows", dsa_rope_rows, ms.p, ms.tok, ms.head, md.p, md.tok, md.head, (int)d_main, ps.p, ps.tok, ps.head, pd.p, pd.tok, pd.head, (int)emb, emb ? cos.const_data_ptr() : nullptr, emb ? sin.const_data_ptr() : nullptr, emb && cos.scalar_type() == at::kFloat, emb ? (const int32_t*)ptr(positions) : nullptr, (int)batch, (int)tokens, (int)heads, (int)in_pairing, (int)out_pairing, inverse, call.stream);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.doc() = "Native host layer of loongforge_amd.ops";
+  py::class_<WindowCheck>(m, "WindowCheck").def("wait", &WindowCheck::wait);
+#define DEF(name) m.def(#name, torch::wrap_pybind_function(name))
+  DEF(quant_rowwise);
+  DEF(rotate_quant);
+  DEF(quant_weights);
+  DEF(indexer_front);
+  DEF(indexer_topk);
+  DEF(topk);
+  DEF(mla_fwd);
+  DEF(mla_bwd);
+  DEF(attn_dist);
+  DEF(kl_loss);
+  DEF(indexer_window);
+  DEF(thd_positions);
+  DEF(absorb_into);
+  DEF(absorb);
+  DEF(absorb_rope_query_into);
+  DEF(absorbed_query);
+  DEF(rope_rows);
+#undef DEF
+}

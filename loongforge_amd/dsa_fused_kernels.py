@@ -289,21 +289,15 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
                 k_p, 1, k_norm_weight, k_norm_bias, front.k_norm_eps, front.cos, front.sin, front.pairing,
                 front.positions_k, front.batch, rotate)
 
-        if packed_seq_params is None:
-            k_start = torch.zeros(seq_q, dtype=torch.int, device=device)
-        else:
+        cu = None
+        if packed_seq_params is not None:
             cu = packed_seq_params.cu_seqlens_kv_padded
             if cu is None:
                 cu = packed_seq_params.cu_seqlens_kv
-            cu = cu.to(device)
-            seqlens = cu[1:] - cu[:-1]
-            full_seq_ids = torch.repeat_interleave(torch.arange(len(seqlens), device=device, dtype=torch.int), seqlens)
-            local_seq_ids = full_seq_ids[chunk_offset:chunk_offset + seq_q]
-            k_start = cu[local_seq_ids.long()].int()
-        k_end = torch.arange(seq_q, dtype=torch.int, device=device) + chunk_offset + 1
-
+        k_start, k_end, covered = ops.indexer_window(cu, seq_q, chunk_offset, q_fp8)
         index_score_topk, topk_indices = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start, k_end,
                                                           index_topk, DSAIndexerKernelFunction.sorted_output)
+        covered.wait()
         ctx.softmax_scale = softmax_scale
         ctx.rotate = rotate
         ctx.index_topk = index_topk
@@ -618,6 +612,11 @@ class FusedAbsorbRopeQuery(torch.autograd.Function):
 def fused_absorb_rope_query(q_up, w_uk_t, cos, sin, cu_seqlens_q=None, cp_rank: int = 0, cp_size: int = 1,
                             rotary_interleaved: bool = False):
     """``[.., h, 192]`` up-projected query -> ``[.., h, 576]`` attention query (see :class:`FusedAbsorbRopeQuery`)."""
+    if not (torch.compiler.is_compiling() or (torch.is_grad_enabled() and (q_up.requires_grad or w_uk_t.requires_grad))):
+        positions = None if cu_seqlens_q is None else _token_positions(cu_seqlens_q, q_up.shape[:-2].numel(), cp_rank, cp_size)
+        query = ops.absorbed_query(q_up, w_uk_t, cos, sin, positions, ops.ROPE_ADJACENT if rotary_interleaved else ops.ROPE_SPLIT)
+        if query is not None:
+            return query
     return FusedAbsorbRopeQuery.apply(q_up, w_uk_t, cos, sin, cu_seqlens_q, cp_rank, cp_size, rotary_interleaved)
 
 
@@ -625,6 +624,10 @@ def absorb_attention_output(core_attn_out, w_uv):
     """``[.., h, 512]`` attention output -> ``[.., h * 128]``: the value up-projection applied per head
     (multi_latent_attention.py:955-975 of the reference: einsum("...hk,hdk->...hd") then flatten), read from
     the attention kernel's own layout and written in the layout the output projection reads."""
+    if not torch.compiler.is_compiling():
+        out = ops.absorb_flat(core_attn_out, w_uv)
+        if out is not None:
+            return out
     lead, nheads = core_attn_out.shape[:-2], core_attn_out.shape[-2]
     o3 = core_attn_out.reshape(-1, nheads, core_attn_out.shape[-1])
     return ops.mla_absorb(o3, w_uv).reshape(*lead, nheads * w_uv.shape[1])

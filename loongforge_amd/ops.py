@@ -1,7 +1,8 @@
 """Tensor-level entry points of the gfx950 DSA kernels.
 
 Every function here checks its arguments, allocates outputs and workspaces with torch (the C
-library allocates nothing), and calls libdsa_hip.so through ctypes on the current HIP stream.
+library allocates nothing), and calls libdsa_hip.so on the current HIP stream; the hot ones do all of that
+in C++ (csrc/host/host.cpp), the others here through ctypes.
 The raw kernels are also registered as torch custom ops in the ``dsa::`` namespace so that they
 can be used from compiled graphs and carry fake-tensor shape functions.
 
@@ -15,6 +16,27 @@ import torch
 from . import _lib
 
 _FP8 = torch.float8_e4m3fn
+
+
+_host = None
+
+
+def _native():
+    """The C++ host layer: checks, allocations and kernel calls (csrc/host/host.cpp)."""
+    global _host
+    if _host is None:
+        _host = _lib.load_host()
+    return _host
+
+
+def _direct(name: str, op, *args):
+    """``op(*args)``, called in C++ without the custom-op dispatcher when this is an ordinary eager call on ordinary
+    tensors (the native function returns None otherwise: fake or traced tensors, dispatch modes, recorded gradients)."""
+    if not torch.compiler.is_compiling():
+        res = getattr(_native(), name)(*args, False)
+        if res is not None:
+            return res
+    return op(*args)
 
 
 def _stream(t: torch.Tensor):
@@ -36,19 +58,7 @@ def _c(t: torch.Tensor) -> torch.Tensor:
 # --------------------------------------------------------------------------------------------
 @torch.library.custom_op("dsa::quant_rowwise_e4m3", mutates_args=())
 def _quant_op(x: torch.Tensor, eps: float, pow2: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    _need_gpu(x)
-    if x.dtype != torch.bfloat16:
-        raise ValueError("quant_rowwise_e4m3 expects bf16 input, got %s" % x.dtype)
-    x = _c(x)
-    cols = x.shape[-1]
-    rows = x.numel() // max(cols, 1)
-    x8 = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    scale_inv = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        _lib.check(lib.dsa_quant_rowwise_e4m3(x.data_ptr(), rows, cols, x8.data_ptr(), scale_inv.data_ptr(),
-                                              float(eps), int(pow2), _stream(x)), "dsa_quant_rowwise_e4m3")
-    return x8, scale_inv
+    return _native().quant_rowwise(x, eps, pow2, True)
 
 
 @_quant_op.register_fake
@@ -58,32 +68,14 @@ def _(x, eps, pow2):
 
 def quant_rowwise_e4m3(x: torch.Tensor, eps: float = 1e-12, pow2: bool = True):
     """bf16 ``[..., 128]`` -> (float8_e4m3fn payload, fp32 ``scale_inv`` per row)."""
-    x8, scale_inv = _quant_op(x, eps, pow2)
-    return x8.view(_FP8), scale_inv
+    x8, scale_inv = _direct("quant_rowwise", _quant_op, x, eps, pow2)
+    return _fp8(x8), scale_inv
 
 
 @torch.library.custom_op("dsa::rotate_quant_e4m3", mutates_args=())
 def _rotate_quant_op(x: torch.Tensor, eps: float, pow2: bool, want_payload: bool,
                      want_rotated: bool) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    _need_gpu(x)
-    if x.dtype != torch.bfloat16:
-        raise ValueError("rotate_quant_e4m3 expects bf16 input, got %s" % x.dtype)
-    if x.shape[-1] != 128:
-        raise ValueError("rotate_quant_e4m3 rotates rows of 128 elements, got %d" % x.shape[-1])
-    if not (want_payload or want_rotated):
-        raise ValueError("rotate_quant_e4m3: no output requested")
-    x = _c(x)
-    rows = x.numel() // 128
-    x8 = torch.empty(x.shape if want_payload else (0,), dtype=torch.uint8, device=x.device)
-    scale_inv = torch.empty(x.shape[:-1] if want_payload else (0,), dtype=torch.float32, device=x.device)
-    y = torch.empty(x.shape if want_rotated else (0,), dtype=torch.bfloat16, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        _lib.check(lib.dsa_rotate_quant_e4m3(x.data_ptr(), rows, 128, x8.data_ptr() if want_payload else None,
-                                             scale_inv.data_ptr() if want_payload else None,
-                                             y.data_ptr() if want_rotated else None, float(eps), int(pow2), _stream(x)),
-                   "dsa_rotate_quant_e4m3")
-    return x8, scale_inv, y
+    return _native().rotate_quant(x, eps, pow2, want_payload, want_rotated, True)
 
 
 @_rotate_quant_op.register_fake
@@ -96,8 +88,8 @@ def _(x, eps, pow2, want_payload, want_rotated):
 def rotate_quant_e4m3(x: torch.Tensor, eps: float = 1e-12, pow2: bool = True, return_rotated: bool = False):
     """Hadamard rotation (x 128^-0.5, rounded to bf16) fused with :func:`quant_rowwise_e4m3`:
     bf16 ``[..., 128]`` -> (fp8 payload, ``scale_inv``[, rotated bf16])."""
-    x8, scale_inv, y = _rotate_quant_op(x, eps, pow2, True, return_rotated)
-    return (x8.view(_FP8), scale_inv, y) if return_rotated else (x8.view(_FP8), scale_inv)
+    x8, scale_inv, y = _direct("rotate_quant", _rotate_quant_op, x, eps, pow2, True, return_rotated)
+    return (_fp8(x8), scale_inv, y) if return_rotated else (_fp8(x8), scale_inv)
 
 
 @torch.library.custom_op("dsa::indexer_front_e4m3", mutates_args=())
@@ -107,51 +99,8 @@ def _indexer_front_op(x: torch.Tensor, rows_per_token: int, ln_weight: Optional[
                       rotate: bool, weights: Optional[torch.Tensor], factor: float, want_payload: bool,
                       want_rows: bool, eps: float,
                       pow2: bool) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    _need_gpu(x)
-    if x.dtype != torch.bfloat16 or x.shape[-1] != 128:
-        raise ValueError("indexer_front_e4m3 expects bf16 rows of 128 elements")
-    x = _c(x)
-    rows = x.numel() // 128
-    if rows % rows_per_token:
-        raise ValueError("indexer_front_e4m3: %d rows are not a multiple of %d rows per token" % (rows, rows_per_token))
-    if (ln_weight is None) != (ln_bias is None):
-        raise ValueError("indexer_front_e4m3: LayerNorm needs weight and bias")
-    f32 = 0
-    if pairing >= 0:
-        if cos is None or sin is None or cos.dtype != sin.dtype or cos.dtype not in (torch.float32, torch.bfloat16):
-            raise ValueError("indexer_front_e4m3: cos / sin must both be fp32 or bf16 tables")
-        cos, sin = _c(cos.reshape(-1, cos.shape[-1])), _c(sin.reshape(-1, sin.shape[-1]))
-        if cos.shape[-1] != 64 or sin.shape != cos.shape:
-            raise ValueError("indexer_front_e4m3: cos / sin rows must have 64 entries")
-        f32 = int(cos.dtype == torch.float32)
-        if positions is not None:
-            positions = _c(positions.to(torch.int32))
-            if positions.numel() != rows // rows_per_token:
-                raise ValueError("indexer_front_e4m3: one position per token expected")
-        elif (rows // rows_per_token + batch - 1) // batch > cos.shape[0]:
-            raise ValueError("indexer_front_e4m3: cos / sin tables are shorter than the sequence")
-    if ln_weight is not None:
-        ln_weight, ln_bias = _c(ln_weight.float()), _c(ln_bias.float())
-        if ln_weight.numel() != 128 or ln_bias.numel() != 128:
-            raise ValueError("indexer_front_e4m3: LayerNorm weight and bias must have 128 entries")
-    if weights is not None:
-        if not want_payload or weights.numel() != rows:
-            raise ValueError("indexer_front_e4m3: one weight per row expected, together with the payload")
-        weights = _c(weights.float())
-    dev = x.device
-    x8 = torch.empty(x.shape if want_payload else (0,), dtype=torch.uint8, device=dev)
-    scale_inv = torch.empty(x.shape[:-1] if want_payload else (0,), dtype=torch.float32, device=dev)
-    y = torch.empty(x.shape if want_rows else (0,), dtype=torch.bfloat16, device=dev)
-    w_scaled = torch.empty(x.shape[:-1] if weights is not None else (0,), dtype=torch.float32, device=dev)
-    ptr = lambda t: t.data_ptr() if t is not None and t.numel() else None   # noqa: E731
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        _lib.check(lib.dsa_indexer_front_e4m3(
-            x.data_ptr(), rows, 128, int(rows_per_token), ptr(ln_weight), ptr(ln_bias), float(ln_eps),
-            ptr(cos) if pairing >= 0 else None, ptr(sin) if pairing >= 0 else None, f32, int(pairing), ptr(positions),
-            int(batch), int(rotate), ptr(x8), ptr(scale_inv), ptr(y), float(eps), int(pow2), ptr(weights), float(factor),
-            ptr(w_scaled), _stream(x)), "dsa_indexer_front_e4m3")
-    return x8, scale_inv, y, w_scaled
+    return _native().indexer_front(x, rows_per_token, ln_weight, ln_bias, ln_eps, cos, sin, pairing, positions, batch, rotate,
+                                   weights, factor, want_payload, want_rows, eps, pow2, True)
 
 
 @_indexer_front_op.register_fake
@@ -172,33 +121,16 @@ def indexer_front_e4m3(x: torch.Tensor, rows_per_token: int = 1, ln_weight=None,
     [Hadamard rotation] -> quantiser.  Returns ``(x8, scale_inv, rows, weight_scaled)``; ``rows`` (the bf16
     values that were quantised) and ``weight_scaled`` (``weights * scale_inv * factor``) are ``None`` unless
     asked for."""
-    x8, scale_inv, y, ws = _indexer_front_op(x, rows_per_token, ln_weight, ln_bias, ln_eps, cos, sin, pairing, positions,
-                                             batch, rotate, weights, float(factor), return_payload, return_rows, eps, pow2)
-    return (x8.view(_FP8) if return_payload else None, scale_inv if return_payload else None,
+    x8, scale_inv, y, ws = _direct("indexer_front", _indexer_front_op, x, rows_per_token, ln_weight, ln_bias, ln_eps, cos, sin, pairing,
+                                   positions, batch, rotate, weights, float(factor), return_payload, return_rows, eps, pow2)
+    return (_fp8(x8) if return_payload else None, scale_inv if return_payload else None,
             y if return_rows else None, ws if weights is not None else None)
 
 
 @torch.library.custom_op("dsa::quant_rowwise_e4m3_weights", mutates_args=())
 def _quant_weights_op(x: torch.Tensor, weights: torch.Tensor, factor: float, rotate: bool, eps: float,
                       pow2: bool) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    _need_gpu(x, weights)
-    if x.dtype != torch.bfloat16 or x.shape[-1] != 128:
-        raise ValueError("quant_rowwise_e4m3_weights expects bf16 rows of 128 elements")
-    if weights.shape != x.shape[:-1]:
-        raise ValueError("quant_rowwise_e4m3_weights: one weight per row expected, got %s for rows %s"
-                         % (tuple(weights.shape), tuple(x.shape[:-1])))
-    x, weights = _c(x), _c(weights.float())
-    rows = x.numel() // 128
-    x8 = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    scale_inv = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    w_scaled = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        _lib.check(lib.dsa_quant_rowwise_e4m3_weights(x.data_ptr(), rows, 128, x8.data_ptr(), scale_inv.data_ptr(),
-                                                      float(eps), int(pow2), int(rotate), weights.data_ptr(),
-                                                      float(factor), w_scaled.data_ptr(), _stream(x)),
-                   "dsa_quant_rowwise_e4m3_weights")
-    return x8, scale_inv, w_scaled
+    return _native().quant_weights(x, weights, factor, rotate, eps, pow2, True)
 
 
 @_quant_weights_op.register_fake
@@ -211,13 +143,17 @@ def quant_rowwise_e4m3_weights(x: torch.Tensor, weights: torch.Tensor, factor: f
                                eps: float = 1e-12, pow2: bool = True):
     """:func:`quant_rowwise_e4m3` (after the Hadamard rotation when ``rotate``) that also returns
     ``(weights * scale_inv) * factor`` per row: (fp8 payload, ``scale_inv``, scaled weights fp32)."""
-    x8, scale_inv, w_scaled = _quant_weights_op(x, weights, float(factor), bool(rotate), eps, pow2)
-    return x8.view(_FP8), scale_inv, w_scaled
+    x8, scale_inv, w_scaled = _direct("quant_weights", _quant_weights_op, x, weights, float(factor), bool(rotate), eps, pow2)
+    return _fp8(x8), scale_inv, w_scaled
 
 
 def rotate_bf16(x: torch.Tensor):
     """Hadamard rotation of bf16 rows of 128 (x 128^-0.5), the kernel form of ``rotate_activation``."""
-    return _rotate_quant_op(x, 1e-12, True, False, True)[2]
+    return _direct("rotate_quant", _rotate_quant_op, x, 1e-12, True, False, True)[2]
+
+
+def _fp8(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype == _FP8 else t.view(_FP8)
 
 
 def _as_u8(t: torch.Tensor) -> torch.Tensor:
@@ -273,24 +209,7 @@ def indexer_logits(q8, q_w, k8, k_scale, ks, ke, width: Optional[int] = None, re
 @torch.library.custom_op("dsa::topk", mutates_args=())
 def _topk_op(logits: torch.Tensor, K: int, row_begin: Optional[torch.Tensor], row_end: Optional[torch.Tensor],
              id_base: Optional[torch.Tensor], sort: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    _need_gpu(logits, row_begin, row_end, id_base)
-    if logits.ndim != 2 or logits.dtype != torch.float32:
-        raise ValueError("topk expects a 2-D fp32 tensor")
-    if logits.stride(1) != 1:
-        logits = logits.contiguous()
-    S, width = logits.shape
-    rb = _c(row_begin.int()) if row_begin is not None else None
-    re = _c(row_end.int()) if row_end is not None else None
-    ib = _c(id_base.int()) if id_base is not None else None
-    scores = torch.empty(S, K, dtype=torch.float32, device=logits.device)
-    ids = torch.empty(S, K, dtype=torch.int32, device=logits.device)
-    lib = _lib.load()
-    with torch.cuda.device(logits.device):
-        _lib.check(lib.dsa_topk(logits.data_ptr(), S, logits.stride(0) if S > 0 else width,
-                                rb.data_ptr() if rb is not None else None, re.data_ptr() if re is not None else None,
-                                width, ib.data_ptr() if ib is not None else None, K, int(sort), scores.data_ptr(),
-                                ids.data_ptr(), _stream(logits)), "dsa_topk")
-    return scores, ids
+    return _native().topk(logits, K, row_begin, row_end, id_base, sort, True)
 
 
 @_topk_op.register_fake
@@ -300,27 +219,13 @@ def _(logits, K, row_begin, row_end, id_base, sort):
 
 def topk(logits, K: int, row_begin=None, row_end=None, id_base=None, sorted: bool = True):
     """Per-row top-K (scores, int32 ids); unused slots are (-inf, -1)."""
-    return _topk_op(logits, int(K), row_begin, row_end, id_base, bool(sorted))
+    return _direct("topk", _topk_op, logits, int(K), row_begin, row_end, id_base, bool(sorted))
 
 
 @torch.library.custom_op("dsa::indexer_topk", mutates_args=())
 def _indexer_topk_op(q8: torch.Tensor, q_w: torch.Tensor, k8: torch.Tensor, k_scale: torch.Tensor, ks: torch.Tensor,
                      ke: torch.Tensor, K: int, sort: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    S, Hi, Sk = _check_indexer(q8, q_w, k8, k_scale, ks, ke)
-    q8, k8 = _c(_as_u8(q8)), _c(_as_u8(k8))
-    q_w, k_scale = _c(q_w.float()), _c(k_scale.float())
-    ks, ke = _c(ks.int()), _c(ke.int())
-    scores = torch.empty(S, K, dtype=torch.float32, device=q8.device)
-    ids = torch.empty(S, K, dtype=torch.int32, device=q8.device)
-    lib = _lib.load()
-    nbytes = lib.dsa_indexer_topk_workspace_bytes(S, Sk, K)
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=q8.device)
-    with torch.cuda.device(q8.device):
-        _lib.check(lib.dsa_indexer_topk_fwd(q8.data_ptr(), q_w.data_ptr(), k8.data_ptr(), k_scale.data_ptr(),
-                                            ks.data_ptr(), ke.data_ptr(), S, Hi, Sk, K, int(sort), scores.data_ptr(),
-                                            ids.data_ptr(), ws.data_ptr(), nbytes, _stream(q8)),
-                   "dsa_indexer_topk_fwd")
-    return scores, ids
+    return _native().indexer_topk(q8, q_w, k8, k_scale, ks, ke, K, sort, True)
 
 
 @_indexer_topk_op.register_fake
@@ -330,7 +235,7 @@ def _(q8, q_w, k8, k_scale, ks, ke, K, sort):
 
 def indexer_topk(q8, q_w, k8, k_scale, ks, ke, K: int, sorted: bool = True):
     """Fused logits + top-K: (scores [S,K] fp32, global key ids [S,K] int32, -1 padded)."""
-    return _indexer_topk_op(q8, q_w, k8, k_scale, ks, ke, int(K), bool(sorted))
+    return _direct("indexer_topk", _indexer_topk_op, q8, q_w, k8, k_scale, ks, ke, int(K), bool(sorted))
 
 
 @torch.library.custom_op("dsa::indexer_bwd", mutates_args=())
@@ -375,6 +280,13 @@ def indexer_bwd(g, q8, k8, k_scale, q_w, ids):
     return _indexer_bwd_op(g, q8, k8, k_scale, q_w, ids)
 
 
+def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offset: int, like: torch.Tensor):
+    """``(ks, ke, check)``: the key window of every causal query ``chunk_offset + i`` (int32, on ``like``'s device) over
+    the packed sequences of ``cu_seqlens`` (None: one sequence).  ``check.wait()`` raises ValueError if the sequences
+    end before the queries do; call it behind the launches that use the window."""
+    return _native().indexer_window(cu_seqlens, int(queries), int(chunk_offset), like)
+
+
 # --------------------------------------------------------------------------------------------
 # sparse MLA
 # --------------------------------------------------------------------------------------------
@@ -396,35 +308,7 @@ def _check_mla(q, kv, ids):
 def _mla_fwd_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, q_start: int, sm_scale: float, d_v: int,
                 p_out_mode: int, attn_sink: Optional[torch.Tensor] = None,
                 p_out_skip: int = 0) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    _check_mla(q, kv, ids)
-    q, kv, ids = _c(q), _c(kv), _c(ids.int())
-    S, H, _ = q.shape
-    if attn_sink is not None:
-        _need_gpu(attn_sink)
-        if attn_sink.numel() != H:
-            raise ValueError("attn_sink must hold one logit per head (%d), got %d" % (H, attn_sink.numel()))
-        attn_sink = _c(attn_sink.float().reshape(H))
-    K = ids.shape[1]
-    out = torch.empty(S, H, d_v, dtype=torch.bfloat16, device=q.device)
-    lse = torch.empty(S, H, dtype=torch.float32, device=q.device)
-    if p_out_mode == 0:
-        p_out = torch.empty(0, dtype=torch.bfloat16, device=q.device)
-    else:
-        if p_out_skip < 0 or p_out_skip >= K or p_out_skip % 32:
-            raise ValueError("p_out_skip must be a multiple of 32 in [0, top-k), got %d" % p_out_skip)
-        p_out = torch.empty(S, H, K - p_out_skip, dtype=torch.float32 if p_out_mode == 2 else torch.bfloat16,
-                            device=q.device)
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        nbytes = lib.dsa_sparse_mla_fwd_workspace_bytes(S, H, kv.shape[0], K)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
-        _lib.check(lib.dsa_sparse_mla_fwd_ws(q.data_ptr(), kv.data_ptr(), ids.data_ptr(), S, H, kv.shape[0], K,
-                                             int(q_start), float(sm_scale), int(d_v), out.data_ptr(), lse.data_ptr(),
-                                             p_out.data_ptr() if p_out_mode else None, int(p_out_mode == 2),
-                                             attn_sink.data_ptr() if attn_sink is not None else None,
-                                             int(p_out_skip), ws.data_ptr() if nbytes else None, nbytes, _stream(q)),
-                   "dsa_sparse_mla_fwd")
-    return out, lse, p_out
+    return _native().mla_fwd(q, kv, ids, q_start, sm_scale, d_v, p_out_mode, attn_sink, p_out_skip, True)
 
 
 @_mla_fwd_op.register_fake
@@ -443,8 +327,8 @@ def sparse_mla_fwd(q, kv, ids, q_start: int = 0, sm_scale: Optional[float] = Non
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
     mode = 0 if not return_p_out else (2 if p_out_dtype == torch.float32 else 1)
-    out, lse, p_out = _mla_fwd_op(q, kv, ids, int(q_start), float(sm_scale), int(d_v), mode, attn_sink,
-                                   int(p_out_skip) if return_p_out else 0)
+    out, lse, p_out = _direct("mla_fwd", _mla_fwd_op, q, kv, ids, int(q_start), float(sm_scale), int(d_v), mode, attn_sink,
+                              int(p_out_skip) if return_p_out else 0)
     return out, lse, (p_out if return_p_out else None)
 
 
@@ -537,29 +421,20 @@ def release_bwd_workspace(device=None):
 @torch.library.custom_op("dsa::sparse_mla_bwd", mutates_args=())
 def _mla_bwd_op(q: torch.Tensor, kv: torch.Tensor, out: torch.Tensor, dout: torch.Tensor, ids: torch.Tensor,
                 lse: torch.Tensor, q_start: int, sm_scale: float, d_v: int) -> Tuple[torch.Tensor, torch.Tensor]:
-    _check_mla(q, kv, ids)
-    _need_gpu(out, dout, lse)
-    q, kv, ids = _c(q), _c(kv), _c(ids.int())
-    out, dout, lse = _c(out), _c(dout.to(torch.bfloat16)), _c(lse.float())
-    S, H, _ = q.shape
-    K = ids.shape[1]
-    if out.shape != (S, H, d_v) or dout.shape != (S, H, d_v) or lse.shape != (S, H):
-        raise ValueError("sparse_mla_bwd: out/dout must be [S,H,d_v] and lse [S,H]")
-    dq = torch.empty_like(q)
-    dkv = torch.empty_like(kv)
-    lib = _lib.load()
-    ws, nbytes = _bwd_workspace(lib.dsa_sparse_mla_bwd_workspace_bytes(S, H, kv.shape[0], K), q.device)
-    with torch.cuda.device(q.device):
-        _lib.check(lib.dsa_sparse_mla_bwd(q.data_ptr(), kv.data_ptr(), out.data_ptr(), dout.data_ptr(), ids.data_ptr(),
-                                          lse.data_ptr(), S, H, kv.shape[0], K, int(q_start), float(sm_scale),
-                                          int(d_v), dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), nbytes, _stream(q)),
-                   "dsa_sparse_mla_bwd")
-    return dq, dkv
+    return _native().mla_bwd(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v, _bwd_workspace, True)
 
 
 @_mla_bwd_op.register_fake
 def _(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v):
     return torch.empty_like(q), torch.empty_like(kv)
+
+
+def _mla_bwd(*args):
+    if not torch.compiler.is_compiling():
+        res = _native().mla_bwd(*args, _bwd_workspace, False)
+        if res is not None:
+            return res
+    return _mla_bwd_op(*args)
 
 
 def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optional[float] = None, d_v: int = 512):
@@ -572,13 +447,13 @@ def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optio
         sm_scale = q.shape[-1] ** -0.5
     K = ids.shape[1]
     if K <= BWD_MAX_SLOTS:
-        return _mla_bwd_op(q, kv, out, dout, ids, lse, int(q_start), float(sm_scale), int(d_v))
+        return _mla_bwd(q, kv, out, dout, ids, lse, int(q_start), float(sm_scale), int(d_v))
     dq32 = dkv32 = None
     for k0 in range(0, K, BWD_MAX_SLOTS):
         part = ids[:, k0:k0 + BWD_MAX_SLOTS]
         if part.shape[1] % 64:
             part = torch.nn.functional.pad(part, (0, 64 - part.shape[1] % 64), value=-1)
-        dq, dkv = _mla_bwd_op(q, kv, out, dout, part.contiguous(), lse, int(q_start), float(sm_scale), int(d_v))
+        dq, dkv = _mla_bwd(q, kv, out, dout, part.contiguous(), lse, int(q_start), float(sm_scale), int(d_v))
         dq32 = dq.float() if dq32 is None else dq32.add_(dq)
         dkv32 = dkv.float() if dkv32 is None else dkv32.add_(dkv)
     return dq32.to(torch.bfloat16), dkv32.to(torch.bfloat16)
@@ -586,19 +461,7 @@ def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optio
 
 @torch.library.custom_op("dsa::attn_dist", mutates_args=())
 def _attn_dist_op(p_out: torch.Tensor, sm_scale: float) -> torch.Tensor:
-    _need_gpu(p_out)
-    if p_out.ndim != 3 or p_out.dtype not in (torch.bfloat16, torch.float32):
-        raise ValueError("attn_dist expects p_out [S,H,K] in bf16 or fp32")
-    if p_out.stride(2) != 1:
-        p_out = p_out.contiguous()
-    S, H, K = p_out.shape
-    target = torch.empty(S, K, dtype=torch.float32, device=p_out.device)
-    lib = _lib.load()
-    with torch.cuda.device(p_out.device):
-        _lib.check(lib.dsa_attn_dist(p_out.data_ptr(), int(p_out.dtype == torch.float32), S, H, K,
-                                     p_out.stride(0) if S > 0 else H * K, p_out.stride(1), float(sm_scale),
-                                     target.data_ptr(), _stream(p_out)), "dsa_attn_dist")
-    return target
+    return _native().attn_dist(p_out, sm_scale, True)
 
 
 @_attn_dist_op.register_fake
@@ -608,7 +471,7 @@ def _(p_out, sm_scale):
 
 def attn_dist(p_out, sm_scale: float):
     """fp32 ``[S,K]``: mean over heads of softmax over slots of ``p_out * sm_scale``."""
-    return _attn_dist_op(p_out, float(sm_scale))
+    return _direct("attn_dist", _attn_dist_op, p_out, float(sm_scale))
 
 
 @torch.library.custom_op("dsa::attn_dist_qk", mutates_args=())
@@ -670,24 +533,7 @@ ROPE_ADJACENT, ROPE_SPLIT = 0, 1   # where pair i sits in a row: (2i, 2i+1) or (
 
 @torch.library.custom_op("dsa::indexer_kl_loss", mutates_args=())
 def _kl_loss_op(scores: torch.Tensor, target: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
-    _need_gpu(scores, target)
-    if scores.ndim != 2 or target.shape != scores.shape:
-        raise ValueError("indexer_kl_loss expects scores and target of one shape [S, K]")
-    S, K = scores.shape
-    scores = scores.float()
-    target = target.float()
-    if scores.stride(1) != 1:
-        scores = scores.contiguous()
-    if target.stride(1) != 1:
-        target = target.contiguous()
-    row_loss = torch.empty(S, dtype=torch.float32, device=scores.device)
-    grad = torch.empty(S, K, dtype=torch.float32, device=scores.device)
-    lib = _lib.load()
-    with torch.cuda.device(scores.device):
-        _lib.check(lib.dsa_indexer_kl_loss(scores.data_ptr(), scores.stride(0) if S > 1 else K, target.data_ptr(),
-                                           target.stride(0) if S > 1 else K, S, K, float(eps), row_loss.data_ptr(),
-                                           grad.data_ptr(), _stream(scores)), "dsa_indexer_kl_loss")
-    return row_loss, grad
+    return _native().kl_loss(scores, target, eps, True)
 
 
 @_kl_loss_op.register_fake
@@ -700,7 +546,7 @@ class _IndexerKLLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, scores, target, eps):
-        row_loss, grad = _kl_loss_op(scores.detach(), target.detach(), eps)
+        row_loss, grad = _direct("kl_loss", _kl_loss_op, scores.detach(), target.detach(), eps)
         ctx.save_for_backward(grad)
         ctx.in_dtype = scores.dtype
         return row_loss.sum()
@@ -736,6 +582,10 @@ def _cos_sin(cos: torch.Tensor, sin: torch.Tensor, emb_dim: int):
 def thd_positions(cu_seqlens: torch.Tensor, tokens: int, offset: int = 0) -> torch.Tensor:
     """Position of every packed token inside its own sequence (int32 [tokens]); token t of the call
     is global token t + offset.  Tokens past the last sequence get position 0."""
+    if cu_seqlens.is_cuda and not torch.compiler.is_compiling():
+        pos = _native().thd_positions(cu_seqlens, tokens, int(offset))
+        if pos is not None:
+            return pos
     cu = cu_seqlens.to(torch.int64)
     t = torch.arange(tokens, device=cu.device, dtype=torch.int64) + int(offset)
     seq = torch.searchsorted(cu[1:].contiguous(), t, right=True)
@@ -755,37 +605,8 @@ def rope_rows(pe_src: Optional[torch.Tensor], pe_dst: Optional[torch.Tensor], co
     in ``pe_src`` broadcasts one row.  cos / sin: [positions, emb_dim] fp32 or bf16.  Writes in place
     into ``pe_dst`` / ``main_dst``.
     """
-    ref = pe_dst if pe_dst is not None else main_dst
-    _need_gpu(pe_src, pe_dst, cos, sin, positions, main_src, main_dst)
-    tokens, heads = ref.shape[0], ref.shape[1]
-    emb = 0
-    ps = pd = (None, 0, 0)
-    cos2 = sin2 = None
-    if pe_dst is not None:
-        emb = pe_dst.shape[-1]
-        if pe_src.shape != pe_dst.shape:
-            raise ValueError("pe_src and pe_dst differ in shape: %s vs %s" % (tuple(pe_src.shape), tuple(pe_dst.shape)))
-        ps, pd = _rows_view(pe_src, "pe_src"), _rows_view(pe_dst, "pe_dst")
-        cos2, sin2 = _cos_sin(cos, sin, emb)
-        if positions is not None:
-            positions = _c(positions.int())
-            if positions.numel() != tokens:
-                raise ValueError("positions must hold one entry per token")
-    ms = md = (None, 0, 0)
-    d_main = 0
-    if main_dst is not None:
-        if main_src.shape != main_dst.shape or main_dst.shape[:2] != ref.shape[:2]:
-            raise ValueError("main_src / main_dst shapes do not match the pe rows")
-        d_main = main_dst.shape[-1]
-        ms, md = _rows_view(main_src, "main_src"), _rows_view(main_dst, "main_dst")
-    lib = _lib.load()
-    with torch.cuda.device(ref.device):
-        _lib.check(lib.dsa_rope_rows(ms[0], ms[1], ms[2], md[0], md[1], md[2], d_main, ps[0], ps[1], ps[2], pd[0], pd[1], pd[2],
-                                     emb, cos2.data_ptr() if emb else None, sin2.data_ptr() if emb else None,
-                                     int(emb and cos2.dtype == torch.float32),
-                                     positions.data_ptr() if (emb and positions is not None) else None, int(batch),
-                                     tokens, heads, int(in_pairing), int(out_pairing), int(bool(inverse)), _stream(ref)),
-                   "dsa_rope_rows")
+    _native().rope_rows(pe_src, pe_dst, cos, sin, int(in_pairing), int(out_pairing), bool(inverse), positions, int(batch),
+                        main_src, main_dst)
 
 
 def rope_headsum_inverse(grad_pe: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, in_pairing: int,
@@ -815,20 +636,7 @@ def mla_absorb_into(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor) -> None:
     """``c[s, h, :] = a[s, h, :] @ w[h].T`` for bf16 views ``a [S, H, k]``, ``c [S, H, n]`` (any token / head
     strides that are multiples of 8 elements, unit stride inside a row) and contiguous ``w [H, n, k]`` with
     ``(k, n)`` = (128, 512) or (512, 128).  Writes into ``c``; no autograd (see :class:`MlaAbsorb`)."""
-    _need_gpu(a, w, c)
-    if a.dtype != torch.bfloat16 or c.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
-        raise ValueError("mla_absorb expects bf16 tensors")
-    if a.ndim != 3 or c.ndim != 3 or w.ndim != 3 or a.shape[:2] != c.shape[:2] or w.shape != (a.shape[1], c.shape[2], a.shape[2]):
-        raise ValueError("mla_absorb: shapes a %s, w %s, c %s do not fit c[s,h,:] = a[s,h,:] @ w[h].T"
-                         % (tuple(a.shape), tuple(w.shape), tuple(c.shape)))
-    if a.stride(2) != 1 or c.stride(2) != 1:
-        raise ValueError("mla_absorb: rows must be contiguous")
-    w = _c(w)
-    S, H, k = a.shape
-    lib = _lib.load()
-    with torch.cuda.device(a.device):
-        _lib.check(lib.dsa_mla_absorb(a.data_ptr(), a.stride(0), a.stride(1), w.data_ptr(), c.data_ptr(), c.stride(0),
-                                      c.stride(1), S, H, k, c.shape[2], _stream(a)), "dsa_mla_absorb")
+    _native().absorb_into(a, w, c)
 
 
 def absorb_rope_query_into(q_up: torch.Tensor, w: torch.Tensor, query: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -836,26 +644,17 @@ def absorb_rope_query_into(q_up: torch.Tensor, w: torch.Tensor, query: torch.Ten
     """``query[s, h, :512] = q_up[s, h, :128] @ w[h].T`` and ``query[s, h, 512:] = rope(q_up[s, h, 128:])`` (pairs adjacent
     in ``q_up``), one kernel: :func:`mla_absorb_into` and :func:`rope_rows` over the rows of ``q_up [S, H, 192]`` and
     ``query [S, H, 576]``.  No autograd."""
-    _need_gpu(q_up, w, query, cos, sin, positions)
-    if q_up.dtype != torch.bfloat16 or query.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
-        raise ValueError("mla_absorb expects bf16 tensors")
-    S, H = q_up.shape[:2]
-    if q_up.ndim != 3 or q_up.shape[2] != 192 or query.shape != (S, H, 576) or w.shape != (H, 512, 128):
-        raise ValueError("absorb_rope_query: shapes q_up %s, w %s, query %s do not fit" % (tuple(q_up.shape), tuple(w.shape), tuple(query.shape)))
-    if q_up.stride(2) != 1 or query.stride(2) != 1:
-        raise ValueError("mla_absorb: rows must be contiguous")
-    w = _c(w)
-    cos2, sin2 = _cos_sin(cos, sin, 64)
-    if positions is not None:
-        positions = _c(positions.int())
-        if positions.numel() != S:
-            raise ValueError("positions must hold one entry per token")
-    lib = _lib.load()
-    with torch.cuda.device(q_up.device):
-        _lib.check(lib.dsa_absorb_rope_query(q_up.data_ptr(), q_up.stride(0), q_up.stride(1), w.data_ptr(), query.data_ptr(),
-                                             query.stride(0), query.stride(1), cos2.data_ptr(), sin2.data_ptr(),
-                                             int(cos2.dtype == torch.float32), positions.data_ptr() if positions is not None else None,
-                                             int(batch), S, H, int(out_pairing), _stream(q_up)), "dsa_absorb_rope_query")
+    _native().absorb_rope_query_into(q_up, w, query, cos, sin, int(out_pairing), positions, int(batch))
+
+
+def absorbed_query(q_up, w, cos, sin, positions, out_pairing: int):
+    """:func:`absorb_rope_query_into` over ``q_up [.., H, 192]`` into a new ``[.., H, 576]``; None if that needs autograd."""
+    return _native().absorbed_query(q_up, w, cos, sin, positions, int(out_pairing))
+
+
+def absorb_flat(a, w):
+    """:func:`mla_absorb` with heads and width flattened, ``[.., H * n]``; None if that needs autograd."""
+    return _native().absorb(a, w, True)
 
 
 class MlaAbsorb(torch.autograd.Function):
@@ -882,5 +681,9 @@ def mla_absorb(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = N
     """Differentiable per-head projection ``a [S, H, k] , w [H, n, k] -> [S, H, n]``; ``out`` may be a view into
     a larger tensor (for instance the latent columns of the attention query)."""
     if out is None:
+        if not torch.compiler.is_compiling():
+            res = _native().absorb(a, w, False)
+            if res is not None:
+                return res
         out = a.new_empty(a.shape[0], a.shape[1], w.shape[1])
     return MlaAbsorb.apply(a, w, out)

@@ -327,3 +327,54 @@ def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
                 want = ref[i, ks[i]: ks[i] + n]
                 assert (row - want).abs().max().item() <= 1e-4 * max(want.abs().max().item(), 1.0) if n else True
                 assert int(torch.isfinite(got[i]).sum()) == n
+
+
+@pytest.mark.parametrize("cu,S,offset", [(None, 5, 3), ([0, 7], 7, 0), ([0, 3, 3, 300, 513], 256, 257), ([0, 1, 2, 700], 700, 0)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_windows_and_positions_of_packed_sequences(gpu, cu, S, offset, dtype):
+    from loongforge_amd import ops
+
+    like = torch.zeros(1, device=gpu)
+    t = torch.arange(offset, offset + S)
+    start = torch.zeros(S, dtype=torch.int64)
+    if cu is not None:
+        bounds = torch.tensor(cu)
+        start = bounds[torch.searchsorted(bounds[1:].contiguous(), t, right=True)]
+        pos = ops.thd_positions(bounds.to(gpu, dtype), S + 4, offset)
+        inside = min(S + 4, cu[-1] - offset)
+        assert torch.equal(pos[:S].cpu().long(), t - start) and not pos[inside:].any()
+    ks, ke, covered = ops.indexer_window(None if cu is None else torch.tensor(cu, dtype=dtype, device=gpu), S, offset, like)
+    covered.wait()
+    assert torch.equal(ks.cpu().long(), start) and torch.equal(ke.cpu().long(), t + 1)
+    if cu is not None:
+        _, _, short = ops.indexer_window(torch.tensor(cu[:-1] + [offset + S - 1], dtype=dtype, device=gpu), S, offset, like)
+        with pytest.raises(ValueError, match="inconsistent shapes"):
+            short.wait()
+
+
+def test_native_host_layer_equals_the_registered_ops(gpu):
+    """Ordinary calls go through the C++ layer, traced ones and those under a dispatch mode through the custom op."""
+    from loongforge_amd import ops
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    logits = torch.randn(3, 500, device=gpu)
+    direct = ops.topk(logits, 40)
+    with Seen():
+        seen = ops.topk(logits, 40)
+    assert any("dsa.topk" in n for n in Seen.names) and all(torch.equal(a, b) for a, b in zip(direct, seen))
+    x = torch.randn(4, 128, device=gpu).to(torch.bfloat16)
+    with FakeTensorMode() as mode:
+        x8, scale = ops.quant_rowwise_e4m3(mode.from_tensor(x))
+    assert x8.dtype == torch.float8_e4m3fn and scale.shape == (4,)
+    with pytest.raises(ValueError, match="2-D fp32"):
+        ops.topk(logits.double(), 4)
+    with pytest.raises(ValueError, match="dsa_topk"):
+        ops.topk(logits, 0)
