@@ -160,6 +160,23 @@ int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, const float*
                     void* stream);
 
 /*
+ * The same together with the way from the payload gradients back to the outputs of the projections: per row / scale
+ * (rows on the quantiser's epsilon floor get 0), [Hadamard rotation], [bf16, transposed rotary embedding of the first 64
+ * channels: cos / sin [positions, 64], `pairing` as dsa_rope_rows or -1; the position of a query / key row is positions_q /
+ * positions_k[row], or row / batch where that is NULL], for keys [LayerNorm backward with input k_in [Sk,128] bf16, weight
+ * ln_w, into d_ln_w, d_ln_b [128]]; d_w = d_qw * q_scale * w_scale.  q8, q_w are padded to Hi heads and 128 channels:
+ * d_q [S,heads,dim], d_k [Sk,dim], d_w [S,heads] hold the real ones (f32 where *_f32, else bf16).
+ * Workspace: dsa_indexer_grads_workspace_bytes (256-byte aligned); less, down to the extra of 64 queries, means chunks.
+ */
+size_t dsa_indexer_grads_workspace_bytes(int S, int Hi, int Sk, int K);
+int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
+                      const int32_t* ids, int S, int Hi, int Sk, int K, const float* q_scale, float w_scale, int rotate,
+                      const void* cos, const void* sin, int tables_f32, int pairing, const int32_t* positions_q,
+                      const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps, int heads,
+                      int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32, float* d_ln_w,
+                      float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Windows of the causal queries [chunk_offset, chunk_offset + S) over packed sequences, cu[ncu] (i32, or i64 if cu_i64)
  * their cumulative lengths (NULL: one sequence): ks[i] = start of the query's sequence, ke[i] = chunk_offset + i + 1;
  * queries past the last sequence get ks = 0.  total (may be NULL; host-visible): the summed length of the sequences.

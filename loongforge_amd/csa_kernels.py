@@ -15,7 +15,7 @@ import torch
 from torch import Tensor
 
 from . import ops
-from .dsa_fused_kernels import _pad_to, _unscale_indexer_grad
+from .dsa_fused_kernels import _pad_to
 from .megatron_compat import PackedSeqParams
 
 
@@ -169,15 +169,10 @@ class CSAIndexerKernelFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_score, grad_topk):
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, global_ids = ctx.saved_tensors
-        # padding slots are constants of the forward: their upstream gradient (often NaN) is dropped
-        grad_score = torch.where(global_ids >= 0, grad_score.float(), torch.zeros_like(grad_score, dtype=torch.float32))
-        d_q, d_k, d_weights = ops.indexer_bwd(grad_score.contiguous(), q_fp8, k_fp8, k_scale, weight_scaled, global_ids)
-        d_weights = d_weights * q_scale * ctx.softmax_scale
-        d_q = _unscale_indexer_grad(d_q, q_scale)
-        d_k = _unscale_indexer_grad(d_k, k_scale)
-        dq_t, dk_t, dw_t = ctx.in_dtypes
-        return (d_q[:, :ctx.head].to(dq_t).unsqueeze(1), d_k.to(dk_t).unsqueeze(1),
-                d_weights[:, :ctx.head].to(dw_t).unsqueeze(1), None, None, None, None)
+        # padding slots (id -1) are constants of the forward: their upstream gradient (often NaN) is dropped by the kernel
+        d_q, d_k, d_weights, _, _ = ops.indexer_grads(grad_score, q_fp8, k_fp8, k_scale, weight_scaled, global_ids, q_scale,
+                                                      ctx.softmax_scale, ctx.head, 128, ctx.in_dtypes)
+        return d_q.unsqueeze(1), d_k.unsqueeze(1), d_weights.unsqueeze(1), None, None, None, None
 
 
 class CSAIndexerKernel(torch.nn.Module):

@@ -224,6 +224,72 @@ py::object topk(const Tensor& logits_, int64_t K, const OptTensor& row_begin, co
   return py::make_tuple(scores, ids);
 }
 
+// Slots are processed 128 at a time: gradients and ids padded with empty slots to a multiple of that.
+std::pair<Tensor, Tensor> padded_slots(const Tensor& g_, const Tensor& ids_) {
+  Tensor g = f32(g_), ids = i32(ids_);
+  const int64_t pad = (128 - ids.size(1) % 128) % 128;
+  if (pad) { g = at::constant_pad_nd(g, {0, pad}, 0.0); ids = at::constant_pad_nd(ids, {0, pad}, -1); }
+  return {g, ids};
+}
+
+py::object indexer_bwd(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, const Tensor& k_scale_, const Tensor& q_w_, const Tensor& ids_,
+                       bool force) {
+  PLAIN_OR_NONE(g_, q8_, k8_, k_scale_, q_w_, ids_);
+  need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_);
+  const int64_t S = q8_.size(0), Hi = q8_.size(1), Sk = k8_.size(0);
+  REQUIRE(ids_.dim() == 2 && g_.sizes() == ids_.sizes() && ids_.size(0) == S, "indexer_bwd: grad and ids must both be [S, K]");
+  const auto [g, ids] = padded_slots(g_, ids_);
+  const Tensor q8 = as_u8(q8_), k8 = as_u8(k8_), q_w = f32(q_w_), k_scale = f32(k_scale_);
+  Call call(q8);
+  Tensor d_q8 = make(q8.sizes(), at::kFloat, q8), d_k8 = make(k8.sizes(), at::kFloat, q8), d_qw = make({S, Hi}, at::kFloat, q8);
+  const size_t nbytes = dsa_indexer_bwd_workspace_bytes((int)S, (int)Hi, (int)Sk, (int)ids.size(1));
+  Tensor ws = make({(int64_t)std::max<size_t>(nbytes, 256)}, at::kByte, q8);
+  run("dsa_indexer_bwd", dsa_indexer_bwd, (const float*)g.const_data_ptr(), q8.const_data_ptr(), k8.const_data_ptr(),
+      (const float*)k_scale.const_data_ptr(), (const float*)q_w.const_data_ptr(), (const int32_t*)ids.const_data_ptr(), (int)S, (int)Hi, (int)Sk,
+      (int)ids.size(1), (float*)d_q8.data_ptr(), (float*)d_k8.data_ptr(), (float*)d_qw.data_ptr(), ws.data_ptr(), nbytes, call.stream);
+  return py::make_tuple(d_q8, d_k8, d_qw);
+}
+
+py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, const Tensor& k_scale_, const Tensor& q_w_, const Tensor& ids_,
+                        const Tensor& q_scale_, double w_scale, bool rotate, const OptTensor& cos_, const OptTensor& sin_, int64_t pairing,
+                        const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& k_in, const OptTensor& ln_w_,
+                        double ln_eps, int64_t heads, int64_t dim, at::ScalarType q_type, at::ScalarType k_type, at::ScalarType w_type) {
+  need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_, q_scale_);
+  const int64_t S = q8_.size(0), Hi = q8_.size(1), Sk = k8_.size(0);
+  REQUIRE(ids_.dim() == 2 && g_.sizes() == ids_.sizes() && ids_.size(0) == S && q_scale_.numel() == S * Hi,
+          "indexer_grads: grad and ids must both be [S, K], q_scale [S, H]");
+  const auto [g, ids] = padded_slots(g_, ids_);
+  const Tensor q8 = as_u8(q8_), k8 = as_u8(k8_), q_w = f32(q_w_), k_scale = f32(k_scale_), q_scale = f32(q_scale_);
+  OptTensor cos, sin, pos_q, pos_k, ln_w;
+  if (pairing >= 0) {
+    cos = cos_->contiguous();
+    sin = sin_->contiguous();
+    if (positions_q) pos_q = i32(*positions_q);
+    if (positions_k) pos_k = i32(*positions_k);
+  }
+  Tensor d_ln_w, d_ln_b;
+  if (k_in) {
+    REQUIRE(k_in->scalar_type() == at::kBFloat16 && k_in->is_contiguous() && k_in->numel() == Sk * 128 && ln_w_ && ln_w_->numel() == 128,
+            "indexer_grads: the LayerNorm's input must be bf16 [Sk, 128], its weight [128]");
+    ln_w = f32(*ln_w_);
+    d_ln_w = make({128}, at::kFloat, q8);
+    d_ln_b = make({128}, at::kFloat, q8);
+  }
+  Call call(q8);
+  auto out_type = [](at::ScalarType t) { return t == at::kBFloat16 ? t : at::kFloat; };
+  Tensor d_q = make({S, heads, dim}, out_type(q_type), q8), d_k = make({Sk, dim}, out_type(k_type), q8), d_w = make({S, heads}, out_type(w_type), q8);
+  const size_t nbytes = dsa_indexer_grads_workspace_bytes((int)S, (int)Hi, (int)Sk, (int)ids.size(1));
+  Tensor ws = make({(int64_t)std::max<size_t>(nbytes, 256)}, at::kByte, q8);
+  auto is_f32 = [](const Tensor& t) { return (int)(t.scalar_type() == at::kFloat); };
+  run("dsa_indexer_grads", dsa_indexer_grads, (const float*)g.const_data_ptr(), q8.const_data_ptr(), k8.const_data_ptr(),
+      (const float*)k_scale.const_data_ptr(), (const float*)q_w.const_data_ptr(), (const int32_t*)ids.const_data_ptr(), (int)S, (int)Hi, (int)Sk,
+      (int)ids.size(1), (const float*)q_scale.const_data_ptr(), (float)w_scale, (int)rotate, ptr(cos), ptr(sin), cos ? is_f32(*cos) : 0,
+      (int)pairing, (const int32_t*)ptr(pos_q), (const int32_t*)ptr(pos_k), (int)batch, ptr(k_in), (const float*)ptr(ln_w), (float)ln_eps,
+      (int)heads, (int)dim, d_q.data_ptr(), is_f32(d_q), d_k.data_ptr(), is_f32(d_k), d_w.data_ptr(), is_f32(d_w),
+      k_in ? (float*)d_ln_w.data_ptr() : nullptr, k_in ? (float*)d_ln_b.data_ptr() : nullptr, ws.data_ptr(), nbytes, call.stream);
+  return py::make_tuple(d_q.to(q_type), d_k.to(k_type), d_w.to(w_type), k_in ? py::cast(d_ln_w) : py::none(), k_in ? py::cast(d_ln_b) : py::none());
+}
+
 // ---- windows of packed sequences ------------------------------------------------------------------------
 // Whether the sequences cover the queries is only known on the device; the kernel leaves their length in pinned memory
 // and wait() looks at it, called after the kernels that use the window were launched: the device has work while the
@@ -490,6 +556,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(indexer_front);
   DEF(indexer_topk);
   DEF(topk);
+  DEF(indexer_bwd);
+  DEF(indexer_grads);
   DEF(mla_fwd);
   DEF(mla_bwd);
   DEF(attn_dist);

@@ -1,21 +1,27 @@
 // Sparse backward of the lightning-indexer logits for gfx950, deterministic.
 //
 // For every selected pair (query i, slot t, key j = ids[i,t]) with upstream gradient g[i,t]:
-//   r_h = q8[i,h,:] . k8[j,:]            a = g[i,t] * k_scale[j]          e_h = a * q_w[i,h] * [r_h > 0]
+//   r_h = q8[i,h,:] . k8[j,:]            a = g[i,t] * k_scale[j]          m_h = [r_h > 0]
 //   d_qw[i,h]   += a * relu(r_h)
-//   d_q8[i,h,:] += e_h * k8[j,:]
-//   d_k8[j,:]   += sum_h e_h * q8[i,h,:]
-// One 256-thread workgroup per query; the four waves each take 32 of the 128 slots of a tile.
-//   r        fp8 MFMA (exact products, as in the forward), one key per lane, heads down the registers
-//   d_k8 row bf16 MFMA  row^T[d, key] = Q^T[d, head] . E[head, key];  E = the r-accumulator layout,
-//            Q^T resident in accumulation registers; the row, rounded to bf16, goes to a pair buffer at
-//            the position of a key-sorted order and a second kernel sums every key's rows in fp32 in
-//            ascending query order
-//   d_q8     bf16 MFMA  dq^T[d, head] += K^T[d, key] . E^T[key, head], both operands by LDS transpose
-//            reads (the wave's key rows converted to bf16, and E written back to LDS)
-// For d_q8 E is carried as a bf16 pair (hi + lo), so the bf16 products lose nothing visible in fp32
-// (q8 and k8 are exact in bf16); the d_k8 rows use the hi part alone, as they are rounded to bf16
-// anyway.  No floating-point atomics: every sum has a fixed order.
+//   d_q8[i,h,:] += q_w[i,h] * (a m_h) * k8[j,:]
+//   d_k8[j,:]   += a * sum_h m_h * (q_w[i,h] q8[i,h,:])
+// The weight of a head and the factor of a pair stand outside the sums they do not depend on, so that what passes from
+// the first product to the other two is a mask.
+//
+// One workgroup of eight waves per query, 128 slots per tile; the waves 2p and 2p + 1 share 32 slots.
+//   r        fp8 MFMA, evaluated in both orientations (keys on the columns, then heads on the columns): the
+//            accumulator layout of each is the operand layout of one of the two following products, so nothing
+//            is transposed through LDS
+//   d_k8 row bf16 MFMA  row^T[d, key] = (q_w Q)^T[d, head] . m[head, key], half of d per wave, times a in fp32; the row,
+//            rounded to bf16, goes to a pair buffer at the position of a key-sorted order and a second kernel sums
+//            every key's rows in fp32 in ascending query order
+//   d_q8     bf16 MFMA  dq^T[d, head] += K^T[d, key] . (a m)[key, head]; K^T by transposing 8-bit LDS reads of the fp8 tile,
+//            converted in registers (exact); a as a bf16 pair (hi + lo), so the products lose nothing visible in fp32
+// No floating-point atomics: every sum has a fixed order.
+//
+// At 8192 queries x 2048 slots x 64 heads: 2.54 ms for the previous form (four waves of one SIMD each, E carried through
+// LDS as a bf16 pair: 48 transposing reads and 40 writes per wave and tile), of which the matrix work is 0.4 ms and
+// the pair rows (3.8 GB written) 0.75 ms.
 #include "dsa_common.h"
 #include "order.h"
 
@@ -24,182 +30,288 @@ namespace {
 constexpr int D = 128;
 constexpr int TK = 128;                 // slots per tile
 constexpr int TILE_BYTES = TK * D;      // fp8 key rows
-constexpr int RED_STRIDE = 132;         // floats per head row of the cross-wave reduction buffer
-constexpr int STRIP_STRIDE = 136;       // bytes per key row of the d_k transpose strip (two d-tiles of 64 bytes + bank spread)
+constexpr int STAGES = 4;               // tiles in the LDS ring
+constexpr int THREADS = 512;
+constexpr int RED_STRIDE = 132;         // floats per head row of the cross-wave reduction buffers
 
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-__device__ __forceinline__ int kb_swz(int key) { return ((key & 3) << 2) | ((key >> 2) & 3); }
-__device__ __forceinline__ int es_swz(int key) { return 2 * ((key >> 1) & 3) + ((key >> 3) & 1); }
 __device__ __forceinline__ void dma16(unsigned lds_base, unsigned goff, const void* gbase) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
 }
-__device__ __forceinline__ void mfma_a_vv(f32x16& acc, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void mfma_v_av_first(f32x16& acc, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc) : "a"(a), "v"(b));
-}
-__device__ __forceinline__ void mfma_v_av(f32x16& acc, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "a"(a), "v"(b));
-}
-__device__ __forceinline__ void mfma_done_v(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
-__device__ __forceinline__ void mfma_done_a(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc)); }
+// The 16-byte chunk c of a 128-byte row r sits in slot c ^ slot_xor(r): eight rows of one parity of any 16 consecutive ones
+// use eight different slots (row reads), and the eight rows of a transposing read four different pairs of slots per
+// parity: neither kind of read has a bank conflict.
+__device__ __forceinline__ int slot_xor(int r) { return ((r >> 2) & 1) | (r & 2) | ((r >> 1) & 4); }
 
-__device__ __forceinline__ bf16x8 tr_pair(const unsigned char* p0, const unsigned char* p1) {
-  i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p0));
-  i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p1));
-  return __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+// e4m3 bytes -> bf16 (exact)
+__device__ __forceinline__ bf16x8 fp8_to_bf16(const i32x2& w) {
+  bf16x8 o;
+#pragma unroll
+  for (int x = 0; x < 2; x++) {
+    const bf16x2 lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[x], 1.0f, false);
+    const bf16x2 hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[x], 1.0f, true);
+    o[4 * x] = lo[0]; o[4 * x + 1] = lo[1]; o[4 * x + 2] = hi[0]; o[4 * x + 3] = hi[1];
+  }
+  return o;
+}
+__device__ __forceinline__ i32x2 read_tr8(const unsigned char* p) { return __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(i32x2, p)); }
+
+// ---- what follows the sums: from payload gradients to gradients of the projections' outputs ------------------
+// 16 lanes per row, 8 consecutive elements per lane:  / scale (rows on the quantiser's epsilon floor: 0), Hadamard
+// rotation (its own transpose), bf16, transposed rotary embedding of the first 64 elements - the steps of the front
+// end backwards, rounding where the separate operations round.
+struct RowFinish {
+  int rotate;
+  const void* cos_t;
+  const void* sin_t;
+  int cs_f32, pairing, batch;            // pairing -1: no rotary part
+};
+
+__device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_inv, const RowFinish& f, const int* positions, int token) {
+  constexpr float FLOOR = 0x1.8p-48f;
+  const bool usable = scale_inv > FLOOR && scale_inv < INFINITY;
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = usable ? v[i] / scale_inv : 0.f;
+  if (f.rotate) {
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1)
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        if (!(i & m)) { const float a = v[i], b = v[i | m]; v[i] = a + b; v[i | m] = a - b; }
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float o = __shfl_xor(v[i], m, 64);
+        v[i] = (sub & m) ? o - v[i] : v[i] + o;
+      }
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] *= 0.08838834764831845f;
+  }
+  if (f.pairing >= 0) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
+    const long pos = positions ? positions[token] : token / f.batch;
+    // element e of a pair (a, b):  a' = a cos[e] + b sin[partner],  b' = b cos[e] - a sin[partner]
+    float other[8];
+    if (f.pairing == 1) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) other[i] = __shfl_xor(v[i], 4, 64);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) other[i] = v[i ^ 1];
+    }
+    if (sub < 8) {
+      float c[8], s[8];
+      const long co = pos * 64 + sub * 8, so = f.pairing == 1 ? pos * 64 + (sub ^ 4) * 8 : co;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int j = f.pairing == 1 ? i : i ^ 1;
+        c[i] = f.cs_f32 ? ((const float*)f.cos_t)[co + i] : bf16_bits_to_f32(((const unsigned short*)f.cos_t)[co + i]);
+        s[i] = f.cs_f32 ? ((const float*)f.sin_t)[so + j] : bf16_bits_to_f32(((const unsigned short*)f.sin_t)[so + j]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const bool second = f.pairing == 1 ? sub >= 4 : (i & 1);
+        const float y = second ? (-other[i]) * s[i] + v[i] * c[i] : v[i] * c[i] + other[i] * s[i];
+        v[i] = bf16_bits_to_f32(f32_to_bf16_bits(y));
+      }
+    }
+  }
 }
 
-template <int NHT>
-__global__ __launch_bounds__(256, 1) void indexer_bwd_kernel(
-    const float* __restrict__ gsc, const unsigned char* __restrict__ q8, const unsigned char* __restrict__ k8,
-    const float* __restrict__ k_scale, const float* __restrict__ q_w, const int* __restrict__ ids,
-    const int* __restrict__ dst, unsigned short* __restrict__ rows, float* __restrict__ d_q8, float* __restrict__ d_qw,
-    int q0, int cnt, int Sk, int K, int dummy_row) {
+// elements [8 sub, 8 sub + 8) of an output row of `dim` elements, bf16 or fp32
+__device__ __forceinline__ void store_row(const float (&v)[8], void* base, int is_f32, size_t row, int dim, int sub) {
+  const int c0 = 8 * sub;
+  if (c0 >= dim) return;
+  if (dim % 8 == 0) {
+    if (is_f32) {
+      float* p = (float*)base + row * dim + c0;
+      *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]};
+      *(f32x4*)(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+    } else {
+      *(uint4*)((unsigned short*)base + row * dim + c0) =
+          make_uint4(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]), cvt_pk_bf16(v[4], v[5]), cvt_pk_bf16(v[6], v[7]));
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    if (c0 + i < dim) {
+      if (is_f32) ((float*)base)[row * dim + c0 + i] = v[i];
+      else ((unsigned short*)base)[row * dim + c0 + i] = f32_to_bf16_bits(v[i]);
+    }
+}
+
+struct BwdArgs {
+  const float* gsc;
+  const unsigned char* q8;
+  const unsigned char* k8;
+  const float* k_scale;
+  const float* q_w;
+  const int* ids;
+  const int* dst;
+  unsigned short* rows;
+  int q0, cnt, Sk, K, dummy_row;
+  // plain payload gradients (q_scale null) ...
+  float* d_q8;                           // [S, HI, 128]
+  float* d_qw;                           // [S, HI]
+  // ... or finished ones
+  const float* q_scale;
+  float w_scale;
+  RowFinish fin;
+  const int* pos_q;
+  int heads, dim;                        // of the outputs
+  void* d_q; int q_f32;                  // [S, heads, dim]
+  void* d_w; int w_f32;                  // [S, heads]
+};
+
+size_t bwd_lds_bytes(int HI, int K) {
+  const size_t loop = (size_t)STAGES * TILE_BYTES + (size_t)HI * D + (size_t)K * 16 + 4 * 64 * 4 + 64 * 4 + 64;
+  const size_t red = (size_t)4 * HI * RED_STRIDE * 4 + 4 * 64 * 4;
+  return loop > red ? loop : red;
+}
+
+template <int NHT>   // head tiles of 32
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void indexer_bwd_kernel(const BwdArgs A) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int HI = 32 * NHT;
-  // [2][TILE_BYTES] fp8 key tiles | kb [4 waves][32 keys][256 B] bf16 keys | es [4 waves][2][32 keys][HI] bf16 E |
-  // idx_s [K] | a_s [K] | dst_s [K] | dw_red [4][64] | strip [4 waves][32][STRIP_STRIDE]
-  unsigned char* kb = smem + 2 * TILE_BYTES;
-  unsigned char* es = kb + 4 * 32 * 256;
-  int* idx_s = (int*)(es + 4 * 2 * 32 * 128);
-  float* a_s = (float*)(idx_s + K);
-  int* dst_s = (int*)(a_s + K);
-  float* dw_red = (float*)(dst_s + K);
-  unsigned char* strip = (unsigned char*)(dw_red + 4 * 64) + (threadIdx.x >> 6) * (32 * STRIP_STRIDE);   // per wave
-  float* red = (float*)smem;                        // [HI][RED_STRIDE], reuses the tile area at the end
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NDT = NHT == 2 ? 4 : 2;  // d-tiles of d_q8 of a wave: all of its head tile's, or half of the only one's
+  // [STAGES][TILE_BYTES] fp8 key tiles | q8 [HI][128] | a_s [K] f32 | ahl_s [K / 4][4 hi, 4 lo] bf16 | idx_s [K] | dst_s [K] |
+  // w_s [64] | last_s
+  unsigned char* qs = smem + STAGES * TILE_BYTES;
+  const int K = A.K;
+  float* a_s = (float*)(qs + HI * D);
+  unsigned short* ahl_s = (unsigned short*)(a_s + K);
+  int* idx_s = (int*)(ahl_s + 2 * K);
+  int* dst_s = idx_s + K;
+  float* w_s = (float*)(dst_s + K);
+  int* last_s = (int*)(w_s + 64);
+  float* dw_red = (float*)smem;                     // [4][64], then red [4][HI][RED_STRIDE], reuse the front at the end
+  float* red = dw_red + 4 * 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave >> 1, jh = wave & 1;          // slots 32 kg .. of a tile; which half of the pair's work
+  const int ht = NHT == 2 ? jh : 0, dt0 = NHT == 2 ? 0 : 2 * jh;
   const int r = lane & 31, g = lane >> 5;
-  const int ql = cnt - 1 - (int)blockIdx.x;
-  const int qi = q0 + ql;
+  const int ql = A.cnt - 1 - (int)blockIdx.x;
+  const int qi = A.q0 + ql;
 
-  for (int t0 = tid; t0 < K; t0 += 8 * 256) {     // eight slots per thread with all their loads in flight
-    int v[8], d[8];
-    float gv[8], kv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int t = min(t0 + i * 256, K - 1);
-      v[i] = ids[(size_t)qi * K + t];
-      gv[i] = gsc[(size_t)qi * K + t];
-      d[i] = dst[(size_t)ql * K + t];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) kv[i] = k_scale[(v[i] >= 0 && v[i] < Sk) ? v[i] : 0];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int t = t0 + i * 256;
-      if (t < K) {
-        const bool ok = v[i] >= 0 && v[i] < Sk;
-        idx_s[t] = ok ? v[i] : -1;
-        a_s[t] = ok ? gv[i] * kv[i] : 0.f;
-        dst_s[t] = (ok && d[i] >= 0) ? d[i] : dummy_row;
-      }
-    }
-  }
-  // stage q8[i] (HI x 128 bytes) in the kb area to build the transposed bf16 operand
-  for (int c = tid; c < HI * 8; c += 256) *(uint4*)(kb + c * 16) = *(const uint4*)(q8 + (size_t)qi * HI * D + c * 16);
-  __syncthreads();
-
-  // ---- register-resident operands ---------------------------------------------------------
-  i32x8 aq[NHT][2];          // fp8 rows of the query: A operand of r
-  float wq[NHT][16];         // q_w of the 16 heads a lane sees per head tile
-  float dwp[NHT][16];
-  bf16x8 qt[4][2 * NHT];     // Q^T: lane = d row (32*dt + r), 8 heads of k-step kk = 2*ht + s
-#pragma unroll
-  for (int t = 0; t < NHT; t++) {
-    const unsigned char* row = q8 + ((size_t)qi * HI + 32 * t + r) * D + 32 * g;
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-      const i32x4 lo = *(const i32x4*)(row + 64 * s);
-      const i32x4 hi = *(const i32x4*)(row + 64 * s + 16);
-      aq[t][s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
-    const float* wrow = q_w + (size_t)qi * HI + 32 * t + 4 * g;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const f32x4 w4 = *(const f32x4*)(wrow + 8 * j);
-#pragma unroll
-      for (int e = 0; e < 4; e++) { wq[t][4 * j + e] = w4[e]; dwp[t][4 * j + e] = 0.f; }
-    }
-  }
-#pragma unroll
-  for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-    for (int kk = 0; kk < 2 * NHT; kk++) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int head = 16 * kk + 8 * (e >> 2) + 4 * g + (e & 3);
-        const int byte = kb[head * D + 32 * dt + r];
-        qt[dt][kk][e] = (__bf16)__builtin_amdgcn_cvt_f32_fp8(byte, 0);
-      }
-      asm volatile("" : "+a"(qt[dt][kk]));
-    }
-  f32x16 dq_acc[NHT][4];
+  // ---- the query: slots, rows, weights ----------------------------------------------------------
+  if (tid == 0) *last_s = -1;
+  const unsigned char* qrow = A.q8 + (size_t)qi * HI * D;
+  i32x8 aq[NHT][2];          // fp8 rows of the query, bytes [64 s + 32 g, + 32) of head r of tile t ^ ht (0: the wave's own)
 #pragma unroll
   for (int t = 0; t < NHT; t++)
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++) {
-#pragma unroll
-      for (int e = 0; e < 16; e++) dq_acc[t][dt][e] = 0.f;
-      asm volatile("" : "+a"(dq_acc[t][dt]));
+    for (int s = 0; s < 2; s++) {
+      const unsigned char* p = qrow + (32 * (t ^ ht) + r) * D + 32 * g + 64 * s;
+      const i32x4 lo = *(const i32x4*)p, hi = *(const i32x4*)(p + 16);
+      aq[t][s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
+  if (tid < HI) w_s[tid] = A.q_w[(size_t)qi * HI + tid];
+  if (tid < HI * 8) *(uint4*)(qs + (tid >> 3) * D + (((tid & 7) ^ slot_xor(tid >> 3)) << 4)) = *(const uint4*)(qrow + tid * 16);
+  __syncthreads();
+  int last = -1;
+  for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {   // four slots per thread with all their loads in flight
+    int v[4], d[4];
+    float gv[4], kv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int t = min(t0 + i * THREADS, K - 1);
+      v[i] = A.ids[(size_t)qi * K + t];
+      gv[i] = A.gsc[(size_t)qi * K + t];
+      d[i] = A.dst[(size_t)ql * K + t];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) kv[i] = A.k_scale[(v[i] >= 0 && v[i] < A.Sk) ? v[i] : 0];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int t = t0 + i * THREADS;
+      if (t < K) {
+        const bool ok = v[i] >= 0 && v[i] < A.Sk;
+        const float a = ok ? gv[i] * kv[i] : 0.f;
+        const unsigned short hi = f32_to_bf16_bits(a);
+        idx_s[t] = ok ? v[i] : 0;
+        a_s[t] = a;
+        ahl_s[(t >> 2) * 8 + (t & 3)] = hi;
+        ahl_s[(t >> 2) * 8 + 4 + (t & 3)] = f32_to_bf16_bits(a - bf16_bits_to_f32(hi));
+        dst_s[t] = (ok && d[i] >= 0) ? d[i] : A.dummy_row;
+        if (ok) last = t;
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) last = max(last, __shfl_xor(last, o, 64));
+  if (lane == 0) atomicMax(last_s, last);
+
+  // (q_w Q)^T operands: lane = d row 32 (2 jh + u) + r, 8 heads of k-step kk = 2 t + s in accumulator order
+  const int blk = lane >> 4, ii = lane & 15;
+  const int tr_row = 8 * (ii >> 3) + 4 * g + ((ii >> 1) & 3);          // row of a transposing read, + 16 per k-step
+  bf16x8 qt[2][2 * NHT];
+#pragma unroll
+  for (int kk = 0; kk < 2 * NHT; kk++) {
+    const int h0 = 32 * ((kk >> 1) ^ ht) + 16 * (kk & 1);
+    const f32x4 w0 = *(const f32x4*)(w_s + h0 + 4 * g), w1 = *(const f32x4*)(w_s + h0 + 8 + 4 * g);
+    const int row = h0 + tr_row;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int chunk = 2 * (2 * jh + u) + (blk & 1);
+      const bf16x8 x = fp8_to_bf16(read_tr8(qs + row * D + ((chunk ^ slot_xor(row)) << 4) + 8 * (ii & 1)));
+      unsigned pk[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const f32x4& w = e < 2 ? w0 : w1;
+        pk[e] = cvt_pk_bf16((float)x[2 * e] * w[(2 * e) & 3], (float)x[2 * e + 1] * w[(2 * e + 1) & 3]);
+      }
+      qt[u][kk] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+    }
+  }
+  f32x16 dq_acc[NDT];
+#pragma unroll
+  for (int u = 0; u < NDT; u++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) dq_acc[u][e] = 0.f;
+  float dw = 0.f;            // d_qw of head 32 ht + r over the keys of this half-wave
   DSA_WAIT_VMCNT(0);
   __syncthreads();
+  const int ntile = (*last_s + TK) / TK;            // tiles behind the last valid slot have nothing to add
 
-  // ---- lane-dependent LDS offsets -------------------------------------------------------------
-  unsigned b_off[2][2];      // B operand of r: key row r of the wave's 32, bytes [64s + 32g, +32)
+  // ---- lane-dependent LDS offsets ------------------------------------------------------------------
+  unsigned b_off[2][2];      // key row r of the wave's 32, bytes [64 s + 32 g, + 32)
 #pragma unroll
   for (int s = 0; s < 2; s++)
 #pragma unroll
-    for (int x = 0; x < 2; x++) b_off[s][x] = (unsigned)((32 * wave + r) * D + (((4 * s + 2 * g + x) ^ swz(r)) << 4));
-  const int blk = lane >> 4, ii = lane & 15;
-  // transpose reads: lane (blk, ii) points at key 16*s2 + 8*t + 4*g + ii/4, column chunk 16*(blk&1) + 4*(ii&3)
-  // Both wave-private buffers XOR the 16-byte slot index with a permutation of the key's bits
-  // (kb_swz: 16 slots per 256-byte row, es_swz: 8 slots per 128-byte row), chosen so that the
-  // row-wise writes by 16 lanes and the transpose reads by 32 lanes spread over all banks.
-  unsigned kt_off[2][2][4], et_off[2][2][NHT];
+    for (int x = 0; x < 2; x++) b_off[s][x] = (unsigned)((32 * kg + r) * D + (((4 * s + 2 * g + x) ^ slot_xor(r)) << 4));
+  unsigned kt_off[2];        // K^T operand of k-step s, d-tile 0 (d-tile dt: XOR dt << 5)
 #pragma unroll
-  for (int s2 = 0; s2 < 2; s2++)
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int key = 16 * s2 + 8 * t + 4 * g + (ii >> 2);
-      const int sub = 2 * (blk & 1) + ((ii & 3) >> 1), half = (ii & 1) * 8;
-#pragma unroll
-      for (int dt = 0; dt < 4; dt++)
-        kt_off[s2][t][dt] = (unsigned)(wave * 8192 + key * 256 + (((4 * dt + sub) ^ kb_swz(key)) << 4) + half);
-#pragma unroll
-      for (int tt = 0; tt < NHT; tt++)
-        et_off[s2][t][tt] = (unsigned)(wave * 8192 + key * 128 + (((4 * tt + sub) ^ es_swz(key)) << 4) + half);
-    }
+  for (int s = 0; s < 2; s++) {
+    const int row = 16 * s + tr_row;
+    kt_off[s] = (unsigned)((32 * kg + row) * D + (((blk & 1) ^ slot_xor(row)) << 4) + 8 * (ii & 1));
+  }
 
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   const int gkey = tid >> 3, gsub = tid & 7;
-  const int ntile = K / TK;
-  auto issue = [&](int t) {
-    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((t & 1) * TILE_BYTES + wave * 1024));
+  auto issue = [&](int n) {
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + wave * 1024));
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const int key = c * 32 + gkey;
-      int kid = idx_s[t * TK + key];
-      kid = kid < 0 ? 0 : kid;
-      dma16(lb + c * 4096, (unsigned)kid * D + (unsigned)((gsub ^ swz(key)) * 16), k8);
+    for (int c = 0; c < 2; c++) {
+      const int key = c * 64 + gkey;
+      dma16(lb + c * 8192, (unsigned)idx_s[n * TK + key] * D + (unsigned)((gsub ^ slot_xor(key)) * 16), A.k8);
     }
   };
-  issue(0);
-  for (int t = 0; t < ntile; t++) {
-    // issued after this tile's 4 transfers: the 16 row stores of the previous tile
-    if (t > 0) { DSA_WAIT_VMCNT(16); } else { DSA_WAIT_VMCNT(0); }
+  for (int n = 0; n < STAGES - 1 && n < ntile; n++) issue(n);
+  for (int n = 0; n < ntile; n++) {
+    // issued behind this tile's two transfers: two per later tile in flight, four row stores per tile since
+    if (n >= 3 && n + 2 < ntile) { DSA_WAIT_VMCNT(16); }
+    else if (n >= 3) { DSA_WAIT_VMCNT(12); }
+    else if (n + 2 < ntile) { DSA_WAIT_VMCNT(4); }
+    else { DSA_WAIT_VMCNT(0); }
     __syncthreads();
-    if (t + 1 < ntile) issue(t + 1);
-    const unsigned char* tb = smem + (t & 1) * TILE_BYTES;
-    const int slot = t * TK + 32 * wave + r;
-    const float a = a_s[slot];
-
-    // ---- r, E, d_qw -----------------------------------------------------------------------------
+    if (n + STAGES - 1 < ntile) issue(n + STAGES - 1);
+    const unsigned char* tb = smem + (n % STAGES) * TILE_BYTES;
+    const int slot0 = n * TK + 32 * kg;
     i32x8 bk[2];
 #pragma unroll
     for (int s = 0; s < 2; s++) {
@@ -207,170 +319,127 @@ __global__ __launch_bounds__(256, 1) void indexer_bwd_kernel(
       const i32x4 hi = *(const i32x4*)(tb + b_off[s][1]);
       bk[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
-    bf16x8 ehi[NHT][2], elo[NHT][2];
+    // ---- keys on the columns: masks over the heads, then the rows of d_k8 ----------------------------
+    bf16x8 mk[2 * NHT];
 #pragma unroll
-    for (int tt = 0; tt < NHT; tt++) {
+    for (int t = 0; t < NHT; t++) {
       f32x16 acc;
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[e] = 0.f;
-      acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[tt][0], bk[0], acc, 0, 0, 0, 127, 0, 127);
-      acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[tt][1], bk[1], acc, 0, 0, 0, 127, 0, 127);
+      acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[t][0], bk[0], acc, 0, 0, 0, 127, 0, 127);
+      acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[t][1], bk[1], acc, 0, 0, 0, 127, 0, 127);
 #pragma unroll
-      for (int e = 0; e < 16; e += 2) {
-        // two neighbouring heads at a time: one packed conversion for the bf16 heads of E, one for what they miss
-        float ev[2];
+      for (int s = 0; s < 2; s++) {
+        unsigned pk[4];
+        // r is a multiple of 2^-18: scaled by 2^40 and clamped it is 0 or 1
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          pk[e] = cvt_pk_bf16(__builtin_amdgcn_fmed3f(acc[8 * s + 2 * e] * 0x1p40f, 0.f, 1.f),
+                              __builtin_amdgcn_fmed3f(acc[8 * s + 2 * e + 1] * 0x1p40f, 0.f, 1.f));
+        mk[2 * t + s] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+      }
+    }
+    const float a = a_s[slot0 + r];
+    unsigned short* rowp = A.rows + (size_t)dst_s[slot0 + r] * D + 64 * jh + 8 * g;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      f32x16 racc;
+#pragma unroll
+      for (int e = 0; e < 16; e++) racc[e] = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 2 * NHT; kk++) racc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt[u][kk], mk[kk], racc, 0, 0, 0);
+      uint4 o[2];
+      acc_row_to_16B(racc, a, o);
+      *(uint4*)(rowp + 32 * u) = o[0];
+      *(uint4*)(rowp + 32 * u + 16) = o[1];
+    }
+    // ---- heads on the columns: d_qw, then d_q8 ---------------------------------------------------------
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+    acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bk[0], aq[0][0], acc, 0, 0, 0, 127, 0, 127);
+    acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bk[1], aq[0][1], acc, 0, 0, 0, 127, 0, 127);
+    bf16x8 eh[2], el[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      unsigned ph[4], pl[4];
+#pragma unroll
+      for (int b = 0; b < 2; b++) {        // keys 16 s + 8 b + 4 g .. + 3
+        const f32x4 a4 = *(const f32x4*)(a_s + slot0 + 16 * s + 8 * b + 4 * g);
+        const uint4 hl = *(const uint4*)(ahl_s + 2 * (slot0 + 16 * s + 8 * b + 4 * g));
+        const unsigned h2[2] = {hl.x, hl.y}, l2[2] = {hl.z, hl.w};
 #pragma unroll
         for (int x = 0; x < 2; x++) {
-          const float rr = acc[e + x];
-          dwp[tt][e + x] = fmaf(a, __builtin_bit_cast(float, max(__builtin_bit_cast(int, rr), 0)), dwp[tt][e + x]);   // relu on the bit pattern
-          ev[x] = rr > 0.f ? a * wq[tt][e + x] : 0.f;
+          const float r0 = acc[8 * s + 4 * b + 2 * x], r1 = acc[8 * s + 4 * b + 2 * x + 1];
+          dw = fmaf(a4[2 * x], __builtin_bit_cast(float, max(__builtin_bit_cast(int, r0), 0)), dw);      // relu on the bit pattern
+          dw = fmaf(a4[2 * x + 1], __builtin_bit_cast(float, max(__builtin_bit_cast(int, r1), 0)), dw);
+          // sign of 2^-20 - r: set where r > 0; spread over the 16 bits of its element
+          typedef short i16x2 __attribute__((ext_vector_type(2)));
+          const unsigned sg = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, 0x1p-20f - r1), __builtin_bit_cast(unsigned, 0x1p-20f - r0), 0x07060302u);
+          const unsigned m = __builtin_bit_cast(unsigned, (i16x2)(__builtin_bit_cast(i16x2, sg) >> (i16x2)15));
+          ph[2 * b + x] = m & h2[x];
+          pl[2 * b + x] = m & l2[x];
         }
-        const unsigned ph = cvt_pk_bf16(ev[0], ev[1]);
-        const unsigned pl = cvt_pk_bf16(ev[0] - __builtin_bit_cast(float, ph << 16), ev[1] - __builtin_bit_cast(float, ph & 0xffff0000u));
-        const bf16x2 h2 = __builtin_bit_cast(bf16x2, ph), l2 = __builtin_bit_cast(bf16x2, pl);
-        ehi[tt][e >> 3][e & 7] = h2[0]; ehi[tt][e >> 3][(e & 7) + 1] = h2[1];
-        elo[tt][e >> 3][e & 7] = l2[0]; elo[tt][e >> 3][(e & 7) + 1] = l2[1];
       }
+      eh[s] = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+      el[s] = __builtin_bit_cast(bf16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
     }
-    __builtin_amdgcn_sched_barrier(0);
-
-    // ---- d_k8 rows: row^T[d, key] = Q^T . E, 32 keys of this wave --------------------------------
-    {
-      // Rows leave as bf16 (the ordered sum over a key's rows runs in fp32; one row carries 2^-9 of
-      // relative rounding, so E enters these products as its bf16 head alone).  Two 32 x 32 d-tiles at a
-      // time are rounded, transposed through a wave-private LDS strip and stored, so that a store
-      // instruction writes eight complete 128-byte row segments (lane: key 8*i + lane/8, 16-byte piece
-      // lane%8) instead of scattered 8-byte pieces.
-      unsigned short* rowp[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        rowp[i] = rows + (size_t)dst_s[t * TK + 32 * wave + 8 * i + (lane >> 3)] * D + 8 * (lane & 7);
-      unsigned char* sw = strip + r * STRIP_STRIDE + 8 * g;
-      const unsigned char* sr = strip + (lane >> 3) * STRIP_STRIDE + (lane & 7) * 16;
-      auto row_mfmas = [&](int dt, f32x16& racc) {
-        mfma_v_av_first(racc, qt[dt][0], ehi[0][0]);
+    for (int s = 0; s < 2; s++)
 #pragma unroll
-        for (int kk = 1; kk < 2 * NHT; kk++) mfma_v_av(racc, qt[dt][kk], ehi[kk >> 1][kk & 1]);
-      };
-      f32x16 racc[2];
-      row_mfmas(0, racc[0]);
-#pragma unroll
-      for (int dt = 0; dt < 4; dt++) {
-        // the next d-tile's MFMAs run while this one is rounded into the strip
-        if (dt + 1 < 4) row_mfmas(dt + 1, racc[(dt + 1) & 1]);
-        else mfma_done_v(racc[dt & 1]);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {                // d = 32*dt + 8*j + 4*g .. +3 of key r
-          const uint2 w = make_uint2(cvt_pk_bf16(racc[dt & 1][4 * j], racc[dt & 1][4 * j + 1]),
-                                     cvt_pk_bf16(racc[dt & 1][4 * j + 2], racc[dt & 1][4 * j + 3]));
-          *(uint2*)(sw + 64 * (dt & 1) + 16 * j) = w;
-        }
-        if (dt & 1) {
-          __builtin_amdgcn_wave_barrier();
-#pragma unroll
-          for (int i = 0; i < 4; i++) *(uint4*)(rowp[i] + 64 * (dt >> 1)) = *(const uint4*)(sr + 8 * i * STRIP_STRIDE);
-          __builtin_amdgcn_wave_barrier();
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      for (int u = 0; u < NDT; u++) {
+        const bf16x8 kt = fp8_to_bf16(read_tr8(tb + (kt_off[s] ^ (unsigned)((dt0 + u) << 5))));
+        dq_acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, eh[s], dq_acc[u], 0, 0, 0);
+        dq_acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, el[s], dq_acc[u], 0, 0, 0);
       }
-    }
-
-    // ---- d_q8: this wave's key rows as bf16, E back to LDS, then transpose reads ------------------
-    {
-      // lane (key r, half g) converts bytes [64g, 64g + 64) of its key row
-      const unsigned char* krow = tb + (32 * wave + r) * D;
-      unsigned char* kdst = kb + wave * 8192 + r * 256;
-      const int ksw = kb_swz(r);
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int slot16 = (4 * g + c) ^ swz(r);
-        const i32x4 w = *(const i32x4*)(krow + slot16 * 16);
-        // e4m3 -> bf16 is exact; one instruction converts two bytes of a word
-        bf16x8 o0, o1;
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-          const bf16x2 lo2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[x], 1.0f, false);
-          const bf16x2 hi2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[x], 1.0f, true);
-          if (x < 2) { o0[4 * x] = lo2[0]; o0[4 * x + 1] = lo2[1]; o0[4 * x + 2] = hi2[0]; o0[4 * x + 3] = hi2[1]; }
-          else { o1[4 * (x - 2)] = lo2[0]; o1[4 * (x - 2) + 1] = lo2[1]; o1[4 * (x - 2) + 2] = hi2[0]; o1[4 * (x - 2) + 3] = hi2[1]; }
-        }
-        *(bf16x8*)(kdst + (((8 * g + 2 * c) ^ ksw) << 4)) = o0;
-        *(bf16x8*)(kdst + (((8 * g + 2 * c + 1) ^ ksw) << 4)) = o1;
-      }
-      // E[key r][heads]: the lane holds heads 32*tt + 8*j + 4*g + (0..3)
-      unsigned char* edst = es + wave * 8192 + r * 128;
-      const int esw = es_swz(r);
-#pragma unroll
-      for (int tt = 0; tt < NHT; tt++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int hb = (((4 * tt + j) ^ esw) << 4) + 8 * g;      // heads 32*tt + 8*j + 4*g .. +3
-          bf16x4 vh, vl;
-#pragma unroll
-          for (int e = 0; e < 4; e++) { vh[e] = ehi[tt][j >> 1][4 * (j & 1) + e]; vl[e] = elo[tt][j >> 1][4 * (j & 1) + e]; }
-          *(bf16x4*)(edst + hb) = vh;
-          *(bf16x4*)(edst + 4096 + hb) = vl;
-        }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int s2 = 0; s2 < 2; s2++) {
-        bf16x8 bh[NHT], bl[NHT];
-#pragma unroll
-        for (int tt = 0; tt < NHT; tt++) {
-          bh[tt] = tr_pair(es + et_off[s2][0][tt], es + et_off[s2][1][tt]);
-          bl[tt] = tr_pair(es + 4096 + et_off[s2][0][tt], es + 4096 + et_off[s2][1][tt]);
-        }
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
-          const bf16x8 ak = tr_pair(kb + kt_off[s2][0][dt], kb + kt_off[s2][1][dt]);
-#pragma unroll
-          for (int tt = 0; tt < NHT; tt++) {
-            mfma_a_vv(dq_acc[tt][dt], ak, bh[tt]);
-            mfma_a_vv(dq_acc[tt][dt], ak, bl[tt]);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
   }
 
-  // ---- d_qw: sum the per-lane partials over the 32 keys of a half-wave, then over waves -----------
-#pragma unroll
-  for (int tt = 0; tt < NHT; tt++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      float v = dwp[tt][e];
-#pragma unroll
-      for (int o = 1; o < 32; o <<= 1) v += __shfl_xor(v, o, 64);
-      if (r == 0) dw_red[wave * 64 + 32 * tt + 8 * (e >> 2) + 4 * g + (e & 3)] = v;
-    }
-  // ---- d_q8: fixed-order sum of the four waves' accumulators through LDS ----------------------------
+  // ---- sums over the four slot groups, in a fixed order, through LDS ---------------------------------
   DSA_WAIT_VMCNT(0);
+  float w_row[2];
+#pragma unroll
+  for (int it = 0; it < NHT; it++) w_row[it] = w_s[32 * it + (tid >> 4)];
+  dw += __shfl_xor(dw, 32, 64);
   __syncthreads();
-  for (int w = 0; w < 4; w++) {
-    if (wave == w) {
+  if (g == 0 && (NHT == 2 || jh == 0)) dw_red[kg * 64 + 32 * ht + r] = dw;
 #pragma unroll
-      for (int tt = 0; tt < NHT; tt++)
+  for (int u = 0; u < NDT; u++) {
+    float* rp = red + ((size_t)kg * HI + 32 * ht + r) * RED_STRIDE + 32 * (dt0 + u) + 4 * g;
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
-          mfma_done_a(dq_acc[tt][dt]);
-          float* rp = red + (32 * tt + r) * RED_STRIDE + 32 * dt + 4 * g;
+    for (int j = 0; j < 4; j++)
+      *(f32x4*)(rp + 8 * j) = f32x4{dq_acc[u][4 * j], dq_acc[u][4 * j + 1], dq_acc[u][4 * j + 2], dq_acc[u][4 * j + 3]};
+  }
+  __syncthreads();
+  const int sub = tid & 15;
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            f32x4 v = {dq_acc[tt][dt][4 * j], dq_acc[tt][dt][4 * j + 1], dq_acc[tt][dt][4 * j + 2], dq_acc[tt][dt][4 * j + 3]};
-            if (w > 0) { const f32x4 old = *(const f32x4*)(rp + 8 * j); v += old; }
-            *(f32x4*)(rp + 8 * j) = v;
-          }
-        }
+  for (int it = 0; it < NHT; it++) {
+    const int h = 32 * it + (tid >> 4);
+    float v[8];
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      f32x4 p[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) p[k] = *(const f32x4*)(red + ((size_t)k * HI + h) * RED_STRIDE + 8 * sub + 4 * x);
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[4 * x + e] = ((p[0][e] + p[1][e]) + (p[2][e] + p[3][e])) * w_row[it];
     }
-    __syncthreads();
+    if (A.q_scale == nullptr) {
+      store_row(v, A.d_q8, 1, (size_t)qi * HI + h, D, sub);
+    } else {
+      finish_row(v, sub, A.q_scale[(size_t)qi * HI + h], A.fin, A.pos_q, qi);
+      if (h < A.heads) store_row(v, A.d_q, A.q_f32, (size_t)qi * A.heads + h, A.dim, sub);
+    }
   }
-  for (int c = tid; c < HI * 32; c += 256) {
-    const int h = c >> 5, d4 = c & 31;
-    *(f32x4*)(d_q8 + ((size_t)qi * HI + h) * D + 4 * d4) = *(const f32x4*)(red + h * RED_STRIDE + 4 * d4);
+  if (tid < HI) {
+    const float s = (dw_red[tid] + dw_red[64 + tid]) + (dw_red[128 + tid] + dw_red[192 + tid]);
+    if (A.q_scale == nullptr) {
+      A.d_qw[(size_t)qi * HI + tid] = s;
+    } else if (tid < A.heads) {
+      const float y = s * A.q_scale[(size_t)qi * HI + tid] * A.w_scale;
+      if (A.w_f32) ((float*)A.d_w)[(size_t)qi * A.heads + tid] = y;
+      else ((unsigned short*)A.d_w)[(size_t)qi * A.heads + tid] = f32_to_bf16_bits(y);
+    }
   }
-  if (tid < HI) d_qw[(size_t)qi * HI + tid] = (dw_red[tid] + dw_red[64 + tid]) + (dw_red[128 + tid] + dw_red[192 + tid]);
 }
 
 // d_k8[key] (+)= sum of the key's bf16 rows in fp32, ascending query order; 128 threads = 16 chunks of 8
@@ -403,6 +472,101 @@ __global__ __launch_bounds__(128) void indexer_reduce_kernel(const unsigned shor
     if (accumulate) s += *p;
     if (*dup_flag) s = __builtin_nanf("");       // a query row held a repeated id: no sum that misses a term
     *p = s;
+  }
+}
+
+// Gradients of the keys' projection from the summed payload gradients: the same steps as for the queries, then back
+// through the LayerNorm (fp32).  16 lanes per row; a workgroup takes every gridDim-th group of 16 rows and leaves its
+// share of the LayerNorm's parameter gradients in part[block][2][128] (summed in block order by the next kernel).
+// Bound by its launch (8192 keys: 6 MB).
+struct KeyArgs {
+  const float* d_k8;
+  const float* k_scale;
+  int Sk;
+  RowFinish fin;
+  const int* positions;
+  const unsigned short* k_in;            // bf16 input of the LayerNorm, or null
+  const float* ln_w;
+  float ln_eps;
+  void* d_k; int k_f32, dim;
+  float* part;
+};
+constexpr int KEY_BLOCKS = 256;
+
+__device__ __forceinline__ float sum16(float v) {
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+__global__ __launch_bounds__(256) void indexer_key_finish_kernel(const KeyArgs A) {
+  __shared__ float red_s[2][16][D];
+  const int sub = threadIdx.x & 15, grp = threadIdx.x >> 4;
+  float lw[8], dlw[8], dlb[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) { lw[i] = A.k_in ? A.ln_w[8 * sub + i] : 0.f; dlw[i] = dlb[i] = 0.f; }
+  for (int row0 = blockIdx.x * 16; row0 < A.Sk; row0 += gridDim.x * 16) {
+    const int row = min(row0 + grp, A.Sk - 1);
+    const bool live = row0 + grp < A.Sk;
+    float v[8];
+    const f32x4 p0 = *(const f32x4*)(A.d_k8 + (size_t)row * D + 8 * sub), p1 = *(const f32x4*)(A.d_k8 + (size_t)row * D + 8 * sub + 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) { v[i] = p0[i]; v[4 + i] = p1[i]; }
+    finish_row(v, sub, A.k_scale[row], A.fin, A.positions, row);
+    if (A.k_in) {
+      const uint4 raw = *(const uint4*)(A.k_in + (size_t)row * D + 8 * sub);
+      const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
+      float x[8], dx[8];
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        x[i] = (i & 1) ? __builtin_bit_cast(float, w[i >> 1] & 0xffff0000u) : __builtin_bit_cast(float, w[i >> 1] << 16);
+        s += x[i];
+      }
+      const float mean = sum16(s) * (1.f / D);
+      s = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) { x[i] -= mean; s += x[i] * x[i]; }
+      const float rstd = rsqrtf(sum16(s) * (1.f / D) + A.ln_eps);
+      float m1 = 0.f, m2 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        x[i] *= rstd;
+        if (live) { dlw[i] += v[i] * x[i]; dlb[i] += v[i]; }
+        dx[i] = v[i] * lw[i];
+        m1 += dx[i];
+        m2 += dx[i] * x[i];
+      }
+      m1 = sum16(m1) * (1.f / D);
+      m2 = sum16(m2) * (1.f / D);
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = rstd * (dx[i] - m1 - x[i] * m2);
+    }
+    if (live) store_row(v, A.d_k, A.k_f32, row, A.dim, sub);
+  }
+  if (!A.k_in) return;
+#pragma unroll
+  for (int i = 0; i < 8; i++) { red_s[0][grp][8 * sub + i] = dlw[i]; red_s[1][grp][8 * sub + i] = dlb[i]; }
+  __syncthreads();
+  const int which = threadIdx.x >> 7, c = threadIdx.x & 127;
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; k++) s += red_s[which][k][c];
+  A.part[(size_t)blockIdx.x * 2 * D + threadIdx.x] = s;
+}
+
+__global__ __launch_bounds__(256) void indexer_ln_sum_kernel(const float* __restrict__ part, int blocks, float* __restrict__ d_w,
+                                                             float* __restrict__ d_b) {
+  __shared__ float red_s[4][64];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;      // column of [2][128]
+  float s = 0.f;
+  for (int b = grp; b < blocks; b += 4) s += part[(size_t)b * 2 * D + c];
+  red_s[grp][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (grp == 0) {
+    const int t = threadIdx.x;
+    s = (red_s[0][t] + red_s[1][t]) + (red_s[2][t] + red_s[3][t]);
+    if (c < D) d_w[c] = s; else d_b[c - D] = s;
   }
 }
 
@@ -445,22 +609,29 @@ extern "C" size_t dsa_indexer_bwd_workspace_bytes(int S, int Hi, int Sk, int K) 
   return make_plan(S, Sk, K, DEFAULT_BUDGET).total;
 }
 
-extern "C" int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
-                               const int32_t* ids, int S, int Hi, int Sk, int K, float* d_q8, float* d_k8, float* d_qw,
-                               void* workspace, size_t workspace_bytes, void* stream) {
-  DSA_REQUIRE(Hi == 32 || Hi == 64, "dsa_indexer_bwd: head count must be 32 or 64, got %d", Hi);
-  DSA_REQUIRE(S >= 0 && Sk > 0, "dsa_indexer_bwd: bad sizes S=%d Sk=%d", S, Sk);
-  DSA_REQUIRE(K > 0 && K % TK == 0 && K <= 4096, "dsa_indexer_bwd: top-k must be a multiple of 128 up to 4096, got %d", K);
-  DSA_REQUIRE((size_t)Sk * D <= 0xffffffffull, "dsa_indexer_bwd: key array too large");
-  DSA_REQUIRE(Sk <= order::MAX_KEYS, "dsa_indexer_bwd: at most %d keys are supported, got %d", order::MAX_KEYS, Sk);
-  DSA_REQUIRE(((uintptr_t)q8 % 16) == 0 && ((uintptr_t)k8 % 16) == 0 && ((uintptr_t)q_w % 16) == 0 &&
-              ((uintptr_t)d_q8 % 16) == 0 && ((uintptr_t)d_k8 % 16) == 0 && ((uintptr_t)workspace % 256) == 0,
-              "dsa_indexer_bwd: misaligned pointer");
+namespace {
+
+// what dsa_indexer_grads asks for on top of the payload gradients
+struct KeyFinish {
+  KeyArgs key;
+  float* d_ln_w;
+  float* d_ln_b;
+};
+
+int run_bwd(const char* name, BwdArgs A, int S, int Hi, float* d_k8, const KeyFinish* kf, void* workspace, size_t workspace_bytes, void* stream) {
+  const int Sk = A.Sk, K = A.K;
+  DSA_REQUIRE(Hi == 32 || Hi == 64, "%s: head count must be 32 or 64, got %d", name, Hi);
+  DSA_REQUIRE(S >= 0 && Sk > 0, "%s: bad sizes S=%d Sk=%d", name, S, Sk);
+  DSA_REQUIRE(K > 0 && K % TK == 0 && K <= 4096, "%s: top-k must be a multiple of 128 up to 4096, got %d", name, K);
+  DSA_REQUIRE((size_t)Sk * D <= 0xffffffffull, "%s: key array too large", name);
+  DSA_REQUIRE(Sk <= order::MAX_KEYS, "%s: at most %d keys are supported, got %d", name, order::MAX_KEYS, Sk);
+  DSA_REQUIRE(((uintptr_t)A.q8 % 16) == 0 && ((uintptr_t)A.k8 % 16) == 0 && ((uintptr_t)A.q_w % 16) == 0 &&
+              ((uintptr_t)A.d_q8 % 16) == 0 && ((uintptr_t)A.d_q % 16) == 0 && ((uintptr_t)d_k8 % 16) == 0 && ((uintptr_t)workspace % 256) == 0,
+              "%s: misaligned pointer", name);
   hipStream_t st = (hipStream_t)stream;
   Plan p = make_plan(S > 0 ? S : 1, Sk, K, workspace_bytes);
   if (p.total > workspace_bytes || workspace == nullptr)
-    DSA_FAIL(DSA_ERR_WORKSPACE, "dsa_indexer_bwd: workspace of %zu bytes is too small (need at least %zu)",
-             workspace_bytes, layout_plan(64, Sk, K).total);
+    DSA_FAIL(DSA_ERR_WORKSPACE, "%s: workspace of %zu bytes is too small (need at least %zu)", name, workspace_bytes, layout_plan(64, Sk, K).total);
   unsigned char* ws = (unsigned char*)workspace;
   unsigned* bitmap = (unsigned*)(ws + p.off_bitmap);
   unsigned* prefix = (unsigned*)(ws + p.off_prefix);
@@ -468,27 +639,79 @@ extern "C" int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, c
   int* start = (int*)(ws + p.off_start);
   int* dup_flag = (int*)(ws + p.off_flag);
   int* dstp = (int*)(ws + p.off_dst);
-  unsigned short* rows = (unsigned short*)(ws + p.off_rows);
-  size_t smem = (size_t)2 * TILE_BYTES + 4 * 32 * 256 + 4 * 2 * 32 * 128 + (size_t)K * 12 + 4 * 64 * 4 + 4 * 32 * STRIP_STRIDE;
-  const size_t red_bytes = (size_t)Hi * RED_STRIDE * 4;
-  if (red_bytes > (size_t)2 * TILE_BYTES + 4 * 32 * 256) smem += red_bytes;
+  A.dst = dstp;
+  A.rows = (unsigned short*)(ws + p.off_rows);
+  A.dummy_row = p.chunk * K;
+  const size_t smem = bwd_lds_bytes(Hi, K);
   auto kern = Hi == 32 ? indexer_bwd_kernel<1> : indexer_bwd_kernel<2>;
-  if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess)
-    DSA_FAIL(DSA_ERR_LAUNCH, "dsa_indexer_bwd: cannot reserve LDS");
+  if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) DSA_FAIL(DSA_ERR_LAUNCH, "%s: cannot reserve LDS", name);
   bool first = true;
   order::clear_flag(dup_flag, st);
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
-    const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
+    A.q0 = q0;
+    A.cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     // every id inside [0, Sk) counts: the causal window was already applied when the ids were selected
-    order::build(ids, q0, cnt, K, Sk, 0x3fffffff, bitmap, prefix, count, start, dstp, p.W, st, dup_flag);
-    DSA_CHECK_LAUNCH("dsa_indexer_bwd(order)");
-    kern<<<dim3(cnt), dim3(256), smem, st>>>(g, (const unsigned char*)q8, (const unsigned char*)k8, k_scale, q_w, ids, dstp,
-                                             rows, d_q8, d_qw, q0, cnt, Sk, K, p.chunk * K);
-    DSA_CHECK_LAUNCH("dsa_indexer_bwd");
-    indexer_reduce_kernel<<<dim3(Sk), dim3(128), 0, st>>>(rows, start, d_k8, first ? 0 : 1, dup_flag);
-    DSA_CHECK_LAUNCH("dsa_indexer_bwd(reduce)");
+    order::build(A.ids, q0, A.cnt, K, Sk, 0x3fffffff, bitmap, prefix, count, start, dstp, p.W, st, dup_flag);
+    DSA_CHECK_LAUNCH("indexer_bwd(order)");
+    kern<<<dim3(A.cnt), dim3(THREADS), smem, st>>>(A);
+    DSA_CHECK_LAUNCH("indexer_bwd");
+    indexer_reduce_kernel<<<dim3(Sk), dim3(128), 0, st>>>(A.rows, start, d_k8, first ? 0 : 1, dup_flag);
+    DSA_CHECK_LAUNCH("indexer_bwd(reduce)");
     first = false;
   }
   if (S == 0) order::zero_u32_kernel<<<dim3(256), dim3(256), 0, st>>>((unsigned*)d_k8, (size_t)Sk * D);
+  if (kf) {
+    const int blocks = dsa_cdiv(Sk, 16) < KEY_BLOCKS ? dsa_cdiv(Sk, 16) : KEY_BLOCKS;
+    indexer_key_finish_kernel<<<dim3(blocks), dim3(256), 0, st>>>(kf->key);
+    if (kf->key.k_in) indexer_ln_sum_kernel<<<dim3(4), dim3(256), 0, st>>>(kf->key.part, blocks, kf->d_ln_w, kf->d_ln_b);
+    DSA_CHECK_LAUNCH("indexer_bwd(keys)");
+  }
   return DSA_OK;
+}
+
+size_t grads_extra_bytes(int Sk) { return align_up((size_t)Sk * D * 4) + align_up((size_t)KEY_BLOCKS * 2 * D * 4); }
+
+}  // namespace
+
+extern "C" int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
+                               const int32_t* ids, int S, int Hi, int Sk, int K, float* d_q8, float* d_k8, float* d_qw,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  BwdArgs A = {};
+  A.gsc = g; A.q8 = (const unsigned char*)q8; A.k8 = (const unsigned char*)k8; A.k_scale = k_scale; A.q_w = q_w; A.ids = ids;
+  A.Sk = Sk; A.K = K; A.d_q8 = d_q8; A.d_qw = d_qw;
+  return run_bwd("dsa_indexer_bwd", A, S, Hi, d_k8, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t dsa_indexer_grads_workspace_bytes(int S, int Hi, int Sk, int K) {
+  if (Sk <= 0 || K <= 0) return 0;
+  return dsa_indexer_bwd_workspace_bytes(S > 0 ? S : 1, Hi, Sk, K) + grads_extra_bytes(Sk);
+}
+
+extern "C" int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
+                                 const int32_t* ids, int S, int Hi, int Sk, int K, const float* q_scale, float w_scale, int rotate,
+                                 const void* cos, const void* sin, int tables_f32, int pairing, const int32_t* positions_q,
+                                 const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps,
+                                 int heads, int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32,
+                                 float* d_ln_w, float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream) {
+  DSA_REQUIRE(heads > 0 && heads <= Hi && dim > 0 && dim <= D, "dsa_indexer_grads: %d heads of %d channels do not fit %d x %d", heads, dim, Hi, D);
+  DSA_REQUIRE(q_scale != nullptr, "dsa_indexer_grads: q_scale is missing");
+  DSA_REQUIRE(pairing < 0 || (cos != nullptr && sin != nullptr && pairing <= 1 && batch > 0), "dsa_indexer_grads: bad rotary arguments");
+  DSA_REQUIRE(k_in == nullptr || (ln_w != nullptr && d_ln_w != nullptr && d_ln_b != nullptr), "dsa_indexer_grads: LayerNorm arguments are missing");
+  DSA_REQUIRE(((uintptr_t)d_k % 16) == 0 && ((uintptr_t)k_in % 16) == 0, "dsa_indexer_grads: misaligned pointer");
+  const size_t extra = grads_extra_bytes(Sk > 0 ? Sk : 1);
+  if (workspace == nullptr || workspace_bytes < extra || ((uintptr_t)workspace % 256) != 0)
+    DSA_FAIL(DSA_ERR_WORKSPACE, "dsa_indexer_grads: workspace of %zu bytes is too small or misaligned", workspace_bytes);
+  float* d_k8 = (float*)workspace;
+  BwdArgs A = {};
+  A.gsc = g; A.q8 = (const unsigned char*)q8; A.k8 = (const unsigned char*)k8; A.k_scale = k_scale; A.q_w = q_w; A.ids = ids;
+  A.Sk = Sk; A.K = K;
+  A.q_scale = q_scale; A.w_scale = w_scale;
+  A.fin = RowFinish{rotate, cos, sin, tables_f32, pairing, batch};
+  A.pos_q = positions_q; A.heads = heads; A.dim = dim;
+  A.d_q = d_q; A.q_f32 = q_f32; A.d_w = d_w; A.w_f32 = w_f32;
+  KeyFinish kf = {};
+  kf.key = KeyArgs{d_k8, k_scale, Sk, A.fin, positions_k, (const unsigned short*)k_in, ln_w, ln_eps, d_k, k_f32, dim,
+                   (float*)((unsigned char*)workspace + align_up((size_t)Sk * D * 4))};
+  kf.d_ln_w = d_ln_w; kf.d_ln_b = d_ln_b;
+  return run_bwd("dsa_indexer_grads", A, S, Hi, d_k8, &kf, (unsigned char*)workspace + extra, workspace_bytes - extra, stream);
 }

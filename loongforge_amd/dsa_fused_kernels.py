@@ -212,27 +212,13 @@ class DSADotProductAttention(MegatronModule):
 
 
 def _unscale_indexer_grad(grad, scale_inv):
-    """``grad / scale_inv`` with rows sitting on the quantiser's epsilon floor forced to zero
-    (loongforge/models/foundation/deepseek_v4/deepseek_v4_csa.py:1525-1541)."""
+    """``grad / scale_inv`` with rows sitting on the quantiser's epsilon floor forced to zero (loongforge/models/foundation/
+    deepseek_v4/deepseek_v4_csa.py:1525-1541); the backward kernel (:func:`ops.indexer_grads`) does the same per row."""
     epsilon_scale_floor = 2.0 ** -48 * 1.5
     scale_inv = scale_inv.unsqueeze(-1)
     usable = torch.isfinite(scale_inv) & (scale_inv > epsilon_scale_floor)
     safe = torch.where(usable, scale_inv, torch.ones_like(scale_inv))
     return (grad / safe).masked_fill(~usable.expand_as(grad), 0.0)
-
-
-_H128 = {}
-
-
-def _hadamard128(device) -> Tensor:
-    """Sylvester Hadamard matrix of order 128 in fp32 (cached per device)."""
-    key = str(device)
-    if key not in _H128:
-        h = torch.ones(1, 1, dtype=torch.float32, device=device)
-        while h.shape[0] < 128:
-            h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
-        _H128[key] = h
-    return _H128[key]
 
 
 def _pad_to(x: Tensor, size: int, dim: int) -> Tensor:
@@ -314,42 +300,13 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
     def backward(ctx, grad_score, grad_topk):
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, topk_indices = ctx.saved_tensors
         head, dim = ctx.shape
-        grad_score = torch.where(topk_indices >= 0, grad_score.float(), torch.zeros_like(grad_score, dtype=torch.float32))
-        d_q, d_k, d_weights = ops.indexer_bwd(grad_score.contiguous(), q_fp8, k_fp8, k_scale, weight_scaled,
-                                              topk_indices.int())
-        d_weights = d_weights * q_scale * ctx.softmax_scale
-        d_q = _unscale_indexer_grad(d_q, q_scale)
-        d_k = _unscale_indexer_grad(d_k, k_scale)
-        if ctx.rotate:      # the rotation is symmetric and orthogonal up to its scale: its transpose is itself
-            h = _hadamard128(d_q.device)
-            d_q = (d_q @ h) * 128 ** -0.5
-            d_k = (d_k @ h) * 128 ** -0.5
-        dq_t, dk_t, dw_t = ctx.in_dtypes
-        d_ln_w = d_ln_b = None
-        front = ctx.front
-        if front is not None:
-            # back through the rotary embedding (its transpose, on bf16 gradients as the separate kernel's
-            # backward sees them) and, on the key side, through the LayerNorm
-            d_q, d_k = d_q.to(torch.bfloat16).contiguous(), d_k.to(torch.bfloat16).contiguous()
-            _rope_q_rows(d_q, front.cos, front.sin, 0, 64, front.pairing, front.positions_q, front.batch, True)
-            _rope_q_rows(d_k.unsqueeze(1), front.cos, front.sin, 0, 64, front.pairing, front.positions_k, front.batch, True)
-            k_in, ln_w, ln_b = ctx.front_saved
-            d_k, d_ln_w, d_ln_b = _layer_norm_backward(d_k.float(), k_in.float(), ln_w.float(), front.k_norm_eps)
+        k_in, ln_w, ln_b = ctx.front_saved if ctx.front is not None else (None, None, None)
+        d_q, d_k, d_weights, d_ln_w, d_ln_b = ops.indexer_grads(
+            grad_score, q_fp8, k_fp8, k_scale, weight_scaled, topk_indices, q_scale, ctx.softmax_scale, head, dim, ctx.in_dtypes,
+            ctx.rotate, ctx.front, k_in, ln_w)
+        if ctx.front is not None:
             d_ln_w, d_ln_b = d_ln_w.to(ln_w.dtype), d_ln_b.to(ln_b.dtype)
-        return (d_q[:, :head, :dim].to(dq_t), d_k[:, :dim].to(dk_t), d_weights[:, :head].to(dw_t), None, None, None,
-                None, None, d_ln_w, d_ln_b)
-
-
-def _layer_norm_backward(dy: Tensor, x: Tensor, weight: Tensor, eps: float):
-    """Gradients of ``y = (x - mean) * rstd * weight + bias`` over the last dimension (fp32)."""
-    mean = x.mean(-1, keepdim=True)
-    xc = x - mean
-    rstd = torch.rsqrt(xc.square().mean(-1, keepdim=True) + eps)
-    xhat = xc * rstd
-    d_w, d_b = (dy * xhat).sum(0), dy.sum(0)
-    dxhat = dy * weight
-    dx = rstd * (dxhat - dxhat.mean(-1, keepdim=True) - xhat * (dxhat * xhat).mean(-1, keepdim=True))
-    return dx, d_w, d_b
+        return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b
 
 
 @dataclass

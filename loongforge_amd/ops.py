@@ -241,32 +241,7 @@ def indexer_topk(q8, q_w, k8, k_scale, ks, ke, K: int, sorted: bool = True):
 @torch.library.custom_op("dsa::indexer_bwd", mutates_args=())
 def _indexer_bwd_op(g: torch.Tensor, q8: torch.Tensor, k8: torch.Tensor, k_scale: torch.Tensor, q_w: torch.Tensor,
                     ids: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    _need_gpu(g, q8, k8, k_scale, q_w, ids)
-    S, Hi, D = q8.shape
-    Sk = k8.shape[0]
-    K = ids.shape[1]
-    if g.shape != ids.shape or ids.shape[0] != S:
-        raise ValueError("indexer_bwd: grad and ids must both be [S, K]")
-    Kp = (K + 127) // 128 * 128
-    g = g.float()
-    ids = ids.int()
-    if Kp != K:                       # slots are processed 128 at a time
-        g = torch.nn.functional.pad(g, (0, Kp - K), value=0.0)
-        ids = torch.nn.functional.pad(ids, (0, Kp - K), value=-1)
-    g, ids = _c(g), _c(ids)
-    q8, k8 = _c(_as_u8(q8)), _c(_as_u8(k8))
-    q_w, k_scale = _c(q_w.float()), _c(k_scale.float())
-    d_q8 = torch.empty(S, Hi, D, dtype=torch.float32, device=q8.device)
-    d_k8 = torch.empty(Sk, D, dtype=torch.float32, device=q8.device)
-    d_qw = torch.empty(S, Hi, dtype=torch.float32, device=q8.device)
-    lib = _lib.load()
-    nbytes = lib.dsa_indexer_bwd_workspace_bytes(S, Hi, Sk, Kp)
-    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=q8.device)
-    with torch.cuda.device(q8.device):
-        _lib.check(lib.dsa_indexer_bwd(g.data_ptr(), q8.data_ptr(), k8.data_ptr(), k_scale.data_ptr(), q_w.data_ptr(),
-                                       ids.data_ptr(), S, Hi, Sk, Kp, d_q8.data_ptr(), d_k8.data_ptr(), d_qw.data_ptr(),
-                                       ws.data_ptr(), nbytes, _stream(q8)), "dsa_indexer_bwd")
-    return d_q8, d_k8, d_qw
+    return _native().indexer_bwd(g, q8, k8, k_scale, q_w, ids, True)
 
 
 @_indexer_bwd_op.register_fake
@@ -277,7 +252,20 @@ def _(g, q8, k8, k_scale, q_w, ids):
 
 def indexer_bwd(g, q8, k8, k_scale, q_w, ids):
     """Gradients of the selected logits w.r.t. the fp8 payloads and the scaled weights (fp32)."""
-    return _indexer_bwd_op(g, q8, k8, k_scale, q_w, ids)
+    return _direct("indexer_bwd", _indexer_bwd_op, g, q8, k8, k_scale, q_w, ids)
+
+
+def indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale: float, heads: int, dim: int, dtypes, rotate: bool = False,
+                  front=None, k_in=None, ln_weight=None):
+    """:func:`indexer_bwd` carried on to the outputs of the projections: ``(d_q [S, heads, dim], d_k [Sk, dim], d_weights
+    [S, heads], d_ln_weight, d_ln_bias)`` in ``dtypes`` (of q, k, weights), the last two fp32 or None.  Unscaled (rows on the
+    quantiser's epsilon floor, loongforge/models/foundation/deepseek_v4/deepseek_v4_csa.py:1525-1541, get zero), back
+    through the Hadamard rotation if ``rotate``, and with ``front`` (an ``IndexerFrontEnd``) through the rotary embedding
+    and the LayerNorm of the keys (input ``k_in``, weight ``ln_weight``)."""
+    f = front
+    return _native().indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, float(w_scale), bool(rotate), f and f.cos, f and f.sin,
+                                   f.pairing if f else -1, f and f.positions_q, f and f.positions_k, f.batch if f else 1,
+                                   k_in, ln_weight, f.k_norm_eps if f else 0.0, int(heads), int(dim), *dtypes)
 
 
 def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offset: int, like: torch.Tensor):

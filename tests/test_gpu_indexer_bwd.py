@@ -98,3 +98,83 @@ def test_indexer_kernel_module_forward_and_backward(gpu):
         err = (got.double().cpu() - ref).abs()
         lim = 2e-2 * ref.abs().max().item()       # bf16 grads; ReLU-gate flips are rarer than 1e-4 of pairs
         assert (err > lim).float().mean().item() < 1e-3, name
+
+
+@pytest.mark.parametrize("S,Sk,heads,dim,K,rotate,pairing,dtypes", [
+    (1, 1, 32, 128, 128, False, -1, "fff"),          # one pair
+    (37, 45, 5, 64, 130, False, -1, "bbb"),          # few heads of few channels, slots padded to a tile
+    (70, 300, 64, 128, 256, True, 0, "bbf"),
+    (129, 129, 64, 128, 129, True, 1, "bfb"),
+    (33, 700, 20, 100, 640, False, -1, "hfb"),       # rows of 100 channels, half precision
+    (300, 40, 32, 128, 40, True, 1, "bbb"),          # rows without a valid slot, more queries than keys
+])
+def test_indexer_grads_equal_the_separate_steps(gpu, S, Sk, heads, dim, K, rotate, pairing, dtypes):
+    """Payload gradients -> unscale -> rotation -> rotary transpose -> LayerNorm backward in the kernels, against the same
+    steps one by one (from the kernels' own payload gradients, which the oracle test above covers)."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import IndexerFrontEnd, _unscale_indexer_grad
+
+    gen = torch.Generator().manual_seed(S + K)
+    hp = 32 if heads <= 32 else 64
+    q = torch.zeros(S, hp, 128)
+    q[:, :heads, :dim] = torch.randn(S, heads, dim, generator=gen)
+    k = torch.zeros(Sk, 128)
+    k[:, :dim] = torch.randn(Sk, dim, generator=gen)
+    k[0] = 0.0                                                  # on the quantiser's epsilon floor
+    w = torch.zeros(S, hp)
+    w[:, :heads] = torch.randn(S, heads, generator=gen)
+    q8, qs = ops.quant_rowwise_e4m3(q.to(torch.bfloat16).to(gpu))
+    k8, ksc = ops.quant_rowwise_e4m3(k.to(torch.bfloat16).to(gpu))
+    ws = (w.to(gpu) * qs * dim ** -0.5).contiguous()
+    ids = torch.stack([torch.randperm(max(Sk, K), generator=gen)[:K] for _ in range(S)]).int()
+    ids[ids >= Sk] = -1
+    ids[S // 2] = -1 if S > 1 else ids[0]
+    g = torch.randn(S, K, generator=gen)
+    g[ids < 0] = float("nan")
+    ids, g = ids.to(gpu), g.to(gpu)
+    front = k_in = ln_w = None
+    if pairing >= 0:
+        ang = torch.rand(max(S, Sk), 64, generator=gen) * 6
+        pos_q = torch.randint(0, max(S, Sk), (S,), generator=gen).int().to(gpu) if pairing == 1 else None
+        front = IndexerFrontEnd(cos=ang.cos().to(gpu), sin=ang.sin().to(gpu, torch.float32), pairing=pairing, positions_q=pos_q, k_norm_eps=1e-5)
+        k_in = torch.randn(Sk, 128, generator=gen).to(torch.bfloat16).to(gpu)
+        ln_w = torch.randn(128, generator=gen).to(gpu)
+    types = [dict(f=torch.float32, b=torch.bfloat16, h=torch.float16)[c] for c in dtypes]
+    got = ops.indexer_grads(g, q8, k8, ksc, ws, ids, qs, dim ** -0.5, heads, dim, types, rotate, front, k_in, ln_w)
+    again = ops.indexer_grads(g, q8, k8, ksc, ws, ids, qs, dim ** -0.5, heads, dim, types, rotate, front, k_in, ln_w)
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, again))
+
+    d_q, d_k, d_w = ops.indexer_bwd(torch.where(ids >= 0, g, torch.zeros_like(g)), q8, k8, ksc, ws, ids)
+    d_w = d_w * qs * dim ** -0.5
+    d_q, d_k = _unscale_indexer_grad(d_q, qs), _unscale_indexer_grad(d_k, ksc)
+    if rotate:
+        h = O.hadamard(128).float().to(gpu) if hasattr(O, "hadamard") else None
+        if h is None:
+            h = torch.ones(1, 1, device=gpu)
+            while h.shape[0] < 128:
+                h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+        d_q, d_k = (d_q @ h) * 128 ** -0.5, (d_k @ h) * 128 ** -0.5
+    ref_ln = [None, None]
+    if front is not None:
+        d_q, d_k = d_q.to(torch.bfloat16).contiguous(), d_k.to(torch.bfloat16).contiguous()
+        ops.rope_rows(d_q[:, :, :64], d_q[:, :, :64], front.cos, front.sin, pairing, pairing, True, front.positions_q)
+        ops.rope_rows(d_k[:, None, :64], d_k[:, None, :64], front.cos, front.sin, pairing, pairing, True)
+        x = k_in.float().requires_grad_(True)
+        lw, lb = ln_w.clone().requires_grad_(True), torch.zeros(128, device=gpu, requires_grad=True)
+        d_k, *ref_ln = torch.autograd.grad(torch.nn.functional.layer_norm(x, (128,), lw, lb, 1e-5), [x, lw, lb], d_k.float())
+    want = [d_q[:, :heads, :dim].to(types[0]), d_k[:, :dim].to(types[1]), d_w[:, :heads].to(types[2])] + ref_ln
+    for a, b, t in zip(got, want, types + [torch.float32] * 2):
+        if b is None:
+            assert a is None
+            continue
+        assert a.shape == b.shape and a.dtype == b.dtype
+        # the same values up to the order of fp32 sums, i.e. now and then one step of the output's grid (or of the bf16
+        # grid that the rotary part works on)
+        scale = b.float().abs().max().item()
+        step = {torch.float32: 2e-6, torch.float16: 2e-3, torch.bfloat16: 8e-3}[t]
+        err = (a.float() - b.float()).abs()
+        assert torch.isfinite(a.float()).all()
+        if front is not None:
+            assert (err <= 8e-3 * b.float().abs() + 8e-3 * scale).all() and err.mean() <= 2e-4 * scale
+        else:
+            assert (err <= step * b.float().abs() + 2e-6 * scale).all()
