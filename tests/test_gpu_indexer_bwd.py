@@ -178,3 +178,35 @@ def test_indexer_grads_equal_the_separate_steps(gpu, S, Sk, heads, dim, K, rotat
             assert (err <= 8e-3 * b.float().abs() + 8e-3 * scale).all() and err.mean() <= 2e-4 * scale
         else:
             assert (err <= step * b.float().abs() + 2e-6 * scale).all()
+
+
+@pytest.mark.parametrize("S,Sk,K", [(1, 40000, 128), (70, 16385, 128), (33, 33000, 2048), (300, 16384, 2304)])
+def test_key_sums_over_many_keys(gpu, S, Sk, K):
+    """More keys than the order's lookup table holds at a time, and slot lists above and below the kernel's ring sizes."""
+    from loongforge_amd import ops
+
+    gen = torch.Generator().manual_seed(S)
+    q8 = torch.randn(S, 32, 128, generator=gen).to(torch.float8_e4m3fn)
+    k8 = torch.randn(Sk, 128, generator=gen).to(torch.float8_e4m3fn)
+    ksc, w, g = torch.rand(Sk, generator=gen) + 0.5, torch.randn(S, 32, generator=gen), torch.randn(S, K, generator=gen)
+    ids = torch.stack([torch.randperm(Sk, generator=gen)[:K] for _ in range(S)]).int()
+    ids[:, K // 2:][torch.rand(S, K - K // 2, generator=gen) < 0.3] = -1
+    for i in range(S):       # no gate within accumulation noise of zero
+        q, k = q8[i].double(), k8[ids[i].clamp(min=0).long()].double()
+        g[i, ((q @ k.T).abs() <= 2.0 ** -16 * (q.abs() @ k.abs().T)).any(0)] = 0.0
+    dq, dk, dw = ops.indexer_bwd(*(t.to(gpu) for t in (g, q8, k8, ksc, w, ids)))
+    rq, rk, rw = torch.zeros(S, 32, 128, dtype=torch.float64), torch.zeros(Sk, 128, dtype=torch.float64), torch.zeros(S, 32, dtype=torch.float64)
+    rk_abs = torch.zeros(Sk, dtype=torch.float64)
+    for i in range(S):
+        live = ids[i] >= 0
+        j = ids[i][live].long()
+        q, k = q8[i].double(), k8[j].double()
+        r = q @ k.T
+        a = (g[i][live] * ksc[j]).double()
+        e = w[i].double()[:, None] * a * (r > 0)
+        rq[i], rw[i] = e @ k, (r.clamp(min=0) * a).sum(1)
+        rk[j] += e.T @ q
+        rk_abs[j] += (e.T @ q).abs().amax(1)
+    assert (dq.cpu() - rq).abs().max() <= 1e-4 * rq.abs().max() and (dw.cpu() - rw).abs().max() <= 1e-4 * rw.abs().max()
+    # pair rows are bf16, from head factors w q in bf16
+    assert ((dk.cpu() - rk).abs() <= 2e-2 * rk_abs[:, None] + 1e-3).all()
