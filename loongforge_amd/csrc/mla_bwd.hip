@@ -22,8 +22,11 @@
 namespace {
 using namespace mla;
 
-constexpr int PDS_TILE_BYTES = 16384;        // P and dS of one (query, tile): 2 x [16 chunk groups][32 keys][8 heads] bf16
-constexpr int PDS_KIND_BYTES = 8192;
+// P and dS of one (query, tile): 2 x [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes
+// are compiled for: 1 or 2, or 4 for 96 and 128 heads.
+constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
+constexpr int pds_tile_bytes(int HG) { return HG * 4096; }
+inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
 
@@ -39,16 +42,22 @@ constexpr int PDS_THREADS = 512;
 // SIMD) are then about level.  A lane ends with 4 heads x 2 half tiles; lanes 32 apart trade halves
 // (one v_permlane32_swap per register pair) so that every lane holds one key's 8 heads in the chunk
 // order pass C reads: chunk group 2w + g = heads 16w + {4g .. 4g+3, 8+4g .. 8+4g+3}.
-template <int STAGES>
+// With up to 64 heads four waves hold them all: waves 4-7 take every other tile (two tiles per step, STAGES = 4 tiles are then
+// two steps).  With up to 32 heads two waves do, and a wave takes one half tile of its tile only.  (Idle or repeated heads
+// cost as much as real ones: 3072 queries x 640 slots x 64 heads took 0.50 ms before.)
+template <int STAGES, int HG>
 __device__ __forceinline__ void pds_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, int q0, int ql, int H, int Skv, int K, int q_start, float sm_scale,
     unsigned char* smem) {
   constexpr int KS = DQK / 32, VS = DV / 32;   // 18 and 16 steps of 32 d-values
+  constexpr int NKT = HG == 1 ? 1 : 2;         // half tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4;
+  const int hw = wave & (2 * HG - 1);          // heads 16 hw ..
+  const int kt0 = HG == 1 ? (wave >> 1) & 1 : 0;
   const int qi = q0 + ql;
   const int NT = K / BI;
   int* idx_s = (int*)(smem + STAGES * TILE_BYTES);
@@ -58,7 +67,7 @@ __device__ __forceinline__ void pds_body(
   float* stat_s = (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
   // All of the query's rows are requested before the ids are staged: one round trip to memory for
   // both, instead of one after the other.
-  const int h = wave * 16 + m;
+  const int h = hw * 16 + m;
   const bool head_ok = h < H;
   const size_t hrow = (size_t)qi * H + (head_ok ? h : 0);
   bf16x8 qreg[KS], doreg[VS], oreg[VS];
@@ -96,22 +105,31 @@ __device__ __forceinline__ void pds_body(
   // Within a 128-byte group the 16-byte chunk c of key row r sits in slot c ^ (r & 7).  (The slot function of
   // the other kernels' tiles also serves their transposing reads; with it this kernel's reads - 16 rows x 4
   // chunks per instruction - take two LDS cycles where one is needed.)
-  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16) + (unsigned)(hh * 5 * 128);
+  // (two tiles per step: each half of the workgroup moves its own tile, all nine groups)
+  const int grp0 = HG == 4 ? hh * 5 : 0;
+  constexpr int NSTEP = HG == 4 ? 5 : 9;
+  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16) + (unsigned)(grp0 * 128);
   unsigned t_goff = 0, t_lb = 0;
   auto issue_prepare = [&](int n) {
     const int tile = tlist[n];
     int kid = idx_s[tile * BI + gkey];
     kid = kid < 0 ? 0 : kid;
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
-    t_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024 + hh * 5 * GRP_BYTES));
+    t_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024 + grp0 * GRP_BYTES));
   };
   auto issue_step = [&](int i) {
-    if (hh == 0 || i < 4) dma16(t_lb + i * GRP_BYTES, t_goff + i * 128, kv);
+    if (HG != 4 || hh == 0 || i < 4) dma16(t_lb + i * GRP_BYTES, t_goff + i * 128, kv);
   };
-  for (int n = 0; n < STAGES - 1 && n < ntiles; n++) {
-    issue_prepare(n);
+  if (HG == 4) {
+    for (int n = 0; n < STAGES - 1 && n < ntiles; n++) {
+      issue_prepare(n);
 #pragma unroll
-    for (int i = 0; i < 5; i++) issue_step(i);
+      for (int i = 0; i < NSTEP; i++) issue_step(i);
+    }
+  } else if (hh < ntiles) {
+    issue_prepare(hh);
+#pragma unroll
+    for (int i = 0; i < NSTEP; i++) issue_step(i);
   }
   // delta = rowsum(O . dO) while the first tiles travel
   {
@@ -128,29 +146,29 @@ __device__ __forceinline__ void pds_body(
     }
   }
   __syncthreads();
-  // accumulator i of a lane is head 16*wave + 4*kg + i, for key 16*kt + m
-  const f32x4 lse2 = *(const f32x4*)(stat_s + wave * 16 + 4 * kg);
-  const f32x4 delta = *(const f32x4*)(stat_s + 128 + wave * 16 + 4 * kg);
+  // accumulator i of a lane is head 16*hw + 4*kg + i, for key 16*kt + m
+  const f32x4 lse2 = *(const f32x4*)(stat_s + hw * 16 + 4 * kg);
+  const f32x4 delta = *(const f32x4*)(stat_s + 128 + hw * 16 + 4 * kg);
 
   // key-row operand of half tile kt and step ks: row 16*kt + m, 16-byte chunk 4*ks + kg of the row
-  unsigned boff[2][2];
+  unsigned boff[NKT][2];
 #pragma unroll
-  for (int kt = 0; kt < 2; kt++)
+  for (int kt = 0; kt < NKT; kt++)
 #pragma unroll
     for (int par = 0; par < 2; par++) {
-      const int row = 16 * kt + m;
+      const int row = 16 * (kt0 + kt) + m;
       boff[kt][par] = (unsigned)(row * 128 + (((4 * par + kg) ^ (row & 7)) << 4));
     }
   const float c2 = sm_scale * LOG2E;
 
-  f32x4 sacc[2], dpacc[2];
+  f32x4 sacc[NKT], dpacc[NKT];
   // P and dS of the accumulated tile: the lane's 4 heads for its key of either half tile are two
   // registers (4 bf16) each
   auto finish = [&](int tile, unsigned mask) {
-    unsigned pw[2][2], dw[2][2];
+    unsigned pw[NKT][2], dw[NKT][2];
 #pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      const bool valid = (mask >> (16 * kt + m)) & 1u;
+    for (int kt = 0; kt < NKT; kt++) {
+      const bool valid = (mask >> (16 * (kt0 + kt) + m)) & 1u;
       float pf[4], df[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -160,18 +178,53 @@ __device__ __forceinline__ void pds_body(
       pw[kt][0] = cvt_pk_bf16(pf[0], pf[1]); pw[kt][1] = cvt_pk_bf16(pf[2], pf[3]);
       dw[kt][0] = cvt_pk_bf16(df[0], df[1]); dw[kt][1] = cvt_pk_bf16(df[2], df[3]);
     }
-    // lanes 32 apart trade: the lower lane keeps half tile 0 and gets the partner's heads of it, the
-    // upper lane keeps half tile 1.  Afterwards (x[0], x[1]) is the chunk of key 16*(lane/32) + m:
-    // heads 4g .. 4g+3 then 8+4g .. 8+4g+3 of the wave's 16, g = kg & 1.
+    unsigned char* base = pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG);
+    if constexpr (NKT == 1) {
+      // half a chunk per lane: heads 4 kg .. of its key
+      base += (size_t)(2 * hw + (kg & 1)) * 512 + (16 * kt0 + m) * 16 + (kg >> 1) * 8;
+      *(uint2*)base = make_uint2(dw[0][0], dw[0][1]);
+      *(uint2*)(base + pds_kind_bytes(HG)) = make_uint2(pw[0][0], pw[0][1]);
+    } else {
+      // lanes 32 apart trade: the lower lane keeps half tile 0 and gets the partner's heads of it, the
+      // upper lane keeps half tile 1.  Afterwards (x[0], x[1]) is the chunk of key 16*(lane/32) + m:
+      // heads 4g .. 4g+3 then 8+4g .. 8+4g+3 of the wave's 16, g = kg & 1.
 #pragma unroll
-    for (int r2 = 0; r2 < 2; r2++) {
-      swap_halves(pw[0][r2], pw[1][r2]);
-      swap_halves(dw[0][r2], dw[1][r2]);
+      for (int r2 = 0; r2 < 2; r2++) {
+        swap_halves(pw[0][r2], pw[1][r2]);
+        swap_halves(dw[0][r2], dw[1][r2]);
+      }
+      const int key = 16 * (lane >> 5) + m, g = kg & 1;
+      base += (size_t)(2 * hw + g) * 512 + key * 16;
+      *(uint4*)base = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
+      *(uint4*)(base + pds_kind_bytes(HG)) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
     }
-    const int key = 16 * (lane >> 5) + m, g = kg & 1;
-    unsigned char* base = pds + ((size_t)ql * NT + tile) * PDS_TILE_BYTES + (size_t)(2 * wave + g) * 512 + key * 16;
-    *(uint4*)base = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
-    *(uint4*)(base + PDS_KIND_BYTES) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
+  };
+  // S and dP of a tile in LDS; `more`: with the transfers of a later tile between the products
+  auto products = [&](const unsigned char* tb, bool more) {
+#pragma unroll
+    for (int kt = 0; kt < NKT; kt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) { sacc[kt][e] = 0.f; dpacc[kt][e] = 0.f; }
+    // step j = NKT * ks + kt; FD operand reads in flight
+    constexpr int FD = 4;
+    bf16x8 f[FD];
+    auto operand = [&](int j) {
+      const int ks = j / NKT, kt = j % NKT;
+      return *(const bf16x8*)(tb + (ks >> 1) * GRP_BYTES + boff[kt][ks & 1]);
+    };
+#pragma unroll
+    for (int j = 0; j < FD; j++) f[j] = operand(j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NKT * KS; j++) {
+      const int ks = j / NKT, kt = j % NKT;
+      sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[ks], f[j % FD], sacc[kt], 0, 0, 0);
+      if (ks < VS) dpacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(doreg[ks], f[j % FD], dpacc[kt], 0, 0, 0);
+      if (j + FD < NKT * KS) f[j % FD] = operand(j + FD);
+      constexpr int EVERY = HG == 4 ? 7 : NKT * KS / NSTEP, AT = HG == 1 ? 1 : 2;
+      if (j % EVERY == AT && more) issue_step(j / EVERY);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
 
   // Between two barriers every wave runs the MFMAs of one tile and one `finish`; waves 0-3 finish the
@@ -179,6 +232,28 @@ __device__ __forceinline__ void pds_body(
   // w + 4) are thus half a step apart: the arithmetic and stores of one run under the other's MFMAs.
   int tile = 0;
   unsigned mask = 0;
+  if constexpr (HG != 4) {
+    // two tiles per step, one per half of the workgroup; the next step's are in flight
+    for (int i = 0; 2 * i < ntiles; i++) {
+      const int n = 2 * i + hh;
+      // behind the tile's transfers: the two stores of the step before (waves 0-3), nothing (waves 4-7)
+      if (hh == 0 && i > 0) { DSA_WAIT_VMCNT(2); } else { DSA_WAIT_VMCNT(0); }
+      __syncthreads();
+      if (hh == 1 && i > 0) finish(tile, mask);
+      if (n < ntiles) {
+        const bool more = n + 2 < ntiles;
+        if (more) issue_prepare(n + 2);
+        tile = __builtin_amdgcn_readfirstlane(tlist[n]);
+        mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+        __builtin_amdgcn_sched_barrier(0);
+        products(smem + (n % STAGES) * TILE_BYTES, more);
+        if (hh == 0) finish(tile, mask);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (hh == 1 && ntiles > 1 && (ntiles & 1) == 0) finish(tile, mask);      // (odd counts: done in the last step)
+    return;
+  }
   for (int n = 0; n < ntiles; n++) {
     // operations a lane issued after this tile's transfers: D per later tile in flight (5 in waves
     // 0-3, 4 in waves 4-7), 2 stores per finished tile (waves 4-7 are one tile behind with those)
@@ -211,31 +286,7 @@ __device__ __forceinline__ void pds_body(
     mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
     if (hh == 1 && n > 0) finish(prev_tile, prev_mask);
     __builtin_amdgcn_sched_barrier(0);
-    const unsigned char* tb = smem + (n % STAGES) * TILE_BYTES;
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) { sacc[kt][e] = 0.f; dpacc[kt][e] = 0.f; }
-    {
-      // step j = 2 * ks + kt; FD operand reads in flight
-      constexpr int FD = 4;
-      bf16x8 f[FD];
-#pragma unroll
-      for (int j = 0; j < FD; j++) f[j] = *(const bf16x8*)(tb + ((j >> 1) >> 1) * GRP_BYTES + boff[j & 1][(j >> 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 2 * KS; j++) {
-        const int ks = j >> 1, kt = j & 1;
-        sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[ks], f[j % FD], sacc[kt], 0, 0, 0);
-        if (ks < VS) dpacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(doreg[ks], f[j % FD], dpacc[kt], 0, 0, 0);
-        if (j + FD < 2 * KS) {
-          const int j2 = j + FD, ks2 = j2 >> 1;
-          f[j % FD] = *(const bf16x8*)(tb + (ks2 >> 1) * GRP_BYTES + boff[j2 & 1][ks2 & 1]);
-        }
-        if (j % 7 == 2 && more) issue_step(j / 7);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+    products(smem + (n % STAGES) * TILE_BYTES, more);
     if (hh == 0) finish(tile, mask);
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -255,13 +306,17 @@ __device__ __forceinline__ void pds_body(
 // the two waves of a SIMD together (1 200 against 1 152 cycles per tile).  Three waves per SIMD at
 // under 168 registers per lane issue them in two thirds of the time, and one wave's transfer issue and
 // waits run under the MFMAs of the other two.
+// With up to 64 heads a wave owns its 3 d-tiles for head group hp only; with up to 32, for one k-step (16 keys) of the only
+// head group, and the two k-steps' sums are added at the end.
 constexpr int DQ_THREADS = 768;
-template <int STAGES>
+template <int STAGES, int HG>
 __device__ __forceinline__ void dq_body(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
     __bf16* __restrict__ dq, int q0, int ql, int H, int Skv, int K, int q_start, const int* __restrict__ dup_flag,
     unsigned char* smem) {
-  constexpr int STAGE_BYTES = TILE_BYTES + PDS_KIND_BYTES;
+  constexpr int STAGE_BYTES = TILE_BYTES + pds_kind_bytes(HG);
+  constexpr int NJ = HG == 4 ? 2 : 1;          // head groups of a wave
+  constexpr int DS_WAVES = 2 * HG;             // waves that move 1 KB of the dS block each
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dg = wave % 6, hp = wave / 6;
@@ -305,7 +360,7 @@ __device__ __forceinline__ void dq_body(
   // block, piece P of the LDS order coming from piece src_piece(P) of the HBM order.  Wave v takes
   // transfers v, v + 12, v + 24 (groups v/4, v/4 + 3, v/4 + 6 of its slot v % 4) and, for v < 8, 36 + v.
   auto src_piece = [](int P) { return (P >> 7) * 128 + ((P >> 1) & 1) * 64 + (P & 1) * 32 + ((P >> 2) & 31); };
-  const unsigned ds_src = (unsigned)src_piece((wave & 7) * 64 + lane) * 16u;
+  const unsigned ds_src = (unsigned)src_piece((wave & (DS_WAVES - 1)) * 64 + lane) * 16u;
   const int gkey = 8 * (wave & 3) + (lane >> 3), gsub = lane & 7;
   const unsigned gslot = (unsigned)((gsub ^ swz(gkey)) * 16) + (unsigned)((wave >> 2) * 128);
   unsigned t_goff = 0, t_lb = 0, t_lbd = 0;
@@ -317,19 +372,21 @@ __device__ __forceinline__ void dq_body(
     kid = kid < 0 ? 0 : kid;
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
     t_lb = __builtin_amdgcn_readfirstlane(sb + (unsigned)((wave & 3) * 1024 + (wave >> 2) * GRP_BYTES));
-    t_lbd = __builtin_amdgcn_readfirstlane(sb + (unsigned)(TILE_BYTES + (wave & 7) * 1024));
-    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * PDS_TILE_BYTES);     // dS half
+    t_lbd = __builtin_amdgcn_readfirstlane(sb + (unsigned)(TILE_BYTES + (wave & (DS_WAVES - 1)) * 1024));
+    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG));     // dS half
   };
-  // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0-7)
+  // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0 .. DS_WAVES - 1)
   auto issue_step = [&](int j) {
     if (j < 3) dma16(t_lb + 3 * j * GRP_BYTES, t_goff + 3 * j * 128, kv);
-    else if (wave < 8) dma16(t_lbd, ds_src, t_src);
+    else if (wave < DS_WAVES) dma16(t_lbd, ds_src, t_src);
   };
 
-  const int hg0 = 2 * hp, hg1 = 2 * hp + 1;
-  f32x16 acc[6];      // u = 2 * i + j: d-tile 3dg + i, head group 2hp + j
+  const int hg0 = HG == 4 ? 2 * hp : HG == 2 ? hp : 0;
+  const int s0 = HG == 1 ? hp : 0;
+  constexpr int NS = HG == 1 ? 1 : 2;          // k-steps of a wave
+  f32x16 acc[3 * NJ];      // u = NJ * i + j: d-tile 3dg + i, head group hg0 + j
 #pragma unroll
-  for (int u = 0; u < 6; u++)
+  for (int u = 0; u < 3 * NJ; u++)
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[u][e] = 0.f;
   typedef short i16x8 __attribute__((ext_vector_type(8)));
@@ -345,44 +402,70 @@ __device__ __forceinline__ void dq_body(
   }
   for (int n = 0; n < ntiles; n++) {
     static_assert(STAGES == 3, "one tile of transfers in flight behind the awaited one");
-    // transfers per wave and tile: 4 for waves 0-7, 3 for waves 8-11
-    if (n + 1 < ntiles) { if (wave < 8) { DSA_WAIT_VMCNT(4); } else { DSA_WAIT_VMCNT(3); } } else { DSA_WAIT_VMCNT(0); }
+    // transfers per wave and tile: 4 for waves 0 .. DS_WAVES - 1, 3 for the others
+    if (n + 1 < ntiles) { if (wave < DS_WAVES) { DSA_WAIT_VMCNT(4); } else { DSA_WAIT_VMCNT(3); } } else { DSA_WAIT_VMCNT(0); }
     __syncthreads();
     const bool more = n + STAGES - 1 < ntiles;
     if (more) { issue_prepare(n + STAGES - 1); issue_step(3); }
     const unsigned char* tb = smem + (n % STAGES) * STAGE_BYTES;
-    // key-tile operands one d-tile ahead, the four dS operands of the wave's two head groups: [hg0 or hg1][k-step]
-    bf16x8 a[2][2], bds[2][2];
+    // key-tile operands one d-tile ahead, the dS operands of the wave's head groups: [head group][k-step]
+    bf16x8 a[2][NS], bds[NJ][NS];
+    auto key_operand = [&](int i, int s) {
+      return HG == 1 ? tr_pair(tb + (hp ? a_off[i][1][0] : a_off[i][0][0]), tb + (hp ? a_off[i][1][1] : a_off[i][0][1]))
+                     : tr_pair(tb + a_off[i][s][0], tb + a_off[i][s][1]);
+    };
 #pragma unroll
-    for (int s = 0; s < 2; s++) a[0][s] = tr_pair(tb + a_off[0][s][0], tb + a_off[0][s][1]);
+    for (int s = 0; s < NS; s++) a[0][s] = key_operand(0, s);
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
-      for (int s = 0; s < 2; s++)
-        bds[j][s] = tr_pair(tb + (j ? hg1 : hg0) * 2048 + ds_off[s][0], tb + (j ? hg1 : hg0) * 2048 + ds_off[s][1]);
+      for (int s = 0; s < NS; s++) {
+        const unsigned o0 = HG == 1 ? (s0 ? ds_off[1][0] : ds_off[0][0]) : ds_off[s][0];
+        const unsigned o1 = HG == 1 ? (s0 ? ds_off[1][1] : ds_off[0][1]) : ds_off[s][1];
+        bds[j][s] = tr_pair(tb + (hg0 + j) * 2048 + o0, tb + (hg0 + j) * 2048 + o1);
+      }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 3; i++) {
       if (i + 1 < 3) {
 #pragma unroll
-        for (int s = 0; s < 2; s++) a[(i + 1) & 1][s] = tr_pair(tb + a_off[i + 1][s][0], tb + a_off[i + 1][s][1]);
+        for (int s = 0; s < NS; s++) a[(i + 1) & 1][s] = key_operand(i + 1, s);
       }
 #pragma unroll
-      for (int s = 0; s < 2; s++)
+      for (int s = 0; s < NS; s++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-          acc[2 * i + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i & 1][s], bds[j][s], acc[2 * i + j], 0, 0, 0);
+        for (int j = 0; j < NJ; j++)
+          acc[NJ * i + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i & 1][s], bds[j][s], acc[NJ * i + j], 0, 0, 0);
       if (more) issue_step(i);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (HG == 1) {       // the second k-step's sums join the first one's
+    __syncthreads();
+    f32x4* box = (f32x4*)smem + (size_t)(dg * 12) * 64 + lane;
+    if (hp == 1) {
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) box[(4 * i + j) * 64] = f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
+    }
+    __syncthreads();
+    if (hp == 1) return;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const f32x4 v = box[(4 * i + j) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[i][4 * j + e] += v[e];
+      }
+  }
   // ---- write dQ: accumulator e of a lane is d = 32*dt + 8*(e/4) + 4*g + (e%4), head = 32*hg + r ----
   const bool poison = *dup_flag != 0;          // a query row with a repeated id: NaN instead of a sum that misses a term
 #pragma unroll
-  for (int u = 0; u < 6; u++) {
-    const int dt = 3 * dg + (u >> 1);
-    const int hg = (u & 1) ? hg1 : hg0;
-    const int h = hg * 32 + r;
+  for (int u = 0; u < 3 * NJ; u++) {
+    const int dt = 3 * dg + u / NJ;
+    const int h = (hg0 + u % NJ) * 32 + r;
     if (h < H) {                               // the same for all lanes of a wave (H is a multiple of 32)
       unsigned short* op = (unsigned short*)dq + ((size_t)qi * H + h) * DQK + 32 * dt + 8 * g;
       uint4 o[2];
@@ -421,14 +504,14 @@ __device__ __forceinline__ void dkv_body(
     int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
   constexpr int CST = DKV_COEF_STAGES;
   constexpr int NU = NC == 5 ? 9 : 8;          // units of 8 MFMAs per tile
-  // [CST][PDS_TILE_BYTES] coefficient ring, shared with the set-up's per-wave X staging [4][8192] |
+  // [CST][pds_tile_bytes(4)] coefficient ring, shared with the set-up's per-wave X staging [4][8192] |
   // ids arrays | dst rows of the query [K + 32]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, g = lane >> 5;
   const int qi = q0 + ql;
   const int NT = K / BI;
   unsigned char* xs = smem + wave * 8192;
-  int* idx_s = (int*)(smem + CST * PDS_TILE_BYTES);
+  int* idx_s = (int*)(smem + CST * pds_tile_bytes(4));
   unsigned* tmask = (unsigned*)(idx_s + K);
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
@@ -506,8 +589,8 @@ __device__ __forceinline__ void dkv_body(
 
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   auto issue = [&](int n) {
-    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % CST) * PDS_TILE_BYTES + wave * 1024));
-    const unsigned char* src = uniform_ptr(pds + ((size_t)ql * NT + tlist[n]) * PDS_TILE_BYTES);
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % CST) * pds_tile_bytes(4) + wave * 1024));
+    const unsigned char* src = uniform_ptr(pds + ((size_t)ql * NT + tlist[n]) * pds_tile_bytes(4));
 #pragma unroll
     for (int c = 0; c < 4; c++) dma16(lb + c * 4096, (unsigned)(c * 4096 + tid * 16), src);
   };
@@ -575,7 +658,7 @@ __device__ __forceinline__ void dkv_body(
   for (int n = 0; n < ntiles; n++) {
     const int tile = tlist[n];
     const int drow = dst_s[tile * BI + r];
-    const unsigned char* nb = smem + ((n + 1) % CST) * PDS_TILE_BYTES;   // next tile's coefficients
+    const unsigned char* nb = smem + ((n + 1) % CST) * pds_tile_bytes(4);   // next tile's coefficients
 #pragma unroll
     for (int u = 0; u < NU; u++) {
       const int ci = u < 8 ? u >> 1 : 4, half = u < 8 ? (u & 1) : 0;
@@ -630,6 +713,128 @@ __device__ __forceinline__ void dkv_body(
   piece_store(NC - 1, 1);
 }
 
+// The same with up to 64 heads (HG = 1, 2): the operands of a query take 72 or 144 registers, two workgroups share a compute
+// unit and hide each other's set-up, barriers and stores, and the products are plain builtins in the compiler's order.  Bound by
+// the rows: 2.26 GB for 3072 queries x 640 slots.
+constexpr int DKV_FEW_STAGES = 4;
+template <int NC, int HG>
+__device__ __forceinline__ void dkv_few_body(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
+    const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
+  constexpr int CST = DKV_FEW_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
+  // [CST][TB] coefficient ring, shared with the set-up's per-wave X staging [4][HG * 2048] | ids arrays | dst rows [K]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, g = lane >> 5;
+  const int qi = q0 + ql;
+  const int NT = K / BI;
+  unsigned char* xs = smem + wave * (HG * 2048);
+  int* idx_s = (int*)(smem + CST * TB);
+  unsigned* tmask = (unsigned*)(idx_s + K);
+  int* tlist = (int*)(tmask + NT);
+  int* ntile_s = tlist + NT;
+  int* dst_s = ntile_s + 4;
+  for (int t0 = tid; t0 < K; t0 += 8 * 256) {        // eight loads in flight per thread
+    int d[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) d[i] = t0 + i * 256 < K ? dst[(size_t)ql * K + t0 + i * 256] : -1;
+#pragma unroll
+    for (int i = 0; i < 8; i++)       // invalid slots land in a scratch row: the store count stays fixed
+      if (t0 + i * 256 < K) dst_s[t0 + i * 256] = d[i] >= 0 ? d[i] : dummy_row;
+  }
+  // X^T operands, k-step kk = 16 heads: column tiles wave + 4 c of Q (c < NC) and of dO (c < 4)
+  bf16x8 xq[NC][M], xo[4][M];
+  {
+    typedef short i16x8 __attribute__((ext_vector_type(8)));
+    const int blk = lane >> 4, ii = lane & 15;
+    const unsigned xoff = (unsigned)((4 * g + (ii >> 2)) * 64 + (16 * (blk & 1) + 4 * (ii & 3)) * 2);
+    constexpr int NP = NC + 4;
+    uint4 ld[3][M];                            // three passes of global loads in flight
+    auto pass_load = [&](int pass, uint4 (&v)[M]) {
+      const bool isq = pass < NC;
+      const int c = wave + 4 * (isq ? pass : pass - NC);
+      const __bf16* src = isq ? q + (size_t)qi * H * DQK + 32 * c : dout + (size_t)qi * H * DV + 32 * c;
+      const int stride = isq ? DQK : DV;
+#pragma unroll
+      for (int it = 0; it < M; it++)           // rows of 64 bytes: lane covers head lane/4 + 16*it, 16-byte piece lane%4
+        v[it] = *(const uint4*)(src + (size_t)((lane >> 2) + 16 * it) * stride + (lane & 3) * 8);
+    };
+    pass_load(0, ld[0]);
+    pass_load(1, ld[1]);
+    pass_load(2, ld[2]);
+#pragma unroll
+    for (int pass = 0; pass < NP; pass++) {
+#pragma unroll
+      for (int it = 0; it < M; it++) *(uint4*)(xs + ((lane >> 2) + 16 * it) * 64 + (lane & 3) * 16) = ld[pass % 3][it];
+      if (pass + 3 < NP) pass_load(pass + 3, ld[pass % 3]);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int kk = 0; kk < M; kk++) {
+        const unsigned char* hb = xs + 16 * kk * 64;
+        const i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + xoff));
+        const i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + 8 * 64 + xoff));
+        const bf16x8 val = __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+        if (pass < NC) xq[pass < NC ? pass : 0][kk] = val;
+        else xo[pass < NC ? 0 : pass - NC][kk] = val;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  // (its barriers also part the X staging from the coefficient ring, which shares LDS with it)
+  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  if (ntiles == 0) return;
+
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  auto issue = [&](int n) {
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % CST) * TB + wave * 1024));
+    const unsigned char* src = uniform_ptr(pds + ((size_t)ql * NT + tlist[n]) * TB);
+#pragma unroll
+    for (int c = 0; c < HG; c++) dma16(lb + c * 4096, (unsigned)(c * 4096 + tid * 16), src);
+  };
+  for (int n = 0; n < CST && n < ntiles; n++) issue(n);
+  const unsigned coff = (unsigned)(g * 512 + r * 16);      // coefficient chunk of k-step kk: [kind][kk][g][key r] 16 bytes
+  bf16x8 cf[2][M];
+  auto read_coefs = [&](int n) {
+    const unsigned char* tb = smem + (n % CST) * TB;
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int kk = 0; kk < M; kk++) cf[k][kk] = *(const bf16x8*)(tb + k * pds_kind_bytes(HG) + kk * 1024 + coff);
+  };
+  DSA_WAIT_VMCNT(0);
+  __syncthreads();
+  read_coefs(0);
+  for (int n = 0; n < ntiles; n++) {
+    unsigned char* rptr = rows + (size_t)dst_s[tlist[n] * BI + r] * ROW_BYTES + wave * 64 + g * 16;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      f32x16 acc;
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < M; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xq[c][kk], cf[0][kk], acc, 0, 0, 0);
+      if (c < 4) {
+#pragma unroll
+        for (int kk = 0; kk < M; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xo[c < 4 ? c : 0][kk], cf[1][kk], acc, 0, 0, 0);
+      }
+      uint4 o[2];
+      acc_row_to_16B(acc, 1.0f, o);
+      *(uint4*)(rptr + c * 256) = o[0];
+      *(uint4*)(rptr + c * 256 + 32) = o[1];
+    }
+    if (n + 1 < ntiles) {
+      // issued behind the next tile's transfers: HG per later tile in flight, 2 NC stores per tile since
+      if (n >= CST - 1 && n + CST - 1 < ntiles) { DSA_WAIT_VMCNT((CST - 2) * HG + (CST - 1) * 2 * NC); }
+      else if (n >= CST - 1) { DSA_WAIT_VMCNT((CST - 1) * 2 * NC); }
+      else { DSA_WAIT_VMCNT(2 * NC); }
+      __syncthreads();
+      if (n + CST < ntiles) issue(n + CST);    // into the slot of tile n, whose coefficients are in registers
+      read_coefs(n + 1);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // pass D: dKV[key] = sum of that key's rows, ascending query order
 // ---------------------------------------------------------------------------------------------
@@ -654,8 +859,8 @@ constexpr int RED_KEYS = 4;                  // consecutive keys per workgroup
 // exposed once a key has few rows per launch: with the queries of 32768 tokens walked in four chunks the launch
 // took 27.1 ms against 18.9 ms for one sweep; per key the sums and their order are the same as before.)
 __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ rows, const int* __restrict__ start,
-                                            float* __restrict__ dkv_acc, int key0, int n_keys, int accumulate,
-                                            unsigned char* smem) {
+                                            float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int key0, int n_keys,
+                                            int accumulate, const int* __restrict__ dup_flag, unsigned char* smem) {
   float* part = (float*)smem;                  // [RED_KEYS][RED_GROUPS][DQK]
   const int tid = threadIdx.x;
   const int ch = tid % 72, grp = tid / 72;
@@ -705,8 +910,12 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
     float sum = part[k * RED_GROUPS * DQK + d];
 #pragma unroll
     for (int gq = 1; gq < RED_GROUPS; gq++) sum += part[(k * RED_GROUPS + gq) * DQK + d];
-    float* p = dkv_acc + (size_t)(key0 + k) * DQK + d;
-    *p = accumulate ? *p + sum : sum;
+    if (dkv) {       // one sweep over all queries: the sum is complete (NaN everywhere when a query row held a repeated id)
+      dkv[(size_t)(key0 + k) * DQK + d] = *dup_flag ? (unsigned short)0x7fc0 : f32_to_bf16_bits(sum);
+    } else {
+      float* p = dkv_acc + (size_t)(key0 + k) * DQK + d;
+      *p = accumulate ? *p + sum : sum;
+    }
   }
 }
 
@@ -735,15 +944,17 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
+template <int HG>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  pds_body<4>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
+  pds_body<4, HG>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
 }
 
-__global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
+template <int HG>
+__global__ __launch_bounds__(256, HG == 4 ? 1 : 2) void bwd_dkv_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
     const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int cnt, int H, int Skv, int K, int q_start, int dummy_row) {
@@ -751,19 +962,25 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
   const int ql = cnt - 1 - (int)blockIdx.x;
   // waves 0 and 1 own five column tiles, waves 2 and 3 four: two copies of the whole body, so that
   // no branch sits between the MFMAs; every copy meets the same barriers
-  if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-  else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+  if constexpr (HG == 4) {
+    if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+    else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+  } else {
+    if (threadIdx.x < 128) dkv_few_body<5, HG>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+    else dkv_few_body<4, HG>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+  }
 }
 
+template <int HG>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
     __bf16* __restrict__ dq, int q0, int cnt, int H, int Skv, int K, int q_start, const int* __restrict__ dup_flag,
-    const unsigned char* __restrict__ rows, const int* __restrict__ start, float* __restrict__ dkv_acc, int n_keys,
-    int accumulate) {
+    const unsigned char* __restrict__ rows, const int* __restrict__ start, float* __restrict__ dkv_acc,
+    unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
-  if (rs.first) dq_body<3>(kv, ids, pds, dq, q0, cnt - 1 - rs.i, H, Skv, K, q_start, dup_flag, smem);
-  else reduce_body(rows, start, dkv_acc, rs.i * RED_KEYS, n_keys, accumulate, smem);
+  if (rs.first) dq_body<3, HG>(kv, ids, pds, dq, q0, cnt - 1 - rs.i, H, Skv, K, q_start, dup_flag, smem);
+  else reduce_body(rows, start, dkv_acc, dkv, rs.i * RED_KEYS, n_keys, accumulate, dup_flag, smem);
 }
 
 // fp32 accumulator -> bf16 dKV; NaN everywhere when a query row held a repeated id
@@ -792,7 +1009,7 @@ struct BwdPlan {
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-BwdPlan layout_plan(int chunk, int Skv, int K) {
+BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
   BwdPlan p;
   p.chunk = chunk;
   p.W = (chunk + 31) / 32;
@@ -804,7 +1021,7 @@ BwdPlan layout_plan(int chunk, int Skv, int K) {
   p.off_flag = o; o = align_up(o + 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
-  p.off_pds = o; o = align_up(o + (size_t)chunk * (K / BI) * PDS_TILE_BYTES);
+  p.off_pds = o; o = align_up(o + (size_t)chunk * (K / BI) * pds_tile_bytes(head_groups(H)));
   p.off_rows = o; o = align_up(o + ((size_t)chunk * K + 1) * ROW_BYTES);
   p.off_acc = o; o = align_up(o + (size_t)Skv * DQK * 4);
   p.total = o;
@@ -813,12 +1030,12 @@ BwdPlan layout_plan(int chunk, int Skv, int K) {
 
 // Largest chunk of queries (all of them if possible, else repeated halving, at least 64) whose
 // buffers fit the budget.
-BwdPlan make_plan(int S, int Skv, int K, size_t budget) {
+BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
   int chunk = S;
-  BwdPlan p = layout_plan(chunk, Skv, K);
+  BwdPlan p = layout_plan(chunk, H, Skv, K);
   while (p.total > budget && chunk > 64) {
     chunk = (chunk + 1) / 2;
-    p = layout_plan(chunk, Skv, K);
+    p = layout_plan(chunk, H, Skv, K);
   }
   return p;
 }
@@ -828,15 +1045,13 @@ constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;
 }  // namespace
 
 extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes(int S, int H, int Skv, int K) {
-  (void)H;
   if (S <= 0 || Skv <= 0 || K <= 0) return 0;
-  return make_plan(S, Skv, K, DEFAULT_BUDGET).total;
+  return make_plan(S, H, Skv, K, DEFAULT_BUDGET).total;
 }
 
 extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes_min(int S, int H, int Skv, int K) {
-  (void)H;
   if (S <= 0 || Skv <= 0 || K <= 0) return 0;
-  return layout_plan(S < 64 ? S : 64, Skv, K).total;
+  return layout_plan(S < 64 ? S : 64, H, Skv, K).total;
 }
 
 static int bwd_impl(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
@@ -853,10 +1068,10 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
               "dsa_sparse_mla_bwd: misaligned pointer");
   hipStream_t st = (hipStream_t)stream;
   // choose the largest chunk the given workspace allows
-  BwdPlan p = make_plan(S > 0 ? S : 1, Skv, K, workspace_bytes);
+  BwdPlan p = make_plan(S > 0 ? S : 1, H, Skv, K, workspace_bytes);
   if (p.total > workspace_bytes || workspace == nullptr)
     DSA_FAIL(DSA_ERR_WORKSPACE, "dsa_sparse_mla_bwd: workspace of %zu bytes is too small (need at least %zu)",
-             workspace_bytes, make_plan(64, Skv, K, 1).total);
+             workspace_bytes, make_plan(64, H, Skv, K, 1).total);
   unsigned char* ws = (unsigned char*)workspace;
   unsigned* bitmap = (unsigned*)(ws + p.off_bitmap);
   unsigned* prefix = (unsigned*)(ws + p.off_prefix);
@@ -868,14 +1083,19 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   unsigned char* pds = ws + p.off_pds;
   unsigned char* rows = ws + p.off_rows;
   float* acc = (float*)(ws + p.off_acc);
-  const int NT = K / BI;
 
+  const int HG = head_groups(H);
   const size_t smemA = (size_t)4 * TILE_BYTES + ids_lds_bytes(K) + 16 + 1024;
-  const size_t smemB = (size_t)3 * (TILE_BYTES + PDS_KIND_BYTES) + ids_lds_bytes(K);
-  const size_t smemC = (size_t)DKV_COEF_STAGES * PDS_TILE_BYTES + ids_lds_bytes(K) + 16 + (size_t)(K + BI) * 4;
-  if (dsa_reserve_lds((const void*)bwd_pds_kernel, smemA) != hipSuccess ||
-      dsa_reserve_lds((const void*)bwd_dkv_kernel, smemC) != hipSuccess ||
-      dsa_reserve_lds((const void*)bwd_dq_reduce_kernel, smemB) != hipSuccess)
+  const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
+  size_t smemB = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
+  if (smemB < reduce_lds) smemB = reduce_lds;
+  const size_t smemC = (size_t)(HG == 4 ? DKV_COEF_STAGES : DKV_FEW_STAGES) * pds_tile_bytes(HG) + ids_lds_bytes(K) + 16 + (size_t)(K + BI) * 4;
+  auto pds_kernel = HG == 1 ? bwd_pds_kernel<1> : HG == 2 ? bwd_pds_kernel<2> : bwd_pds_kernel<4>;
+  auto dkv_kernel = HG == 1 ? bwd_dkv_kernel<1> : HG == 2 ? bwd_dkv_kernel<2> : bwd_dkv_kernel<4>;
+  auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
+  if (dsa_reserve_lds((const void*)pds_kernel, smemA) != hipSuccess ||
+      dsa_reserve_lds((const void*)dkv_kernel, smemC) != hipSuccess ||
+      dsa_reserve_lds((const void*)dq_reduce_kernel, smemB) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
 
   // optional timing (profiling entry point only): events between the launch groups
@@ -905,17 +1125,18 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
-    bwd_pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
+    pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
                                                        (const __bf16*)dout, lse, pds, q0, cnt, H, Skv, K, q_start, sm_scale);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS)");
     DSA_MARK(2);
-    bwd_dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
+    dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
                                                        H, Skv, K, q_start, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dKV rows)");
     DSA_MARK(3);
     // Pass B of every query beside pass D of every key.
-    bwd_dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smemB, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
-                                                                   K, q_start, dup_flag, rows, start, acc, Skv, first ? 0 : 1);
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smemB, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
+                                                                   K, q_start, dup_flag, rows, start, acc,
+                                                                   S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");
     DSA_MARK(4);
     if (pass_ms) {
@@ -927,11 +1148,10 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   if (S == 0) {
     order::zero_u32_kernel<<<dim3(256), dim3(256), 0, st>>>((unsigned*)acc, (size_t)Skv * DQK);
   }
-  cast_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>(acc, (unsigned short*)dkv, (size_t)Skv * DQK, dup_flag);
+  if (S == 0 || S > p.chunk) cast_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>(acc, (unsigned short*)dkv, (size_t)Skv * DQK, dup_flag);
   if (S > p.chunk)      // more than one chunk: the flag may have come up after earlier chunks wrote their dQ
     poison_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>((unsigned short*)dq, (size_t)S * H * DQK, dup_flag);
   DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(cast)");
-  (void)NT;
   if (pass_ms) for (int i = 0; i < 5; i++) hipEventDestroy(ev[i]);
 #undef DSA_MARK
   return DSA_OK;

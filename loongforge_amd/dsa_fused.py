@@ -503,8 +503,8 @@ class DSAttentionFused(MegatronModule):
         self.sparse_attention = build_module(DSADotProductAttention, config=self.config,
                                              softmax_scale=self.softmax_scale)
         self.attn_sink = None
-        _DSA_MIN_HEAD_DIM = 128  # head count the sparse attention kernel is tiled for
-        self.num_attention_heads_padded = max(config.num_attention_heads, _DSA_MIN_HEAD_DIM)
+        # the sparse attention kernels take any multiple of 32 heads (the reference's pads to 128)
+        self.num_attention_heads_padded = (config.num_attention_heads + 31) // 32 * 32
         self.num_attention_heads = config.num_attention_heads
 
     def forward(self, query, key, value, attention_mask, x, qr, attn_mask_type: AttnMaskType = None,

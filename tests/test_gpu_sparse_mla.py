@@ -184,6 +184,33 @@ def test_backward_against_oracle_and_deterministic(gpu, S, H, K, q_start, skv, s
     assert torch.equal(dq, dq2) and torch.equal(dkv, dkv2)          # bit-identical
 
 
+@pytest.mark.parametrize("H", [32, 64])
+@pytest.mark.parametrize("S,K,q_start,skv", [
+    (1, 64, 0, None),                 # one valid slot
+    (67, 64, 0, None),                # one and two tiles per query
+    (70, 320, 0, None),               # up to ten tiles: odd and even counts, more than the rings hold
+    (9, 2048, 3000, None),            # the longest lists
+])
+def test_backward_of_few_heads(gpu, H, S, K, q_start, skv):
+    """Up to 64 heads the passes share tiles, k-steps and compute units differently; one workspace sweep and several give the
+    sums of the oracle, and an empty row or a tile without valid slots adds nothing."""
+    from loongforge_amd import ops
+
+    inp = O.make_mla_inputs(S, H, K, seed=S + H, skv=skv, q_start=q_start)
+    inp.idx = inp.idx.clone()
+    inp.idx[:, 40:50] = -1
+    if S > 2:
+        inp.idx[2] = -1
+    q, kv, idx, do = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu)
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, q_start, inp.sm_scale)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, inp.sm_scale)
+    assert_mla_grads(dq, dkv, inp.q, inp.kv, inp.idx, inp.dout, q_start, inp.sm_scale, out=out, lse=lse)
+    dq2, dkv2 = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, inp.sm_scale)
+    assert torch.equal(dq, dq2) and torch.equal(dkv, dkv2)
+    if S > 2:
+        assert (dq[2] == 0).all()
+
+
 def test_backward_does_not_depend_on_the_slot_order(gpu):
     """The backward walks each query's ids in ascending key order whatever order they arrive in, so
     permuting the slots (independently per query) and scattering unused slots between the used ones
