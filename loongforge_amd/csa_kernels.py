@@ -164,10 +164,13 @@ class CSAIndexerKernelFunction(torch.autograd.Function):
         ctx.in_dtypes = (index_q.dtype, index_k.dtype, weights.dtype)
         ctx.save_for_backward(q_fp8, k_fp8, q_scale, k_scale, weight_scaled, global_ids)
         ctx.mark_non_differentiable(topk_indices)
+        ctx.set_materialize_grads(False)
         return index_score_topk, topk_indices
 
     @staticmethod
     def backward(ctx, grad_score, grad_topk):
+        if grad_score is None:
+            return (None,) * 7
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, global_ids = ctx.saved_tensors
         # padding slots (id -1) are constants of the forward: their upstream gradient (often NaN) is dropped by the kernel
         d_q, d_k, d_weights, _, _ = ops.indexer_grads(grad_score, q_fp8, k_fp8, k_scale, weight_scaled, global_ids, q_scale,

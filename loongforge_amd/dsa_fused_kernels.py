@@ -108,6 +108,7 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
             out, lse, p_out = ops.sparse_mla_fwd(q, kv2, ids, chunk_offset, sm_scale, d_v, return_p_out or dist_from_logits,
                                                  attn_sink=attn_sink, p_out_skip=window_size)
         ctx.save_for_backward(q, kv, ids, out, lse)
+        ctx.set_materialize_grads(False)      # no zeros for the outputs without a gradient
         ctx.sm_scale = sm_scale
         ctx.chunk_offset = chunk_offset
         ctx.d_v = d_v
@@ -129,6 +130,8 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out, grad_p_out=None):
+        if grad_out is None:
+            return (None,) * 13
         q, kv, ids, out, lse = ctx.saved_tensors
         grad_out = grad_out.squeeze(0).contiguous()
         kv2 = kv.reshape(kv.shape[0], kv.shape[-1])
@@ -294,10 +297,13 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
             ctx.front_saved = (k_p, k_norm_weight, k_norm_bias)
         ctx.save_for_backward(q_fp8, k_fp8, q_scale, k_scale, weight_scaled, topk_indices)
         ctx.mark_non_differentiable(topk_indices)
+        ctx.set_materialize_grads(False)
         return index_score_topk, topk_indices
 
     @staticmethod
     def backward(ctx, grad_score, grad_topk):
+        if grad_score is None:
+            return (None,) * 10
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, topk_indices = ctx.saved_tensors
         head, dim = ctx.shape
         k_in, ln_w, ln_b = ctx.front_saved if ctx.front is not None else (None, None, None)

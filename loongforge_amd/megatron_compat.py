@@ -161,9 +161,8 @@ class DSAIndexerLossAutoScaler(torch.autograd.Function):
     def backward(ctx, grad_output):
         (indexer_loss,) = ctx.saved_tensors
         scale = DSAIndexerLossAutoScaler.main_loss_backward_scale
-        if scale is None:
-            scale = torch.tensor(1.0, device=indexer_loss.device)
-        return grad_output, torch.ones_like(indexer_loss) * scale.to(indexer_loss.device)
+        grad = torch.ones_like(indexer_loss)
+        return grad_output, grad if scale is None else grad * scale.to(indexer_loss.device)
 
     @staticmethod
     def set_loss_scale(scale):
