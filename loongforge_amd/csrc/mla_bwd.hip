@@ -980,7 +980,13 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
   if (rs.first) dq_body<3, HG>(kv, ids, pds, dq, q0, cnt - 1 - rs.i, H, Skv, K, q_start, dup_flag, smem);
-  else reduce_body(rows, start, dkv_acc, dkv, rs.i * RED_KEYS, n_keys, accumulate, dup_flag, smem);
+  else {
+    // longest work first: from the first key on where the first half of the keys has most of the rows (causal windows), else
+    // from the last key (compressed keys behind a sliding window)
+    const int groups = (n_keys + RED_KEYS - 1) / RED_KEYS;
+    const bool forward = 2 * (long long)start[n_keys / 2] >= start[n_keys];
+    reduce_body(rows, start, dkv_acc, dkv, (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS, n_keys, accumulate, dup_flag, smem);
+  }
 }
 
 // fp32 accumulator -> bf16 dKV; NaN everywhere when a query row held a repeated id
