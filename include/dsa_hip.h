@@ -66,6 +66,31 @@ int dsa_quant_rowwise_e4m3_weights(const void* x, int64_t rows, int cols, void* 
                                    float* weight_scaled, void* stream);
 
 /*
+ * The quantiser over rows padded on the way: x [tokens, heads_in, dim_in] bf16 -> x8 [tokens, heads_out, 128], zeros in
+ * between.  weights (NULL, or [tokens, heads_in] f32 / bf16): weight_scaled [tokens, heads_out] = (w * scale_inv) * factor.
+ */
+int dsa_quant_padded_e4m3(const void* x, int64_t tokens, int heads_in, int dim_in, int heads_out, void* x8, float* scale_inv,
+                          float eps, int pow2, const void* weights, int weights_bf16, float factor, float* weight_scaled,
+                          void* stream);
+
+/*
+ * Rotary tables [n, 2 half]: angle[i][c] = (i + offset) * inv_freq[c % half] (what = 0, into a, f32), or cosines into a and
+ * sines into b (what = 1: f32, 2: bf16).
+ */
+int dsa_rotary_tables(const float* inv_freq, int half, int n, float offset, int what, void* a, void* b, void* stream);
+
+/*
+ * y = t cos + rotate_half(t) sin over bf16 rows [rows, heads, d] (strides in elements, unit inside a row), cos / sin =
+ * bf16(cos / sin(angles[row / batch]) * mscale), every product and the sum rounded to bf16 as separate tensor operations
+ * round.  interleaved: pairs are adjacent in t, halves in y.  transpose: the gradient (pairs adjacent in y then).
+ */
+int dsa_rope_steps(const void* x, int64_t x_tok, int64_t x_head, void* y, int64_t y_tok, int64_t y_head, const float* angles,
+                   float mscale, int interleaved, int batch, int64_t rows, int heads, int d, int transpose, void* stream);
+
+/* Hadamard rotation of bf16 rows of n = 32 .. 512 elements: fp32 butterfly, times n^-0.5, rounded to bf16. */
+int dsa_hadamard(const void* x, void* y, int64_t rows, int n, void* stream);
+
+/*
  * The indexer front end behind its projections in one pass per 128-element row:
  *   [LayerNorm ->] [RoPE on the leading 64 elements ->] [Hadamard rotation ->] quantiser [-> weight scaling]
  * Replaces, on the key side, k_norm -> _apply_rope -> rotate_activation at

@@ -182,6 +182,69 @@ py::object indexer_front(const Tensor& x_, int64_t rows_per_token, const OptTens
   return py::make_tuple(x8, scale_inv, y, scaled);
 }
 
+py::tuple quant_padded(const Tensor& x_, int64_t heads_out, const OptTensor& weights_, double factor) {
+  need_gpus(x_, weights_);
+  REQUIRE(x_.dim() == 3, "quant_padded expects [tokens, heads, dim]");
+  const Tensor x = x_.to(at::kBFloat16).contiguous();
+  OptTensor weights;
+  if (weights_) {
+    REQUIRE(weights_->numel() == x.size(0) * x.size(1), "quant_padded: one weight per row expected");
+    weights = weights_->scalar_type() == at::kBFloat16 ? weights_->contiguous() : f32(*weights_);
+  }
+  Call call(x);
+  const int64_t T = x.size(0);
+  Tensor x8 = make({T, heads_out, 128}, at::kFloat8_e4m3fn, x), scale_inv = make({T, heads_out}, at::kFloat, x), scaled;
+  if (weights) scaled = make({T, heads_out}, at::kFloat, x);
+  run("dsa_quant_padded_e4m3", dsa_quant_padded_e4m3, x.const_data_ptr(), T, (int)x.size(1), (int)x.size(2), (int)heads_out, x8.data_ptr(),
+      (float*)scale_inv.data_ptr(), 1e-12f, 1, ptr(weights), weights && weights->scalar_type() == at::kBFloat16, (float)factor,
+      weights ? (float*)scaled.data_ptr() : nullptr, call.stream);
+  return py::make_tuple(x8, scale_inv, weights ? py::cast(scaled) : py::none());
+}
+
+// ---- separate operations of the indexer's front end ---------------------------------------------------
+py::object rotary_angles(const Tensor& inv_freq, int64_t n, double offset) {
+  if (!inv_freq.is_cuda() || !plain(inv_freq) || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous()) return py::none();
+  Call call(inv_freq);
+  Tensor a = make({n, 1, 1, 2 * inv_freq.numel()}, at::kFloat, inv_freq);
+  run("dsa_rotary_tables", dsa_rotary_tables, (const float*)inv_freq.const_data_ptr(), (int)inv_freq.numel(), (int)n, (float)offset, 0,
+      out_ptr<void>(a), (void*)nullptr, call.stream);
+  return py::cast(a);
+}
+
+py::object rotary_cos_sin(const Tensor& inv_freq, int64_t n, double offset, at::ScalarType type) {
+  if (!inv_freq.is_cuda() || !plain(inv_freq) || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous() ||
+      (type != at::kFloat && type != at::kBFloat16)) return py::none();
+  Call call(inv_freq);
+  Tensor c = make({n, 1, 1, 2 * inv_freq.numel()}, type, inv_freq), s = at::empty_like(c);
+  run("dsa_rotary_tables", dsa_rotary_tables, (const float*)inv_freq.const_data_ptr(), (int)inv_freq.numel(), (int)n, (float)offset,
+      type == at::kFloat ? 1 : 2, out_ptr<void>(c), out_ptr<void>(s), call.stream);
+  return py::make_tuple(c, s);
+}
+
+// t [s, (b,) h, d] with unit stride inside rows -> contiguous result of the same shape
+Tensor rope_steps(const Tensor& t, const Tensor& angles, double mscale, bool interleaved, bool transpose) {
+  need_gpus(t, angles);
+  const Tensor x = t.stride(-1) == 1 && (t.dim() == 3 || t.stride(0) == t.size(1) * t.stride(1)) ? t : t.contiguous();
+  const int64_t batch = x.dim() == 4 ? x.size(1) : 1, rows = x.size(0) * batch, d = x.size(-1), heads = x.size(-2);
+  REQUIRE(x.scalar_type() == at::kBFloat16 && angles.scalar_type() == at::kFloat && angles.is_contiguous() && angles.size(-1) == d &&
+          angles.size(0) >= x.size(0) && angles.numel() == angles.size(0) * d, "rope_steps: inconsistent arguments");
+  Call call(x);
+  Tensor y = make(x.sizes(), at::kBFloat16, x);
+  run("dsa_rope_steps", dsa_rope_steps, x.const_data_ptr(), x.dim() == 4 ? x.stride(1) : x.stride(0), x.stride(-2), out_ptr<void>(y), heads * d, d,
+      (const float*)angles.const_data_ptr(), (float)mscale, (int)interleaved, (int)batch, rows, (int)heads, (int)d, (int)transpose, call.stream);
+  return y;
+}
+
+Tensor hadamard(const Tensor& x_) {
+  need_gpus(x_);
+  REQUIRE(x_.scalar_type() == at::kBFloat16, "hadamard expects bf16 rows");
+  const Tensor x = x_.contiguous();
+  Call call(x);
+  Tensor y = at::empty_like(x);
+  run("dsa_hadamard", dsa_hadamard, x.const_data_ptr(), out_ptr<void>(y), x.numel() / std::max<int64_t>(x.size(-1), 1), (int)x.size(-1), call.stream);
+  return y;
+}
+
 // ---- indexer ----------------------------------------------------------------------------------------
 struct IndexerShape { int S, Hi, Sk; };
 IndexerShape indexer_shape(const Tensor& q8, const Tensor& q_w, const Tensor& k8, const Tensor& k_scale, const Tensor& ks, const Tensor& ke) {
@@ -554,6 +617,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(rotate_quant);
   DEF(quant_weights);
   DEF(indexer_front);
+  DEF(quant_padded);
+  DEF(rotary_angles);
+  DEF(rotary_cos_sin);
+  DEF(rope_steps);
+  DEF(hadamard);
   DEF(indexer_topk);
   DEF(topk);
   DEF(indexer_bwd);

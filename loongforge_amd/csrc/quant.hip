@@ -123,6 +123,51 @@ __global__ __launch_bounds__(256) void rotate_quant128_kernel(const uint4* __res
 }
 
 
+// The quantiser over rows that are padded on the way: token t's heads_in rows of dim_in elements become heads_out rows of 128,
+// zeros in between (as if the bf16 tensor had been padded first: zero rows get the scale of the epsilon floor, and the
+// weight 0).  Weights may be bf16.
+__global__ __launch_bounds__(256) void quant_padded_kernel(const unsigned short* __restrict__ x, int heads_in, int dim_in, int heads_out,
+                                                           uint2* __restrict__ x8, float* __restrict__ scale_inv, int64_t rows,
+                                                           float eps, int pow2, const void* __restrict__ w_in, int w_bf16, float w_factor,
+                                                           float* __restrict__ w_scaled) {
+  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int sub = threadIdx.x & 15;
+  if (row >= rows) return;               // (the 16 lanes of a row leave together)
+  const int64_t tok = row / heads_out;
+  const int h = (int)(row % heads_out);
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    v[i] = h < heads_in && 8 * sub + i < dim_in ? bf16_bits_to_f32(x[(tok * heads_in + h) * dim_in + 8 * sub + i]) : 0.f;
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
+  amax = fmaxf(wave_max16(amax), eps);
+  float scale = 448.0f / amax;
+  if (pow2) scale = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, scale) & 0xff800000u);
+  float q[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) q[i] = fminf(fmaxf(v[i] * scale, -448.0f), 448.0f);
+  int lo = 0, hi = 0;
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], lo, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], hi, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
+  x8[row * 16 + sub] = make_uint2((unsigned)lo, (unsigned)hi);
+  if (sub == 0) {
+    const float si = 1.0f / scale;
+    scale_inv[row] = si;
+    if (w_scaled) {
+      float w = 0.f;
+      if (h < heads_in) {
+        const int64_t e = tok * heads_in + h;
+        w = w_bf16 ? bf16_bits_to_f32(((const unsigned short*)w_in)[e]) : ((const float*)w_in)[e];
+      }
+      w_scaled[row] = (w * si) * w_factor;
+    }
+  }
+}
+
 // The indexer front end behind its projections, one pass over a 128-element row:
 //   LN    (key rows)  y = ((x - mean) * rstd) * gamma + beta, statistics in fp32, rounded to bf16
 //   ROPE              rotation of the leading 64 elements by the row's position (pairs adjacent or split,
@@ -293,6 +338,22 @@ extern "C" int dsa_quant_rowwise_e4m3(const void* x, int64_t rows, int cols, voi
   quant128_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(
       (const uint4*)x, (uint2*)x8, scale_inv, rows, eps, pow2, nullptr, 0.f, nullptr);
   DSA_CHECK_LAUNCH("dsa_quant_rowwise_e4m3");
+  return DSA_OK;
+}
+
+extern "C" int dsa_quant_padded_e4m3(const void* x, int64_t tokens, int heads_in, int dim_in, int heads_out, void* x8, float* scale_inv,
+                                     float eps, int pow2, const void* weights, int weights_bf16, float factor, float* weight_scaled,
+                                     void* stream) {
+  DSA_REQUIRE(tokens >= 0 && heads_in > 0 && heads_in <= heads_out && dim_in > 0 && dim_in <= 128,
+              "dsa_quant_padded_e4m3: %d heads of %d elements do not fit %d of 128", heads_in, dim_in, heads_out);
+  DSA_REQUIRE(x8 != nullptr && scale_inv != nullptr && (weights == nullptr) == (weight_scaled == nullptr), "dsa_quant_padded_e4m3: null pointer");
+  DSA_REQUIRE(((uintptr_t)x8 % 8) == 0, "dsa_quant_padded_e4m3: misaligned pointer");
+  const int64_t rows = tokens * heads_out, blocks = (rows + 15) / 16;
+  if (rows == 0) return DSA_OK;
+  DSA_REQUIRE(blocks < (1ll << 31), "dsa_quant_padded_e4m3: too many rows");
+  quant_padded_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(
+      (const unsigned short*)x, heads_in, dim_in, heads_out, (uint2*)x8, scale_inv, rows, eps, pow2, weights, weights_bf16, factor, weight_scaled);
+  DSA_CHECK_LAUNCH("dsa_quant_padded_e4m3");
   return DSA_OK;
 }
 

@@ -61,6 +61,11 @@ def rotate_activation(x: torch.Tensor) -> torch.Tensor:
     """Hadamard rotation of the last dimension scaled by ``dim ** -0.5`` (dsa_fused.py:74-90)."""
     assert x.dtype == torch.bfloat16, f"rotate_activation only support bf16 input, but got {x.dtype}"
     hidden_size = x.size(-1)
+    if x.is_cuda and not torch.compiler.is_compiling():
+        from . import ops
+
+        if hidden_size in ops.HADAMARD_SIZES:
+            return ops.hadamard(x)
     h = _hadamard(hidden_size, x.device, torch.float32)
     return ((x.float() @ h) * hidden_size ** -0.5).to(x.dtype)
 
@@ -308,14 +313,13 @@ class DSAIndexerFused(MegatronModule):
                                        cu_seqlens, self.pg_collection.cp.rank(), self.pg_collection.cp.size(),
                                        pe_first=True, sp_offset=0)
             return out.view(x.shape)
-        x_pe, x_nope = torch.split(
-            x, [self.qk_pos_emb_head_dim, self.index_head_dim - self.qk_pos_emb_head_dim], dim=-1
-        )
+        all_rotary = self.index_head_dim == self.qk_pos_emb_head_dim
+        x_pe = x if all_rotary else x[..., :self.qk_pos_emb_head_dim]
         indexer_rope_config = copy.copy(self.config)
         indexer_rope_config.multi_latent_attention = getattr(self.config, "dsa_indexer_rope_interleaved", False)
         x_pe = apply_rotary_pos_emb(x_pe, rotary_pos_emb, config=indexer_rope_config, cu_seqlens=cu_seqlens,
                                     mscale=mscale, cp_group=self.pg_collection.cp)
-        return torch.cat([x_pe, x_nope], dim=-1)
+        return x_pe if all_rotary else torch.cat([x_pe, x[..., self.qk_pos_emb_head_dim:]], dim=-1)
 
     def get_query_key_weight_tensors(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None,
                                      defer_rotation: bool = False):

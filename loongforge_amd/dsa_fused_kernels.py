@@ -256,12 +256,21 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
 
         head_p = 32 if head <= 32 else 64
         assert head <= 64, "the indexer kernel supports at most 64 heads"
-        q_p = _pad_to(_pad_to(index_q.to(torch.bfloat16), 128, 2), head_p, 1).contiguous()
-        k_p = _pad_to(index_k.to(torch.bfloat16), 128, 1).contiguous()
         # rotate: the Hadamard rotation of the indexer front end is applied here, fused with the
         # quantiser (a zero-padded head dimension cannot be rotated after padding: 128 only)
         assert not rotate or dim == 128, "the fused rotation needs head dim 128"
-        if front is None:
+
+        def padded():
+            return (_pad_to(_pad_to(index_q.to(torch.bfloat16), 128, 2), head_p, 1).contiguous(),
+                    _pad_to(index_k.to(torch.bfloat16), 128, 1).contiguous())
+
+        k_p = None
+        if front is None and not rotate and (head != head_p or dim != 128):
+            q_fp8, q_scale, weight_scaled = ops.quant_padded_e4m3(index_q, head_p, weights, softmax_scale)
+            k_fp8, k_scale, _ = ops.quant_padded_e4m3(index_k.unsqueeze(1), 1)
+            k_fp8, k_scale = k_fp8.squeeze(1), k_scale.squeeze(1)
+        elif front is None:
+            q_p, k_p = padded()
             quant = ops.rotate_quant_e4m3 if rotate else ops.quant_rowwise_e4m3
             # weight_scaled = weights * q_scale * softmax_scale comes out of the query's quantiser kernel
             q_fp8, q_scale, weight_scaled = ops.quant_rowwise_e4m3_weights(q_p, _pad_to(weights.float(), head_p, 1),
@@ -271,6 +280,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
             # index_q / index_k are the projections' outputs: key LayerNorm, rotary embedding and rotation
             # happen inside the quantiser kernel (a zero-padded head stays zero through all of them)
             assert dim == 128, "the fused front end needs head dim 128"
+            q_p, k_p = padded()
             q_fp8, q_scale, _, weight_scaled = ops.indexer_front_e4m3(
                 q_p, head_p, None, None, 0.0, front.cos, front.sin, front.pairing, front.positions_q, front.batch, rotate,
                 _pad_to(weights.float(), head_p, 1), softmax_scale)

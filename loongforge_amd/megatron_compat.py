@@ -101,6 +101,12 @@ class RotaryEmbedding(torch.nn.Module):
         return x.size(0)
 
     def forward(self, max_seq_len, offset=0, packed_seq=False):
+        if self.inv_freq.is_cuda and not torch.compiler.is_compiling():
+            from . import ops
+
+            angles = ops.rotary_angles(self.inv_freq, max_seq_len, offset)
+            if angles is not None:
+                return angles
         seq = torch.arange(max_seq_len, device=self.inv_freq.device, dtype=torch.float32) + offset
         freqs = torch.outer(seq, self.inv_freq)
         emb = torch.cat((freqs, freqs), dim=-1)
@@ -109,6 +115,12 @@ class RotaryEmbedding(torch.nn.Module):
 
     def get_cached_cos_sin(self, max_seq_len, dtype=torch.float32, packed_seq=False):
         """``(cos, sin)`` of the angles, each ``[seq, 1, 1, dim]`` in ``dtype`` (what the fused rotary kernels take)."""
+        if self.inv_freq.is_cuda and not torch.compiler.is_compiling():
+            from . import ops
+
+            tables = ops.rotary_cos_sin(self.inv_freq, max_seq_len, 0.0, dtype)
+            if tables is not None:
+                return tables
         emb = self.forward(max_seq_len, packed_seq=packed_seq)
         return emb.cos().to(dtype).contiguous(), emb.sin().to(dtype).contiguous()
 
@@ -126,6 +138,13 @@ def apply_rotary_pos_emb(t, freqs, config=None, cu_seqlens=None, mscale=1.0, cp_
     positions restart at every document (packed layout ``[t, h, d]``).  When
     ``config.multi_latent_attention`` is set the input is de-interleaved first, as Megatron does."""
     interleaved_in = bool(getattr(config, "multi_latent_attention", False))
+    if (cu_seqlens is None and t.is_cuda and t.dtype == torch.bfloat16 and t.ndim in (3, 4) and t.shape[-1] % 2 == 0
+            and freqs.dtype == torch.float32 and freqs.is_contiguous() and not freqs.requires_grad
+            and freqs.shape[-1] == t.shape[-1] and freqs.shape[0] >= t.shape[0] and freqs.numel() == freqs.shape[0] * freqs.shape[-1]
+            and not torch.compiler.is_compiling()):
+        from . import ops
+
+        return ops.rope_steps(t, freqs, mscale, interleaved_in)
     if interleaved_in:
         t = torch.cat((t[..., 0::2], t[..., 1::2]), dim=-1)
     if cu_seqlens is None:

@@ -152,6 +152,63 @@ def rotate_bf16(x: torch.Tensor):
     return _direct("rotate_quant", _rotate_quant_op, x, 1e-12, True, False, True)[2]
 
 
+def quant_padded_e4m3(x, heads: int, weights=None, factor: float = 1.0):
+    """:func:`quant_rowwise_e4m3_weights` of ``x [tokens, heads_in, dim]`` padded with zeros to ``[tokens, heads, 128]``, the
+    padding done on the way: (fp8 payload, ``scale_inv``, scaled weights or None)."""
+    return _native().quant_padded(x, int(heads), weights, float(factor))
+
+
+# --------------------------------------------------------------------------------------------
+# separate operations of the indexer's front end
+# --------------------------------------------------------------------------------------------
+def rotary_angles(inv_freq, n: int, offset: float = 0.0):
+    """``[n, 1, 1, dim]`` angles ``(i + offset) * inv_freq`` (twice side by side), one kernel; None for tensors it does not take."""
+    return _native().rotary_angles(inv_freq, int(n), float(offset))
+
+
+def rotary_cos_sin(inv_freq, n: int, offset: float, dtype):
+    """Cosines and sines of :func:`rotary_angles` in ``dtype`` (fp32 or bf16), one kernel; None for tensors it does not take."""
+    return _native().rotary_cos_sin(inv_freq, int(n), float(offset), dtype)
+
+
+class _RopeSteps(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, t, angles, mscale, interleaved):
+        ctx.save_for_backward(angles)
+        ctx.args = (mscale, interleaved)
+        return _native().rope_steps(t, angles, mscale, interleaved, False)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _native().rope_steps(grad, ctx.saved_tensors[0], *ctx.args, True), None, None, None
+
+
+def rope_steps(t, angles, mscale: float = 1.0, interleaved: bool = False):
+    """``t * cos + rotate_half(t) * sin`` for bf16 ``t [s, (b,) h, d]`` and fp32 ``angles [>= s, 1, 1, d]``, with the rounding of
+    the separate bf16 operations; differentiable in ``t``.  ``interleaved``: the pairs of ``t`` are adjacent elements."""
+    return _RopeSteps.apply(t, angles, float(mscale), bool(interleaved))
+
+
+HADAMARD_SIZES = (32, 64, 128, 256, 512)
+
+
+class _Hadamard(torch.autograd.Function):
+    """The rotation is symmetric: its transpose is itself."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return _native().hadamard(x)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _native().hadamard(grad.to(torch.bfloat16))
+
+
+def hadamard(x):
+    """bf16 rows of 32 .. 512 elements times the Hadamard matrix and ``n ** -0.5``; differentiable."""
+    return _Hadamard.apply(x)
+
+
 def _fp8(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == _FP8 else t.view(_FP8)
 

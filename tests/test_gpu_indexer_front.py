@@ -151,3 +151,68 @@ def test_indexer_module_with_the_front_end_inside_the_kernel(gpu, packed):
         assert a.grad is not None and b.grad is not None, n
         scale = b.grad.float().abs().max().item()
         assert (a.grad.float() - b.grad.float()).abs().max().item() <= 3e-2 * scale, n
+
+
+@pytest.mark.parametrize("heads_in,dim,heads_out", [(1, 64, 1), (4, 64, 32), (5, 100, 32), (33, 128, 64), (64, 7, 64)])
+def test_quantiser_pads_on_the_way(gpu, heads_in, dim, heads_out):
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(dim)
+    x = torch.randn(37, heads_in, dim, generator=g).to(torch.bfloat16).to(gpu)
+    x[3] = 0.0
+    padded = torch.nn.functional.pad(x, (0, 128 - dim, 0, heads_out - heads_in)).contiguous()
+    for w in (torch.randn(37, heads_in, generator=g).to(gpu), torch.randn(37, heads_in, generator=g).to(gpu, torch.bfloat16)):
+        want = ops.quant_rowwise_e4m3_weights(padded, torch.nn.functional.pad(w.float(), (0, heads_out - heads_in)), 0.3)
+        got = ops.quant_padded_e4m3(x, heads_out, w, 0.3)
+        assert torch.equal(got[0].view(torch.uint8), want[0].view(torch.uint8))
+        assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    assert ops.quant_padded_e4m3(x, heads_out)[2] is None
+
+
+@pytest.mark.parametrize("shape,interleaved,mscale", [((1, 1, 1, 2), False, 1.0), ((65, 1, 4, 64), False, 1.0), ((33, 2, 3, 62), True, 1.25),
+                                                      ((7, 5, 64), True, 1.0)])
+def test_rope_in_rounded_steps_equals_the_separate_operations(gpu, shape, interleaved, mscale):
+    """One kernel for the unfused rotary embedding: bit for bit what the bf16 tensor operations give, forward and gradient."""
+    from loongforge_amd import megatron_compat as M, ops
+
+    g = torch.Generator().manual_seed(5)
+    rot = M.RotaryEmbedding(shape[-1]).to(gpu)
+    ang = rot(shape[0] + 3, offset=11)
+    ref_ang = torch.outer(torch.arange(shape[0] + 3, dtype=torch.float32, device=gpu) + 11, rot.inv_freq)
+    assert torch.equal(ang, torch.cat((ref_ang, ref_ang), -1)[:, None, None, :])
+    for dt in (torch.float32, torch.bfloat16):
+        cos, sin = rot.get_cached_cos_sin(shape[0], dtype=dt)
+        a = rot(shape[0])
+        assert torch.equal(cos, a.cos().to(dt)) and torch.equal(sin, a.sin().to(dt))
+    base = torch.randn(*shape[:-1], shape[-1] + 6, generator=g).to(torch.bfloat16).to(gpu)
+    dout = torch.randn(*shape, generator=g).to(torch.bfloat16).to(gpu)
+
+    def separate(t):
+        if interleaved:
+            t = torch.cat((t[..., 0::2], t[..., 1::2]), dim=-1)
+        f = ang[: t.shape[0]].reshape(t.shape[0], *([1] * (t.ndim - 2)), t.shape[-1])
+        cos, sin = (torch.cos(f) * mscale).to(t.dtype), (torch.sin(f) * mscale).to(t.dtype)
+        x1, x2 = torch.chunk(t, 2, dim=-1)
+        return t * cos + torch.cat((-x2, x1), dim=-1) * sin
+
+    res = []
+    for fn in (separate, lambda t: ops.rope_steps(t, ang, mscale, interleaved)):
+        x = base.clone().requires_grad_(True)
+        y = fn(x[..., : shape[-1]])
+        res.append((y.detach(), torch.autograd.grad(y, x, dout)[0]))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("n", [32, 64, 128, 256, 512])
+def test_hadamard_rotation_of_other_widths(gpu, n):
+    from loongforge_amd import dsa_fused
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(19, 3, n, generator=g).to(torch.bfloat16).to(gpu).requires_grad_(True)
+    dout = torch.randn(19, 3, n, generator=g).to(torch.bfloat16).to(gpu)
+    y = dsa_fused.rotate_activation(x)
+    (dx,) = torch.autograd.grad(y, x, dout)
+    h = dsa_fused._hadamard(n, torch.device("cpu"), torch.float64)
+    for got, ref in ((y, x), (dx, dout)):
+        want = ref.detach().double().cpu() @ h * n ** -0.5
+        assert ((got.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all()
