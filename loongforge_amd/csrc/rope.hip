@@ -53,6 +53,49 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RopeArgs a) {
   }
 }
 
+// The same for the rows of the absorbed MLA layouts, 512 main and 64 rotary elements.  Bound by memory: 4 B per element.  The
+// kernel above has one 16-byte load per thread in flight behind an integer division, 3.2 TB/s; here a workgroup takes a tile
+// of 32 rows, 2^tok_log2 tokens by the rest in heads, and a wave eight of them: the 64 lanes move a 1 KB main part per
+// instruction and the eight rotary parts in one, all loads requested before the first store.  us, HSD -> SHD / back:
+// 4096 tokens x 128 heads 379 / 383 -> 216 / 228 (5.6 TB/s), 700 x 128 63 / 62 -> 30 / 30, 8192 x 32 183 / 177 -> 108 / 109,
+// 60 x 128 33 / 33 -> 4.7 / 5.1.  Tiles of 1, 2, 4 or 8 tokens measured within 2 %, of 32 tokens 5 % slower.
+constexpr int MLA_MAIN = 512, MLA_EMB = 64, TILE_ROWS = 32, TOK_LOG2 = 1;
+// Non-temporal loads where the rows exceed the memory-side cache (4096 x 128: 216 against 227 us); below it the data may
+// still be there from the kernel that wrote it (700 x 128: 34 against 30 us).
+constexpr long CACHE_BYTES = 256l << 20;
+template <int IN, int OUT, bool INVERSE>
+__global__ __launch_bounds__(256) void rope_mla_rows_kernel(RopeArgs a, int tok_log2, int head_tiles, bool streamed) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tok0 = ((int)blockIdx.x / head_tiles) << tok_log2;
+  const int head0 = ((int)blockIdx.x % head_tiles) * (TILE_ROWS >> tok_log2);
+  auto token = [&](int row) { return tok0 + (row & ((1 << tok_log2) - 1)); };
+  auto head = [&](int row) { return head0 + (row >> tok_log2); };
+  // rows beyond the end are read as the last one and not written
+  auto at = [&](const unsigned short* base, long per_tok, long per_head, int row) {
+    return base + min(token(row), a.tokens - 1) * per_tok + min(head(row), a.heads - 1) * per_head;
+  };
+  auto there = [&](int row) { return token(row) < a.tokens && head(row) < a.heads; };
+  const int pe_row = wave * 8 + (lane >> 3), q = lane & 7;
+  const int t = min(token(pe_row), a.tokens - 1);
+  const long pos = a.positions ? a.positions[t] : t / a.batch;
+  i32x4 v[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const i32x4* src = (const i32x4*)at(a.main_src, a.ms_tok, a.ms_head, wave * 8 + i) + lane;
+    if (streamed) v[i] = __builtin_nontemporal_load(src);
+    else v[i] = *src;
+  }
+  const Quad x = load_quad<IN>(at(a.pe_src, a.ps_tok, a.ps_head, pe_row), q, MLA_EMB);
+  const QuadTables tables = load_tables<INVERSE ? IN : OUT>(a.cos, a.sin, a.cs_f32, pos, q, MLA_EMB);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    if (there(wave * 8 + i))
+      *((i32x4*)(a.main_dst + (long)token(wave * 8 + i) * a.md_tok + (long)head(wave * 8 + i) * a.md_head) + lane) = v[i];
+  if (there(pe_row))
+    store_quad<OUT>(rotate<INVERSE>(x, tables), a.pe_dst + (long)token(pe_row) * a.pd_tok + (long)head(pe_row) * a.pd_head, q, MLA_EMB);
+}
+
 // Gradient of a pe row that the forward broadcast to every head: the head-sum of the incoming
 // gradient (fp32, heads added in ascending order within 256 / emb_dim interleaved groups, the groups
 // then in order), rounded to bf16, then the inverse rotation; written with adjacent pairing.
@@ -135,18 +178,30 @@ extern "C" int dsa_rope_rows(const void* main_src, int64_t ms_tok, int64_t ms_he
   a.cos = cos; a.sin = sin; a.cs_f32 = cos_sin_f32; a.positions = positions; a.batch = batch;
   a.tokens = tokens; a.heads = heads;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid(tokens < (1 << 20) ? tokens : (1 << 20)), block(256);
+  const dim3 block(256);
   const int sel = (in_pairing << 2) | (out_pairing << 1) | (inverse ? 1 : 0);
+  int tok_log2 = TOK_LOG2;
+  while (tok_log2 < 5 && heads <= (TILE_ROWS >> (tok_log2 + 1))) tok_log2++;
+  const int head_tiles = dsa_cdiv(heads, TILE_ROWS >> tok_log2);
+  const long tiles = (long)dsa_cdiv(tokens, 1 << tok_log2) * head_tiles;
+  const bool mla = main_src && d_main == MLA_MAIN && emb_dim == MLA_EMB && tiles < (1 << 24);
+  const bool streamed = (long)tokens * heads * (MLA_MAIN + MLA_EMB) * 4 > CACHE_BYTES;
+  const dim3 grid(mla ? (unsigned)tiles : tokens < (1 << 20) ? tokens : (1 << 20));
+#define DSA_ROPE(IN, OUT, INV) do { \
+    if (mla) rope_mla_rows_kernel<IN, OUT, INV><<<grid, block, 0, st>>>(a, tok_log2, head_tiles, streamed); \
+    else rope_rows_kernel<IN, OUT, INV><<<grid, block, 0, st>>>(a); \
+  } while (0)
   switch (sel) {
-    case 0: rope_rows_kernel<ADJ, ADJ, false><<<grid, block, 0, st>>>(a); break;
-    case 1: rope_rows_kernel<ADJ, ADJ, true><<<grid, block, 0, st>>>(a); break;
-    case 2: rope_rows_kernel<ADJ, SPLIT, false><<<grid, block, 0, st>>>(a); break;
-    case 3: rope_rows_kernel<ADJ, SPLIT, true><<<grid, block, 0, st>>>(a); break;
-    case 4: rope_rows_kernel<SPLIT, ADJ, false><<<grid, block, 0, st>>>(a); break;
-    case 5: rope_rows_kernel<SPLIT, ADJ, true><<<grid, block, 0, st>>>(a); break;
-    case 6: rope_rows_kernel<SPLIT, SPLIT, false><<<grid, block, 0, st>>>(a); break;
-    default: rope_rows_kernel<SPLIT, SPLIT, true><<<grid, block, 0, st>>>(a); break;
+    case 0: DSA_ROPE(ADJ, ADJ, false); break;
+    case 1: DSA_ROPE(ADJ, ADJ, true); break;
+    case 2: DSA_ROPE(ADJ, SPLIT, false); break;
+    case 3: DSA_ROPE(ADJ, SPLIT, true); break;
+    case 4: DSA_ROPE(SPLIT, ADJ, false); break;
+    case 5: DSA_ROPE(SPLIT, ADJ, true); break;
+    case 6: DSA_ROPE(SPLIT, SPLIT, false); break;
+    default: DSA_ROPE(SPLIT, SPLIT, true); break;
   }
+#undef DSA_ROPE
   DSA_CHECK_LAUNCH("dsa_rope_rows");
   return DSA_OK;
 }

@@ -94,6 +94,26 @@ def test_absorbed_key_rope_and_its_backward(gpu, inter, thd):
     assert (err == 0).float().mean().item() > 0.9
 
 
+@pytest.mark.parametrize("S,h,inter,positions", [(1, 1, False, False), (3, 5, True, True), (33, 1, True, False), (35, 33, False, True),
+                                                 (920, 128, False, False)])     # the last: beyond the memory-side cache
+def test_mla_rows_in_tiles(gpu, S, h, inter, positions):
+    """Rows of 512 + 64 elements go by tiles of tokens and heads: ragged tiles and one head, both directions, bit for bit."""
+    from loongforge_amd.dsa_fused_kernels import fused_rope_permute_cat
+
+    cos, sin = _tables(S, 64, inter, BF, True)
+    qc, pe = _rand(h, S, 512, seed=10), _rand(S, h, 64, seed=11)
+    cu = torch.tensor([0, S // 3, S], dtype=torch.int32) if positions else None
+    pos = R.thd_positions(cu, S) if positions else torch.arange(S)
+    lead = (S,) if positions else (S, 1)
+    qcg, peg = qc.to(gpu).requires_grad_(True), pe.view(*lead, h, 64).to(gpu).requires_grad_(True)
+    out = fused_rope_permute_cat(qcg, peg, cos.to(gpu), sin.to(gpu), cu.to(gpu) if positions else None, 0, 1, inter)
+    assert torch.equal(out.detach().cpu().view(S, h, 576), R.fused_rope_permute_cat(qc, pe, cos, sin, pos, inter))
+    g = _rand(*out.shape, seed=12)
+    out.backward(g.to(gpu))
+    gqc, gpe = R.fused_rope_permute_cat_bwd(g.view(S, h, 576), 512, cos, sin, pos, inter)
+    assert torch.equal(qcg.grad.cpu(), gqc) and torch.equal(peg.grad.cpu().view(S, h, 64), gpe)
+
+
 def test_argument_errors_of_the_rope_entry(gpu):
     from loongforge_amd import ops
 
