@@ -43,6 +43,24 @@ def test_absorb_kernel_in_place_views_and_gradients(gpu):
         ops.mla_absorb_into(a.detach(), w.detach()[:, :100], torch.empty(200, 8, 100, dtype=torch.bfloat16, device=gpu))
 
 
+@pytest.mark.parametrize("S,H", [(1, 1), (33, 7), (64, 128), (65, 128), (257, 32), (8192, 1), (8193, 1), (31, 96)])
+@pytest.mark.parametrize("k,n", [(128, 512), (512, 128)])
+def test_absorb_of_few_and_many_rows(gpu, S, H, k, n):
+    """Row blocks and waves that share a sum, on both sides of the rule that chooses the kernel."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(S + k)
+    a = torch.randn(S, H, k, generator=g).to(torch.bfloat16).to(gpu)
+    w = torch.randn(H, n, k, generator=g).to(torch.bfloat16).to(gpu)
+    c = torch.full((S, H, n + 8), 7.0, dtype=torch.bfloat16, device=gpu)
+    ops.mla_absorb_into(a, w, c[:, :, :n])
+    ref = torch.stack([a[:, h].double() @ w[h].double().t() for h in range(H)], 1)
+    size = torch.stack([a[:, h].double().abs() @ w[h].double().abs().t() for h in range(H)], 1)
+    # one rounding to bf16, and k fp32 additions
+    assert ((c[:, :, :n].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + k * 2.0 ** -24 * size).all()
+    assert (c[:, :, n:] == 7.0).all()
+
+
 @pytest.mark.parametrize("S,H", [(1, 3), (33, 16), (64, 2), (65, 5), (300, 128), (777, 1)])
 @pytest.mark.parametrize("pairing,dtype", [(0, torch.bfloat16), (1, torch.float32)])
 def test_absorb_and_rope_in_one_kernel(gpu, S, H, pairing, dtype):
