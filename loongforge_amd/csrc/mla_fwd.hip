@@ -532,17 +532,32 @@ __global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
   }
 }
 
-// Sum of the ksplit partial results of a query: one wave per (query, 32-head block, value column tile), reading
-// the accumulator layout in which they were stored (1 KB per instruction).  HBM / L2-bound: ksplit * H * 2 KB per query.
+// Sum of the ksplit partial results of a query, reading the accumulator layout in which they were stored (1 KB per
+// instruction).  HBM / L2-bound with many queries (ksplit * H * 2 KB each): one wave per (query, 32-head block, value column
+// tile).  A few queries are bound by the chain of round trips to memory and by the compute units at work: SHARED gives the
+// tile to the four waves of a workgroup, a quarter of the ranges each, whose sums meet in LDS.
+template <bool SHARED>
 __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31;
   const int HB = a.H / 32;
-  const int dt = ((int)blockIdx.x & 3) * 4 + wave;
-  const int hb = ((int)blockIdx.x >> 2) % HB, qi = ((int)blockIdx.x >> 2) / HB;
-  const int ns = a.ksplit;
+  const int per = SHARED ? DTILES : DTILES / 4;
+  const int dt = SHARED ? (int)blockIdx.x % per : ((int)blockIdx.x % per) * 4 + wave;
+  const int hb = ((int)blockIdx.x / per) % HB, qi = ((int)blockIdx.x / per) / HB;
+  const int ns = a.ksplit, s0 = SHARED ? wave : 0, s_step = SHARED ? 4 : 1;
   const float* ml = a.part_ml + ((size_t)qi * ns * a.H + hb * 32 + r) * 2;
   const f32x4* po = a.part_o + (((size_t)qi * ns * HB + hb) * DTILES + dt) * 256 + lane;
   const size_t o_step = (size_t)HB * DTILES * 256;
+  constexpr int AHEAD = SHARED ? 4 : 2;      // ranges requested together; the first ones beside the statistics
+  f32x4 v[AHEAD][4];
+  auto load = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+      if (s + i * s_step < ns) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[i][j] = po[(s + i * s_step) * o_step + j * 64];
+      }
+  };
+  load(s0);
   float m = -1e30f;
   bool again = false;                        // the same for all threads of the workgroup
 #pragma unroll 8
@@ -557,16 +572,42 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
   for (int e = 0; e < 16; e++) acc[e] = 0.f;
   if (__ballot(again) != 0ull) {
     redo_block(a, qi, hb, dt, acc, m, l);
+    if (SHARED && wave != 0) return;         // all waves have the same block
   } else {
-#pragma unroll 4
-    for (int s = 0; s < ns; s++) {
-      const float f = __builtin_amdgcn_exp2f(ml[(size_t)s * a.H * 2] - m);
-      l = fmaf(ml[(size_t)s * a.H * 2 + 1], f, l);
+    for (int s = s0; s < ns; s += AHEAD * s_step) {
+      if (s != s0) load(s);
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const f32x4 v = po[s * o_step + j * 64];
+      for (int i = 0; i < AHEAD; i++) {
+        const int si = s + i * s_step;
+        if (si >= ns) break;
+        const float f = __builtin_amdgcn_exp2f(ml[(size_t)si * a.H * 2] - m);
+        l = fmaf(ml[(size_t)si * a.H * 2 + 1], f, l);
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[4 * j + e] = fmaf(v[e], f, acc[4 * j + e]);
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[4 * j + e] = fmaf(v[i][j][e], f, acc[4 * j + e]);
+      }
+    }
+    if (SHARED) {
+      extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+      f32x4* box = (f32x4*)smem + lane;                                  // [wave - 1][4][lane], then the sums l
+      float* box_l = (float*)(smem + 3 * 4096) + lane;
+      if (wave != 0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) box[((wave - 1) * 4 + j) * 64] = f32x4{acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
+        box_l[(wave - 1) * 64] = l;
+      }
+      __syncthreads();
+      if (wave != 0) return;
+#pragma unroll
+      for (int w = 0; w < 3; w++) {
+        l += box_l[w * 64];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const f32x4 o = box[(w * 4 + j) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[4 * j + e] += o[e];
+        }
       }
     }
   }
@@ -583,18 +624,23 @@ int max_slots(int mode, int stages) {        // slots of a range whose id arrays
   return (160 * 1024 - ring - 16) * 16 / 68 / 64 * 64;                  // 4 B per slot + 8 B per tile of 32
 }
 
+// The combine kernel shares a tile's ranges among waves for few head blocks (2048 slots, us with it / without: 1 query x 128
+// heads 18.4 / 20.2, 1 x 32 17.3 / 18.9, 4 x 128 22.2 / 22.6, 8 x 128 24.6 / 24.6, 16 x 128 32.3 / 30.2).
+constexpr int SHARE_RANGES = 4, SHARE_BLOCKS = 16;
+bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES && (long)S * (H / 32) <= SHARE_BLOCKS; }
+
 FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
 
 // The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
 // units, each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel that follows.
 // The constants are measured times in us (random rows; a pair of tiles on an idle chip and on a full one: the gathers
-// of 256 workgroups share the fabric): at 2048 slots and 128 heads one query takes 104 us in mode 0 and 17 us as
-// 32 workgroups of mode 2, 48 queries 104 and 45 us (mode 1 in two ranges), 200 queries of 64 heads 114 and 67 us
+// of 256 workgroups share the fabric): at 2048 slots and 128 heads one query takes 104 us in mode 0 and 17.7 us as
+// 64 workgroups of mode 2 (in 16 ranges; 18.4 in 11), 48 queries 104 and 45 us (mode 1 in two ranges), 200 queries of 64 heads 114 and 67 us
 // (mode 1), 4096 of 32 heads 1840 and 980 us (mode 2); 1500 queries of 128 heads stay in mode 0 (810 against 905 us).
 // A query with one pair of tiles has nothing to share out: mode 0.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   if (K <= 2 * BI) return one_workgroup_per_query(K);
-  constexpr float FIXED = 6.0f, REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, COMBINE_BYTES_PER_US = 6e6f;
+  constexpr float FIXED = 6.0f, REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
   constexpr float PAIR_IDLE[3] = {2.95f, 1.6f, 1.3f}, PAIR_FULL[3] = {4.1f, 2.15f, 1.65f};
   const int heads[3] = {128, 64, 32};
   const int pairs = K / (2 * BI);
@@ -608,7 +654,8 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const long wgs = (long)S * n_hg * ksplit;
       const float full = wgs < 256 ? (float)wgs / 256.0f : 1.0f;
       float t = (float)((wgs + 255) / 256) * (FIXED + per * (PAIR_IDLE[mode] + full * (PAIR_FULL[mode] - PAIR_IDLE[mode])));
-      t += ksplit == 1 ? REDO : COMBINE + COMBINE_RANGE * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
+      t += ksplit == 1 ? REDO
+                       : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
       if (wgs >= 4096) break;                // more ranges only add rounds
     }
@@ -636,9 +683,10 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   else DSA_FWD_LAUNCH(2);
 #undef DSA_FWD_LAUNCH
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
-  if (dsa_reserve_lds(SPLIT ? (const void*)mla_fwd_combine_kernel : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess)
-    return -2;
-  if (SPLIT) mla_fwd_combine_kernel<<<dim3(a.S * (a.H / 32) * 4), block, tail, st>>>(a);
+  const bool shared = combine_shares(a.S, a.H, a.ksplit);
+  auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
+  if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
+  if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), block, tail, st>>>(a);
   else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), block, tail, st>>>(a);
   return 0;
 }
