@@ -50,6 +50,17 @@ __device__ __forceinline__ unsigned cvt_pk_bf16(float lo, float hi) {
   const f32x2_t v = {lo, hi};
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
 }
+// The value of lane ^ m (m = 1, 2, 4 or 8, a constant after unrolling) by moves inside rows of 16 lanes, which must all be
+// active: vector instructions that the consumer mostly absorbs, where a shuffle is a trip through LDS.
+__device__ __forceinline__ float xor16(float x, int m) {
+  const int i = __builtin_bit_cast(int, x);
+  int o;
+  if (m == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xb1, 0xf, 0xf, true);              // quad_perm [1, 0, 3, 2]
+  else if (m == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4e, 0xf, 0xf, true);         // quad_perm [2, 3, 0, 1]
+  else if (m == 4) o = __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, i, 0x141, 0xf, 0xf, true), 0x1b, 0xf, 0xf, true);
+  else o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, true);                    // row_ror:8 (m = 4: i ^ 7, then i ^ 3)
+  return __builtin_bit_cast(float, o);
+}
 // v_permlane32_swap: the upper half-wave of a trades places with the lower half-wave of b.
 __device__ __forceinline__ void swap_halves(unsigned& a, unsigned& b) {
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));

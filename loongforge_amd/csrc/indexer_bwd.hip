@@ -87,7 +87,7 @@ __device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_i
     for (int m = 1; m < 16; m <<= 1)
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        const float o = __shfl_xor(v[i], m, 64);
+        const float o = xor16(v[i], m);
         v[i] = (sub & m) ? o - v[i] : v[i] + o;
       }
 #pragma unroll
@@ -102,7 +102,7 @@ __device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_i
     float other[8];
     if (f.pairing == 1) {
 #pragma unroll
-      for (int i = 0; i < 8; i++) other[i] = __shfl_xor(v[i], 4, 64);
+      for (int i = 0; i < 8; i++) other[i] = xor16(v[i], 4);
     } else {
 #pragma unroll
       for (int i = 0; i < 8; i++) other[i] = v[i ^ 1];

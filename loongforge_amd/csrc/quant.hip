@@ -6,10 +6,10 @@
 namespace {
 
 __device__ __forceinline__ float wave_max16(float v) {   // max over the 16 lanes sharing a row
-  v = fmaxf(v, __shfl_xor(v, 1, 64));
-  v = fmaxf(v, __shfl_xor(v, 2, 64));
-  v = fmaxf(v, __shfl_xor(v, 4, 64));
-  v = fmaxf(v, __shfl_xor(v, 8, 64));
+  v = fmaxf(v, xor16(v, 1));
+  v = fmaxf(v, xor16(v, 2));
+  v = fmaxf(v, xor16(v, 4));
+  v = fmaxf(v, xor16(v, 8));
   return v;
 }
 
@@ -84,16 +84,15 @@ __global__ __launch_bounds__(256) void rotate_quant128_kernel(const uint4* __res
   for (int m = 1; m < 16; m <<= 1)
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const float o = __shfl_xor(v[i], m, 64);
+      const float o = xor16(v[i], m);
       v[i] = (sub & m) ? o - v[i] : v[i] + o;
     }
   unsigned yb[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const unsigned lo = f32_to_bf16_bits(v[2 * i] * 0.08838834764831845f), hi = f32_to_bf16_bits(v[2 * i + 1] * 0.08838834764831845f);
-    yb[i] = lo | (hi << 16);
-    v[2 * i] = __builtin_bit_cast(float, lo << 16);
-    v[2 * i + 1] = __builtin_bit_cast(float, hi << 16);
+    yb[i] = cvt_pk_bf16(v[2 * i] * 0.08838834764831845f, v[2 * i + 1] * 0.08838834764831845f);
+    v[2 * i] = __builtin_bit_cast(float, yb[i] << 16);
+    v[2 * i + 1] = __builtin_bit_cast(float, yb[i] & 0xffff0000u);
   }
   if (live && y) y[row * 16 + sub] = make_uint4(yb[0], yb[1], yb[2], yb[3]);
   if (!x8) return;
@@ -200,12 +199,16 @@ __global__ __launch_bounds__(256) void indexer_front128_kernel(
 #pragma unroll
     for (int i = 1; i < 8; i++) s = s + t[i];
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) s = s + __shfl_xor(s, m, 64);
+    for (int m = 1; m < 16; m <<= 1) s = s + xor16(s, m);
     return s;
   };
   auto round_bf16 = [&]() {
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
+    for (int i = 0; i < 8; i += 2) {
+      const unsigned u = cvt_pk_bf16(v[i], v[i + 1]);
+      v[i] = __builtin_bit_cast(float, u << 16);
+      v[i + 1] = __builtin_bit_cast(float, u & 0xffff0000u);
+    }
   };
   if (LN) {
     const float mean = row_sum(v) * 0.0078125f;
@@ -221,8 +224,8 @@ __global__ __launch_bounds__(256) void indexer_front128_kernel(
     round_bf16();
   }
   if (PAIRING >= 0) {
-    const int64_t tok = row / rows_per_token;
-    const int64_t pos = live ? (positions ? positions[tok] : tok / batch) : 0;
+    const unsigned tok = (unsigned)row / (unsigned)rows_per_token;       // in 32 bits: a 64-bit division is a long routine
+    const int64_t pos = live ? (positions ? positions[tok] : tok / (unsigned)batch) : 0;
     auto table8 = [&](const void* t, int col, float (&o)[8]) {     // 8 consecutive entries of the position's row
       if (cs_f32) {
         const f32x4 a = *(const f32x4*)((const float*)t + pos * 64 + col), b = *(const f32x4*)((const float*)t + pos * 64 + col + 4);
@@ -250,7 +253,7 @@ __global__ __launch_bounds__(256) void indexer_front128_kernel(
     } else {
       float o[8];               // element e of lane s pairs with element e of lane s ^ 4 (lanes 0..7 hold the 64 rotary elements)
 #pragma unroll
-      for (int i = 0; i < 8; i++) o[i] = __shfl_xor(v[i], 4, 64);
+      for (int i = 0; i < 8; i++) o[i] = xor16(v[i], 4);
       if (sub < 8) {
         float c[8], s[8];
         table8(cos_t, 8 * sub, c);
@@ -272,7 +275,7 @@ __global__ __launch_bounds__(256) void indexer_front128_kernel(
     for (int m = 1; m < 16; m <<= 1)
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        const float o = __shfl_xor(v[i], m, 64);
+        const float o = xor16(v[i], m);
         v[i] = (sub & m) ? o - v[i] : v[i] + o;
       }
 #pragma unroll
@@ -397,7 +400,7 @@ extern "C" int dsa_indexer_front_e4m3(const void* x, int64_t rows, int cols, int
               ((uintptr_t)sin % 16) == 0, "dsa_indexer_front_e4m3: misaligned pointer");
   if (rows == 0) return DSA_OK;
   const int64_t blocks = (rows + 15) / 16;
-  DSA_REQUIRE(blocks < (1ll << 31), "dsa_indexer_front_e4m3: too many rows");
+  DSA_REQUIRE(rows < (1ll << 32), "dsa_indexer_front_e4m3: too many rows");
 #define DSA_FRONT_LAUNCH(LN, P) indexer_front128_kernel<LN, P><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>( \
       (const uint4*)x, rows, rows_per_token, ln_weight, ln_bias, ln_eps, cos, sin, cos_sin_f32, positions, batch, rotate, \
       (uint2*)x8, scale_inv, (uint4*)y, eps, pow2, weights, factor, weight_scaled)
