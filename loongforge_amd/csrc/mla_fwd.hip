@@ -62,7 +62,9 @@ struct FwdArgs {
 // O^T accumulators are never rescaled (a rescaling branch in the loop, even one never taken, costs the
 // register allocator hundreds of spills).  Where a later tile exceeds it by more than 2^64 (exp2 then nears
 // the end of fp32) the wave marks its heads - a NaN with a payload in lse, or in the statistics of its
-// slot range - and the kernel that follows does them again relative to the true row maximum.
+// slot range - and the kernel that follows does them again relative to the true row maximum.  In mode 2 with all slots in
+// one workgroup, where the waves' registers have room for it, the workgroup does so itself: the kernel that follows takes
+// 4.5 us also when nothing is marked.
 constexpr float REDO_ABOVE = 64.0f;
 constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
 __device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
@@ -128,6 +130,73 @@ __device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned
   acc_row_to_16B(t, scale, o);
   *(uint4*)p = o[0];
   *(uint4*)(p + 16) = o[1];
+}
+
+// One 32-head block of a query relative to the true maximum of every head, all slots, one tile at a time: every
+// wave computes S^T of the block and sums its own value column tile dt.  For the marked blocks only: simple, and
+// light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.
+__device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int dt, f32x16& acc, float& m, float& l) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int NT = a.K / BI;
+  int* idx_s = (int*)(smem + TILE_BYTES);
+  unsigned* tmask = (unsigned*)(idx_s + a.K);
+  int* tlist = (int*)(tmask + NT);
+  __syncthreads();
+  const int ntiles = stage_ids(a.ids, qi, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  const LaneOffsets lo = lane_offsets();
+  const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * a.H + hb * 32 + r) * DQK) + g;
+  const float c2 = a.sm_scale * LOG2E;
+  unsigned v_off[2][2];                      // the wave's value columns: lo.tr_off[s][t][dt & 1]
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      v_off[s][t] = (unsigned)((dt >> 1) * GRP_BYTES) + lo.tr_off[s][t][0] + (unsigned)(dt & 1) * (lo.tr_off[s][t][1] - lo.tr_off[s][t][0]);
+  m = -1e30f;
+  l = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll 1
+  for (int step = 0; step < 2 * ntiles; step++) {            // first sweep: the maximum; second: the sums
+    const int tile = tlist[step < ntiles ? step : step - ntiles];
+    __syncthreads();
+    gather_tile(a.kv, idx_s, tile, (unsigned)(uintptr_t)smem);
+    DSA_WAIT_VMCNT(0);
+    __syncthreads();
+    f32x16 sacc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) sacc[e] = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < KSTEPS / 4; c++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(smem + c * GRP_BYTES + lo.row_off[j]),
+                                                       qp[2 * (4 * c + j)], sacc, 0, 0, 0);
+    const unsigned mg = tmask[tile] >> (4 * g);
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+      if (!((mg >> (8 * (e >> 2) + (e & 3))) & 1u)) sacc[e] = -INFINITY;
+    if (step < ntiles) {
+      m = fmaxf(m, tile_max(sacc) * c2);
+    } else {
+      bf16x8 pb[2];
+      softmax_numerators(sacc, c2, m, l, pb);
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            value_operand(read_tr(smem + v_off[s][0]), read_tr(smem + v_off[s][1])), pb[s], acc, 0, 0, 0);
+    }
+  }
+  l += __shfl_xor(l, 32, 64);
+}
+
+__device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, int dt, const f32x16& acc, float m, float l) {
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int h = hb * 32 + r;
+  const Final fin = finish_head(m, l, a.sink ? a.sink + h : nullptr);
+  if (dt == 0 && g == 0) a.lse[(size_t)qi * a.H + h] = fin.lse;
+  store_out(acc, fin.inv, (unsigned short*)a.out + ((size_t)qi * a.H + h) * DV + 32 * dt + 8 * g);
 }
 
 template <int MODE, int STAGES, bool SPLIT, int POUT>   // SPLIT: ksplit > 1; POUT: 0 none, 1 bf16, 2 f32
@@ -381,6 +450,16 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     __syncthreads();
     const float m_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2], l_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2 + 1];
     again |= is_marked(m_o);
+    if (MODE == 2 && !SPLIT && again) {      // the same for all waves: they have the same heads
+#pragma unroll 1
+      for (int dt = wave; dt < DTILES; dt += 4) {
+        f32x16 acc;
+        float m, l;
+        redo_block(a, qi, hb, dt, acc, m, l);
+        write_block(a, qi, hb, dt, acc, m, l);
+      }
+      return;
+    }
     const float nm = fmaxf(m_ref, m_o);
     const float f = __builtin_amdgcn_exp2f(m_ref - nm);
     l_tot = l_tot * f + l_o * __builtin_amdgcn_exp2f(m_o - nm);
@@ -444,74 +523,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   }
 }
 
-// One 32-head block of a query relative to the true maximum of every head, all slots, one tile at a time: every
-// wave computes S^T of the block and sums its own value column tile dt.  For the marked blocks only: simple, and
-// light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.
-__device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int dt, f32x16& acc, float& m, float& l) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
-  const int NT = a.K / BI;
-  int* idx_s = (int*)(smem + TILE_BYTES);
-  unsigned* tmask = (unsigned*)(idx_s + a.K);
-  int* tlist = (int*)(tmask + NT);
-  __syncthreads();
-  const int ntiles = stage_ids(a.ids, qi, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
-  const LaneOffsets lo = lane_offsets();
-  const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * a.H + hb * 32 + r) * DQK) + g;
-  const float c2 = a.sm_scale * LOG2E;
-  unsigned v_off[2][2];                      // the wave's value columns: lo.tr_off[s][t][dt & 1]
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int t = 0; t < 2; t++)
-      v_off[s][t] = (unsigned)((dt >> 1) * GRP_BYTES) + lo.tr_off[s][t][0] + (unsigned)(dt & 1) * (lo.tr_off[s][t][1] - lo.tr_off[s][t][0]);
-  m = -1e30f;
-  l = 0.f;
-#pragma unroll
-  for (int e = 0; e < 16; e++) acc[e] = 0.f;
-#pragma unroll 1
-  for (int step = 0; step < 2 * ntiles; step++) {            // first sweep: the maximum; second: the sums
-    const int tile = tlist[step < ntiles ? step : step - ntiles];
-    __syncthreads();
-    gather_tile(a.kv, idx_s, tile, (unsigned)(uintptr_t)smem);
-    DSA_WAIT_VMCNT(0);
-    __syncthreads();
-    f32x16 sacc;
-#pragma unroll
-    for (int e = 0; e < 16; e++) sacc[e] = 0.f;
-#pragma unroll 1
-    for (int c = 0; c < KSTEPS / 4; c++)
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(smem + c * GRP_BYTES + lo.row_off[j]),
-                                                       qp[2 * (4 * c + j)], sacc, 0, 0, 0);
-    const unsigned mg = tmask[tile] >> (4 * g);
-#pragma unroll
-    for (int e = 0; e < 16; e++)
-      if (!((mg >> (8 * (e >> 2) + (e & 3))) & 1u)) sacc[e] = -INFINITY;
-    if (step < ntiles) {
-      m = fmaxf(m, tile_max(sacc) * c2);
-    } else {
-      bf16x8 pb[2];
-      softmax_numerators(sacc, c2, m, l, pb);
-#pragma unroll
-      for (int s = 0; s < 2; s++)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            value_operand(read_tr(smem + v_off[s][0]), read_tr(smem + v_off[s][1])), pb[s], acc, 0, 0, 0);
-    }
-  }
-  l += __shfl_xor(l, 32, 64);
-}
-
-__device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, int dt, const f32x16& acc, float m, float l) {
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
-  const int h = hb * 32 + r;
-  const Final fin = finish_head(m, l, a.sink ? a.sink + h : nullptr);
-  if (dt == 0 && g == 0) a.lse[(size_t)qi * a.H + h] = fin.lse;
-  store_out(acc, fin.inv, (unsigned short*)a.out + ((size_t)qi * a.H + h) * DV + 32 * dt + 8 * g);
-}
-
-// ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
+// Modes 0 and 1, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
 // redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
 __global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
   const int wave = threadIdx.x >> 6;
@@ -654,7 +666,7 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const long wgs = (long)S * n_hg * ksplit;
       const float full = wgs < 256 ? (float)wgs / 256.0f : 1.0f;
       float t = (float)((wgs + 255) / 256) * (FIXED + per * (PAIR_IDLE[mode] + full * (PAIR_FULL[mode] - PAIR_IDLE[mode])));
-      t += ksplit == 1 ? REDO
+      t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
       if (wgs >= 4096) break;                // more ranges only add rounds
@@ -685,6 +697,7 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
   const bool shared = combine_shares(a.S, a.H, a.ksplit);
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
+  if (MODE == 2 && !SPLIT) return 0;
   if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
   if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), block, tail, st>>>(a);
   else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), block, tail, st>>>(a);
