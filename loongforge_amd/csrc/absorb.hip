@@ -19,9 +19,9 @@
 // bytes per lane, next block requested before this block's MFMAs).  With C^T in the accumulators a lane
 // owns one output row; four column tiles go through an 8 KB strip per wave, so that a store instruction
 // writes four 256-byte row segments instead of 32 of 32 bytes.
-// Few rows (absorb_few_kernel): one wave (query side) or two (output side) per (head, 32 columns) read
-// their weight rows straight into registers and walk the row blocks: 4 - 8x the waves, no trip of the
-// weights through LDS.
+// Few rows (absorb_few_kernel): one wave per (head, 64 columns) on the query side, two per (head, 32
+// columns) on the output side read their weight rows straight into registers and walk the row blocks:
+// more waves, no trip of the weights through LDS.
 #include <algorithm>
 
 #include "mla_tile.h"
@@ -154,21 +154,21 @@ __global__ __launch_bounds__(64 * WAVES, 1) void absorb_kernel(AbsorbArgs p, int
   }
 }
 
-// One task per (head, 32 output columns) and range of row blocks, plus one per head for the rotary part.  With K = 512 two
-// waves share a task, half of the sum each: half the registers (the next rows are requested before these rows' products)
-// and twice the waves; the halves meet in LDS, the two waves storing every other block.
+// One workgroup per (head, column tiles) and range of row blocks, plus one per head for the rotary part.  Query side: one wave
+// and two 32-column tiles, so that it fills whole 128-byte lines of the output (us, one / two / four tiles: 48 rows x 128 heads
+// 13.1 / 11.1 / 11.6; waves in workgroups of their own: 1 row 4.8, in pairs 5.5, in fours 7.1).  Output side (K = 512): two
+// waves share a tile, half of the sum each: half the registers (the next rows are requested before these rows' products) and
+// twice the waves; the halves meet in LDS, the two waves storing every other block.
 template <int K> constexpr int FEW_SHARE = K == 512 ? 2 : 1;
-template <int K> constexpr int FEW_TASKS = K == 512 ? 1 : 4;          // tasks of a workgroup
+template <int K> constexpr int FEW_COLS = K == 512 ? 1 : 2;
 template <int K, int N>
-__global__ __launch_bounds__(64 * FEW_SHARE<K> * FEW_TASKS<K>, 2) void absorb_few_kernel(AbsorbArgs p) {
-  constexpr int SHARE = FEW_SHARE<K>, KS = K / 16 / SHARE, NT = N / 32;
+__global__ __launch_bounds__(64 * FEW_SHARE<K>, 2) void absorb_few_kernel(AbsorbArgs p) {
+  constexpr int SHARE = FEW_SHARE<K>, KS = K / 16 / SHARE, COLS = FEW_COLS<K>, NT = N / (32 * COLS);
   __shared__ f32x4 box[SHARE == 1 ? 1 : 2 * 4 * 64];         // [block % 2][4][lane]
   const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int task = SHARE == 1 ? (int)blockIdx.x * FEW_TASKS<K> + wave : (int)blockIdx.x, part = SHARE == 1 ? 0 : wave;
+  const int part = SHARE == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int per = p.pe_src ? NT + 1 : NT;
-  const int h = task / per, nt = task % per;
-  if (h >= p.H) return;                      // (one task per workgroup where waves share it: all of them leave)
+  const int h = (int)blockIdx.x / per, nt = (int)blockIdx.x % per;
   const int nblk = (p.S + 31) / 32;
   const int b_lo = (int)((long)nblk * blockIdx.y / gridDim.y), b_hi = (int)((long)nblk * (blockIdx.y + 1) / gridDim.y);
   if (nt == NT) {
@@ -178,10 +178,13 @@ __global__ __launch_bounds__(64 * FEW_SHARE<K> * FEW_TASKS<K>, 2) void absorb_fe
                     tables_of(p, position_of(p, s), q), s, h, q);
     return;
   }
-  bf16x8 wv[KS], cur[KS], nxt[KS];
-  const bf16x8* wp = (const bf16x8*)(p.w + ((size_t)h * N + 32 * nt + r) * K) + 2 * KS * part + g;
+  bf16x8 wv[COLS][KS], cur[KS], nxt[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) wv[ks] = wp[2 * ks];
+  for (int c = 0; c < COLS; c++) {
+    const bf16x8* wp = (const bf16x8*)(p.w + ((size_t)h * N + 32 * (COLS * nt + c) + r) * K) + 2 * KS * part + g;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) wv[c][ks] = wp[2 * ks];
+  }
   auto load_rows = [&](int blk, bf16x8 (&t)[KS]) {
     const bf16x8* ap = (const bf16x8*)(p.a + (size_t)min(32 * blk + r, p.S - 1) * p.a_tok + (size_t)h * p.a_head) + 2 * KS * part + g;
 #pragma unroll
@@ -192,38 +195,41 @@ __global__ __launch_bounds__(64 * FEW_SHARE<K> * FEW_TASKS<K>, 2) void absorb_fe
   for (int blk = b_lo; blk < b_hi; blk++) {
     if (blk + 1 < b_hi) load_rows(blk + 1, nxt);
     __builtin_amdgcn_sched_barrier(0);       // all loads in flight before the first product
-    f32x16 acc;
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+    for (int c = 0; c < COLS; c++) {
+      f32x16 acc;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[ks], cur[ks], acc, 0, 0, 0);
-    bool mine = true;
-    if (SHARE == 2) {
-      // one barrier per block: a box is written again two blocks on, behind the barrier that follows its reading
-      f32x4* b = box + (blk & 1) * 256 + lane;
-      mine = part == (blk & 1);
-      if (!mine) {
+      for (int e = 0; e < 16; e++) acc[e] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) b[j * 64] = f32x4{acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
-      }
-      __syncthreads();
-      if (mine) {
+      for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[c][ks], cur[ks], acc, 0, 0, 0);
+      bool mine = true;
+      if (SHARE == 2) {
+        // one barrier per block: a box is written again two blocks on, behind the barrier that follows its reading
+        f32x4* b = box + (blk & 1) * 256 + lane;
+        mine = part == (blk & 1);
+        if (!mine) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const f32x4 o = b[j * 64];
+          for (int j = 0; j < 4; j++) b[j * 64] = f32x4{acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
+        }
+        __syncthreads();
+        if (mine) {
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[4 * j + e] += o[e];
+          for (int j = 0; j < 4; j++) {
+            const f32x4 o = b[j * 64];
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[4 * j + e] += o[e];
+          }
         }
       }
-    }
-    if (mine) {
-      uint4 o[2];
-      acc_row_to_16B(acc, 1.0f, o);          // every lane takes part; rows past the end are not stored
-      const int s = 32 * blk + r;
-      if (s < p.S) {
-        unsigned short* out = (unsigned short*)p.c + (size_t)s * p.c_tok + (size_t)h * p.c_head + 32 * nt + 8 * g;
-        *(uint4*)out = o[0];
-        *(uint4*)(out + 16) = o[1];
+      if (mine) {
+        uint4 o[2];
+        acc_row_to_16B(acc, 1.0f, o);        // every lane takes part; rows past the end are not stored
+        const int s = 32 * blk + r;
+        if (s < p.S) {
+          unsigned short* out = (unsigned short*)p.c + (size_t)s * p.c_tok + (size_t)h * p.c_head + 32 * (COLS * nt + c) + 8 * g;
+          *(uint4*)out = o[0];
+          *(uint4*)(out + 16) = o[1];
+        }
       }
     }
 #pragma unroll
@@ -233,21 +239,21 @@ __global__ __launch_bounds__(64 * FEW_SHARE<K> * FEW_TASKS<K>, 2) void absorb_fe
 
 // Up to this many (row, head) pairs the weights are better re-read by the waves than brought through LDS once per head: there the
 // other kernel is one workgroup per head that mostly waits for its weights.  us, this kernel against the other, query side with
-// rotary part / output side: 128 heads x 1 row 5.6 / 4.9 against 12.5 / 9.5, x 64 rows 14.9 / 10.7 against 15.8 / 11.3, x 100
-// 20.9 / 14.2 against 17.1 / 12.1; 64 heads x 100 13.2 / 8.1 against 14.0 / 10.4, x 200 20.1 / 13.3 against 16.6 / 12.6;
-// 32 heads x 200 12.4 / 8.6 against 15.4 / 10.9, x 300 16.5 / 11.2 against 17.1 / 11.0.
-constexpr int FEW_ROW_HEADS = 8192;
+// rotary part / output side: 128 heads x 1 row 4.8 / 4.9 against 12.5 / 9.5, x 64 rows 12.5 / 10.7 against 15.8 / 11.3, x 100
+// 17.0 / 14.2 against 17.1 / 12.1; 64 heads x 100 11.0 / 8.1 against 14.0 / 10.4, x 200 16.6 / 13.3 against 16.6 / 12.6;
+// 32 heads x 200 10.2 / 8.6 against 15.4 / 10.9, x 300 13.1 / 11.2 against 17.1 / 11.0.
+template <int K> constexpr int FEW_ROW_HEADS = K == 512 ? 8192 : 12288;
 // Row ranges until there are so many workgroups.  The query side's share of the weights is read in one round trip, so every
-// row block has its own waves (32 heads x 200 rows in 4 ranges instead of 7: 14.6 us); the output side's is not (48 rows x 128
-// heads 11.4 us with the weights read by both blocks' waves, 9.0 in one range).
-template <int K> constexpr int FEW_GROUPS = K == 512 ? 512 : 2048;
+// row block has its own waves; the output side's is not (48 rows x 128 heads 11.4 us with the weights read by both blocks'
+// waves, 9.0 in one range).
+template <int K> constexpr int FEW_GROUPS = K == 512 ? 512 : 1 << 16;
 
 template <int K, int N>
 int launch(const AbsorbArgs& p, hipStream_t st) {
-  if ((long)p.S * p.H <= FEW_ROW_HEADS) {
-    const int groups = dsa_cdiv((long)p.H * (N / 32 + (p.pe_src ? 1 : 0)), FEW_TASKS<K>);
+  if ((long)p.S * p.H <= FEW_ROW_HEADS<K>) {
+    const int groups = p.H * (N / (32 * FEW_COLS<K>) + (p.pe_src ? 1 : 0));
     const int ranges = std::max(1, std::min(FEW_GROUPS<K> / groups, (p.S + 31) / 32));
-    absorb_few_kernel<K, N><<<dim3(groups, ranges), dim3(64 * FEW_SHARE<K> * FEW_TASKS<K>), 0, st>>>(p);
+    absorb_few_kernel<K, N><<<dim3(groups, ranges), dim3(64 * FEW_SHARE<K>), 0, st>>>(p);
     return 0;
   }
   constexpr int WAVES = K == 128 ? 8 : 4;    // rows of 1 KB in registers twice: four waves

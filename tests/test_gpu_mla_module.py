@@ -43,7 +43,7 @@ def test_absorb_kernel_in_place_views_and_gradients(gpu):
         ops.mla_absorb_into(a.detach(), w.detach()[:, :100], torch.empty(200, 8, 100, dtype=torch.bfloat16, device=gpu))
 
 
-@pytest.mark.parametrize("S,H", [(1, 1), (33, 7), (64, 128), (65, 128), (257, 32), (8192, 1), (8193, 1), (31, 96)])
+@pytest.mark.parametrize("S,H", [(1, 1), (33, 7), (64, 128), (65, 128), (257, 32), (8192, 1), (8193, 1), (12289, 1), (31, 96)])
 @pytest.mark.parametrize("k,n", [(128, 512), (512, 128)])
 def test_absorb_of_few_and_many_rows(gpu, S, H, k, n):
     """Row blocks and waves that share a sum, on both sides of the rule that chooses the kernel."""
