@@ -17,7 +17,7 @@ constexpr int BLOCK = 256;
 // sums (or maxima) over the workgroup; every thread gets the result.  `scratch` holds 8 floats.
 __device__ __forceinline__ float block_max(float v, float* scratch) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, o > 8 ? __shfl_xor(v, o, 64) : xor16(v, o));
   __syncthreads();                                   // the previous reduction's reads are done
   if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -25,7 +25,7 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 }
 __device__ __forceinline__ void block_sum2(float& a, float& b, float* scratch) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { a += __shfl_xor(a, o, 64); b += __shfl_xor(b, o, 64); }
+  for (int o = 32; o > 0; o >>= 1) { a += o > 8 ? __shfl_xor(a, o, 64) : xor16(a, o); b += o > 8 ? __shfl_xor(b, o, 64) : xor16(b, o); }
   __syncthreads();
   if ((threadIdx.x & 63) == 0) { scratch[threadIdx.x >> 6] = a; scratch[4 + (threadIdx.x >> 6)] = b; }
   __syncthreads();
