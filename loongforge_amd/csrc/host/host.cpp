@@ -24,13 +24,15 @@ namespace {
 bool plain_call() {
   if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
   constexpr c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::Tracer,
-                                     c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchVmapMode});
+                                     c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchVmapMode,
+                                     c10::DispatchKey::VmapMode});
   return !c10::impl::tls_local_dispatch_key_set().included_.has_any(odd);
 }
 bool plain_tensor(const Tensor& t, bool grad) {
   constexpr c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchBatched,
+                                     c10::DispatchKey::Batched,
                                      c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
-  return !t.key_set().has_any(odd) && !(grad && t.requires_grad());
+  return !t.key_set().has_any(odd) && !(grad && t.requires_grad()) && !t._fw_grad(0).defined();
 }
 bool plain_tensor(const OptTensor& t, bool grad) { return !t || plain_tensor(*t, grad); }
 template <class... T>
@@ -39,11 +41,19 @@ bool plain(const T&... t) {
   const bool grad = at::GradMode::is_enabled();
   return (plain_tensor(t, grad) && ...);
 }
+bool ordinary(const std::vector<OptTensor>& tensors) {
+  if (!plain_call()) return false;
+  for (const OptTensor& t : tensors)
+    if (!plain_tensor(t, false)) return false;
+  return true;
+}
 #define PLAIN_OR_NONE(...) do { if (!force && !plain(__VA_ARGS__)) return py::none(); } while (0)
 
 // ---- checks ---------------------------------------------------------------------------------------
 void need_gpu(const Tensor& t) {
   TORCH_CHECK(t.is_cuda(), "DSA kernels need tensors on a HIP device; got a ", c10::DeviceTypeName(t.device().type(), true), " tensor");
+  // (fake tensors and wrappers of transforms have a device but no memory)
+  TORCH_CHECK(t.numel() == 0 || (t.has_storage() && t.storage().data() != nullptr), "DSA kernels need tensors with memory of their own");
 }
 void need_gpu(const OptTensor& t) { if (t) need_gpu(*t); }
 template <class... T>
@@ -238,7 +248,8 @@ Tensor rope_steps(const Tensor& t, const Tensor& angles, double mscale, bool int
 Tensor hadamard(const Tensor& x_) {
   need_gpus(x_);
   REQUIRE(x_.scalar_type() == at::kBFloat16, "hadamard expects bf16 rows");
-  const Tensor x = x_.contiguous();
+  Tensor x = x_.contiguous();
+  if ((uintptr_t)x.const_data_ptr() % 16) x = x.clone();        // a view that starts inside a 16-byte piece
   Call call(x);
   Tensor y = at::empty_like(x);
   run("dsa_hadamard", dsa_hadamard, x.const_data_ptr(), out_ptr<void>(y), x.numel() / std::max<int64_t>(x.size(-1), 1), (int)x.size(-1), call.stream);
@@ -610,6 +621,7 @@ void rope_rows(const OptTensor& pe_src, const OptTensor& pe_dst, const OptTensor
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("ordinary", &ordinary);
   m.doc() = "Native host layer of loongforge_amd.ops";
   py::class_<WindowCheck>(m, "WindowCheck").def("wait", &WindowCheck::wait);
 #define DEF(name) m.def(#name, torch::wrap_pybind_function(name))

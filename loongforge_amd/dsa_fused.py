@@ -61,10 +61,10 @@ def rotate_activation(x: torch.Tensor) -> torch.Tensor:
     """Hadamard rotation of the last dimension scaled by ``dim ** -0.5`` (dsa_fused.py:74-90)."""
     assert x.dtype == torch.bfloat16, f"rotate_activation only support bf16 input, but got {x.dtype}"
     hidden_size = x.size(-1)
-    if x.is_cuda and not torch.compiler.is_compiling():
+    if x.is_cuda:
         from . import ops
 
-        if hidden_size in ops.HADAMARD_SIZES:
+        if hidden_size in ops.HADAMARD_SIZES and ops.ordinary(x):
             return ops.hadamard(x)
     h = _hadamard(hidden_size, x.device, torch.float32)
     return ((x.float() @ h) * hidden_size ** -0.5).to(x.dtype)

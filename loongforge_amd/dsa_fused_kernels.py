@@ -265,7 +265,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
                     _pad_to(index_k.to(torch.bfloat16), 128, 1).contiguous())
 
         k_p = None
-        if front is None and not rotate and (head != head_p or dim != 128):
+        if front is None and not rotate and (head != head_p or dim != 128) and ops.ordinary(index_q, index_k, weights):
             q_fp8, q_scale, weight_scaled = ops.quant_padded_e4m3(index_q, head_p, weights, softmax_scale)
             k_fp8, k_scale, _ = ops.quant_padded_e4m3(index_k.unsqueeze(1), 1)
             k_fp8, k_scale = k_fp8.squeeze(1), k_scale.squeeze(1)

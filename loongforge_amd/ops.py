@@ -39,6 +39,16 @@ def _direct(name: str, op, *args):
     return op(*args)
 
 
+def ordinary(*tensors) -> bool:
+    """Whether this is an eager call on ordinary tensors, which kernels may take past the dispatcher: not compiled or traced, no
+    functorch transform, forward-mode level or dispatch mode, no batched, fake or otherwise dispatched tensor."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return _native().ordinary(tensors)
+
+
 def _stream(t: torch.Tensor):
     return torch.cuda.current_stream(t.device).cuda_stream
 
@@ -173,20 +183,33 @@ def rotary_cos_sin(inv_freq, n: int, offset: float, dtype):
 
 class _RopeSteps(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, t, angles, mscale, interleaved):
+    def forward(ctx, t, angles, mscale, interleaved, transpose):
         ctx.save_for_backward(angles)
-        ctx.args = (mscale, interleaved)
-        return _native().rope_steps(t, angles, mscale, interleaved, False)
+        ctx.args = (mscale, interleaved, not transpose)
+        return _native().rope_steps(t, angles, mscale, interleaved, transpose)
 
     @staticmethod
     def backward(ctx, grad):
-        return _native().rope_steps(grad, ctx.saved_tensors[0], *ctx.args, True), None, None, None
+        return rope_steps(grad, ctx.saved_tensors[0], *ctx.args), None, None, None, None
 
 
-def rope_steps(t, angles, mscale: float = 1.0, interleaved: bool = False):
+def rope_steps(t, angles, mscale: float = 1.0, interleaved: bool = False, transpose: bool = False):
     """``t * cos + rotate_half(t) * sin`` for bf16 ``t [s, (b,) h, d]`` and fp32 ``angles [>= s, 1, 1, d]``, with the rounding of
-    the separate bf16 operations; differentiable in ``t``.  ``interleaved``: the pairs of ``t`` are adjacent elements."""
-    return _RopeSteps.apply(t, angles, float(mscale), bool(interleaved))
+    the separate bf16 operations, or the transpose of that map; differentiable in ``t`` any number of times.
+    ``interleaved``: the pairs of ``t`` are adjacent elements.  Tensors that are not :func:`ordinary` (a batched gradient, for
+    instance) take the separate operations."""
+    if ordinary(t, angles):
+        return _RopeSteps.apply(t, angles, float(mscale), bool(interleaved), bool(transpose))
+    half = t.shape[-1] // 2
+    f = angles[:t.shape[0]].reshape(t.shape[0], *([1] * (t.ndim - 2)), angles.shape[-1])
+    cos, sin = (torch.cos(f) * mscale).to(t.dtype), (torch.sin(f) * mscale).to(t.dtype)
+    if transpose:
+        u = t * sin
+        y = t * cos + torch.cat((u[..., half:], -u[..., :half]), dim=-1)
+        return torch.stack((y[..., :half], y[..., half:]), dim=-1).reshape(t.shape) if interleaved else y
+    if interleaved:
+        t = torch.cat((t[..., 0::2], t[..., 1::2]), dim=-1)
+    return t * cos + torch.cat((-t[..., half:], t[..., :half]), dim=-1) * sin
 
 
 HADAMARD_SIZES = (32, 64, 128, 256, 512)
@@ -201,11 +224,14 @@ class _Hadamard(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):
-        return _native().hadamard(grad.to(torch.bfloat16))
+        from .dsa_fused import rotate_activation      # this kernel, or tensor operations for what it does not take
+
+        return rotate_activation(grad.to(torch.bfloat16))
 
 
 def hadamard(x):
-    """bf16 rows of 32 .. 512 elements times the Hadamard matrix and ``n ** -0.5``; differentiable."""
+    """bf16 rows of 32 .. 512 elements (an :func:`ordinary` tensor) times the Hadamard matrix and ``n ** -0.5``; differentiable
+    any number of times."""
     return _Hadamard.apply(x)
 
 
@@ -320,15 +346,45 @@ def indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale: float, heads: 
     through the Hadamard rotation if ``rotate``, and with ``front`` (an ``IndexerFrontEnd``) through the rotary embedding
     and the LayerNorm of the keys (input ``k_in``, weight ``ln_weight``)."""
     f = front
+    if f is None and not ordinary(g, q8, k8, k_scale, q_w, ids, q_scale):
+        return _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, rotate)
     return _native().indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, float(w_scale), bool(rotate), f and f.cos, f and f.sin,
                                    f.pairing if f else -1, f and f.positions_q, f and f.positions_k, f.batch if f else 1,
                                    k_in, ln_weight, f.k_norm_eps if f else 0.0, int(heads), int(dim), *dtypes)
+
+
+def _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, rotate):
+    """:func:`indexer_grads` without a front end as the custom op and tensor operations, for traced and fake tensors."""
+    from .dsa_fused import _hadamard
+    from .dsa_fused_kernels import _unscale_indexer_grad
+
+    g = torch.where(ids >= 0, g.float(), torch.zeros_like(g, dtype=torch.float32))
+    d_q, d_k, d_w = indexer_bwd(g.contiguous(), q8, k8, k_scale, q_w, ids.int())
+    d_w, d_q, d_k = d_w * q_scale * w_scale, _unscale_indexer_grad(d_q, q_scale), _unscale_indexer_grad(d_k, k_scale)
+    if rotate:
+        h = _hadamard(128, d_q.device, torch.float32)
+        d_q, d_k = (d_q @ h) * 128 ** -0.5, (d_k @ h) * 128 ** -0.5
+    return d_q[:, :heads, :dim].to(dtypes[0]), d_k[:, :dim].to(dtypes[1]), d_w[:, :heads].to(dtypes[2]), None, None
+
+
+class _Unchecked:
+    def wait(self):
+        pass
 
 
 def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offset: int, like: torch.Tensor):
     """``(ks, ke, check)``: the key window of every causal query ``chunk_offset + i`` (int32, on ``like``'s device) over
     the packed sequences of ``cu_seqlens`` (None: one sequence).  ``check.wait()`` raises ValueError if the sequences
     end before the queries do; call it behind the launches that use the window."""
+    if not ordinary(cu_seqlens, like):
+        dev = like.device
+        ke = torch.arange(queries, dtype=torch.int32, device=dev) + chunk_offset + 1
+        if cu_seqlens is None:
+            return torch.zeros(queries, dtype=torch.int32, device=dev), ke, _Unchecked()
+        cu = cu_seqlens.to(dev)
+        lens = cu[1:] - cu[:-1]
+        seq = torch.repeat_interleave(torch.arange(len(lens), device=dev, dtype=torch.int32), lens)
+        return cu[seq[chunk_offset:chunk_offset + queries].long()].int(), ke, _Unchecked()
     return _native().indexer_window(cu_seqlens, int(queries), int(chunk_offset), like)
 
 

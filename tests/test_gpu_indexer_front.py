@@ -216,3 +216,35 @@ def test_hadamard_rotation_of_other_widths(gpu, n):
     for got, ref in ((y, x), (dx, dout)):
         want = ref.detach().double().cpu() @ h * n ** -0.5
         assert ((got.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_separate_operations_under_transforms(gpu, interleaved):
+    """What the tensor operations took before there were kernels: gradients of gradients, batched gradients, vmap, forward mode,
+    views that start inside a 16-byte piece."""
+    from types import SimpleNamespace
+
+    from loongforge_amd.dsa_fused import rotate_activation
+    from loongforge_amd.megatron_compat import RotaryEmbedding, apply_rotary_pos_emb
+
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(gpu)                  # noqa: E731
+    angles = RotaryEmbedding(64, 1.0).to(gpu)(9)
+    cfg = SimpleNamespace(multi_latent_attention=interleaved)
+    near = dict(rtol=2.0 ** -7, atol=2.0 ** -6)          # two roundings to bf16 of values up to 2
+    for f in (rotate_activation, lambda t: apply_rotary_pos_emb(t, angles, config=cfg)):
+        x, go, v = rnd(9, 2, 3, 64).requires_grad_(), rnd(9, 2, 3, 64).requires_grad_(), rnd(9, 2, 3, 64)
+        y = f(x)
+        (gx,) = torch.autograd.grad(y, x, go, create_graph=True)
+        (gg,) = torch.autograd.grad(gx, go, v)
+        assert torch.equal(gg, f(v))
+        rows = torch.stack([rnd(9, 2, 3, 64) for _ in range(2)])
+        (many,) = torch.autograd.grad(f(x), x, rows, is_grads_batched=True)
+        for i in range(2):
+            torch.testing.assert_close(many[i], torch.autograd.grad(f(x), x, rows[i])[0], **near)
+        torch.testing.assert_close(torch.func.vmap(f)(rows), torch.stack([f(r) for r in rows]), **near)
+        out, tangent = torch.func.jvp(f, (x.detach(),), (v,))
+        torch.testing.assert_close(out, y.detach(), **near)
+        torch.testing.assert_close(tangent, f(v), **near)
+    odd = rnd(4 * 64 + 1)[1:].view(4, 64)
+    assert torch.equal(rotate_activation(odd), rotate_activation(odd.clone()))
