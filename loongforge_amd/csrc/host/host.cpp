@@ -231,16 +231,24 @@ py::object rotary_cos_sin(const Tensor& inv_freq, int64_t n, double offset, at::
   return py::make_tuple(c, s);
 }
 
-// t [s, (b,) h, d] with unit stride inside rows -> contiguous result of the same shape
+// t [s, (b,) h, d] as rows [s * b, h][d] of unit stride with one token pitch, copied if it does not lie like that.  Where s or b
+// is 1 its stride says nothing, and contiguous() keeps it: [s, 1, h, d] out of a batch-first tensor has the whole sequence there.
+std::pair<Tensor, int64_t> token_rows(const Tensor& t) {
+  const bool one_pitch = t.dim() == 3 || t.size(0) == 1 || t.size(1) == 1 || t.stride(0) == t.size(1) * t.stride(1);
+  const Tensor x = t.stride(-1) == 1 && one_pitch ? t : t.contiguous();
+  return {x, x.dim() == 3 || x.size(1) == 1 ? x.stride(0) : x.stride(1)};
+}
+
+// -> contiguous result of t's shape
 Tensor rope_steps(const Tensor& t, const Tensor& angles, double mscale, bool interleaved, bool transpose) {
   need_gpus(t, angles);
-  const Tensor x = t.stride(-1) == 1 && (t.dim() == 3 || t.stride(0) == t.size(1) * t.stride(1)) ? t : t.contiguous();
+  const auto [x, pitch] = token_rows(t);
   const int64_t batch = x.dim() == 4 ? x.size(1) : 1, rows = x.size(0) * batch, d = x.size(-1), heads = x.size(-2);
   REQUIRE(x.scalar_type() == at::kBFloat16 && angles.scalar_type() == at::kFloat && angles.is_contiguous() && angles.size(-1) == d &&
           angles.size(0) >= x.size(0) && angles.numel() == angles.size(0) * d, "rope_steps: inconsistent arguments");
   Call call(x);
   Tensor y = make(x.sizes(), at::kBFloat16, x);
-  run("dsa_rope_steps", dsa_rope_steps, x.const_data_ptr(), x.dim() == 4 ? x.stride(1) : x.stride(0), x.stride(-2), out_ptr<void>(y), heads * d, d,
+  run("dsa_rope_steps", dsa_rope_steps, x.const_data_ptr(), pitch, x.stride(-2), out_ptr<void>(y), heads * d, d,
       (const float*)angles.const_data_ptr(), (float)mscale, (int)interleaved, (int)batch, rows, (int)heads, (int)d, (int)transpose, call.stream);
   return y;
 }
@@ -632,6 +640,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(quant_padded);
   DEF(rotary_angles);
   DEF(rotary_cos_sin);
+  DEF(token_rows);
   DEF(rope_steps);
   DEF(hadamard);
   DEF(indexer_topk);

@@ -203,6 +203,28 @@ def test_rope_in_rounded_steps_equals_the_separate_operations(gpu, shape, interl
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("batch", [1, 2])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_rope_in_rounded_steps_of_batch_first_views(gpu, batch, interleaved):
+    """[s, b, h, d] as a transposed view of [b, s, h, d], and a gradient that comes back through such a transpose: with one
+    sequence in the batch the view counts as contiguous and its batch stride is that of the whole sequence."""
+    from types import SimpleNamespace
+
+    from loongforge_amd.megatron_compat import RotaryEmbedding, apply_rotary_pos_emb
+
+    g = torch.Generator().manual_seed(9)
+    angles, cfg = RotaryEmbedding(64).to(gpu)(5), SimpleNamespace(multi_latent_attention=interleaved)
+    base, dout = (torch.randn(batch, 5, 2, 64, generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    res = []
+    for lay in (lambda t: t.transpose(0, 1), lambda t: t.transpose(0, 1).clone(memory_format=torch.contiguous_format)):
+        x = base.clone().requires_grad_(True)
+        y = apply_rotary_pos_emb(lay(x), angles, config=cfg)
+        res.append((y.detach(), torch.autograd.grad(y.transpose(0, 1), x, dout)[0]))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    one = torch.cat([apply_rotary_pos_emb(base[i], angles, config=cfg).unsqueeze(1) for i in range(batch)], 1)
+    assert torch.equal(res[0][0], one)
+
+
 @pytest.mark.parametrize("n", [32, 64, 128, 256, 512])
 def test_hadamard_rotation_of_other_widths(gpu, n):
     from loongforge_amd import dsa_fused

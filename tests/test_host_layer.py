@@ -1,0 +1,37 @@
+"""The native host layer's decisions that need no device: layouts, refusals."""
+import pytest
+import torch
+
+BF = torch.bfloat16
+
+
+def _views():
+    r = lambda *shape: torch.arange(torch.Size(shape).numel(), dtype=torch.float32).to(BF).view(shape)             # noqa: E731
+    yield "contiguous", r(5, 2, 3, 8)
+    yield "packed", r(5, 3, 8)
+    yield "one sequence, batch first", r(1, 5, 2, 64).transpose(0, 1)
+    yield "two sequences, batch first", r(2, 5, 2, 64).transpose(0, 1)
+    yield "one token, batch first", r(2, 1, 3, 8).transpose(0, 1)
+    yield "one token of one sequence", r(1, 1, 3, 8).as_strided((1, 1, 3, 8), (7, 5, 8, 1))
+    yield "one head, head first", r(1, 5, 2, 8).permute(1, 2, 0, 3)
+    yield "heads first", r(3, 5, 2, 8).permute(1, 2, 0, 3)
+    yield "leading part of a row", r(5, 2, 3, 12)[..., :8]
+    yield "every other element of a row", r(5, 2, 3, 16)[..., ::2]
+    yield "one sequence, batch first, leading part", r(1, 5, 2, 12).transpose(0, 1)[..., :8]
+    yield "every other token", r(10, 1, 3, 8)[::2]
+    yield "every other sequence", r(5, 4, 3, 8)[:, ::2]
+    yield "shared by the heads", r(5, 2, 1, 8).expand(5, 2, 3, 8)
+    yield "shared by the tokens", r(1, 1, 3, 8).expand(5, 1, 3, 8)
+
+
+@pytest.mark.parametrize("name,t", list(_views()), ids=lambda v: v if isinstance(v, str) else "")
+def test_rows_with_one_token_pitch_are_the_tensor(name, t):
+    """What the kernel reads at pitch * token + head stride * head + element is the tensor, and lies inside its storage."""
+    from loongforge_amd import _lib
+
+    x, pitch = _lib.load_host().token_rows(t)
+    tokens, (heads, d) = t.shape[:-2].numel(), t.shape[-2:]
+    assert x.stride(-1) == 1
+    last = x.storage_offset() + (tokens - 1) * pitch + (heads - 1) * x.stride(-2) + d - 1
+    assert last < x.untyped_storage().nbytes() // x.element_size()
+    assert torch.equal(x.as_strided((tokens, heads, d), (pitch, x.stride(-2), 1)), t.reshape(tokens, heads, d))
