@@ -561,10 +561,12 @@ void absorb_rope_query_into(const Tensor& q_up, const Tensor& w_, const Tensor& 
   run("dsa_absorb_rope_query", dsa_absorb_rope_query, q_up.const_data_ptr(), q_up.stride(0), q_up.stride(1), w.const_data_ptr(), query.data_ptr(), query.stride(0), query.stride(1), cos.const_data_ptr(), sin.const_data_ptr(), cos.scalar_type() == at::kFloat, (const int32_t*)ptr(positions), (int)batch, (int)S, (int)H, (int)out_pairing, call.stream);
 }
 
-// The two projections around the attention without autograd: output allocation and kernel in one call.
+// The two projections around the attention without autograd: output allocation and kernel in one call.  (The query side's kernel
+// has one shape; the other pair of widths that the projection takes goes through the two kernels.)
 py::object absorbed_query(const Tensor& q_up, const Tensor& w, const Tensor& cos, const Tensor& sin, const OptTensor& positions,
                           int64_t out_pairing) {
-  if (!plain(q_up, w, cos, sin, positions) || q_up.dim() < 3 || w.dim() != 3 || q_up.size(-1) != w.size(2) + 64) return py::none();
+  if (!plain(q_up, w, cos, sin, positions) || q_up.dim() < 3 || w.dim() != 3 || w.size(1) != 512 || w.size(2) != 128 ||
+      q_up.size(-1) != 192) return py::none();
   std::vector<int64_t> shape = q_up.sizes().vec();
   const int64_t batch = q_up.dim() == 4 ? q_up.size(1) : 1;
   const Tensor q3 = q_up.dim() == 3 ? q_up : q_up.reshape({-1, q_up.size(-2), q_up.size(-1)});

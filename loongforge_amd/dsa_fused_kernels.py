@@ -560,7 +560,7 @@ class FusedAbsorbRopeQuery(torch.autograd.Function):
         query = q_up.new_empty(S, nheads, d_out + emb)
         positions = _token_positions(cu_seqlens_q, S, cp_rank, cp_size)
         out_pairing = ops.ROPE_ADJACENT if rotary_interleaved else ops.ROPE_SPLIT
-        if emb == 64:
+        if (d_nope, d_out, emb) == (128, 512, 64):
             ops.absorb_rope_query_into(q3, w_uk_t, query, cos, sin, out_pairing, positions, batch)
         else:
             ops.mla_absorb_into(q3[:, :, :d_nope], w_uk_t, query[:, :, :d_out])

@@ -749,7 +749,8 @@ def absorb_rope_query_into(q_up: torch.Tensor, w: torch.Tensor, query: torch.Ten
 
 
 def absorbed_query(q_up, w, cos, sin, positions, out_pairing: int):
-    """:func:`absorb_rope_query_into` over ``q_up [.., H, 192]`` into a new ``[.., H, 576]``; None if that needs autograd."""
+    """:func:`absorb_rope_query_into` over ``q_up [.., H, 192]`` into a new ``[.., H, 576]``; None if that needs autograd or
+    the widths are others."""
     return _native().absorbed_query(q_up, w, cos, sin, positions, int(out_pairing))
 
 

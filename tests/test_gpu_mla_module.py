@@ -80,6 +80,24 @@ def test_absorb_and_rope_in_one_kernel(gpu, S, H, pairing, dtype):
         assert torch.equal(query, ref)
 
 
+@pytest.mark.parametrize("n,k,emb", [(512, 128, 64), (128, 512, 64), (512, 128, 32)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_absorbed_query_of_every_supported_width(gpu, n, k, emb, grad):
+    """The widths of the fused kernel and the others that the projection and the rotary kernel take: bit-equal to these two."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import fused_absorb_rope_query
+
+    g = torch.Generator().manual_seed(n)
+    q_up = torch.randn(9, 2, 3, k + emb, generator=g).to(torch.bfloat16).to(gpu).requires_grad_(grad)
+    w = (torch.randn(3, n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(gpu)
+    cos, sin = (torch.randn(9, emb, generator=g).to(gpu) for _ in range(2))
+    query = fused_absorb_rope_query(q_up, w, cos, sin)
+    q3, ref = q_up.detach().view(18, 3, k + emb), torch.zeros(18, 3, n + emb, dtype=torch.bfloat16, device=gpu)
+    ops.mla_absorb_into(q3[:, :, :k], w, ref[:, :, :n])
+    ops.rope_rows(q3[:, :, k:], ref[:, :, n:], cos, sin, ops.ROPE_ADJACENT, ops.ROPE_SPLIT, False, None, 2)
+    assert query.requires_grad == grad and torch.equal(query.detach().view(18, 3, n + emb), ref)
+
+
 class _Linear(torch.nn.Module):
     def __init__(self, n_in, n_out, **_):
         super().__init__()

@@ -35,3 +35,11 @@ def test_rows_with_one_token_pitch_are_the_tensor(name, t):
     last = x.storage_offset() + (tokens - 1) * pitch + (heads - 1) * x.stride(-2) + d - 1
     assert last < x.untyped_storage().nbytes() // x.element_size()
     assert torch.equal(x.as_strided((tokens, heads, d), (pitch, x.stride(-2), 1)), t.reshape(tokens, heads, d))
+
+
+@pytest.mark.parametrize("n,k,emb", [(128, 512, 64), (512, 128, 32)])
+def test_absorbed_query_leaves_other_widths_to_the_two_kernels(n, k, emb):
+    from loongforge_amd import ops
+
+    q_up, w = torch.zeros(3, 2, k + emb, dtype=BF), torch.zeros(2, n, k, dtype=BF)
+    assert ops.absorbed_query(q_up, w, torch.zeros(3, emb), torch.zeros(3, emb), None, ops.ROPE_SPLIT) is None
