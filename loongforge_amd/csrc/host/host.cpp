@@ -147,6 +147,7 @@ py::object indexer_front(const Tensor& x_, int64_t rows_per_token, const OptTens
                          bool rotate, const OptTensor& weights_, double factor, bool want_payload, bool want_rows, double eps, bool pow2,
                          bool force) {
   PLAIN_OR_NONE(x_, ln_weight_, ln_bias_, cos_, sin_, positions_, weights_);
+  REQUIRE(batch > 0, "indexer_front_e4m3: batch must be positive, got ", batch);       // (divided by below)
   need_gpus(x_, ln_weight_, ln_bias_, cos_, sin_, positions_, weights_);
   REQUIRE(x_.scalar_type() == at::kBFloat16 && x_.size(-1) == 128, "indexer_front_e4m3 expects bf16 rows of 128 elements");
   const Tensor x = x_.contiguous();

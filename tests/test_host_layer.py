@@ -43,3 +43,13 @@ def test_absorbed_query_leaves_other_widths_to_the_two_kernels(n, k, emb):
 
     q_up, w = torch.zeros(3, 2, k + emb, dtype=BF), torch.zeros(2, n, k, dtype=BF)
     assert ops.absorbed_query(q_up, w, torch.zeros(3, emb), torch.zeros(3, emb), None, ops.ROPE_SPLIT) is None
+
+
+def test_indexer_front_end_refuses_an_empty_batch():
+    """The positions' default is token // batch: no batch is an error of the caller's, not a division by zero."""
+    from loongforge_amd import ops
+
+    x, table = torch.zeros(4, 128, dtype=BF), torch.zeros(4, 64)
+    for batch in (0, -1):
+        with pytest.raises(ValueError, match="batch must be positive"):
+            ops.indexer_front_e4m3(x, cos=table, sin=table, pairing=ops.ROPE_SPLIT, batch=batch)
