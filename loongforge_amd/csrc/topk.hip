@@ -664,7 +664,7 @@ static int fused_block_rows(int Sk) {
   // one block's logits stay within the 256 MiB memory-side cache where that still leaves a block 8192 queries:
   // 1024 workgroups of 8 queries, four rounds over the 256 compute units (blocks of 2048 queries - one workgroup per
   // compute unit, half of what fits - took 2.6 ms for 32768 packed tokens where blocks of 8192 take 1.9 ms)
-  long rows = (256l << 20) / ((long)Sk * 4);
+  long rows = (256l << 20) / ((long)(Sk > 0 ? Sk : 1) * 4);         // (no keys: refused by the logits kernel's checks)
   rows = rows < 8192 ? 8192 : rows;
   return (int)(rows / 8 * 8);
 }

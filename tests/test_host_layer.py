@@ -53,3 +53,13 @@ def test_indexer_front_end_refuses_an_empty_batch():
     for batch in (0, -1):
         with pytest.raises(ValueError, match="batch must be positive"):
             ops.indexer_front_e4m3(x, cos=table, sin=table, pairing=ops.ROPE_SPLIT, batch=batch)
+
+
+def test_workspace_of_an_indexer_without_keys():
+    """The size is asked for before the arguments are checked: no keys must not be divided by."""
+    from loongforge_amd import _lib
+
+    lib = _lib.load()
+    assert lib.dsa_indexer_topk_workspace_bytes(5, 0, 64) == 0
+    with pytest.raises(ValueError, match="Sk=0"):
+        _lib.check(lib.dsa_indexer_topk_fwd(None, None, None, None, None, None, 5, 64, 0, 64, 1, None, None, 256, 0, None), "no keys")
