@@ -235,6 +235,7 @@ py::object rotary_cos_sin(const Tensor& inv_freq, int64_t n, double offset, at::
 // t [s, (b,) h, d] as rows [s * b, h][d] of unit stride with one token pitch, copied if it does not lie like that.  Where s or b
 // is 1 its stride says nothing, and contiguous() keeps it: [s, 1, h, d] out of a batch-first tensor has the whole sequence there.
 std::pair<Tensor, int64_t> token_rows(const Tensor& t) {
+  REQUIRE(t.dim() == 3 || t.dim() == 4, "expected [s, h, d] or [s, b, h, d], got ", t.sizes());
   const bool one_pitch = t.dim() == 3 || t.size(0) == 1 || t.size(1) == 1 || t.stride(0) == t.size(1) * t.stride(1);
   const Tensor x = t.stride(-1) == 1 && one_pitch ? t : t.contiguous();
   return {x, x.dim() == 3 || x.size(1) == 1 ? x.stride(0) : x.stride(1)};
@@ -242,8 +243,8 @@ std::pair<Tensor, int64_t> token_rows(const Tensor& t) {
 
 // -> contiguous result of t's shape
 Tensor rope_steps(const Tensor& t, const Tensor& angles, double mscale, bool interleaved, bool transpose) {
-  need_gpus(t, angles);
   const auto [x, pitch] = token_rows(t);
+  need_gpus(x, angles);
   const int64_t batch = x.dim() == 4 ? x.size(1) : 1, rows = x.size(0) * batch, d = x.size(-1), heads = x.size(-2);
   REQUIRE(x.scalar_type() == at::kBFloat16 && angles.scalar_type() == at::kFloat && angles.is_contiguous() && angles.size(-1) == d &&
           angles.size(0) >= x.size(0) && angles.numel() == angles.size(0) * d, "rope_steps: inconsistent arguments");

@@ -37,6 +37,15 @@ def test_rows_with_one_token_pitch_are_the_tensor(name, t):
     assert torch.equal(x.as_strided((tokens, heads, d), (pitch, x.stride(-2), 1)), t.reshape(tokens, heads, d))
 
 
+@pytest.mark.parametrize("shape", [(8,), (5, 8), (2, 5, 2, 3, 8)])
+def test_rope_in_rounded_steps_refuses_other_dimensions(shape):
+    """Two dimensions would be walked as if the tokens were heads as well, behind the storage."""
+    from loongforge_amd import ops
+
+    with pytest.raises(ValueError, match="expected"):
+        ops.rope_steps(torch.zeros(shape, dtype=BF), torch.zeros(5, 1, 1, 8))
+
+
 @pytest.mark.parametrize("n,k,emb", [(128, 512, 64), (512, 128, 32)])
 def test_absorbed_query_leaves_other_widths_to_the_two_kernels(n, k, emb):
     from loongforge_amd import ops
