@@ -250,6 +250,7 @@ Tensor rope_steps(const Tensor& t, const Tensor& angles, double mscale, bool int
           angles.size(0) >= x.size(0) && angles.numel() == angles.size(0) * d, "rope_steps: inconsistent arguments");
   Call call(x);
   Tensor y = make(x.sizes(), at::kBFloat16, x);
+  if (x.numel() == 0) return y;
   run("dsa_rope_steps", dsa_rope_steps, x.const_data_ptr(), pitch, x.stride(-2), out_ptr<void>(y), heads * d, d,
       (const float*)angles.const_data_ptr(), (float)mscale, (int)interleaved, (int)batch, rows, (int)heads, (int)d, (int)transpose, call.stream);
   return y;

@@ -225,6 +225,20 @@ def test_rope_in_rounded_steps_of_batch_first_views(gpu, batch, interleaved):
     assert torch.equal(res[0][0], one)
 
 
+@pytest.mark.parametrize("shape", [(0, 1, 2, 64), (5, 0, 2, 64), (5, 1, 0, 64), (0, 2, 64)])
+def test_rotary_embedding_and_rotation_of_nothing(gpu, shape):
+    """Empty tensors go through, forward and backward, as through the tensor operations."""
+    from loongforge_amd.dsa_fused import rotate_activation
+    from loongforge_amd.megatron_compat import RotaryEmbedding, apply_rotary_pos_emb
+
+    x = torch.zeros(shape, dtype=torch.bfloat16, device=gpu, requires_grad=True)
+    angles = RotaryEmbedding(64).to(gpu)(5)
+    for f in (rotate_activation, lambda t: apply_rotary_pos_emb(t, angles)):
+        y = f(x)
+        assert y.shape == x.shape and y.dtype == x.dtype
+        assert torch.autograd.grad(y, x, torch.zeros_like(y))[0].shape == x.shape
+
+
 @pytest.mark.parametrize("n", [32, 64, 128, 256, 512])
 def test_hadamard_rotation_of_other_widths(gpu, n):
     from loongforge_amd import dsa_fused
