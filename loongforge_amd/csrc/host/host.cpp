@@ -213,8 +213,12 @@ py::tuple quant_padded(const Tensor& x_, int64_t heads_out, const OptTensor& wei
 }
 
 // ---- separate operations of the indexer's front end ---------------------------------------------------
+bool frequencies(const Tensor& t) {
+  return t.is_cuda() && plain(t) && t.scalar_type() == at::kFloat && t.dim() == 1 && t.numel() > 0 && t.is_contiguous();
+}
+
 py::object rotary_angles(const Tensor& inv_freq, int64_t n, double offset) {
-  if (!inv_freq.is_cuda() || !plain(inv_freq) || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous()) return py::none();
+  if (!frequencies(inv_freq)) return py::none();
   Call call(inv_freq);
   Tensor a = make({n, 1, 1, 2 * inv_freq.numel()}, at::kFloat, inv_freq);
   run("dsa_rotary_tables", dsa_rotary_tables, (const float*)inv_freq.const_data_ptr(), (int)inv_freq.numel(), (int)n, (float)offset, 0,
@@ -223,8 +227,7 @@ py::object rotary_angles(const Tensor& inv_freq, int64_t n, double offset) {
 }
 
 py::object rotary_cos_sin(const Tensor& inv_freq, int64_t n, double offset, at::ScalarType type) {
-  if (!inv_freq.is_cuda() || !plain(inv_freq) || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous() ||
-      (type != at::kFloat && type != at::kBFloat16)) return py::none();
+  if (!frequencies(inv_freq) || (type != at::kFloat && type != at::kBFloat16)) return py::none();
   Call call(inv_freq);
   Tensor c = make({n, 1, 1, 2 * inv_freq.numel()}, type, inv_freq), s = at::empty_like(c);
   run("dsa_rotary_tables", dsa_rotary_tables, (const float*)inv_freq.const_data_ptr(), (int)inv_freq.numel(), (int)n, (float)offset,

@@ -172,13 +172,18 @@ def quant_padded_e4m3(x, heads: int, weights=None, factor: float = 1.0):
 # separate operations of the indexer's front end
 # --------------------------------------------------------------------------------------------
 def rotary_angles(inv_freq, n: int, offset: float = 0.0):
-    """``[n, 1, 1, dim]`` angles ``(i + offset) * inv_freq`` (twice side by side), one kernel; None for tensors it does not take."""
-    return _native().rotary_angles(inv_freq, int(n), float(offset))
+    """``[n, 1, 1, dim]`` angles ``(i + offset) * inv_freq`` (twice side by side), one kernel; None for arguments it does not take
+    (other tensors, a length that is no integer, an offset on the device or one per position)."""
+    if not isinstance(n, int) or not isinstance(offset, (int, float)):
+        return None
+    return _native().rotary_angles(inv_freq, n, float(offset))
 
 
 def rotary_cos_sin(inv_freq, n: int, offset: float, dtype):
-    """Cosines and sines of :func:`rotary_angles` in ``dtype`` (fp32 or bf16), one kernel; None for tensors it does not take."""
-    return _native().rotary_cos_sin(inv_freq, int(n), float(offset), dtype)
+    """Cosines and sines of :func:`rotary_angles` in ``dtype`` (fp32 or bf16), one kernel; None for arguments it does not take."""
+    if not isinstance(n, int) or not isinstance(offset, (int, float)):
+        return None
+    return _native().rotary_cos_sin(inv_freq, n, float(offset), dtype)
 
 
 class _RopeSteps(torch.autograd.Function):

@@ -225,6 +225,21 @@ def test_rope_in_rounded_steps_of_batch_first_views(gpu, batch, interleaved):
     assert torch.equal(res[0][0], one)
 
 
+def test_rotary_angles_with_other_arguments(gpu):
+    """Lengths, offsets and frequencies that the kernel does not take give what the tensor operations give."""
+    from loongforge_amd.megatron_compat import RotaryEmbedding
+
+    rot, ref = RotaryEmbedding(64).to(gpu), RotaryEmbedding(64)
+    offsets = torch.tensor([7.0, 7.0, 3.0, 0.5])
+    for length, offset in ((4, offsets), (4, torch.tensor(9.0)), (3.5, 2), (0, 0)):
+        got = rot(length, offset.to(gpu) if torch.is_tensor(offset) else offset)
+        assert torch.equal(got.cpu(), ref(length, offset))
+    assert RotaryEmbedding(0).to(gpu)(4).shape == (4, 1, 1, 0)
+    with pytest.raises(RuntimeError):
+        rot.inv_freq = rot.inv_freq.view(2, 16)
+        rot(4)
+
+
 @pytest.mark.parametrize("shape", [(0, 1, 2, 64), (5, 0, 2, 64), (5, 1, 0, 64), (0, 2, 64)])
 def test_rotary_embedding_and_rotation_of_nothing(gpu, shape):
     """Empty tensors go through, forward and backward, as through the tensor operations."""
