@@ -138,7 +138,7 @@ def apply_rotary_pos_emb(t, freqs, config=None, cu_seqlens=None, mscale=1.0, cp_
     positions restart at every document (packed layout ``[t, h, d]``).  When
     ``config.multi_latent_attention`` is set the input is de-interleaved first, as Megatron does."""
     interleaved_in = bool(getattr(config, "multi_latent_attention", False))
-    if (cu_seqlens is None and t.is_cuda and t.dtype == torch.bfloat16 and t.ndim in (3, 4) and t.shape[-1] % 2 == 0
+    if (cu_seqlens is None and isinstance(mscale, (int, float)) and t.is_cuda and t.dtype == torch.bfloat16 and t.ndim in (3, 4) and t.shape[-1] % 2 == 0
             and freqs.dtype == torch.float32 and freqs.is_contiguous() and not freqs.requires_grad
             and freqs.shape[-1] == t.shape[-1] and freqs.shape[0] >= t.shape[0] and freqs.numel() == freqs.shape[0] * freqs.shape[-1]):
         from . import ops

@@ -240,6 +240,22 @@ def test_rotary_angles_with_other_arguments(gpu):
         rot(4)
 
 
+def test_rotary_embedding_with_a_scale_on_the_device(gpu):
+    """A scale that is a tensor gets its gradient and is not read on the host."""
+    from loongforge_amd.megatron_compat import RotaryEmbedding, apply_rotary_pos_emb
+
+    x = torch.randn(5, 2, 3, 64, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(gpu)
+    angles = RotaryEmbedding(64).to(gpu)(5)
+    scale = torch.tensor(1.25, device=gpu, requires_grad=True)
+    y = apply_rotary_pos_emb(x, angles, mscale=scale)
+    assert torch.equal(y.detach(), apply_rotary_pos_emb(x, angles, mscale=1.25))
+    (got,) = torch.autograd.grad(y.double().sum(), scale)
+    half = x.double().roll(32, -1) * torch.cat((-torch.ones(32), torch.ones(32))).to(gpu)
+    terms = x.double() * angles.double().cos() + half * angles.double().sin()
+    # sums and gradients pass through bf16: per term a few roundings, and the sum over tokens and heads one per addend
+    assert (got.double() - terms.sum()).abs() <= 2.0 ** -5 * terms.abs().sum()
+
+
 @pytest.mark.parametrize("shape", [(0, 1, 2, 64), (5, 0, 2, 64), (5, 1, 0, 64), (0, 2, 64)])
 def test_rotary_embedding_and_rotation_of_nothing(gpu, shape):
     """Empty tensors go through, forward and backward, as through the tensor operations."""
