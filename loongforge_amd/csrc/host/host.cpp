@@ -50,14 +50,23 @@ bool ordinary(const std::vector<OptTensor>& tensors) {
 #define PLAIN_OR_NONE(...) do { if (!force && !plain(__VA_ARGS__)) return py::none(); } while (0)
 
 // ---- checks ---------------------------------------------------------------------------------------
-void need_gpu(const Tensor& t) {
-  TORCH_CHECK(t.is_cuda(), "DSA kernels need tensors on a HIP device; got a ", c10::DeviceTypeName(t.device().type(), true), " tensor");
-  // (fake tensors and wrappers of transforms have a device but no memory)
-  TORCH_CHECK(t.numel() == 0 || (t.has_storage() && t.storage().data() != nullptr), "DSA kernels need tensors with memory of their own");
-}
-void need_gpu(const OptTensor& t) { if (t) need_gpu(*t); }
+const Tensor* present(const Tensor& t) { return &t; }
+const Tensor* present(const OptTensor& t) { return t ? &*t : nullptr; }
+// All tensors that a kernel is given: with memory, on one device.
 template <class... T>
-void need_gpus(const T&... t) { (need_gpu(t), ...); }
+void need_gpus(const T&... t) {
+  const Tensor* const all[] = {present(t)...};
+  const Tensor* first = nullptr;
+  for (const Tensor* p : all) {
+    if (!p) continue;
+    TORCH_CHECK(p->is_cuda(), "DSA kernels need tensors on a HIP device; got a ", c10::DeviceTypeName(p->device().type(), true), " tensor");
+    if (!first) first = p;
+    TORCH_CHECK(p->device() == first->device(), "DSA kernels need tensors on one device; got ", first->device(), " and ", p->device());
+  }
+  // (fake tensors and wrappers of transforms have a device but no memory)
+  for (const Tensor* p : all)
+    TORCH_CHECK(!p || p->numel() == 0 || (p->has_storage() && p->storage().data() != nullptr), "DSA kernels need tensors with memory of their own");
+}
 
 void check(int rc, const char* what) {
   if (rc == 0) return;
@@ -342,7 +351,7 @@ py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, 
                         const Tensor& q_scale_, double w_scale, bool rotate, const OptTensor& cos_, const OptTensor& sin_, int64_t pairing,
                         const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& k_in, const OptTensor& ln_w_,
                         double ln_eps, int64_t heads, int64_t dim, at::ScalarType q_type, at::ScalarType k_type, at::ScalarType w_type) {
-  need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_, q_scale_);
+  need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_, q_scale_, cos_, sin_, positions_q, positions_k, k_in, ln_w_);
   const int64_t S = q8_.size(0), Hi = q8_.size(1), Sk = k8_.size(0);
   REQUIRE(ids_.dim() == 2 && g_.sizes() == ids_.sizes() && ids_.size(0) == S && q_scale_.numel() == S * Hi,
           "indexer_grads: grad and ids must both be [S, K], q_scale [S, H]");
@@ -459,7 +468,7 @@ py::object mla_fwd(const Tensor& q_, const Tensor& kv_, const Tensor& ids_, int6
   const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);
   OptTensor sink;
   if (attn_sink) {
-    need_gpus(attn_sink);
+    need_gpus(q, attn_sink);
     REQUIRE(attn_sink->numel() == H, "attn_sink must hold one logit per head (", H, "), got ", attn_sink->numel());
     sink = f32(attn_sink->reshape({H}));
   }
@@ -480,7 +489,7 @@ py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, cons
                    int64_t q_start, double sm_scale, int64_t d_v, const py::function& workspace, bool force) {
   PLAIN_OR_NONE(q_, kv_, out_, dout_, ids_, lse_);
   mla_shape(q_, kv_, ids_);
-  need_gpus(out_, dout_, lse_);
+  need_gpus(q_, out_, dout_, lse_);
   const Tensor q = q_.contiguous(), kv = kv_.contiguous(), ids = i32(ids_), out = out_.contiguous(), lse = f32(lse_);
   const Tensor dout = dout_.to(at::kBFloat16).contiguous();
   const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);

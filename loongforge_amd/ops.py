@@ -54,9 +54,12 @@ def _stream(t: torch.Tensor):
 
 
 def _need_gpu(*tensors):
+    tensors = [t for t in tensors if t is not None]
     for t in tensors:
-        if t is not None and not t.is_cuda:
+        if not t.is_cuda:
             raise RuntimeError("DSA kernels need tensors on a HIP device; got a %s tensor" % t.device.type)
+        if t.device != tensors[0].device:
+            raise RuntimeError("DSA kernels need tensors on one device; got %s and %s" % (tensors[0].device, t.device))
 
 
 def _c(t: torch.Tensor) -> torch.Tensor:
@@ -446,7 +449,7 @@ def _mla_fwd_dist_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, q_sta
     S, H, _ = q.shape
     K = ids.shape[1]
     if attn_sink is not None:
-        _need_gpu(attn_sink)
+        _need_gpu(q, attn_sink)
         attn_sink = _c(attn_sink.float().reshape(H))
     out = torch.empty(S, H, d_v, dtype=torch.bfloat16, device=q.device)
     lse = torch.empty(S, H, dtype=torch.float32, device=q.device)

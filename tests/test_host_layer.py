@@ -72,3 +72,23 @@ def test_workspace_of_an_indexer_without_keys():
     assert lib.dsa_indexer_topk_workspace_bytes(5, 0, 64) == 0
     with pytest.raises(ValueError, match="Sk=0"):
         _lib.check(lib.dsa_indexer_topk_fwd(None, None, None, None, None, None, 5, 64, 0, 64, 1, None, None, 256, 0, None), "no keys")
+
+
+def test_tensors_of_one_call_live_on_one_device():
+    """A kernel would read the other device's memory.  (Fake tensors: two devices without any.)"""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from loongforge_amd import _lib, ops
+
+    with FakeTensorMode():
+        new = lambda *shape, dtype=BF, dev=0: torch.empty(shape, dtype=dtype, device="cuda:%d" % dev)             # noqa: E731
+        t, angles = new(5, 1, 2, 64), new(5, 1, 1, 64, dtype=torch.float32, dev=1)
+        p, cos = new(5, 2, 64), new(5, 64, dtype=torch.float32, dev=1)
+        logits, k8 = new(5, 32, 128, dtype=torch.uint8), new(9, 128, dtype=torch.uint8, dev=1)
+    host = _lib.load_host()
+    with pytest.raises(RuntimeError, match="on one device; got cuda:0 and cuda:1"):
+        host.rope_steps(t, angles, 1.0, False, False)
+    with pytest.raises(RuntimeError, match="on one device; got cuda:0 and cuda:1"):
+        ops.rope_rows(p, p, cos, cos, 0, 0)
+    with pytest.raises(RuntimeError, match="on one device; got cuda:0 and cuda:1"):
+        ops._need_gpu(None, logits, None, k8)
