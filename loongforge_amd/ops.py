@@ -586,7 +586,7 @@ def attn_dist(p_out, sm_scale: float):
 @torch.library.custom_op("dsa::attn_dist_qk", mutates_args=())
 def _attn_dist_qk_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, lse: torch.Tensor, q_start: int,
                      sm_scale: float, heads_in_mean: int) -> torch.Tensor:
-    _need_gpu(q)
+    _need_gpu(q, kv, ids, lse)
     if q.ndim != 3 or q.shape[-1] != 576 or q.dtype != torch.bfloat16:
         raise ValueError("attn_dist_qk expects q [S,H,576] in bf16")
     if kv.ndim != 2 or kv.shape[-1] != 576 or kv.dtype != torch.bfloat16:

@@ -484,3 +484,14 @@ def test_random_shapes_forward_backward_distribution(gpu):
         target = ops.attn_dist_qk(q, kv, idx, lse, q_start, inp.sm_scale, H)
         ref = O.attn_dist_from_lse(inp.q, inp.kv, inp.idx, lse.cpu(), q_start, inp.sm_scale, H)
         assert_close(target, ref, name + " attn_dist", atol=1e-3, rtol=1e-2)
+
+
+def test_recomputed_distribution_refuses_host_tensors(gpu):
+    """Keys, ids and statistics are read by the kernel as well as the queries: none of them may be host memory."""
+    from loongforge_amd import ops
+
+    args = [torch.zeros(4, 32, 576, dtype=torch.bfloat16), torch.zeros(9, 576, dtype=torch.bfloat16), torch.zeros(4, 64, dtype=torch.int32),
+            torch.zeros(4, 32)]
+    for host in range(4):
+        with pytest.raises(RuntimeError, match="HIP device"):
+            ops.attn_dist_qk(*[t if i == host else t.to(gpu) for i, t in enumerate(args)], 0, 0.1)
