@@ -45,14 +45,26 @@ def _deps():
             + [os.path.join(HERE, "mla_bwd.hip")])          # csrc/bench/bwd_profile.hip includes it
 
 
+def _run_if_stale(cmd, obj, inputs, force, built_for=""):
+    """Runs the compiler unless ``obj`` is newer than its inputs and came out of the same command (and of the same ``built_for``:
+    what it depends on besides); returns the result or None."""
+    made, record = "\n".join([built_for] + cmd), obj + ".cmd"
+    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= max(os.path.getmtime(p) for p in inputs):
+        if os.path.exists(record) and open(record).read() == made:
+            return None
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode == 0:
+        with open(record, "w") as f:
+            f.write(made)
+    return res
+
+
 def _compile(src, force):
     prefix = "bench_" if os.path.basename(os.path.dirname(src)) == "bench" else ""
     obj = os.path.join(OBJ_DIR, prefix + os.path.basename(src)[:-4] + ".o")
-    newest = max(os.path.getmtime(p) for p in [src] + _deps())
-    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= newest:
+    res = _run_if_stale([HIPCC] + FLAGS + ["-c", src, "-o", obj], obj, [src] + _deps(), force)
+    if res is None:
         return obj, ""
-    cmd = [HIPCC] + FLAGS + ["-c", src, "-o", obj]
-    res = subprocess.run(cmd, capture_output=True, text=True)
     log = "\n".join(l for l in (res.stdout + res.stderr).splitlines() if "not a recognized feature" not in l)
     if res.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s" % (src, log))
@@ -60,18 +72,18 @@ def _compile(src, force):
 
 
 def _compile_host(force):
-    """csrc/host/host.cpp -> object file (host code only: g++)."""
-    src, obj = os.path.join(HERE, "host", "host.cpp"), os.path.join(OBJ_DIR, "host.o")
-    newest = max(os.path.getmtime(p) for p in [src, os.path.join(os.path.dirname(PKG), "include", "dsa_hip.h")])
-    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= newest:
-        return obj
+    """csrc/host/host.cpp -> object file (host code only: g++).  An extension works with the torch it was compiled against."""
+    import torch
     from torch.utils.cpp_extension import include_paths
 
+    src, obj = os.path.join(HERE, "host", "host.cpp"), os.path.join(OBJ_DIR, "host.o")
     includes = include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"]]
-    res = subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
-                          "-DUSE_ROCM", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_dsa_host"]
-                         + ["-I" + p for p in includes] + ["-c", src, "-o", obj], capture_output=True, text=True)
-    if res.returncode != 0:
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+           "-DUSE_ROCM", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_dsa_host"]
+    cmd += ["-I" + p for p in includes] + ["-c", src, "-o", obj]
+    res = _run_if_stale(cmd, obj, [src, os.path.join(os.path.dirname(PKG), "include", "dsa_hip.h")], force,
+                        "torch %s, python %s" % (torch.__version__, sys.version))
+    if res is not None and res.returncode != 0:
         raise RuntimeError("compiling host.cpp failed:\n" + res.stdout + res.stderr)
     return obj
 

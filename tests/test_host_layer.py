@@ -92,3 +92,29 @@ def test_tensors_of_one_call_live_on_one_device():
         ops.rope_rows(p, p, cos, cos, 0, 0)
     with pytest.raises(RuntimeError, match="on one device; got cuda:0 and cuda:1"):
         ops._need_gpu(None, logits, None, k8)
+
+
+def test_host_layer_is_rebuilt_for_another_torch(tmp_path, monkeypatch):
+    """An extension compiled against another torch does not load; a build without --force has to notice."""
+    from types import SimpleNamespace
+
+    from loongforge_amd.csrc import build
+
+    runs = []
+
+    def compiler(cmd, **_):
+        runs.append(cmd)
+        open(cmd[cmd.index("-o") + 1], "w").close()
+        return SimpleNamespace(returncode=0, stdout="", stderr="")
+
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path))
+    monkeypatch.setattr(build.subprocess, "run", compiler)
+    for version, compiles in (("1.0", 1), ("1.0", 1), ("1.1", 2), ("1.1", 2)):
+        monkeypatch.setattr(torch, "__version__", version)
+        build._compile_host(False)
+        assert len(runs) == compiles, version
+    monkeypatch.setenv("CXX", "another")
+    build._compile_host(False)
+    assert len(runs) == 3
+    build._compile_host(True)
+    assert len(runs) == 4
