@@ -204,7 +204,8 @@ int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const floa
 /*
  * Windows of the causal queries [chunk_offset, chunk_offset + S) over packed sequences, cu[ncu] (i32, or i64 if cu_i64)
  * their cumulative lengths (NULL: one sequence): ks[i] = start of the query's sequence, ke[i] = chunk_offset + i + 1;
- * queries past the last sequence get ks = 0.  total (may be NULL; host-visible): the summed length of the sequences.
+ * queries past the last sequence get ks = ke = 0, an empty window.  total (may be NULL; host-visible): the summed length of
+ * the sequences, -1 if the cumulative lengths decrease somewhere.
  */
 int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, int chunk_offset, int32_t* ks, int32_t* ke,
                        int32_t* total, void* stream);

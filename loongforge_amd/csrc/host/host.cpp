@@ -390,7 +390,7 @@ py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, 
 // ---- windows of packed sequences ------------------------------------------------------------------------
 // Whether the sequences cover the queries is only known on the device; the kernel leaves their length in pinned memory
 // and wait() looks at it, called after the kernels that use the window were launched: the device has work while the
-// host waits.  (Under graph capture nothing is checked.)
+// host waits.  Under graph capture nothing can be checked: queries that no sequence holds then have empty windows.
 struct WindowCheck {
   Tensor total;
   int64_t need = 0;
@@ -406,6 +406,7 @@ struct WindowCheck {
       rc = hipEventSynchronize(done);
     }
     TORCH_CHECK(rc == hipSuccess, "indexer window: ", hipGetErrorString(rc));
+    REQUIRE(*total.const_data_ptr<int>() >= 0, "indexer: the cumulative lengths of the packed sequences decrease");
     REQUIRE(*total.const_data_ptr<int>() >= need, "indexer: inconsistent shapes (the packed sequences hold ", *total.const_data_ptr<int>(),
             " tokens, the queries end at ", need, ")");
   }
@@ -421,10 +422,11 @@ py::tuple indexer_window(const OptTensor& cu_, int64_t S, int64_t chunk_offset, 
   need_gpus(like);
   OptTensor cu;
   if (cu_) cu = seqlens(*cu_, like.device());
+  REQUIRE(!cu || S == 0 || cu->numel() > 1, "indexer: inconsistent shapes (no packed sequence)");
   Call call(like);
   Tensor window = make({2, S}, at::kInt, like);
   auto check = std::make_unique<WindowCheck>();
-  if (cu) {
+  if (cu && S > 0) {
     hipStreamCaptureStatus capturing;
     if (hipStreamIsCapturing((hipStream_t)call.stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
       check->total = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));

@@ -16,19 +16,26 @@ __device__ __forceinline__ int sequence_of(const T* cu, int ncu, long long t) {
   return lo;
 }
 
+// A query behind the last sequence has an empty window, not the keys of another sequence: nothing stops a captured launch.
 template <typename T>
-__global__ void window_kernel(const T* __restrict__ cu, int ncu, int S, int chunk_offset, int* __restrict__ ks, int* __restrict__ ke,
-                              int* __restrict__ total) {
+__global__ __launch_bounds__(256) void window_kernel(const T* __restrict__ cu, int ncu, int S, int chunk_offset, int* __restrict__ ks,
+                                                     int* __restrict__ ke, int* __restrict__ total) {
+  if (total && blockIdx.x == 0) {
+    bool falls = false;
+    for (int k = threadIdx.x; k + 1 < ncu; k += blockDim.x) falls |= cu[k + 1] < cu[k];
+    falls = __syncthreads_or(falls);
+    if (threadIdx.x == 0) *total = falls ? -1 : ncu > 0 ? (int)min((long long)cu[ncu - 1] - (long long)cu[0], 0x7fffffffll) : 0;
+  }
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0 && total) *total = ncu > 0 ? (int)(cu[ncu - 1] - cu[0]) : 0;
   if (i >= S) return;
-  int start = 0;
-  if (ncu > 1) {
+  int start = 0, end = chunk_offset + i + 1;
+  if (ncu > 0) {
     const int seq = sequence_of(cu, ncu, (long long)i + chunk_offset + (long long)cu[0]);   // lengths count from cu[0]
     if (seq < ncu - 1) start = (int)cu[seq];
+    else end = 0;
   }
   ks[i] = start;
-  ke[i] = chunk_offset + i + 1;
+  ke[i] = end;
 }
 
 template <typename T>

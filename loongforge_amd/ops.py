@@ -383,7 +383,9 @@ class _Unchecked:
 def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offset: int, like: torch.Tensor):
     """``(ks, ke, check)``: the key window of every causal query ``chunk_offset + i`` (int32, on ``like``'s device) over
     the packed sequences of ``cu_seqlens`` (None: one sequence).  ``check.wait()`` raises ValueError if the sequences
-    end before the queries do; call it behind the launches that use the window."""
+    end before the queries do, or their cumulative lengths decrease; call it behind the launches that use the window.
+    While a HIP graph is captured nothing can be checked; in any case a query behind the last sequence has an empty window
+    (no keys, ids -1)."""
     if not ordinary(cu_seqlens, like):
         dev = like.device
         ke = torch.arange(queries, dtype=torch.int32, device=dev) + chunk_offset + 1

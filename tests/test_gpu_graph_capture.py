@@ -52,3 +52,34 @@ def test_pipeline_replays_from_a_graph(gpu):
         torch.cuda.synchronize()
         for name, ref in eager.items():
             assert torch.equal(captured[name], ref), "replay with seed %d differs from the eager run in %s" % (seed, name)
+
+
+def test_packed_indexer_replays_with_other_sequences(gpu):
+    """The windows of packed sequences are part of the graph: a replay follows the lengths that are in the tensor then.  Queries
+    that no sequence holds, which an eager call refuses, select nothing."""
+    from loongforge_amd import dsa_fused_kernels as K
+    from loongforge_amd.megatron_compat import PackedSeqParams
+
+    S, topk = 300, 64
+    iq, ik, w = (t.to(gpu) for t in O.make_indexer_inputs(S, 32, 128, seed=3))
+    cu = torch.tensor([0, 100, S], dtype=torch.int32, device=gpu)
+    run = lambda c: K.DSAIndexerKernel()(iq, ik, w, topk, 0, PackedSeqParams(qkv_format="thd", cu_seqlens_q=c, cu_seqlens_kv=c))   # noqa: E731
+    run(cu)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        scores, ids = run(cu)
+    for lengths in ([0, 100, S], [0, 7, S], [0, 250, S], [0, 100, 200]):
+        now = torch.tensor(lengths, dtype=torch.int32, device=gpu)
+        full = now.clone()
+        full[-1] = S                                   # the held queries' windows do not depend on where the last sequence ends
+        want_s, want_i = run(full)
+        torch.cuda.synchronize()
+        cu.copy_(now)
+        graph.replay()
+        torch.cuda.synchronize()
+        held = lengths[-1]
+        assert torch.equal(ids[:held], want_i[:held]) and torch.equal(scores[:held], want_s[:held]), lengths
+        assert (ids[held:] == -1).all() and (scores[held:] == float("-inf")).all(), lengths
+    with pytest.raises(ValueError, match="200 tokens"):
+        run(cu)

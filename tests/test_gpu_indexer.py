@@ -352,6 +352,31 @@ def test_windows_and_positions_of_packed_sequences(gpu, cu, S, offset, dtype):
             short.wait()
 
 
+def test_packed_sequences_that_end_before_the_queries(gpu):
+    """What the windows are where nothing can raise (a launch under capture): none for the queries that no sequence holds.  What
+    is refused: sequences that are too short, decreasing lengths, no sequence; no query needs none."""
+    import ctypes
+
+    from loongforge_amd import _lib, ops
+
+    like = torch.zeros(1, device=gpu)
+    for cu, offset in (([0, 3, 9], 4), ([5, 8, 14], 4), ([0], 0), ([0, 0], 0)):
+        ks, ke = (torch.full((300,), 7, dtype=torch.int32, device=gpu) for _ in range(2))
+        t = torch.tensor(cu, dtype=torch.int32, device=gpu)
+        _lib.check(_lib.load().dsa_indexer_window(t.data_ptr(), 0, len(cu), 300, offset, ks.data_ptr(), ke.data_ptr(), None,
+                                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "window")
+        held = max(cu[-1] - cu[0] - offset, 0)
+        assert ke[:held].tolist() == list(range(offset + 1, offset + 1 + held)) and (ks[:held] < ke[:held] + cu[0]).all()
+        assert not ks[held:].any() and not ke[held:].any()
+    for bad, match in (([0, 5, 4, 20], "decrease"), ([0, 9], "9 tokens"), ([0], "no packed sequence"), ([], "no packed sequence")):
+        with pytest.raises(ValueError, match=match):
+            ops.indexer_window(torch.tensor(bad, dtype=torch.int64, device=gpu), 10, 3, like)[2].wait()
+    long = torch.cat((torch.arange(700), torch.tensor([600])))                     # the fall lies behind the first 256 entries
+    with pytest.raises(ValueError, match="decrease"):
+        ops.indexer_window(long.to(gpu), 10, 3, like)[2].wait()
+    ops.indexer_window(torch.tensor([0, 2], device=gpu), 0, 3, like)[2].wait()
+
+
 def test_native_host_layer_equals_the_registered_ops(gpu):
     """Ordinary calls go through the C++ layer, traced ones and those under a dispatch mode through the custom op."""
     from loongforge_amd import ops
