@@ -448,25 +448,26 @@ __device__ __forceinline__ bool linear_select_sort_regs(const float* __restrict_
   return select_regs_tolerant<BL, NV>(v, off, K, base_id, hist, scratch, obuf, sv, si);
 }
 
-// LEAN (sorted rows held in registers; implies !STAGED).  1: rows of up to REG_ROW elements, the kernel keeps to
-// 128 registers so that four workgroups share a compute unit.  2: rows of up to REG_ROW_BIG elements at up to 256
-// registers (two workgroups per compute unit).  3: BL = 1024, rows of up to REG_ROW_BIG elements at 64 registers per
-// thread: one or two rows per compute unit, each four times as fast.  A launch looks only at the rows whose length
-// lies in (n_above, n_upto] and leaves the others to the launch of the other variant; rows the single-sweep path
-// turns down take the general path on global memory and the plain LDS sorting network.  Rows are taken in ascending
-// order (with causal windows the short ones first: 0.118 ms at 8192 x 8192 against 0.161 ms longest first and
-// 0.141 ms with short and long rows alternating).
+// LEAN 0: unsorted output, the row staged in LDS where it fits.  1, 2, 3: sorted output, rows held in registers.  1: rows of up
+// to REG_ROW elements, the kernel keeps to 128 registers so that four workgroups share a compute unit.  2: rows of up to
+// REG_ROW_BIG elements at up to 256 registers (two workgroups per compute unit).  3: BL = 1024, rows of up to REG_ROW_BIG
+// elements at up to 128 registers: one row per compute unit, four times as fast.  A launch looks only at the rows whose length
+// lies in (n_above, n_upto] and leaves the others to the launch of the other variant.  Rows that the single-sweep path turns
+// down or that are too long for it take the general path on global memory and a sorting network: in LDS with 256 threads,
+// whose registers are the row's, in registers with 1024 (us, top-k 2048, in LDS / in registers: one row of 40000 81 / 73, 48 of
+// 131072 210 / 202, 300 of 65536 398 / 382).  Rows are taken in ascending order (with causal windows the short ones first:
+// 0.118 ms at 8192 x 8192 against 0.161 ms longest first and 0.141 ms with short and long rows alternating).
 template <int BL, bool STAGED, int LEAN>
 __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 : 1) void topk_kernel(
     const float* __restrict__ logits, long ld, const int* __restrict__ row_begin, const int* __restrict__ row_end,
-    int width, const int* __restrict__ id_base, int K, int Kp2, int sorted, float* __restrict__ scores,
-    int* __restrict__ ids, int nmax, int n_above, int n_upto) {
+    int width, const int* __restrict__ id_base, int K, int Kp2, float* __restrict__ scores, int* __restrict__ ids,
+    int n_above, int n_upto) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   int* hist = (int*)smem;                          // HBINS
   int* scratch = hist + HBINS;                     // SCRATCH<BL>
   float* outv = (float*)(scratch + SCRATCH<BL>);   // Kp2
   int* outi = (int*)(outv + Kp2);                  // Kp2
-  unsigned* keys = (unsigned*)(outi + Kp2 + 2 * LIN_SPARE);   // nmax (STAGED only); the gap extends the (score, id) buffer
+  unsigned* keys = (unsigned*)(outi + Kp2 + 2 * LIN_SPARE);   // width (STAGED only); the gap extends the (score, id) buffer
   const int tid = threadIdx.x;
   const long row = blockIdx.x;
   const int cb = max(row_begin ? row_begin[row] : 0, 0);
@@ -477,14 +478,13 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
   const float* src = logits + row * ld + cb;
   float* sv = scores + row * (long)K;
   int* si = ids + row * (long)K;
-  (void)nmax;
 
   auto key_at = [&](int e) -> unsigned { return STAGED ? keys[e] : f2key(src[e]); };
 
-  if (sorted && n > 0 && n <= SHORT_ROW) {
+  if (LEAN != 0 && n > 0 && n <= SHORT_ROW) {
     if (rank_short_row<BL>(src, n, K, base_id, (unsigned long long*)outv, sv, si)) return;
     __syncthreads();
-  } else if (sorted && n > 0) {   // single-sweep path, also for rows shorter than K
+  } else if (LEAN != 0 && n > 0) {   // single-sweep path, also for rows shorter than K
     if (LEAN == 1 && n + 3 <= REG_ROW) {
       bool done;
       unsigned long long* obuf = (unsigned long long*)outv;
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
       outi[t] = (t < n && v != -INFINITY) ? base_id + t : -1;
     }
   } else {
-    if (STAGED && !sorted) {
+    if (STAGED) {
       for (int e = tid; e < n; e += BL) keys[e] = f2key(src[e]);
     }
     // ---- pass 1: bits [31:20] ------------------------------------------------------------
@@ -576,27 +576,27 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
   }
   __syncthreads();
 
-  if (sorted) {   // bitonic sort, descending score, ascending id among equal scores
-    const int ept = LEAN != 0 ? 0 : Kp2 / BL;
-    if (ept == 8) { bitonic_regs<BL, 8>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 4) { bitonic_regs<BL, 4>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 2) { bitonic_regs<BL, 2>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 1) { bitonic_regs<BL, 1>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 16) { bitonic_regs<BL, 16>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else if (ept == 32) { bitonic_regs<BL, 32>(outv, outi, (unsigned long long*)outv, Kp2, sv, si, K); return; }
-    else {
-      for (int size = 2; size <= Kp2; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-          for (int t = tid; t < (Kp2 >> 1); t += BL) {
-            const int lo = 2 * t - (t & (stride - 1));
-            const int hi = lo + stride;
-            const bool desc = ((lo & size) == 0);
-            const float a = outv[lo], b = outv[hi];
-            const int ia = outi[lo], ib = outi[hi];
-            if (comes_first(a, ia, b, ib) != desc) { outv[lo] = b; outv[hi] = a; outi[lo] = ib; outi[hi] = ia; }
-          }
-          __syncthreads();
+  if (LEAN != 0) {   // bitonic sort, descending score, ascending id among equal scores
+    // in registers where the kernel has them to spare: every row too long for the single sweep comes this way
+    if (LEAN == 3 && Kp2 >= BL) {
+      unsigned long long* xbuf = (unsigned long long*)outv;
+      if (Kp2 == BL) bitonic_regs<BL, 1>(outv, outi, xbuf, Kp2, sv, si, K);
+      else if (Kp2 == 2 * BL) bitonic_regs<BL, 2>(outv, outi, xbuf, Kp2, sv, si, K);
+      else if (Kp2 == 4 * BL) bitonic_regs<BL, 4>(outv, outi, xbuf, Kp2, sv, si, K);
+      else bitonic_regs<BL, 8>(outv, outi, xbuf, Kp2, sv, si, K);
+      return;
+    }
+    for (int size = 2; size <= Kp2; size <<= 1) {
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        for (int t = tid; t < (Kp2 >> 1); t += BL) {
+          const int lo = 2 * t - (t & (stride - 1));
+          const int hi = lo + stride;
+          const bool desc = ((lo & size) == 0);
+          const float a = outv[lo], b = outv[hi];
+          const int ia = outi[lo], ib = outi[hi];
+          if (comes_first(a, ia, b, ib) != desc) { outv[lo] = b; outv[hi] = a; outi[lo] = ib; outi[hi] = ia; }
         }
+        __syncthreads();
       }
     }
   }
@@ -624,8 +624,8 @@ int dsa_topk_launch(const float* logits, int S, int64_t ld, const int32_t* row_b
   const int none = 0x7fffffff, split = REG_ROW - 3;
   auto launch = [&](auto kern, int block, size_t smem, int n_above, int n_upto) {
     if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return false;
-    kern<<<dim3(S), dim3(block), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, sorted, scores, ids,
-                                             width, n_above, n_upto);
+    kern<<<dim3(S), dim3(block), smem, st>>>(logits, (long)ld, row_begin, row_end, width, id_base, K, Kp2, scores, ids,
+                                             n_above, n_upto);
     return true;
   };
   bool ok;

@@ -304,6 +304,42 @@ def test_topk_row_lengths_at_the_edges_of_its_variants(gpu, copies, K):
             assert (got_i[k:] == -1).all() and torch.isinf(got_s[k:]).all(), (n, c)
 
 
+@pytest.mark.parametrize("copies", [1, 45])       # 6 rows: the 1024-thread kernel alone; 270 rows: behind the 256-thread one
+@pytest.mark.parametrize("K", [64, 1000, 2048, 4096, 8192])
+@pytest.mark.parametrize("sorted_out", [True, False])
+def test_topk_of_rows_beyond_the_register_variants(gpu, copies, K, sorted_out):
+    """Around the longest row held in registers and beyond it: the general path with the sorting networks, ties by ascending
+    column, columns that cannot be selected, fewer of the others than slots."""
+    from loongforge_amd import ops
+
+    lengths = [36861, 36862, 41000, 41000, 41000, 41000]
+    width = 41003
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(len(lengths), width, generator=g)
+    x[3] = torch.randint(0, 5, (width,), generator=g).float()
+    x[4, ::2] = float("-inf")
+    x[5, 700:] = float("-inf")
+    begin = torch.tensor([i % 4 for i in range(len(lengths))], dtype=torch.int32)
+    end = begin + torch.tensor(lengths, dtype=torch.int32)
+    rep = lambda t: t.repeat(copies, *([1] * (t.ndim - 1))).to(gpu)                    # noqa: E731
+    sc, ids = ops.topk(rep(x), K, rep(begin), rep(end), sorted=sorted_out)
+    sc, ids = sc.view(copies, len(lengths), K), ids.view(copies, len(lengths), K)
+    assert all(torch.equal(sc[c], sc[0]) and torch.equal(ids[c], ids[0]) for c in range(copies))
+    for i, n in enumerate(lengths):
+        row = x[i, int(begin[i]): int(end[i])]
+        v, order = torch.sort(row, descending=True, stable=True)
+        k = min(K, int(torch.isfinite(row).sum()))
+        got_s, got_i = sc[0, i].cpu(), ids[0, i].cpu().long()
+        if sorted_out:
+            assert torch.equal(got_s[:k], v[:k]) and torch.equal(got_i[:k], order[:k] + int(begin[i])), n
+            assert (got_i[k:] == -1).all() and torch.isinf(got_s[k:]).all(), n
+        else:                                           # in ascending column order
+            want = torch.sort(order[:k])[0]
+            live = got_i >= 0
+            assert torch.equal(got_i[live], want + int(begin[i])) and torch.equal(got_s[live], row[want]), n
+            assert torch.isinf(got_s[~live]).all(), n
+
+
 @pytest.mark.parametrize("Hi", [32, 64])
 def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
     """Windows cut into parts over workgroups: shared ones (a chunk behind cached keys), unrelated ones (sequences of a
