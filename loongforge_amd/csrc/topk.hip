@@ -170,6 +170,7 @@ __device__ __forceinline__ void bitonic_regs(float* outv, int* outi, unsigned lo
 constexpr int LIN_SPARE = 960;               // extra buffer entries for the threshold bin's surplus
 constexpr int REG_ROW = 8192 + 4 * 256;      // longest row (plus alignment slack) the register variant holds
 constexpr int REG_ROW_BIG = 32768 + 4 * 256; // the same for the variant with twice the registers
+constexpr int REG_ROW_WIDE = 9 * 4 * 1024;   // the same for the 1024-thread variant
 constexpr int WIDE_ROWS = 256;               // at most so many rows: the 1024-thread kernel
 constexpr int LIN_MAX_BIN = 256;             // largest segment ranked by pairwise counting
 
@@ -450,11 +451,12 @@ __device__ __forceinline__ bool linear_select_sort_regs(const float* __restrict_
 
 // LEAN 0: unsorted output, the row staged in LDS where it fits.  1, 2, 3: sorted output, rows held in registers.  1: rows of up
 // to REG_ROW elements, the kernel keeps to 128 registers so that four workgroups share a compute unit.  2: rows of up to
-// REG_ROW_BIG elements at up to 256 registers (two workgroups per compute unit).  3: BL = 1024, rows of up to REG_ROW_BIG
-// elements at up to 128 registers: one row per compute unit, four times as fast.  A launch looks only at the rows whose length
-// lies in (n_above, n_upto] and leaves the others to the launch of the other variant.  Rows that the single-sweep path turns
-// down or that are too long for it take the general path on global memory and a sorting network: in LDS with 256 threads,
-// whose registers are the row's, in registers with 1024 (us, top-k 2048, in LDS / in registers: one row of 40000 81 / 73, 48 of
+// REG_ROW_BIG elements at up to 256 registers (two workgroups per compute unit).  3: BL = 1024, rows of up to REG_ROW_WIDE
+// elements at up to 128 registers: one row per compute unit, four times as fast (between the two limits, 300 rows of
+// 34000, top-k 64: 171 us on the general path, 25 here).  A launch looks only at the rows whose length lies in
+// (n_above, n_upto] and leaves the others to the launch of the other variant.  Rows that the single-sweep path turns down or
+// that are too long for it take the general path on global memory and a sorting network: in LDS with 256 threads, whose
+// registers are the row's, in registers with 1024 (us, top-k 2048, in LDS / in registers: one row of 40000 81 / 73, 48 of
 // 131072 210 / 202, 300 of 65536 398 / 382).  Rows are taken in ascending order (with causal windows the short ones first:
 // 0.118 ms at 8192 x 8192 against 0.161 ms longest first and 0.141 ms with short and long rows alternating).
 template <int BL, bool STAGED, int LEAN>
@@ -501,13 +503,13 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
       else done = linear_select_sort_regs<BL, REG_ROW_BIG / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       if (done) return;
       __syncthreads();
-    } else if (LEAN == 3 && n + 3 <= REG_ROW_BIG) {
+    } else if (LEAN == 3 && n + 3 <= REG_ROW_WIDE) {
       bool done;
       unsigned long long* obuf = (unsigned long long*)outv;
       if (n + 3 <= 4 * BL) done = linear_select_sort_regs<BL, 1>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       else if (n + 3 <= 2 * 4 * BL) done = linear_select_sort_regs<BL, 2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       else if (n + 3 <= 4 * 4 * BL) done = linear_select_sort_regs<BL, 4>(src, n, K, base_id, hist, scratch, obuf, sv, si);
-      else done = linear_select_sort_regs<BL, (REG_ROW_BIG + 4 * BL - 1) / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else done = linear_select_sort_regs<BL, REG_ROW_WIDE / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       if (done) return;
       __syncthreads();
     }
