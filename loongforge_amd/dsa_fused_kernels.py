@@ -576,9 +576,10 @@ class FusedAbsorbRopeQuery(torch.autograd.Function):
         g3 = grad.reshape(-1, grad.shape[-2], grad.shape[-1])
         d_up = torch.empty_like(q3)
         g_c = g3[:, :, :d_out].transpose(0, 1)                                   # [h, S, 512]
-        d_up[:, :, :d_nope] = torch.bmm(g_c, w_uk_t).transpose(0, 1)
+        d_up[:, :, :d_nope] = torch.bmm(g_c, w_uk_t.contiguous()).transpose(0, 1)
         ops.rope_rows(g3[:, :, d_out:], d_up[:, :, d_nope:], cos, sin, out_pairing, ops.ROPE_ADJACENT, True, positions, batch)
-        d_w = torch.bmm(g_c.transpose(1, 2), q3[:, :, :d_nope].transpose(0, 1)) if ctx.needs_input_grad[1] else None
+        # (right operands contiguous, as in MlaAbsorb)
+        d_w = torch.bmm(g_c.transpose(1, 2), q3[:, :, :d_nope].transpose(0, 1).contiguous()) if ctx.needs_input_grad[1] else None
         return d_up.view(shape), d_w, None, None, None, None, None, None
 
 

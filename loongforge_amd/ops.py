@@ -784,8 +784,9 @@ class MlaAbsorb(torch.autograd.Function):
     def backward(ctx, grad):
         a, w = ctx.saved_tensors
         g = grad.transpose(0, 1)                       # [H, S, n]
-        d_a = torch.bmm(g, w).transpose(0, 1) if ctx.needs_input_grad[0] else None          # [S, H, k]
-        d_w = torch.bmm(g.transpose(1, 2), a.transpose(0, 1)) if ctx.needs_input_grad[1] else None   # [H, n, k]
+        d_a = torch.bmm(g, _c(w)).transpose(0, 1) if ctx.needs_input_grad[0] else None          # [S, H, k]
+        # [H, n, k]; the right operand of a batched bf16 product is laid out contiguously: as a transposed view it has faulted
+        d_w = torch.bmm(g.transpose(1, 2), a.transpose(0, 1).contiguous()) if ctx.needs_input_grad[1] else None
         return d_a, d_w, None
 
 

@@ -118,3 +118,32 @@ def test_host_layer_is_rebuilt_for_another_torch(tmp_path, monkeypatch):
     assert len(runs) == 3
     build._compile_host(True)
     assert len(runs) == 4
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_batched_products_of_the_absorption_have_contiguous_right_operands(fused, monkeypatch):
+    """A bf16 batched product whose right operand is a transposed view has faulted the device; the gradients' products are
+    given contiguous ones, whatever the layouts of the weights and the activations."""
+    from types import SimpleNamespace
+
+    from loongforge_amd import dsa_fused_kernels as K, ops
+
+    seen, bmm = [], torch.bmm
+
+    def product(a, b):
+        seen.append(b.is_contiguous())
+        return bmm(a, b)
+
+    monkeypatch.setattr(torch, "bmm", product)
+    monkeypatch.setattr(ops, "rope_rows", lambda *a, **k: None)
+    rnd = lambda *shape: torch.randn(*shape, generator=torch.Generator().manual_seed(0), dtype=torch.float64)      # noqa: E731
+    a, w, grad = rnd(5, 3, 192 if fused else 128), rnd(3, 128, 512).transpose(1, 2), rnd(5, 3, 576 if fused else 512)
+    if fused:
+        ctx = SimpleNamespace(saved_tensors=(a, w, None, None), args=(None, 1, 0, 128, 512, 64, a.shape), needs_input_grad=(True, True))
+        d_a, d_w = K.FusedAbsorbRopeQuery.backward(ctx, grad)[:2]
+    else:
+        ctx = SimpleNamespace(saved_tensors=(a, w), needs_input_grad=(True, True, False))
+        d_a, d_w = ops.MlaAbsorb.backward(ctx, grad)[:2]
+    assert seen == [True, True]
+    torch.testing.assert_close(d_a[..., :128], torch.einsum("shn,hnk->shk", grad[..., :512], w))
+    torch.testing.assert_close(d_w, torch.einsum("shn,shk->hnk", grad[..., :512], a[..., :128]))
