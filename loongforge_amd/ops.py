@@ -488,7 +488,7 @@ def sparse_mla_fwd_dist(q, kv, ids, q_start: int, sm_scale: float, d_v: int, dis
     return _mla_fwd_dist_op(q, kv, ids, int(q_start), float(sm_scale), int(d_v), int(dist_heads), int(block), attn_sink)
 
 
-_BWD_WS = {}      # device index -> workspace kept between calls
+_BWD_WS = {}      # device index -> workspace kept between calls; its `stream` is the one it was allocated and used on
 BWD_MAX_SLOTS = 2048      # slots per query the backward kernels take in one call
 ATTN_DIST_QK_MAX_SLOTS = 4096
 
@@ -498,24 +498,28 @@ def _bwd_workspace(full_bytes: int, device):
     tokens, top-k 2048; 105 GiB at 32k); given less, the library walks the queries in chunks.  The size handed to
     the library - and with it the chunking, on which the last bits of dKV depend - follows from the shapes and
     from ``DSA_BWD_WORKSPACE_GIB`` (default 48) alone, never from what happens to be free or from earlier calls.
-    The buffer is kept per device and reused by later calls (held until :func:`release_bwd_workspace`; calls that
-    overlap on one device - other streams - must not share it: set ``DSA_BWD_WORKSPACE_CACHE=0``).  Nothing is
-    kept while a HIP graph is being captured."""
+    The buffer is kept per device and reused by later calls on the same stream (held until :func:`release_bwd_workspace`;
+    ``DSA_BWD_WORKSPACE_CACHE=0`` keeps none).  A call on another stream, which may overlap, lets go of it - the allocator
+    hands it out again behind the work of its own stream only - and allocates one there.  A graph that is being captured gets
+    one of its own, which lives as long as the graph."""
     want = max(int(full_bytes), 256)
     cap = os.environ.get("DSA_BWD_WORKSPACE_GIB", "48")
     want = min(want, max(int(float(cap) * 2 ** 30), 256))
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    kept = _BWD_WS.get(idx)
-    if kept is not None and kept.numel() >= want:
-        return kept, want
-    _BWD_WS.pop(idx, None)
-    del kept
+    capturing, stream = torch.cuda.is_current_stream_capturing(), torch.cuda.current_stream(device).cuda_stream
+    if not capturing:
+        kept = _BWD_WS.get(idx)
+        if kept is not None and kept.numel() >= want and kept.stream == stream:
+            return kept, want
+        _BWD_WS.pop(idx, None)
+        del kept
     try:
         ws = torch.empty(want, dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError as e:
         raise RuntimeError("sparse_mla_bwd: cannot allocate its %.1f GiB workspace; lower DSA_BWD_WORKSPACE_GIB "
                            "(the library then walks the queries in more chunks)" % (want / 2 ** 30)) from e
-    if os.environ.get("DSA_BWD_WORKSPACE_CACHE", "1") != "0" and not torch.cuda.is_current_stream_capturing():
+    if os.environ.get("DSA_BWD_WORKSPACE_CACHE", "1") != "0" and not capturing:
+        ws.stream = stream
         _BWD_WS[idx] = ws
     return ws, want
 

@@ -392,6 +392,29 @@ def test_backward_op_workspace_is_capped_and_kept(gpu, monkeypatch):
     ops._BWD_WS.clear()
 
 
+def test_backward_on_two_streams_at_once(gpu):
+    """Backward passes that overlap on two streams do not share a workspace: the results are those of passes one by one."""
+    from loongforge_amd import ops
+
+    inp = [O.make_mla_inputs(300, 64, 128, seed=s) for s in (1, 2)]
+    args = []
+    for i in inp:
+        q, kv, idx, do = i.q.to(gpu), i.kv.to(gpu), i.idx.to(gpu), i.dout.to(gpu)
+        out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, 0, i.sm_scale)
+        args.append((q, kv, out, do, idx, lse, 0, i.sm_scale))
+    want = [ops.sparse_mla_bwd(*a) for a in args]
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream(), torch.cuda.Stream()], [[], []]
+    for _ in range(4):
+        for n, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[n].append(ops.sparse_mla_bwd(*args[n]))
+    torch.cuda.synchronize()
+    for n in range(2):
+        assert all(torch.equal(g, w) for pair in got[n] for g, w in zip(pair, want[n]))
+    ops._BWD_WS.clear()
+
+
 def test_argument_errors(gpu):
     from loongforge_amd import ops
 

@@ -147,3 +147,29 @@ def test_batched_products_of_the_absorption_have_contiguous_right_operands(fused
     assert seen == [True, True]
     torch.testing.assert_close(d_a[..., :128], torch.einsum("shn,hnk->shk", grad[..., :512], w))
     torch.testing.assert_close(d_w, torch.einsum("shn,shk->hnk", grad[..., :512], a[..., :128]))
+
+
+def test_backward_workspace_is_not_shared_between_streams(monkeypatch):
+    """One buffer is kept per device, for the stream it was used on; another stream and a graph capture get their own."""
+    from types import SimpleNamespace
+
+    from loongforge_amd import ops
+
+    now, empty = SimpleNamespace(stream=1, capturing=False), torch.empty
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=now.stream))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now.capturing)
+    monkeypatch.setattr(torch, "empty", lambda n, dtype, device: empty(n, dtype=dtype))
+    monkeypatch.setattr(ops, "_BWD_WS", {})
+    get = lambda n: ops._bwd_workspace(n, torch.device("cuda", 0))[0]                # noqa: E731
+    first = get(1000)
+    assert get(500) is first and get(1000) is first
+    now.stream = 2
+    second = get(500)
+    assert second is not first and get(400) is second
+    now.capturing = True
+    captured = get(300)
+    assert captured is not second and ops._BWD_WS[0] is second      # the graph's buffer is nobody else's, the kept one stays
+    now.capturing = False
+    assert get(300) is second
+    now.stream = 1
+    assert get(300) is not second and len(ops._BWD_WS) == 1
