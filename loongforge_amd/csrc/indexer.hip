@@ -93,11 +93,11 @@ __device__ __forceinline__ void load_query(const unsigned char* __restrict__ q8,
   }
 }
 
-template <int NHT>   // groups of 32 heads
+template <int NHT, bool RELATIVE>   // groups of 32 heads; columns counted from the start of the window
 __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kernel(
     const unsigned char* __restrict__ q8, const float* __restrict__ q_w, const unsigned char* __restrict__ k8,
     const float* __restrict__ k_scale, const int* __restrict__ ks, const int* __restrict__ ke,
-    int S, int Sk, float* __restrict__ logits, long ld, int relative, int q_begin, int q_count, int parts) {
+    int S, int Sk, int width, float* __restrict__ logits, long ld, int q_begin, int q_count, int parts) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * TILE_BYTES + 2 * BK * 4];
   constexpr int NWAVE = QB;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -107,13 +107,18 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
   const int blk = nblk - 1 - (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;            // longest windows first
   const int qb0 = q_begin + blk * QB;
   const int q_end = q_begin + q_count;
+  // end of the window that starts at lo: no key has a column beyond the row's (absolute columns: Sk is at most the width)
+  auto window_end = [&](int i, int lo) {
+    const int hi = min(ke[i], Sk);
+    return RELATIVE && hi - lo > width ? lo + width : hi;
+  };
 
   // window union of the block
   int jlo = 0x7fffffff, jhi = 0, total = 0;
   for (int t = 0; t < QB; t++) {
     const int i = qb0 + t;
     if (i < q_end) {
-      const int lo = max(ks[i], 0), hi = min(ke[i], Sk);
+      const int lo = max(ks[i], 0), hi = window_end(i, lo);
       jlo = min(jlo, ks[i]);
       jhi = max(jhi, hi);
       total += (max(hi - lo, 0) + 31) / 32;
@@ -130,7 +135,7 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
     int before = 0;
 #pragma unroll 1
     for (int i = qb0; i < min(qb0 + QB, q_end); i++) {
-      const int w_lo = max(ks[i], 0), w_hi = min(ke[i], Sk), n = (max(w_hi - w_lo, 0) + 31) / 32;
+      const int w_lo = max(ks[i], 0), w_hi = window_end(i, w_lo), n = (max(w_hi - w_lo, 0) + 31) / 32;
       const int u_lo = max(a - before, 0), u_hi = min(b - before, n);
       before += n;
       if (u_lo >= u_hi) continue;
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
       i32x8 aq[NHT][2];
       float wq[NHT][16];
       load_query(q8, q_w, i, r, g, aq, wq);
-      float* lrow = logits + (size_t)(i - q_begin) * ld - (relative ? w_lo : 0);
+      float* lrow = logits + (size_t)(i - q_begin) * ld - (RELATIVE ? w_lo : 0);
 #pragma unroll 1
       for (int u = u_lo; u < u_hi; u++) {
         i32x8 bk[2];
@@ -170,7 +175,7 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
   const bool live = i_q < q_end;
   const int qi = live ? i_q : -1;
   const int qks = live ? max(ks[i_q], 0) : 0;
-  const int qke = live ? min(ke[i_q], Sk) : 0;
+  const int qke = live ? window_end(i_q, qks) : 0;
   const int wlo = live ? qks : 0x7fffffff, whi = live ? qke : 0;     // the wave's window
   i32x8 aq[NHT][2];
   float wq[NHT][16];
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
       for (int tt = 0; tt < NHT; tt++) sum = head_sum(aq[tt], bk, wq[tt], sum);
       sum = add_halves(sum) * ksc;
       if (g == 0 && j >= qks && j < qke) {
-        const int col = relative ? j - qks : j;
+        const int col = RELATIVE ? j - qks : j;
         logits[(size_t)(qi - q_begin) * ld + col] = sum;
       }
     }
@@ -262,14 +267,15 @@ int dsa_indexer_logits_block(const void* q8, const float* q_w, const void* k8, c
   // of shorter ones beyond (us before -> after, 64 heads: one query x 4096 keys 52 -> 5, 61 x 20000 292 -> 18, 48
   // unrelated windows of 7000 keys 807 -> 15, 500 x 8000 129 -> 39, 1500 x 7500 131 -> 89, 3000 x 7500 200 -> 166).
   const int nblk = (q_count + QB - 1) / QB;
+  if (!relative && width < Sk) Sk = width;                   // the keys beyond have no column
   int parts = (nblk < 128 ? 512 : 768) / nblk;
   if (parts > (Sk + BK - 1) / BK) parts = (Sk + BK - 1) / BK;
   if (parts < 1) parts = 1;
   dim3 grid(nblk * parts), block(64 * QB);
-#define DSA_IDX_LAUNCH(N) indexer_logits_kernel<N><<<grid, block, 0, st>>>( \
-    (const unsigned char*)q8, q_w, (const unsigned char*)k8, k_scale, ks, ke, S, Sk, logits, (long)ld, relative, q_begin, q_count, parts)
-  if (Hi == 32) DSA_IDX_LAUNCH(1);
-  else DSA_IDX_LAUNCH(2);
+#define DSA_IDX_LAUNCH(N, R) indexer_logits_kernel<N, R><<<grid, block, 0, st>>>( \
+    (const unsigned char*)q8, q_w, (const unsigned char*)k8, k_scale, ks, ke, S, Sk, width, logits, (long)ld, q_begin, q_count, parts)
+  if (Hi == 32) { if (relative) DSA_IDX_LAUNCH(1, true); else DSA_IDX_LAUNCH(1, false); }
+  else { if (relative) DSA_IDX_LAUNCH(2, true); else DSA_IDX_LAUNCH(2, false); }
 #undef DSA_IDX_LAUNCH
   DSA_CHECK_LAUNCH("dsa_indexer_logits");
   return DSA_OK;

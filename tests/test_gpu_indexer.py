@@ -365,6 +365,28 @@ def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
                 assert int(torch.isfinite(got[i]).sum()) == n
 
 
+@pytest.mark.parametrize("relative", [False, True])
+@pytest.mark.parametrize("S", [3, 300])                  # unrelated and shared windows
+def test_logits_in_rows_narrower_than_the_windows(gpu, relative, S):
+    """Keys that have no column in the row are left out, and nothing is written behind it."""
+    from loongforge_amd import _lib, ops
+
+    g = torch.Generator().manual_seed(S)
+    sk, width = 700, 333
+    q = torch.randn(S, 64, 128, generator=g).to(torch.float8_e4m3fn).to(gpu)
+    k = torch.randn(sk, 128, generator=g).to(torch.float8_e4m3fn).to(gpu)
+    w, sc = torch.randn(S, 64, generator=g).to(gpu), torch.rand(sk, generator=g).to(gpu)
+    ks = torch.tensor([(37 * i) % 400 if S < 10 else i // 8 for i in range(S)], dtype=torch.int32, device=gpu)
+    ke = torch.full((S,), sk, dtype=torch.int32, device=gpu)
+    full = ops.indexer_logits(q, w, k, sc, ks, ke, relative=relative)
+    ld = width + 5
+    out = torch.full((S + 1, ld), 7.0, device=gpu)
+    _lib.check(_lib.load().dsa_indexer_logits(q.data_ptr(), w.data_ptr(), k.data_ptr(), sc.data_ptr(), ks.data_ptr(), ke.data_ptr(), S, 64, sk,
+                                              out.data_ptr(), ld, width, int(relative), torch.cuda.current_stream().cuda_stream), "logits")
+    assert torch.equal(out[:S, :width], full[:, :width])
+    assert (out[:S, width:] == 7.0).all() and (out[S] == 7.0).all()
+
+
 @pytest.mark.parametrize("cu,S,offset", [(None, 5, 3), ([0, 7], 7, 0), ([0, 3, 3, 300, 513], 256, 257), ([0, 1, 2, 700], 700, 0)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 def test_windows_and_positions_of_packed_sequences(gpu, cu, S, offset, dtype):
