@@ -3,7 +3,7 @@
 //
 //   logits[i, j] = k_scale[j] * sum_h q_w[i,h] * relu(q8[i,h,:] . k8[j,:])      ks[i] <= j < ke[i]
 //
-// One workgroup owns 8 consecutive queries, one per wave (512 threads; at 122 registers per lane
+// One workgroup owns 8 consecutive queries, one per wave (512 threads; at 128 registers per lane
 // four waves share a SIMD), and streams the keys its queries can see through LDS in tiles of 128
 // rows (global_load_lds, double buffered, 16-byte slots XOR-swizzled per row).  For every 32-key
 // sub-tile a wave issues, per group of 32 heads, two v_mfma_f32_32x32x64_f8f6f4 (A = the query's fp8
