@@ -13,6 +13,7 @@
 //                              bf16 row of 576 values
 //                              in a pair buffer, at the position given by a key-sorted order
 //   pass D  (bwd_reduce_kernel) dKV[key] = sum of that key's rows, in ascending query order
+// With 64 heads both orientations fit, and passes A and C are one (bwd_pds_rows_kernel).
 // The key-sorted order (pass 0) comes from a bitmap key x query, its row-wise prefix popcounts and
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
@@ -22,10 +23,10 @@
 namespace {
 using namespace mla;
 
-// P and dS of one (query, tile): 2 x [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes
-// are compiled for: 1 or 2, or 4 for 96 and 128 heads.
+// P or dS of one (query, tile): [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes are
+// compiled for: 1 or 2, or 4 for 96 and 128 heads.  In memory a tile is dS and then P; dS alone where passes A and C are one.
 constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
-constexpr int pds_tile_bytes(int HG) { return HG * 4096; }
+constexpr int pds_tile_bytes(int HG) { return HG == 2 ? pds_kind_bytes(HG) : 2 * pds_kind_bytes(HG); }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
@@ -42,9 +43,8 @@ constexpr int PDS_THREADS = 512;
 // SIMD) are then about level.  A lane ends with 4 heads x 2 half tiles; lanes 32 apart trade halves
 // (one v_permlane32_swap per register pair) so that every lane holds one key's 8 heads in the chunk
 // order pass C reads: chunk group 2w + g = heads 16w + {4g .. 4g+3, 8+4g .. 8+4g+3}.
-// With up to 64 heads four waves hold them all: waves 4-7 take every other tile (two tiles per step, STAGES = 4 tiles are then
-// two steps).  With up to 32 heads two waves do, and a wave takes one half tile of its tile only.  (Idle or repeated heads
-// cost as much as real ones: 3072 queries x 640 slots x 64 heads took 0.50 ms before.)
+// With up to 32 heads two waves hold them all: waves 4-7 take every other tile (two tiles per step, STAGES = 4 tiles are then
+// two steps), and a wave takes one half tile of its tile only.  (Idle or repeated heads cost as much as real ones.)
 template <int STAGES, int HG>
 __device__ __forceinline__ void pds_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
@@ -373,7 +373,7 @@ __device__ __forceinline__ void dq_body(
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
     t_lb = __builtin_amdgcn_readfirstlane(sb + (unsigned)((wave & 3) * 1024 + (wave >> 2) * GRP_BYTES));
     t_lbd = __builtin_amdgcn_readfirstlane(sb + (unsigned)(TILE_BYTES + (wave & (DS_WAVES - 1)) * 1024));
-    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG));     // dS half
+    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG));     // dS
   };
   // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0 .. DS_WAVES - 1)
   auto issue_step = [&](int j) {
@@ -713,16 +713,15 @@ __device__ __forceinline__ void dkv_body(
   piece_store(NC - 1, 1);
 }
 
-// The same with up to 64 heads (HG = 1, 2): the operands of a query take 72 or 144 registers, two workgroups share a compute
-// unit and hide each other's set-up, barriers and stores, and the products are plain builtins in the compiler's order.  Bound by
-// the rows: 2.26 GB for 3072 queries x 640 slots.
+// The same with up to 32 heads: the operands of a query take 72 registers, two workgroups share a compute unit and hide each
+// other's set-up, barriers and stores, and the products are plain builtins in the compiler's order.  Bound by the rows.
 constexpr int DKV_FEW_STAGES = 4;
-template <int NC, int HG>
+template <int NC>
 __device__ __forceinline__ void dkv_few_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
     const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
-  constexpr int CST = DKV_FEW_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
+  constexpr int HG = 1, CST = DKV_FEW_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
   // [CST][TB] coefficient ring, shared with the set-up's per-wave X staging [4][HG * 2048] | ids arrays | dst rows [K]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -831,6 +830,290 @@ __device__ __forceinline__ void dkv_few_body(
       __syncthreads();
       if (n + CST < ntiles) issue(n + CST);    // into the slot of tile n, whose coefficients are in registers
       read_coefs(n + 1);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// passes A and C in one, for 64 heads
+// ---------------------------------------------------------------------------------------------
+// Q and dO of 64 heads fit the registers of a compute unit in both orientations: 136 per lane for the products over d (wave
+// (hw, hh) = (wave % 4, wave / 4): 16 heads, the 16 keys of half tile hh) and 64 for those over the heads (wave w: the columns
+// 64 w .. 64 w + 63 of both; 16 columns of the rotary part come from LDS).  So P never leaves the compute unit, dS is written for
+// pass B only, and a pair costs 1152 + 128 bytes of writes where the two passes wrote 1152 + 256 and read 256.
+// Between two barriers a wave works on S, dP of tile n and on the rows of tile n - 1, whose P and dS all waves have put into
+// LDS (two buffers) before the barrier; waves 0-3 take them in this order, waves 4-7 in the other one, so that the two waves
+// of a SIMD issue stores and exponentials under each other's MFMAs.  The transfers of tile n + 2 come first in a step: between
+// the MFMAs behind the row stores of a step they held waves 4-7 for 2600 cycles per tile instead of 1100.
+// Bound by the row writes: a step of 5000 cycles writes 41 KB per compute unit, 4.7 TB/s, and the set-up of a query (208 KB
+// read, 36 000 cycles) does not overlap it.  3072 queries x 128 + 512 slots of compressed keys: 0.68 ms against 0.41 + 0.51; 2077 x 512: 0.35 against 0.23 + 0.26.
+constexpr int FUSED_STAGES = 3;
+// 16x16x32 MFMAs with accumulators in architectural registers and operand A in either file.  The compiler does not see an MFMA
+// in them: the wait states after a move that it may put in front of one (VALU write to MFMA read) are part of the string.
+#define DSA_MFMA16_FN(name, A)                                                                         \
+  __device__ __forceinline__ void name(f32x4& acc, const bf16x8& a, const bf16x8& b, bool first) {     \
+    if (first) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : A(a), "v"(b));      \
+    else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : A(a), "v"(b));            \
+  }
+DSA_MFMA16_FN(mfma16_a, "a")
+DSA_MFMA16_FN(mfma16_v, "v")
+#undef DSA_MFMA16_FN
+__device__ __forceinline__ void mfma16_done(f32x4& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
+__device__ __forceinline__ void mfma16_done(f32x4& x, f32x4& y) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x), "+v"(y)); }
+constexpr int FUSED_XCH = 2 * pds_kind_bytes(2);      // P and dS of a tile
+constexpr int FUSED_ROT = 16384;                      // every wave's operands of the rotary columns
+static_assert(64 * (DQK + DV) * 2 <= FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT, "Q and dO of a query pass through this part of LDS");
+__host__ __device__ inline size_t fused_lds_bytes(int K) {
+  return (size_t)FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT + ids_lds_bytes(K) + 512 + (size_t)K * 4;
+}
+template <int hh>
+__device__ __forceinline__ void pds_rows_body(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
+    const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    int q0, int ql, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
+  constexpr int H = 64, KS = DQK / 32, VS = DV / 32, STAGES = FUSED_STAGES;
+  constexpr int DO_ACC = 12;                   // steps of dO in accumulation registers, beside all of Q: 120
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15, kg = lane >> 4, g = lane >> 5;
+  const int hw = wave & 3;
+  const int qi = q0 + ql;
+  const int NT = K / BI;
+  // [ring][P and dS, two buffers][rotary operands], all of it Q and dO of the query at first | ids arrays | statistics | dst rows [K]
+  unsigned char* xch = smem + STAGES * TILE_BYTES;
+  bf16x8* xr_s = (bf16x8*)(xch + 2 * FUSED_XCH) + wave * 128 + lane;
+  int* idx_s = (int*)(xch + 2 * FUSED_XCH + FUSED_ROT);
+  unsigned* tmask = (unsigned*)(idx_s + K);
+  int* tlist = (int*)(tmask + NT);
+  int* ntile_s = tlist + NT;
+  float* stat_s = (float*)(ntile_s + 4);       // [2][64]: lse * log2(e), delta
+  int* dst_s = (int*)(stat_s + 128);
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+
+  // Q and dO travel to LDS as they are, in groups of 128 bytes of all 64 rows (Q: 9, dO: 8), chunk c of row r in slot c ^ (r & 7):
+  // both orientations are read from there.  Wave w moves rows 8 w .. 8 w + 7.
+  {
+    const __bf16* q_rows = uniform_ptr(q + (size_t)qi * H * DQK);
+    const __bf16* do_rows = uniform_ptr(dout + (size_t)qi * H * DV);
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
+    const unsigned row = (unsigned)(8 * wave + (lane >> 3)), col = (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
+#pragma unroll
+    for (int k = 0; k < 9; k++) dma16(lb + k * 8192, row * (DQK * 2) + col + k * 128, q_rows);
+#pragma unroll
+    for (int k = 0; k < 8; k++) dma16(lb + (9 + k) * 8192, row * (DV * 2) + col + k * 128, do_rows);
+  }
+  const int h = hw * 16 + m;
+  const size_t hrow = (size_t)qi * H + h;
+  bf16x8 qreg[KS], doreg[VS], oreg[VS];
+  {
+    const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++) oreg[ks] = op[4 * ks];
+  }
+  const float lse_h = lse[hrow];
+  __builtin_amdgcn_sched_barrier(0);
+  for (int t = tid; t < K; t += PDS_THREADS) {        // invalid slots land in a scratch row: the store count stays fixed
+    const int d = dst[(size_t)ql * K + t];
+    dst_s[t] = d >= 0 ? d : dummy_row;
+  }
+  // (the helper is written for four waves; the other four repeat part of its work with equal results)
+  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  DSA_WAIT_VMCNT(0);
+  if (ntiles == 0) return;
+  __syncthreads();
+  {
+    const unsigned char* rb = smem + h * 128;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qreg[ks] = *(const bf16x8*)(rb + (ks >> 1) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++) doreg[ks] = *(const bf16x8*)(rb + (9 + (ks >> 1)) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
+  }
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+a"(qreg[ks]));
+#pragma unroll
+  for (int ks = 0; ks < VS; ks++) {
+    if (ks < DO_ACC) asm volatile("" : "+a"(doreg[ks]));
+    else asm volatile("" : "+v"(doreg[ks]));
+  }
+  {                                            // delta = rowsum(O . dO)
+    float part = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) part = fmaf((float)oreg[ks][e], (float)doreg[ks][e], part);
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    if (kg == 0) {
+      stat_s[h] = lse_h * LOG2E;
+      stat_s[64 + h] = part;
+    }
+  }
+  // ---- operands of the rows: 16 columns by k-step ks of 32 heads, in the chunk order of P and dS ----
+  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  auto tr_pair = [&](const unsigned char* p0, const unsigned char* p1) {
+    const i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p0));
+    const i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p1));
+    return __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // Row 4 j + e of the operand is column {0, 8, 4, 12}[j] + e of the 16, so that lanes 32 apart end up with neighbouring columns.
+  // The heads of lane chunk kg are 32 ks + 16 (kg / 2) + 4 (kg % 2) + {0 .. 3, 8 .. 11}.
+  bf16x8 xq[4][2], xo[4][2];
+  {
+    const int ii = lane & 15, jj = ((ii & 1) << 1) | ((ii >> 1) & 1);
+    const int hd = 16 * (kg >> 1) + 4 * (kg & 1) + (ii >> 2);
+    auto column_operand = [&](int group, int c, int ks) {
+      const unsigned char* p = smem + group * 8192 + (32 * ks + hd) * 128 + (((2 * c + (jj >> 1)) ^ (hd & 7)) << 4) + (jj & 1) * 8;
+      return tr_pair(p, p + 8 * 128);
+    };
+    bf16x8 xr[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        xq[c][ks] = column_operand(wave, c, ks);
+        xo[c][ks] = column_operand(9 + wave, c, ks);
+      }
+      xr[ks] = column_operand(8, wave & 3, ks);      // rotary columns 16 (wave % 4) ..
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      asm volatile("" : "+v"(xq[0][ks]), "+v"(xq[1][ks]), "+v"(xq[2][ks]), "+v"(xq[3][ks]), "+v"(xr[ks]));
+      asm volatile("" : "+v"(xo[0][ks]), "+v"(xo[1][ks]), "+v"(xo[2][ks]), "+v"(xo[3][ks]));
+    }
+    __syncthreads();                           // every wave has its operands: the space is the ring's from here on
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) xr_s[64 * ks] = xr[ks];
+  }
+
+  // transfers of a tile, as in pass A: waves 0-3 take groups 0-4, waves 4-7 groups 5-8
+  const int gkey = (tid & 255) >> 3, gsub = tid & 7;
+  const int grp0 = hh * 5;
+  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16) + (unsigned)(grp0 * 128);
+  auto issue = [&](int n) {
+    int kid = idx_s[tlist[n] * BI + gkey];
+    kid = kid < 0 ? 0 : kid;
+    const unsigned goff = __umul24((unsigned)kid, DQK * 2) + gslot;       // (fewer than 2^24 rows: kv is at most 4 GiB)
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024 + grp0 * GRP_BYTES));
+#pragma unroll
+    for (int i = 0; i < 5 - hh; i++) dma16(lb + i * GRP_BYTES, goff + i * 128, kv);
+  };
+  for (int n = 0; n < STAGES - 1 && n < ntiles; n++) issue(n);
+
+  // accumulator i of a lane is head 16 hw + 4 kg + i, for key 16 hh + m
+  const float* stat = stat_s + hw * 16 + 4 * kg;
+  const int krow = 16 * hh + m;
+  unsigned boff[2];
+#pragma unroll
+  for (int par = 0; par < 2; par++) boff[par] = (unsigned)(krow * 128 + (((4 * par + kg) ^ (krow & 7)) << 4));
+  const unsigned half_chunk = (unsigned)((2 * hw + (kg & 1)) * 512 + krow * 16 + (kg >> 1) * 8);   // of the lane's key and 4 heads
+  const unsigned coff = (unsigned)(kg * 512 + m * 16);                 // coefficients of k-step ks (32 heads) and half tile kt: + 2048 ks + 256 kt
+  // the lane's 16 bytes of a row for a pair of column tiles: the lower half-wave has the first one's, lanes kg + 2 and kg trade
+  const unsigned coloff = (unsigned)(wave * 128 + g * 32 + (kg & 1) * 16);
+  const unsigned rotoff = (unsigned)(DV * 2 + (wave & 3) * 32 + ((kg & 1) * 2 + (kg >> 1)) * 8);
+  const float c2 = sm_scale * LOG2E;
+
+  // S, dP -> P, dS of tile n
+  auto phase_pds = [&](int n) {
+    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]);
+    const unsigned mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+    const unsigned char* tb = smem + (n % STAGES) * TILE_BYTES;
+    f32x4 sacc, dpacc;
+    constexpr int FD = 3;                      // operand reads in flight
+    bf16x8 f[FD];
+    auto operand = [&](int ks) { return *(const bf16x8*)(tb + (ks >> 1) * GRP_BYTES + boff[ks & 1]); };
+#pragma unroll
+    for (int j = 0; j < FD; j++) f[j] = operand(j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      mfma16_a(sacc, qreg[ks], f[ks % FD], ks == 0);
+      if (ks < DO_ACC) mfma16_a(dpacc, doreg[ks], f[ks % FD], ks == 0);
+      else if (ks < VS) mfma16_v(dpacc, doreg[ks], f[ks % FD], false);
+      if (ks + FD < KS) f[ks % FD] = operand(ks + FD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mfma16_done(sacc, dpacc);
+    const f32x4 lse2 = *(const f32x4*)stat, delta = *(const f32x4*)(stat + 64);
+    const bool valid = (mask >> krow) & 1u;
+    float pf[4], df[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[i], c2, -lse2[i])) : 0.f;
+      df[i] = pf[i] * (dpacc[i] - delta[i]) * sm_scale;
+    }
+    const uint2 pw = make_uint2(cvt_pk_bf16(pf[0], pf[1]), cvt_pk_bf16(pf[2], pf[3]));
+    const uint2 dw = make_uint2(cvt_pk_bf16(df[0], df[1]), cvt_pk_bf16(df[2], df[3]));
+    unsigned char* xb = xch + (n & 1) * FUSED_XCH + half_chunk;
+    *(uint2*)xb = dw;
+    *(uint2*)(xb + pds_kind_bytes(2)) = pw;
+    *(uint2*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(2) + half_chunk) = dw;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the rows of tile n
+  auto phase_rows = [&](int n) {
+    const unsigned char* xb = xch + (n & 1) * FUSED_XCH;
+    const int* drow = dst_s + tlist[n] * BI;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      bf16x8 cs[2], cp[2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        cs[ks] = *(const bf16x8*)(xb + ks * 2048 + coff + kt * 256);
+        cp[ks] = *(const bf16x8*)(xb + pds_kind_bytes(2) + ks * 2048 + coff + kt * 256);
+      }
+      unsigned char* row = rows + (size_t)drow[16 * kt + m] * ROW_BYTES;
+#pragma unroll
+      for (int cp2 = 0; cp2 < 2; cp2++) {
+        f32x4 acc[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) mfma16_v(acc[i], xq[2 * cp2 + i][ks], cs[ks], ks == 0);
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) mfma16_v(acc[i], xo[2 * cp2 + i][ks], cp[ks], false);
+        mfma16_done(acc[0], acc[1]);
+        unsigned w0[2], w1[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          w0[e] = cvt_pk_bf16(acc[0][2 * e], acc[0][2 * e + 1]);
+          w1[e] = cvt_pk_bf16(acc[1][2 * e], acc[1][2 * e + 1]);
+          swap_halves(w0[e], w1[e]);
+        }
+        *(uint4*)(row + cp2 * 64 + coloff) = make_uint4(w0[0], w0[1], w1[0], w1[1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (kt == hh) {
+        f32x4 acc;
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) mfma16_v(acc, xr_s[64 * ks], cs[ks], ks == 0);
+        mfma16_done(acc);
+        *(uint2*)(row + rotoff) = make_uint2(cvt_pk_bf16(acc[0], acc[1]), cvt_pk_bf16(acc[2], acc[3]));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+#pragma clang loop unroll(disable)
+  for (int n = 0; n <= ntiles; n++) {
+    asm volatile("" : "+s"(n));                // one copy of the loop: peeled ones cost registers
+    // A wave's operations behind the transfer of tile n, which went out two steps ago.  A step is 5 transfers (4 of waves 4-7), the
+    // dS store and 5 row stores.  The first tiles and the last one, behind which there are fewer, wait for all.
+    if (n < ntiles) {
+      if (n >= 3 && n + 1 < ntiles) { if (hh == 0) { DSA_WAIT_VMCNT(17); } else { DSA_WAIT_VMCNT(16); } }
+      else { DSA_WAIT_VMCNT(0); }
+    }
+    __syncthreads();
+    if (n + STAGES - 1 < ntiles) issue(n + STAGES - 1);       // ahead of the step's stores, which the transfers would queue behind
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (hh == 0) {
+      if (n < ntiles) phase_pds(n);
+      if (n > 0) phase_rows(n - 1);
+    } else {
+      if (n > 0) phase_rows(n - 1);
+      if (n < ntiles) phase_pds(n);
     }
   }
 }
@@ -953,6 +1236,18 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_kernel(
   pds_body<4, HG>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
 }
 
+__global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
+    const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    int q0, int cnt, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int ql = cnt - 1 - (int)blockIdx.x;
+  // (two copies of the body: every copy meets the same barriers)
+  if (threadIdx.x < 256) pds_rows_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+  else pds_rows_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+}
+
 template <int HG>
 __global__ __launch_bounds__(256, HG == 4 ? 1 : 2) void bwd_dkv_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
@@ -966,8 +1261,8 @@ __global__ __launch_bounds__(256, HG == 4 ? 1 : 2) void bwd_dkv_kernel(
     if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
     else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
   } else {
-    if (threadIdx.x < 128) dkv_few_body<5, HG>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-    else dkv_few_body<4, HG>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+    if (threadIdx.x < 128) dkv_few_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+    else dkv_few_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
   }
 }
 
@@ -1096,11 +1391,13 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   size_t smemB = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
   if (smemB < reduce_lds) smemB = reduce_lds;
   const size_t smemC = (size_t)(HG == 4 ? DKV_COEF_STAGES : DKV_FEW_STAGES) * pds_tile_bytes(HG) + ids_lds_bytes(K) + 16 + (size_t)(K + BI) * 4;
-  auto pds_kernel = HG == 1 ? bwd_pds_kernel<1> : HG == 2 ? bwd_pds_kernel<2> : bwd_pds_kernel<4>;
-  auto dkv_kernel = HG == 1 ? bwd_dkv_kernel<1> : HG == 2 ? bwd_dkv_kernel<2> : bwd_dkv_kernel<4>;
+  auto pds_kernel = HG == 1 ? bwd_pds_kernel<1> : bwd_pds_kernel<4>;
+  auto dkv_kernel = HG == 1 ? bwd_dkv_kernel<1> : bwd_dkv_kernel<4>;
   auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
-  if (dsa_reserve_lds((const void*)pds_kernel, smemA) != hipSuccess ||
-      dsa_reserve_lds((const void*)dkv_kernel, smemC) != hipSuccess ||
+  const bool one_pass = HG == 2;               // passes A and C
+  if ((one_pass ? dsa_reserve_lds((const void*)bwd_pds_rows_kernel, fused_lds_bytes(K)) != hipSuccess
+                : dsa_reserve_lds((const void*)pds_kernel, smemA) != hipSuccess ||
+                  dsa_reserve_lds((const void*)dkv_kernel, smemC) != hipSuccess) ||
       dsa_reserve_lds((const void*)dq_reduce_kernel, smemB) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
 
@@ -1131,13 +1428,21 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
-    pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
-                                                       (const __bf16*)dout, lse, pds, q0, cnt, H, Skv, K, q_start, sm_scale);
-    DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS)");
-    DSA_MARK(2);
-    dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
-                                                       H, Skv, K, q_start, p.chunk * K);
-    DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dKV rows)");
+    if (one_pass) {
+      bwd_pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), fused_lds_bytes(K), st>>>(
+          (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, Skv, K, q_start,
+          sm_scale, p.chunk * K);
+      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
+      DSA_MARK(2);
+    } else {
+      pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
+                                                         (const __bf16*)dout, lse, pds, q0, cnt, H, Skv, K, q_start, sm_scale);
+      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS)");
+      DSA_MARK(2);
+      dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
+                                                         H, Skv, K, q_start, p.chunk * K);
+      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dKV rows)");
+    }
     DSA_MARK(3);
     // Pass B of every query beside pass D of every key.
     dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smemB, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
