@@ -272,7 +272,7 @@ def main():
     torch.cuda.synchronize()
 
     t_idx = t_fwd = t_bwd = 0.0
-    t_pass = [0.0] * 5           # launch groups of the backward: order, pass A, pass C, passes B | D
+    t_pass = [0.0] * 5           # launch groups of the backward: order, passes A and C (one launch, then [2] is 0), passes B | D
     t_logits = t_topk = 0.0
     wall = 0.0
     for step in range(args.warmup + args.steps):
@@ -420,24 +420,25 @@ def main():
     del q_up, w_uk, w_uv, w_uk_t
 
     # what plain data movers with the traffic shape of the two bandwidth-bound backward passes reach:
-    # as many 1152-byte rows as the dKV pass writes, at scattered positions, beside a streaming read
-    # of 0.6 x that size (P, dS, Q, dO); and a streaming read of the rows (the ordered sum).  Source
-    # and destination are carved out of the backward's workspace, which is scratch between calls.
+    # as many 1152-byte rows as the launch that computes them writes, at scattered positions, beside a streaming read
+    # of 0.6 x that size (P, dS, Q, dO); and a streaming read of the rows (the ordered sum).  The
+    # destination lies in the backward's workspace, which is scratch between calls.
     rows_per_wg = int(pairs // S) // 4 * 4
     row_bytes = S * rows_per_wg * 1152
     steps4 = rows_per_wg // 4
     src_bytes = S * (steps4 // 5 * 3 + min(steps4 % 5, 3)) * 4608
     mover = None
-    if row_bytes + src_bytes + 256 <= wsb:
-        src_ptr = ws.data_ptr() + (row_bytes + 255) // 256 * 256
+    if row_bytes <= wsb:
+        mover_src = torch.empty(src_bytes, dtype=torch.uint8, device=dev)
         sink = torch.zeros(16, dtype=torch.uint8, device=dev)
-        t_rows, _ = timed(lambda: _lib.check(blib.dsa_probe_hbm_rows(src_ptr, ws.data_ptr(), S, rows_per_wg, 3, 1, stream),
+        t_rows, _ = timed(lambda: _lib.check(blib.dsa_probe_hbm_rows(mover_src.data_ptr(), ws.data_ptr(), S, rows_per_wg, 3, 1, stream),
                                              "probe rows", blib))
         t_read, _ = timed(lambda: _lib.check(blib.dsa_probe_hbm_read(ws.data_ptr(), row_bytes, sink.data_ptr(), stream),
                                              "probe read", blib))
+        del mover_src
         mover = {"rows_written_scattered_plus_stream_read_gbps": round((row_bytes + src_bytes) / (t_rows * 1e-3) / 1e9, 1),
                  "stream_read_gbps": round(row_bytes / (t_read * 1e-3) / 1e9, 1),
-                 "note": "plain movers with the byte counts and access shape of bwd_dkv_kernel and bwd_reduce_kernel"}
+                 "note": "plain movers with the byte counts and access shape of the row writes of bwd_pds_rows_kernel and of the ordered sum"}
 
     # what the matrix pipes sustain when a kernel issues nothing but bf16 MFMAs (about 20 ms of them)
     probe_flops = ctypes.c_double(0.0)
@@ -454,16 +455,15 @@ def main():
     # move, and - when a counter profile of exactly these sources is committed - the measured traffic.
     nq = float(S)
     b_q, b_do, b_o = nq * H * DQK * 2, nq * H * DV * 2, nq * H * DV * 2
-    b_pds = 512.0 * pairs                     # bf16 P and dS, 128 heads, per pair
+    b_ds = 256.0 * pairs                      # bf16 dS, 128 heads, per pair
     b_rows = 1152.0 * pairs                   # one bf16 row of 576 per pair
     b_dq, b_dkv = nq * H * DQK * 2, float(S) * DQK * 2
-    pass_names = ["order", "bwd_pds_kernel (S, dP -> P, dS)", "bwd_dkv_kernel (dKV rows)",
-                  "bwd_dq_reduce_kernel (dQ beside the ordered dKV sum)"]
-    pass_flops = [0.0, 2.0 * H * (DQK + DV) * pairs, 2.0 * H * (DQK + DV) * pairs, 2.0 * H * DQK * pairs]
-    pass_bytes = [8.0 * pairs, b_q + b_do + b_o + b_pds, b_pds + b_rows + b_q + b_do,
-                  0.5 * b_pds + b_dq + b_rows + S * DQK * 4.0]
+    pass_names = ["order", "bwd_pds_rows_kernel (S, dP -> dS, dKV rows)", "bwd_dq_reduce_kernel (dQ beside the ordered dKV sum)"]
+    t_pass = [t_pass[0], t_pass[1] + t_pass[2], t_pass[3]]
+    pass_flops = [0.0, 4.0 * H * (DQK + DV) * pairs, 2.0 * H * DQK * pairs]
+    pass_bytes = [8.0 * pairs, b_q + b_do + b_o + b_ds + b_rows, b_ds + b_dq + b_rows + S * DQK * 4.0]
     kernels = [("mla_fwd_kernel", t_fwd, flops_fwd, b_q + b_o)]
-    kernels += [(pass_names[i], t_pass[i], pass_flops[i], pass_bytes[i]) for i in range(4)]
+    kernels += [(pass_names[i], t_pass[i], pass_flops[i], pass_bytes[i]) for i in range(3)]
     name, t_dom, f_dom, b_dom = max(kernels, key=lambda k: k[1])
     traffic, traffic_note = None, "no counter profile committed for these kernel sources"
     tpath = os.path.join(ROOT, "profiles", "traffic.json")   # HBM bytes per launch from rocprofv3 counter runs
@@ -527,7 +527,7 @@ def main():
         "mla_fwd_ms": round(t_fwd, 3), "mla_bwd_ms": round(t_bwd, 3),
         "mla_fwd_tflops": round(flops_fwd / (t_fwd * 1e-3) / 1e12, 1),
         "mla_bwd_tflops": round(flops_bwd / (t_bwd * 1e-3) / 1e12, 1),
-        "mla_bwd_pass_ms": {pass_names[i]: round(t_pass[i], 3) for i in range(4)},
+        "mla_bwd_pass_ms": {pass_names[i]: round(t_pass[i], 3) for i in range(3)},
         "indexer_topk_ms": round(t_idx, 3), "indexer_topk_launch": "one HIP graph of the four launches (quantise q, quantise k, logits, top-k)",
         "indexer_topk_tokens_per_s": round(S / (t_idx * 1e-3), 1),
         "indexer_topk_ms_back_to_back": round(t_idx_alone, 3),

@@ -2,18 +2,18 @@
 //
 // Per (query, selected key) pair the backward needs five products:
 //   S  = Q.KV^T (576)   dP = dO.V^T (512)   dQ += dS.KV (576)   dKV[key] += dS^T.Q (576) + P^T.dO (512)
-// The operands Q and dO of one query (278 KB in bf16) plus the fp32 dQ accumulators (295 KB) do
-// not fit one compute unit (512 KB of registers, 160 KB of LDS) next to the gathered key tiles, and
-// the products over d and over heads need the same operands in two register orientations.  The
-// work is therefore split into passes that each keep ONE orientation resident in registers:
-//   pass A  (bwd_pds_kernel)   S and dP per 32-key tile -> P and dS, written to HBM as bf16 in the
-//                              exact MFMA operand layout of pass C (16 KB per query and tile)
-//   pass B  (bwd_dq_kernel)    dQ^T += KV^T.dS^T, both operands by LDS transpose reads
-//   pass C  (bwd_dkv_kernel)   per-pair rows  dS^T.Q + P^T.dO  (sum over all 128 heads) -> one
-//                              bf16 row of 576 values
-//                              in a pair buffer, at the position given by a key-sorted order
-//   pass D  (bwd_reduce_kernel) dKV[key] = sum of that key's rows, in ascending query order
-// With 64 heads both orientations fit, and passes A and C are one (bwd_pds_rows_kernel).
+// The operands Q and dO of one query (278 KB in bf16 with 128 heads) plus the fp32 dQ accumulators
+// (295 KB) do not fit one compute unit (512 KB of registers, 160 KB of LDS) next to the gathered key
+// tiles, and the products over d and over heads need the same operands in two orientations.  The work
+// is therefore split into passes:
+//   pass A  S and dP per 32-key tile -> P and dS; dS goes to HBM as bf16 for pass B, 8 KB per query and tile
+//   pass B  dQ^T += KV^T.dS^T, both operands by LDS transpose reads
+//   pass C  per-pair rows  dS^T.Q + P^T.dO  (sum over all heads) -> one bf16 row of 576 values in a pair
+//           buffer, at the position given by a key-sorted order
+//   pass D  dKV[key] = sum of that key's rows, in ascending query order
+// Passes A and C are one kernel (bwd_pds_rows_kernel) where both orientations can be kept, from 64 heads
+// on; with 32 heads they are two (bwd_pds_kernel, bwd_dkv_kernel), and P and dS pass through HBM in the
+// MFMA operand layout of pass C.  Passes B and D share a launch (bwd_dq_reduce_kernel).
 // The key-sorted order (pass 0) comes from a bitmap key x query, its row-wise prefix popcounts and
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
@@ -26,7 +26,7 @@ using namespace mla;
 // P or dS of one (query, tile): [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes are
 // compiled for: 1 or 2, or 4 for 96 and 128 heads.  In memory a tile is dS and then P; dS alone where passes A and C are one.
 constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
-constexpr int pds_tile_bytes(int HG) { return HG == 2 ? pds_kind_bytes(HG) : 2 * pds_kind_bytes(HG); }
+constexpr int pds_tile_bytes(int HG) { return HG >= 2 ? pds_kind_bytes(HG) : 2 * pds_kind_bytes(HG); }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
@@ -34,30 +34,23 @@ constexpr int PDS_THREADS = 512;
 // ---------------------------------------------------------------------------------------------
 // pass A: P and dS of every (query, tile)
 // ---------------------------------------------------------------------------------------------
-// One workgroup of eight waves per query; wave w owns heads [16w, 16w+16).  S = Q.KV^T and dP = dO.V^T
-// are 16x16x32 MFMAs with the heads on the rows (Q and dO rows resident in registers, 8 d-values per
-// lane and step) and the 16 keys of a half tile on the columns (key rows read from LDS, one 1 KB read
-// feeding both products).  At under 256 registers per lane two waves share a SIMD.  Measured against
-// four waves of 32 heads with 32x32x16 MFMAs (one wave per SIMD, half the LDS reads): the backward
-// takes 14.5 instead of 15.1 ms; LDS reads (288 KB per tile) and the MFMAs (2176 clocks per tile and
-// SIMD) are then about level.  A lane ends with 4 heads x 2 half tiles; lanes 32 apart trade halves
-// (one v_permlane32_swap per register pair) so that every lane holds one key's 8 heads in the chunk
-// order pass C reads: chunk group 2w + g = heads 16w + {4g .. 4g+3, 8+4g .. 8+4g+3}.
-// With up to 32 heads two waves hold them all: waves 4-7 take every other tile (two tiles per step, STAGES = 4 tiles are then
-// two steps), and a wave takes one half tile of its tile only.  (Idle or repeated heads cost as much as real ones.)
-template <int STAGES, int HG>
+// With up to 32 heads, one workgroup of eight waves per query.  S = Q.KV^T and dP = dO.V^T are 16x16x32 MFMAs with the heads on the
+// rows (Q and dO rows resident in registers, 8 d-values per lane and step) and the 16 keys of a half tile on the columns (key rows
+// read from LDS, one 1 KB read feeding both products).  Two waves hold all heads, so waves 4-7 take every other tile (two tiles per
+// step, STAGES = 4 tiles are then two steps), and a wave takes one half tile of its tile only.  (Idle or repeated heads cost as much
+// as real ones.)  A lane ends with 4 heads of one key, half a chunk in the order pass C reads: chunk group 2w + g = heads 16w +
+// {4g .. 4g+3, 8+4g .. 8+4g+3}.
+template <int STAGES>
 __device__ __forceinline__ void pds_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, int q0, int ql, int H, int Skv, int K, int q_start, float sm_scale,
     unsigned char* smem) {
   constexpr int KS = DQK / 32, VS = DV / 32;   // 18 and 16 steps of 32 d-values
-  constexpr int NKT = HG == 1 ? 1 : 2;         // half tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4;
-  const int hw = wave & (2 * HG - 1);          // heads 16 hw ..
-  const int kt0 = HG == 1 ? (wave >> 1) & 1 : 0;
+  const int hw = wave & 1, kt = (wave >> 1) & 1;       // heads 16 hw .., half tile of the tile
   const int qi = q0 + ql;
   const int NT = K / BI;
   int* idx_s = (int*)(smem + STAGES * TILE_BYTES);
@@ -98,35 +91,24 @@ __device__ __forceinline__ void pds_body(
   for (int ks = 0; ks < VS; ks++) asm volatile("" : "+v"(oreg[ks]));
 
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  // transfers of a tile: thread (key, sub) of either half of the workgroup moves 16 bytes of a 128-byte
-  // group of the key's row; waves 0-3 take groups 0-4, waves 4-7 groups 5-8 (a fifth step does nothing)
-  const int hh = wave >> 2;
-  const int gkey = (tid & 255) >> 3, gsub = tid & 7;
-  // Within a 128-byte group the 16-byte chunk c of key row r sits in slot c ^ (r & 7).  (The slot function of
+  // Transfers of a tile: each half of the workgroup moves its own; thread (key, sub) moves 16 bytes of every 128-byte group of the
+  // key's row.  Within a group the 16-byte chunk c of key row r sits in slot c ^ (r & 7).  (The slot function of
   // the other kernels' tiles also serves their transposing reads; with it this kernel's reads - 16 rows x 4
   // chunks per instruction - take two LDS cycles where one is needed.)
-  // (two tiles per step: each half of the workgroup moves its own tile, all nine groups)
-  const int grp0 = HG == 4 ? hh * 5 : 0;
-  constexpr int NSTEP = HG == 4 ? 5 : 9;
-  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16) + (unsigned)(grp0 * 128);
+  const int hh = wave >> 2;
+  const int gkey = (tid & 255) >> 3, gsub = tid & 7;
+  constexpr int NSTEP = 9;
+  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16);
   unsigned t_goff = 0, t_lb = 0;
   auto issue_prepare = [&](int n) {
     const int tile = tlist[n];
     int kid = idx_s[tile * BI + gkey];
     kid = kid < 0 ? 0 : kid;
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
-    t_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024 + grp0 * GRP_BYTES));
+    t_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024));
   };
-  auto issue_step = [&](int i) {
-    if (HG != 4 || hh == 0 || i < 4) dma16(t_lb + i * GRP_BYTES, t_goff + i * 128, kv);
-  };
-  if (HG == 4) {
-    for (int n = 0; n < STAGES - 1 && n < ntiles; n++) {
-      issue_prepare(n);
-#pragma unroll
-      for (int i = 0; i < NSTEP; i++) issue_step(i);
-    }
-  } else if (hh < ntiles) {
+  auto issue_step = [&](int i) { dma16(t_lb + i * GRP_BYTES, t_goff + i * 128, kv); };
+  if (hh < ntiles) {
     issue_prepare(hh);
 #pragma unroll
     for (int i = 0; i < NSTEP; i++) issue_step(i);
@@ -150,79 +132,43 @@ __device__ __forceinline__ void pds_body(
   const f32x4 lse2 = *(const f32x4*)(stat_s + hw * 16 + 4 * kg);
   const f32x4 delta = *(const f32x4*)(stat_s + 128 + hw * 16 + 4 * kg);
 
-  // key-row operand of half tile kt and step ks: row 16*kt + m, 16-byte chunk 4*ks + kg of the row
-  unsigned boff[NKT][2];
+  // key-row operand of step ks: row 16*kt + m, 16-byte chunk 4*ks + kg of the row
+  const int krow = 16 * kt + m;
+  unsigned boff[2];
 #pragma unroll
-  for (int kt = 0; kt < NKT; kt++)
-#pragma unroll
-    for (int par = 0; par < 2; par++) {
-      const int row = 16 * (kt0 + kt) + m;
-      boff[kt][par] = (unsigned)(row * 128 + (((4 * par + kg) ^ (row & 7)) << 4));
-    }
+  for (int par = 0; par < 2; par++) boff[par] = (unsigned)(krow * 128 + (((4 * par + kg) ^ (krow & 7)) << 4));
   const float c2 = sm_scale * LOG2E;
 
-  f32x4 sacc[NKT], dpacc[NKT];
-  // P and dS of the accumulated tile: the lane's 4 heads for its key of either half tile are two
-  // registers (4 bf16) each
+  f32x4 sacc, dpacc;
+  // P and dS of the accumulated tile: the lane's 4 heads for its key, two registers (4 bf16) each
   auto finish = [&](int tile, unsigned mask) {
-    unsigned pw[NKT][2], dw[NKT][2];
+    const bool valid = (mask >> krow) & 1u;
+    float pf[4], df[4];
 #pragma unroll
-    for (int kt = 0; kt < NKT; kt++) {
-      const bool valid = (mask >> (16 * (kt0 + kt) + m)) & 1u;
-      float pf[4], df[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], c2, -lse2[i])) : 0.f;
-        df[i] = pf[i] * (dpacc[kt][i] - delta[i]) * sm_scale;
-      }
-      pw[kt][0] = cvt_pk_bf16(pf[0], pf[1]); pw[kt][1] = cvt_pk_bf16(pf[2], pf[3]);
-      dw[kt][0] = cvt_pk_bf16(df[0], df[1]); dw[kt][1] = cvt_pk_bf16(df[2], df[3]);
+    for (int i = 0; i < 4; i++) {
+      pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[i], c2, -lse2[i])) : 0.f;
+      df[i] = pf[i] * (dpacc[i] - delta[i]) * sm_scale;
     }
-    unsigned char* base = pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG);
-    if constexpr (NKT == 1) {
-      // half a chunk per lane: heads 4 kg .. of its key
-      base += (size_t)(2 * hw + (kg & 1)) * 512 + (16 * kt0 + m) * 16 + (kg >> 1) * 8;
-      *(uint2*)base = make_uint2(dw[0][0], dw[0][1]);
-      *(uint2*)(base + pds_kind_bytes(HG)) = make_uint2(pw[0][0], pw[0][1]);
-    } else {
-      // lanes 32 apart trade: the lower lane keeps half tile 0 and gets the partner's heads of it, the
-      // upper lane keeps half tile 1.  Afterwards (x[0], x[1]) is the chunk of key 16*(lane/32) + m:
-      // heads 4g .. 4g+3 then 8+4g .. 8+4g+3 of the wave's 16, g = kg & 1.
-#pragma unroll
-      for (int r2 = 0; r2 < 2; r2++) {
-        swap_halves(pw[0][r2], pw[1][r2]);
-        swap_halves(dw[0][r2], dw[1][r2]);
-      }
-      const int key = 16 * (lane >> 5) + m, g = kg & 1;
-      base += (size_t)(2 * hw + g) * 512 + key * 16;
-      *(uint4*)base = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
-      *(uint4*)(base + pds_kind_bytes(HG)) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
-    }
+    unsigned char* base = pds + ((size_t)ql * NT + tile) * pds_tile_bytes(1) + (size_t)(2 * hw + (kg & 1)) * 512 + krow * 16 + (kg >> 1) * 8;
+    *(uint2*)base = make_uint2(cvt_pk_bf16(df[0], df[1]), cvt_pk_bf16(df[2], df[3]));
+    *(uint2*)(base + pds_kind_bytes(1)) = make_uint2(cvt_pk_bf16(pf[0], pf[1]), cvt_pk_bf16(pf[2], pf[3]));
   };
   // S and dP of a tile in LDS; `more`: with the transfers of a later tile between the products
   auto products = [&](const unsigned char* tb, bool more) {
 #pragma unroll
-    for (int kt = 0; kt < NKT; kt++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) { sacc[kt][e] = 0.f; dpacc[kt][e] = 0.f; }
-    // step j = NKT * ks + kt; FD operand reads in flight
-    constexpr int FD = 4;
+    for (int e = 0; e < 4; e++) { sacc[e] = 0.f; dpacc[e] = 0.f; }
+    constexpr int FD = 4;                      // operand reads in flight
     bf16x8 f[FD];
-    auto operand = [&](int j) {
-      const int ks = j / NKT, kt = j % NKT;
-      return *(const bf16x8*)(tb + (ks >> 1) * GRP_BYTES + boff[kt][ks & 1]);
-    };
+    auto operand = [&](int ks) { return *(const bf16x8*)(tb + (ks >> 1) * GRP_BYTES + boff[ks & 1]); };
 #pragma unroll
     for (int j = 0; j < FD; j++) f[j] = operand(j);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < NKT * KS; j++) {
-      const int ks = j / NKT, kt = j % NKT;
-      sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[ks], f[j % FD], sacc[kt], 0, 0, 0);
-      if (ks < VS) dpacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(doreg[ks], f[j % FD], dpacc[kt], 0, 0, 0);
-      if (j + FD < NKT * KS) f[j % FD] = operand(j + FD);
-      constexpr int EVERY = HG == 4 ? 7 : NKT * KS / NSTEP, AT = HG == 1 ? 1 : 2;
-      if (j % EVERY == AT && more) issue_step(j / EVERY);
+    for (int ks = 0; ks < KS; ks++) {
+      sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[ks], f[ks % FD], sacc, 0, 0, 0);
+      if (ks < VS) dpacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(doreg[ks], f[ks % FD], dpacc, 0, 0, 0);
+      if (ks + FD < KS) f[ks % FD] = operand(ks + FD);
+      if (ks % 2 == 1 && more) issue_step(ks / 2);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -232,65 +178,25 @@ __device__ __forceinline__ void pds_body(
   // w + 4) are thus half a step apart: the arithmetic and stores of one run under the other's MFMAs.
   int tile = 0;
   unsigned mask = 0;
-  if constexpr (HG != 4) {
-    // two tiles per step, one per half of the workgroup; the next step's are in flight
-    for (int i = 0; 2 * i < ntiles; i++) {
-      const int n = 2 * i + hh;
-      // behind the tile's transfers: the two stores of the step before (waves 0-3), nothing (waves 4-7)
-      if (hh == 0 && i > 0) { DSA_WAIT_VMCNT(2); } else { DSA_WAIT_VMCNT(0); }
-      __syncthreads();
-      if (hh == 1 && i > 0) finish(tile, mask);
-      if (n < ntiles) {
-        const bool more = n + 2 < ntiles;
-        if (more) issue_prepare(n + 2);
-        tile = __builtin_amdgcn_readfirstlane(tlist[n]);
-        mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
-        __builtin_amdgcn_sched_barrier(0);
-        products(smem + (n % STAGES) * TILE_BYTES, more);
-        if (hh == 0) finish(tile, mask);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    if (hh == 1 && ntiles > 1 && (ntiles & 1) == 0) finish(tile, mask);      // (odd counts: done in the last step)
-    return;
-  }
-  for (int n = 0; n < ntiles; n++) {
-    // operations a lane issued after this tile's transfers: D per later tile in flight (5 in waves
-    // 0-3, 4 in waves 4-7), 2 stores per finished tile (waves 4-7 are one tile behind with those)
-    {
-      const int ahead = min(STAGES - 2, ntiles - 1 - n);
-      if (hh == 0) {
-        constexpr int D = 5;
-        const int behind = min(n, STAGES - 1);
-        if (ahead == STAGES - 2 && behind == STAGES - 1) { DSA_WAIT_VMCNT(D * (STAGES - 2) + 2 * (STAGES - 1)); }
-        else if (ahead == STAGES - 2) { DSA_WAIT_VMCNT(D * (STAGES - 2)); }
-        else if (ahead >= 1) { DSA_WAIT_VMCNT(D); }
-        else { DSA_WAIT_VMCNT(0); }
-      } else {
-        constexpr int D = 4;             // (their stores of a step come before its transfers)
-        const int behind = min(n - 1, STAGES - 2);
-        if (ahead == STAGES - 2 && behind == STAGES - 2) { DSA_WAIT_VMCNT(D * (STAGES - 2) + 2 * (STAGES - 2)); }
-        else if (ahead == STAGES - 2) { DSA_WAIT_VMCNT(D * (STAGES - 2)); }
-        else if (ahead >= 1) { DSA_WAIT_VMCNT(D); }
-        else { DSA_WAIT_VMCNT(0); }
-      }
-    }
+  // two tiles per step, one per half of the workgroup; the next step's are in flight
+  for (int i = 0; 2 * i < ntiles; i++) {
+    const int n = 2 * i + hh;
+    // behind the tile's transfers: the two stores of the step before (waves 0-3), nothing (waves 4-7)
+    if (hh == 0 && i > 0) { DSA_WAIT_VMCNT(2); } else { DSA_WAIT_VMCNT(0); }
     __syncthreads();
-    // the next tile's transfers go out one at a time between the MFMA steps below: issued together they
-    // would hold every wave at the address unit, which takes 64 bytes per clock for the compute unit
-    const bool more = n + STAGES - 1 < ntiles;
-    if (more) issue_prepare(n + STAGES - 1);
-    const int prev_tile = tile;
-    const unsigned prev_mask = mask;
-    tile = __builtin_amdgcn_readfirstlane(tlist[n]);
-    mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
-    if (hh == 1 && n > 0) finish(prev_tile, prev_mask);
-    __builtin_amdgcn_sched_barrier(0);
-    products(smem + (n % STAGES) * TILE_BYTES, more);
-    if (hh == 0) finish(tile, mask);
-    __builtin_amdgcn_sched_barrier(0);
+    if (hh == 1 && i > 0) finish(tile, mask);
+    if (n < ntiles) {
+      const bool more = n + 2 < ntiles;
+      if (more) issue_prepare(n + 2);
+      tile = __builtin_amdgcn_readfirstlane(tlist[n]);
+      mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+      __builtin_amdgcn_sched_barrier(0);
+      products(smem + (n % STAGES) * TILE_BYTES, more);
+      if (hh == 0) finish(tile, mask);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
-  if (hh == 1 && ntiles > 0) finish(tile, mask);
+  if (hh == 1 && ntiles > 1 && (ntiles & 1) == 0) finish(tile, mask);      // (odd counts: done in the last step)
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -480,248 +386,20 @@ __device__ __forceinline__ void dq_body(
 // ---------------------------------------------------------------------------------------------
 // pass C: per-pair dKV rows
 // ---------------------------------------------------------------------------------------------
-// row[key, d] = sum_h dS[h,key] Q[h,d] + (d < 512) sum_h P[h,key] dO[h,d], all 128 heads, as
-// row^T = X^T . coef with X = [Q; dO] (k = heads).  X^T is the register-resident operand: wave w
-// owns the 32-column d-tiles {w, w+4, w+8, w+12, w+16} (the last only for w < 2) and loads its
-// columns once per query through LDS transpose reads.  The 16 coefficient operands of a tile
-// (pass-A layout, read from LDS as stored) also sit in registers, so a column tile is finished by
-// 16 (or 8) back-to-back MFMAs on one accumulator.  Everything else runs in the shadow of the
-// matrix pipe, a few instructions after each MFMA: while column tile c+1 accumulates, tile c is
-// rounded to bf16, its four 8-byte pieces per lane are turned into two 16-byte pieces by a trade
-// between the half-waves (the accumulator already holds one key per lane), and these are stored
-// as 32-byte halves of the tile's 64 bytes in each of its 32 rows, at the positions of the
-// key-sorted order; while the last column tile of a tile accumulates, the coefficient registers are
-// refilled for the next tile.  The loop touches LDS for the coefficients only (16 reads per wave
-// and tile).  One barrier per tile (the coefficient transfer is shared by the four waves); the
-// per-pair rows are bf16.
-constexpr int DKV_COEF_STAGES = 5;           // coefficient tiles in the LDS ring
-
-// NC = column tiles of this wave (5 for waves 0 and 1, else 4).
+// row[key, d] = sum_h dS[h,key] Q[h,d] + (d < 512) sum_h P[h,key] dO[h,d], as row^T = X^T . coef with
+// X = [Q; dO] (k = heads).  With up to 32 heads X^T takes 72 registers: wave w owns the 32-column d-tiles
+// {w, w+4, w+8, w+12, w+16} (the last only for w < 2) and loads its columns once per query through LDS
+// transpose reads; two workgroups share a compute unit and hide each other's set-up, barriers and stores.
+// The coefficients arrive in pass A's layout, read from LDS as stored; a column tile is rounded to bf16, its four 8-byte
+// pieces per lane are turned into two 16-byte pieces by a trade between the half-waves, and these are stored as 32-byte halves of
+// the tile's 64 bytes in each of its 32 rows.  Bound by the rows.
+constexpr int DKV_STAGES = 4;            // coefficient tiles in the LDS ring
 template <int NC>
 __device__ __forceinline__ void dkv_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
     const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
-  constexpr int CST = DKV_COEF_STAGES;
-  constexpr int NU = NC == 5 ? 9 : 8;          // units of 8 MFMAs per tile
-  // [CST][pds_tile_bytes(4)] coefficient ring, shared with the set-up's per-wave X staging [4][8192] |
-  // ids arrays | dst rows of the query [K + 32]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 31, g = lane >> 5;
-  const int qi = q0 + ql;
-  const int NT = K / BI;
-  unsigned char* xs = smem + wave * 8192;
-  int* idx_s = (int*)(smem + CST * pds_tile_bytes(4));
-  unsigned* tmask = (unsigned*)(idx_s + K);
-  int* tlist = (int*)(tmask + NT);
-  int* ntile_s = tlist + NT;
-  int* dst_s = ntile_s + 4;
-  for (int t0 = tid; t0 < K + BI; t0 += 8 * 256) {   // eight loads in flight per thread
-    int d[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) d[i] = t0 + i * 256 < K ? dst[(size_t)ql * K + t0 + i * 256] : -1;
-#pragma unroll
-    for (int i = 0; i < 8; i++)       // invalid slots land in a scratch row: the store count stays fixed
-      if (t0 + i * 256 < K + BI) dst_s[t0 + i * 256] = d[i] >= 0 ? d[i] : dummy_row;
-  }
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
-  if (ntiles == 0) return;
-
-  // ---- X^T operands: x?[c][kk], kk = 2*w' + s' over the 8 groups of 16 heads ------------------
-  // Q columns 0..3 and all dO columns live in accumulation registers (MFMA reads them there), the
-  // fifth Q column, the coefficients and the accumulators in architectural registers.
-  bf16x8 xqa[4][8], xqv[8], xo[4][8];
-  {
-    typedef short i16x8 __attribute__((ext_vector_type(8)));
-    const int blk = lane >> 4, ii = lane & 15;
-    // transpose read of a [128 heads][32 d] block (64-byte rows): lane points at head
-    // 32w' + 8(2s'+t) + 4g + ii/4, d chunk 16*(blk&1) + 4*(ii&3)
-    const unsigned xoff = (unsigned)((4 * g + (ii >> 2)) * 64 + (16 * (blk & 1) + 4 * (ii & 3)) * 2);
-    constexpr int NP = NC + 4;                 // passes: Q column tiles, then dO column tiles
-    uint4 ld[3][8];                            // three passes of global loads in flight
-    auto pass_load = [&](int pass, uint4 (&dstv)[8]) {
-      const bool isq = pass < NC;
-      const int ci = isq ? pass : pass - NC;
-      const int c = wave + 4 * ci;
-      const __bf16* src = isq ? q + (size_t)qi * H * DQK + 32 * c : dout + (size_t)qi * H * DV + 32 * c;
-      const int stride = isq ? DQK : DV;
-      // rows of 64 bytes: lane covers head (lane/4 + 16*it), 16-byte piece lane%4
-#pragma unroll
-      for (int it = 0; it < 8; it++) {
-        const int hh = (lane >> 2) + 16 * it;
-        dstv[it] = make_uint4(0, 0, 0, 0);
-        if (hh < H) dstv[it] = *(const uint4*)(src + (size_t)hh * stride + (lane & 3) * 8);
-      }
-    };
-    pass_load(0, ld[0]);
-    pass_load(1, ld[1]);
-    pass_load(2, ld[2]);
-#pragma unroll
-    for (int pass = 0; pass < NP; pass++) {
-      const bool isq = pass < NC;
-      const int ci = isq ? pass : pass - NC;
-#pragma unroll
-      for (int it = 0; it < 8; it++) *(uint4*)(xs + ((lane >> 2) + 16 * it) * 64 + (lane & 3) * 16) = ld[pass % 3][it];
-      if (pass + 3 < NP) pass_load(pass + 3, ld[pass % 3]);
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int kk = 0; kk < 8; kk++) {
-        const unsigned char* hb = xs + (32 * (kk >> 1) + 16 * (kk & 1)) * 64;
-        i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + xoff));
-        i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + 8 * 64 + xoff));
-        const bf16x8 val = __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
-        if (!isq) xo[ci][kk] = val;
-        else if (ci < 4) xqa[ci][kk] = val;
-        else xqv[kk] = val;
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-#pragma unroll
-    for (int kk = 0; kk < 8; kk++) {
-#pragma unroll
-      for (int ci = 0; ci < 4; ci++) asm volatile("" : "+a"(xqa[ci][kk]));
-      if (NC == 5) asm volatile("" : "+v"(xqv[kk]));
-#pragma unroll
-      for (int ci = 0; ci < 4; ci++) asm volatile("" : "+a"(xo[ci][kk]));
-    }
-  }
-  __syncthreads();                             // the X staging shares LDS with the coefficient ring
-
-  const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  auto issue = [&](int n) {
-    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % CST) * pds_tile_bytes(4) + wave * 1024));
-    const unsigned char* src = uniform_ptr(pds + ((size_t)ql * NT + tlist[n]) * pds_tile_bytes(4));
-#pragma unroll
-    for (int c = 0; c < 4; c++) dma16(lb + c * 4096, (unsigned)(c * 4096 + tid * 16), src);
-  };
-  // Vector-memory operations retire in issue order, so "the transfer of tile t has landed" is a
-  // bound on the number of operations issued after it: `issued` counts every operation of this
-  // wave, mk[j] is the count right after the transfer of the (j+1)-th tile ahead.  Stores younger
-  // than the awaited transfer stay in flight: the deeper the ring, the more of them.
-  int issued = 0;
-  int mk[CST - 1];
-#pragma unroll
-  for (int j = 0; j < CST - 1; j++) mk[j] = 0;
-  auto issue_marked = [&](int n) {
-    if (n < ntiles) {
-      issue(n);
-      issued += 4;
-    }
-    return issued;
-  };
-  // coefficient chunk of k-step kk: [kind][kk][g][key r] 16 bytes
-  const unsigned coff = (unsigned)(g * 512 + r * 16);
-  bf16x8 cf[16];
-  issue_marked(0);
-  mk[0] = issue_marked(1);
-  if (ntiles > 1) { DSA_WAIT_VMCNT(4); } else { DSA_WAIT_VMCNT(0); }
-  __syncthreads();
-#pragma unroll
-  for (int j = 1; j < CST - 1; j++) mk[j] = issue_marked(j + 1);
-#pragma unroll
-  for (int k = 0; k < 16; k++) cf[k] = *(const bf16x8*)(smem + k * 1024 + coff);
-
-  // copy-out state: the rounded column tile in flight (four 8-byte pieces, then two 16-byte ones) and
-  // the pointer to this lane's 16 bytes in the row of its key (lane & 31), first column tile of the wave
-  const size_t lane_off = (size_t)(wave * 64 + g * 16);
-  unsigned char* rptr = rows + (size_t)dummy_row * ROW_BYTES + lane_off;
-  unsigned pc[4][2];
-#pragma unroll
-  for (int j = 0; j < 4; j++) pc[j][0] = pc[j][1] = 0u;
-  uint4 piece[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-  f32x16 acc[5];
-#pragma unroll
-  for (int e = 0; e < 16; e++) acc[NC - 1][e] = 0.f;   // rounded (to the scratch row) before its first MFMA
-
-  // tasks of column tile ci, spread over MFMA slots: round (4 slots), trade between the half-waves
-  // (2 slots: piece it = elements 16*it + 8*g .. +7 of the lane's key), store (2 slots of the following unit)
-  auto conv = [&](int ci, int j) {
-    pc[j][0] = cvt_pk_bf16(acc[ci][4 * j], acc[ci][4 * j + 1]);
-    pc[j][1] = cvt_pk_bf16(acc[ci][4 * j + 2], acc[ci][4 * j + 3]);
-  };
-  auto piece_read = [&](int it) {
-    const int jj = 2 * it;
-    swap_halves(pc[jj][0], pc[jj + 1][0]);
-    swap_halves(pc[jj][1], pc[jj + 1][1]);
-    piece[it] = make_uint4(pc[jj][0], pc[jj][1], pc[jj + 1][0], pc[jj + 1][1]);
-  };
-  auto piece_store = [&](int ci, int it) {
-    *(uint4*)(rptr + ci * 256 + it * 32) = piece[it];
-    issued += 1;
-  };
-  // Operations a wave has issued, in the steady state, since the transfer it waits for at unit 6 of a
-  // tile (that of the next tile, issued CST - 1 tiles earlier): the stores of unit 7 (and 8) of that
-  // tile, CST - 2 whole tiles of 4 transfers + 2 NC stores, and this tile's stores before unit 6.
-  constexpr int STEADY = 2 + (CST - 2) * (4 + 2 * NC) + (NC == 5 ? 8 : 6);
-  static_assert(STEADY <= 63, "the vector-memory counter holds 63 at most");
-
-  for (int n = 0; n < ntiles; n++) {
-    const int tile = tlist[n];
-    const int drow = dst_s[tile * BI + r];
-    const unsigned char* nb = smem + ((n + 1) % CST) * pds_tile_bytes(4);   // next tile's coefficients
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int ci = u < 8 ? u >> 1 : 4, half = u < 8 ? (u & 1) : 0;
-      // column tile finished one unit ago (rounded now) and two units ago (stored now)
-      const int p1 = (u + NU - 1) % NU, p2 = (u + NU - 2) % NU;
-      const int conv_ci = p1 == 8 ? 4 : ((p1 & 1) ? p1 >> 1 : -1);
-      const int store_ci = p2 == 8 ? 4 : ((p2 & 1) ? p2 >> 1 : -1);
-      const bool reload = half == 1 ? u == 7 : u == (NC == 5 ? 8 : 6);
-      if (u == 6) {
-        // the next tile's coefficients have landed once at most (issued - mk[0]) younger operations
-        // are in flight; anything below the steady-state count (first and last tiles of a query)
-        // waits for everything, which is always enough
-        if (n + 1 < ntiles) {
-          if (issued - mk[0] >= STEADY) { DSA_WAIT_VMCNT(STEADY); } else { DSA_WAIT_VMCNT(0); }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j + 1 < CST - 1; j++) mk[j] = mk[j + 1];
-        mk[CST - 2] = issue_marked(n + CST);
-      }
-      if (u == 2) rptr = rows + (size_t)drow * ROW_BYTES + lane_off;      // all stores of the previous tile are issued
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int m = 0; m < 8; m++) {
-        const bf16x8 b = cf[half * 8 + m];
-        if (half == 1) {
-          mfma_v_av(acc[ci], xo[ci][m], b);
-        } else if (ci == 4) {
-          if (m == 0) mfma_v_vv_first(acc[4], xqv[m], b); else mfma_v_vv(acc[4], xqv[m], b);
-        } else {
-          if (m == 0) mfma_v_av_first(acc[ci], xqa[ci][m], b); else mfma_v_av(acc[ci], xqa[ci][m], b);
-        }
-        if (reload) cf[half * 8 + m] = *(const bf16x8*)(nb + (half * 8 + m) * 1024 + coff);
-        if (conv_ci >= 0 && m >= 2 && m < 6) conv(conv_ci, m - 2);
-        if (conv_ci >= 0 && m >= 6) piece_read(m - 6);
-        if (store_ci >= 0 && (m == 3 || m == 4)) piece_store(store_ci, m - 3);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-  }
-  // ---- drain: the last tile's final column tiles -------------------------------------------------
-  if (NC == 5) {
-    piece_store(3, 0);
-    piece_store(3, 1);
-  }
-  mfma_done_v(acc[NC - 1]);
-#pragma unroll
-  for (int j = 0; j < 4; j++) conv(NC - 1, j);
-  piece_read(0);
-  piece_read(1);
-  piece_store(NC - 1, 0);
-  piece_store(NC - 1, 1);
-}
-
-// The same with up to 32 heads: the operands of a query take 72 registers, two workgroups share a compute unit and hide each
-// other's set-up, barriers and stores, and the products are plain builtins in the compiler's order.  Bound by the rows.
-constexpr int DKV_FEW_STAGES = 4;
-template <int NC>
-__device__ __forceinline__ void dkv_few_body(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
-    const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
-  constexpr int HG = 1, CST = DKV_FEW_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
+  constexpr int HG = 1, CST = DKV_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
   // [CST][TB] coefficient ring, shared with the set-up's per-wave X staging [4][HG * 2048] | ids arrays | dst rows [K]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1119,6 +797,325 @@ __device__ __forceinline__ void pds_rows_body(
 }
 
 // ---------------------------------------------------------------------------------------------
+// passes A and C in one, for 96 and 128 heads
+// ---------------------------------------------------------------------------------------------
+// Both orientations of 128 heads are 557 KB; registers (512 KB) and LDS (160 KB) hold them together with the tile because what
+// lies in LDS serves either orientation: row reads for the products over d, transposing reads for those over the heads.  In LDS:
+// the first 32 of every 64 columns of dO (64 KB) and the rotary columns of Q (16 KB).  In registers (192 per lane): Q and the
+// other columns of dO by rows (wave w: heads 16 w ..) and by columns (wave w: columns 64 w ..).
+// That leaves room for one tile and one buffer of P and dS, so a step has two halves with a barrier each: S, dP -> P, dS of the
+// tile; then the transfer of the next tile starts and the rows are multiplied and stored under it.
+// 7700 cycles a step at 8192 queries x 2048 slots x 128 heads, 4352 of them in the matrix pipe (46 % busy; a pass costs 75 000
+// more for its set-up, 557 KB through LDS): the 816 LDS reads, 36 KB of transfers and 37 KB of stores of a step share the way
+// between the registers and LDS or cache, and hold each other up: LDS reads slow down by half while a tile arrives.  8.7 ms where
+// the two passes took 4.15 + 5.55, with 8 KB less to write and 16 KB less to read per tile.  Slower than this form, though each
+// has fewer LDS reads: 32x32x16 products for the rows (644, stores of 32 bytes in 32 rows), all column tiles at once (704, the
+// stores of a step together at its end), and waves 0-3 for P, dS beside waves 4-7 for the rows, with the next tile's first groups
+// ahead (640): 8 - 12 % each.
+constexpr int WIDE_ROT = 65536;                        // behind dO's columns [4 pairs of 64][128 heads][2 x 32 columns]
+constexpr int WIDE_TILE = WIDE_ROT + 16384;
+constexpr int WIDE_XCH = WIDE_TILE + TILE_BYTES;
+constexpr int WIDE_LISTS = 128 * DQK * 2;              // Q of the query fits in front of the lists before the rest is there
+static_assert(WIDE_XCH + 2 * pds_kind_bytes(4) <= WIDE_LISTS && WIDE_TILE + 65536 <= WIDE_LISTS, "the lists lie behind everything else");
+inline size_t wide_lds_bytes(int K) { return (size_t)WIDE_LISTS + ids_lds_bytes(K) + 1024 + 2048; }
+
+template <int hh>
+__device__ __forceinline__ void pds_rows_wide_body(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
+    const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    int q0, int ql, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
+  constexpr int VS = DV / 32;
+  constexpr int XQ_ACC = 7;                    // column operands of Q in accumulation registers, beside all row operands: 124
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qi = q0 + ql;
+  const int NT = K / BI;
+  unsigned char* xch = smem + WIDE_XCH;
+  int* idx_s = (int*)(smem + WIDE_LISTS);
+  unsigned* tmask = (unsigned*)(idx_s + K);
+  int* tlist = (int*)(tmask + NT);
+  int* ntile_s = tlist + NT;
+  float* stat_s = (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
+  int* dst_s = (int*)(stat_s + 256);           // [2][256]: destination rows from the tile's first slot on
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  // Registers are short: what depends on the lane is worked out anew for every part.
+  auto fresh_lane = []() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+  };
+
+  // Rows of Q and dO travel to LDS in groups of 128 bytes of all 128 rows, chunk c of row r in slot c ^ (r & 7).  Wave w moves rows
+  // 8 w .. 8 w + 7 and 64 + 8 w ..; heads beyond H repeat the last one (their P and dS are zero).
+  const unsigned char* q_rows = (const unsigned char*)uniform_ptr(q + (size_t)qi * H * DQK);
+  const unsigned char* do_rows = (const unsigned char*)uniform_ptr(dout + (size_t)qi * H * DV);
+  const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
+  auto group_base = [](int p) { return p < 4 ? p * 16384 : p < 8 ? WIDE_TILE + (p - 4) * 16384 : WIDE_ROT; };
+  {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++) {
+      const unsigned src = (unsigned)min(64 * rb + 8 * wave + (l >> 3), H - 1) * (DQK * 2) + ((l & 7) ^ (l >> 3)) * 16;
+#pragma unroll
+      for (int p = 0; p < 9; p++) dma16(lb + rb * 8192 + group_base(p), src + p * 128, q_rows);
+    }
+  }
+  bf16x8 doreg[VS / 2];                        // dO, the odd 32 columns
+  {
+    const int m = lane & 15, kg = lane >> 4;
+    const int h = wave * 16 + m;
+    const bool head_ok = h < H;
+    const size_t hrow = (size_t)qi * H + (head_ok ? h : 0);
+    const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
+    const bf16x8* dp = (const bf16x8*)(dout + hrow * DV) + kg;
+    bf16x8 o[VS], d[VS];
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++) { d[ks] = dp[4 * ks]; o[ks] = op[4 * ks]; }
+    const float lse_h = lse[hrow];
+    __builtin_amdgcn_sched_barrier(0);
+    float part = 0.f;                          // delta = rowsum(O . dO)
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) part = fmaf((float)o[ks][e], (float)d[ks][e], part);
+      if (ks & 1) {
+        doreg[ks >> 1] = d[ks];
+        asm volatile("" : "+a"(doreg[ks >> 1]));
+      }
+    }
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    if (kg == 0) {
+      stat_s[h] = head_ok ? lse_h * LOG2E : INFINITY;
+      stat_s[128 + h] = head_ok ? part : 0.f;
+    }
+  }
+  // (the helper is written for four waves; the other four repeat part of its work with equal results)
+  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  DSA_WAIT_VMCNT(0);
+  if (ntiles == 0) return;
+  __syncthreads();
+
+  // ---- resident operands: rows of Q (32 columns each) and of dO (the columns that are not in LDS), columns of both ----
+  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  auto tr_pair = [&](const unsigned char* p) {             // 16 columns by the heads of chunk kg: 8 rows apart
+    const i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p));
+    const i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, p + 8 * 128));
+    return __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // Operand rows as in the body for 64 heads: row 4 j + e is column {0, 8, 4, 12}[j] + e of 16, chunk kg of k-step ks holds heads
+  // 32 ks + 16 (kg / 2) + 4 (kg % 2) + {0 .. 3, 8 .. 11}
+  auto tr_off = [](int l, int chunk) {
+    const int ii = l & 15, jj = ((ii & 1) << 1) | ((ii >> 1) & 1), hd = 16 * (l >> 5) + 4 * ((l >> 4) & 1) + (ii >> 2);
+    return (unsigned)(hd * 128 + (((chunk + (jj >> 1)) ^ (hd & 7)) << 4) + (jj & 1) * 8);
+  };
+  auto row_off = [](int l, int par) {          // row l % 16 of 16, an even or odd 32 columns of a group
+    return (unsigned)((l & 15) * 128 + (((4 * par + (l >> 4)) ^ (l & 7)) << 4));
+  };
+  bf16x8 qreg[VS], xq[4][4], xo[2][4];
+  {
+    const int l = fresh_lane();
+    const unsigned off[2] = {2048 * wave + row_off(l, 0), 2048 * wave + row_off(l, 1)};
+#pragma unroll
+    for (int ks = 0; ks < VS; ks++) {
+      qreg[ks] = *(const bf16x8*)(smem + group_base(ks >> 1) + off[ks & 1]);
+      asm volatile("" : "+a"(qreg[ks]));
+    }
+  }
+  {
+    const int l = fresh_lane();
+    const unsigned char* xg = smem + (wave < 4 ? wave * 16384 : WIDE_TILE + (wave - 4) * 16384);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) {
+        xq[c][ks] = tr_pair(xg + ks * 4096 + tr_off(l, 2 * c));
+        if (4 * c + ks < XQ_ACC) asm volatile("" : "+a"(xq[c][ks]));
+        else asm volatile("" : "+v"(xq[c][ks]));
+      }
+  }
+  __syncthreads();                             // dO takes the place of Q's first groups
+  // dO: pair j of 64 columns, its first 32 of either to stay, the second 32 to pass through
+  {
+    const int l = fresh_lane(), sw = (l & 7) ^ (l >> 3);
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++) {
+      const unsigned src = (unsigned)min(64 * rb + 8 * wave + (l >> 3), H - 1) * (DV * 2) + (sw >> 2) * 128 + (sw & 3) * 16;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        dma16(lb + rb * 8192 + j * 16384, src + j * 256, do_rows);
+        dma16(lb + rb * 8192 + WIDE_TILE + j * 16384, src + j * 256 + 64, do_rows);
+      }
+    }
+  }
+  DSA_WAIT_VMCNT(0);
+  __syncthreads();
+  {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) {
+        xo[c][ks] = tr_pair(smem + WIDE_TILE + (wave >> 1) * 16384 + ks * 4096 + tr_off(l, 4 * (wave & 1) + 2 * c));
+        asm volatile("" : "+v"(xo[c][ks]));
+      }
+  }
+  __syncthreads();
+
+  const int ln = fresh_lane();
+  const int lm = ln & 15, lk = ln >> 4, lg = ln >> 5;
+  // transfers of a tile: waves 0-3 take groups 0-4, waves 4-7 groups 5-8; wave 7 the tile's destination rows
+  const int grp0 = hh * 5;
+  const unsigned tile_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(WIDE_TILE + (wave & 3) * 1024 + grp0 * GRP_BYTES));
+  auto issue = [&](int n) {
+    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]), l = fresh_lane();
+    int kid = idx_s[tile * BI + 8 * (wave & 3) + (l >> 3)];
+    kid = kid < 0 ? 0 : kid;
+    const unsigned goff = __umul24((unsigned)kid, DQK * 2) + (unsigned)(((l & 7) ^ (l >> 3)) * 16 + grp0 * 128);       // (fewer than 2^24 rows: kv is at most 4 GiB)
+#pragma unroll
+    for (int i = 0; i < 5 - hh; i++) dma16(tile_lb + i * GRP_BYTES, goff + i * 128, kv);
+    // 1 KB from the tile's first slot on (behind the last query's slots the workspace goes on with the sorted list)
+    if (wave == 7) dma16(lds0 + (unsigned)((unsigned char*)dst_s - smem) + (n & 1) * 1024, (unsigned)l * 16, dst + (size_t)ql * K + tile * BI);
+  };
+  issue(0);
+
+  // accumulator i of a lane is head 16 wave + 4 lk + i, for key 16 kt + lm
+  unsigned boff[2], loff[2];                   // row operands of even and odd 32 columns: of a key, of the lane's head
+#pragma unroll
+  for (int par = 0; par < 2; par++) {
+    boff[par] = (unsigned)WIDE_TILE + row_off(ln, par);
+    loff[par] = (unsigned)(2048 * wave) + row_off(ln, par);
+  }
+  const unsigned chunk = (unsigned)((2 * wave + (lk & 1)) * 512 + (16 * lg + lm) * 16);  // after the trade: 8 heads of key 16 lg + lm
+  const unsigned coff = (unsigned)(lk * 512 + lm * 16);                // coefficients of k-step ks and half tile kt: + 2048 ks + 256 kt
+  const unsigned coloff = (unsigned)(wave * 128 + lg * 32 + (lk & 1) * 16);
+  const unsigned rotoff = (unsigned)(DV * 2 + (wave & 3) * 32 + ((lk & 1) * 2 + (lk >> 1)) * 8);
+  // column operands: dO of the first column tile (the second one's: ^ 32), rotary columns
+  const unsigned tr_do = (unsigned)((wave >> 1) * 16384) + tr_off(ln, 4 * (wave & 1)), tr_rot = (unsigned)WIDE_ROT + tr_off(ln, 2 * (wave & 3));
+  const float c2 = sm_scale * LOG2E;
+
+  // S, dP -> P, dS of tile n
+  auto phase_pds = [&](int n) {
+    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]);
+    const unsigned mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+    f32x4 sacc[2], dpacc[2];
+    constexpr int NJ = 2 * (DQK / 32), FD = 3;
+    bf16x8 f[FD], x;                           // key rows of step j = 2 ks + kt; row operand from LDS: dO of even ks, Q of the rotary ks
+    auto operand = [&](int j) { return *(const bf16x8*)(smem + (j >> 2) * GRP_BYTES + (j & 1) * 2048 + boff[(j >> 1) & 1]); };
+    x = *(const bf16x8*)(smem + loff[0]);
+#pragma unroll
+    for (int j = 0; j < FD; j++) f[j] = operand(j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      const int ks = j >> 1, kt = j & 1;
+      if (ks < VS) {
+        mfma16_a(sacc[kt], qreg[ks < VS ? ks : 0], f[j % FD], ks == 0);
+        if (ks & 1) mfma16_a(dpacc[kt], doreg[ks < VS ? ks >> 1 : 0], f[j % FD], false);
+        else mfma16_v(dpacc[kt], x, f[j % FD], ks == 0);
+      } else {
+        mfma16_v(sacc[kt], x, f[j % FD], false);
+      }
+      if (j + FD < NJ) f[j % FD] = operand(j + FD);
+      if (kt == 1 && ks < VS - 2 && (ks & 1) == 0) x = *(const bf16x8*)(smem + ((ks + 2) >> 2) * 16384 + loff[((ks + 2) >> 1) & 1]);
+      if (kt == 1 && (ks == VS - 2 || ks == VS)) x = *(const bf16x8*)(smem + WIDE_ROT + loff[ks == VS]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_nop 15\n\ts_nop 3" : "+v"(sacc[0]), "+v"(sacc[1]), "+v"(dpacc[0]), "+v"(dpacc[1]));
+    const f32x4 lse2 = *(const f32x4*)(stat_s + wave * 16 + 4 * lk), delta = *(const f32x4*)(stat_s + 128 + wave * 16 + 4 * lk);
+    unsigned pw[2][2], dw[2][2];
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const bool valid = (mask >> (16 * kt + lm)) & 1u;
+      float pf[4], df[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], c2, -lse2[i])) : 0.f;
+        df[i] = pf[i] * (dpacc[kt][i] - delta[i]) * sm_scale;
+      }
+      pw[kt][0] = cvt_pk_bf16(pf[0], pf[1]); pw[kt][1] = cvt_pk_bf16(pf[2], pf[3]);
+      dw[kt][0] = cvt_pk_bf16(df[0], df[1]); dw[kt][1] = cvt_pk_bf16(df[2], df[3]);
+    }
+    // lanes 32 apart trade half tiles, as in pass A
+#pragma unroll
+    for (int r2 = 0; r2 < 2; r2++) {
+      swap_halves(pw[0][r2], pw[1][r2]);
+      swap_halves(dw[0][r2], dw[1][r2]);
+    }
+    const uint4 d16 = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
+    *(uint4*)(xch + chunk) = d16;
+    *(uint4*)(xch + pds_kind_bytes(4) + chunk) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
+    *(uint4*)(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(4) + chunk) = d16;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the rows of tile n
+  auto phase_rows = [&](int n) {
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const int drow = dst_s[(n & 1) * 256 + 16 * kt + lm];
+      f32x4 acc[4], rot;
+      bf16x8 cf[2], x[2];                      // coefficients of step k = 0 .. 3: dS . Q, 4 .. 7: P . dO; column operands from LDS
+      auto coef = [&](int k) { return *(const bf16x8*)(xch + k * 2048 + kt * 256 + coff); };
+      cf[0] = coef(0);
+      if (kt == hh) x[0] = tr_pair(smem + tr_rot);
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        if (k < 7) cf[(k + 1) & 1] = coef(k + 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int c = (i + 2) & 3;           // dO of column tiles 0 and 1 comes from LDS: those last
+          if (k >= 4) mfma16_v(acc[c], c < 2 ? x[c & 1] : xo[c & 1][k & 3], cf[k & 1], false);
+          else if (4 * c + k < XQ_ACC) mfma16_a(acc[c], xq[c][k & 3], cf[k & 1], k == 0);
+          else mfma16_v(acc[c], xq[c][k & 3], cf[k & 1], k == 0);
+          if (k >= 4 && k < 7 && c < 2) x[c & 1] = tr_pair(smem + (k - 3) * 4096 + (tr_do ^ (32u * c)));
+        }
+        if (kt == hh && k < 4) {
+          mfma16_v(rot, x[k & 1], cf[k & 1], k == 0);
+          if (k < 3) x[(k + 1) & 1] = tr_pair(smem + tr_rot + (k + 1) * 4096);
+        }
+        if (k == 3) {
+          x[0] = tr_pair(smem + tr_do);
+          x[1] = tr_pair(smem + (tr_do ^ 32u));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+      unsigned char* row = rows + (size_t)(drow >= 0 ? drow : dummy_row) * ROW_BYTES;       // invalid slots: a scratch row
+#pragma unroll
+      for (int pr = 0; pr < 2; pr++) {
+        unsigned w0[2], w1[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          w0[e] = cvt_pk_bf16(acc[2 * pr][2 * e], acc[2 * pr][2 * e + 1]);
+          w1[e] = cvt_pk_bf16(acc[2 * pr + 1][2 * e], acc[2 * pr + 1][2 * e + 1]);
+          swap_halves(w0[e], w1[e]);
+        }
+        *(uint4*)(row + pr * 64 + coloff) = make_uint4(w0[0], w0[1], w1[0], w1[1]);
+      }
+      if (kt == hh) {
+        mfma16_done(rot);
+        *(uint2*)(row + rotoff) = make_uint2(cvt_pk_bf16(rot[0], rot[1]), cvt_pk_bf16(rot[2], rot[3]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+#pragma clang loop unroll(disable)
+  for (int n = 0; n < ntiles; n++) {
+    asm volatile("" : "+s"(n));                // one copy of the loop: peeled ones cost registers
+    // behind the tile's transfers: the five row stores of the tile before
+    if (n > 0) { DSA_WAIT_VMCNT(5); } else { DSA_WAIT_VMCNT(0); }
+    __syncthreads();
+    phase_pds(n);
+    __syncthreads();
+    if (n + 1 < ntiles) issue(n + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    phase_rows(n);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // pass D: dKV[key] = sum of that key's rows, ascending query order
 // ---------------------------------------------------------------------------------------------
 // One key per workgroup (504 of its threads): 72 column chunks of 8 elements x 7 row groups (row r of the
@@ -1211,12 +1208,6 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
 // dispatch order, so that both kinds of work are in flight from the first workgroup to the last:
 //   bwd_dq_reduce_kernel   pass B of all queries | pass D of all keys      (4.5 ms against 2.6 + 2.75)
 // Within a role, the longest work (latest query, earliest key) comes first.
-// Passes A and C, carried by one launch in the same way (pass A of one block of queries beside
-// pass C of the block before it, 2 - 64 interleaved blocks), took as long side by side as one after
-// the other: neither gets faster when it has fewer compute units - a compute unit that alternates
-// cold loads (the P / dS tiles) with stores (the rows) drains either queue before it serves the
-// other, which bounds pass C per compute unit at about the rate at which HBM bounds it for the
-// whole chip.  They are separate kernels.
 struct RoleSlot { bool first; int i; };
 // nX workgroups of the first role and nY of the second, spread evenly over the launch: workgroup b belongs to the
 // second role when the count floor(b * nY / (nX + nY)) steps up after it.
@@ -1227,29 +1218,33 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-template <int HG>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  pds_body<4, HG>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
+  pds_body<4>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
 }
 
+template <int HG>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int cnt, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
+    int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int ql = cnt - 1 - (int)blockIdx.x;
   // (two copies of the body: every copy meets the same barriers)
-  if (threadIdx.x < 256) pds_rows_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-  else pds_rows_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+  if constexpr (HG == 2) {
+    if (threadIdx.x < 256) pds_rows_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+  } else {
+    if (threadIdx.x < 256) pds_rows_wide_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_wide_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
+  }
 }
 
-template <int HG>
-__global__ __launch_bounds__(256, HG == 4 ? 1 : 2) void bwd_dkv_kernel(
+__global__ __launch_bounds__(256, 2) void bwd_dkv_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
     const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int cnt, int H, int Skv, int K, int q_start, int dummy_row) {
@@ -1257,13 +1252,8 @@ __global__ __launch_bounds__(256, HG == 4 ? 1 : 2) void bwd_dkv_kernel(
   const int ql = cnt - 1 - (int)blockIdx.x;
   // waves 0 and 1 own five column tiles, waves 2 and 3 four: two copies of the whole body, so that
   // no branch sits between the MFMAs; every copy meets the same barriers
-  if constexpr (HG == 4) {
-    if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-    else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-  } else {
-    if (threadIdx.x < 128) dkv_few_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-    else dkv_few_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-  }
+  if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
+  else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
 }
 
 template <int HG>
@@ -1390,14 +1380,14 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
   size_t smemB = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
   if (smemB < reduce_lds) smemB = reduce_lds;
-  const size_t smemC = (size_t)(HG == 4 ? DKV_COEF_STAGES : DKV_FEW_STAGES) * pds_tile_bytes(HG) + ids_lds_bytes(K) + 16 + (size_t)(K + BI) * 4;
-  auto pds_kernel = HG == 1 ? bwd_pds_kernel<1> : bwd_pds_kernel<4>;
-  auto dkv_kernel = HG == 1 ? bwd_dkv_kernel<1> : bwd_dkv_kernel<4>;
+  const size_t smemC = (size_t)DKV_STAGES * pds_tile_bytes(1) + ids_lds_bytes(K) + 16 + (size_t)K * 4;
   auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
-  const bool one_pass = HG == 2;               // passes A and C
-  if ((one_pass ? dsa_reserve_lds((const void*)bwd_pds_rows_kernel, fused_lds_bytes(K)) != hipSuccess
-                : dsa_reserve_lds((const void*)pds_kernel, smemA) != hipSuccess ||
-                  dsa_reserve_lds((const void*)dkv_kernel, smemC) != hipSuccess) ||
+  const bool one_pass = HG >= 2;               // passes A and C
+  auto pds_rows_kernel = HG == 2 ? bwd_pds_rows_kernel<2> : bwd_pds_rows_kernel<4>;
+  const size_t smemAC = HG == 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
+  if ((one_pass ? dsa_reserve_lds((const void*)pds_rows_kernel, smemAC) != hipSuccess
+                : dsa_reserve_lds((const void*)bwd_pds_kernel, smemA) != hipSuccess ||
+                  dsa_reserve_lds((const void*)bwd_dkv_kernel, smemC) != hipSuccess) ||
       dsa_reserve_lds((const void*)dq_reduce_kernel, smemB) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
 
@@ -1429,17 +1419,17 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
     if (one_pass) {
-      bwd_pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), fused_lds_bytes(K), st>>>(
-          (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, Skv, K, q_start,
+      pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemAC, st>>>(
+          (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, H, Skv, K, q_start,
           sm_scale, p.chunk * K);
       DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
       DSA_MARK(2);
     } else {
-      pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
+      bwd_pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
                                                          (const __bf16*)dout, lse, pds, q0, cnt, H, Skv, K, q_start, sm_scale);
       DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS)");
       DSA_MARK(2);
-      dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
+      bwd_dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
                                                          H, Skv, K, q_start, p.chunk * K);
       DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dKV rows)");
     }

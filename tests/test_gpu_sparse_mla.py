@@ -211,6 +211,18 @@ def test_backward_of_few_heads(gpu, H, S, K, q_start, skv):
         assert (dq[2] == 0).all()
 
 
+@pytest.mark.parametrize("S,H,K,q_start", [
+    (1, 128, 64, 0),                  # one valid slot
+    (68, 96, 64, 0),                  # heads that repeat the last one; one and two tiles per query
+    (70, 128, 320, 0),                # up to ten tiles
+    (5, 128, 2048, 3000),             # the longest lists
+])
+def test_backward_of_many_heads_in_one_pass(gpu, S, H, K, q_start):
+    """P, dS and the rows of the pairs in one kernel: the first and the last tiles of a query, empty rows, the end of the order's
+    list, against the oracle, with the bounds of the other backward tests."""
+    test_backward_of_few_heads(gpu, H, S, K, q_start, None)
+
+
 def test_backward_does_not_depend_on_the_slot_order(gpu):
     """The backward walks each query's ids in ascending key order whatever order they arrive in, so
     permuting the slots (independently per query) and scattering unused slots between the used ones
