@@ -12,18 +12,16 @@
 // of the keys inside a tile, the B-operand layout of the second product, so P never touches LDS.
 // MFMA-bound: 2*H*(576+512) flop per (query, key) pair against 1152 gathered bytes.
 //
-// A 256-thread workgroup has four waves of up to 512 registers, one per SIMD.  How they share a
-// query's heads and slots is the MODE:
-//   0  128 heads, one tile at a time: wave w owns heads [32w, 32w + 32).
+// How a workgroup shares a query's heads and slots is the MODE:
+//   0  128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
 //   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
 //      of every other tile; the two streams' sums are merged through LDS at the end.
 //   2  32 heads, two tiles at a time: waves (stream, b) compute S^T of the same heads and own half
 //      of the value columns.
-// With fewer than 128 heads mode 0 leaves waves without work, at the same time per tile; modes 1
-// and 2 spend 68 / 52 matrix instructions per wave on two tiles instead of one and are then bound
-// by the gather.  A query's heads may also be spread over several workgroups, and its slots over
-// `ksplit` of them (few queries: one workgroup per query would leave most of the 256 compute units
-// idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
+// Modes 1 and 2 are mla_fwd_kernel: four waves of up to 512 registers, one per SIMD.  They spend 68 / 52 matrix
+// instructions per wave on two tiles and are then bound by the gather.  A query's heads may also be spread over several
+// workgroups, and its slots over `ksplit` of them (few queries: one workgroup per query would leave most of the 256
+// compute units idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
 #include "mla_tile.h"
 
 namespace {
@@ -65,7 +63,7 @@ struct FwdArgs {
 // slot range - and the kernel that follows does them again relative to the true row maximum.  In mode 2 with all slots in
 // one workgroup, where the waves' registers have room for it, the workgroup does so itself: the kernel that follows takes
 // 4.5 us also when nothing is marked.
-constexpr float REDO_ABOVE = 64.0f;
+constexpr float REDO_ABOVE = 64.0f, REDO_TERM = 0x1p64f;
 constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
 __device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
 
@@ -104,8 +102,8 @@ __device__ __forceinline__ float tile_max(const f32x16& sacc) {
   for (int e = 1; e < 16; e++) mx = fmaxf(mx, sacc[e]);
   return fmaxf(mx, __shfl_xor(mx, 32, 64));
 }
-// P of a tile relative to `ref` (base 2) as the B operand of the second product; l gains the lane's share of the sum
-__device__ __forceinline__ void softmax_numerators(const f32x16& sacc, float c2, float ref, float& l, bf16x8 (&pb)[2]) {
+// P of a tile relative to `ref` (base 2) as the B operand of the second product; returns the lane's share of the sum
+__device__ __forceinline__ float softmax_numerators(const f32x16& sacc, float c2, float ref, bf16x8 (&pb)[2]) {
   float psum = 0.f;
 #pragma unroll
   for (int s = 0; s < 2; s++)
@@ -115,7 +113,7 @@ __device__ __forceinline__ void softmax_numerators(const f32x16& sacc, float c2,
       psum += pe;
       pb[s][e] = (__bf16)pe;
     }
-  l += psum;
+  return psum;
 }
 // one 32 x 32 block of O^T (lane = head): to the workspace as it lies, or normalised to the lane's output row
 __device__ __forceinline__ void store_partial(const f32x16& t, f32x4* p) {
@@ -181,7 +179,7 @@ __device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int
       m = fmaxf(m, tile_max(sacc) * c2);
     } else {
       bf16x8 pb[2];
-      softmax_numerators(sacc, c2, m, l, pb);
+      l += softmax_numerators(sacc, c2, m, pb);
 #pragma unroll
       for (int s = 0; s < 2; s++)
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
@@ -199,37 +197,31 @@ __device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, in
   store_out(acc, fin.inv, (unsigned short*)a.out + ((size_t)qi * a.H + h) * DV + 32 * dt + 8 * g);
 }
 
-template <int MODE, int STAGES, bool SPLIT, int POUT>   // SPLIT: ksplit > 1; POUT: 0 none, 1 bf16, 2 f32
+template <int MODE, bool SPLIT, int POUT>    // MODE 1, 2; SPLIT: ksplit > 1; POUT: 0 none, 1 bf16, 2 f32
 __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
-  constexpr int STREAMS = MODE == 0 ? 1 : 2;
   constexpr int NDT = MODE == 2 ? DTILES / 2 : DTILES;      // value column tiles of a wave
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, g = lane >> 5;
-  const int stream = STREAMS == 2 ? wave >> 1 : 0, sub = wave & 1;
+  const int stream = wave >> 1, sub = wave & 1;
   const int S = a.S, H = a.H, K = a.K, p_skip = a.p_skip;
 
   // Workgroup -> (query, head group, slot range).  The head groups of one slot range gather the same rows:
   // they sit eight workgroups apart, i.e. on the same XCD and its L2.  Longest prefixes first.
-  int qi, hg = 0, sp = 0;
-  if (MODE == 0 && !SPLIT) {
-    qi = S - 1 - (int)blockIdx.x;
-  } else {
-    const int i = (int)blockIdx.x >> 3;
-    hg = i % a.n_hg;
-    const int u = (i / a.n_hg) * 8 + ((int)blockIdx.x & 7);
-    if (u >= S * (SPLIT ? a.ksplit : 1)) return;
-    qi = S - 1 - (SPLIT ? u / a.ksplit : u);
-    sp = SPLIT ? u % a.ksplit : 0;
-  }
+  const int i = (int)blockIdx.x >> 3;
+  const int hg = i % a.n_hg;
+  const int u = (i / a.n_hg) * 8 + ((int)blockIdx.x & 7);
+  if (u >= S * (SPLIT ? a.ksplit : 1)) return;
+  const int qi = S - 1 - (SPLIT ? u / a.ksplit : u);
+  const int sp = SPLIT ? u % a.ksplit : 0;
   const int qpos = a.q_start + qi;
   const int k0 = sp * a.k_loc;
   const int KL = min(a.k_loc, K - k0), NT = KL / BI;         // slots and tiles of this range
   const int tile0 = k0 / BI;
-  const int hb = MODE == 0 ? wave : (MODE == 1 ? 2 * hg + sub : hg);   // 32-head block of the wave
+  const int hb = MODE == 1 ? 2 * hg + sub : hg;              // 32-head block of the wave
 
-  constexpr int RING = STREAMS * STAGES * TILE_BYTES;
+  constexpr int RING = 4 * TILE_BYTES;       // the two tiles at work, the two on their way
   int* idx_s = (int*)(smem + RING);
   unsigned* tmask = (unsigned*)(idx_s + KL);
   int* tlist = (int*)(tmask + NT);
@@ -249,7 +241,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
 
   // ---- stage the ids, mark valid slots, list the tiles that have any ---------------------
   const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, qpos, idx_s, tmask, tlist, ntile_s);
-  const int nsteps = (ntiles + STREAMS - 1) / STREAMS;
+  const int nsteps = (ntiles + 1) / 2;
   // the slice must have landed before the gather pipeline starts: the loop below counts
   // outstanding vector-memory operations by hand
   DSA_WAIT_VMCNT(0);
@@ -260,7 +252,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
   if (POUT != 0 && head_ok && ntiles < NT) {
     for (int t = 0; t < NT; t++) {
-      if (tmask[t] != 0u || (tile0 + t) * BI < p_skip || (STREAMS == 2 && (t & 1) != stream)) continue;
+      if (tmask[t] != 0u || (tile0 + t) * BI < p_skip || (t & 1) != stream) continue;
       const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + t) * BI - p_skip) + 16 * g;
       if (POUT == 2) {
         const f32x4 ninf = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -274,25 +266,25 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
   }
 
-  // ---- gather of tile n of the list into ring slot n % (STREAMS * STAGES); lane-dependent LDS offsets ----
+  // ---- gather of tile n of the list into ring slot n % 4; lane-dependent LDS offsets ----
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   auto issue = [&](int n) {
-    gather_tile(a.kv, idx_s, tlist[min(n, ntiles - 1)], lds0 + (unsigned)((n % (STREAMS * STAGES)) * TILE_BYTES));
+    gather_tile(a.kv, idx_s, tlist[min(n, ntiles - 1)], lds0 + (unsigned)((n % 4) * TILE_BYTES));
   };
   // The same gather in single steps (one 128-byte group of the key rows of a tile each), issued between
   // MFMAs: nine transfers in a row hold the wave until the memory pipeline has taken them all (about 520
   // clocks per tile of 4200).
-  // (Two streams and an odd tile count: the last tile is gathered twice and masked out in the second stream.)
-  unsigned g_goff[STREAMS], g_lb[STREAMS];
+  // (An odd tile count: the last tile is gathered twice and masked out in the second stream.)
+  unsigned g_goff[2], g_lb[2];
   auto gather_prepare = [&](int n0) {
 #pragma unroll
-    for (int s = 0; s < STREAMS; s++) {
+    for (int s = 0; s < 2; s++) {
       const int n = n0 + s;
       const int gkey = tid >> 3, gsub = tid & 7;
       int kid = idx_s[tlist[min(n, ntiles - 1)] * BI + gkey];
       kid = kid < 0 ? 0 : kid;
       g_goff[s] = (unsigned)kid * (DQK * 2) + (unsigned)((gsub ^ swz(gkey)) * 16);
-      g_lb[s] = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % (STREAMS * STAGES)) * TILE_BYTES + wave * 1024));
+      g_lb[s] = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % 4) * TILE_BYTES + wave * 1024));
     }
   };
   auto gather_step = [&](int s, int grp) {
@@ -319,11 +311,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
       if (ks == 0) mfma_first(sacc, f[0], qreg[0]);
       else mfma_next(sacc, f[ks & 3], qreg[ks]);
       if (ks + 4 < KSTEPS) f[ks & 3] = *(const bf16x8*)(tb + ((ks + 4) >> 2) * GRP_BYTES + qk_off[ks & 3]);
-      if (STREAMS == 1) {
-        if (ks % 7 == 3 && gather) gather_step(0, ks / 7);                // groups 0 .. 4
-      } else {
-        if (ks % 2 == 1 && gather) gather_step((ks / 2) / 9, (ks / 2) % 9);   // all 18 of the next two tiles
-      }
+      if (ks % 2 == 1 && gather) gather_step((ks / 2) / 9, (ks / 2) % 9);     // all 18 of the next two tiles
       __builtin_amdgcn_sched_barrier(0);
     }
     mfma_chain_done(sacc);
@@ -336,43 +324,31 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
   };
 
-  auto issue_first = [&]() {
-    for (int n = 0; n < STREAMS * (STAGES - 1) && n < STREAMS * nsteps; n++) issue(n);
-  };
-
 #pragma unroll
   for (int dt = 0; dt < NDT; dt++) {
 #pragma unroll
     for (int e = 0; e < 16; e++) oacc[dt][e] = 0.f;
   }
-  issue_first();
+  for (int n = 0; n < 2 && n < 2 * nsteps; n++) issue(n);
   bool overflow = false;
-  int stores_after = 0;                      // p_out stores a wave issued after the transfers it waits for (two streams)
+  int stores_after = 0;                      // p_out stores a wave issued after the transfers it waits for
   for (int step = 0; step < nsteps; step++) {
-    if (STREAMS == 1) {
-      const int ahead = min(STAGES - 2, ntiles - 1 - step);   // tiles allowed to stay in flight
-      if (ahead >= 2) { DSA_WAIT_VMCNT(18); }
-      else if (ahead == 1) { DSA_WAIT_VMCNT(9); }
-      else { DSA_WAIT_VMCNT(0); }
-    } else {
-      static_assert(STREAMS == 1 || STAGES == 2, "one step of transfers in flight");
-      if (POUT != 0 && stores_after == 4) { DSA_WAIT_VMCNT(4); }
-      else if (POUT != 0 && stores_after == 2) { DSA_WAIT_VMCNT(2); }
-      else { DSA_WAIT_VMCNT(0); }
-    }
+    if (POUT != 0 && stores_after == 4) { DSA_WAIT_VMCNT(4); }
+    else if (POUT != 0 && stores_after == 2) { DSA_WAIT_VMCNT(2); }
+    else { DSA_WAIT_VMCNT(0); }
     __syncthreads();
-    const int next0 = STREAMS == 1 ? step + STAGES - 1 : STREAMS * (step + STAGES - 1);
+    const int next0 = 2 * (step + 1);
     const bool more = next0 < ntiles;
     if (more) gather_prepare(next0);
-    const int n = STREAMS * step + stream;
-    const bool real = STREAMS == 1 || n < ntiles;
+    const int n = 2 * step + stream;
+    const bool real = n < ntiles;
     const int tile = tlist[real ? n : ntiles - 1];
     const unsigned mask = real ? tmask[tile] : 0u;
-    const unsigned char* tb = smem + (n % (STREAMS * STAGES)) * TILE_BYTES;
+    const unsigned char* tb = smem + (n % 4) * TILE_BYTES;
 
     f32x16 sacc;
     qk_tile(tb, mask, sacc, more);
-    if (STREAMS == 2) stores_after = 0;
+    stores_after = 0;
     if (POUT != 0 && head_ok && real && (tile0 + tile) * BI >= p_skip) {
       const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + tile) * BI - p_skip);
       if (POUT == 2) {
@@ -389,17 +365,17 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
         if (MODE != 2 || sub == 0) *(uint4*)((unsigned short*)a.p_out + prow + 8 * g) = o[0];
         if (MODE != 2 || sub == 1) *(uint4*)((unsigned short*)a.p_out + prow + 16 + 8 * g) = o[1];
       }
-      if (STREAMS == 2) stores_after = POUT == 2 ? (MODE == 2 ? 2 : 4) : (MODE == 2 ? 0 : 2);
+      stores_after = POUT == 2 ? (MODE == 2 ? 2 : 4) : (MODE == 2 ? 0 : 2);
     }
 
     // ---- softmax numerators (base 2), one head per lane -----------------------------------
     {
       const float mx = tile_max(sacc) * c2;
-      if (step == 0) m_ref = STREAMS == 1 ? mx : fmaxf(mx, -1e30f);       // (a masked-out tile has the maximum -inf)
+      if (step == 0) m_ref = fmaxf(mx, -1e30f);       // (a masked-out tile has the maximum -inf)
       overflow |= (mx > m_ref + REDO_ABOVE);
     }
     bf16x8 pb[2];
-    softmax_numerators(sacc, c2, m_ref, l_run, pb);
+    l_run += softmax_numerators(sacc, c2, m_ref, pb);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- O^T += V^T . P^T -----------------------------------------------------------------
@@ -426,7 +402,6 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
             for (int t = 0; t < 2; t++)
               v[dt & 1][s][t] = read_tr(vb + ((dt + 2) >> 1) * GRP_BYTES + pv_off[s][t][dt & 1]);
         }
-        if (STREAMS == 1 && dt % 4 == 1 && more) gather_step(0, 5 + dt / 4);        // groups 5 .. 8
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -436,51 +411,47 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   bool again = __ballot(overflow) != 0ull;   // the same for all lanes of a wave
 
   f32x4* box = (f32x4*)(smem + (size_t)sub * NDT * 4096) + lane;
-  float mine = 1.0f;
   // ---- two streams: the second one's sums reach the first through the (now free) tile ring, scaled to the
   // common reference point; the first one's waves finish --------------------------------------------------
-  if (STREAMS == 2) {
-    __syncthreads();                         // the last tiles and the id arrays have been read
-    static_assert(STREAMS == 1 || 2 * NDT * 4096 + 1024 <= RING, "the hand-over fits the tile ring");
-    float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the two waves' boxes
-    if (g == 0) {
-      ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
-      ml[((stream * 2 + sub) * 32 + r) * 2 + 1] = l_tot;
-    }
-    __syncthreads();
-    const float m_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2], l_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2 + 1];
-    again |= is_marked(m_o);
-    if (MODE == 2 && !SPLIT && again) {      // the same for all waves: they have the same heads
-#pragma unroll 1
-      for (int dt = wave; dt < DTILES; dt += 4) {
-        f32x16 acc;
-        float m, l;
-        redo_block(a, qi, hb, dt, acc, m, l);
-        write_block(a, qi, hb, dt, acc, m, l);
-      }
-      return;
-    }
-    const float nm = fmaxf(m_ref, m_o);
-    const float f = __builtin_amdgcn_exp2f(m_ref - nm);
-    l_tot = l_tot * f + l_o * __builtin_amdgcn_exp2f(m_o - nm);
-    m_ref = nm;
-    if (stream == 1) {
-#pragma unroll
-      for (int dt = 0; dt < NDT; dt++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          f32x4 v;
-#pragma unroll
-          for (int e = 0; e < 4; e++) v[e] = oacc[dt][4 * j + e] * f;
-          box[(dt * 4 + j) * 64] = v;
-        }
-    }
-    __syncthreads();
-    if (stream == 1) return;
-    mine = f;
+  __syncthreads();                         // the last tiles and the id arrays have been read
+  static_assert(2 * NDT * 4096 + 1024 <= RING, "the hand-over fits the tile ring");
+  float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the two waves' boxes
+  if (g == 0) {
+    ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
+    ml[((stream * 2 + sub) * 32 + r) * 2 + 1] = l_tot;
   }
+  __syncthreads();
+  const float m_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2], l_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2 + 1];
+  again |= is_marked(m_o);
+  if (MODE == 2 && !SPLIT && again) {      // the same for all waves: they have the same heads
+#pragma unroll 1
+    for (int dt = wave; dt < DTILES; dt += 4) {
+      f32x16 acc;
+      float m, l;
+      redo_block(a, qi, hb, dt, acc, m, l);
+      write_block(a, qi, hb, dt, acc, m, l);
+    }
+    return;
+  }
+  const float nm = fmaxf(m_ref, m_o);
+  const float f = __builtin_amdgcn_exp2f(m_ref - nm);
+  l_tot = l_tot * f + l_o * __builtin_amdgcn_exp2f(m_o - nm);
+  m_ref = nm;
+  if (stream == 1) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = oacc[dt][4 * j + e] * f;
+        box[(dt * 4 + j) * 64] = v;
+      }
+  }
+  __syncthreads();
+  if (stream == 1) return;
+  const float mine = f;
   auto merged = [&](int dt) {                // column tile dt of the wave's heads, both streams
-    if (STREAMS == 1) return oacc[dt];
     f32x16 t;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -519,8 +490,309 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
 #pragma unroll
   for (int dt = 0; dt < NDT; dt++) {
     store_out(merged(dt), fin.inv, op + 32 * dt);
-    if (STREAMS == 2) __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// 128 heads: eight waves of up to 256 registers, two per SIMD, in two roles.
+//
+// Wave w < 4 makes the scores of heads 32 w ..: S^T of a tile (the Q slice, 144 registers, stays in place), the softmax, P to
+// LDS.  Wave 4 + w sums value columns 128 w .. of all heads, one tile behind, and issues the transfers.  So one wave's softmax,
+// transfers and waits pass under the other's matrix instructions; a wave that did both, alone on its SIMD, left the matrix
+// pipe idle for 1700 of the 3900 cycles a tile took.  Splitting the values by columns and not by heads also feeds four products from a
+// transposed operand instead of one: 16 such reads a tile and wave instead of 64, for 8 reads of P.  The value sums of four head
+// blocks and 128 columns are 256 registers; three of the sixteen 32 x 32 blocks (heads 0 .. 95, the last 32 columns) therefore live
+// in the scores' waves, which leaves 208 + 40 there and 144 + 48 + 32 here.  Accumulators and the first half of Q sit in
+// accumulation registers, the rest in architectural ones.
+// Measured with 8192 queries and 2048 slots, cycles a tile: scores 1350, softmax 630, their share of the values 440; the other
+// role transfers 640, products 1900: near 2650 in all, 2176 of them matrix instructions; LDS (77 reads a tile on each SIMD,
+// and the arriving tile) is close behind.  Forward 3.70 -> 3.33 ms, with the logits 4.39 -> 3.97; 1500 queries behind
+// a long prefix 809 -> 715 us.  Transfers spread over the products instead of first in the step: products
+// 2550 cycles (a transfer holds the wave, and the operand reads behind it); wave priorities: no difference.
+// ---------------------------------------------------------------------------------------------
+constexpr int WIDE_RING = 3;                 // tiles: the values of n, the scores of n + 1, the transfers of n + 2
+constexpr int P_BYTES = 4 * 2 * 1024;        // P of a tile, [32-head block][16 keys][lane] of 16 bytes
+constexpr int WIDE_LDS = WIDE_RING * TILE_BYTES + 2 * P_BYTES;
+constexpr int Q_ACC = 18;                    // k-steps of the Q slice in accumulation registers
+
+template <bool SCORES, bool SPLIT, int POUT>
+__device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsigned char* smem) {
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  const int H = a.H, K = a.K;
+  const int k0 = sp * a.k_loc;
+  const int KL = min(a.k_loc, K - k0), NT = KL / BI;
+  unsigned char* const pbuf = smem + WIDE_RING * TILE_BYTES;
+  int* idx_s = (int*)(smem + WIDE_LDS);
+  unsigned* tmask = (unsigned*)(idx_s + KL);
+  int* tlist = (int*)(tmask + NT);
+  float* const inv_s = (float*)pbuf;         // after the last tile
+
+  const int h = 32 * w + r;                  // of the scores
+  const bool head_ok = h < H;                // the same for all lanes of a wave
+  bf16x8 qreg[SCORES ? KSTEPS : 1];
+  if constexpr (SCORES) {
+    const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : 0)) * DQK) + g;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  if constexpr (SCORES) {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ks++) {
+      if (ks < Q_ACC) asm volatile("" : "+a"(qreg[ks]));
+      else asm volatile("" : "+v"(qreg[ks]));
+    }
+  }
+  if constexpr (SCORES) {
+    const unsigned row0 = (unsigned)(r * 128 + ((g ^ swz(r)) << 4));     // chunk 2 j + g of a group: row0 ^ 32 j
+    const int tile0 = k0 / BI, p_skip = a.p_skip;
+    // slots of tiles that are never visited still need their -inf in p_out
+    // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
+    if (POUT != 0 && head_ok && ntiles < NT) {
+      for (int t = 0; t < NT; t++) {
+        if (tmask[t] != 0u || (tile0 + t) * BI < p_skip) continue;
+        const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + t) * BI - p_skip) + 16 * g;
+        if (POUT == 2) {
+          const f32x4 ninf = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+          for (int j = 0; j < 4; j++) *(f32x4*)((float*)a.p_out + pbase + 4 * j) = ninf;
+        } else {
+          const uint4 ninf = make_uint4(0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u);
+#pragma unroll
+          for (int j = 0; j < 2; j++) *(uint4*)((unsigned short*)a.p_out + pbase + 8 * j) = ninf;
+        }
+      }
+    }
+    const float c2 = a.sm_scale * LOG2E;
+    float m_ref = -1e30f, l_run = 0.f;
+    bool overflow = false;
+    f32x16 o[3];                             // value columns 128 w + 96 .. of heads 0 .. 95
+#pragma unroll
+    for (int hb = 0; hb < 3; hb++) {
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[hb][e] = 0.f;
+      asm volatile("" : "+a"(o[hb]));
+    }
+    f32x16 s_acc;
+    auto chain = [&](unsigned tb) {
+      bf16x8 f[4];
+      const unsigned tb0 = tb + row0;
+      auto row = [&](int ks) { return *LDS_PTR(const bf16x8, (uintptr_t)((tb0 ^ (32 * (ks & 3))) + (ks >> 2) * GRP_BYTES)); };
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) f[ks] = row(ks);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++) {
+        if (ks == 0) mfma_v_va_first(s_acc, f[0], qreg[0]);
+        else if (ks < Q_ACC) mfma_v_va(s_acc, f[ks & 3], qreg[ks]);
+        else mfma_v_vv(s_acc, f[ks & 3], qreg[ks]);
+        if (ks + 4 < KSTEPS) f[ks & 3] = row(ks + 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      mfma_done_v(s_acc);
+    };
+    auto soft = [&](int n, int tile, unsigned mask) {        // the chain's tile n of the list: p_out, statistics, P to LDS
+      // accumulator e of this lane is key 8*(e/4) + 4*g + (e%4) of the tile
+      if (mask != 0xffffffffu) {
+        const unsigned mg = mask >> (4 * g);
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+          if (!((mg >> (8 * (e >> 2) + (e & 3))) & 1u)) s_acc[e] = -INFINITY;
+      }
+      if (POUT != 0 && head_ok && (tile0 + tile) * BI >= p_skip) {
+        const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + tile) * BI - p_skip);
+        if (POUT == 2) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            f32x4 v = {s_acc[4 * j], s_acc[4 * j + 1], s_acc[4 * j + 2], s_acc[4 * j + 3]};
+            *(f32x4*)((float*)a.p_out + prow + 4 * g + 8 * j) = v;
+          }
+        } else {
+          // A lane holds keys 8j + 4g .. +3 of its head (j = 0..3): 8-byte pieces.  The two half-waves
+          // trade pieces so that each lane ends up with 8 consecutive keys, twice: 16-byte stores.
+          uint4 t[2];
+          acc_row_to_16B(s_acc, 1.0f, t);
+          *(uint4*)((unsigned short*)a.p_out + prow + 8 * g) = t[0];
+          *(uint4*)((unsigned short*)a.p_out + prow + 16 + 8 * g) = t[1];
+        }
+      }
+      if (n == 0) m_ref = tile_max(s_acc) * c2;
+      bf16x8 pb[2];
+      const float sum = softmax_numerators(s_acc, c2, m_ref, pb);
+      l_run += sum;
+      overflow |= sum > REDO_TERM;           // one of the terms, or a few just below
+      bf16x8* const p = (bf16x8*)(pbuf + (n & 1) * P_BYTES + w * 2048) + lane;
+      p[0] = pb[0];
+      p[64] = pb[1];
+    };
+    unsigned tr0[2];                         // transposed reads of value columns 128 w + 96 .., [t]; 16 keys on: + 2048
+    { const LaneOffsets lo = lane_offsets(); tr0[0] = lo.tr_off[0][0][1]; tr0[1] = lo.tr_off[0][1][1]; }
+    auto values = [&](int n, int slot) {
+      const unsigned char* vb = smem + slot * TILE_BYTES + (2 * w + 1) * GRP_BYTES;
+      const bf16x8* const p = (const bf16x8*)(pbuf + (n & 1) * P_BYTES) + lane;
+      bf16x8 v[2], pr[2][3];
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        v[s] = value_operand(read_tr(vb + tr0[0] + 2048 * s), read_tr(vb + tr0[1] + 2048 * s));
+#pragma unroll
+        for (int hb = 0; hb < 3; hb++) pr[s][hb] = p[hb * 128 + s * 64];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int hb = 0; hb < 3; hb++) mfma_a_vv(o[hb], v[s], pr[s][hb]);
+    };
+    __syncthreads();                         // tile 0 has landed
+    int slot = -1;                           // of tile n
+    if (ntiles > 0) {
+      int tile_v = tlist[0];
+#pragma clang loop unroll(disable)
+      for (int n = -1; n < ntiles; n++) {
+        asm volatile("" : "+s"(n));          // one copy of the body: a peeled one costs registers
+        const int next = slot == WIDE_RING - 1 ? 0 : slot + 1;
+        const int tile = tile_v;
+        const unsigned mask = tmask[tile_v];
+        tile_v = tlist[min(n + 2, ntiles - 1)];
+        const unsigned tb = (unsigned)(uintptr_t)smem + next * TILE_BYTES;
+        if (n >= 0) values(n, slot);
+        if (n + 1 < ntiles) {
+          chain(tb);
+          soft(n + 1, __builtin_amdgcn_readfirstlane(tile), __builtin_amdgcn_readfirstlane(mask));
+        }
+        slot = next;
+        __syncthreads();
+      }
+    }
+    const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+    const bool again = __ballot(overflow) != 0ull;
+    if (SPLIT) {
+      if (head_ok && g == 0) {
+        float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
+        part_ml[0] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
+        part_ml[1] = l_tot;
+      }
+    } else {
+      const Final fin = finish_head(m_ref, l_tot, a.sink && head_ok ? a.sink + h : nullptr);
+      if (head_ok && g == 0) a.lse[(size_t)qi * H + h] = again ? __builtin_bit_cast(float, REDO_MARK) : fin.lse;
+      if (g == 0) inv_s[h] = fin.inv;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int hb = 0; hb < 3; hb++) {
+      mfma_done_a(o[hb]);
+      if (32 * hb < H) {
+        const int dt = 4 * w + 3;
+        if (SPLIT) store_partial(o[hb], a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt) * 256 + lane);
+        else store_out(o[hb], inv_s[32 * hb + r], (unsigned short*)a.out + ((size_t)qi * H + 32 * hb + r) * DV + 32 * dt + 8 * g);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    const LaneOffsets lo = lane_offsets();
+    const unsigned lds0 = (unsigned)(uintptr_t)smem;
+    const int gkey = (threadIdx.x & 255) >> 3, gsub = lane & 7;
+    const unsigned gsl = (unsigned)((gsub ^ swz(gkey)) * 16);
+    auto gather = [&](int n, int slot) {     // tile n of the list
+      const unsigned goff = (unsigned)max(idx_s[tlist[n] * BI + gkey], 0) * (DQK * 2) + gsl;
+      const unsigned lb = lds0 + slot * TILE_BYTES + w * 1024;
+#pragma unroll
+      for (int grp = 0; grp < 9; grp++) dma16(lb + grp * GRP_BYTES, goff + grp * 128, a.kv);
+    };
+    f32x16 oa[2][4], ov[4], o3;              // value columns 128 w + 32 i of head block hb: i = 0, 1; i = 2; i = 3, the last block
+#pragma unroll
+    for (int hb = 0; hb < 4; hb++) {
+#pragma unroll
+      for (int e = 0; e < 16; e++) oa[0][hb][e] = oa[1][hb][e] = ov[hb][e] = o3[e] = 0.f;
+      asm volatile("" : "+a"(oa[0][hb]), "+a"(oa[1][hb]));
+      asm volatile("" : "+v"(ov[hb]));
+    }
+    asm volatile("" : "+v"(o3));
+#pragma unroll
+    for (int n = 0; n < WIDE_RING; n++)
+      if (n < ntiles) gather(n, n);
+    if (ntiles >= 3) { DSA_WAIT_VMCNT(18); }
+    else if (ntiles == 2) { DSA_WAIT_VMCNT(9); }
+    else { DSA_WAIT_VMCNT(0); }
+    __syncthreads();
+    if (ntiles > 0) {
+      if (ntiles >= 3) { DSA_WAIT_VMCNT(9); }
+      else { DSA_WAIT_VMCNT(0); }
+      __syncthreads();
+      int slot = 0;
+#pragma clang loop unroll(disable)
+      for (int n = 0; n < ntiles; n++) {
+        const int before = slot == 0 ? WIDE_RING - 1 : slot - 1;
+        if (n > 0 && n + 2 < ntiles) gather(n + 2, before);
+        const unsigned char* vb = smem + slot * TILE_BYTES + 2 * w * GRP_BYTES;
+        const bf16x8* const pp = (const bf16x8*)(pbuf + (n & 1) * P_BYTES) + lane;
+        auto read_v = [&](int u) {           // unit u = 4 s + i
+          const unsigned char* b = vb + ((u & 3) >> 1) * GRP_BYTES;
+          return value_operand(read_tr(b + lo.tr_off[u >> 2][0][u & 1]), read_tr(b + lo.tr_off[u >> 2][1][u & 1]));
+        };
+        bf16x8 p[4], v[2];
+#pragma unroll
+        for (int hb = 0; hb < 4; hb++) p[hb] = pp[hb * 128];
+        v[0] = read_v(0);
+        v[1] = read_v(1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int i = u & 3;
+          if (i < 2) {
+#pragma unroll
+            for (int hb = 0; hb < 4; hb++) mfma_a_vv(oa[i][hb], v[u & 1], p[hb]);
+          } else if (i == 2) {
+#pragma unroll
+            for (int hb = 0; hb < 4; hb++) mfma_v_vv(ov[hb], v[u & 1], p[hb]);
+          } else {
+            mfma_v_vv(o3, v[u & 1], p[3]);
+          }
+          if (u + 2 < 8) v[u & 1] = read_v(u + 2);
+          if (u == 2) {
+#pragma unroll
+            for (int hb = 0; hb < 3; hb++) p[hb] = pp[hb * 128 + 64];
+          }
+          if (u == 3) p[3] = pp[3 * 128 + 64];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        slot = slot == WIDE_RING - 1 ? 0 : slot + 1;
+        DSA_WAIT_VMCNT(0);                   // tile n + 2 has landed
+        __syncthreads();
+      }
+    }
+    __syncthreads();                         // the heads' factors
+    auto store = [&](const f32x16& t, int hb, int i) {
+      if (32 * hb >= H) return;
+      const int dt = 4 * w + i;
+      if (SPLIT) store_partial(t, a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt) * 256 + lane);
+      else store_out(t, inv_s[32 * hb + r], (unsigned short*)a.out + ((size_t)qi * H + 32 * hb + r) * DV + 32 * dt + 8 * g);
+    };
+#pragma unroll
+    for (int hb = 0; hb < 4; hb++) {
+      mfma_done_a(oa[0][hb]);
+      store(oa[0][hb], hb, 0);
+      mfma_done_a(oa[1][hb]);
+      store(oa[1][hb], hb, 1);
+      mfma_done_v(ov[hb]);
+      store(ov[hb], hb, 2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mfma_done_v(o3);
+    store(o3, 3, 3);
+  }
+}
+
+template <bool SPLIT, int POUT>
+__global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int u = (int)blockIdx.x;             // longest prefixes first
+  const int qi = a.S - 1 - (SPLIT ? u / a.ksplit : u), sp = SPLIT ? u % a.ksplit : 0;
+  if (threadIdx.x < 256) wide_body<true, SPLIT, POUT>(a, qi, sp, smem);
+  else wide_body<false, SPLIT, POUT>(a, qi, sp, smem);
 }
 
 // Modes 0 and 1, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
@@ -631,8 +903,8 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
 // ---------------------------------------------------------------------------------------------
 struct FwdPlan { int mode, n_hg, ksplit, k_loc; };
 
-int max_slots(int mode, int stages) {        // slots of a range whose id arrays fit LDS beside the tile ring
-  const int ring = (mode == 0 ? stages : 2 * stages) * TILE_BYTES;
+int max_slots(int mode) {                    // slots of a range whose id arrays fit LDS beside the tile ring
+  const int ring = mode == 0 ? WIDE_LDS : 4 * TILE_BYTES;
   return (160 * 1024 - ring - 16) * 16 / 68 / 64 * 64;                  // 4 B per slot + 8 B per tile of 32
 }
 
@@ -646,14 +918,16 @@ FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
 // The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
 // units, each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel that follows.
 // The constants are measured times in us (random rows; a pair of tiles on an idle chip and on a full one: the gathers
-// of 256 workgroups share the fabric): at 2048 slots and 128 heads one query takes 104 us in mode 0 and 17.7 us as
-// 64 workgroups of mode 2 (in 16 ranges; 18.4 in 11), 48 queries 104 and 45 us (mode 1 in two ranges), 200 queries of 64 heads 114 and 67 us
-// (mode 1), 4096 of 32 heads 1840 and 980 us (mode 2); 1500 queries of 128 heads stay in mode 0 (810 against 905 us).
+// of 256 workgroups share the fabric, and a last round that is half empty runs a pair nearly as fast as an idle chip does, hence
+// the square).  At 2048 slots and 128 heads one query takes 86 us in mode 0 and 18 as
+// 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0, 50 - 52 in mode 0 of four ranges or mode 1 of two; 128 queries 100 and 86
+// (mode 1), 160 queries 100 and 148; 300 queries 211 and 227, 600 queries 334 and 392; 48 queries of 96 heads 45 in mode 0 of four
+// ranges and 49 in mode 1 of two; 200 queries of 64 heads 77 (mode 1), 1500 of 32 heads 390 (mode 2).
 // A query with one pair of tiles has nothing to share out: mode 0.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   if (K <= 2 * BI) return one_workgroup_per_query(K);
   constexpr float FIXED = 6.0f, REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
-  constexpr float PAIR_IDLE[3] = {2.95f, 1.6f, 1.3f}, PAIR_FULL[3] = {4.1f, 2.15f, 1.65f};
+  constexpr float PAIR_IDLE[3] = {2.35f, 1.6f, 1.3f}, PAIR_FULL[3] = {3.65f, 2.3f, 1.8f};
   const int heads[3] = {128, 64, 32};
   const int pairs = K / (2 * BI);
   FwdPlan best = one_workgroup_per_query(K);
@@ -662,10 +936,11 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
     const int n_hg = (H + heads[mode] - 1) / heads[mode];
     for (int want = 1; want <= (may_split ? 32 : 1) && want <= pairs; want++) {
       const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
-      if (ksplit != want || 64 * per > max_slots(mode, mode == 0 ? 3 : 2)) continue;
+      if (ksplit != want || 64 * per > max_slots(mode)) continue;
       const long wgs = (long)S * n_hg * ksplit;
-      const float full = wgs < 256 ? (float)wgs / 256.0f : 1.0f;
-      float t = (float)((wgs + 255) / 256) * (FIXED + per * (PAIR_IDLE[mode] + full * (PAIR_FULL[mode] - PAIR_IDLE[mode])));
+      const float rest = (float)(wgs % 256) / 256.0f;
+      float t = (float)(wgs / 256) * (FIXED + per * PAIR_FULL[mode]);
+      if (rest > 0.0f) t += FIXED + per * (PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode]));
       t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
@@ -679,14 +954,20 @@ size_t part_bytes(const FwdPlan& p, int S, int H) {
   return p.ksplit > 1 ? (size_t)S * p.ksplit * H * (DV * 4 + 8) + 256 : 0;
 }
 
-template <int MODE, int STAGES, bool SPLIT>
+template <int MODE, bool SPLIT, int POUT>
+constexpr auto fwd_kernel() {
+  if constexpr (MODE == 0) return mla_fwd_wide_kernel<SPLIT, POUT>;
+  else return mla_fwd_kernel<MODE, SPLIT, POUT>;
+}
+
+template <int MODE, bool SPLIT>
 int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
-  const size_t smem = (size_t)(MODE == 0 ? STAGES : 2 * STAGES) * TILE_BYTES + ids_lds_bytes(a.k_loc);
+  const size_t smem = (size_t)(MODE == 0 ? WIDE_LDS : 4 * TILE_BYTES) + ids_lds_bytes(a.k_loc);
   if (smem > 160 * 1024) return -1;
   const int units = a.S * a.ksplit;
-  const dim3 grid(MODE == 0 && !SPLIT ? a.S : 8 * ((units + 7) / 8) * a.n_hg), block(256);
+  const dim3 grid(MODE == 0 ? units : 8 * ((units + 7) / 8) * a.n_hg), block(MODE == 0 ? 512 : 256);
 #define DSA_FWD_LAUNCH(P) do { \
-    auto kern = mla_fwd_kernel<MODE, STAGES, SPLIT, P>; \
+    auto kern = fwd_kernel<MODE, SPLIT, P>(); \
     if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return -2; \
     kern<<<grid, block, smem, st>>>(a); \
   } while (0)
@@ -699,8 +980,8 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
   if (MODE == 2 && !SPLIT) return 0;
   if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
-  if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), block, tail, st>>>(a);
-  else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), block, tail, st>>>(a);
+  if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), 256, tail, st>>>(a);
+  else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), 256, tail, st>>>(a);
   return 0;
 }
 
@@ -727,10 +1008,9 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, in
             (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4)};
   int rc;
   const bool split = p.ksplit > 1;
-  if (p.mode == 1) rc = split ? launch_fwd<1, 2, true>(a, p_out_f32, st) : launch_fwd<1, 2, false>(a, p_out_f32, st);
-  else if (p.mode == 2) rc = split ? launch_fwd<2, 2, true>(a, p_out_f32, st) : launch_fwd<2, 2, false>(a, p_out_f32, st);
-  else if (p.k_loc > 2048) rc = split ? launch_fwd<0, 3, true>(a, p_out_f32, st) : launch_fwd<0, 3, false>(a, p_out_f32, st);
-  else rc = split ? launch_fwd<0, 4, true>(a, p_out_f32, st) : launch_fwd<0, 4, false>(a, p_out_f32, st);
+  if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, st) : launch_fwd<0, false>(a, p_out_f32, st);
+  else if (p.mode == 1) rc = split ? launch_fwd<1, true>(a, p_out_f32, st) : launch_fwd<1, false>(a, p_out_f32, st);
+  else rc = split ? launch_fwd<2, true>(a, p_out_f32, st) : launch_fwd<2, false>(a, p_out_f32, st);
   DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d does not fit LDS", K);
   if (rc == -2) DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_fwd: cannot reserve LDS");
   DSA_CHECK_LAUNCH("dsa_sparse_mla_fwd");

@@ -155,6 +155,18 @@ def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
                 assert ((p.cpu() - rp)[torch.isfinite(rp)].abs() / rp[torch.isfinite(rp)].abs().clamp_min(1)).max().item() < 1e-3
 
 
+@pytest.mark.parametrize("S,H,K,q_start,skv", [
+    (3, 128, 64, 0, None),            # one tile, then none
+    (40, 128, 64, 30, None),          # one and two tiles
+    (260, 128, 192, 0, None),         # up to six tiles, fewer than the ring in the early rows; a second round of workgroups
+    (170, 96, 320, 400, 500),         # the fourth 32-head block is not there
+    (48, 96, 2048, 3000, None),       # in ranges of slots
+])
+def test_forward_of_many_heads(gpu, S, H, K, q_start, skv):
+    """The two-role kernel at the edges of its tile ring and of its heads, with the slot lists and the bounds of the forms above."""
+    test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv)
+
+
 def test_forward_slot_permutation_invariance(gpu):
     inp = O.make_mla_inputs(100, 128, 128, seed=7)
     out1, lse1, _ = _run_fwd(inp, gpu)
