@@ -76,12 +76,13 @@ __device__ __forceinline__ void acc_row_to_16B(const f32x16& acc, float scale, u
     pc[j][0] = cvt_pk_bf16(acc[4 * j] * scale, acc[4 * j + 1] * scale);
     pc[j][1] = cvt_pk_bf16(acc[4 * j + 2] * scale, acc[4 * j + 3] * scale);
   }
-#pragma unroll
-  for (int jj = 0; jj < 4; jj += 2) {
-    swap_halves(pc[jj][0], pc[jj + 1][0]);
-    swap_halves(pc[jj][1], pc[jj + 1][1]);
-    o[jj >> 1] = make_uint4(pc[jj][0], pc[jj][1], pc[jj + 1][0], pc[jj + 1][1]);
-  }
+  // four v_permlane32_swap (swap_halves) that do not depend on one another: one wait in front, one behind
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\tv_permlane32_swap_b32 %4, %5\n\t"
+               "v_permlane32_swap_b32 %6, %7\n\ts_nop 1"
+               : "+v"(pc[0][0]), "+v"(pc[1][0]), "+v"(pc[0][1]), "+v"(pc[1][1]), "+v"(pc[2][0]), "+v"(pc[3][0]), "+v"(pc[2][1]),
+                 "+v"(pc[3][1]));
+  o[0] = make_uint4(pc[0][0], pc[0][1], pc[1][0], pc[1][1]);
+  o[1] = make_uint4(pc[2][0], pc[2][1], pc[3][0], pc[3][1]);
 }
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding).
 #define DSA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 0xf) | (((n) >> 4) << 14)) | (0x7 << 4) | (0xf << 8))
