@@ -227,26 +227,20 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
 
-  // ---- this wave's Q slice as the B operand of S^T = KV . Q^T, requested before the ids are staged
-  // so that both come back in one round trip to memory ---------------------------------------------
+  // ---- Q of the workgroup's heads, requested before the ids are staged so that both come back in one round trip
+  // to memory: 32-head blocks in the tiles' layout, where tiles 2 and 3 will lie.  (mla_fwd_wide_kernel gains nothing from
+  // this: its queries come in rounds of 256 and their rows at the rate of the memory, 3.33 ms either way.) ----------
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
   const int h = hb * 32 + r;
   const bool head_ok = h < H;
-  bf16x8 qreg[KSTEPS];
-  {
-    const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : 0)) * DQK) + g;
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
-  }
+  for (int b = 0; b < (MODE == 1 ? 2 : 1); b++)
+    gather_rows(a.q + ((size_t)qi * H + min((MODE == 1 ? 2 * hg + b : hg) * 32, H - 32)) * DQK, lds0 + (unsigned)((2 + b) * TILE_BYTES));
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- stage the ids, mark valid slots, list the tiles that have any ---------------------
   const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, qpos, idx_s, tmask, tlist, ntile_s);
   const int nsteps = (ntiles + 1) / 2;
-  // the slice must have landed before the gather pipeline starts: the loop below counts
-  // outstanding vector-memory operations by hand
-  DSA_WAIT_VMCNT(0);
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ks++) asm volatile("" : "+v"(qreg[ks]));
 
   // slots of tiles that are never visited still need their -inf in p_out
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
@@ -267,7 +261,6 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   }
 
   // ---- gather of tile n of the list into ring slot n % 4; lane-dependent LDS offsets ----
-  const unsigned lds0 = (unsigned)(uintptr_t)smem;
   auto issue = [&](int n) {
     gather_tile(a.kv, idx_s, tlist[min(n, ntiles - 1)], lds0 + (unsigned)((n % 4) * TILE_BYTES));
   };
@@ -296,6 +289,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
 
   const float c2 = a.sm_scale * LOG2E;
   float m_ref = -1e30f, l_run = 0.f;
+  bf16x8 qreg[KSTEPS];                               // the wave's Q slice, B operand of S^T = KV . Q^T
   f32x16 oacc[NDT];
 
   // S^T of the tile in stage buffer tb.  Operand reads run four k-steps ahead of the MFMAs; the
@@ -330,6 +324,17 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     for (int e = 0; e < 16; e++) oacc[dt][e] = 0.f;
   }
   for (int n = 0; n < 2 && n < 2 * nsteps; n++) issue(n);
+  if (nsteps > 0) { DSA_WAIT_VMCNT(18); }
+  else { DSA_WAIT_VMCNT(0); }
+  __syncthreads();
+  {
+    const unsigned char* qb = smem + (2 + (MODE == 1 ? sub : 0)) * TILE_BYTES;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ks++) {
+      qreg[ks] = *(const bf16x8*)(qb + (ks >> 2) * GRP_BYTES + qk_off[ks & 3]);
+      asm volatile("" : "+v"(qreg[ks]));
+    }
+  }
   bool overflow = false;
   int stores_after = 0;                      // p_out stores a wave issued after the transfers it waits for
   for (int step = 0; step < nsteps; step++) {

@@ -97,6 +97,18 @@ __device__ __forceinline__ void gather_tile(const void* kv, const int* idx_s, in
   for (int grp = 0; grp < 9; grp++) dma16(lb + grp * GRP_BYTES, goff + grp * 128, kv);
 }
 
+// 32 consecutive rows of an array, in the layout of a tile: thread (row = tid / 8, sub = tid % 8).  Every transfer moves whole
+// 128-byte lines.  Loads in the operands' own layout take 32 bytes of each of 32 rows and keep the address path busy for twice
+// their bytes and more: one query's forward (32 heads a workgroup, all four waves reading the same block) 17.6 -> 14.8 us.
+__device__ __forceinline__ void gather_rows(const void* rows, unsigned lds_tile_base) {
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const unsigned goff = (unsigned)(tid >> 3) * (DQK * 2) + (unsigned)(((tid & 7) ^ swz(tid >> 3)) * 16);
+  const unsigned lb = __builtin_amdgcn_readfirstlane(lds_tile_base + (unsigned)(wave * 1024));
+  const void* base = uniform_ptr((const unsigned char*)rows);
+#pragma unroll
+  for (int grp = 0; grp < 9; grp++) dma16(lb + grp * GRP_BYTES, goff + grp * 128, base);
+}
+
 // Tile-relative LDS byte offsets for this lane.
 //   row_off[j]: 128-bit read of row (lane & 31), chunk c with (c & 7) == 2*j + (lane >> 5); add
 //               (c >> 3) * GRP_BYTES.  This is the MFMA operand "32 rows x 16 contiguous d".
