@@ -526,18 +526,6 @@ __device__ __forceinline__ void dkv_body(
 // Bound by the row writes: a step of 5000 cycles writes 41 KB per compute unit, 4.7 TB/s, and the set-up of a query (208 KB
 // read, 36 000 cycles) does not overlap it.  3072 queries x 128 + 512 slots of compressed keys: 0.68 ms against 0.41 + 0.51; 2077 x 512: 0.35 against 0.23 + 0.26.
 constexpr int FUSED_STAGES = 3;
-// 16x16x32 MFMAs with accumulators in architectural registers and operand A in either file.  The compiler does not see an MFMA
-// in them: the wait states after a move that it may put in front of one (VALU write to MFMA read) are part of the string.
-#define DSA_MFMA16_FN(name, A)                                                                         \
-  __device__ __forceinline__ void name(f32x4& acc, const bf16x8& a, const bf16x8& b, bool first) {     \
-    if (first) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : A(a), "v"(b));      \
-    else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : A(a), "v"(b));            \
-  }
-DSA_MFMA16_FN(mfma16_a, "a")
-DSA_MFMA16_FN(mfma16_v, "v")
-#undef DSA_MFMA16_FN
-__device__ __forceinline__ void mfma16_done(f32x4& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
-__device__ __forceinline__ void mfma16_done(f32x4& x, f32x4& y) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x), "+v"(y)); }
 constexpr int FUSED_XCH = 2 * pds_kind_bytes(2);      // P and dS of a tile
 constexpr int FUSED_ROT = 16384;                      // every wave's operands of the rotary columns
 static_assert(64 * (DQK + DV) * 2 <= FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT, "Q and dO of a query pass through this part of LDS");

@@ -14,6 +14,7 @@
 //
 // How a workgroup shares a query's heads and slots is the MODE:
 //   0  128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
+//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel.
 //   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
 //      of every other tile; the two streams' sums are merged through LDS at the end.
 //   2  32 heads, two tiles at a time: waves (stream, b) compute S^T of the same heads and own half
@@ -800,7 +801,305 @@ __global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
   else wide_body<false, SPLIT, POUT>(a, qi, sp, smem);
 }
 
-// Modes 0 and 1, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
+// ---------------------------------------------------------------------------------------------
+// 64 heads and more queries than compute units: four waves of up to 256 registers, two workgroups on a compute unit.
+//
+// With one workgroup of 512 registers a lane on a compute unit (mode 1) nothing fills what a query spends outside its tiles - Q, ids,
+// the hand-over between the streams, the output: 12 us of the 31 that 640 slots took - nor a wave's softmax and transfers.  Here
+// wave w has the scores of 16 heads (16x16x32 products: 72 registers of Q) and the value columns 128 w .. of all 64 (128
+// accumulation registers), P passes through LDS, and a workgroup takes 79 KB: two tiles, P, and of the slot list only the masks,
+// so that the longest one fits; the ids are read again a tile ahead of the transfers.  While one workgroup waits the other one works.
+// Cycles a tile, two workgroups at work: transfers 740, scores 1440 (36 row reads of LDS for 576 matrix cycles), softmax
+// 360, values 840, waits 330: bound by LDS, 56 reads a wave and tile, and by the gather where the keys lie far apart (65536 keys: no
+// gain over mode 1).  3072 queries x 640 slots 372 -> 303 us (with the logits), 2048 x 512 220 -> 175, 3072 x 2048 1005 -> 940.
+// ---------------------------------------------------------------------------------------------
+constexpr int HALF_P = 4096;                 // P of a tile, [32-head block][16 keys][lane] of 16 bytes
+constexpr int HALF_LDS = 2 * TILE_BYTES + HALF_P;
+constexpr int HALF_AHEAD = 6;                // row reads in flight
+__host__ __device__ inline size_t mask_lds_bytes(int K) { return (size_t)(K / BI) * 8 + 16; }
+static_assert(HALF_LDS + 8192 / BI * 8 + 16 <= 80 * 1024, "two workgroups on a compute unit at the longest list");
+
+// The tiles' slot function with bit 0 of the row alone below: 16 rows x 4 chunks (an operand of 16x16x32) and the transposed
+// reads of lane_offsets are both free of bank conflicts.
+__device__ __forceinline__ int swz16(int r) { return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | (r & 1); }
+
+// stage_ids without the ids: the masks and the list of the tiles that have a valid slot
+__device__ __forceinline__ int stage_masks(const int* __restrict__ ids, int K, unsigned limit, unsigned* tmask, int* tlist, int* ntile_s) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int NT = K / BI;
+  for (int t0 = wave * 64; t0 < K; t0 += 8 * 256) {          // eight loads in flight
+    int v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 64) + lane];
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const unsigned long long b = __ballot((unsigned)v[i] < limit);
+      if (lane == 0 && t0 + i * 256 < K) {
+        tmask[(t0 + i * 256) / BI] = (unsigned)b;
+        tmask[(t0 + i * 256) / BI + 1] = (unsigned)(b >> 32);
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int base = 0;
+    for (int t0 = 0; t0 < NT; t0 += 64) {
+      const int t = t0 + lane;
+      const bool nz = t < NT && tmask[t] != 0u;
+      const unsigned long long b = __ballot(nz);
+      if (nz) tlist[base + __popcll(b & ((1ull << lane) - 1ull))] = t;
+      base += __popcll(b);
+    }
+    if (lane == 0) *ntile_s = base;
+  }
+  __syncthreads();
+  return *ntile_s;
+}
+
+template <int POUT>
+__global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  constexpr int KS = DQK / 32;               // 18 k-steps of 32
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15, kg = lane >> 4;   // scores: head m of the wave's 16, keys 4 kg .. + 3 of each half tile
+  const int r = lane & 31, g = lane >> 5;    // values: head r of a block of 32
+  const int S = a.S, H = a.H, K = a.K, p_skip = a.p_skip;
+
+  // the head groups of a query eight workgroups apart, i.e. on the same XCD and its L2; longest prefixes first
+  const int i8 = (int)blockIdx.x >> 3;
+  const int hg = i8 % a.n_hg;
+  const int u = (i8 / a.n_hg) * 8 + ((int)blockIdx.x & 7);
+  if (u >= S) return;
+  const int qi = S - 1 - u;
+  const int NT = K / BI;
+  const unsigned limit = (unsigned)min(a.Skv, a.q_start + qi + 1);       // valid ids are below
+
+  unsigned char* const pbuf = smem + 2 * TILE_BYTES;
+  unsigned* tmask = (unsigned*)(smem + HALF_LDS);
+  int* tlist = (int*)(tmask + NT);
+
+  const int h = 64 * hg + 16 * w + m;        // of the scores
+  const bool head_ok = 64 * hg + 16 * w < H; // the same for all lanes of a wave
+  bf16x8 qreg[KS];
+  {
+    const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : m)) * DQK) + kg;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qreg[ks] = qp[4 * ks];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int* const row_ids = a.ids + (size_t)qi * K;
+  const int ntiles = stage_masks(row_ids, K, limit, tmask, tlist, tlist + NT);
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qreg[ks]));
+
+  // slots of tiles that are never visited still need their -inf in p_out
+  // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
+  if (POUT != 0 && head_ok && ntiles < NT) {
+    for (int t = 0; t < NT; t++) {
+      if (tmask[t] != 0u || t * BI < p_skip) continue;
+      const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(t * BI - p_skip) + 8 * kg;
+      if (POUT == 2) {
+        const f32x4 ninf = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+        for (int j = 0; j < 2; j++) *(f32x4*)((float*)a.p_out + pbase + 4 * j) = ninf;
+      } else {
+        *(uint4*)((unsigned short*)a.p_out + pbase) = make_uint4(0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u);
+      }
+    }
+  }
+
+  // ---- transfers: thread (key = tid / 8, sub = tid % 8) moves slot `sub` of each of the 9 groups.  The ids come from memory,
+  // a tile ahead of the transfers that need them: beside two tiles LDS has no room for those of a long list ----
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  const int gkey = tid >> 3;
+  const unsigned gsl = (unsigned)(((tid & 7) ^ swz16(gkey)) * 16);
+  auto id_of = [&](int n) { return row_ids[tlist[min(n, ntiles - 1)] * BI + gkey]; };
+  auto offset_of = [&](int id) { return ((unsigned)id < limit ? (unsigned)id : 0u) * (DQK * 2) + gsl; };
+  auto gather = [&](unsigned goff, int slot) {
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(slot * TILE_BYTES + w * 1024));
+#pragma unroll
+    for (int grp = 0; grp < 9; grp++) dma16(lb + grp * GRP_BYTES, goff + grp * 128, a.kv);
+  };
+
+  // operand A of the scores: key 16 hh + m, chunk 4 (ks % 2) + kg of group ks / 2; hh: + 2048 (the slot function repeats after 8 rows)
+  const unsigned row0 = (unsigned)(m * 128 + ((kg ^ swz16(m)) << 4));
+  // transposed reads of a value tile, as in lane_offsets with this kernel's slots: keys 16 s + 8 t + 4 g .. + 3; s: + 2048, t: + 1024
+  unsigned tr0;
+  {
+    const int blk = lane >> 4, ii = lane & 15;
+    const int key = 4 * g + (ii >> 2), cl = 2 * (blk & 1) + ((ii & 3) >> 1);
+    tr0 = (unsigned)(key * 128 + ((cl ^ swz16(key)) << 4) + (ii & 1) * 8);             // odd column tile of a group: ^ 64
+  }
+  const float c2 = a.sm_scale * LOG2E;
+  float m_ref = -1e30f, l_run = 0.f;
+  bool overflow = false;
+  f32x16 o[4][2];                            // value columns 128 w + 32 i of head block hb
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++) {
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[i][hb][e] = 0.f;
+      asm volatile("" : "+a"(o[i][hb]));
+    }
+  const unsigned p_lds = lds0 + 2 * TILE_BYTES;
+  const unsigned p_wr = p_lds + (unsigned)((w >> 1) * 2048 + ((kg & 1) * 32 + 16 * (w & 1) + m) * 16 + (kg >> 1) * 8);
+  const unsigned p_rd = p_lds + (unsigned)(lane * 16);
+
+  int id_next = 0;
+  if (ntiles > 0) {
+    const int id0 = id_of(0);
+    id_next = id_of(1);
+    gather(offset_of(id0), 0);
+  }
+  int stores_after = 0;                      // p_out stores a wave issued after the transfers it waits for
+#pragma clang loop unroll(disable)
+  for (int n = 0; n < ntiles; n++) {
+    asm volatile("" : "+s"(n));              // one copy of the body
+    if (POUT == 1 && stores_after) { DSA_WAIT_VMCNT(1); }
+    else if (POUT == 2 && stores_after) { DSA_WAIT_VMCNT(2); }
+    else { DSA_WAIT_VMCNT(0); }
+    __syncthreads();                         // the tile has landed; the other one and P have been read
+    if (n + 1 < ntiles) {
+      unsigned goff = offset_of(id_next);
+      asm volatile("" : "+v"(goff));         // before the next load is on its way: the wait for this one would be for both
+      id_next = id_of(n + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      gather(goff, (n + 1) & 1);
+    }
+    const unsigned tb = lds0 + (unsigned)((n & 1) * TILE_BYTES);
+    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]);
+    const unsigned mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+
+    // ---- S^T of the wave's 16 heads: half tiles alternate ----
+    f32x4 sa[2];
+    {
+      const unsigned t0 = tb + row0;
+      auto row = [&](int x) {                // x = 2 ks + hh
+        const int ks = x >> 1;
+        return *LDS_PTR(const bf16x8, (uintptr_t)((t0 ^ (64 * (ks & 1))) + (ks >> 1) * GRP_BYTES + 2048 * (x & 1)));
+      };
+      bf16x8 f[HALF_AHEAD];
+#pragma unroll
+      for (int x = 0; x < HALF_AHEAD; x++) f[x] = row(x);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 2 * KS; x++) {
+        mfma16_v(sa[x & 1], f[x % HALF_AHEAD], qreg[x >> 1], x < 2);
+        if (x + HALF_AHEAD < 2 * KS) f[x % HALF_AHEAD] = row(x + HALF_AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      mfma16_done(sa[0], sa[1]);
+    }
+    // accumulator e of half hh is key 16 hh + 4 kg + e of the tile
+    if (mask != 0xffffffffu) {
+      const unsigned mg = mask >> (4 * kg);
+#pragma unroll
+      for (int hh = 0; hh < 2; hh++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (!((mg >> (16 * hh + e)) & 1u)) sa[hh][e] = -INFINITY;
+    }
+    stores_after = 0;
+    if (POUT != 0 && head_ok && tile * BI >= p_skip) {
+      const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(tile * BI - p_skip);
+      if (POUT == 2) {
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) *(f32x4*)((float*)a.p_out + prow + 16 * hh + 4 * kg) = sa[hh];
+      } else {
+        // 8-byte pieces of each half tile; lanes 16 apart trade them, so that a lane stores 8 consecutive keys: those from
+        // 0, 16, 8, 24 on for kg = 0 .. 3
+        unsigned x0 = cvt_pk_bf16(sa[0][0], sa[0][1]), x1 = cvt_pk_bf16(sa[0][2], sa[0][3]);
+        unsigned y0 = cvt_pk_bf16(sa[1][0], sa[1][1]), y1 = cvt_pk_bf16(sa[1][2], sa[1][3]);
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1"
+                     : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1));
+        *(uint4*)((unsigned short*)a.p_out + prow + 16 * (kg & 1) + 8 * (kg >> 1)) = make_uint4(x0, x1, y0, y1);
+      }
+      stores_after = 1;
+    }
+    // ---- softmax numerators (base 2); P to LDS ----
+    if (n == 0) {
+      float mx = sa[0][0];
+#pragma unroll
+      for (int e = 1; e < 8; e++) mx = fmaxf(mx, sa[e >> 2][e & 3]);
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      m_ref = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int hh = 0; hh < 2; hh++) {
+      float p[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        p[e] = __builtin_amdgcn_exp2f(fmaf(sa[hh][e], c2, -m_ref));
+        sum += p[e];
+      }
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      *LDS_PTR(u32x2, (uintptr_t)(p_wr + 1024 * hh)) = u32x2{cvt_pk_bf16(p[0], p[1]), cvt_pk_bf16(p[2], p[3])};
+    }
+    l_run += sum;
+    overflow |= sum > REDO_TERM;             // one of the terms, or a few just below
+    __syncthreads();
+
+    // ---- O^T += V^T . P^T ----
+    {
+      const unsigned vb = tb + tr0 + (unsigned)(2 * w * GRP_BYTES);
+      auto read_v = [&](int x) {             // x = 4 s + i
+        const unsigned b = (vb ^ (64 * (x & 1))) + ((x & 3) >> 1) * GRP_BYTES + 2048 * (x >> 2);
+        return value_operand(__builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, (uintptr_t)b)),
+                             __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, (uintptr_t)(b + 1024))));
+      };
+      bf16x8 p[2][2], v[3];
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int hb = 0; hb < 2; hb++) p[s][hb] = *LDS_PTR(const bf16x8, (uintptr_t)(p_rd + hb * 2048 + s * 1024));
+#pragma unroll
+      for (int x = 0; x < 3; x++) v[x] = read_v(x);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 8; x++) {
+#pragma unroll
+        for (int hb = 0; hb < 2; hb++) mfma_a_vv(o[x & 3][hb], v[x % 3], p[x >> 2][hb]);
+        if (x + 3 < 8) v[x % 3] = read_v(x + 3);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+
+  // ---- epilogue: a mark is of a whole 32-head block, i.e. of two waves ----
+  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
+  l_tot += __shfl_xor(l_tot, 32, 64);
+  float* const inv_s = (float*)pbuf;         // [64] factors, then [4] marks
+  int* const again_s = (int*)(inv_s + 64);
+  __syncthreads();                           // P has been read
+  const bool mine = __ballot(overflow) != 0ull;
+  if (lane == 0) again_s[w] = mine;
+  __syncthreads();
+  const bool again = (again_s[w] | again_s[w ^ 1]) != 0;
+  const Final fin = finish_head(m_ref, l_tot, a.sink && head_ok ? a.sink + h : nullptr);
+  if (kg == 0) {
+    if (head_ok) a.lse[(size_t)qi * H + h] = again ? __builtin_bit_cast(float, REDO_MARK) : fin.lse;
+    inv_s[16 * w + m] = fin.inv;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int hb = 0; hb < 2; hb++) {
+    if (64 * hg + 32 * hb >= H) break;
+    const float inv = inv_s[32 * hb + r];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int dt = 4 * w + i;
+      mfma_done_a(o[i][hb]);
+      store_out(o[i][hb], inv, (unsigned short*)a.out + ((size_t)qi * H + 64 * hg + 32 * hb + r) * DV + 32 * dt + 8 * g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// Modes 0, 1 and 3, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
 // redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
 __global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
   const int wave = threadIdx.x >> 6;
@@ -909,6 +1208,7 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
 struct FwdPlan { int mode, n_hg, ksplit, k_loc; };
 
 int max_slots(int mode) {                    // slots of a range whose id arrays fit LDS beside the tile ring
+  if (mode == 3) return 8192;                // (it reads them from memory)
   const int ring = mode == 0 ? WIDE_LDS : 4 * TILE_BYTES;
   return (160 * 1024 - ring - 16) * 16 / 68 / 64 * 64;                  // 4 B per slot + 8 B per tile of 32
 }
@@ -928,24 +1228,30 @@ FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
 // 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0, 50 - 52 in mode 0 of four ranges or mode 1 of two; 128 queries 100 and 86
 // (mode 1), 160 queries 100 and 148; 300 queries 211 and 227, 600 queries 334 and 392; 48 queries of 96 heads 45 in mode 0 of four
 // ranges and 49 in mode 1 of two; 200 queries of 64 heads 77 (mode 1), 1500 of 32 heads 390 (mode 2).
+// Mode 3 gains by its second workgroup on a compute unit: 256 queries of 64 heads 94 us against 83 in mode 1, 300 queries 123 and
+// 140, 512 147 and 158, 3000 817 and 900.  A round of 512 that is at most half full is priced as what it takes where the keys
+// lie far apart (700 queries, 65536 keys: 281 and 251; 8192 keys: 215 and 224).
 // A query with one pair of tiles has nothing to share out: mode 0.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   if (K <= 2 * BI) return one_workgroup_per_query(K);
-  constexpr float FIXED = 6.0f, REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
-  constexpr float PAIR_IDLE[3] = {2.35f, 1.6f, 1.3f}, PAIR_FULL[3] = {3.65f, 2.3f, 1.8f};
-  const int heads[3] = {128, 64, 32};
+  constexpr float FIXED[4] = {6.0f, 6.0f, 6.0f, 12.0f};
+  constexpr float REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
+  constexpr float PAIR_IDLE[3] = {2.35f, 1.6f, 1.3f}, PAIR_FULL[4] = {3.65f, 2.3f, 1.8f, 4.0f};
+  constexpr int HEADS[4] = {128, 64, 32, 64}, SLOTS[4] = {256, 256, 256, 512};
   const int pairs = K / (2 * BI);
   FwdPlan best = one_workgroup_per_query(K);
   float best_t = 1e30f;
-  for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 3; mode++) {
-    const int n_hg = (H + heads[mode] - 1) / heads[mode];
-    for (int want = 1; want <= (may_split ? 32 : 1) && want <= pairs; want++) {
+  for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < (H > 32 ? 4 : 3); mode++) {
+    const int n_hg = (H + HEADS[mode] - 1) / HEADS[mode];
+    for (int want = 1; want <= (may_split && mode != 3 ? 32 : 1) && want <= pairs; want++) {
       const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
       if (ksplit != want || 64 * per > max_slots(mode)) continue;
       const long wgs = (long)S * n_hg * ksplit;
-      const float rest = (float)(wgs % 256) / 256.0f;
-      float t = (float)(wgs / 256) * (FIXED + per * PAIR_FULL[mode]);
-      if (rest > 0.0f) t += FIXED + per * (PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode]));
+      const float rest = (float)(wgs % SLOTS[mode]) / (float)SLOTS[mode];
+      const float pair = mode == 3 ? (rest > 0.5f ? 3.3f + 1.4f * (rest - 0.5f) : 2.7f)
+                                   : PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode]);
+      float t = (float)(wgs / SLOTS[mode]) * (FIXED[mode] + per * PAIR_FULL[mode]);
+      if (rest > 0.0f) t += FIXED[mode] + per * pair;
       t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
@@ -962,12 +1268,15 @@ size_t part_bytes(const FwdPlan& p, int S, int H) {
 template <int MODE, bool SPLIT, int POUT>
 constexpr auto fwd_kernel() {
   if constexpr (MODE == 0) return mla_fwd_wide_kernel<SPLIT, POUT>;
+  else if constexpr (MODE == 3) return mla_fwd_half_kernel<POUT>;
   else return mla_fwd_kernel<MODE, SPLIT, POUT>;
 }
 
 template <int MODE, bool SPLIT>
 int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
-  const size_t smem = (size_t)(MODE == 0 ? WIDE_LDS : 4 * TILE_BYTES) + ids_lds_bytes(a.k_loc);
+  const size_t smem = MODE == 0   ? WIDE_LDS + ids_lds_bytes(a.k_loc)
+                      : MODE == 3 ? HALF_LDS + mask_lds_bytes(a.k_loc)
+                                  : 4 * TILE_BYTES + ids_lds_bytes(a.k_loc);
   if (smem > 160 * 1024) return -1;
   const int units = a.S * a.ksplit;
   const dim3 grid(MODE == 0 ? units : 8 * ((units + 7) / 8) * a.n_hg), block(MODE == 0 ? 512 : 256);
@@ -1014,6 +1323,7 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, in
   int rc;
   const bool split = p.ksplit > 1;
   if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, st) : launch_fwd<0, false>(a, p_out_f32, st);
+  else if (p.mode == 3) rc = launch_fwd<3, false>(a, p_out_f32, st);
   else if (p.mode == 1) rc = split ? launch_fwd<1, true>(a, p_out_f32, st) : launch_fwd<1, false>(a, p_out_f32, st);
   else rc = split ? launch_fwd<2, true>(a, p_out_f32, st) : launch_fwd<2, false>(a, p_out_f32, st);
   DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d does not fit LDS", K);

@@ -52,7 +52,8 @@ __device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, in
   for (int t0 = tid; t0 < K; t0 += 8 * 256) {     // eight loads in flight per thread
     int v[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = t0 + i * 256 < K ? ids[(size_t)qi * K + t0 + i * 256] : -1;
+    for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(t0 + i * 256, K - 1)];      // (under its condition each load is waited for by itself)
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const bool ok = (v[i] >= 0) && (v[i] < Skv) && (v[i] <= qpos);
@@ -159,5 +160,17 @@ DSA_MFMA_FN(mfma_a_vv, "a", "v", "v")
 __device__ __forceinline__ void mfma_done_v(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
 __device__ __forceinline__ void mfma_done_a(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc)); }
 
+// 16x16x32 MFMAs with accumulators in architectural registers and operand A in either file.  The compiler does not see an MFMA
+// in them: the wait states after a move that it may put in front of one (VALU write to MFMA read) are part of the string.
+#define DSA_MFMA16_FN(name, A)                                                                         \
+  __device__ __forceinline__ void name(f32x4& acc, const bf16x8& a, const bf16x8& b, bool first) {     \
+    if (first) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : A(a), "v"(b));      \
+    else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : A(a), "v"(b));            \
+  }
+DSA_MFMA16_FN(mfma16_a, "a")
+DSA_MFMA16_FN(mfma16_v, "v")
+#undef DSA_MFMA16_FN
+__device__ __forceinline__ void mfma16_done(f32x4& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
+__device__ __forceinline__ void mfma16_done(f32x4& x, f32x4& y) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x), "+v"(y)); }
 
 }  // namespace mla

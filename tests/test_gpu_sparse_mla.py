@@ -167,6 +167,23 @@ def test_forward_of_many_heads(gpu, S, H, K, q_start, skv):
     test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv)
 
 
+@pytest.mark.parametrize("S,K,q_start,skv", [
+    (300, 64 * 3, 0, None),           # one tile in the early rows: the other half of the ring stays empty
+    (257, 128, 700, 300),             # the last workgroup that has a compute unit to itself, ids beyond the keys
+    (530, 320, 900, None),
+])
+def test_forward_of_64_heads_two_workgroups_to_a_unit(gpu, S, K, q_start, skv):
+    """More queries than compute units: the forms and bounds of the tests above, and bf16 logits that are the fp32 ones rounded."""
+    from loongforge_amd import ops
+
+    test_forward_shares_a_query_among_workgroups(gpu, S, 64, K, q_start, skv)
+    inp = O.make_mla_inputs(S, 64, K, seed=5, skv=skv, q_start=q_start)
+    for skip in (0, 64):
+        p16, p32 = (ops.sparse_mla_fwd(inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), q_start, inp.sm_scale, 512, True, dt, p_out_skip=skip)[2]
+                    for dt in (torch.bfloat16, torch.float32))
+        assert p32.shape[2] == K - skip and torch.equal(p16, p32.to(torch.bfloat16))
+
+
 def test_forward_slot_permutation_invariance(gpu):
     inp = O.make_mla_inputs(100, 128, 128, seed=7)
     out1, lse1, _ = _run_fwd(inp, gpu)
