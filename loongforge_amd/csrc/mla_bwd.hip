@@ -557,6 +557,10 @@ __device__ __forceinline__ void pds_rows_body(
   int* dst_s = (int*)(stat_s + 128);
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
 
+  int slot_id[4], slot_row[4];
+  request_ids(ids, ql, K, slot_id);
+  request_ids(dst, ql, K, slot_row);
+  __builtin_amdgcn_sched_barrier(0);
   // Q and dO travel to LDS as they are, in groups of 128 bytes of all 64 rows (Q: 9, dO: 8), chunk c of row r in slot c ^ (r & 7):
   // both orientations are read from there.  Wave w moves rows 8 w .. 8 w + 7.
   {
@@ -579,12 +583,10 @@ __device__ __forceinline__ void pds_rows_body(
   }
   const float lse_h = lse[hrow];
   __builtin_amdgcn_sched_barrier(0);
-  for (int t = tid; t < K; t += PDS_THREADS) {        // invalid slots land in a scratch row: the store count stays fixed
-    const int d = dst[(size_t)ql * K + t];
-    dst_s[t] = d >= 0 ? d : dummy_row;
-  }
-  // (the helper is written for four waves; the other four repeat part of its work with equal results)
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  const int ntiles = stage_requested_ids(slot_id, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+#pragma unroll
+  for (int i = 0; i < 4; i++)                  // invalid slots land in a scratch row: the store count stays fixed
+    if (tid + 512 * i < K) dst_s[tid + 512 * i] = slot_row[i] >= 0 ? slot_row[i] : dummy_row;
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();

@@ -830,7 +830,7 @@ __device__ __forceinline__ int stage_masks(const int* __restrict__ ids, int K, u
   for (int t0 = wave * 64; t0 < K; t0 += 8 * 256) {          // eight loads in flight
     int v[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 64) + lane];
+    for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 64) + lane];    // (under its condition each would be waited for by itself)
     asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 #pragma unroll
     for (int i = 0; i < 8; i++) {

@@ -52,8 +52,7 @@ __device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, in
   for (int t0 = tid; t0 < K; t0 += 8 * 256) {     // eight loads in flight per thread
     int v[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(t0 + i * 256, K - 1)];      // (under its condition each load is waited for by itself)
-    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+    for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(t0 + i * 256, K - 1)];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const bool ok = (v[i] >= 0) && (v[i] < Skv) && (v[i] <= qpos);
@@ -78,6 +77,38 @@ __device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, in
       base += __popcll(b);
     }
     if (lane == 0) *ntile_s = base;
+  }
+  __syncthreads();
+  return *ntile_s;
+}
+
+// stage_ids for 512 threads and at most 2048 slots, in two steps: the ids are requested before the operands of a query, so that
+// the lists are made while those are on their way.
+__device__ __forceinline__ void request_ids(const int* __restrict__ ids, int qi, int K, int (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = ids[(size_t)qi * K + min((int)threadIdx.x + 512 * i, K - 1)];
+}
+__device__ __forceinline__ int stage_requested_ids(int (&v)[4], int K, int Skv, int qpos, int* idx_s, unsigned* tmask, int* tlist,
+                                                   int* ntile_s) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int NT = K / BI;
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int t = tid + 512 * i;             // 64 consecutive slots per wave: the masks of two tiles
+    const bool ok = (v[i] >= 0) && (v[i] < Skv) && (v[i] <= qpos);
+    const unsigned long long b = __ballot(ok);
+    if (t < K) {
+      idx_s[t] = ok ? v[i] : -1;
+      if (lane == 0) { tmask[t / BI] = (unsigned)b; tmask[t / BI + 1] = (unsigned)(b >> 32); }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {                           // at most 64 tiles
+    const bool nz = lane < NT && tmask[lane] != 0u;
+    const unsigned long long b = __ballot(nz);
+    if (nz) tlist[__popcll(b & ((1ull << lane) - 1ull))] = lane;
+    if (lane == 0) *ntile_s = __popcll(b);
   }
   __syncthreads();
   return *ntile_s;
