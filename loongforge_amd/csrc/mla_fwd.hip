@@ -14,7 +14,8 @@
 //
 // How a workgroup shares a query's heads and slots is the MODE:
 //   0  128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
-//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel.
+//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel<2>.
+//   4  32 heads, likewise: mla_fwd_half_kernel<1>.
 //   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
 //      of every other tile; the two streams' sums are merged through LDS at the end.
 //   2  32 heads, two tiles at a time: waves (stream, b) compute S^T of the same heads and own half
@@ -802,7 +803,7 @@ __global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 64 heads and more queries than compute units: four waves of up to 256 registers, two workgroups on a compute unit.
+// 64 or 32 heads and more queries than compute units: four waves of up to 256 registers, two workgroups on a compute unit.
 //
 // With one workgroup of 512 registers a lane on a compute unit (mode 1) nothing fills what a query spends outside its tiles - Q, ids,
 // the hand-over between the streams, the output: 12 us of the 31 that 640 slots took - nor a wave's softmax and transfers.  Here
@@ -812,6 +813,8 @@ __global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
 // Cycles a tile, two workgroups at work: transfers 740, scores 1440 (36 row reads of LDS for 576 matrix cycles), softmax
 // 360, values 840, waits 330: bound by LDS, 56 reads a wave and tile, and by the gather where the keys lie far apart (65536 keys: no
 // gain over mode 1).  3072 queries x 640 slots 372 -> 303 us (with the logits), 2048 x 512 220 -> 175, 3072 x 2048 1005 -> 940.
+// 32 heads: a wave has the scores of 16 heads and one half of a tile's keys; 3000 queries x 640 slots 288 -> 216 us, x 2048 747 -> 575,
+// 1024 x 256 62 -> 45 (against mode 2).
 // ---------------------------------------------------------------------------------------------
 constexpr int HALF_P = 4096;                 // P of a tile, [32-head block][16 keys][lane] of 16 bytes
 constexpr int HALF_LDS = 2 * TILE_BYTES + HALF_P;
@@ -857,13 +860,15 @@ __device__ __forceinline__ int stage_masks(const int* __restrict__ ids, int K, u
   return *ntile_s;
 }
 
-template <int POUT>
+template <int HB, int POUT>                // HB 32-head blocks of a workgroup: 2, or 1
 __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int KS = DQK / 32;               // 18 k-steps of 32
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4;   // scores: head m of the wave's 16, keys 4 kg .. + 3 of each half tile
+  const int hw = HB == 2 ? w : w & 1;        // its 16 heads; one block: it has half tile w / 2 alone, the other one is in wave w ^ 2
+  const int h0 = HB == 2 ? 0 : w >> 1;       // its first half tile
   const int r = lane & 31, g = lane >> 5;    // values: head r of a block of 32
   const int S = a.S, H = a.H, K = a.K, p_skip = a.p_skip;
 
@@ -880,8 +885,8 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   unsigned* tmask = (unsigned*)(smem + HALF_LDS);
   int* tlist = (int*)(tmask + NT);
 
-  const int h = 64 * hg + 16 * w + m;        // of the scores
-  const bool head_ok = 64 * hg + 16 * w < H; // the same for all lanes of a wave
+  const int h = 32 * HB * hg + 16 * hw + m;  // of the scores
+  const bool head_ok = 32 * HB * hg + 16 * hw < H;           // the same for all lanes of a wave
   bf16x8 qreg[KS];
   {
     const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : m)) * DQK) + kg;
@@ -896,7 +901,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
 
   // slots of tiles that are never visited still need their -inf in p_out
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
-  if (POUT != 0 && head_ok && ntiles < NT) {
+  if (POUT != 0 && head_ok && h0 == 0 && ntiles < NT) {
     for (int t = 0; t < NT; t++) {
       if (tmask[t] != 0u || t * BI < p_skip) continue;
       const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(t * BI - p_skip) + 8 * kg;
@@ -924,7 +929,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   };
 
   // operand A of the scores: key 16 hh + m, chunk 4 (ks % 2) + kg of group ks / 2; hh: + 2048 (the slot function repeats after 8 rows)
-  const unsigned row0 = (unsigned)(m * 128 + ((kg ^ swz16(m)) << 4));
+  const unsigned row0 = (unsigned)(2048 * h0 + m * 128 + ((kg ^ swz16(m)) << 4));
   // transposed reads of a value tile, as in lane_offsets with this kernel's slots: keys 16 s + 8 t + 4 g .. + 3; s: + 2048, t: + 1024
   unsigned tr0;
   {
@@ -935,17 +940,17 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   const float c2 = a.sm_scale * LOG2E;
   float m_ref = -1e30f, l_run = 0.f;
   bool overflow = false;
-  f32x16 o[4][2];                            // value columns 128 w + 32 i of head block hb
+  f32x16 o[4][HB];                           // value columns 128 w + 32 i of head block hb
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int hb = 0; hb < 2; hb++) {
+    for (int hb = 0; hb < HB; hb++) {
 #pragma unroll
       for (int e = 0; e < 16; e++) o[i][hb][e] = 0.f;
       asm volatile("" : "+a"(o[i][hb]));
     }
   const unsigned p_lds = lds0 + 2 * TILE_BYTES;
-  const unsigned p_wr = p_lds + (unsigned)((w >> 1) * 2048 + ((kg & 1) * 32 + 16 * (w & 1) + m) * 16 + (kg >> 1) * 8);
+  const unsigned p_wr = p_lds + (unsigned)((HB == 2 ? (w >> 1) * 2048 : h0 * 1024) + ((kg & 1) * 32 + 16 * (w & 1) + m) * 16 + (kg >> 1) * 8);
   const unsigned p_rd = p_lds + (unsigned)(lane * 16);
 
   int id_next = 0;
@@ -959,7 +964,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   for (int n = 0; n < ntiles; n++) {
     asm volatile("" : "+s"(n));              // one copy of the body
     if (POUT == 1 && stores_after) { DSA_WAIT_VMCNT(1); }
-    else if (POUT == 2 && stores_after) { DSA_WAIT_VMCNT(2); }
+    else if (POUT == 2 && stores_after) { DSA_WAIT_VMCNT(HB); }
     else { DSA_WAIT_VMCNT(0); }
     __syncthreads();                         // the tile has landed; the other one and P have been read
     if (n + 1 < ntiles) {
@@ -973,31 +978,36 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
     const int tile = __builtin_amdgcn_readfirstlane(tlist[n]);
     const unsigned mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
 
-    // ---- S^T of the wave's 16 heads: half tiles alternate ----
+    // ---- S^T of the wave's 16 heads; two chains: the half tiles, or the even and the odd k-steps of one ----
     f32x4 sa[2];
     {
+      constexpr int NX = HB * KS;
       const unsigned t0 = tb + row0;
-      auto row = [&](int x) {                // x = 2 ks + hh
-        const int ks = x >> 1;
-        return *LDS_PTR(const bf16x8, (uintptr_t)((t0 ^ (64 * (ks & 1))) + (ks >> 1) * GRP_BYTES + 2048 * (x & 1)));
+      auto row = [&](int x) {
+        const int ks = HB == 2 ? x >> 1 : x, hh = HB == 2 ? x & 1 : 0;
+        return *LDS_PTR(const bf16x8, (uintptr_t)((t0 ^ (64 * (ks & 1))) + (ks >> 1) * GRP_BYTES + 2048 * hh));
       };
       bf16x8 f[HALF_AHEAD];
 #pragma unroll
       for (int x = 0; x < HALF_AHEAD; x++) f[x] = row(x);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int x = 0; x < 2 * KS; x++) {
-        mfma16_v(sa[x & 1], f[x % HALF_AHEAD], qreg[x >> 1], x < 2);
-        if (x + HALF_AHEAD < 2 * KS) f[x % HALF_AHEAD] = row(x + HALF_AHEAD);
+      for (int x = 0; x < NX; x++) {
+        mfma16_v(sa[x & 1], f[x % HALF_AHEAD], qreg[HB == 2 ? x >> 1 : x], x < 2);
+        if (x + HALF_AHEAD < NX) f[x % HALF_AHEAD] = row(x + HALF_AHEAD);
         __builtin_amdgcn_sched_barrier(0);
       }
       mfma16_done(sa[0], sa[1]);
+      if (HB == 1) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) sa[0][e] += sa[1][e];
+      }
     }
     // accumulator e of half hh is key 16 hh + 4 kg + e of the tile
     if (mask != 0xffffffffu) {
-      const unsigned mg = mask >> (4 * kg);
+      const unsigned mg = mask >> (16 * h0 + 4 * kg);
 #pragma unroll
-      for (int hh = 0; hh < 2; hh++)
+      for (int hh = 0; hh < HB; hh++)
 #pragma unroll
         for (int e = 0; e < 4; e++)
           if (!((mg >> (16 * hh + e)) & 1u)) sa[hh][e] = -INFINITY;
@@ -1007,7 +1017,10 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
       const size_t prow = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(tile * BI - p_skip);
       if (POUT == 2) {
 #pragma unroll
-        for (int hh = 0; hh < 2; hh++) *(f32x4*)((float*)a.p_out + prow + 16 * hh + 4 * kg) = sa[hh];
+        for (int hh = 0; hh < HB; hh++) *(f32x4*)((float*)a.p_out + prow + 16 * (h0 + hh) + 4 * kg) = sa[hh];
+      } else if (HB == 1) {
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        *(u32x2*)((unsigned short*)a.p_out + prow + 16 * h0 + 4 * kg) = u32x2{cvt_pk_bf16(sa[0][0], sa[0][1]), cvt_pk_bf16(sa[0][2], sa[0][3])};
       } else {
         // 8-byte pieces of each half tile; lanes 16 apart trade them, so that a lane stores 8 consecutive keys: those from
         // 0, 16, 8, 24 on for kg = 0 .. 3
@@ -1023,13 +1036,20 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
     if (n == 0) {
       float mx = sa[0][0];
 #pragma unroll
-      for (int e = 1; e < 8; e++) mx = fmaxf(mx, sa[e >> 2][e & 3]);
+      for (int e = 1; e < 4 * HB; e++) mx = fmaxf(mx, sa[e >> 2][e & 3]);
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      m_ref = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if (HB == 1) {                         // and of the other half tile
+        float* const half_s = (float*)(pbuf + 2048);         // [4][16], behind the one block's P
+        if (kg == 0) half_s[16 * w + m] = mx;
+        __syncthreads();
+        mx = fmaxf(mx, half_s[16 * (w ^ 2) + m]);
+      }
+      m_ref = mx * c2;
     }
     float sum = 0.f;
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < HB; hh++) {
       float p[4];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -1051,55 +1071,58 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
         return value_operand(__builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, (uintptr_t)b)),
                              __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, (uintptr_t)(b + 1024))));
       };
-      bf16x8 p[2][2], v[3];
+      bf16x8 p[2][HB], v[3];
 #pragma unroll
       for (int s = 0; s < 2; s++)
 #pragma unroll
-        for (int hb = 0; hb < 2; hb++) p[s][hb] = *LDS_PTR(const bf16x8, (uintptr_t)(p_rd + hb * 2048 + s * 1024));
+        for (int hb = 0; hb < HB; hb++) p[s][hb] = *LDS_PTR(const bf16x8, (uintptr_t)(p_rd + hb * 2048 + s * 1024));
 #pragma unroll
       for (int x = 0; x < 3; x++) v[x] = read_v(x);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int x = 0; x < 8; x++) {
 #pragma unroll
-        for (int hb = 0; hb < 2; hb++) mfma_a_vv(o[x & 3][hb], v[x % 3], p[x >> 2][hb]);
+        for (int hb = 0; hb < HB; hb++) mfma_a_vv(o[x & 3][hb], v[x % 3], p[x >> 2][hb]);
         if (x + 3 < 8) v[x % 3] = read_v(x + 3);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
 
-  // ---- epilogue: a mark is of a whole 32-head block, i.e. of two waves ----
+  // ---- epilogue: a mark is of a whole 32-head block, i.e. of two waves, or of all four ----
   float l_tot = l_run + __shfl_xor(l_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
   float* const inv_s = (float*)pbuf;         // [64] factors, then [4] marks
   int* const again_s = (int*)(inv_s + 64);
+  float* const l_s = inv_s + 128;            // [4][16]
   __syncthreads();                           // P has been read
   const bool mine = __ballot(overflow) != 0ull;
   if (lane == 0) again_s[w] = mine;
+  if (HB == 1 && kg == 0) l_s[16 * w + m] = l_tot;
   __syncthreads();
-  const bool again = (again_s[w] | again_s[w ^ 1]) != 0;
+  const bool again = HB == 2 ? (again_s[w] | again_s[w ^ 1]) != 0 : (again_s[0] | again_s[1] | again_s[2] | again_s[3]) != 0;
+  if (HB == 1) l_tot = l_s[16 * hw + m] + l_s[16 * hw + 32 + m];
   const Final fin = finish_head(m_ref, l_tot, a.sink && head_ok ? a.sink + h : nullptr);
-  if (kg == 0) {
+  if (kg == 0 && h0 == 0) {
     if (head_ok) a.lse[(size_t)qi * H + h] = again ? __builtin_bit_cast(float, REDO_MARK) : fin.lse;
-    inv_s[16 * w + m] = fin.inv;
+    inv_s[16 * hw + m] = fin.inv;
   }
   __syncthreads();
 #pragma unroll
-  for (int hb = 0; hb < 2; hb++) {
-    if (64 * hg + 32 * hb >= H) break;
+  for (int hb = 0; hb < HB; hb++) {
+    if (32 * (HB * hg + hb) >= H) break;
     const float inv = inv_s[32 * hb + r];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int dt = 4 * w + i;
       mfma_done_a(o[i][hb]);
-      store_out(o[i][hb], inv, (unsigned short*)a.out + ((size_t)qi * H + 64 * hg + 32 * hb + r) * DV + 32 * dt + 8 * g);
+      store_out(o[i][hb], inv, (unsigned short*)a.out + ((size_t)qi * H + 32 * (HB * hg + hb) + r) * DV + 32 * dt + 8 * g);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
-// Modes 0, 1 and 3, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
+// All modes but 2, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
 // redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
 __global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
   const int wave = threadIdx.x >> 6;
@@ -1208,7 +1231,7 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
 struct FwdPlan { int mode, n_hg, ksplit, k_loc; };
 
 int max_slots(int mode) {                    // slots of a range whose id arrays fit LDS beside the tile ring
-  if (mode == 3) return 8192;                // (it reads them from memory)
+  if (mode >= 3) return 8192;                // (they read them from memory)
   const int ring = mode == 0 ? WIDE_LDS : 4 * TILE_BYTES;
   return (160 * 1024 - ring - 16) * 16 / 68 / 64 * 64;                  // 4 B per slot + 8 B per tile of 32
 }
@@ -1230,26 +1253,29 @@ FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
 // ranges and 49 in mode 1 of two; 200 queries of 64 heads 77 (mode 1), 1500 of 32 heads 390 (mode 2).
 // Mode 3 gains by its second workgroup on a compute unit: 256 queries of 64 heads 94 us against 83 in mode 1, 300 queries 123 and
 // 140, 512 147 and 158, 3000 817 and 900.  A round of 512 that is at most half full is priced as what it takes where the keys
-// lie far apart (700 queries, 65536 keys: 281 and 251; 8192 keys: 215 and 224).
+// lie far apart (700 queries, 65536 keys: 281 and 251; 8192 keys: 215 and 224).  Mode 4 likewise: 257 queries of 32 heads 78 us
+// against 112 in mode 2, 600 queries 167 and 177 (65536 keys: 233 and 222), 800 queries 175 and 236.
 // A query with one pair of tiles has nothing to share out: mode 0.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   if (K <= 2 * BI) return one_workgroup_per_query(K);
-  constexpr float FIXED[4] = {6.0f, 6.0f, 6.0f, 12.0f};
   constexpr float REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
-  constexpr float PAIR_IDLE[3] = {2.35f, 1.6f, 1.3f}, PAIR_FULL[4] = {3.65f, 2.3f, 1.8f, 4.0f};
-  constexpr int HEADS[4] = {128, 64, 32, 64}, SLOTS[4] = {256, 256, 256, 512};
+  constexpr float FIXED[5] = {6.0f, 6.0f, 6.0f, 12.0f, 8.5f}, PAIR_FULL[5] = {3.65f, 2.3f, 1.8f, 4.0f, 2.8f};
+  constexpr float PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.1f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
+  constexpr int HEADS[5] = {128, 64, 32, 64, 32}, SLOTS[5] = {256, 256, 256, 512, 512};
   const int pairs = K / (2 * BI);
   FwdPlan best = one_workgroup_per_query(K);
   float best_t = 1e30f;
-  for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < (H > 32 ? 4 : 3); mode++) {
+  for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 5; mode++) {
+    if (mode == (H > 32 ? 4 : 3)) continue;
     const int n_hg = (H + HEADS[mode] - 1) / HEADS[mode];
-    for (int want = 1; want <= (may_split && mode != 3 ? 32 : 1) && want <= pairs; want++) {
+    for (int want = 1; want <= (may_split && mode < 3 ? 32 : 1) && want <= pairs; want++) {
       const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
       if (ksplit != want || 64 * per > max_slots(mode)) continue;
       const long wgs = (long)S * n_hg * ksplit;
       const float rest = (float)(wgs % SLOTS[mode]) / (float)SLOTS[mode];
-      const float pair = mode == 3 ? (rest > 0.5f ? 3.3f + 1.4f * (rest - 0.5f) : 2.7f)
-                                   : PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode]);
+      const float pair = mode < 3      ? PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode])
+                         : rest > 0.5f ? PAIR_SHARED[mode] + 2.0f * (rest - 0.5f) * (PAIR_FULL[mode] - PAIR_SHARED[mode])
+                                       : PAIR_IDLE[mode];
       float t = (float)(wgs / SLOTS[mode]) * (FIXED[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += FIXED[mode] + per * pair;
       t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
@@ -1268,14 +1294,14 @@ size_t part_bytes(const FwdPlan& p, int S, int H) {
 template <int MODE, bool SPLIT, int POUT>
 constexpr auto fwd_kernel() {
   if constexpr (MODE == 0) return mla_fwd_wide_kernel<SPLIT, POUT>;
-  else if constexpr (MODE == 3) return mla_fwd_half_kernel<POUT>;
+  else if constexpr (MODE >= 3) return mla_fwd_half_kernel<MODE == 3 ? 2 : 1, POUT>;
   else return mla_fwd_kernel<MODE, SPLIT, POUT>;
 }
 
 template <int MODE, bool SPLIT>
 int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   const size_t smem = MODE == 0   ? WIDE_LDS + ids_lds_bytes(a.k_loc)
-                      : MODE == 3 ? HALF_LDS + mask_lds_bytes(a.k_loc)
+                      : MODE >= 3 ? HALF_LDS + mask_lds_bytes(a.k_loc)
                                   : 4 * TILE_BYTES + ids_lds_bytes(a.k_loc);
   if (smem > 160 * 1024) return -1;
   const int units = a.S * a.ksplit;
@@ -1324,6 +1350,7 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, in
   const bool split = p.ksplit > 1;
   if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, st) : launch_fwd<0, false>(a, p_out_f32, st);
   else if (p.mode == 3) rc = launch_fwd<3, false>(a, p_out_f32, st);
+  else if (p.mode == 4) rc = launch_fwd<4, false>(a, p_out_f32, st);
   else if (p.mode == 1) rc = split ? launch_fwd<1, true>(a, p_out_f32, st) : launch_fwd<1, false>(a, p_out_f32, st);
   else rc = split ? launch_fwd<2, true>(a, p_out_f32, st) : launch_fwd<2, false>(a, p_out_f32, st);
   DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d does not fit LDS", K);

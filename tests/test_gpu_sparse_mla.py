@@ -167,17 +167,24 @@ def test_forward_of_many_heads(gpu, S, H, K, q_start, skv):
     test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv)
 
 
+@pytest.mark.parametrize("H", [64, 32])
 @pytest.mark.parametrize("S,K,q_start,skv", [
     (300, 64 * 3, 0, None),           # one tile in the early rows: the other half of the ring stays empty
-    (257, 128, 700, 300),             # the last workgroup that has a compute unit to itself, ids beyond the keys
+    (257, 128, 700, None),            # just more than there are compute units
     (530, 320, 900, None),
 ])
-def test_forward_of_64_heads_two_workgroups_to_a_unit(gpu, S, K, q_start, skv):
+def test_forward_two_workgroups_to_a_unit(gpu, S, K, q_start, skv, H):
     """More queries than compute units: the forms and bounds of the tests above, and bf16 logits that are the fp32 ones rounded."""
     from loongforge_amd import ops
 
-    test_forward_shares_a_query_among_workgroups(gpu, S, 64, K, q_start, skv)
-    inp = O.make_mla_inputs(S, 64, K, seed=5, skv=skv, q_start=q_start)
+    test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv)
+    inp = O.make_mla_inputs(S, H, K, seed=5, skv=skv, q_start=q_start)
+    inp.idx[:, ::7] += S + q_start    # beyond the keys: no valid slots
+    ro, rl, _ = O.sparse_mla_fwd(inp.q, inp.kv, inp.idx, q_start, inp.sm_scale, 512)
+    out, lse, _ = _run_fwd(inp, gpu, q_start)
+    assert_close(out, ro, "out")
+    fin = torch.isfinite(rl)
+    assert torch.equal(torch.isfinite(lse.cpu()), fin) and (lse.cpu() - rl)[fin].abs().max().item() < 1e-4
     for skip in (0, 64):
         p16, p32 = (ops.sparse_mla_fwd(inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), q_start, inp.sm_scale, 512, True, dt, p_out_skip=skip)[2]
                     for dt in (torch.bfloat16, torch.float32))
