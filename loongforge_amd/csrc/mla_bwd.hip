@@ -11,9 +11,8 @@
 //   pass C  per-pair rows  dS^T.Q + P^T.dO  (sum over all heads) -> one bf16 row of 576 values in a pair
 //           buffer, at the position given by a key-sorted order
 //   pass D  dKV[key] = sum of that key's rows, in ascending query order
-// Passes A and C are one kernel (bwd_pds_rows_kernel) where both orientations can be kept, from 64 heads
-// on; with 32 heads they are two (bwd_pds_kernel, bwd_dkv_kernel), and P and dS pass through HBM in the
-// MFMA operand layout of pass C.  Passes B and D share a launch (bwd_dq_reduce_kernel).
+// Passes A and C are one kernel (bwd_pds_rows_kernel) that keeps both orientations and P on the compute unit, passes B and D
+// share a launch (bwd_dq_reduce_kernel).
 // The key-sorted order (pass 0) comes from a bitmap key x query, its row-wise prefix popcounts and
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
@@ -24,180 +23,11 @@ namespace {
 using namespace mla;
 
 // P or dS of one (query, tile): [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes are
-// compiled for: 1 or 2, or 4 for 96 and 128 heads.  In memory a tile is dS and then P; dS alone where passes A and C are one.
+// compiled for: 1 or 2, or 4 for 96 and 128 heads.
 constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
-constexpr int pds_tile_bytes(int HG) { return HG >= 2 ? pds_kind_bytes(HG) : 2 * pds_kind_bytes(HG); }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
-
-// ---------------------------------------------------------------------------------------------
-// pass A: P and dS of every (query, tile)
-// ---------------------------------------------------------------------------------------------
-// With up to 32 heads, one workgroup of eight waves per query.  S = Q.KV^T and dP = dO.V^T are 16x16x32 MFMAs with the heads on the
-// rows (Q and dO rows resident in registers, 8 d-values per lane and step) and the 16 keys of a half tile on the columns (key rows
-// read from LDS, one 1 KB read feeding both products).  Two waves hold all heads, so waves 4-7 take every other tile (two tiles per
-// step, STAGES = 4 tiles are then two steps), and a wave takes one half tile of its tile only.  (Idle or repeated heads cost as much
-// as real ones.)  A lane ends with 4 heads of one key, half a chunk in the order pass C reads: chunk group 2w + g = heads 16w +
-// {4g .. 4g+3, 8+4g .. 8+4g+3}.
-template <int STAGES>
-__device__ __forceinline__ void pds_body(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
-    const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, int q0, int ql, int H, int Skv, int K, int q_start, float sm_scale,
-    unsigned char* smem) {
-  constexpr int KS = DQK / 32, VS = DV / 32;   // 18 and 16 steps of 32 d-values
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m = lane & 15, kg = lane >> 4;
-  const int hw = wave & 1, kt = (wave >> 1) & 1;       // heads 16 hw .., half tile of the tile
-  const int qi = q0 + ql;
-  const int NT = K / BI;
-  int* idx_s = (int*)(smem + STAGES * TILE_BYTES);
-  unsigned* tmask = (unsigned*)(idx_s + K);
-  int* tlist = (int*)(tmask + NT);
-  int* ntile_s = tlist + NT;
-  float* stat_s = (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
-  // All of the query's rows are requested before the ids are staged: one round trip to memory for
-  // both, instead of one after the other.
-  const int h = hw * 16 + m;
-  const bool head_ok = h < H;
-  const size_t hrow = (size_t)qi * H + (head_ok ? h : 0);
-  bf16x8 qreg[KS], doreg[VS], oreg[VS];
-  {
-    const bf16x8* qp = (const bf16x8*)(q + hrow * DQK) + kg;
-    const bf16x8* dp = (const bf16x8*)(dout + hrow * DV) + kg;
-    const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) qreg[ks] = qp[4 * ks];
-#pragma unroll
-    for (int ks = 0; ks < VS; ks++) doreg[ks] = dp[4 * ks];
-#pragma unroll
-    for (int ks = 0; ks < VS; ks++) oreg[ks] = op[4 * ks];
-  }
-  const float lse_h = lse[hrow];
-  __builtin_amdgcn_sched_barrier(0);
-  // (the helper is written for four waves; the other four repeat part of its work with equal results)
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
-  // Q and part of dO live in accumulation registers, which MFMA reads directly
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+a"(qreg[ks]));
-#pragma unroll
-  for (int ks = 0; ks < VS; ks++) {
-    if (ks < 6) asm volatile("" : "+a"(doreg[ks]));
-    else asm volatile("" : "+v"(doreg[ks]));
-  }
-#pragma unroll
-  for (int ks = 0; ks < VS; ks++) asm volatile("" : "+v"(oreg[ks]));
-
-  const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  // Transfers of a tile: each half of the workgroup moves its own; thread (key, sub) moves 16 bytes of every 128-byte group of the
-  // key's row.  Within a group the 16-byte chunk c of key row r sits in slot c ^ (r & 7).  (The slot function of
-  // the other kernels' tiles also serves their transposing reads; with it this kernel's reads - 16 rows x 4
-  // chunks per instruction - take two LDS cycles where one is needed.)
-  const int hh = wave >> 2;
-  const int gkey = (tid & 255) >> 3, gsub = tid & 7;
-  constexpr int NSTEP = 9;
-  const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16);
-  unsigned t_goff = 0, t_lb = 0;
-  auto issue_prepare = [&](int n) {
-    const int tile = tlist[n];
-    int kid = idx_s[tile * BI + gkey];
-    kid = kid < 0 ? 0 : kid;
-    t_goff = (unsigned)kid * (DQK * 2) + gslot;
-    t_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % STAGES) * TILE_BYTES + (wave & 3) * 1024));
-  };
-  auto issue_step = [&](int i) { dma16(t_lb + i * GRP_BYTES, t_goff + i * 128, kv); };
-  if (hh < ntiles) {
-    issue_prepare(hh);
-#pragma unroll
-    for (int i = 0; i < NSTEP; i++) issue_step(i);
-  }
-  // delta = rowsum(O . dO) while the first tiles travel
-  {
-    float part = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < VS; ks++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) part = fmaf((float)oreg[ks][e], (float)doreg[ks][e], part);
-    part += __shfl_xor(part, 16, 64);
-    part += __shfl_xor(part, 32, 64);
-    if (kg == 0) {
-      stat_s[h] = head_ok ? lse_h * LOG2E : INFINITY;
-      stat_s[128 + h] = head_ok ? part : 0.f;
-    }
-  }
-  __syncthreads();
-  // accumulator i of a lane is head 16*hw + 4*kg + i, for key 16*kt + m
-  const f32x4 lse2 = *(const f32x4*)(stat_s + hw * 16 + 4 * kg);
-  const f32x4 delta = *(const f32x4*)(stat_s + 128 + hw * 16 + 4 * kg);
-
-  // key-row operand of step ks: row 16*kt + m, 16-byte chunk 4*ks + kg of the row
-  const int krow = 16 * kt + m;
-  unsigned boff[2];
-#pragma unroll
-  for (int par = 0; par < 2; par++) boff[par] = (unsigned)(krow * 128 + (((4 * par + kg) ^ (krow & 7)) << 4));
-  const float c2 = sm_scale * LOG2E;
-
-  f32x4 sacc, dpacc;
-  // P and dS of the accumulated tile: the lane's 4 heads for its key, two registers (4 bf16) each
-  auto finish = [&](int tile, unsigned mask) {
-    const bool valid = (mask >> krow) & 1u;
-    float pf[4], df[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[i], c2, -lse2[i])) : 0.f;
-      df[i] = pf[i] * (dpacc[i] - delta[i]) * sm_scale;
-    }
-    unsigned char* base = pds + ((size_t)ql * NT + tile) * pds_tile_bytes(1) + (size_t)(2 * hw + (kg & 1)) * 512 + krow * 16 + (kg >> 1) * 8;
-    *(uint2*)base = make_uint2(cvt_pk_bf16(df[0], df[1]), cvt_pk_bf16(df[2], df[3]));
-    *(uint2*)(base + pds_kind_bytes(1)) = make_uint2(cvt_pk_bf16(pf[0], pf[1]), cvt_pk_bf16(pf[2], pf[3]));
-  };
-  // S and dP of a tile in LDS; `more`: with the transfers of a later tile between the products
-  auto products = [&](const unsigned char* tb, bool more) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) { sacc[e] = 0.f; dpacc[e] = 0.f; }
-    constexpr int FD = 4;                      // operand reads in flight
-    bf16x8 f[FD];
-    auto operand = [&](int ks) { return *(const bf16x8*)(tb + (ks >> 1) * GRP_BYTES + boff[ks & 1]); };
-#pragma unroll
-    for (int j = 0; j < FD; j++) f[j] = operand(j);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[ks], f[ks % FD], sacc, 0, 0, 0);
-      if (ks < VS) dpacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(doreg[ks], f[ks % FD], dpacc, 0, 0, 0);
-      if (ks + FD < KS) f[ks % FD] = operand(ks + FD);
-      if (ks % 2 == 1 && more) issue_step(ks / 2);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-
-  // Between two barriers every wave runs the MFMAs of one tile and one `finish`; waves 0-3 finish the
-  // tile they just accumulated, waves 4-7 first finish the previous one.  The two waves of a SIMD (w and
-  // w + 4) are thus half a step apart: the arithmetic and stores of one run under the other's MFMAs.
-  int tile = 0;
-  unsigned mask = 0;
-  // two tiles per step, one per half of the workgroup; the next step's are in flight
-  for (int i = 0; 2 * i < ntiles; i++) {
-    const int n = 2 * i + hh;
-    // behind the tile's transfers: the two stores of the step before (waves 0-3), nothing (waves 4-7)
-    if (hh == 0 && i > 0) { DSA_WAIT_VMCNT(2); } else { DSA_WAIT_VMCNT(0); }
-    __syncthreads();
-    if (hh == 1 && i > 0) finish(tile, mask);
-    if (n < ntiles) {
-      const bool more = n + 2 < ntiles;
-      if (more) issue_prepare(n + 2);
-      tile = __builtin_amdgcn_readfirstlane(tlist[n]);
-      mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
-      __builtin_amdgcn_sched_barrier(0);
-      products(smem + (n % STAGES) * TILE_BYTES, more);
-      if (hh == 0) finish(tile, mask);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  if (hh == 1 && ntiles > 1 && (ntiles & 1) == 0) finish(tile, mask);      // (odd counts: done in the last step)
-}
 
 // ---------------------------------------------------------------------------------------------
 // pass B: dQ
@@ -279,7 +109,7 @@ __device__ __forceinline__ void dq_body(
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
     t_lb = __builtin_amdgcn_readfirstlane(sb + (unsigned)((wave & 3) * 1024 + (wave >> 2) * GRP_BYTES));
     t_lbd = __builtin_amdgcn_readfirstlane(sb + (unsigned)(TILE_BYTES + (wave & (DS_WAVES - 1)) * 1024));
-    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(HG));     // dS
+    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(HG));     // dS
   };
   // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0 .. DS_WAVES - 1)
   auto issue_step = [&](int j) {
@@ -384,136 +214,7 @@ __device__ __forceinline__ void dq_body(
 }
 
 // ---------------------------------------------------------------------------------------------
-// pass C: per-pair dKV rows
-// ---------------------------------------------------------------------------------------------
-// row[key, d] = sum_h dS[h,key] Q[h,d] + (d < 512) sum_h P[h,key] dO[h,d], as row^T = X^T . coef with
-// X = [Q; dO] (k = heads).  With up to 32 heads X^T takes 72 registers: wave w owns the 32-column d-tiles
-// {w, w+4, w+8, w+12, w+16} (the last only for w < 2) and loads its columns once per query through LDS
-// transpose reads; two workgroups share a compute unit and hide each other's set-up, barriers and stores.
-// The coefficients arrive in pass A's layout, read from LDS as stored; a column tile is rounded to bf16, its four 8-byte
-// pieces per lane are turned into two 16-byte pieces by a trade between the half-waves, and these are stored as 32-byte halves of
-// the tile's 64 bytes in each of its 32 rows.  Bound by the rows.
-constexpr int DKV_STAGES = 4;            // coefficient tiles in the LDS ring
-template <int NC>
-__device__ __forceinline__ void dkv_body(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
-    const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int ql, int H, int Skv, int K, int q_start, int dummy_row, unsigned char* smem) {
-  constexpr int HG = 1, CST = DKV_STAGES, M = 2 * HG, TB = pds_tile_bytes(HG);
-  // [CST][TB] coefficient ring, shared with the set-up's per-wave X staging [4][HG * 2048] | ids arrays | dst rows [K]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 31, g = lane >> 5;
-  const int qi = q0 + ql;
-  const int NT = K / BI;
-  unsigned char* xs = smem + wave * (HG * 2048);
-  int* idx_s = (int*)(smem + CST * TB);
-  unsigned* tmask = (unsigned*)(idx_s + K);
-  int* tlist = (int*)(tmask + NT);
-  int* ntile_s = tlist + NT;
-  int* dst_s = ntile_s + 4;
-  for (int t0 = tid; t0 < K; t0 += 8 * 256) {        // eight loads in flight per thread
-    int d[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) d[i] = t0 + i * 256 < K ? dst[(size_t)ql * K + t0 + i * 256] : -1;
-#pragma unroll
-    for (int i = 0; i < 8; i++)       // invalid slots land in a scratch row: the store count stays fixed
-      if (t0 + i * 256 < K) dst_s[t0 + i * 256] = d[i] >= 0 ? d[i] : dummy_row;
-  }
-  // X^T operands, k-step kk = 16 heads: column tiles wave + 4 c of Q (c < NC) and of dO (c < 4)
-  bf16x8 xq[NC][M], xo[4][M];
-  {
-    typedef short i16x8 __attribute__((ext_vector_type(8)));
-    const int blk = lane >> 4, ii = lane & 15;
-    const unsigned xoff = (unsigned)((4 * g + (ii >> 2)) * 64 + (16 * (blk & 1) + 4 * (ii & 3)) * 2);
-    constexpr int NP = NC + 4;
-    uint4 ld[3][M];                            // three passes of global loads in flight
-    auto pass_load = [&](int pass, uint4 (&v)[M]) {
-      const bool isq = pass < NC;
-      const int c = wave + 4 * (isq ? pass : pass - NC);
-      const __bf16* src = isq ? q + (size_t)qi * H * DQK + 32 * c : dout + (size_t)qi * H * DV + 32 * c;
-      const int stride = isq ? DQK : DV;
-#pragma unroll
-      for (int it = 0; it < M; it++)           // rows of 64 bytes: lane covers head lane/4 + 16*it, 16-byte piece lane%4
-        v[it] = *(const uint4*)(src + (size_t)((lane >> 2) + 16 * it) * stride + (lane & 3) * 8);
-    };
-    pass_load(0, ld[0]);
-    pass_load(1, ld[1]);
-    pass_load(2, ld[2]);
-#pragma unroll
-    for (int pass = 0; pass < NP; pass++) {
-#pragma unroll
-      for (int it = 0; it < M; it++) *(uint4*)(xs + ((lane >> 2) + 16 * it) * 64 + (lane & 3) * 16) = ld[pass % 3][it];
-      if (pass + 3 < NP) pass_load(pass + 3, ld[pass % 3]);
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int kk = 0; kk < M; kk++) {
-        const unsigned char* hb = xs + 16 * kk * 64;
-        const i16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + xoff));
-        const i16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(i16x4, hb + 8 * 64 + xoff));
-        const bf16x8 val = __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
-        if (pass < NC) xq[pass < NC ? pass : 0][kk] = val;
-        else xo[pass < NC ? 0 : pass - NC][kk] = val;
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
-  // (its barriers also part the X staging from the coefficient ring, which shares LDS with it)
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
-  if (ntiles == 0) return;
-
-  const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  auto issue = [&](int n) {
-    const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((n % CST) * TB + wave * 1024));
-    const unsigned char* src = uniform_ptr(pds + ((size_t)ql * NT + tlist[n]) * TB);
-#pragma unroll
-    for (int c = 0; c < HG; c++) dma16(lb + c * 4096, (unsigned)(c * 4096 + tid * 16), src);
-  };
-  for (int n = 0; n < CST && n < ntiles; n++) issue(n);
-  const unsigned coff = (unsigned)(g * 512 + r * 16);      // coefficient chunk of k-step kk: [kind][kk][g][key r] 16 bytes
-  bf16x8 cf[2][M];
-  auto read_coefs = [&](int n) {
-    const unsigned char* tb = smem + (n % CST) * TB;
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-#pragma unroll
-      for (int kk = 0; kk < M; kk++) cf[k][kk] = *(const bf16x8*)(tb + k * pds_kind_bytes(HG) + kk * 1024 + coff);
-  };
-  DSA_WAIT_VMCNT(0);
-  __syncthreads();
-  read_coefs(0);
-  for (int n = 0; n < ntiles; n++) {
-    unsigned char* rptr = rows + (size_t)dst_s[tlist[n] * BI + r] * ROW_BYTES + wave * 64 + g * 16;
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      f32x16 acc;
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[e] = 0.f;
-#pragma unroll
-      for (int kk = 0; kk < M; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xq[c][kk], cf[0][kk], acc, 0, 0, 0);
-      if (c < 4) {
-#pragma unroll
-        for (int kk = 0; kk < M; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xo[c < 4 ? c : 0][kk], cf[1][kk], acc, 0, 0, 0);
-      }
-      uint4 o[2];
-      acc_row_to_16B(acc, 1.0f, o);
-      *(uint4*)(rptr + c * 256) = o[0];
-      *(uint4*)(rptr + c * 256 + 32) = o[1];
-    }
-    if (n + 1 < ntiles) {
-      // issued behind the next tile's transfers: HG per later tile in flight, 2 NC stores per tile since
-      if (n >= CST - 1 && n + CST - 1 < ntiles) { DSA_WAIT_VMCNT((CST - 2) * HG + (CST - 1) * 2 * NC); }
-      else if (n >= CST - 1) { DSA_WAIT_VMCNT((CST - 1) * 2 * NC); }
-      else { DSA_WAIT_VMCNT(2 * NC); }
-      __syncthreads();
-      if (n + CST < ntiles) issue(n + CST);    // into the slot of tile n, whose coefficients are in registers
-      read_coefs(n + 1);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// passes A and C in one, for 64 heads
+// passes A and C in one, for 32 and 64 heads
 // ---------------------------------------------------------------------------------------------
 // Q and dO of 64 heads fit the registers of a compute unit in both orientations: 136 per lane for the products over d (wave
 // (hw, hh) = (wave % 4, wave / 4): 16 heads, the 16 keys of half tile hh) and 64 for those over the heads (wave w: the columns
@@ -524,7 +225,9 @@ __device__ __forceinline__ void dkv_body(
 // of a SIMD issue stores and exponentials under each other's MFMAs.  The transfers of tile n + 2 come first in a step: between
 // the MFMAs behind the row stores of a step they held waves 4-7 for 2600 cycles per tile instead of 1100.
 // Bound by the row writes: a step of 5000 cycles writes 41 KB per compute unit, 4.7 TB/s, and the set-up of a query (208 KB
-// read, 36 000 cycles) does not overlap it.  3072 queries x 128 + 512 slots of compressed keys: 0.68 ms against 0.41 + 0.51; 2077 x 512: 0.35 against 0.23 + 0.26.
+// read, 31 000 cycles) does not overlap it.  3072 queries x 128 + 512 slots of compressed keys: 0.68 ms against 0.41 + 0.51; 2077 x 512: 0.35 against 0.23 + 0.26.
+// 32 heads have the same rows to write; four waves then have no scores to make.  The whole backward of 3072 queries x 640 slots 1501 ->
+// 1108 us against two passes with P and dS in memory, 3000 x 2048 3172 -> 2474, 1024 x 256 254 -> 204.
 constexpr int FUSED_STAGES = 3;
 constexpr int FUSED_XCH = 2 * pds_kind_bytes(2);      // P and dS of a tile
 constexpr int FUSED_ROT = 16384;                      // every wave's operands of the rotary columns
@@ -532,18 +235,20 @@ static_assert(64 * (DQK + DV) * 2 <= FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH +
 __host__ __device__ inline size_t fused_lds_bytes(int K) {
   return (size_t)FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT + ids_lds_bytes(K) + 512 + (size_t)K * 4;
 }
-template <int hh>
+template <int hh, int HG>                    // HG: groups of 32 heads, 2 or 1
 __device__ __forceinline__ void pds_rows_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int ql, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
-  constexpr int H = 64, KS = DQK / 32, VS = DV / 32, STAGES = FUSED_STAGES;
+  constexpr int H = 32 * HG, KS = DQK / 32, VS = DV / 32, STAGES = FUSED_STAGES;
   constexpr int DO_ACC = 12;                   // steps of dO in accumulation registers, beside all of Q: 120
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4, g = lane >> 5;
-  const int hw = wave & 3;
+  // One group: two waves of each half have S and dP, on SIMDs 0, 1 and 2, 3; the other four the rows alone.
+  const int hw = HG == 2 ? wave & 3 : wave & 1;
+  const bool scores = HG == 2 || (wave & 3) >> 1 == hh;
   const int qi = q0 + ql;
   const int NT = K / BI;
   // [ring][P and dS, two buffers][rotary operands], all of it Q and dO of the query at first | ids arrays | statistics | dst rows [K]
@@ -563,7 +268,7 @@ __device__ __forceinline__ void pds_rows_body(
   __builtin_amdgcn_sched_barrier(0);
   // Q and dO travel to LDS as they are, in groups of 128 bytes of all 64 rows (Q: 9, dO: 8), chunk c of row r in slot c ^ (r & 7):
   // both orientations are read from there.  Wave w moves rows 8 w .. 8 w + 7.
-  {
+  if (8 * wave < H) {
     const __bf16* q_rows = uniform_ptr(q + (size_t)qi * H * DQK);
     const __bf16* do_rows = uniform_ptr(dout + (size_t)qi * H * DV);
     const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
@@ -576,7 +281,7 @@ __device__ __forceinline__ void pds_rows_body(
   const int h = hw * 16 + m;
   const size_t hrow = (size_t)qi * H + h;
   bf16x8 qreg[KS], doreg[VS], oreg[VS];
-  {
+  if (scores) {
     const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
 #pragma unroll
     for (int ks = 0; ks < VS; ks++) oreg[ks] = op[4 * ks];
@@ -590,26 +295,22 @@ __device__ __forceinline__ void pds_rows_body(
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();
-  {
+  if (scores) {
     const unsigned char* rb = smem + h * 128;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qreg[ks] = *(const bf16x8*)(rb + (ks >> 1) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
+    for (int ks = 0; ks < KS; ks++) {
+      qreg[ks] = *(const bf16x8*)(rb + (ks >> 1) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
+      asm volatile("" : "+a"(qreg[ks]));
+    }
+    float part = 0.f;                          // delta = rowsum(O . dO)
 #pragma unroll
-    for (int ks = 0; ks < VS; ks++) doreg[ks] = *(const bf16x8*)(rb + (9 + (ks >> 1)) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
-  }
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+a"(qreg[ks]));
-#pragma unroll
-  for (int ks = 0; ks < VS; ks++) {
-    if (ks < DO_ACC) asm volatile("" : "+a"(doreg[ks]));
-    else asm volatile("" : "+v"(doreg[ks]));
-  }
-  {                                            // delta = rowsum(O . dO)
-    float part = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < VS; ks++)
+    for (int ks = 0; ks < VS; ks++) {
+      doreg[ks] = *(const bf16x8*)(rb + (9 + (ks >> 1)) * 8192 + (((4 * (ks & 1) + kg) ^ (h & 7)) << 4));
 #pragma unroll
       for (int e = 0; e < 8; e++) part = fmaf((float)oreg[ks][e], (float)doreg[ks][e], part);
+      if (ks < DO_ACC) asm volatile("" : "+a"(doreg[ks]));
+      else asm volatile("" : "+v"(doreg[ks]));
+    }
     part += __shfl_xor(part, 16, 64);
     part += __shfl_xor(part, 32, 64);
     if (kg == 0) {
@@ -626,7 +327,7 @@ __device__ __forceinline__ void pds_rows_body(
   };
   // Row 4 j + e of the operand is column {0, 8, 4, 12}[j] + e of the 16, so that lanes 32 apart end up with neighbouring columns.
   // The heads of lane chunk kg are 32 ks + 16 (kg / 2) + 4 (kg % 2) + {0 .. 3, 8 .. 11}.
-  bf16x8 xq[4][2], xo[4][2];
+  bf16x8 xq[4][HG], xo[4][HG];
   {
     const int ii = lane & 15, jj = ((ii & 1) << 1) | ((ii >> 1) & 1);
     const int hd = 16 * (kg >> 1) + 4 * (kg & 1) + (ii >> 2);
@@ -634,9 +335,9 @@ __device__ __forceinline__ void pds_rows_body(
       const unsigned char* p = smem + group * 8192 + (32 * ks + hd) * 128 + (((2 * c + (jj >> 1)) ^ (hd & 7)) << 4) + (jj & 1) * 8;
       return tr_pair(p, p + 8 * 128);
     };
-    bf16x8 xr[2];
+    bf16x8 xr[HG];
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
+    for (int ks = 0; ks < HG; ks++) {
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         xq[c][ks] = column_operand(wave, c, ks);
@@ -645,13 +346,13 @@ __device__ __forceinline__ void pds_rows_body(
       xr[ks] = column_operand(8, wave & 3, ks);      // rotary columns 16 (wave % 4) ..
     }
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
+    for (int ks = 0; ks < HG; ks++) {
       asm volatile("" : "+v"(xq[0][ks]), "+v"(xq[1][ks]), "+v"(xq[2][ks]), "+v"(xq[3][ks]), "+v"(xr[ks]));
       asm volatile("" : "+v"(xo[0][ks]), "+v"(xo[1][ks]), "+v"(xo[2][ks]), "+v"(xo[3][ks]));
     }
     __syncthreads();                           // every wave has its operands: the space is the ring's from here on
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) xr_s[64 * ks] = xr[ks];
+    for (int ks = 0; ks < HG; ks++) xr_s[64 * ks] = xr[ks];
   }
 
   // transfers of a tile, as in pass A: waves 0-3 take groups 0-4, waves 4-7 groups 5-8
@@ -715,7 +416,7 @@ __device__ __forceinline__ void pds_rows_body(
     unsigned char* xb = xch + (n & 1) * FUSED_XCH + half_chunk;
     *(uint2*)xb = dw;
     *(uint2*)(xb + pds_kind_bytes(2)) = pw;
-    *(uint2*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(2) + half_chunk) = dw;
+    *(uint2*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(HG) + half_chunk) = dw;
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
@@ -724,9 +425,9 @@ __device__ __forceinline__ void pds_rows_body(
     const int* drow = dst_s + tlist[n] * BI;
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      bf16x8 cs[2], cp[2];
+      bf16x8 cs[HG], cp[HG];
 #pragma unroll
-      for (int ks = 0; ks < 2; ks++) {
+      for (int ks = 0; ks < HG; ks++) {
         cs[ks] = *(const bf16x8*)(xb + ks * 2048 + coff + kt * 256);
         cp[ks] = *(const bf16x8*)(xb + pds_kind_bytes(2) + ks * 2048 + coff + kt * 256);
       }
@@ -735,11 +436,11 @@ __device__ __forceinline__ void pds_rows_body(
       for (int cp2 = 0; cp2 < 2; cp2++) {
         f32x4 acc[2];
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++)
+        for (int ks = 0; ks < HG; ks++)
 #pragma unroll
           for (int i = 0; i < 2; i++) mfma16_v(acc[i], xq[2 * cp2 + i][ks], cs[ks], ks == 0);
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++)
+        for (int ks = 0; ks < HG; ks++)
 #pragma unroll
           for (int i = 0; i < 2; i++) mfma16_v(acc[i], xo[2 * cp2 + i][ks], cp[ks], false);
         mfma16_done(acc[0], acc[1]);
@@ -756,7 +457,7 @@ __device__ __forceinline__ void pds_rows_body(
       if (kt == hh) {
         f32x4 acc;
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++) mfma16_v(acc, xr_s[64 * ks], cs[ks], ks == 0);
+        for (int ks = 0; ks < HG; ks++) mfma16_v(acc, xr_s[64 * ks], cs[ks], ks == 0);
         mfma16_done(acc);
         *(uint2*)(row + rotoff) = make_uint2(cvt_pk_bf16(acc[0], acc[1]), cvt_pk_bf16(acc[2], acc[3]));
       }
@@ -768,20 +469,24 @@ __device__ __forceinline__ void pds_rows_body(
   for (int n = 0; n <= ntiles; n++) {
     asm volatile("" : "+s"(n));                // one copy of the loop: peeled ones cost registers
     // A wave's operations behind the transfer of tile n, which went out two steps ago.  A step is 5 transfers (4 of waves 4-7), the
-    // dS store and 5 row stores.  The first tiles and the last one, behind which there are fewer, wait for all.
+    // dS store (not of every wave with one group) and 5 row stores.  The first tiles and the last one, behind which there are fewer,
+    // wait for all.
     if (n < ntiles) {
-      if (n >= 3 && n + 1 < ntiles) { if (hh == 0) { DSA_WAIT_VMCNT(17); } else { DSA_WAIT_VMCNT(16); } }
+      if (n >= 3 && n + 1 < ntiles) {
+        if (HG == 2) { if (hh == 0) { DSA_WAIT_VMCNT(17); } else { DSA_WAIT_VMCNT(16); } }
+        else { if (hh == 0) { DSA_WAIT_VMCNT(15); } else { DSA_WAIT_VMCNT(14); } }
+      }
       else { DSA_WAIT_VMCNT(0); }
     }
     __syncthreads();
     if (n + STAGES - 1 < ntiles) issue(n + STAGES - 1);       // ahead of the step's stores, which the transfers would queue behind
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (hh == 0) {
-      if (n < ntiles) phase_pds(n);
+      if (n < ntiles && scores) phase_pds(n);
       if (n > 0) phase_rows(n - 1);
     } else {
       if (n > 0) phase_rows(n - 1);
-      if (n < ntiles) phase_pds(n);
+      if (n < ntiles && scores) phase_pds(n);
     }
   }
 }
@@ -1036,7 +741,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
     const uint4 d16 = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
     *(uint4*)(xch + chunk) = d16;
     *(uint4*)(xch + pds_kind_bytes(4) + chunk) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
-    *(uint4*)(pds + ((size_t)ql * NT + tile) * pds_tile_bytes(4) + chunk) = d16;
+    *(uint4*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(4) + chunk) = d16;
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
@@ -1208,14 +913,6 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-__global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_kernel(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
-    const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  pds_body<4>(q, kv, ids, out, dout, lse, pds, q0, cnt - 1 - (int)blockIdx.x, H, Skv, K, q_start, sm_scale, smem);
-}
-
 template <int HG>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
@@ -1225,25 +922,13 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int ql = cnt - 1 - (int)blockIdx.x;
   // (two copies of the body: every copy meets the same barriers)
-  if constexpr (HG == 2) {
-    if (threadIdx.x < 256) pds_rows_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-    else pds_rows_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+  if constexpr (HG <= 2) {
+    if (threadIdx.x < 256) pds_rows_body<0, HG>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_body<1, HG>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
   } else {
     if (threadIdx.x < 256) pds_rows_wide_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
     else pds_rows_wide_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
   }
-}
-
-__global__ __launch_bounds__(256, 2) void bwd_dkv_kernel(
-    const __bf16* __restrict__ q, const __bf16* __restrict__ dout, const int* __restrict__ ids,
-    const unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int cnt, int H, int Skv, int K, int q_start, int dummy_row) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int ql = cnt - 1 - (int)blockIdx.x;
-  // waves 0 and 1 own five column tiles, waves 2 and 3 four: two copies of the whole body, so that
-  // no branch sits between the MFMAs; every copy meets the same barriers
-  if (threadIdx.x < 128) dkv_body<5>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
-  else dkv_body<4>(q, dout, ids, pds, dst, rows, q0, ql, H, Skv, K, q_start, dummy_row, smem);
 }
 
 template <int HG>
@@ -1302,7 +987,7 @@ BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
   p.off_flag = o; o = align_up(o + 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
-  p.off_pds = o; o = align_up(o + (size_t)chunk * (K / BI) * pds_tile_bytes(head_groups(H)));
+  p.off_pds = o; o = align_up(o + (size_t)chunk * (K / BI) * pds_kind_bytes(head_groups(H)));
   p.off_rows = o; o = align_up(o + ((size_t)chunk * K + 1) * ROW_BYTES);
   p.off_acc = o; o = align_up(o + (size_t)Skv * DQK * 4);
   p.total = o;
@@ -1366,18 +1051,13 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   float* acc = (float*)(ws + p.off_acc);
 
   const int HG = head_groups(H);
-  const size_t smemA = (size_t)4 * TILE_BYTES + ids_lds_bytes(K) + 16 + 1024;
   const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
   size_t smemB = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
   if (smemB < reduce_lds) smemB = reduce_lds;
-  const size_t smemC = (size_t)DKV_STAGES * pds_tile_bytes(1) + ids_lds_bytes(K) + 16 + (size_t)K * 4;
   auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
-  const bool one_pass = HG >= 2;               // passes A and C
-  auto pds_rows_kernel = HG == 2 ? bwd_pds_rows_kernel<2> : bwd_pds_rows_kernel<4>;
-  const size_t smemAC = HG == 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
-  if ((one_pass ? dsa_reserve_lds((const void*)pds_rows_kernel, smemAC) != hipSuccess
-                : dsa_reserve_lds((const void*)bwd_pds_kernel, smemA) != hipSuccess ||
-                  dsa_reserve_lds((const void*)bwd_dkv_kernel, smemC) != hipSuccess) ||
+  auto pds_rows_kernel = HG == 1 ? bwd_pds_rows_kernel<1> : HG == 2 ? bwd_pds_rows_kernel<2> : bwd_pds_rows_kernel<4>;
+  const size_t smemAC = HG <= 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
+  if (dsa_reserve_lds((const void*)pds_rows_kernel, smemAC) != hipSuccess ||
       dsa_reserve_lds((const void*)dq_reduce_kernel, smemB) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
 
@@ -1408,21 +1088,11 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
-    if (one_pass) {
-      pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemAC, st>>>(
-          (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, H, Skv, K, q_start,
-          sm_scale, p.chunk * K);
-      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
-      DSA_MARK(2);
-    } else {
-      bwd_pds_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemA, st>>>((const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out,
-                                                         (const __bf16*)dout, lse, pds, q0, cnt, H, Skv, K, q_start, sm_scale);
-      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS)");
-      DSA_MARK(2);
-      bwd_dkv_kernel<<<dim3(cnt), dim3(256), smemC, st>>>((const __bf16*)q, (const __bf16*)dout, sids, pds, dstp, rows, q0, cnt,
-                                                         H, Skv, K, q_start, p.chunk * K);
-      DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dKV rows)");
-    }
+    pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemAC, st>>>(
+        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, H, Skv, K, q_start,
+        sm_scale, p.chunk * K);
+    DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
+    DSA_MARK(2);
     DSA_MARK(3);
     // Pass B of every query beside pass D of every key.
     dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smemB, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
