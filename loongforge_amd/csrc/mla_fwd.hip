@@ -14,7 +14,7 @@
 //
 // How a workgroup shares a query's heads and slots is the MODE:
 //   0  128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
-//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel<2>.
+//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel<2>; with one pair of tiles any heads.
 //   4  32 heads, likewise: mla_fwd_half_kernel<1>.
 //   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
 //      of every other tile; the two streams' sums are merged through LDS at the end.
@@ -1241,8 +1241,6 @@ int max_slots(int mode) {                    // slots of a range whose id arrays
 constexpr int SHARE_RANGES = 4, SHARE_BLOCKS = 16;
 bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES && (long)S * (H / 32) <= SHARE_BLOCKS; }
 
-FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
-
 // The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
 // units, each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel that follows.
 // The constants are measured times in us (random rows; a pair of tiles on an idle chip and on a full one: the gathers
@@ -1255,15 +1253,17 @@ FwdPlan one_workgroup_per_query(int K) { return {0, 1, 1, K}; }
 // 140, 512 147 and 158, 3000 817 and 900.  A round of 512 that is at most half full is priced as what it takes where the keys
 // lie far apart (700 queries, 65536 keys: 281 and 251; 8192 keys: 215 and 224).  Mode 4 likewise: 257 queries of 32 heads 78 us
 // against 112 in mode 2, 600 queries 167 and 177 (65536 keys: 233 and 222), 800 queries 175 and 236.
-// A query with one pair of tiles has nothing to share out: mode 0.
+// The fixed part is what a full round takes with two to four pairs (the rows of 256 queries come in together); 4000 queries of 128 heads:
+// 256 slots 440 us in mode 0 and 390 in mode 3, 640 slots 760 and 800.  One pair of tiles is always mode 3, so that a query has
+// the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
-  if (K <= 2 * BI) return one_workgroup_per_query(K);
   constexpr float REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
-  constexpr float FIXED[5] = {6.0f, 6.0f, 6.0f, 12.0f, 8.5f}, PAIR_FULL[5] = {3.65f, 2.3f, 1.8f, 4.0f, 2.8f};
-  constexpr float PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.1f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
+  constexpr float FIXED_IDLE = 6.0f, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
+  constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.2f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
   constexpr int HEADS[5] = {128, 64, 32, 64, 32}, SLOTS[5] = {256, 256, 256, 512, 512};
+  if (K <= 2 * BI) return {3, (H + HEADS[3] - 1) / HEADS[3], 1, K};
   const int pairs = K / (2 * BI);
-  FwdPlan best = one_workgroup_per_query(K);
+  FwdPlan best = {0, 1, 1, K};
   float best_t = 1e30f;
   for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 5; mode++) {
     if (mode == (H > 32 ? 4 : 3)) continue;
@@ -1276,8 +1276,9 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const float pair = mode < 3      ? PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode])
                          : rest > 0.5f ? PAIR_SHARED[mode] + 2.0f * (rest - 0.5f) * (PAIR_FULL[mode] - PAIR_SHARED[mode])
                                        : PAIR_IDLE[mode];
-      float t = (float)(wgs / SLOTS[mode]) * (FIXED[mode] + per * PAIR_FULL[mode]);
-      if (rest > 0.0f) t += FIXED[mode] + per * pair;
+      const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE;
+      float t = (float)(wgs / SLOTS[mode]) * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
+      if (rest > 0.0f) t += fixed + per * pair;
       t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }

@@ -156,14 +156,16 @@ def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
 
 
 @pytest.mark.parametrize("S,H,K,q_start,skv", [
-    (3, 128, 64, 0, None),            # one tile, then none
-    (40, 128, 64, 30, None),          # one and two tiles
+    (3, 128, 64, 0, None),            # one pair of tiles, whatever the heads: one tile, then none
+    (40, 96, 64, 30, None),           # one and two tiles, the fourth 32-head block is not there
+    (5, 32, 64, 60, None),
     (260, 128, 192, 0, None),         # up to six tiles, fewer than the ring in the early rows; a second round of workgroups
     (170, 96, 320, 400, 500),         # the fourth 32-head block is not there
+    (300, 128, 768, 0, None),         # from one tile in the early rows to 24
     (48, 96, 2048, 3000, None),       # in ranges of slots
 ])
 def test_forward_of_many_heads(gpu, S, H, K, q_start, skv):
-    """The two-role kernel at the edges of its tile ring and of its heads, with the slot lists and the bounds of the forms above."""
+    """The two-role kernel, and the one for a pair of tiles, at the edges of their rings and heads; slot lists and bounds as above."""
     test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv)
 
 
