@@ -62,9 +62,9 @@ struct FwdArgs {
 // O^T accumulators are never rescaled (a rescaling branch in the loop, even one never taken, costs the
 // register allocator hundreds of spills).  Where a later tile exceeds it by more than 2^64 (exp2 then nears
 // the end of fp32) the wave marks its heads - a NaN with a payload in lse, or in the statistics of its
-// slot range - and the kernel that follows does them again relative to the true row maximum.  In mode 2 with all slots in
-// one workgroup, where the waves' registers have room for it, the workgroup does so itself: the kernel that follows takes
-// 4.5 us also when nothing is marked.
+// slot range - and the kernel that follows does them again relative to the true row maximum.  In modes 3 and 4, and in mode
+// 2 with all slots in one workgroup, where the waves' registers have room for it, the workgroup does so itself: the kernel that
+// follows takes 4.5 us also when nothing is marked.
 constexpr float REDO_ABOVE = 64.0f, REDO_TERM = 0x1p64f;
 constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
 __device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
@@ -821,6 +821,7 @@ constexpr int HALF_LDS = 2 * TILE_BYTES + HALF_P;
 constexpr int HALF_AHEAD = 6;                // row reads in flight
 __host__ __device__ inline size_t mask_lds_bytes(int K) { return (size_t)(K / BI) * 8 + 16; }
 static_assert(HALF_LDS + 8192 / BI * 8 + 16 <= 80 * 1024, "two workgroups on a compute unit at the longest list");
+static_assert(TILE_BYTES + 8192 * 4 + 8192 / BI * 8 + 16 <= HALF_LDS, "a tile and the ids of a block done again");
 
 // The tiles' slot function with bit 0 of the row alone below: 16 rows x 4 chunks (an operand of 16x16x32) and the transposed
 // reads of lane_offsets are both free of bank conflicts.
@@ -1100,17 +1101,18 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   if (lane == 0) again_s[w] = mine;
   if (HB == 1 && kg == 0) l_s[16 * w + m] = l_tot;
   __syncthreads();
-  const bool again = HB == 2 ? (again_s[w] | again_s[w ^ 1]) != 0 : (again_s[0] | again_s[1] | again_s[2] | again_s[3]) != 0;
+  const bool lower = __builtin_amdgcn_readfirstlane(again_s[0] | again_s[1]) != 0, upper = __builtin_amdgcn_readfirstlane(again_s[2] | again_s[3]) != 0;
+  const bool again[2] = {HB == 2 ? lower : lower || upper, upper};       // of the workgroup's blocks
   if (HB == 1) l_tot = l_s[16 * hw + m] + l_s[16 * hw + 32 + m];
   const Final fin = finish_head(m_ref, l_tot, a.sink && head_ok ? a.sink + h : nullptr);
   if (kg == 0 && h0 == 0) {
-    if (head_ok) a.lse[(size_t)qi * H + h] = again ? __builtin_bit_cast(float, REDO_MARK) : fin.lse;
+    if (head_ok && !again[HB == 2 ? w >> 1 : 0]) a.lse[(size_t)qi * H + h] = fin.lse;
     inv_s[16 * hw + m] = fin.inv;
   }
   __syncthreads();
 #pragma unroll
   for (int hb = 0; hb < HB; hb++) {
-    if (32 * (HB * hg + hb) >= H) break;
+    if (32 * (HB * hg + hb) >= H || again[hb]) continue;
     const float inv = inv_s[32 * hb + r];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -1120,9 +1122,19 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  for (int hb = 0; hb < HB; hb++) {          // here and not in a kernel behind this one: that takes 4.5 us also when nothing is marked
+    if (32 * (HB * hg + hb) >= H || !again[hb]) continue;
+#pragma unroll 1
+    for (int dt = w; dt < DTILES; dt += 4) {
+      f32x16 acc;
+      float m1, l1;
+      redo_block(a, qi, HB * hg + hb, dt, acc, m1, l1);
+      write_block(a, qi, HB * hg + hb, dt, acc, m1, l1);
+    }
+  }
 }
 
-// All modes but 2, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
+// Modes 0 and 1, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
 // redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
 __global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
   const int wave = threadIdx.x >> 6;
@@ -1279,7 +1291,7 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE;
       float t = (float)(wgs / SLOTS[mode]) * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += fixed + per * pair;
-      t += ksplit == 1 ? (mode == 2 ? 0.0f : REDO)
+      t += ksplit == 1 ? (mode >= 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
       if (wgs >= 4096) break;                // more ranges only add rounds
@@ -1319,7 +1331,7 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
   const bool shared = combine_shares(a.S, a.H, a.ksplit);
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
-  if (MODE == 2 && !SPLIT) return 0;
+  if (MODE >= 2 && !SPLIT) return 0;
   if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
   if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), 256, tail, st>>>(a);
   else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), 256, tail, st>>>(a);
