@@ -1254,24 +1254,23 @@ constexpr int SHARE_RANGES = 4, SHARE_BLOCKS = 16;
 bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES && (long)S * (H / 32) <= SHARE_BLOCKS; }
 
 // The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
-// units, each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel that follows.
-// The constants are measured times in us (random rows; a pair of tiles on an idle chip and on a full one: the gathers
-// of 256 workgroups share the fabric, and a last round that is half empty runs a pair nearly as fast as an idle chip does, hence
-// the square).  At 2048 slots and 128 heads one query takes 86 us in mode 0 and 18 as
-// 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0, 50 - 52 in mode 0 of four ranges or mode 1 of two; 128 queries 100 and 86
-// (mode 1), 160 queries 100 and 148; 300 queries 211 and 227, 600 queries 334 and 392; 48 queries of 96 heads 45 in mode 0 of four
-// ranges and 49 in mode 1 of two; 200 queries of 64 heads 77 (mode 1), 1500 of 32 heads 390 (mode 2).
-// Mode 3 gains by its second workgroup on a compute unit: 256 queries of 64 heads 94 us against 83 in mode 1, 300 queries 123 and
-// 140, 512 147 and 158, 3000 817 and 900.  A round of 512 that is at most half full is priced as what it takes where the keys
-// lie far apart (700 queries, 65536 keys: 281 and 251; 8192 keys: 215 and 224).  Mode 4 likewise: 257 queries of 32 heads 78 us
-// against 112 in mode 2, 600 queries 167 and 177 (65536 keys: 233 and 222), 800 queries 175 and 236.
-// The fixed part is what a full round takes with two to four pairs (the rows of 256 queries come in together); 4000 queries of 128 heads:
-// 256 slots 440 us in mode 0 and 390 in mode 3, 640 slots 760 and 800.  One pair of tiles is always mode 3, so that a query has
-// the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
+// units (512 places in modes 3 and 4), each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel
+// that follows.  The constants are measured times in us, random rows.  A round among others, FULL: the rows of all its queries come in
+// together, and the gathers of 256 workgroups share the fabric.  A single or last round, LAST: IDLE on an empty chip, and nearly that
+// while it is half empty, hence the square.  Modes 3 and 4 by whether workgroups share a compute unit; where few do, what they take
+// with keys that lie far apart.
+// 2048 slots, 128 heads: one query 86 us in mode 0 and 15 as 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0, 50 in mode
+// 0 of four ranges, 47 in mode 1 of two; 128 queries 100 and 82 (mode 1), 160 queries 100 and 148, 600 queries 334 and 392.  64 heads: 256 queries
+// 94 us in mode 3 and 83 in mode 1, 300 queries 123 and 140, 3000 817 and 900; 700 queries 215 and 224, with 65536 keys 281 and 251.
+// 32 heads: 257 queries 78 us in mode 4 and 112 in mode 2, 800 queries 175 and 236.  4000 queries of 128 heads: 256 slots 440 us in
+// mode 0 and 390 in mode 3, 640 slots 760 and 800.
+// One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
+// mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   constexpr float REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
   constexpr float FIXED_IDLE = 6.0f, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
-  constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.2f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
+  constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.2f};
+  constexpr float PAIR_LAST[3] = {3.65f, 2.15f, 1.65f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
   constexpr int HEADS[5] = {128, 64, 32, 64, 32}, SLOTS[5] = {256, 256, 256, 512, 512};
   if (K <= 2 * BI) return {3, (H + HEADS[3] - 1) / HEADS[3], 1, K};
   const int pairs = K / (2 * BI);
@@ -1284,12 +1283,13 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
       if (ksplit != want || 64 * per > max_slots(mode)) continue;
       const long wgs = (long)S * n_hg * ksplit;
-      const float rest = (float)(wgs % SLOTS[mode]) / (float)SLOTS[mode];
-      const float pair = mode < 3      ? PAIR_IDLE[mode] + rest * rest * (PAIR_FULL[mode] - PAIR_IDLE[mode])
+      const long rounds = wgs <= SLOTS[mode] ? 0 : wgs / SLOTS[mode];                  // full ones, with others behind or before
+      const float rest = (float)(wgs - rounds * SLOTS[mode]) / (float)SLOTS[mode];
+      const float pair = mode < 3      ? PAIR_IDLE[mode] + rest * rest * (PAIR_LAST[mode] - PAIR_IDLE[mode])
                          : rest > 0.5f ? PAIR_SHARED[mode] + 2.0f * (rest - 0.5f) * (PAIR_FULL[mode] - PAIR_SHARED[mode])
                                        : PAIR_IDLE[mode];
       const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE;
-      float t = (float)(wgs / SLOTS[mode]) * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
+      float t = (float)rounds * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += fixed + per * pair;
       t += ksplit == 1 ? (mode >= 2 ? 0.0f : REDO)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
