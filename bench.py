@@ -462,7 +462,7 @@ def main():
     t_pass = [t_pass[0], t_pass[1] + t_pass[2], t_pass[3]]
     pass_flops = [0.0, 4.0 * H * (DQK + DV) * pairs, 2.0 * H * DQK * pairs]
     pass_bytes = [8.0 * pairs, b_q + b_do + b_o + b_ds + b_rows, b_ds + b_dq + b_rows + S * DQK * 4.0]
-    kernels = [("mla_fwd_kernel", t_fwd, flops_fwd, b_q + b_o)]
+    kernels = [("mla_fwd_wide_kernel", t_fwd, flops_fwd, b_q + b_o)]
     kernels += [(pass_names[i], t_pass[i], pass_flops[i], pass_bytes[i]) for i in range(3)]
     name, t_dom, f_dom, b_dom = max(kernels, key=lambda k: k[1])
     traffic, traffic_note = None, "no counter profile committed for these kernel sources"
