@@ -1263,7 +1263,7 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // 0 of four ranges, 47 in mode 1 of two; 128 queries 100 and 82 (mode 1), 160 queries 100 and 148, 600 queries 334 and 392.  64 heads: 256 queries
 // 94 us in mode 3 and 83 in mode 1, 300 queries 123 and 140, 3000 817 and 900; 700 queries 215 and 224, with 65536 keys 281 and 251.
 // 32 heads: 257 queries 78 us in mode 4 and 112 in mode 2, 800 queries 175 and 236.  4000 queries of 128 heads: 256 slots 440 us in
-// mode 0 and 390 in mode 3, 640 slots 760 and 800.
+// mode 0 and 390 in mode 3, 640 slots 760 and 800 (150 queries x 256 slots 28.6 and 31.2).
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
 // mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
@@ -1278,6 +1278,8 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   float best_t = 1e30f;
   for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 5; mode++) {
     if (mode == (H > 32 ? 4 : 3)) continue;
+    // 128 heads: by the slots alone, so that blocks of queries have the bits of the whole; 96 fill two thirds of mode 3
+    if (H > 64 && mode == (H > 96 && K <= 256 ? 0 : 3)) continue;
     const int n_hg = (H + HEADS[mode] - 1) / HEADS[mode];
     for (int want = 1; want <= (may_split && mode < 3 ? 32 : 1) && want <= pairs; want++) {
       const int per = (pairs + want - 1) / want, ksplit = (pairs + per - 1) / per;
