@@ -257,6 +257,12 @@ int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int
                           int K, int q_start, float sm_scale, int d_v, void* out, float* lse,
                           void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
                           void* workspace, size_t workspace_bytes, void* stream);
+/*
+ * How the forward goes about a call of these sizes, for tests and measurements: the form (0: one workgroup in two wave roles
+ * for all heads, 1 / 2: 64 / 32 heads, two tiles at a time, 3 / 4: 64 / 32 heads, two workgroups on a compute unit), and in
+ * *ranges (may be NULL) over how many workgroups it spreads a query's slots.  -1 for sizes that the forward does not take.
+ */
+int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges);
 
 /*
  * Sparse MQA-MLA attention backward: dQ and dKV of dsa_sparse_mla_fwd given dO, the saved out and

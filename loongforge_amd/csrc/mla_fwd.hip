@@ -880,7 +880,9 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
   if (u >= S) return;
   const int qi = S - 1 - u;
   const int NT = K / BI;
-  const unsigned limit = (unsigned)min(a.Skv, a.q_start + qi + 1);       // valid ids are below
+  // valid ids are below: none for a query in front of the keys (a negative bound would be a huge one here), and no sum past INT_MAX
+  const int qpos = a.q_start + qi;
+  const unsigned limit = qpos < 0 ? 0u : (unsigned)min(a.Skv - 1, qpos) + 1u;
 
   unsigned char* const pbuf = smem + 2 * TILE_BYTES;
   unsigned* tmask = (unsigned*)(smem + HALF_LDS);
@@ -1391,6 +1393,13 @@ extern "C" size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int 
   (void)Skv;
   if (S <= 0 || H <= 0 || H % 32 || K <= 0 || K % 64) return 0;
   return part_bytes(plan_fwd(S, H, K, true), S, H);
+}
+
+extern "C" int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges) {
+  if (S <= 0 || H <= 0 || H > 128 || H % 32 || K <= 0 || K % 64 || K > 8192) return -1;
+  const FwdPlan p = plan_fwd(S, H, K, with_workspace != 0);
+  if (ranges) *ranges = p.ksplit;
+  return p.mode;
 }
 
 extern "C" int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,

@@ -2,6 +2,22 @@
 import torch
 
 
+# A small call for every form of the sparse-MLA forward: (form, slot ranges, queries, heads, slots); tests/test_boundary_cpu.py
+# checks that these sizes take the form they stand for
+MLA_FORMS = [(0, 1, 140, 128, 320), (0, 3, 70, 128, 2048), (1, 1, 130, 64, 320), (1, 4, 40, 64, 2048), (2, 1, 130, 32, 192),
+             (2, 8, 1, 128, 512), (3, 1, 300, 64, 192), (3, 1, 5, 128, 64), (4, 1, 260, 32, 128)]
+
+
+def mla_form(S, H, K, with_workspace=True):
+    """(form, slot ranges) of a forward call (dsa_sparse_mla_fwd_form)."""
+    import ctypes
+
+    from loongforge_amd import _lib
+
+    ranges = ctypes.c_int(0)
+    return _lib.load().dsa_sparse_mla_fwd_form(S, H, K, int(with_workspace), ctypes.addressof(ranges)), ranges.value
+
+
 def assert_close(got, ref, name, atol=2e-2, rtol=1e-2):
     """|got - ref| <= atol + rtol * |ref| for every element (the tolerance the path is specified
     with: max-abs 2e-2, relative 1e-2 against an fp32 reference)."""

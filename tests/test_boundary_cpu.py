@@ -50,6 +50,16 @@ def test_binding_arity_matches_header():
         assert n == len(argtypes), (name, n, len(argtypes))
 
 
+def test_forms_of_the_sparse_mla_forward():
+    """The sizes with which the GPU tests mean to reach every form of the forward do so."""
+    from tests.gpu_util import MLA_FORMS, mla_form
+
+    for form, ranges, S, H, K in MLA_FORMS:
+        assert mla_form(S, H, K) == (form, ranges), (S, H, K)
+    assert {f for f, _, _, _, _ in MLA_FORMS} == {0, 1, 2, 3, 4}
+    assert mla_form(4, 48, 64)[0] == mla_form(4, 64, 96)[0] == mla_form(4, 64, 16384)[0] == mla_form(0, 64, 64)[0] == -1
+
+
 def test_no_cpu_fallback():
     from loongforge_amd import ops
 

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from oracle import dsa_oracle as O
-from tests.gpu_util import assert_close, assert_mla_grads
+from tests.gpu_util import MLA_FORMS, assert_close, assert_mla_grads, mla_form
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +96,46 @@ def test_forward_invalid_ids_and_empty_rows(gpu):
     m = torch.isfinite(rl)
     assert (lse.cpu()[m] - rl[m]).abs().max().item() < 1e-4
     assert torch.equal(torch.isfinite(p.cpu()), torch.isfinite(rp))
+
+
+@pytest.mark.parametrize("form,ranges,S,H,K", MLA_FORMS)
+@pytest.mark.parametrize("end", ["before", "last"])
+def test_forward_at_the_ends_of_the_query_positions(gpu, form, ranges, S, H, K, end):
+    """Queries in front of the keys (a negative position: no valid slot, a zero row, lse = +inf), and positions up to the
+    largest int, in every form; with ids at and beyond the number of keys, and negative ones other than -1."""
+    from loongforge_amd import ops
+
+    assert mla_form(S, H, K) == (form, ranges)
+    skv, q_start = 90, -(S + 1) // 2 if end == "before" else 2 ** 31 - S
+    inp = O.make_mla_inputs(S, H, 64, seed=S + H, skv=skv, q_start=skv)
+    g = torch.Generator().manual_seed(K)
+    idx = torch.randint(0, skv, (S, K), generator=g).int()
+    for bad in (skv, skv + 1, 1 << 20, 2 ** 31 - 1, -1, -2, -77, -2 ** 31):
+        idx[torch.rand(idx.shape, generator=g) < 0.05] = bad
+    ro, rl, rp = O.sparse_mla_fwd(inp.q, inp.kv, idx, q_start, inp.sm_scale, 512)
+    assert torch.isinf(rl[: -q_start if end == "before" else 0]).all()
+    for dt in (None, torch.float32):
+        out, lse, p = ops.sparse_mla_fwd(inp.q.to(gpu), inp.kv.to(gpu), idx.to(gpu), q_start, inp.sm_scale, 512, dt is not None,
+                                         dt or torch.bfloat16)
+        assert_close(out, ro, "out")
+        fin = torch.isfinite(rl)
+        assert torch.equal(torch.isposinf(lse.cpu()), ~fin) and (out.cpu()[~fin] == 0).all()
+        assert not fin.any() or (lse.cpu() - rl)[fin].abs().max().item() < 1e-4
+        if dt is not None:
+            assert torch.equal(torch.isneginf(p.cpu()), torch.isneginf(rp))
+
+
+def test_backward_of_queries_in_front_of_the_keys(gpu):
+    """The backward has the same rule: their dQ is zero and they add nothing to dKV."""
+    from loongforge_amd import ops
+
+    inp = O.make_mla_inputs(100, 64, 64, seed=3, skv=70, q_start=70)
+    q_start = -41
+    q, kv, idx, do = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu)
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, q_start, inp.sm_scale)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, inp.sm_scale)
+    assert_mla_grads(dq, dkv, inp.q, inp.kv, inp.idx, inp.dout, q_start, inp.sm_scale, out=out, lse=lse)
+    assert (dq[:41] == 0).all()
 
 
 def test_forward_survives_a_late_dominant_key(gpu):
