@@ -69,6 +69,10 @@ constexpr float REDO_ABOVE = 64.0f, REDO_TERM = 0x1p64f;
 constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
 __device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
 
+// The reference point from a maximum (base 2).  It stays finite where that is -inf: relative to -inf a term would be
+// exp2(-inf + inf), while a row whose valid logits are all -inf has the sum 0, a zero output row and lse = +inf.
+__device__ __forceinline__ float reference_point(float mx) { return fmaxf(mx, -1e30f); }
+
 struct Final { float o_scale; float inv; float lse; };
 // Denominator, output factor and natural-log lse of a head from its reference point m (base 2) and sum l.
 // A sink logit is one more term exp(sink) in the denominator with no value row; the reference moves to
@@ -378,7 +382,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     // ---- softmax numerators (base 2), one head per lane -----------------------------------
     {
       const float mx = tile_max(sacc) * c2;
-      if (step == 0) m_ref = fmaxf(mx, -1e30f);       // (a masked-out tile has the maximum -inf)
+      if (step == 0) m_ref = reference_point(mx);     // (a masked-out tile has the maximum -inf)
       overflow |= (mx > m_ref + REDO_ABOVE);
     }
     bf16x8 pb[2];
@@ -626,7 +630,7 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
           *(uint4*)((unsigned short*)a.p_out + prow + 16 + 8 * g) = t[1];
         }
       }
-      if (n == 0) m_ref = tile_max(s_acc) * c2;
+      if (n == 0) m_ref = reference_point(tile_max(s_acc) * c2);
       bf16x8 pb[2];
       const float sum = softmax_numerators(s_acc, c2, m_ref, pb);
       l_run += sum;
@@ -1050,7 +1054,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
         __syncthreads();
         mx = fmaxf(mx, half_s[16 * (w ^ 2) + m]);
       }
-      m_ref = mx * c2;
+      m_ref = reference_point(mx * c2);
     }
     float sum = 0.f;
 #pragma unroll

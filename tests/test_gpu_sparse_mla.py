@@ -125,6 +125,37 @@ def test_forward_at_the_ends_of_the_query_positions(gpu, form, ranges, S, H, K, 
             assert torch.equal(torch.isneginf(p.cpu()), torch.isneginf(rp))
 
 
+@pytest.mark.parametrize("form,ranges,S,H,K", MLA_FORMS)
+def test_forward_of_logits_that_are_minus_infinity(gpu, form, ranges, S, H, K):
+    """Logits beyond the range of fp32 on the lower side count for nothing in every form: a row that has no others is like one
+    without a valid slot, and where they come first the others decide, in the same tile or a later one."""
+    from loongforge_amd import ops
+
+    assert mla_form(S, H, K) == (form, ranges)
+    skv = 2 * K
+    inp = O.make_mla_inputs(S, H, 64, seed=S + H, skv=skv, q_start=skv)
+    q, kv = inp.q.clone(), inp.kv.clone()
+    q[:, :, 0], kv[:, 0] = 0, 0
+    kv[:K, 0] = 8                                         # times -2^127: keys 0 .. K - 1 have a logit of -inf
+    idx = torch.stack([torch.randperm(K)[:K] + K for _ in range(S)]).int()
+    for i in range(S):                                    # none, all, those in front of a tile's middle, of all tiles but one, of half
+        idx[i, :[0, K, 16, K - 32, K // 2][(i + 1) % 5]] -= K
+        q[i, ::2 if i % 2 else 1, 0] = -2.0 ** 127        # odd rows: half of the heads
+    sink = torch.linspace(-2, 2, H)
+    for sk in (None, sink):
+        ro, rl, rp = O.sparse_mla_fwd(q, kv, idx, skv, inp.sm_scale, 512, attn_sink=sk)
+        assert torch.isneginf(rp).any() and not torch.isnan(ro).any()
+        for dt in (None, torch.float32):
+            out, lse, p = ops.sparse_mla_fwd(q.to(gpu), kv.to(gpu), idx.to(gpu), skv, inp.sm_scale, 512, dt is not None,
+                                             dt or torch.bfloat16, attn_sink=None if sk is None else sk.to(gpu))
+            assert_close(out, ro, "out")
+            fin = torch.isfinite(rl)
+            assert torch.equal(torch.isposinf(lse.cpu()), ~fin) and (out.cpu()[~fin] == 0).all()
+            assert not fin.any() or (lse.cpu() - rl)[fin].abs().max().item() < 1e-4
+            if dt is not None:
+                assert torch.equal(torch.isneginf(p.cpu()), torch.isneginf(rp))
+
+
 def test_backward_of_queries_in_front_of_the_keys(gpu):
     """The backward has the same rule: their dQ is zero and they add nothing to dKV."""
     from loongforge_amd import ops
