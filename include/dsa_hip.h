@@ -258,6 +258,16 @@ int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int
                           void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
                           void* workspace, size_t workspace_bytes, void* stream);
 /*
+ * The same for a block of S queries of a call of S_all: those rows of its results (out, lse, p_out), bit for bit.  The last bits
+ * of a query depend on how the work is shared out, and that on the number of queries; here S_all decides, and as of
+ * dsa_sparse_mla_fwd_ws it does so with a workspace of the size that the call of S_all, or a block of it, can use.
+ */
+size_t dsa_sparse_mla_fwd_block_workspace_bytes(int S_all, int S, int H, int Skv, int K);
+int dsa_sparse_mla_fwd_block(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv,
+                             int K, int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
+                             int p_out_f32, const float* attn_sink, int p_out_skip,
+                             void* workspace, size_t workspace_bytes, void* stream);
+/*
  * How the forward goes about a call of these sizes, for tests and measurements: the form (0: one workgroup in two wave roles
  * for all heads, 1 / 2: 64 / 32 heads, two tiles at a time, 3 / 4: 64 / 32 heads, two workgroups on a compute unit), and in
  * *ranges (may be NULL) over how many workgroups it spreads a query's slots.  -1 for sizes that the forward does not take.

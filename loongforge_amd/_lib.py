@@ -40,6 +40,8 @@ SIGNATURES = {
     "dsa_sparse_mla_fwd": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp]),
     "dsa_sparse_mla_fwd_ex": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _i, _vp]),
     "dsa_sparse_mla_fwd_workspace_bytes": (_sz, [_i, _i, _i, _i]),
+    "dsa_sparse_mla_fwd_block_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "dsa_sparse_mla_fwd_block": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _sz, _vp]),
     "dsa_sparse_mla_fwd_form": (_i, [_i, _i, _i, _i, _vp]),
     "dsa_sparse_mla_fwd_ws": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _sz, _vp]),
     "dsa_sparse_mla_bwd_workspace_bytes": (_sz, [_i, _i, _i, _i]),

@@ -1295,7 +1295,7 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
   float best_t = 1e30f;
   for (int mode = H > 64 ? 0 : H > 32 ? 1 : 2; mode < 5; mode++) {
     if (mode == (H > 32 ? 4 : 3)) continue;
-    // 128 heads: by the slots alone, so that blocks of queries have the bits of the whole; 96 fill two thirds of mode 3
+    // 128 heads: mode 3 up to 256 slots, mode 0 from there on; 96 fill two thirds of mode 3
     if (H > 64 && mode == (H > 96 && K <= 256 ? 0 : 3)) continue;
     const int n_hg = (H + HEADS[mode] - 1) / HEADS[mode];
     for (int want = 1; want <= (may_split && mode < 3 ? 32 : 1) && want <= pairs; want++) {
@@ -1331,7 +1331,7 @@ constexpr auto fwd_kernel() {
 }
 
 template <int MODE, bool SPLIT>
-int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
+int launch_fwd(const FwdArgs& a, int p_out_f32, bool shared, hipStream_t st) {
   const size_t smem = MODE == 0   ? WIDE_LDS + ids_lds_bytes(a.k_loc)
                       : MODE >= 3 ? HALF_LDS + mask_lds_bytes(a.k_loc)
                                   : 4 * TILE_BYTES + ids_lds_bytes(a.k_loc);
@@ -1348,7 +1348,6 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   else DSA_FWD_LAUNCH(2);
 #undef DSA_FWD_LAUNCH
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
-  const bool shared = combine_shares(a.S, a.H, a.ksplit);
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
   if (MODE >= 2 && !SPLIT) return 0;
   if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
@@ -1357,11 +1356,14 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, hipStream_t st) {
   return 0;
 }
 
-int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K, int q_start, float sm_scale,
+// S_all: the queries of the call of which these S are a block (S where it is the whole).  They, not S, choose the form, the ranges
+// and the way the ranges' sums are put together, so a query has the same bits in a block of any size.
+int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv, int K, int q_start, float sm_scale,
              int d_v, void* out, float* lse, void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
              void* workspace, size_t workspace_bytes, void* stream) {
   DSA_REQUIRE(d_v == DV, "dsa_sparse_mla_fwd: only d_v = 512 (d_qk = 576) is supported, got d_v = %d", d_v);
   DSA_REQUIRE(S >= 0 && Skv > 0, "dsa_sparse_mla_fwd: bad sequence sizes S=%d Skv=%d", S, Skv);
+  DSA_REQUIRE(S_all >= S, "dsa_sparse_mla_fwd: a block of %d queries of %d", S, S_all);
   DSA_REQUIRE(H > 0 && H <= 128 && H % 32 == 0, "dsa_sparse_mla_fwd: head count must be 32, 64, 96 or 128, got %d", H);
   DSA_REQUIRE(K > 0 && K % 64 == 0, "dsa_sparse_mla_fwd: top-k must be a positive multiple of 64, got %d", K);
   DSA_REQUIRE(p_out_skip >= 0 && p_out_skip < K && p_out_skip % BI == 0,
@@ -1373,18 +1375,18 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, in
   DSA_REQUIRE(K <= 8192, "dsa_sparse_mla_fwd: top-k %d exceeds the supported maximum 8192", K);
   if (S == 0) return DSA_OK;
   hipStream_t st = (hipStream_t)stream;
-  FwdPlan p = plan_fwd(S, H, K, true);
-  if (part_bytes(p, S, H) > workspace_bytes || (p.ksplit > 1 && workspace == nullptr)) p = plan_fwd(S, H, K, false);
+  FwdPlan p = plan_fwd(S_all, H, K, true);
+  if (part_bytes(p, S, H) > workspace_bytes || (p.ksplit > 1 && workspace == nullptr)) p = plan_fwd(S_all, H, K, false);
   FwdArgs a{(const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, attn_sink,
             p_out ? p_out_skip : 0, p.n_hg, p.ksplit, p.k_loc, (f32x4*)workspace,
             (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4)};
   int rc;
-  const bool split = p.ksplit > 1;
-  if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, st) : launch_fwd<0, false>(a, p_out_f32, st);
-  else if (p.mode == 3) rc = launch_fwd<3, false>(a, p_out_f32, st);
-  else if (p.mode == 4) rc = launch_fwd<4, false>(a, p_out_f32, st);
-  else if (p.mode == 1) rc = split ? launch_fwd<1, true>(a, p_out_f32, st) : launch_fwd<1, false>(a, p_out_f32, st);
-  else rc = split ? launch_fwd<2, true>(a, p_out_f32, st) : launch_fwd<2, false>(a, p_out_f32, st);
+  const bool split = p.ksplit > 1, shared = combine_shares(S_all, H, p.ksplit);
+  if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, shared, st) : launch_fwd<0, false>(a, p_out_f32, shared, st);
+  else if (p.mode == 3) rc = launch_fwd<3, false>(a, p_out_f32, shared, st);
+  else if (p.mode == 4) rc = launch_fwd<4, false>(a, p_out_f32, shared, st);
+  else if (p.mode == 1) rc = split ? launch_fwd<1, true>(a, p_out_f32, shared, st) : launch_fwd<1, false>(a, p_out_f32, shared, st);
+  else rc = split ? launch_fwd<2, true>(a, p_out_f32, shared, st) : launch_fwd<2, false>(a, p_out_f32, shared, st);
   DSA_REQUIRE(rc != -1, "dsa_sparse_mla_fwd: top-k %d does not fit LDS", K);
   if (rc == -2) DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_fwd: cannot reserve LDS");
   DSA_CHECK_LAUNCH("dsa_sparse_mla_fwd");
@@ -1393,10 +1395,14 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S, int H, in
 
 }  // namespace
 
-extern "C" size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int K) {
+extern "C" size_t dsa_sparse_mla_fwd_block_workspace_bytes(int S_all, int S, int H, int Skv, int K) {
   (void)Skv;
-  if (S <= 0 || H <= 0 || H % 32 || K <= 0 || K % 64) return 0;
-  return part_bytes(plan_fwd(S, H, K, true), S, H);
+  if (S <= 0 || S_all < S || H <= 0 || H % 32 || K <= 0 || K % 64) return 0;
+  return part_bytes(plan_fwd(S_all, H, K, true), S, H);
+}
+
+extern "C" size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int K) {
+  return dsa_sparse_mla_fwd_block_workspace_bytes(S, S, H, Skv, K);
 }
 
 extern "C" int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges) {
@@ -1406,23 +1412,31 @@ extern "C" int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, 
   return p.mode;
 }
 
+extern "C" int dsa_sparse_mla_fwd_block(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv, int K,
+                                        int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
+                                        int p_out_f32, const float* attn_sink, int p_out_skip, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+  return fwd_impl(q, kv, ids, S_all, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
+                  workspace, workspace_bytes, stream);
+}
+
 extern "C" int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
                                      int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
                                      int p_out_f32, const float* attn_sink, int p_out_skip, void* workspace,
                                      size_t workspace_bytes, void* stream) {
-  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
+  return fwd_impl(q, kv, ids, S, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
                   workspace, workspace_bytes, stream);
 }
 
 extern "C" int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
                                      int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
                                      int p_out_f32, const float* attn_sink, int p_out_skip, void* stream) {
-  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
+  return fwd_impl(q, kv, ids, S, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
                   nullptr, 0, stream);
 }
 
 extern "C" int dsa_sparse_mla_fwd(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,
                                   int q_start, float sm_scale, int d_v, void* out, float* lse, void* p_out,
                                   int p_out_f32, void* stream) {
-  return fwd_impl(q, kv, ids, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, nullptr, 0, nullptr, 0, stream);
+  return fwd_impl(q, kv, ids, S, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, nullptr, 0, nullptr, 0, stream);
 }

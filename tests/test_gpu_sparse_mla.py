@@ -581,6 +581,32 @@ def test_attn_dist_from_q_kv_lse_matches_oracle_and_the_logits_path(gpu, S, H, K
     assert ((got.sum(-1) - 1.0).abs() <= 1e-4).all() and (got[5, 3] == 0).all()
 
 
+@pytest.mark.parametrize("S,H,K,block", [
+    (300, 64, 192, 100),              # the whole: two workgroups to a unit; a block by itself would share its queries' heads out
+    (300, 64, 192, 256),              # the last block of 44 alone
+    (300, 32, 128, 200),
+    (200, 128, 256, 64),
+    (140, 128, 320, 96),              # two roles; blocks of 96 and 44
+    (40, 64, 2048, 16),               # in four ranges of slots; a block alone in eight
+    (20, 32, 2048, 9),                # the same, and the ranges' sums of few queries are put together another way
+    (10, 128, 512, 3),                # one workgroup for a query's slots; a block alone in ranges
+])
+def test_forward_with_distribution_in_blocks_is_that_of_the_whole(gpu, S, H, K, block):
+    from loongforge_amd import ops
+
+    heads = H - 5
+    q_start = K + 50
+    inp = O.make_mla_inputs(S, H, K, seed=S + H, q_start=q_start)
+    q, kv, ids, sink = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), torch.linspace(-2, 2, H).to(gpu)
+    assert any(mla_form(n, H, K) != mla_form(S, H, K) for n in (block, S % block))          # by themselves
+    for sk in (None, sink):
+        out, lse, p_out = ops.sparse_mla_fwd(q, kv, ids, q_start, inp.sm_scale, 512, True, attn_sink=sk)
+        want = out, lse, ops.attn_dist(p_out[:, :heads], inp.sm_scale)
+        for n in (block, S):
+            got = ops.sparse_mla_fwd_dist(q, kv, ids, q_start, inp.sm_scale, 512, heads, n, sk)
+            assert all(torch.equal(g, w) for g, w in zip(got, want)), n
+
+
 def test_attn_dist_from_q_kv_lse_with_sink_is_the_softmax_over_the_slots(gpu):
     from loongforge_amd import ops
 
