@@ -240,7 +240,7 @@ def main():
     dq, dkv = torch.empty_like(q), torch.empty_like(kv)
     out = torch.empty(S, H, DV, dtype=torch.bfloat16, device=dev)
     lse = torch.empty(S, H, dtype=torch.float32, device=dev)
-    pass_ms = (ctypes.c_float * 5)()
+    pass_ms = (ctypes.c_float * 3)()
     q8 = torch.empty(S, HI, 128, dtype=torch.uint8, device=dev)
     k8 = torch.empty(S, 128, dtype=torch.uint8, device=dev)
     qs = torch.empty(S, HI, dtype=torch.float32, device=dev)
@@ -272,7 +272,7 @@ def main():
     torch.cuda.synchronize()
 
     t_idx = t_fwd = t_bwd = 0.0
-    t_pass = [0.0] * 5           # launch groups of the backward: order, passes A and C (one launch, then [2] is 0), passes B | D
+    t_pass = [0.0] * 3           # launch groups of the backward: order; P, dS and rows; dQ | dKV
     t_logits = t_topk = 0.0
     wall = 0.0
     for step in range(args.warmup + args.steps):
@@ -310,7 +310,7 @@ def main():
                                                    dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), wsb, stream, pass_ms),
                    "bwd", blib)
         torch.cuda.synchronize()
-        for i in range(5):
+        for i in range(3):
             t_pass[i] += pass_ms[i]
     t_pass = [x / n_prof for x in t_pass]
     # the indexer part alone, twenty replays in a row: inside a step it starts on caches and clocks the backward
@@ -459,7 +459,6 @@ def main():
     b_rows = 1152.0 * pairs                   # one bf16 row of 576 per pair
     b_dq, b_dkv = nq * H * DQK * 2, float(S) * DQK * 2
     pass_names = ["order", "bwd_pds_rows_kernel (S, dP -> dS, dKV rows)", "bwd_dq_reduce_kernel (dQ beside the ordered dKV sum)"]
-    t_pass = [t_pass[0], t_pass[1] + t_pass[2], t_pass[3]]
     pass_flops = [0.0, 4.0 * H * (DQK + DV) * pairs, 2.0 * H * DQK * pairs]
     pass_bytes = [8.0 * pairs, b_q + b_do + b_o + b_ds + b_rows, b_ds + b_dq + b_rows + S * DQK * 4.0]
     kernels = [("mla_fwd_wide_kernel", t_fwd, flops_fwd, b_q + b_o)]

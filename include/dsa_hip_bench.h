@@ -16,8 +16,7 @@ extern "C" {
 /*
  * Profiling variant of dsa_sparse_mla_bwd: same arguments and results, plus the time of each launch
  * group in milliseconds, measured with HIP events on `stream` and summed over query chunks:
- *   pass_ms[0] key-sorted order   [1] P and dS, from 64 heads on with the per-pair dKV rows   [2] the rows where they are a launch
- *   of their own   [3] dQ beside the ordered dKV reduce   [4] 0
+ *   pass_ms[0] key-sorted order   [1] P, dS and the per-pair dKV rows   [2] dQ beside the ordered dKV reduce
  * It creates and destroys HIP events and waits for the stream before returning, so it is for
  * benchmarks only.  No counterpart in the reference (its kernels are timed with do_bench from
  * Python, ops/tilelang_ops/sparse_mla_bwd.py:359-368).

@@ -6,14 +6,13 @@
 // (295 KB) do not fit one compute unit (512 KB of registers, 160 KB of LDS) next to the gathered key
 // tiles, and the products over d and over heads need the same operands in two orientations.  The work
 // is therefore split into passes:
-//   pass A  S and dP per 32-key tile -> P and dS; dS goes to HBM as bf16 for pass B, 8 KB per query and tile
-//   pass B  dQ^T += KV^T.dS^T, both operands by LDS transpose reads
-//   pass C  per-pair rows  dS^T.Q + P^T.dO  (sum over all heads) -> one bf16 row of 576 values in a pair
-//           buffer, at the position given by a key-sorted order
-//   pass D  dKV[key] = sum of that key's rows, in ascending query order
-// Passes A and C are one kernel (bwd_pds_rows_kernel) that keeps both orientations and P on the compute unit, passes B and D
-// share a launch (bwd_dq_reduce_kernel).
-// The key-sorted order (pass 0) comes from a bitmap key x query, its row-wise prefix popcounts and
+//   P, dS, rows  (bwd_pds_rows_kernel)  S and dP per 32-key tile -> P and dS; the tile's pair rows dS^T.Q + P^T.dO (sum over all
+//                heads) -> one bf16 row of 576 values in a pair buffer, at the position given by a key-sorted order.  Both
+//                orientations of Q and dO and P stay on the compute unit; dS goes to HBM as bf16, 2 KB per 32 heads and tile
+//   dQ           dQ^T += KV^T.dS^T, both operands by LDS transpose reads
+//   dKV          dKV[key] = sum of that key's rows, in ascending query order
+// The last two share a launch (bwd_dq_reduce_kernel).
+// The key-sorted order comes from a bitmap key x query, its row-wise prefix popcounts and
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
 #include "mla_tile.h"
@@ -22,7 +21,7 @@
 namespace {
 using namespace mla;
 
-// P or dS of one (query, tile): [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes are
+// dS of one (query, tile) in memory, P and dS of a tile in LDS: [4 HG chunk groups][32 keys][8 heads] bf16.  HG is the number of 32-head groups the passes are
 // compiled for: 1 or 2, or 4 for 96 and 128 heads.
 constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
@@ -30,11 +29,11 @@ constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
 
 // ---------------------------------------------------------------------------------------------
-// pass B: dQ
+// dQ
 // ---------------------------------------------------------------------------------------------
 // dQ^T[d, head] += KV^T[d, key] . dS^T[key, head] per 32-key tile.  Both operands are LDS transpose
-// reads: of the gathered key tile (18 d-tiles) and of the tile's dS block copied verbatim from the
-// pass-A buffer.  Twelve waves share the 72 accumulator tiles (18 d-tiles x 4 head groups): wave
+// reads: of the gathered key tile (18 d-tiles) and of the tile's dS block copied verbatim from
+// memory.  Twelve waves share the 72 accumulator tiles (18 d-tiles x 4 head groups): wave
 // (dg, hp) = (wave % 6, wave / 6) owns d-tiles 3dg .. 3dg+2 for the head groups 2hp, 2hp+1: 6 tiles
 // (96 accumulator registers), 12 MFMAs and 20 transposing reads per wave and tile.  A wave issues one
 // LDS instruction per 40-odd cycles whatever its width, and a transposing read carries 8 bytes per
@@ -214,12 +213,13 @@ __device__ __forceinline__ void dq_body(
 }
 
 // ---------------------------------------------------------------------------------------------
-// passes A and C in one, for 32 and 64 heads
+// P, dS and the rows of the pairs, for 32 and 64 heads
 // ---------------------------------------------------------------------------------------------
 // Q and dO of 64 heads fit the registers of a compute unit in both orientations: 136 per lane for the products over d (wave
 // (hw, hh) = (wave % 4, wave / 4): 16 heads, the 16 keys of half tile hh) and 64 for those over the heads (wave w: the columns
 // 64 w .. 64 w + 63 of both; 16 columns of the rotary part come from LDS).  So P never leaves the compute unit, dS is written for
-// pass B only, and a pair costs 1152 + 128 bytes of writes where the two passes wrote 1152 + 256 and read 256.
+// the dQ products only, and a pair costs 1152 + 128 bytes of writes where two kernels with P and dS in memory between them wrote
+// 1152 + 256 and read 256.
 // Between two barriers a wave works on S, dP of tile n and on the rows of tile n - 1, whose P and dS all waves have put into
 // LDS (two buffers) before the barrier; waves 0-3 take them in this order, waves 4-7 in the other one, so that the two waves
 // of a SIMD issue stores and exponentials under each other's MFMAs.  The transfers of tile n + 2 come first in a step: between
@@ -355,7 +355,7 @@ __device__ __forceinline__ void pds_rows_body(
     for (int ks = 0; ks < HG; ks++) xr_s[64 * ks] = xr[ks];
   }
 
-  // transfers of a tile, as in pass A: waves 0-3 take groups 0-4, waves 4-7 groups 5-8
+  // transfers of a tile: waves 0-3 take groups 0-4, waves 4-7 groups 5-8
   const int gkey = (tid & 255) >> 3, gsub = tid & 7;
   const int grp0 = hh * 5;
   const unsigned gslot = (unsigned)((gsub ^ (gkey & 7)) * 16) + (unsigned)(grp0 * 128);
@@ -492,7 +492,7 @@ __device__ __forceinline__ void pds_rows_body(
 }
 
 // ---------------------------------------------------------------------------------------------
-// passes A and C in one, for 96 and 128 heads
+// P, dS and the rows of the pairs, for 96 and 128 heads
 // ---------------------------------------------------------------------------------------------
 // Both orientations of 128 heads are 557 KB; registers (512 KB) and LDS (160 KB) hold them together with the tile because what
 // lies in LDS serves either orientation: row reads for the products over d, transposing reads for those over the heads.  In LDS:
@@ -732,7 +732,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
       pw[kt][0] = cvt_pk_bf16(pf[0], pf[1]); pw[kt][1] = cvt_pk_bf16(pf[2], pf[3]);
       dw[kt][0] = cvt_pk_bf16(df[0], df[1]); dw[kt][1] = cvt_pk_bf16(df[2], df[3]);
     }
-    // lanes 32 apart trade half tiles, as in pass A
+    // lanes 32 apart trade half tiles: 16 bytes of a key's heads for a lane
 #pragma unroll
     for (int r2 = 0; r2 < 2; r2++) {
       swap_halves(pw[0][r2], pw[1][r2]);
@@ -811,7 +811,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
 }
 
 // ---------------------------------------------------------------------------------------------
-// pass D: dKV[key] = sum of that key's rows, ascending query order
+// dKV[key] = sum of that key's rows, ascending query order
 // ---------------------------------------------------------------------------------------------
 // One key per workgroup (504 of its threads): 72 column chunks of 8 elements x 7 row groups (row r of the
 // segment goes to group r % 7); the seven partial sums are combined in a fixed order, so the result
@@ -897,11 +897,11 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
 // ---------------------------------------------------------------------------------------------
 // kernels: two roles each, chosen per workgroup
 // ---------------------------------------------------------------------------------------------
-// Pass B is bound by LDS reads and leaves HBM nearly idle; pass D is a pure stream of HBM reads and
-// leaves everything else idle; each occupies a whole compute unit (140 KB of LDS, or all its
+// The dQ products are bound by LDS reads and leave HBM nearly idle; the sums are a pure stream of HBM reads and
+// leave everything else idle; each occupies a whole compute unit (140 KB of LDS, or all its
 // memory-level parallelism).  One launch carries the workgroups of both, spread evenly over the
 // dispatch order, so that both kinds of work are in flight from the first workgroup to the last:
-//   bwd_dq_reduce_kernel   pass B of all queries | pass D of all keys      (4.5 ms against 2.6 + 2.75)
+//   bwd_dq_reduce_kernel   dQ of all queries | dKV of all keys      (4.5 ms against 2.6 + 2.75)
 // Within a role, the longest work (latest query, earliest key) comes first.
 struct RoleSlot { bool first; int i; };
 // nX workgroups of the first role and nY of the second, spread evenly over the launch: workgroup b belongs to the
@@ -1052,22 +1052,22 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
 
   const int HG = head_groups(H);
   const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
-  size_t smemB = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
-  if (smemB < reduce_lds) smemB = reduce_lds;
+  size_t smem_dq = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
+  if (smem_dq < reduce_lds) smem_dq = reduce_lds;
   auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
   auto pds_rows_kernel = HG == 1 ? bwd_pds_rows_kernel<1> : HG == 2 ? bwd_pds_rows_kernel<2> : bwd_pds_rows_kernel<4>;
-  const size_t smemAC = HG <= 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
-  if (dsa_reserve_lds((const void*)pds_rows_kernel, smemAC) != hipSuccess ||
-      dsa_reserve_lds((const void*)dq_reduce_kernel, smemB) != hipSuccess)
+  const size_t smem_rows = HG <= 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
+  if (dsa_reserve_lds((const void*)pds_rows_kernel, smem_rows) != hipSuccess ||
+      dsa_reserve_lds((const void*)dq_reduce_kernel, smem_dq) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
 
   // optional timing (profiling entry point only): events between the launch groups
-  hipEvent_t ev[5];
+  hipEvent_t ev[4];
   if (pass_ms) {
-    for (int i = 0; i < 5; i++) pass_ms[i] = 0.f;
+    for (int i = 0; i < 3; i++) pass_ms[i] = 0.f;
     int made = 0;
-    for (; made < 5; made++) if (hipEventCreate(&ev[made]) != hipSuccess) break;
-    if (made < 5) {
+    for (; made < 4; made++) if (hipEventCreate(&ev[made]) != hipSuccess) break;
+    if (made < 4) {
       for (int i = 0; i < made; i++) hipEventDestroy(ev[i]);
       DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd_profile: cannot create events");
     }
@@ -1088,21 +1088,20 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
-    pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smemAC, st>>>(
+    pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smem_rows, st>>>(
         (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, H, Skv, K, q_start,
         sm_scale, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
-    DSA_MARK(3);
-    // Pass B of every query beside pass D of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smemB, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
+    // dQ of every query beside the sums of every key.
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
                                                                    K, q_start, dup_flag, rows, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");
-    DSA_MARK(4);
+    DSA_MARK(3);
     if (pass_ms) {
-      hipEventSynchronize(ev[4]);
-      for (int i = 0; i < 4; i++) { float ms = 0.f; hipEventElapsedTime(&ms, ev[i], ev[i + 1]); pass_ms[i] += ms; }
+      hipEventSynchronize(ev[3]);
+      for (int i = 0; i < 3; i++) { float ms = 0.f; hipEventElapsedTime(&ms, ev[i], ev[i + 1]); pass_ms[i] += ms; }
     }
     first = false;
   }
@@ -1113,7 +1112,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   if (S > p.chunk)      // more than one chunk: the flag may have come up after earlier chunks wrote their dQ
     poison_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>((unsigned short*)dq, (size_t)S * H * DQK, dup_flag);
   DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(cast)");
-  if (pass_ms) for (int i = 0; i < 5; i++) hipEventDestroy(ev[i]);
+  if (pass_ms) for (int i = 0; i < 4; i++) hipEventDestroy(ev[i]);
 #undef DSA_MARK
   return DSA_OK;
 }
@@ -1130,7 +1129,7 @@ extern "C" int dsa_sparse_mla_bwd_profile(const void* q, const void* kv, const v
                                           const int32_t* ids, const float* lse, int S, int H, int Skv, int K, int q_start,
                                           float sm_scale, int d_v, void* dq, void* dkv, void* workspace,
                                           size_t workspace_bytes, void* stream, float* pass_ms) {
-  DSA_REQUIRE(pass_ms != nullptr, "dsa_sparse_mla_bwd_profile: pass_ms must point at 5 floats");
+  DSA_REQUIRE(pass_ms != nullptr, "dsa_sparse_mla_bwd_profile: pass_ms must point at 3 floats");
   return bwd_impl(q, kv, out, dout, ids, lse, S, H, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
                   stream, pass_ms);
 }
