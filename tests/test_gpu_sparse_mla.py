@@ -30,7 +30,7 @@ def test_forward_against_oracle(gpu, S, H, K, q_start, skv, seed):
 
 @pytest.mark.parametrize("K", [4096, 8192])
 def test_top_k_beyond_2048(gpu, K):
-    """Wider slot lists: the forward runs them with a three-stage tile ring; the backward and the recomputed attention
+    """Wider slot lists: the forward of a few queries shares them out in ranges; the backward and the recomputed attention
     distribution take 2048 / 4096 slots per call and the host walks the list in parts (the gradients are sums over the
     slots once lse and out of the whole list are given)."""
     from loongforge_amd import ops
@@ -188,8 +188,10 @@ def test_forward_survives_a_late_dominant_key(gpu):
     (3, 64, 320, 500, 700),           # five pairs of tiles per query
     (5, 96, 192, 300, None),          # the last 64-head workgroup holds 32 heads
     (2, 32, 128, 400, None),
-    (300, 64, 192, 0, None),          # two tiles at a time without ranges, odd tile counts in the early rows
+    (300, 64, 192, 0, None),          # two workgroups on a unit, odd tile counts in the early rows
     (300, 32, 256, 0, None),
+    (140, 64, 320, 0, None),          # two tiles at a time without ranges, odd tile counts in the early rows
+    (140, 32, 256, 0, None),
     (2, 128, 4096, 5000, None),       # ranges that fit the two-tile ring though the whole list does not
 ])
 def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
@@ -233,7 +235,9 @@ def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
     (260, 128, 192, 0, None),         # up to six tiles, fewer than the ring in the early rows; a second round of workgroups
     (170, 96, 320, 400, 500),         # the fourth 32-head block is not there
     (300, 128, 768, 0, None),         # from one tile in the early rows to 24
-    (48, 96, 2048, 3000, None),       # in ranges of slots
+    (48, 96, 2048, 3000, None),       # in ranges of slots, by 64 heads
+    (88, 96, 2048, 3000, None),       # in ranges, in two roles
+    (70, 128, 2048, 0, 2100),         # the same; ranges without a tile in the early rows
 ])
 def test_forward_of_many_heads(gpu, S, H, K, q_start, skv):
     """The two-role kernel, and the one for a pair of tiles, at the edges of their rings and heads; slot lists and bounds as above."""
@@ -262,6 +266,57 @@ def test_forward_two_workgroups_to_a_unit(gpu, S, K, q_start, skv, H):
         p16, p32 = (ops.sparse_mla_fwd(inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), q_start, inp.sm_scale, 512, True, dt, p_out_skip=skip)[2]
                     for dt in (torch.bfloat16, torch.float32))
         assert p32.shape[2] == K - skip and torch.equal(p16, p32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("form,ranges,S,H,K", [
+    (3, 1, 270, 64, 2112),            # more slots than one sweep of the masks takes, more tiles than a wave has lanes
+    (4, 1, 258, 32, 2112),
+    (3, 1, 350, 64, 8192),            # the longest list, which a block done again holds beside a tile
+    (4, 1, 258, 32, 8192),
+    (0, 1, 130, 128, 4096),
+    (0, 5, 45, 128, 4096),
+    (0, 2, 90, 96, 8192),
+])
+def test_forward_of_long_lists_in_every_form_for_many_queries(gpu, form, ranges, S, H, K):
+    """The forms that own a query's slots with lists of more than 2048, in some of the rows: holes, tiles without a valid slot, an
+    empty row, causal bounds, sinks, logits, and for one row a key in the last slot that beats all others by far more than 2^64."""
+    from loongforge_amd import ops
+
+    assert mla_form(S, H, K) == (form, ranges)
+    skv = K + 900
+    q_start = skv - S // 2                                # half of the queries have keys behind them
+    g = torch.Generator().manual_seed(S + K)
+    q = torch.randn(S, H, 576, generator=g).to(torch.bfloat16)
+    kv = torch.randn(skv, 576, generator=g).to(torch.bfloat16)
+    idx = torch.stack([torch.randperm(skv, generator=g)[:K] for _ in range(S)]).int()
+    idx[torch.rand(idx.shape, generator=g) < 0.3] = -1
+    idx[1, 32:K - 64] = -1                                # the first tile and the last two
+    idx[2] = -1
+    idx[S - 2, :2080] = -1
+    idx[: S - 2][idx[: S - 2] == skv - 1] = -1
+    idx[S - 3, K - 1] = skv - 1
+    kv[skv - 1] = (q[S - 3, H - 1].float() * 40.0).to(torch.bfloat16)
+    rows = [0, 1, 2, 3, S // 2, S - 3, S - 2, S - 1]
+    sink = torch.linspace(-2, 2, H)
+    for sk in (None, sink):
+        ref = [O.sparse_mla_fwd(q[i:i + 1], kv, idx[i:i + 1], q_start + i, 192 ** -0.5, 512, attn_sink=sk) for i in rows]
+        ro, rl, rp = (torch.cat(x) for x in zip(*ref))
+        for dt in (None, torch.bfloat16, torch.float32):
+            out, lse, p = ops.sparse_mla_fwd(q.to(gpu), kv.to(gpu), idx.to(gpu), q_start, 192 ** -0.5, 512, dt is not None,
+                                             dt or torch.bfloat16, attn_sink=None if sk is None else sk.to(gpu))
+            assert_close(out[rows], ro, "out", atol=4e-2)
+            lse, fin = lse[rows].cpu(), torch.isfinite(rl)
+            assert torch.equal(torch.isposinf(lse), ~fin)
+            assert ((lse - rl)[fin].abs() / rl[fin].abs().clamp_min(1)).max().item() < 1e-3
+            assert torch.isfinite(out.float()).all()
+            if dt is not None:
+                p = p[rows].cpu()
+                assert torch.equal(torch.isfinite(p), torch.isfinite(rp))
+            if dt == torch.bfloat16:
+                p16 = p
+            if dt == torch.float32:
+                assert ((p - rp)[torch.isfinite(rp)].abs() / rp[torch.isfinite(rp)].abs().clamp_min(1)).max().item() < 1e-3
+                assert torch.equal(p.to(torch.bfloat16), p16)
 
 
 def test_forward_slot_permutation_invariance(gpu):
