@@ -13,8 +13,9 @@
 // MFMA-bound: 2*H*(576+512) flop per (query, key) pair against 1152 gathered bytes.
 //
 // How a workgroup shares a query's heads and slots is the MODE:
-//   0  128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
-//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel<2>; with one pair of tiles any heads.
+//   0  96 or 128 heads, one tile at a time: mla_fwd_wide_kernel, eight waves of up to 256 registers in two roles.
+//   3  64 heads, one tile at a time, two workgroups on a compute unit: mla_fwd_half_kernel<2>; 128 heads with up to
+//      256 slots as two groups of heads, and any heads with one pair of tiles.
 //   4  32 heads, likewise: mla_fwd_half_kernel<1>.
 //   1  64 heads, two tiles at a time: waves (stream, b) = (w / 2, w % 2) own heads [32b, 32b + 32)
 //      of every other tile; the two streams' sums are merged through LDS at the end.
@@ -1276,9 +1277,13 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // together, and the gathers of 256 workgroups share the fabric.  A single or last round, LAST: IDLE on an empty chip, and nearly that
 // while it is half empty, hence the square.  Modes 3 and 4 by whether workgroups share a compute unit; where few do, what they take
 // with keys that lie far apart.
-// 2048 slots, 128 heads: one query 86 us in mode 0 and 15 as 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0, 50 in mode
-// 0 of four ranges, 47 in mode 1 of two; 128 queries 100 and 82 (mode 1), 160 queries 100 and 148, 600 queries 334 and 392.  64 heads: 256 queries
-// 94 us in mode 3 and 83 in mode 1, 300 queries 123 and 140, 3000 817 and 900; 700 queries 215 and 224, with 65536 keys 281 and 251.
+// 2048 slots, 128 heads: one query 86 us in mode 0 and 15 as 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0 and
+// 47 in mode 1 of two ranges; 128 queries 100 and 82 (mode 1), 160 queries 100 and 148, 600 queries 334 and 392.  64 heads: 256 queries
+// 94 us in mode 3 and 83 in mode 1, 300 queries 123 and 140, 3000 817 and 900; 513 - 738 queries, one
+// round of mode 3's 512 places and a short second one, are as fast in mode 1 (600 queries 218 and 216, with 65536 keys 243 and 256) and take it.
+// Mode 0 in ranges: up to 2048 slots it is the best form for 65 - 76 queries only (70 queries 65 us, mode 1 73); lists beyond what
+// modes 1 and 2 hold (3840) have it up to some hundred queries: 100 queries x 4096 slots 121 us and 152 in mode 1 of two ranges, x 8192
+// 215 and 285 (303 in mode 0 undivided), 300 x 4096 357 and 391 (381).
 // 32 heads: 257 queries 78 us in mode 4 and 112 in mode 2, 800 queries 175 and 236.  4000 queries of 128 heads: 256 slots 440 us in
 // mode 0 and 390 in mode 3, 640 slots 760 and 800 (150 queries x 256 slots 28.6 and 31.2).
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
