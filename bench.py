@@ -143,7 +143,7 @@ def config_row(n):
                    config={"workload": "config 1"})
     elif n == 5:
         T = 32768
-        os.environ.setdefault("DSA_BWD_WORKSPACE_GIB", "128")        # one sweep over all queries (105 GiB of workspace)
+        os.environ.setdefault("DSA_BWD_WORKSPACE_GIB", "128")        # one sweep over all queries (89 GiB of workspace)
         cu = O.make_packed_cu_seqlens(T, 4, 2048, seed=7)
         iq, ik, w = O.make_indexer_inputs(T, HI, 128, seed=7)
         ks, ke = (x.to(dev) for x in O.indexer_window(T, 0, cu))

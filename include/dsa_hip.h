@@ -216,7 +216,8 @@ int dsa_thd_positions(const void* cu, int cu_i64, int ncu, int tokens, int64_t o
 
 /*
  * Sparse MQA-MLA attention forward.  Slot t of query i (global position q_start + i) is valid iff
- * ids[i,t] != -1, 0 <= ids[i,t] < Skv and ids[i,t] <= q_start + i.  Over the valid slots:
+ * ids[i,t] != -1, 0 <= ids[i,t] < Skv and ids[i,t] <= q_start + i (none where that is
+ * negative).  Over the valid slots:
  *   s = q[i,h,:] . kv[ids[i,t],:]   P = softmax_t(s * sm_scale)   out[i,h,:] = sum_t P kv[ids[i,t], :d_v]
  *   lse[i,h] = natural-log sum-exp of s * sm_scale  (+inf, with out = 0, when no slot is valid)
  *   p_out[i,h,t] = s (raw logit) on valid slots, -inf elsewhere; optional (NULL to skip);
@@ -286,7 +287,7 @@ int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges
  * (math: loongforge/models/common/experimental_attention_variant/sparse_mla_bwd.py:292-356).
  *   dout [S, H, 512] bf16   dq [S, H, 576] bf16   dkv [Skv, 576] bf16
  * Workspace: dsa_sparse_mla_bwd_workspace_bytes is the largest size the call can use - all queries in one
- * sweep (26 GiB at S = Skv = 8192, K = 2048; 105 GiB at 32768 tokens).  Any size from
+ * sweep (22 GiB at S = Skv = 8192, K = 2048; 89 GiB at 32768 tokens).  Any size from
  * dsa_sparse_mla_bwd_workspace_bytes_min on is accepted: with less than the full size the queries are walked in
  * chunks (the largest of S, S/2, S/4, ... that fits, at least 64), a few per cent slower per extra chunk; the
  * chunking follows from the sizes alone, and dKV is bit-reproducible for a given workspace size.

@@ -52,11 +52,18 @@ def test_binding_arity_matches_header():
 
 def test_forms_of_the_sparse_mla_forward():
     """The sizes with which the GPU tests mean to reach every form of the forward do so."""
+    from loongforge_amd import _lib
     from tests.gpu_util import MLA_FORMS, mla_form
 
     for form, ranges, S, H, K in MLA_FORMS:
         assert mla_form(S, H, K) == (form, ranges), (S, H, K)
     assert {f for f, _, _, _, _ in MLA_FORMS} == {0, 1, 2, 3, 4}
+    # a block of a call: not of fewer queries than it has; nothing to spread, no workspace
+    lib = _lib.load()
+    assert lib.dsa_sparse_mla_fwd_block(None, None, None, 4, 5, 64, 9, 64, 0, 1.0, 512, None, None, None, 0, None, 0, None, 0, None) == -1
+    assert lib.dsa_sparse_mla_fwd_block_workspace_bytes(4, 5, 64, 9, 2048) == 0
+    assert lib.dsa_sparse_mla_fwd_block_workspace_bytes(40, 10, 64, 9, 2048) == 10 * 4 * 64 * (512 * 4 + 8) + 256
+    assert lib.dsa_sparse_mla_fwd_workspace_bytes(40, 64, 9, 2048) == 40 * 4 * 64 * (512 * 4 + 8) + 256
     assert mla_form(4, 48, 64)[0] == mla_form(4, 64, 96)[0] == mla_form(4, 64, 16384)[0] == mla_form(0, 64, 64)[0] == -1
 
 
