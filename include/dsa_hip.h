@@ -260,8 +260,9 @@ int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int
                           void* workspace, size_t workspace_bytes, void* stream);
 /*
  * The same for a block of S queries of a call of S_all: those rows of its results (out, lse, p_out), bit for bit.  The last bits
- * of a query depend on how the work is shared out, and that on the number of queries; here S_all decides, and as of
- * dsa_sparse_mla_fwd_ws it does so with a workspace of the size that the call of S_all, or a block of it, can use.
+ * of a query depend on how the work is shared out, and that on the number of queries: here S_all decides.  The rows are those of
+ * dsa_sparse_mla_fwd_ws with its full workspace if the block has dsa_sparse_mla_fwd_block_workspace_bytes, and those of
+ * dsa_sparse_mla_fwd_ex if it has none.
  */
 size_t dsa_sparse_mla_fwd_block_workspace_bytes(int S_all, int S, int H, int Skv, int K);
 int dsa_sparse_mla_fwd_block(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv,
