@@ -15,6 +15,8 @@
 // The key-sorted order comes from a bitmap key x query, its row-wise prefix popcounts and
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
+#include <algorithm>
+
 #include "mla_tile.h"
 #include "order.h"
 
@@ -27,6 +29,37 @@ constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
 constexpr int PDS_THREADS = 512;
+
+// Joint units.  With 64 or 32 heads, 2 or 4 consecutive queries may be worked as one query of 128 heads: their rows of Q, dO, O, lse and
+// dQ follow one another in memory just like that.  The unit's slots are the union of the queries' keys, ascending; an entry carries
+// in bits 24 .. 27 which of the queries have it (UNIT_KEY masks the key), and P and dS are zero for the heads of the others.  One
+// pair row then stands for the key's pairs with all of them, and a key tile is gathered once.  order::qmap_unit_kernel decides
+// for every group; `units` holds its padded slot count, or 0 where the queries stay by themselves.
+// Why: the backward of few heads is bound by its pair rows, 1152 bytes written and read whatever the heads, and neighbouring queries share
+// keys - a sliding window all but one, a selection of K out of L at least K / L of them.  The matrix work of the heads that have not
+// selected a slot is wasted, which the pipes have room for.  Whole backward, us, by themselves / joint / as the rule takes them (u:
+// union over sum of the lists): 3072 queries x 640 slots, window and compressed keys, 64 heads (u 0.54) 1219 / 937 / 933, 32 heads (0.27)
+// 1010 / 507 / 506; 2077 x 512 at random, 64 heads (0.73) 827 / 775 / 736, 32 heads (0.48) 683 / 512 / 494; 4000 x 512, 64 heads (0.83)
+// 1557 / 1619 / 1504, 32 heads (0.63) 1301 / 1178 / 1145; 8000 x 256, 64 heads (0.94) 1970 / 2189 / 1969; 3000 x 2048, 32 heads (0.28)
+// 2483 / 1105 / 1113.
+constexpr int unit_queries(int HG) { return 4 / HG; }
+constexpr int UNIT_SLOTS = 3072;             // what the lists in LDS behind the operands of 128 heads have room for
+constexpr int UNIT_KEY = 0xffffff;
+inline int unit_slots(int HG, int K) { return unit_queries(HG) * K < UNIT_SLOTS ? unit_queries(HG) * K : UNIT_SLOTS; }
+// dS of a group of G queries in memory: of the queries by themselves or of their unit
+inline size_t group_pds_bytes(int HG, int G, int K) {
+  const size_t apart = (size_t)G * (K / BI) * pds_kind_bytes(HG), joint = (size_t)(unit_slots(HG, K) / BI) * pds_kind_bytes(4);
+  return G == 1 || apart > joint ? apart : joint;
+}
+// A unit's list of `n` slots (a multiple of 32) to LDS.  Slots behind the last key repeat the first one, for none of the queries.
+__device__ __forceinline__ void stage_unit(const int* __restrict__ list, int n, int* idx_s) {
+  const int pad = list[0] & UNIT_KEY;
+  for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    const int v = list[t];
+    idx_s[t] = v < 0 ? pad : v;
+  }
+  __syncthreads();
+}
 
 // ---------------------------------------------------------------------------------------------
 // dQ
@@ -44,10 +77,11 @@ constexpr int PDS_THREADS = 512;
 // With up to 64 heads a wave owns its 3 d-tiles for head group hp only; with up to 32, for one k-step (16 keys) of the only
 // head group, and the two k-steps' sums are added at the end.
 constexpr int DQ_THREADS = 768;
-template <int STAGES, int HG>
+// ids, pds, dq: the query's (UNIT: the joint unit's) slots, dS tiles and rows of dQ; qpos: its position
+template <int STAGES, int HG, bool UNIT>
 __device__ __forceinline__ void dq_body(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, int q0, int ql, int H, int Skv, int K, int q_start, const int* __restrict__ dup_flag,
+    __bf16* __restrict__ dq, int H, int Skv, int K, int qpos, const int* __restrict__ dup_flag,
     unsigned char* smem) {
   constexpr int STAGE_BYTES = TILE_BYTES + pds_kind_bytes(HG);
   constexpr int NJ = HG == 4 ? 2 : 1;          // head groups of a wave
@@ -56,14 +90,15 @@ __device__ __forceinline__ void dq_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dg = wave % 6, hp = wave / 6;
   const int r = lane & 31, g = lane >> 5;
-  const int qi = q0 + ql;
   const int NT = K / BI;
   int* idx_s = (int*)(smem + STAGES * STAGE_BYTES);
   unsigned* tmask = (unsigned*)(idx_s + K);
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
+  int ntiles = NT;
   // (the helper is written for four waves; the others repeat part of its work with equal results)
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  if constexpr (UNIT) stage_unit(ids, K, idx_s);
+  else ntiles = stage_ids(ids, 0, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
 
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   // transposed read of the dS block: lane (blk, ii) points at key 16s + 8t + 4g + ii/4 and the 4 heads
@@ -101,14 +136,14 @@ __device__ __forceinline__ void dq_body(
   unsigned t_goff = 0, t_lb = 0, t_lbd = 0;
   const unsigned char* t_src = nullptr;
   auto issue_prepare = [&](int n) {
-    const int tile = tlist[n];
+    const int tile = UNIT ? n : tlist[n];
     const unsigned sb = lds0 + (unsigned)((n % STAGES) * STAGE_BYTES);
     int kid = idx_s[tile * BI + gkey];
-    kid = kid < 0 ? 0 : kid;
+    kid = UNIT ? kid & UNIT_KEY : kid < 0 ? 0 : kid;
     t_goff = (unsigned)kid * (DQK * 2) + gslot;
     t_lb = __builtin_amdgcn_readfirstlane(sb + (unsigned)((wave & 3) * 1024 + (wave >> 2) * GRP_BYTES));
     t_lbd = __builtin_amdgcn_readfirstlane(sb + (unsigned)(TILE_BYTES + (wave & (DS_WAVES - 1)) * 1024));
-    t_src = uniform_ptr(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(HG));     // dS
+    t_src = uniform_ptr(pds + (size_t)tile * pds_kind_bytes(HG));     // dS
   };
   // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0 .. DS_WAVES - 1)
   auto issue_step = [&](int j) {
@@ -202,7 +237,7 @@ __device__ __forceinline__ void dq_body(
     const int dt = 3 * dg + u / NJ;
     const int h = (hg0 + u % NJ) * 32 + r;
     if (h < H) {                               // the same for all lanes of a wave (H is a multiple of 32)
-      unsigned short* op = (unsigned short*)dq + ((size_t)qi * H + h) * DQK + 32 * dt + 8 * g;
+      unsigned short* op = (unsigned short*)dq + (size_t)h * DQK + 32 * dt + 8 * g;
       uint4 o[2];
       acc_row_to_16B(acc[u], 1.0f, o);
       if (poison) o[0] = o[1] = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
@@ -416,7 +451,7 @@ __device__ __forceinline__ void pds_rows_body(
     unsigned char* xb = xch + (n & 1) * FUSED_XCH + half_chunk;
     *(uint2*)xb = dw;
     *(uint2*)(xb + pds_kind_bytes(2)) = pw;
-    *(uint2*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(HG) + half_chunk) = dw;
+    *(uint2*)(pds + (size_t)tile * pds_kind_bytes(HG) + half_chunk) = dw;
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
@@ -513,25 +548,42 @@ constexpr int WIDE_XCH = WIDE_TILE + TILE_BYTES;
 constexpr int WIDE_LISTS = 128 * DQK * 2;              // Q of the query fits in front of the lists before the rest is there
 static_assert(WIDE_XCH + 2 * pds_kind_bytes(4) <= WIDE_LISTS && WIDE_TILE + 65536 <= WIDE_LISTS, "the lists lie behind everything else");
 inline size_t wide_lds_bytes(int K) { return (size_t)WIDE_LISTS + ids_lds_bytes(K) + 1024 + 2048; }
+inline size_t unit_lds_bytes(int slots) { return (size_t)WIDE_LISTS + (size_t)slots * 4 + 1024 + 2048; }
+static_assert(WIDE_LISTS + UNIT_SLOTS * 4 + 1024 + 2048 <= 160 * 1024, "the list of a joint unit");
 
-template <int hh>
+// Zero where a bf16 value is not finite (exponent all ones), in 16 bytes of LDS
+__device__ __forceinline__ void drop_nonfinite(unsigned char* p) {
+  uint4 v = *(uint4*)p;
+  unsigned* w = (unsigned*)&v;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if ((w[i] & 0x7f80u) == 0x7f80u) w[i] &= 0xffff0000u;
+    if ((w[i] & 0x7f800000u) == 0x7f800000u) w[i] &= 0xffffu;
+  }
+  *(uint4*)p = v;
+}
+
+// All arrays from the query's first head on.  G > 1: a joint unit of G queries with 128 / G heads each (H = 128, K its slots).  The
+// products over the heads then meet heads whose query has not selected the key: their P and dS are zero, and what is not finite in
+// their rows of Q and dO would still make the pair row NaN.  Such values become zero in LDS, where the column operands are read; the
+// query's own pairs are NaN all the same, through lse (NaN for a head with such a value in Q) or delta (not finite with one in dO).
+template <int hh, int G>
 __device__ __forceinline__ void pds_rows_wide_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int ql, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
+    int H, int Skv, int K, int qpos, float sm_scale, int dummy_row, unsigned char* smem) {
   constexpr int VS = DV / 32;
   constexpr int XQ_ACC = 7;                    // column operands of Q in accumulation registers, beside all row operands: 124
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int qi = q0 + ql;
   const int NT = K / BI;
   unsigned char* xch = smem + WIDE_XCH;
   int* idx_s = (int*)(smem + WIDE_LISTS);
-  unsigned* tmask = (unsigned*)(idx_s + K);
+  unsigned* tmask = (unsigned*)(idx_s + K);    // (no masks and list of tiles in a joint unit: its slots are dense)
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
-  float* stat_s = (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
+  float* stat_s = G > 1 ? (float*)(idx_s + K) : (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
   int* dst_s = (int*)(stat_s + 256);           // [2][256]: destination rows from the tile's first slot on
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   // Registers are short: what depends on the lane is worked out anew for every part.
@@ -543,8 +595,8 @@ __device__ __forceinline__ void pds_rows_wide_body(
 
   // Rows of Q and dO travel to LDS in groups of 128 bytes of all 128 rows, chunk c of row r in slot c ^ (r & 7).  Wave w moves rows
   // 8 w .. 8 w + 7 and 64 + 8 w ..; heads beyond H repeat the last one (their P and dS are zero).
-  const unsigned char* q_rows = (const unsigned char*)uniform_ptr(q + (size_t)qi * H * DQK);
-  const unsigned char* do_rows = (const unsigned char*)uniform_ptr(dout + (size_t)qi * H * DV);
+  const unsigned char* q_rows = (const unsigned char*)uniform_ptr(q);
+  const unsigned char* do_rows = (const unsigned char*)uniform_ptr(dout);
   const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
   auto group_base = [](int p) { return p < 4 ? p * 16384 : p < 8 ? WIDE_TILE + (p - 4) * 16384 : WIDE_ROT; };
   {
@@ -557,11 +609,13 @@ __device__ __forceinline__ void pds_rows_wide_body(
     }
   }
   bf16x8 doreg[VS / 2];                        // dO, the odd 32 columns
+  unsigned bad_do = 0;                         // G > 1: which of the wave's heads have values in dO that are not finite
+  auto of_heads = [](unsigned long long b) { return (unsigned)((b | b >> 16 | b >> 32 | b >> 48) & 0xffffu); };   // lanes (m, kg) -> heads m
   {
     const int m = lane & 15, kg = lane >> 4;
     const int h = wave * 16 + m;
     const bool head_ok = h < H;
-    const size_t hrow = (size_t)qi * H + (head_ok ? h : 0);
+    const size_t hrow = head_ok ? h : 0;
     const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
     const bf16x8* dp = (const bf16x8*)(dout + hrow * DV) + kg;
     bf16x8 o[VS], d[VS];
@@ -585,9 +639,12 @@ __device__ __forceinline__ void pds_rows_wide_body(
       stat_s[h] = head_ok ? lse_h * LOG2E : INFINITY;
       stat_s[128 + h] = head_ok ? part : 0.f;
     }
+    if (G > 1) bad_do = of_heads(__ballot(!(fabsf(part) < INFINITY)));
   }
+  int ntiles = NT;
   // (the helper is written for four waves; the other four repeat part of its work with equal results)
-  const int ntiles = stage_ids(ids, ql, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
+  if constexpr (G > 1) stage_unit(ids, K, idx_s);
+  else ntiles = stage_ids(ids, 0, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();
@@ -612,10 +669,32 @@ __device__ __forceinline__ void pds_rows_wide_body(
   {
     const int l = fresh_lane();
     const unsigned off[2] = {2048 * wave + row_off(l, 0), 2048 * wave + row_off(l, 1)};
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 most = {0, 0};                       // largest magnitude, as bits
+    auto look = [&](const bf16x8& x) {
+      const uint4 v = __builtin_bit_cast(uint4, x);
+      const unsigned wd[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, wd[i] & 0x7fff7fffu));
+    };
 #pragma unroll
     for (int ks = 0; ks < VS; ks++) {
       qreg[ks] = *(const bf16x8*)(smem + group_base(ks >> 1) + off[ks & 1]);
+      if (G > 1) look(qreg[ks]);
       asm volatile("" : "+a"(qreg[ks]));
+    }
+    if constexpr (G > 1) {
+#pragma unroll
+      for (int par = 0; par < 2; par++) look(*(const bf16x8*)(smem + WIDE_ROT + off[par]));
+      const unsigned bad = of_heads(__ballot(most[0] >= 0x7f80 || most[1] >= 0x7f80));
+      if (bad) {                               // the wave's own rows, all columns
+        if (l < 16 && (bad >> l & 1u)) stat_s[16 * wave + l] = NAN;
+#pragma unroll 1
+        for (int p = 0; p < 9; p++)
+#pragma unroll 1
+          for (int c = l; c < 128; c += 64) drop_nonfinite(smem + group_base(p) + 2048 * wave + c * 16);
+      }
+      __syncthreads();
     }
   }
   {
@@ -646,6 +725,16 @@ __device__ __forceinline__ void pds_rows_wide_body(
   }
   DSA_WAIT_VMCNT(0);
   __syncthreads();
+  if constexpr (G > 1) {
+    if (bad_do) {
+      const int l = fresh_lane();
+#pragma unroll 1
+      for (int j = 0; j < 8; j++)
+#pragma unroll 1
+        for (int c = l; c < 128; c += 64) drop_nonfinite(smem + (j < 4 ? 0 : WIDE_TILE) + (j & 3) * 16384 + 2048 * wave + c * 16);
+    }
+    __syncthreads();
+  }
   {
     const int l = fresh_lane();
 #pragma unroll
@@ -664,14 +753,14 @@ __device__ __forceinline__ void pds_rows_wide_body(
   const int grp0 = hh * 5;
   const unsigned tile_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(WIDE_TILE + (wave & 3) * 1024 + grp0 * GRP_BYTES));
   auto issue = [&](int n) {
-    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]), l = fresh_lane();
+    const int tile = G > 1 ? n : __builtin_amdgcn_readfirstlane(tlist[n]), l = fresh_lane();
     int kid = idx_s[tile * BI + 8 * (wave & 3) + (l >> 3)];
-    kid = kid < 0 ? 0 : kid;
+    kid = G > 1 ? kid & UNIT_KEY : kid < 0 ? 0 : kid;
     const unsigned goff = __umul24((unsigned)kid, DQK * 2) + (unsigned)(((l & 7) ^ (l >> 3)) * 16 + grp0 * 128);       // (fewer than 2^24 rows: kv is at most 4 GiB)
 #pragma unroll
     for (int i = 0; i < 5 - hh; i++) dma16(tile_lb + i * GRP_BYTES, goff + i * 128, kv);
     // 1 KB from the tile's first slot on (behind the last query's slots the workspace goes on with the sorted list)
-    if (wave == 7) dma16(lds0 + (unsigned)((unsigned char*)dst_s - smem) + (n & 1) * 1024, (unsigned)l * 16, dst + (size_t)ql * K + tile * BI);
+    if (wave == 7) dma16(lds0 + (unsigned)((unsigned char*)dst_s - smem) + (n & 1) * 1024, (unsigned)l * 16, dst + tile * BI);
   };
   issue(0);
 
@@ -692,8 +781,8 @@ __device__ __forceinline__ void pds_rows_wide_body(
 
   // S, dP -> P, dS of tile n
   auto phase_pds = [&](int n) {
-    const int tile = __builtin_amdgcn_readfirstlane(tlist[n]);
-    const unsigned mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+    const int tile = G > 1 ? n : __builtin_amdgcn_readfirstlane(tlist[n]);
+    const unsigned mask = G > 1 ? 0u : __builtin_amdgcn_readfirstlane(tmask[tile]);
     f32x4 sacc[2], dpacc[2];
     constexpr int NJ = 2 * (DQK / 32), FD = 3;
     bf16x8 f[FD], x;                           // key rows of step j = 2 ks + kt; row operand from LDS: dO of even ks, Q of the rotary ks
@@ -722,12 +811,13 @@ __device__ __forceinline__ void pds_rows_wide_body(
     unsigned pw[2][2], dw[2][2];
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      const bool valid = (mask >> (16 * kt + lm)) & 1u;
+      // (G > 1: the query of the wave's heads is wave * G / 8)
+      const bool valid = G > 1 ? (idx_s[n * BI + 16 * kt + lm] >> (24 + wave * G / 8)) & 1 : (mask >> (16 * kt + lm)) & 1u;
       float pf[4], df[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         pf[i] = valid ? __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], c2, -lse2[i])) : 0.f;
-        df[i] = pf[i] * (dpacc[kt][i] - delta[i]) * sm_scale;
+        df[i] = G > 1 && !valid ? 0.f : pf[i] * (dpacc[kt][i] - delta[i]) * sm_scale;
       }
       pw[kt][0] = cvt_pk_bf16(pf[0], pf[1]); pw[kt][1] = cvt_pk_bf16(pf[2], pf[3]);
       dw[kt][0] = cvt_pk_bf16(df[0], df[1]); dw[kt][1] = cvt_pk_bf16(df[2], df[3]);
@@ -741,7 +831,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
     const uint4 d16 = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
     *(uint4*)(xch + chunk) = d16;
     *(uint4*)(xch + pds_kind_bytes(4) + chunk) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
-    *(uint4*)(pds + ((size_t)ql * NT + tile) * pds_kind_bytes(4) + chunk) = d16;
+    *(uint4*)(pds + (size_t)tile * pds_kind_bytes(4) + chunk) = d16;
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
@@ -913,34 +1003,71 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-template <int HG>
+// The query of workgroup i, from the last one on; with groups of G in G turns over the groups with one query of each, so that the
+// workgroups that do joint units follow one another.  Neighbouring workgroups go to different XCDs: with the groups' queries side by side
+// every G-th workgroup did the work, on 8 / G of the XCDs (3072 x 32 heads x 640 slots: scores and rows 865 us instead of 296).
+template <int G>
+__device__ __forceinline__ int query_of(int i, int cnt) {
+  const int groups = cnt / G, rest = cnt - groups * G;
+  if (G == 1 || i < rest) return cnt - 1 - i;
+  const int turn = (i - rest) / groups;
+  return (groups - 1 - (i - rest - turn * groups)) * G + turn;
+}
+
+// G: queries of a group that may be a joint unit (4 / HG), or 1.  units: padded slot counts of the groups' units, 0 where the queries
+// are by themselves.
+template <int HG, int G>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
-    int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, const int* __restrict__ units,
+    size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int ql = cnt - 1 - (int)blockIdx.x;
-  // (two copies of the body: every copy meets the same barriers)
+  const int ql = query_of<G>((int)blockIdx.x, cnt);
+  // (two copies of every body: each copy meets the same barriers)
+  if constexpr (HG == 4 || G > 1) {            // 128 heads: of the query or of a unit
+    const int slots = G > 1 ? units[ql / G] : K;
+    if (slots > 0) {
+      if (G > 1 && ql % G) return;
+      const size_t hrow = (size_t)(q0 + ql) * H;
+      unsigned char* unit = pds + (size_t)(ql / G) * group_pds;
+      const __bf16 *q_rows = q + hrow * DQK, *out_rows = out + hrow * DV, *do_rows = dout + hrow * DV;
+      const int *list = ids + (size_t)ql * K, *drow = dst + (size_t)ql * K;
+      if (threadIdx.x < 256) pds_rows_wide_body<0, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
+      else pds_rows_wide_body<1, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
+      return;
+    }
+  }
   if constexpr (HG <= 2) {
-    if (threadIdx.x < 256) pds_rows_body<0, HG>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-    else pds_rows_body<1, HG>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-  } else {
-    if (threadIdx.x < 256) pds_rows_wide_body<0>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
-    else pds_rows_wide_body<1>(q, kv, ids, out, dout, lse, pds, dst, rows, q0, ql, H, Skv, K, q_start, sm_scale, dummy_row, smem);
+    unsigned char* own = pds + (size_t)(ql / G) * group_pds + (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
+    if (threadIdx.x < 256) pds_rows_body<0, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_body<1, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
   }
 }
 
-template <int HG>
+template <int HG, int G>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, int q0, int cnt, int H, int Skv, int K, int q_start, const int* __restrict__ dup_flag,
-    const unsigned char* __restrict__ rows, const int* __restrict__ start, float* __restrict__ dkv_acc,
+    __bf16* __restrict__ dq, const int* __restrict__ units, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
+    const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const int* __restrict__ start, float* __restrict__ dkv_acc,
     unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
-  if (rs.first) dq_body<3, HG>(kv, ids, pds, dq, q0, cnt - 1 - rs.i, H, Skv, K, q_start, dup_flag, smem);
-  else {
+  if (rs.first) {
+    const int ql = query_of<G>(rs.i, cnt);
+    const int* list = ids + (size_t)ql * K;
+    __bf16* dq_rows = dq + (size_t)(q0 + ql) * H * DQK;
+    const unsigned char* own = pds + (size_t)(ql / G) * group_pds;
+    if constexpr (G > 1) {
+      const int slots = units[ql / G];
+      if (slots > 0) {
+        if (ql % G == 0) dq_body<3, 4, true>(kv, list, own, dq_rows, 128, Skv, slots, 0, dup_flag, smem);
+        return;
+      }
+      own += (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
+    }
+    dq_body<3, HG, false>(kv, list, own, dq_rows, H, Skv, K, q_start + q0 + ql, dup_flag, smem);
+  } else {
     // longest work first: from the first key on where the first half of the keys has most of the rows (causal windows), else
     // from the last key (compressed keys behind a sliding window)
     const int groups = (n_keys + RED_KEYS - 1) / RED_KEYS;
@@ -967,10 +1094,15 @@ __global__ void poison_bf16_kernel(unsigned short* __restrict__ p, size_t n, con
 // ---------------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------------
+// Units pay from 192 groups on, where their lists fit.  Below, too many of the 256 compute units are left without one: 150 pairs of queries
+// 82 us by themselves and 85 joint, 75 groups of four 72 and 82, and looking for them costs 2 - 8 us.
+bool use_units(int HG, int S, int Skv) { return HG < 4 && S >= 192 * unit_queries(HG) && order::unit_lists_fit(unit_queries(HG), Skv); }
+
 struct BwdPlan {
   int chunk;            // queries per pass over the buffers
+  int G;                // queries of a group that may be a unit, or 1
   int W;                // bitmap words per key
-  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_dst, off_sorted, off_pds, off_rows, off_acc, total;
+  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_bad, off_dst, off_sorted, off_pds, off_rows, off_acc, total;
 };
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -985,9 +1117,12 @@ BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
   p.off_count = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_start = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_flag = o; o = align_up(o + 4);
+  const int HG = head_groups(H), G = p.G = use_units(HG, chunk, Skv) ? unit_queries(HG) : 1;
+  p.off_units = o; o = align_up(o + (size_t)(chunk + G - 1) / G * 4);
+  p.off_bad = o; o = align_up(o + (size_t)((Skv + 31) / 32) * 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
-  p.off_pds = o; o = align_up(o + (size_t)chunk * (K / BI) * pds_kind_bytes(head_groups(H)));
+  p.off_pds = o; o = align_up(o + (size_t)((chunk + G - 1) / G) * group_pds_bytes(HG, G, K));
   p.off_rows = o; o = align_up(o + ((size_t)chunk * K + 1) * ROW_BYTES);
   p.off_acc = o; o = align_up(o + (size_t)Skv * DQK * 4);
   p.total = o;
@@ -1004,6 +1139,17 @@ BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
     p = layout_plan(chunk, H, Skv, K);
   }
   return p;
+}
+
+// What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, fitted to
+// whole backward passes of 1000 - 8000 queries with 8 - 47 tiles (by themselves 62.8 us at 8 tiles, 98.5 at 15, 236 at 42 of 64 heads, 52 /
+// 81 / 216 of 32; units 135 at 15, 200 at 25, 337 at 46).  Units come in rounds of 256 like queries, G times as few: of up to
+// G x 256 queries there is only one.
+order::UnitCost unit_cost(int HG, int S) {       // (HG 1 or 2)
+  const int G = unit_queries(HG), CUS = 256;
+  const float unit = std::max(1.0f, (float)(G * CUS) / S), apart = std::max(1.0f, (float)CUS / S);
+  const float fixed = HG == 2 ? 226.f : 140.f, tile = HG == 2 ? 50.f : 48.f;
+  return {(int)(420.f * unit), (int)(66.f * unit), (int)(fixed * apart), (int)(tile * apart)};
 }
 
 constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;
@@ -1051,12 +1197,27 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   float* acc = (float*)(ws + p.off_acc);
 
   const int HG = head_groups(H);
+  // The passes are free to choose their slot order (P, dS and the dKV rows never leave the workspace): they walk each query's valid
+  // ids in ascending key order, so that the queries in flight on an XCD gather neighbouring latent rows at the same time, and
+  // may work several queries as one.  (The lists are put together in LDS next to a bitmap over all keys; with more keys than
+  // fit there the passes walk the caller's slot order instead.)
+  const bool sort_ids = order::sorted_list_fits(Skv, K);
+  const int G = p.G;
+  const size_t group_pds = group_pds_bytes(HG, G, K);
+  int* units = (int*)(ws + p.off_units);
+  unsigned* bad = (unsigned*)(ws + p.off_bad);
   const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
   size_t smem_dq = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
   if (smem_dq < reduce_lds) smem_dq = reduce_lds;
-  auto dq_reduce_kernel = HG == 1 ? bwd_dq_reduce_kernel<1> : HG == 2 ? bwd_dq_reduce_kernel<2> : bwd_dq_reduce_kernel<4>;
-  auto pds_rows_kernel = HG == 1 ? bwd_pds_rows_kernel<1> : HG == 2 ? bwd_pds_rows_kernel<2> : bwd_pds_rows_kernel<4>;
-  const size_t smem_rows = HG <= 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
+  if (G > 1) smem_dq = std::max(smem_dq, (size_t)3 * (TILE_BYTES + pds_kind_bytes(4)) + (size_t)unit_slots(HG, K) * 4);
+  auto dq_reduce_kernel = HG == 4   ? bwd_dq_reduce_kernel<4, 1>
+                          : HG == 2 ? (G > 1 ? bwd_dq_reduce_kernel<2, 2> : bwd_dq_reduce_kernel<2, 1>)
+                                    : (G > 1 ? bwd_dq_reduce_kernel<1, 4> : bwd_dq_reduce_kernel<1, 1>);
+  auto pds_rows_kernel = HG == 4   ? bwd_pds_rows_kernel<4, 1>
+                         : HG == 2 ? (G > 1 ? bwd_pds_rows_kernel<2, 2> : bwd_pds_rows_kernel<2, 1>)
+                                   : (G > 1 ? bwd_pds_rows_kernel<1, 4> : bwd_pds_rows_kernel<1, 1>);
+  size_t smem_rows = HG <= 2 ? fused_lds_bytes(K) : wide_lds_bytes(K);
+  if (G > 1) smem_rows = std::max(smem_rows, unit_lds_bytes(unit_slots(HG, K)));
   if (dsa_reserve_lds((const void*)pds_rows_kernel, smem_rows) != hipSuccess ||
       dsa_reserve_lds((const void*)dq_reduce_kernel, smem_dq) != hipSuccess)
     DSA_FAIL(DSA_ERR_LAUNCH, "dsa_sparse_mla_bwd: cannot reserve LDS");
@@ -1074,27 +1235,23 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   }
 #define DSA_MARK(i) do { if (pass_ms) hipEventRecord(ev[i], st); } while (0)
   bool first = true;
-  order::clear_flag(dup_flag, st);
+  if (G > 1) order::kv_check_kernel<<<dim3((Skv + 31) / 32), dim3(256), 0, st>>>((const uint4*)kv, Skv, DQK * 2 / 16, bad, dup_flag);
+  else order::clear_flag(dup_flag, st);
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
     const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     DSA_MARK(0);
-    // The passes are free to choose their slot order (P, dS and the dKV rows never leave the workspace):
-    // they walk each query's valid ids in ascending key order, so that the queries in flight on an XCD
-    // gather neighbouring latent rows at the same time.
-    // (The list is put together in LDS next to a bitmap over all keys; with more keys than fit there the
-    // passes walk the caller's slot order instead.)
-    const bool sort_ids = order::sorted_list_fits(Skv, K);
-    order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
+    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units, unit_slots(HG, K), unit_cost(HG, p.chunk));
+    else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
     pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smem_rows, st>>>(
-        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, q0, cnt, H, Skv, K, q_start,
-        sm_scale, p.chunk * K);
+        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, units, group_pds, q0, cnt, H, Skv, K,
+        q_start, sm_scale, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, q0, cnt, H, Skv,
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, units, group_pds, q0, cnt, H, Skv,
                                                                    K, q_start, dup_flag, rows, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");

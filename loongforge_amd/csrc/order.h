@@ -74,6 +74,165 @@ static __global__ __launch_bounds__(256) void qmap_kernel(const int* __restrict_
   for (int t = threadIdx.x; t < K; t += 256) row[t] = list[t];
 }
 
+// ---- groups of G consecutive queries that may be worked as one unit ----
+// bad[w] bit b  <=>  row 32 w + b of kv (row16 pieces of 16 bytes, bf16) holds a value that is not finite.  Also clears the flag of
+// repeated ids.
+static __global__ __launch_bounds__(256) void kv_check_kernel(const uint4* __restrict__ kv, int Skv, int row16, unsigned* __restrict__ bad,
+                                                              int* __restrict__ dup_flag) {
+  __shared__ unsigned word;
+  if (threadIdx.x == 0) {
+    word = 0u;
+    if (blockIdx.x == 0) *dup_flag = 0;
+  }
+  __syncthreads();
+  const int n = min(32, Skv - 32 * (int)blockIdx.x) * row16;
+  const uint4* p = kv + (size_t)blockIdx.x * 32 * row16;
+  constexpr int AHEAD = 9;                   // all of 32 rows of 576 values
+  for (int e0 = threadIdx.x; e0 < n; e0 += AHEAD * 256) {
+    uint4 v[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) v[i] = p[min(e0 + i * 256, n - 1)];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) {
+      const unsigned w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+      bool inf = false;
+#pragma unroll
+      for (int j = 0; j < 4; j++) inf |= (w[j] & 0x7f80u) == 0x7f80u || (w[j] & 0x7f800000u) == 0x7f800000u;
+      if (inf) atomicOr(&word, 1u << (min(e0 + i * 256, n - 1) / row16));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) bad[blockIdx.x] = word;
+}
+
+// What a group costs as one unit and as single queries: a fixed part and a part per 32 slots each
+struct UnitCost { int unit_fixed, unit_tile, fixed, tile; };
+
+// qmap_kernel for a group of G queries per workgroup.  units[group] = slots of the unit, a multiple of 32, or 0 for single queries.  A
+// unit has the bits of all its queries in its first one's row of qmap, so that it counts as one query in everything behind; its
+// list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query at the end, more than
+// max_slots keys, keys with values that are not finite (a product over the slots would carry them to the queries that do not have
+// them), and what costs less query by query.
+template <int G>
+static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __restrict__ ids, int q0, int cnt, int K, int Skv, int q_start,
+                                                               unsigned* __restrict__ qmap, int Wk, int* __restrict__ sorted,
+                                                               int* __restrict__ dup_flag, const unsigned* __restrict__ bad,
+                                                               int* __restrict__ units, int max_slots, UnitCost cost) {
+  extern __shared__ unsigned qbits[];        // [G][Wk] bits, [G / 2][Wk] prefix counts, 16 bits each
+  __shared__ unsigned wave_tot[G / 2 + 1][8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ql0 = blockIdx.x * G, nq = min(G, cnt - ql0);
+  unsigned* pre = qbits + G * Wk;
+  for (int w = tid; w < G * Wk; w += 512) qbits[w] = 0u;
+  __syncthreads();
+  const int* src = ids + (size_t)(q0 + ql0) * K;
+  for (int t0 = tid; t0 < nq * K; t0 += 8 * 512) {
+    int v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = t0 + i * 512 < nq * K ? src[t0 + i * 512] : -1;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int j = __builtin_amdgcn_readfirstlane((t0 + i * 512) / K);        // (K is a multiple of 64: the same for a wave)
+      if (v[i] >= 0 && v[i] < Skv && v[i] <= q_start + q0 + ql0 + j) {
+        const unsigned bit = 1u << (v[i] & 31);
+        if (atomicOr(&qbits[j * Wk + (v[i] >> 5)], bit) & bit) *dup_flag = 1;
+      }
+    }
+  }
+  __syncthreads();
+  const int per = (Wk + 511) / 512, w0 = tid * per, w1 = min(w0 + per, Wk);
+  auto any = [&](int w) {
+    unsigned b = qbits[w];
+#pragma unroll
+    for (int j = 1; j < G; j++) b |= qbits[j * Wk + w];
+    return b;
+  };
+  // one scan over the threads: the queries' counts in pairs (a query has at most 2048 keys), then the union's beside the number of
+  // threads that saw a key with values that are not finite
+  constexpr int NC = G / 2 + 1;
+  unsigned mine[NC], inc[NC], total[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) mine[c] = 0u;
+  for (int w = w0; w < w1; w++) {
+#pragma unroll
+    for (int j = 0; j < G; j++) mine[j / 2] += (unsigned)__popc(qbits[j * Wk + w]) << (16 * (j & 1));
+    const unsigned b = any(w);
+    mine[NC - 1] += __popc(b);
+    if (b & bad[w]) mine[NC - 1] |= 0x10000u;
+  }
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    inc[c] = mine[c];
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) { const unsigned x = __shfl_up(inc[c], o, 64); if (lane >= o) inc[c] += x; }
+    if (lane == 63) wave_tot[c][wave] = inc[c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    inc[c] -= mine[c];
+    total[c] = 0u;
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      if (w < wave) inc[c] += wave_tot[c][w];
+      total[c] += wave_tot[c][w];
+    }
+  }
+  const int keys = (int)(total[NC - 1] & 0xffffu), tiles = (keys + 31) / 32;
+  int n[G], apart = 0;
+#pragma unroll
+  for (int j = 0; j < G; j++) {
+    n[j] = (int)(total[j / 2] >> (16 * (j & 1)) & 0xffffu);
+    apart += n[j] ? cost.fixed + cost.tile * ((n[j] + 31) / 32) : 0;
+  }
+  const bool unit = nq == G && keys > 0 && 32 * tiles <= max_slots && total[NC - 1] >> 16 == 0u && cost.unit_fixed + cost.unit_tile * tiles <= apart;
+  if (tid == 0) units[blockIdx.x] = unit ? 32 * tiles : 0;
+  for (int w = w0; w < w1; w++) {
+    if (unit) {
+      pre[w] = inc[NC - 1] & 0xffffu;
+      inc[NC - 1] += __popc(any(w));
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC - 1; c++) {
+        pre[c * Wk + w] = inc[c];
+        inc[c] += (unsigned)__popc(qbits[2 * c * Wk + w]) + ((unsigned)__popc(qbits[(2 * c + 1) * Wk + w]) << 16);
+      }
+    }
+  }
+  for (int j = 0; j < nq; j++)
+    for (int w = tid; w < Wk; w += 512) qmap[(size_t)(ql0 + j) * Wk + w] = !unit ? qbits[j * Wk + w] : j == 0 ? any(w) : 0u;
+  __syncthreads();
+  // the lists, ascending: a thread per key, whose place is the number of set bits below it
+  int* row = sorted + (size_t)ql0 * K;
+  for (int k = tid; k < 32 * Wk; k += 512) {
+    const int w = k >> 5, b = k & 31;
+    const unsigned below = (1u << b) - 1u;
+    unsigned own[G], bits = 0u;
+    int v = k;
+#pragma unroll
+    for (int j = 0; j < G; j++) {
+      own[j] = qbits[j * Wk + w];
+      bits |= own[j];
+      v |= (int)(own[j] >> b & 1u) << (24 + j);
+    }
+    if (unit) {
+      if (bits >> b & 1u) row[pre[w] + __popc(bits & below)] = v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < G; j++)
+        if (own[j] >> b & 1u) row[j * K + (int)(pre[(j / 2) * Wk + w] >> (16 * (j & 1)) & 0xffffu) + __popc(own[j] & below)] = k;
+    }
+  }
+  if (unit) {
+    for (int t = keys + tid; t < G * K; t += 512) row[t] = -1;
+  } else {
+#pragma unroll
+    for (int j = 0; j < G; j++)
+      if (j < nq)
+        for (int t = n[j] + tid; t < K; t += 512) row[j * K + t] = -1;
+  }
+}
+
 // grid (ceil(cnt / 256), Wk); workgroup = 4 waves = 256 queries of one key word
 static __global__ __launch_bounds__(256) void bm_transpose_kernel(const unsigned* __restrict__ qmap, int cnt, int Skv, int Wk,
                                                                   unsigned* __restrict__ bitmap, int W) {
@@ -149,11 +308,12 @@ static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __rest
 
 // dst[ql][slot] = row of the pair in key-sorted order (-1 for invalid slots).  A workgroup takes the 32 queries of a word, or
 // a part of them (blockIdx.y) where there are few words, and has the word's bits and first rows of `range` keys at a time in
-// LDS, where the lookups by id go: from memory they were two dependent random reads of 4 bytes per pair (8192 queries x
+// LDS, where the lookups by id go (units: ids are the lists of qmap_unit_kernel, and a unit's pairs are its first query's): from memory they were two dependent random reads of 4 bytes per pair (8192 queries x
 // 2048 slots: 0.165 ms; 32768 x 2048: 1.29 ms).
 static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict__ ids, int row0, int q0, int cnt, int K, int Skv, int q_start,
                                                            const unsigned* __restrict__ bitmap, const unsigned* __restrict__ prefix,
-                                                           const int* __restrict__ start, int range, int* __restrict__ dst) {
+                                                           const int* __restrict__ start, int range, int* __restrict__ dst,
+                                                           const int* __restrict__ units, int G) {
   extern __shared__ uint2 tab[];             // {first row of the word's queries, bits}
   const int w = blockIdx.x, share = 32 / gridDim.y;
   const int q_lo = 32 * w + blockIdx.y * share, q_hi = min(q_lo + share, cnt);
@@ -167,8 +327,9 @@ static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict
     }
     __syncthreads();
     for (int ql = q_lo + sub; ql < q_hi; ql += 4) {
-      const unsigned below = (1u << (ql & 31)) - 1u;
-      const int last = min(Skv - 1, q_start + q0 + ql);
+      const int owner = units && units[ql / G] ? ql / G * G : ql;
+      const unsigned below = (1u << (owner & 31)) - 1u;
+      const int last = units ? Skv - 1 : min(Skv - 1, q_start + q0 + ql);
       const int* row = ids + (size_t)(row0 + ql) * K;       // row0: row of local query 0 in the id array handed in
       for (int t0 = lane; t0 < K; t0 += 8 * 256) {
         int v[8];
@@ -177,8 +338,9 @@ static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           if (t0 + i * 256 >= K) break;
-          const bool ok = v[i] >= 0 && v[i] <= last;
-          const int k = v[i] - k0;
+          const int id = units && v[i] >= 0 ? v[i] & 0xffffff : v[i];
+          const bool ok = id >= 0 && id <= last;
+          const int k = id - k0;
           if (ok && k >= 0 && k < nk) {
             const uint2 e = tab[k];
             dst[(size_t)ql * K + t0 + i * 256] = (int)e.x + __popc(e.y & below);
@@ -213,23 +375,40 @@ inline bool sorted_list_fits(int Skv, int K) {
 }
 // dup_flag: one int the caller has cleared (clear_flag) before the first block of queries of a call.
 inline void clear_flag(int* dup_flag, hipStream_t st) { zero_u32_kernel<<<dim3(1), dim3(64), 0, st>>>((unsigned*)dup_flag, 1); }
-inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
-                  int* count, int* start, int* dst, int W, hipStream_t st, int* dup_flag, int* sorted = nullptr) {
+inline void build_ranks(const int* lists, int row0, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
+                        int* count, int* start, int* dst, int W, const int* units, int G, hipStream_t st) {
   const int Wk = (Skv + 31) / 32;
-  unsigned* qmap = prefix;
-  const size_t lds = (size_t)Wk * 4 * (sorted ? 2 : 1) + (sorted ? (size_t)K * 4 : 0);
-  if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)qmap_kernel, lds);
-  qmap_kernel<<<dim3(cnt), dim3(256), lds, st>>>(ids, q0, cnt, K, Skv, q_start, qmap, Wk, sorted, dup_flag);
   // every word of the bitmap is written (zeros beyond the last query), so no clearing pass is needed
-  bm_transpose_kernel<<<dim3((W + 7) / 8, Wk), dim3(256), 0, st>>>(qmap, cnt, Skv, Wk, bitmap, W);
+  bm_transpose_kernel<<<dim3((W + 7) / 8, Wk), dim3(256), 0, st>>>(prefix, cnt, Skv, Wk, bitmap, W);
   bm_prefix_kernel<<<dim3((Skv + 63) / 64), dim3(1024), 0, st>>>(bitmap, prefix, count, Skv, W);
   key_scan_kernel<<<dim3(1), dim3(1024), 0, st>>>(count, start, Skv);
-  // with `sorted` (rows of the block's queries, [cnt][K]) the ranks are those of the sorted slots
   const int range = Skv < RANK_KEYS ? Skv : RANK_KEYS;
   if (range * 8 > 48 * 1024) (void)dsa_reserve_lds((const void*)rank_kernel, (size_t)range * 8);
   const int words = (cnt + 31) / 32, parts = words >= 256 ? 1 : words >= 128 ? 2 : words >= 64 ? 4 : 8;
-  rank_kernel<<<dim3(words, parts), dim3(1024), (size_t)range * 8, st>>>(sorted ? sorted : ids, sorted ? 0 : q0, q0, cnt, K, Skv, q_start,
-                                                                         bitmap, prefix, start, range, dst);
+  rank_kernel<<<dim3(words, parts), dim3(1024), (size_t)range * 8, st>>>(lists, row0, q0, cnt, K, Skv, q_start, bitmap, prefix, start, range, dst,
+                                                                         units, G);
+}
+inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
+                  int* count, int* start, int* dst, int W, hipStream_t st, int* dup_flag, int* sorted = nullptr) {
+  const int Wk = (Skv + 31) / 32;
+  const size_t lds = (size_t)Wk * 4 * (sorted ? 2 : 1) + (sorted ? (size_t)K * 4 : 0);
+  if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)qmap_kernel, lds);
+  qmap_kernel<<<dim3(cnt), dim3(256), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag);
+  // with `sorted` (rows of the block's queries, [cnt][K]) the ranks are those of the sorted slots
+  build_ranks(sorted ? sorted : ids, sorted ? 0 : q0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, nullptr, 1, st);
+}
+// LDS of qmap_unit_kernel
+inline bool unit_lists_fit(int G, int Skv) { return (size_t)((Skv + 31) / 32) * 4 * (G + G / 2) <= (size_t)150 * 1024; }
+// build with the sorted lists, for groups of G (2 or 4) queries that may be units
+inline void build_units(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix, int* count, int* start,
+                        int* dst, int W, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
+                        UnitCost cost) {
+  const int Wk = (Skv + 31) / 32;
+  const size_t lds = (size_t)Wk * 4 * (G + G / 2);
+  auto kernel = G == 2 ? qmap_unit_kernel<2> : qmap_unit_kernel<4>;
+  if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)kernel, lds);
+  kernel<<<dim3((cnt + G - 1) / G), dim3(512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
+  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st);
 }
 
 }  // namespace order

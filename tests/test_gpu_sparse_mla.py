@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from oracle import dsa_oracle as O
-from tests.gpu_util import MLA_FORMS, assert_close, assert_mla_grads, mla_form
+from tests.gpu_util import MLA_FORMS, REF_DKV_EXCESS_LIMIT, assert_close, assert_mla_grads, mla_form
 
 pytestmark = pytest.mark.gpu
 
@@ -385,6 +385,169 @@ def test_backward_of_many_heads_in_one_pass(gpu, S, H, K, q_start):
     """P, dS and the rows of the pairs in one kernel: the first and the last tiles of a query, empty rows, the end of the order's
     list, against the oracle, with the bounds of the other backward tests."""
     test_backward_of_few_heads(gpu, H, S, K, q_start, None)
+
+
+def _overlapping_ids(S, K, skv, turn, far, seed):
+    """Causal ids of queries at positions skv - S + i: K of the K + K / 8 keys behind a place that moves by a key every ``turn``
+    queries (0: never), and for every ``far``-th run of 16 queries ids at random, which neighbours hardly share."""
+    g = torch.Generator().manual_seed(seed)
+    ids = torch.full((S, K), -1, dtype=torch.int32)
+    for i in range(S):
+        last = skv - S + i
+        if far and i // 16 % far == far - 1:
+            pool = torch.arange(last + 1)
+        else:
+            pool = torch.arange(max(0, i // turn - 8) if turn else 0, last + 1)[:K + K // 8]
+        pick = pool[torch.randperm(len(pool), generator=g)[:K]]
+        ids[i, :len(pick)] = pick.int()
+    return ids
+
+
+def _joint_groups(ids, H):
+    """(groups worked as one query, groups) by the rule of the library: tenths of us per unit against its queries one by one."""
+    G = 128 // H
+    S, full = ids.shape[0], ids.shape[0] // G
+    wide, apart = max(1.0, G * 256 / S), max(1.0, 256 / S)
+    joint = 0
+    for g in range(full):
+        rows = [r[r >= 0] for r in ids[g * G:(g + 1) * G]]
+        tiles = (len(torch.unique(torch.cat(rows))) + 31) // 32
+        one_by_one = sum(int((226 if H == 64 else 140) * apart) + int((50 if H == 64 else 48) * apart) * ((len(r) + 31) // 32) for r in rows if len(r))
+        joint += 0 < 32 * tiles <= 3072 and int(420 * wide) + int(66 * wide) * tiles <= one_by_one
+    return joint, full
+
+
+@pytest.mark.parametrize("H,S,K,skv,turn,far", [
+    (64, 515, 128, 900, 1, 0),        # pairs of queries as one, one query left over
+    (64, 520, 192, 1400, 1, 3),       # both kinds of groups
+    (64, 513, 128, 520, 2, 0),        # lists that begin short
+    (32, 768, 64, 1100, 1, 0),        # four queries as one
+    (32, 771, 64, 1500, 1, 2),        # three queries left over, both kinds
+])
+def test_backward_of_joint_queries(gpu, H, S, K, skv, turn, far):
+    """Consecutive queries of 64 or 32 heads that share most of their keys are worked as one query of 128 heads: holes, empty
+    rows and groups of either kind against the oracle.  dKV against bf16 P and dS and fp32 rows: a row per unit instead of one per
+    query is rounded to bf16, so the bound with the oracle's own rounded rows does not apply; an element may be off by the
+    largest excess any of these tests knows for them, all together by the 2**-9 / sqrt(3) of a rounding for the rows and for
+    the result, 1.1e-3 each, times 2 where rows cancel."""
+    from loongforge_amd import ops
+
+    q_start = skv - S
+    inp = O.make_mla_inputs(S, H, K, seed=S + H, skv=skv, q_start=q_start)
+    inp.idx = _overlapping_ids(S, K, skv, turn, far, S)
+    inp.idx[2] = -1
+    inp.idx[8:12] = -1
+    inp.idx[20:40, 10:13] = -1
+    joint, groups = _joint_groups(inp.idx, H)
+    assert joint > groups // 4 and joint < groups - groups // 8 * (far > 0)
+    q, kv, idx, do = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu)
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, q_start, inp.sm_scale)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, inp.sm_scale)
+    dq_b, dkv_b = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, inp.idx, inp.dout, q_start, inp.sm_scale, 512, out=out.cpu(),
+                                                   lse=lse.cpu(), dtype=torch.float64)
+    assert_close(dq, dq_b, "dQ")
+    d = dkv.double().cpu() - dkv_b
+    assert (d.abs() - 2e-2 - 1e-2 * dkv_b.abs()).max().item() <= REF_DKV_EXCESS_LIMIT
+    assert d.norm() <= 2 * (2 * (2.0 ** -9 / 3 ** 0.5) ** 2) ** 0.5 * dkv_b.norm()
+    dq2, dkv2 = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, inp.sm_scale)
+    assert torch.equal(dq, dq2) and torch.equal(dkv, dkv2)
+    assert (dq[2] == 0).all() and (dq[8:12] == 0).all()
+    # a repeated id in one query of a group: NaN everywhere, as ever
+    dup = idx.clone()
+    dup[S // 2, 5] = dup[S // 2, 9]
+    dq3, dkv3 = ops.sparse_mla_bwd(q, kv, out, do, dup, lse, q_start, inp.sm_scale)
+    assert torch.isnan(dq3.float()).all() and torch.isnan(dkv3.float()).all()
+
+
+@pytest.mark.parametrize("H,S,K,skv,causal", [
+    (64, 700, 2048, 4076, False),     # unions beyond the longest list of a unit, and within it
+    (64, 1030, 512, 1200, True),
+    (32, 1100, 2048, 2900, False),    # nearly the longest list
+    (32, 1537, 192, 1537, True),      # from one key on
+    (32, 1540, 256, 6000, False),     # little in common: no units
+])
+def test_backward_of_joint_queries_is_that_of_wider_queries(gpu, H, S, K, skv, causal):
+    """The same gradients as through the kernels for 128 heads with heads of zeros beside the queries' own, in one sweep and in
+    several.  dQ: the order of its fp32 sums, rounded to bf16 - 2**-8 of an element, or an fp32 step of the largest ones where terms
+    cancel.  dKV: pair rows rounded to bf16 once per query or once per unit, 2**-9 of a row each, independent of one another."""
+    from loongforge_amd import _lib, ops
+
+    g = torch.Generator(device=gpu).manual_seed(S + H)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu).to(torch.bfloat16)                     # noqa: E731
+    q, kv, do = rnd(S, H, 576), rnd(skv, 576), rnd(S, H, 512)
+    score = torch.rand(S, skv, generator=g, device=gpu)
+    q_start = skv - S if causal else skv
+    if causal:
+        score.masked_fill_(torch.arange(skv, device=gpu)[None] > (q_start + torch.arange(S, device=gpu))[:, None], -1.0)
+    val, idx = score.topk(K, -1)
+    idx = torch.where(val >= 0, idx, -1).int()
+    joint, groups = _joint_groups(idx.cpu(), H)
+    assert joint == 0 if skv == 6000 else joint > groups // 4
+    sm = 192 ** -0.5
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, q_start, sm)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, q_start, sm)
+    wide = lambda t: torch.cat([t, torch.zeros(S, 128 - H, *t.shape[2:], dtype=t.dtype, device=gpu)], 1).contiguous()      # noqa: E731
+    dq_w, dkv_w = ops.sparse_mla_bwd(wide(q), kv, wide(out), wide(do), idx, wide(lse), q_start, sm)
+    a, b = dq.float(), dq_w[:, :H].float()
+    assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -14 * b.abs().max()).all()
+    a, b = dkv.float(), dkv_w.float()
+    assert (a - b).norm() <= 5e-3 * b.norm()
+    lib = _lib.load()
+    part = lib.dsa_sparse_mla_bwd_workspace_bytes((S + 1) // 2, H, skv, K)
+    ws = torch.empty(part, dtype=torch.uint8, device=gpu)
+    dq2, dkv2 = torch.empty_like(q), torch.empty_like(kv)
+    rc = lib.dsa_sparse_mla_bwd(q.data_ptr(), kv.data_ptr(), out.data_ptr(), do.data_ptr(), idx.data_ptr(), lse.data_ptr(), S, H, skv, K,
+                                q_start, sm, 512, dq2.data_ptr(), dkv2.data_ptr(), ws.data_ptr(), part,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.dsa_last_error()
+    a, b = dq2.float(), dq_w[:, :H].float()
+    assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -14 * b.abs().max()).all()
+    a, b = dkv2.float(), dkv_w.float()
+    assert (a - b).norm() <= 5e-3 * b.norm()
+
+
+@pytest.mark.parametrize("H,S", [(64, 520), (32, 800)])
+@pytest.mark.parametrize("where,value", [("dout", float("nan")), ("dout", float("inf")), ("q", float("nan")), ("q_rope", float("inf")),
+                                         ("kv", float("nan"))])
+def test_backward_of_joint_queries_keeps_nonfinite_values_apart(gpu, H, S, where, value):
+    """A value that is not finite in one query's row reaches that query's dQ and the keys it selected and nothing else, as if
+    the queries it is worked with were not there; in a key row, the queries that selected the key."""
+    from loongforge_amd import ops
+
+    K, skv = 128, 700
+    inp = O.make_mla_inputs(S, H, K, seed=S, skv=skv, q_start=skv)
+    idx = _overlapping_ids(S, K, skv + S, 0, 0, 5)        # K of 144 keys
+    assert _joint_groups(idx, H)[0] > S * H // 128 // 2
+    q, kv, do = inp.q.to(gpu), inp.kv.to(gpu), inp.dout.to(gpu)
+    ids, sm = idx.to(gpu), inp.sm_scale
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, skv, sm)
+    dq0, dkv0 = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, skv, sm)
+    assert torch.isfinite(dq0.float()).all() and torch.isfinite(dkv0.float()).all()
+    bad = 101
+    if where == "dout":
+        do[bad, H // 2, 77] = value
+    elif where == "kv":
+        kv[int(idx[bad, 3]), 5] = value
+    else:
+        q[bad, 3, 40 if where == "q" else 570] = value
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, skv, sm)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, skv, sm)
+    hit = torch.zeros(S, dtype=torch.bool)
+    if where == "kv":
+        hit = (idx == int(idx[bad, 3])).any(1)
+        keys = torch.unique(idx[hit]).long()
+    else:
+        hit[bad] = True
+        keys = idx[bad].long()
+    assert 0 < hit.sum() < S
+    touched = torch.zeros(skv, dtype=torch.bool)
+    touched[keys] = True
+    dq, dkv = dq.float().cpu(), dkv.float().cpu()
+    assert torch.isfinite(dq[~hit]).all()
+    assert (~torch.isfinite(dq[hit])).flatten(1).any(1).all()
+    assert torch.isfinite(dkv[~touched]).all()
+    if where != "kv":                          # (every pair of the query has a non-finite row)
+        assert (~torch.isfinite(dkv[touched])).any(1).all() and torch.equal(dkv[~touched], dkv0.float().cpu()[~touched])
 
 
 def test_backward_does_not_depend_on_the_slot_order(gpu):
