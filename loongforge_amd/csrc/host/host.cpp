@@ -418,7 +418,9 @@ Tensor seqlens(const Tensor& cu, const c10::Device& device) {
   return t.contiguous();
 }
 
-py::tuple indexer_window(const OptTensor& cu_, int64_t S, int64_t chunk_offset, const Tensor& like) {
+struct Window { Tensor bounds; std::unique_ptr<WindowCheck> check; };      // [2, S]: first key, key behind the last
+
+Window key_windows(const OptTensor& cu_, int64_t S, int64_t chunk_offset, const Tensor& like) {
   need_gpus(like);
   OptTensor cu;
   if (cu_) cu = seqlens(*cu_, like.device());
@@ -439,7 +441,42 @@ py::tuple indexer_window(const OptTensor& cu_, int64_t S, int64_t chunk_offset, 
   if (check->need && (hipEventCreateWithFlags(&check->done, hipEventDisableTiming) != hipSuccess ||
                       hipEventRecord(check->done, (hipStream_t)call.stream) != hipSuccess))
     throw std::runtime_error("indexer window: no event");
-  return py::make_tuple(window.select(0, 0), window.select(0, 1), std::move(check));
+  return {window, std::move(check)};
+}
+
+py::tuple indexer_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, const Tensor& like) {
+  Window w = key_windows(cu, S, chunk_offset, like);
+  return py::make_tuple(w.bounds.select(0, 0), w.bounds.select(0, 1), std::move(w.check));
+}
+
+// The indexer's forward in one call: quantisers (behind the front end if there are rotary tables, else behind the rotation if
+// asked for), key windows, logits and top-k.  Five calls from Python cost 35 - 40 us of host time, more than the kernels of a few
+// queries take.  None for shapes and types that need padding or conversion first.  -> (scores, ids, q8, q_scale, scaled weights,
+// k8, k_scale, check or None): check.wait() belongs behind it, as with indexer_window.
+py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weights, bool rotate, double factor, const OptTensor& cu,
+                           int64_t chunk_offset, int64_t K, bool sort, const OptTensor& cos, const OptTensor& sin, int64_t pairing,
+                           const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& ln_weight,
+                           const OptTensor& ln_bias, double ln_eps) {
+  if (!plain(q, k, weights, cu, cos, sin, positions_q, positions_k, ln_weight, ln_bias)) return py::none();
+  if (!q.is_cuda() || q.dim() != 3 || k.dim() != 2 || q.size(2) != 128 || k.size(1) != 128 || (q.size(1) != 32 && q.size(1) != 64) ||
+      q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || weights.sizes() != q.sizes().slice(0, 2)) return py::none();
+  using Three = std::tuple<Tensor, Tensor, Tensor>;
+  using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+  Tensor q8, q_scale, scaled, k8, k_scale, rows;
+  if (cos) {
+    std::tie(q8, q_scale, rows, scaled) = py::cast<Four>(indexer_front(q, q.size(1), {}, {}, 0.0, cos, sin, pairing, positions_q, batch, rotate,
+                                                                       weights, factor, true, false, 1e-12, true, false));
+    std::tie(k8, k_scale, rows, rows) = py::cast<Four>(indexer_front(k, 1, ln_weight, ln_bias, ln_eps, cos, sin, pairing, positions_k, batch, rotate,
+                                                                     {}, 1.0, true, false, 1e-12, true, false));
+  } else {
+    std::tie(q8, q_scale, scaled) = py::cast<Three>(quant_weights(q, weights, factor, rotate, 1e-12, true, false));
+    if (rotate) std::tie(k8, k_scale, rows) = py::cast<Three>(rotate_quant(k, 1e-12, true, true, false, false));
+    else std::tie(k8, k_scale) = py::cast<std::pair<Tensor, Tensor>>(quant_rowwise(k, 1e-12, true, false));
+  }
+  Window w = key_windows(cu, q.size(0), chunk_offset, q8);
+  const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
+      indexer_topk(q8, scaled, k8, k_scale, w.bounds.select(0, 0), w.bounds.select(0, 1), K, sort, false));
+  return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale, w.check->done ? py::cast(std::move(w.check)) : py::none());
 }
 
 py::object thd_positions(const Tensor& cu_, int64_t tokens, int64_t offset) {
@@ -593,6 +630,22 @@ py::object absorbed_query(const Tensor& q_up, const Tensor& w, const Tensor& cos
   return py::cast(q_up.dim() == 3 ? query : query.view(shape));
 }
 
+void rope_rows(const OptTensor& pe_src, const OptTensor& pe_dst, const OptTensor& cos_, const OptTensor& sin_, int64_t in_pairing,
+               int64_t out_pairing, bool inverse, const OptTensor& positions_, int64_t batch, const OptTensor& main_src, const OptTensor& main_dst);
+
+// kv [s, b, h, d] (packed: [t, h, d]) and the rotated k_pe that the heads share, side by side in new rows
+py::object absorbed_key(const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin, const OptTensor& positions, int64_t emb,
+                        bool packed, int64_t out_pairing) {
+  if (!plain(kv, k_pe, cos, sin, positions) || kv.dim() != (packed ? 3 : 4) || !kv.is_contiguous() || !k_pe.is_contiguous() ||
+      !cos.is_contiguous() || !sin.is_contiguous() || emb % 4) return py::none();
+  const int64_t heads = kv.size(-2), d = kv.size(-1), T = packed ? kv.size(0) : kv.size(0) * kv.size(1);
+  if (k_pe.numel() != T * emb) return py::none();
+  Tensor key = make({T, heads, d + emb}, kv.scalar_type(), kv);
+  rope_rows(k_pe.view({T, 1, emb}).expand({T, heads, emb}), key.narrow(2, d, emb), cos, sin, 0, out_pairing, false, positions,
+            packed ? 1 : kv.size(1), kv.view({T, heads, d}), key.narrow(2, 0, d));
+  return py::cast(packed ? key : key.view({kv.size(0), kv.size(1), heads, d + emb}));
+}
+
 py::object absorb(const Tensor& a, const Tensor& w, bool flat) {
   if (!plain(a, w) || a.dim() < 3 || w.dim() != 3) return py::none();
   const Tensor a3 = a.dim() == 3 ? a : a.reshape({-1, a.size(-2), a.size(-1)});
@@ -671,11 +724,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(attn_dist);
   DEF(kl_loss);
   DEF(indexer_window);
+  DEF(indexer_forward);
   DEF(thd_positions);
   DEF(absorb_into);
   DEF(absorb);
   DEF(absorb_rope_query_into);
   DEF(absorbed_query);
+  DEF(absorbed_key);
   DEF(rope_rows);
 #undef DEF
 }

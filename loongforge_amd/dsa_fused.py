@@ -575,7 +575,7 @@ class DSAttentionFused(MegatronModule):
             # softmax, F.kl_div(log(pred + 1e-10), target + 1e-10, "sum") and their backward in one kernel
             from . import ops
             loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10)
-            indexer_loss = indexer_loss_coeff * loss / sq
+            indexer_loss = loss * (indexer_loss_coeff / sq) if sq else indexer_loss_coeff * loss / sq      # (one launch each way)
             if indexer_loss_coeff > 0:
                 DSAIndexerLossLoggingHelperFused.save_loss_to_tracker(
                     loss=indexer_loss,

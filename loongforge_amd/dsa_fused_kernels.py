@@ -51,6 +51,23 @@ def padded_flashinfer_topk(logits, topk, sk, *, sorted=True):
     return vals.reshape(*lead, topk), idx.reshape(*lead, topk)
 
 
+class _NoNode:
+    """The context of an autograd function's forward in a call that records nothing."""
+
+    def save_for_backward(self, *tensors):
+        pass
+
+    mark_non_differentiable = set_materialize_grads = save_for_backward
+
+
+def _apply(function, tensors, *args):
+    """``function.apply(*args)``.  With gradients switched off an eager call on ordinary tensors has nothing to record or to
+    transform, and goes to the forward itself (6 us of host time less; ``tensors``: those among ``args``)."""
+    if not torch.is_grad_enabled() and ops.ordinary(*tensors):
+        return function.forward(_NoNode(), *args)
+    return function.apply(*args)
+
+
 class DSADotProductAttentionFunction(torch.autograd.Function):
     """Sparse MLA attention over the selected latent rows (forward and backward on the HIP kernels).
 
@@ -199,9 +216,9 @@ class DSADotProductAttention(MegatronModule):
         d_qk = query.size(-1)
         d_v = self.config.v_head_dim if d_qk == self.config.v_head_dim else self.config.kv_lora_rank
 
-        res = DSADotProductAttentionFunction.apply(query, kv, indices, chunk_offset, self.softmax_scale, d_v,
-                                                   return_p_out, packed_seq_params, topk_length, attn_sink,
-                                                   window_size, True, int(return_attn_dist))
+        res = _apply(DSADotProductAttentionFunction, (query, kv, indices, topk_length, attn_sink), query, kv, indices, chunk_offset,
+                     self.softmax_scale, d_v, return_p_out, packed_seq_params, topk_length, attn_sink, window_size, True,
+                     int(return_attn_dist))
         core_attn_out, p_out = (res if (return_p_out or return_attn_dist) else (res, None))
         if qkv_format == "thd":
             core_attn_out = core_attn_out.squeeze(0).contiguous()
@@ -264,8 +281,21 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
             return (_pad_to(_pad_to(index_q.to(torch.bfloat16), 128, 2), head_p, 1).contiguous(),
                     _pad_to(index_k.to(torch.bfloat16), 128, 1).contiguous())
 
-        k_p = None
-        if front is None and not rotate and (head != head_p or dim != 128) and ops.ordinary(index_q, index_k, weights):
+        cu = None
+        if packed_seq_params is not None:
+            cu = packed_seq_params.cu_seqlens_kv_padded
+            if cu is None:
+                cu = packed_seq_params.cu_seqlens_kv
+        sort = DSAIndexerKernelFunction.sorted_output
+        k_p = topk_indices = None
+        whole = ops.indexer_forward(index_q, index_k, weights, rotate, softmax_scale, cu, chunk_offset, index_topk, sort, front,
+                                    k_norm_weight if front is not None else None, k_norm_bias if front is not None else None)
+        if whole is not None:
+            index_score_topk, topk_indices, q_fp8, q_scale, weight_scaled, k_fp8, k_scale, covered = whole
+            k_p = index_k.contiguous()
+            if covered is not None:
+                covered.wait()
+        elif front is None and not rotate and (head != head_p or dim != 128) and ops.ordinary(index_q, index_k, weights):
             q_fp8, q_scale, weight_scaled = ops.quant_padded_e4m3(index_q, head_p, weights, softmax_scale)
             k_fp8, k_scale, _ = ops.quant_padded_e4m3(index_k.unsqueeze(1), 1)
             k_fp8, k_scale = k_fp8.squeeze(1), k_scale.squeeze(1)
@@ -288,15 +318,10 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
                 k_p, 1, k_norm_weight, k_norm_bias, front.k_norm_eps, front.cos, front.sin, front.pairing,
                 front.positions_k, front.batch, rotate)
 
-        cu = None
-        if packed_seq_params is not None:
-            cu = packed_seq_params.cu_seqlens_kv_padded
-            if cu is None:
-                cu = packed_seq_params.cu_seqlens_kv
-        k_start, k_end, covered = ops.indexer_window(cu, seq_q, chunk_offset, q_fp8)
-        index_score_topk, topk_indices = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start, k_end,
-                                                          index_topk, DSAIndexerKernelFunction.sorted_output)
-        covered.wait()
+        if topk_indices is None:
+            k_start, k_end, covered = ops.indexer_window(cu, seq_q, chunk_offset, q_fp8)
+            index_score_topk, topk_indices = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start, k_end, index_topk, sort)
+            covered.wait()
         ctx.softmax_scale = softmax_scale
         ctx.rotate = rotate
         ctx.index_topk = index_topk
@@ -355,8 +380,8 @@ class DSAIndexerKernel(torch.nn.Module):
         """``front`` (an extension, :class:`IndexerFrontEnd`): ``index_q`` / ``index_k`` are the outputs of the
         projections and the key LayerNorm (``k_norm_weight``, ``k_norm_bias``), the rotary embedding and the rotation
         run inside the quantiser kernels."""
-        return DSAIndexerKernelFunction.apply(index_q, index_k, weights, index_topk, chunk_offset, packed_seq_params,
-                                              rotate, front, k_norm_weight, k_norm_bias)
+        return _apply(DSAIndexerKernelFunction, (index_q, index_k, weights, k_norm_weight, k_norm_bias), index_q, index_k, weights,
+                      index_topk, chunk_offset, packed_seq_params, rotate, front, k_norm_weight, k_norm_bias)
 
 
 # ---------------------------------------------------------------------------------------------------
@@ -611,5 +636,11 @@ def fused_apply_mla_rope_for_absorb_kv(kv, k_pos_emb, cos, sin, emb_dim: int, k_
                                        cp_rank: int = 0, cp_size: int = 1, rotary_interleaved: bool = False):
     """Key rows of the absorbed MLA form: copy of ``kv`` plus the rotated, head-shared ``k_pos_emb``
     (reference: dsa_fused_kernels.py:1796-1841)."""
+    if not (torch.compiler.is_compiling() or (torch.is_grad_enabled() and (kv.requires_grad or k_pos_emb.requires_grad))) and kv.shape[-1] == k_dim:
+        packed = cu_seqlens_kv is not None
+        positions = _token_positions(cu_seqlens_kv, kv.shape[0], cp_rank, cp_size) if packed else None
+        key = ops.absorbed_key(kv, k_pos_emb, cos, sin, positions, emb_dim, packed, ops.ROPE_ADJACENT if rotary_interleaved else ops.ROPE_SPLIT)
+        if key is not None:
+            return key
     return ApplyMLARotaryEmbAbsorbKV.apply(kv, k_pos_emb, cos, sin, emb_dim, k_dim, cu_seqlens_kv, cp_rank, cp_size,
                                            rotary_interleaved)

@@ -398,6 +398,19 @@ def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offse
     return _native().indexer_window(cu_seqlens, int(queries), int(chunk_offset), like)
 
 
+def indexer_forward(index_q, index_k, weights, rotate: bool, factor: float, cu_seqlens, chunk_offset: int, K: int, sorted: bool, front=None,
+                    ln_weight=None, ln_bias=None):
+    """Quantisers (with ``front``, an ``IndexerFrontEnd``, behind the front end), :func:`indexer_window` and :func:`indexer_topk` of bf16
+    ``index_q [S, 32 or 64, 128]`` and ``index_k [Sk, 128]`` in one native call: (scores, ids, q8, q_scale, scaled weights, k8,
+    k_scale, check or None); None for other arguments and for calls that are not eager ones on ordinary tensors."""
+    if torch.compiler.is_compiling():
+        return None
+    f = front
+    return _native().indexer_forward(index_q, index_k, weights, bool(rotate), float(factor), cu_seqlens, int(chunk_offset), int(K), bool(sorted),
+                                     f and f.cos, f and f.sin, f.pairing if f else -1, f and f.positions_q, f and f.positions_k,
+                                     f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0)
+
+
 # --------------------------------------------------------------------------------------------
 # sparse MLA
 # --------------------------------------------------------------------------------------------
@@ -770,6 +783,12 @@ def absorbed_query(q_up, w, cos, sin, positions, out_pairing: int):
     """:func:`absorb_rope_query_into` over ``q_up [.., H, 192]`` into a new ``[.., H, 576]``; None if that needs autograd or
     the widths are others."""
     return _native().absorbed_query(q_up, w, cos, sin, positions, int(out_pairing))
+
+
+def absorbed_key(kv, k_pos_emb, cos, sin, positions, emb_dim: int, packed: bool, out_pairing: int):
+    """``cat(kv, rope(k_pos_emb))`` over the heads of ``kv [s, b, h, d]`` (``packed``: ``[t, h, d]``) as a new tensor; None if that needs
+    autograd, or for layouts and widths that are looked at one by one elsewhere."""
+    return _native().absorbed_key(kv, k_pos_emb, cos, sin, positions, int(emb_dim), bool(packed), int(out_pairing))
 
 
 def absorb_flat(a, w):

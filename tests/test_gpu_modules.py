@@ -323,3 +323,83 @@ def test_chunkpipe_chunks_through_the_kernels_match_the_whole_sequence(gpu):
         scale = pw.grad.abs().max().item()
         err = (pc.grad / C - pw.grad).abs().max().item()
         assert err <= 2e-2 * scale, "%s: %.3e against %.3e" % (n, err, scale)
+
+
+@pytest.mark.parametrize("case", ["rotate", "plain", "packed", "packed_host", "front"])
+def test_indexer_forward_in_one_call_is_that_of_the_separate_calls(gpu, case, monkeypatch):
+    """Quantisers, key windows and selection issued by one native call: the same bits, saved tensors and gradients as step by step,
+    with gradients recorded and without."""
+    from loongforge_amd import dsa_fused_kernels as K, ops
+    from loongforge_amd.megatron_compat import PackedSeqParams
+
+    S, off = 70, 0 if case.startswith("packed") else 130
+    Sk = S + off
+    g = torch.Generator().manual_seed(3)
+    q, k, w = (torch.randn(*s, generator=g).to(gpu, torch.bfloat16) for s in ((S, 32, 128), (Sk, 128), (S, 32)))
+    packed, front, ln = None, None, (None, None)
+    if case.startswith("packed"):
+        cu = torch.tensor([0, 9, 9, 41, 70], dtype=torch.int32, device="cpu" if case == "packed_host" else gpu)
+        packed = PackedSeqParams(qkv_format="thd", cu_seqlens_q=cu, cu_seqlens_kv=cu, max_seqlen_q=32, max_seqlen_kv=32)
+    if case == "front":
+        ang = torch.rand(Sk, 64, generator=g).to(gpu)
+        ln = (torch.rand(128, generator=g).to(gpu), torch.rand(128, generator=g).to(gpu))
+        front = K.IndexerFrontEnd(cos=ang.cos(), sin=ang.sin(), pairing=ops.ROPE_SPLIT)
+    kern, rotate = K.DSAIndexerKernel(), case != "plain"
+
+    def both(record):
+        leaves = [t.clone().requires_grad_(record) for t in (q, k, w) + tuple(x for x in ln if x is not None)]
+        with torch.set_grad_enabled(record):
+            s, i = kern(leaves[0], leaves[1], leaves[2], 64, off, packed, rotate, front, *(leaves[3:] or (None, None)))
+        grads = torch.autograd.grad(s, leaves, torch.where(i >= 0, torch.ones_like(s), torch.zeros_like(s))) if record else ()
+        return (s, i) + tuple(grads)
+
+    whole = [both(r) for r in (False, True)]
+    monkeypatch.setattr(ops, "indexer_forward", lambda *a, **k: None)
+    steps = both(True)
+    assert all(torch.equal(a, b) for res in whole for a, b in zip(res, steps))
+    if packed is not None:
+        monkeypatch.undo()
+        short = PackedSeqParams(qkv_format="thd", cu_seqlens_q=packed.cu_seqlens_q[:4], cu_seqlens_kv=packed.cu_seqlens_kv[:4],
+                                max_seqlen_q=32, max_seqlen_kv=32)
+        with torch.no_grad(), pytest.raises(ValueError, match="packed sequences"):
+            kern(q, k, w, 64, 0, short, True)
+
+
+@pytest.mark.parametrize("shape,interleaved", [((5, 2, 3), False), ((1, 1, 1), True), ((7,), False)])
+def test_absorbed_key_without_gradients_is_that_of_the_autograd_function(gpu, shape, interleaved):
+    """Also for strided inputs, which the one native call leaves to the autograd function."""
+    from loongforge_amd import dsa_fused_kernels as K, ops
+
+    packed = len(shape) == 1
+    lead, heads = (shape, 2) if packed else (shape[:2], shape[2])
+    kv = torch.randn(*lead, heads, 512, device=gpu).to(torch.bfloat16)
+    pe = torch.randn(*lead, 1, 64, device=gpu).to(torch.bfloat16)
+    ang = torch.rand(8, 1, 1, 64, device=gpu)
+    cu = torch.tensor([0, 3, 7], dtype=torch.int32, device=gpu) if packed else None
+    args = (ang.cos().contiguous(), ang.sin().contiguous(), 64, 512, cu, 0, 1, interleaved)
+    want = K.fused_apply_mla_rope_for_absorb_kv(kv.clone().requires_grad_(True), pe, *args)
+    wide = torch.cat([kv, kv], -1)[..., :512]
+    with torch.no_grad():
+        for x in (kv, wide) if packed else (kv,):
+            assert torch.equal(K.fused_apply_mla_rope_for_absorb_kv(x, pe, *args), want)
+    with pytest.raises((AssertionError, RuntimeError)):
+        with torch.no_grad():
+            K.fused_apply_mla_rope_for_absorb_kv(kv, pe, ang.cos(), ang.sin()[:, :, :, ::2], 64, 512, cu, 0, 1, interleaved)
+
+
+def test_calls_that_are_not_eager_take_the_functions(gpu):
+    """Under a transform, a dispatch mode or a trace the native calls do nothing."""
+    from torch._subclasses import FakeTensorMode
+
+    from loongforge_amd import ops
+
+    mk = lambda: (torch.zeros(4, 32, 128, device=gpu, dtype=torch.bfloat16), torch.zeros(9, 128, device=gpu, dtype=torch.bfloat16),     # noqa: E731
+                  torch.zeros(4, 32, device=gpu))
+    q, k, w = mk()
+    assert ops.indexer_forward(q, k, w, True, 1.0, None, 0, 64, True) is not None
+    assert ops.indexer_forward(q.requires_grad_(True), k, w, True, 1.0, None, 0, 64, True) is None
+    with FakeTensorMode():
+        assert ops.indexer_forward(*mk(), True, 1.0, None, 0, 64, True) is None
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(ops.indexer_forward(x, k, w, True, 1.0, None, 0, 64, True)), x)[1])(torch.stack([q.detach(), q.detach()]))
+    assert seen == [None]
