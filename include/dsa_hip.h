@@ -270,6 +270,15 @@ int dsa_sparse_mla_fwd_block(const void* q, const void* kv, const int32_t* ids, 
                              int p_out_f32, const float* attn_sink, int p_out_skip,
                              void* workspace, size_t workspace_bytes, void* stream);
 /*
+ * dsa_sparse_mla_fwd_block together with the head-averaged attention distribution over the slots, target [S, K] f32: the mean over
+ * the first dist_heads heads of the softmax of the forward's bf16 logits, bit for bit dsa_attn_dist of them (K <= 4096).  The
+ * logits pass through `logits` [S, H, K] bf16, whose contents are undefined afterwards: tiles of 32 slots without a valid one
+ * are neither written nor read.
+ */
+int dsa_sparse_mla_fwd_dist(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv, int K,
+                            int q_start, float sm_scale, int d_v, void* out, float* lse, const float* attn_sink,
+                            int dist_heads, float* target, void* logits, void* workspace, size_t workspace_bytes, void* stream);
+/*
  * How the forward goes about a call of these sizes, for tests and measurements: the form (0: one workgroup in two wave roles
  * for all heads, 1 / 2: 64 / 32 heads, two tiles at a time, 3 / 4: 64 / 32 heads, two workgroups on a compute unit), and in
  * *ranges (may be NULL) over how many workgroups it spreads a query's slots.  -1 for sizes that the forward does not take.

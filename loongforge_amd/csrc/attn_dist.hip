@@ -72,13 +72,40 @@ __global__ __launch_bounds__(256) void attn_dist_kernel(const void* __restrict__
 // maximum is taken on the raw logits).  Logits beyond the memory-side cache are read with the non-temporal hint
 // (STREAMED; [8192, 128, 2048] bf16: 0.79 -> 0.76 ms, 5.7 TB/s; 0.1 - 0.2 GB, still cached from the forward that wrote
 // them, read no faster with it).
-template <bool F32, int NC, bool STREAMED>
+// LIVE: the ids of the slots are given, and of the 32-slot tiles without a valid one (0 <= id < min(Skv, q_start + i + 1)) the logits
+// have not been written.  They are -inf without being read: short documents and prefixes then cost what their slots cost.  With the
+// forward that writes them, us: [912, 128, 1024] of five documents 132 + 59 -> 85 + 36, [1091, 128, 2048] 307 + 146 -> 230 + 89, [871, 64,
+// 2048] of five 86 + 46 -> 41 + 22, [8192, 128, 2048] 3843 + 756 -> 3758 + 706; full lists the same.
+template <bool F32, int NC, bool STREAMED, bool LIVE>
 __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restrict__ p_out, int H, int K,
                                                             int64_t ld_s, int64_t ld_h, float c2,
-                                                            float* __restrict__ target) {
+                                                            float* __restrict__ target, const int* __restrict__ ids, int Skv, int q_start) {
   extern __shared__ float acc_s[];            // [4 waves][K]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t i = blockIdx.x;
+  bool has[NC];                               // the lane's slots of chunk v have logits
+  int chunks = NC;                            // chunks in front of the last one that any lane has
+  if constexpr (LIVE) {
+    const int last = min((int64_t)Skv - 1, (int64_t)q_start + i);
+    chunks = 0;
+    int4 a[NC], b[NC];
+#pragma unroll
+    for (int v = 0; v < NC; v++) {
+      const int t = min(8 * (v * 64 + lane), K - 8);
+      a[v] = *(const int4*)(ids + i * K + t);
+      b[v] = *(const int4*)(ids + i * K + t + 4);
+    }
+#pragma unroll
+    for (int v = 0; v < NC; v++) {
+      const int id[8] = {a[v].x, a[v].y, a[v].z, a[v].w, b[v].x, b[v].y, b[v].z, b[v].w};
+      bool any = false;
+#pragma unroll
+      for (int e = 0; e < 8; e++) any |= id[e] >= 0 && id[e] <= last;
+      const unsigned long long m = __ballot(any && 8 * (v * 64 + lane) < K);
+      has[v] = (m >> (lane & ~3)) & 0xfull;   // four lanes share a tile
+      if (m) chunks = v + 1;
+    }
+  }
   float acc[NC][8];
 #pragma unroll
   for (int v = 0; v < NC; v++)
@@ -95,7 +122,7 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
 #pragma unroll
     for (int v = 0; v < NC; v++) {
       const int t = 8 * (v * 64 + lane);
-      if (t < K && h < H) {
+      if (t < K && h < H && (!LIVE || has[v])) {
         if (F32) {
           r.a[v] = piece((const float*)p_out + base + t);
           r.b[v] = piece((const float*)p_out + base + t + 4);
@@ -111,8 +138,9 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < NC; v++) {
+      if (LIVE && v >= chunks) break;
       const int t = 8 * (v * 64 + lane);
-      if (t < K) {
+      if (t < K && (!LIVE || has[v])) {
         if (F32) {
           const unsigned w[8] = {cur.a[v].x, cur.a[v].y, cur.a[v].z, cur.a[v].w, cur.b[v].x, cur.b[v].y, cur.b[v].z, cur.b[v].w};
 #pragma unroll
@@ -138,15 +166,19 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
     const float off = -mx * c2;
     float sum = 0.f;
 #pragma unroll
-    for (int v = 0; v < NC; v++)
+    for (int v = 0; v < NC; v++) {
+      if (LIVE && v >= chunks) break;
 #pragma unroll
       for (int e = 0; e < 8; e++) { z[v][e] = __builtin_amdgcn_exp2f(fmaf(z[v][e], c2, off)); sum += z[v][e]; }
+    }
     sum = wave_sum(sum);
     const float inv = 1.0f / sum;
 #pragma unroll
-    for (int v = 0; v < NC; v++)
+    for (int v = 0; v < NC; v++) {
+      if (LIVE && v >= chunks) break;
 #pragma unroll
       for (int e = 0; e < 8; e++) acc[v][e] += z[v][e] * inv;
+    }
   };
   // two buffers take turns (no register copies): while one head is worked on, the next is on its way
   Raw r0, r1;
@@ -173,24 +205,34 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
     target[i * K + t] = ((acc_s[t] + acc_s[K + t]) + (acc_s[2 * K + t] + acc_s[3 * K + t])) * invh;
 }
 
+// ids: null, or those whose dead tiles have no logits
 template <bool F32>
-int launch(const void* p_out, int S, int H, int K, int64_t ld_s, int64_t ld_h, float sm_scale, float* target,
-           hipStream_t st) {
+int launch(const void* p_out, int S, int H, int K, int64_t ld_s, int64_t ld_h, float sm_scale, float* target, const int* ids, int Skv,
+           int q_start, hipStream_t st) {
   const float c2 = sm_scale * 1.4426950408889634f;
   size_t smem = (size_t)4 * K * sizeof(float);
   const bool vec = K % 8 == 0 && ld_s % 8 == 0 && ld_h % 8 == 0 && ((uintptr_t)p_out % 32) == 0 && c2 > 0.f;
   if (vec) {
     const int nc = (K + 511) / 512;
     const bool streamed = (int64_t)S * H * K * (F32 ? 4 : 2) > (256ll << 20);
+#define DSA_ADV_LAUNCH(N, STR, LIVE) \
+    attn_dist_vec_kernel<F32, N, STR, LIVE><<<dim3(S), dim3(256), smem, st>>>(p_out, H, K, ld_s, ld_h, c2, target, ids, Skv, q_start)
 #define DSA_ADV_CASE(N) \
     if (nc <= N) { \
-      if (streamed) attn_dist_vec_kernel<F32, N, true><<<dim3(S), dim3(256), smem, st>>>(p_out, H, K, ld_s, ld_h, c2, target); \
-      else attn_dist_vec_kernel<F32, N, false><<<dim3(S), dim3(256), smem, st>>>(p_out, H, K, ld_s, ld_h, c2, target); \
+      if constexpr (!F32) { \
+        if (ids) { \
+          if (streamed) DSA_ADV_LAUNCH(N, true, true); else DSA_ADV_LAUNCH(N, false, true); \
+          return 0; \
+        } \
+      } \
+      if (streamed) DSA_ADV_LAUNCH(N, true, false); else DSA_ADV_LAUNCH(N, false, false); \
       return 0; \
     }
     DSA_ADV_CASE(1) DSA_ADV_CASE(2) DSA_ADV_CASE(4) DSA_ADV_CASE(8)
 #undef DSA_ADV_CASE
+#undef DSA_ADV_LAUNCH
   }
+  if (ids) return -1;
   int nv = (K + 63) / 64;
 #define DSA_AD_CASE(N) \
   if (nv <= N) { attn_dist_kernel<F32, N><<<dim3(S), dim3(256), smem, st>>>(p_out, H, K, ld_s, ld_h, c2, target); return 0; }
@@ -207,9 +249,15 @@ extern "C" int dsa_attn_dist(const void* p_out, int p_out_f32, int S, int H, int
   DSA_REQUIRE(K <= 64 * MAXV, "dsa_attn_dist: K=%d exceeds the supported maximum %d", K, 64 * MAXV);
   DSA_REQUIRE(ld_h >= K && ld_s >= ld_h, "dsa_attn_dist: bad strides");
   if (S == 0) return DSA_OK;
-  int rc = p_out_f32 ? launch<true>(p_out, S, H, K, ld_s, ld_h, sm_scale, target, (hipStream_t)stream)
-                     : launch<false>(p_out, S, H, K, ld_s, ld_h, sm_scale, target, (hipStream_t)stream);
+  int rc = p_out_f32 ? launch<true>(p_out, S, H, K, ld_s, ld_h, sm_scale, target, nullptr, 0, 0, (hipStream_t)stream)
+                     : launch<false>(p_out, S, H, K, ld_s, ld_h, sm_scale, target, nullptr, 0, 0, (hipStream_t)stream);
   DSA_REQUIRE(rc == 0, "dsa_attn_dist: unsupported K");
   DSA_CHECK_LAUNCH("dsa_attn_dist");
   return DSA_OK;
+}
+
+// Of logits [S, heads of ld_s / K, K] whose tiles without a valid slot have not been written (K % 64 == 0, 32-byte aligned, sm_scale > 0)
+int dsa_attn_dist_live(const void* logits, const int32_t* ids, int S, int H, int Skv, int K, int64_t ld_s, int q_start, float sm_scale,
+                       float* target, hipStream_t st) {
+  return launch<false>(logits, S, H, K, ld_s, K, sm_scale, target, ids, Skv, q_start, st);
 }

@@ -524,6 +524,34 @@ py::object mla_fwd(const Tensor& q_, const Tensor& kv_, const Tensor& ids_, int6
   return py::make_tuple(out, lse, p_out);
 }
 
+// The forward with the head-averaged distribution, `block` queries' logits at a time
+py::object mla_fwd_dist(const Tensor& q_, const Tensor& kv_, const Tensor& ids_, int64_t q_start, double sm_scale, int64_t d_v, int64_t dist_heads,
+                        int64_t block, const OptTensor& attn_sink, bool force) {
+  PLAIN_OR_NONE(q_, kv_, ids_, attn_sink);
+  mla_shape(q_, kv_, ids_);
+  const Tensor q = q_.contiguous(), kv = kv_.contiguous(), ids = i32(ids_);
+  const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);
+  OptTensor sink;
+  if (attn_sink) {
+    need_gpus(q, attn_sink);
+    REQUIRE(attn_sink->numel() == H, "attn_sink must hold one logit per head (", H, "), got ", attn_sink->numel());
+    sink = f32(attn_sink->reshape({H}));
+  }
+  Call call(q);
+  Tensor out = make({S, H, d_v}, at::kBFloat16, q), lse = make({S, H}, at::kFloat, q), dist = make({S, K}, at::kFloat, q);
+  block = std::max<int64_t>(1, std::min(block, S));
+  Tensor logits = make({block, H, K}, at::kBFloat16, q);
+  const size_t nbytes = dsa_sparse_mla_fwd_block_workspace_bytes((int)S, (int)block, (int)H, (int)Skv, (int)K);
+  Tensor ws;
+  if (nbytes) ws = make({(int64_t)nbytes}, at::kByte, q);
+  for (int64_t s0 = 0; s0 < S; s0 += block)
+    run("dsa_sparse_mla_fwd_dist", dsa_sparse_mla_fwd_dist, (const char*)q.const_data_ptr() + s0 * H * 576 * 2, kv.const_data_ptr(),
+        (const int32_t*)ids.const_data_ptr() + s0 * K, (int)S, (int)std::min(block, S - s0), (int)H, (int)Skv, (int)K, (int)(q_start + s0),
+        (float)sm_scale, (int)d_v, (char*)out.data_ptr() + s0 * H * d_v * 2, (float*)lse.data_ptr() + s0 * H, (const float*)ptr(sink),
+        (int)dist_heads, (float*)dist.data_ptr() + s0 * K, logits.data_ptr(), nbytes ? ws.data_ptr() : nullptr, nbytes, call.stream);
+  return py::make_tuple(out, lse, dist);
+}
+
 py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, const Tensor& dout_, const Tensor& ids_, const Tensor& lse_,
                    int64_t q_start, double sm_scale, int64_t d_v, const py::function& workspace, bool force) {
   PLAIN_OR_NONE(q_, kv_, out_, dout_, ids_, lse_);
@@ -720,6 +748,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(indexer_bwd);
   DEF(indexer_grads);
   DEF(mla_fwd);
+  DEF(mla_fwd_dist);
   DEF(mla_bwd);
   DEF(attn_dist);
   DEF(kl_loss);

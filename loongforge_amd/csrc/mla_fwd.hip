@@ -27,6 +27,10 @@
 // compute units idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
 #include "mla_tile.h"
 
+// attn_dist.hip
+int dsa_attn_dist_live(const void* logits, const int32_t* ids, int S, int H, int Skv, int K, int64_t ld_s, int q_start, float sm_scale,
+                       float* target, hipStream_t st);
+
 namespace {
 using namespace mla;
 
@@ -55,6 +59,7 @@ struct FwdArgs {
   float sm_scale;
   const float* sink;
   int p_skip;
+  bool p_all;                                // p_out: tiles without a valid slot are filled with -inf (else left as they are)
   int n_hg, ksplit, k_loc;                   // head groups per query, slot ranges per query, slots of a range
   int span;                                  // modes 1 - 4: neighbouring queries (ranges) on one XCD
   f32x4* part_o; float* part_ml;             // ksplit > 1: sums [S][ksplit][H/32][16][4][64] x 4, (m, l) [S][ksplit][H][2]
@@ -259,7 +264,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
 
   // slots of tiles that are never visited still need their -inf in p_out
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
-  if (POUT != 0 && head_ok && ntiles < NT) {
+  if (POUT != 0 && a.p_all && head_ok && ntiles < NT) {
     for (int t = 0; t < NT; t++) {
       if (tmask[t] != 0u || (tile0 + t) * BI < p_skip || (t & 1) != stream) continue;
       const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + t) * BI - p_skip) + 16 * g;
@@ -571,7 +576,7 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
     const int tile0 = k0 / BI, p_skip = a.p_skip;
     // slots of tiles that are never visited still need their -inf in p_out
     // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
-    if (POUT != 0 && head_ok && ntiles < NT) {
+    if (POUT != 0 && a.p_all && head_ok && ntiles < NT) {
       for (int t = 0; t < NT; t++) {
         if (tmask[t] != 0u || (tile0 + t) * BI < p_skip) continue;
         const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)((tile0 + t) * BI - p_skip) + 16 * g;
@@ -915,7 +920,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
 
   // slots of tiles that are never visited still need their -inf in p_out
   // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
-  if (POUT != 0 && head_ok && h0 == 0 && ntiles < NT) {
+  if (POUT != 0 && a.p_all && head_ok && h0 == 0 && ntiles < NT) {
     for (int t = 0; t < NT; t++) {
       if (tmask[t] != 0u || t * BI < p_skip) continue;
       const size_t pbase = ((size_t)qi * H + h) * (K - p_skip) + (size_t)(t * BI - p_skip) + 8 * kg;
@@ -1380,7 +1385,7 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, bool shared, hipStream_t st) {
 // and the way the ranges' sums are put together, so a query has the same bits in a block of any size.
 int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv, int K, int q_start, float sm_scale,
              int d_v, void* out, float* lse, void* p_out, int p_out_f32, const float* attn_sink, int p_out_skip,
-             void* workspace, size_t workspace_bytes, void* stream) {
+             void* workspace, size_t workspace_bytes, void* stream, bool p_all = true) {
   DSA_REQUIRE(d_v == DV, "dsa_sparse_mla_fwd: only d_v = 512 (d_qk = 576) is supported, got d_v = %d", d_v);
   DSA_REQUIRE(S >= 0 && Skv > 0, "dsa_sparse_mla_fwd: bad sequence sizes S=%d Skv=%d", S, Skv);
   DSA_REQUIRE(S_all >= S, "dsa_sparse_mla_fwd: a block of %d queries of %d", S, S_all);
@@ -1398,7 +1403,7 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S_all, int S
   FwdPlan p = plan_fwd(S_all, H, K, true);
   if (part_bytes(p, S, H) > workspace_bytes || (p.ksplit > 1 && workspace == nullptr)) p = plan_fwd(S_all, H, K, false);
   FwdArgs a{(const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, attn_sink,
-            p_out ? p_out_skip : 0, p.n_hg, p.ksplit, p.k_loc, unit_span(p, S), (f32x4*)workspace,
+            p_out ? p_out_skip : 0, p_all, p.n_hg, p.ksplit, p.k_loc, unit_span(p, S), (f32x4*)workspace,
             (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4)};
   int rc;
   const bool split = p.ksplit > 1, shared = combine_shares(S_all, H, p.ksplit);
@@ -1438,6 +1443,24 @@ extern "C" int dsa_sparse_mla_fwd_block(const void* q, const void* kv, const int
                                         size_t workspace_bytes, void* stream) {
   return fwd_impl(q, kv, ids, S_all, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, p_out, p_out_f32, attn_sink, p_out_skip,
                   workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsa_sparse_mla_fwd_dist(const void* q, const void* kv, const int32_t* ids, int S_all, int S, int H, int Skv, int K,
+                                       int q_start, float sm_scale, int d_v, void* out, float* lse, const float* attn_sink,
+                                       int dist_heads, float* target, void* logits, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+  DSA_REQUIRE(logits != nullptr && target != nullptr && dist_heads > 0 && dist_heads <= H, "dsa_sparse_mla_fwd_dist: bad arguments (%d of %d heads)", dist_heads, H);
+  DSA_REQUIRE(K <= 4096, "dsa_sparse_mla_fwd_dist: K=%d exceeds the supported maximum 4096", K);
+  // what the reduction does not read, the forward does not write: the tiles of short prefixes behind their last slot
+  const bool live = ((uintptr_t)logits % 32) == 0 && ((uintptr_t)ids % 16) == 0 && sm_scale > 0.f;
+  const int rc = fwd_impl(q, kv, ids, S_all, S, H, Skv, K, q_start, sm_scale, d_v, out, lse, logits, 0, attn_sink, 0, workspace,
+                          workspace_bytes, stream, !live);
+  if (rc != DSA_OK || S == 0) return rc;
+  if (!live) return dsa_attn_dist(logits, 0, S, dist_heads, K, (int64_t)H * K, K, sm_scale, target, stream);
+  DSA_REQUIRE(dsa_attn_dist_live(logits, ids, S, dist_heads, Skv, K, (int64_t)H * K, q_start, sm_scale, target, (hipStream_t)stream) == 0,
+              "dsa_sparse_mla_fwd_dist: unsupported K");
+  DSA_CHECK_LAUNCH("dsa_sparse_mla_fwd_dist");
+  return DSA_OK;
 }
 
 extern "C" int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv, int K,

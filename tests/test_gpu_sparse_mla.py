@@ -825,6 +825,45 @@ def test_forward_with_distribution_in_blocks_is_that_of_the_whole(gpu, S, H, K, 
             assert all(torch.equal(g, w) for g, w in zip(got, want)), n
 
 
+@pytest.mark.parametrize("form,ranges,S,H,K", MLA_FORMS)
+@pytest.mark.parametrize("misaligned", [False, True])
+def test_distribution_of_short_rows_reads_only_what_the_forward_wrote(gpu, form, ranges, S, H, K, misaligned):
+    """The passing logits of tiles without a valid slot are neither written nor read: with NaN in their place, rows that end early,
+    have holes of whole tiles or no slot at all give the distribution of the logits that the caller can ask for, bit for bit.
+    (A buffer that starts between two 32-byte pieces is written and read whole.)"""
+    from loongforge_amd import _lib, ops
+
+    assert mla_form(S, H, K) == (form, ranges)
+    inp = O.make_mla_inputs(S, H, K, seed=S, skv=K + S, q_start=K)
+    idx = inp.idx.clone()
+    for i in range(0, S, 2):
+        idx[i, (37 * i) % K:] = -1
+    idx[S // 2, :32] = -1
+    idx[S // 3] = K + S + 5                     # behind the keys
+    if S > 2:
+        idx[1, 32:] = K + 2                     # behind the query
+        idx[2, 5:] = -1
+    q, kv, ids = inp.q.to(gpu), inp.kv.to(gpu), idx.to(gpu)
+    out, lse, p_out = ops.sparse_mla_fwd(q, kv, ids, K, inp.sm_scale, 512, True)
+    heads = H - 3
+    want = ops.attn_dist(p_out[:, :heads], inp.sm_scale)
+    got = ops.sparse_mla_fwd_dist(q, kv, ids, K, inp.sm_scale, 512, heads, S)
+    assert torch.equal(got[0], out) and torch.equal(got[1], lse) and torch.equal(got[2], want)
+    lib = _lib.load()
+    off = 8 if misaligned else 0
+    logits = torch.full((S * H * K + 16,), float("nan"), dtype=torch.bfloat16, device=gpu)[off:]
+    out2, lse2, dist2 = torch.empty_like(out), torch.empty_like(lse), torch.full_like(want, float("nan"))
+    n = lib.dsa_sparse_mla_fwd_workspace_bytes(S, H, K + S, K)
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=gpu)
+    rc = lib.dsa_sparse_mla_fwd_dist(q.data_ptr(), kv.data_ptr(), ids.data_ptr(), S, S, H, K + S, K, K, inp.sm_scale, 512, out2.data_ptr(),
+                                     lse2.data_ptr(), None, heads, dist2.data_ptr(), logits.data_ptr(), ws.data_ptr(), n,
+                                     torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.dsa_last_error()
+    assert torch.equal(out2, out) and torch.equal(lse2, lse)
+    # (element by element the sums of a head are grouped differently: a few roundings of 2**-24 of values of one sign)
+    assert torch.equal(dist2, want) if not misaligned else torch.allclose(dist2, want, rtol=2e-6, atol=0)
+
+
 def test_attn_dist_from_q_kv_lse_with_sink_is_the_softmax_over_the_slots(gpu):
     from loongforge_amd import ops
 
