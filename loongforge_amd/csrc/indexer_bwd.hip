@@ -19,9 +19,11 @@
 //            converted in registers (exact); a as a bf16 pair (hi + lo), so the products lose nothing visible in fp32
 // No floating-point atomics: every sum has a fixed order.
 //
-// At 8192 queries x 2048 slots x 64 heads 1.31 ms: 0.20 for the queries' set-up and final sums, 0.85 for the loop without
-// its row stores (2048 matrix cycles of 3600 per tile and SIMD), the rest for the 3.8 GB of rows (4.4 TB/s where the row
-// waves run alone).  (2.54 ms for four waves, one per SIMD, that carried m a q_w through LDS as a bf16 pair: 48 transposing
+// At 8192 queries x 2048 slots x 64 heads 1.28 ms in a training pass: 0.85 for the loop without its row stores (2048 matrix cycles of
+// 3600 per tile and SIMD), most of the rest for the 3.8 GB of rows (4.4 TB/s where the row waves run alone).  The queries'
+// set-up and final sums run alone on their compute unit.  With the slots behind the query's rows, the first transfers behind the keys'
+// scales and weights, scales and angles of the final steps out of memory it took 1.45 ms (2077 x 512 x 32 heads 107 us and now 88,
+// 3072 x 512 compressed keys x 64 heads 169 and 147).  (2.54 ms for four waves, one per SIMD, that carried m a q_w through LDS as a bf16 pair: 48 transposing
 // reads and 40 writes per wave and tile.)  Rows written in slot order instead of scattered: the same; non-temporal: 2.9 ms.
 #include "dsa_common.h"
 #include "order.h"
@@ -72,7 +74,12 @@ struct RowFinish {
   int cs_f32, pairing, batch;            // pairing -1: no rotary part
 };
 
-__device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_inv, const RowFinish& f, const int* positions, int token) {
+__device__ __forceinline__ float table_entry(const void* t, int is_f32, long i) {
+  return is_f32 ? ((const float*)t)[i] : bf16_bits_to_f32(((const unsigned short*)t)[i]);
+}
+// cs: the token's 64 cosines and 64 sines where they are at hand already, else null
+__device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_inv, const RowFinish& f, const int* positions, int token,
+                                           const float* cs) {
   constexpr float FLOOR = 0x1.8p-48f;
   const bool usable = scale_inv > FLOOR && scale_inv < INFINITY;
 #pragma unroll
@@ -97,7 +104,7 @@ __device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_i
 #pragma clang fp contract(off)
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
-    const long pos = positions ? positions[token] : token / f.batch;
+    const long row = cs ? 0 : (positions ? positions[token] : token / f.batch) * 64l;
     // element e of a pair (a, b):  a' = a cos[e] + b sin[partner],  b' = b cos[e] - a sin[partner]
     float other[8];
     if (f.pairing == 1) {
@@ -109,12 +116,12 @@ __device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_i
     }
     if (sub < 8) {
       float c[8], s[8];
-      const long co = pos * 64 + sub * 8, so = f.pairing == 1 ? pos * 64 + (sub ^ 4) * 8 : co;
+      const long co = row + sub * 8, so = f.pairing == 1 ? row + (sub ^ 4) * 8 : co;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
         const int j = f.pairing == 1 ? i : i ^ 1;
-        c[i] = f.cs_f32 ? ((const float*)f.cos_t)[co + i] : bf16_bits_to_f32(((const unsigned short*)f.cos_t)[co + i]);
-        s[i] = f.cs_f32 ? ((const float*)f.sin_t)[so + j] : bf16_bits_to_f32(((const unsigned short*)f.sin_t)[so + j]);
+        c[i] = cs ? cs[co + i] : table_entry(f.cos_t, f.cs_f32, co + i);
+        s[i] = cs ? cs[64 + so + j] : table_entry(f.sin_t, f.cs_f32, so + j);
       }
 #pragma unroll
       for (int i = 0; i < 8; i++) {
@@ -176,11 +183,15 @@ struct BwdArgs {
 // store rows, whose transfers are awaited behind their stores, and two for the others: the same time.)
 int bwd_stages(int K) { return K <= 2048 ? 3 : 2; }
 
-size_t bwd_lds_bytes(int HI, int K) {
-  const size_t loop = (size_t)bwd_stages(K) * 8 * WAVE_BYTES + (size_t)HI * D + (size_t)K * 16 + 4 * 64 * 4 + 64 * 4 + 64;
+// What a workgroup needs to the end lies behind both the loop's arrays and the reduction buffers that take their place: weights [64],
+// scales [64], cosines and sines [2][64], last slot.
+constexpr size_t KEPT_BYTES = 4 * 64 * 4 + 64;
+__host__ __device__ constexpr size_t kept_offset(int HI, int stages, int K) {
+  const size_t loop = (size_t)stages * 8 * WAVE_BYTES + (size_t)HI * D + (size_t)K * 16;
   const size_t red = (size_t)4 * HI * RED_STRIDE * 4 + 4 * 64 * 4;
   return loop > red ? loop : red;
 }
+size_t bwd_lds_bytes(int HI, int K) { return kept_offset(HI, bwd_stages(K), K) + KEPT_BYTES; }
 
 // The waves share nothing inside the loop: each brings the 32 key rows of its slots into a ring of its own and there is no
 // barrier, so that one wave's vector work runs under the matrix work of the other wave of its SIMD.  The loop is bound by
@@ -191,16 +202,17 @@ template <int NHT, int STAGES>   // head tiles of 32
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void indexer_bwd_kernel(const BwdArgs A) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int HI = 32 * NHT;
-  // [8 waves][STAGES][WAVE_BYTES] fp8 key rows | q8 [HI][128] | a_s [K] f32 | ahl_s [K / 4][4 hi, 4 lo] bf16 | idx_s [K] | dst_s [K] |
-  // w_s [64] | last_s
+  // [8 waves][STAGES][WAVE_BYTES] fp8 key rows | q8 [HI][128] | a_s [K] f32 | ahl_s [K / 4][4 hi, 4 lo] bf16 | idx_s [K] | dst_s [K] ||
+  // w_s [64] | scale_s [64] | cs_s [2][64] | last_s
   unsigned char* qs = smem + 8 * STAGES * WAVE_BYTES;
   const int K = A.K;
   float* a_s = (float*)(qs + HI * D);
   unsigned short* ahl_s = (unsigned short*)(a_s + K);
   int* idx_s = (int*)(ahl_s + 2 * K);
   int* dst_s = idx_s + K;
-  float* w_s = (float*)(dst_s + K);
-  int* last_s = (int*)(w_s + 64);
+  float* w_s = (float*)(smem + kept_offset(HI, STAGES, K));
+  float *scale_s = w_s + 64, *cs_s = w_s + 128;
+  int* last_s = (int*)(w_s + 256);
   float* dw_red = (float*)smem;                     // [4][64], then red [4][HI][RED_STRIDE], reuse the front at the end
   float* red = dw_red + 4 * 64;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -210,45 +222,57 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const int ql = A.cnt - 1 - (int)blockIdx.x;
   const int qi = A.q0 + ql;
 
-  // ---- the query: slots, rows, weights ----------------------------------------------------------
+  // ---- the query: slots, rows, weights.  Nothing else runs on the compute unit meanwhile, so the chain of round trips to memory is
+  // kept short: the slots, the query's rows and weights in one, then the first key rows beside the keys' scales. --------------
   if (tid == 0) *last_s = -1;
   const unsigned char* qrow = A.q8 + (size_t)qi * HI * D;
-  if (tid < HI) w_s[tid] = A.q_w[(size_t)qi * HI + tid];
-  if (tid < HI * 8) *(uint4*)(qs + (tid >> 3) * D + (((tid & 7) ^ slot_xor(tid >> 3)) << 4)) = *(const uint4*)(qrow + tid * 16);
-  __syncthreads();
-  int last = -1;
-  for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {   // four slots per thread with all their loads in flight
-    int v[4], d[4];
-    float gv[4], kv[4];
+  const int* ids = A.ids + (size_t)qi * K;
+  const float* gsc = A.gsc + (size_t)qi * K;
+  const int* dst = A.dst + (size_t)ql * K;
+  int v[4], d[4];
+  float gv[4];
+  auto request_slots = [&](int t0) {                // four slots per thread with all their loads in flight
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int t = min(t0 + i * THREADS, K - 1);
-      v[i] = A.ids[(size_t)qi * K + t];
-      gv[i] = A.gsc[(size_t)qi * K + t];
-      d[i] = A.dst[(size_t)ql * K + t];
+      v[i] = ids[t];
+      gv[i] = gsc[t];
+      d[i] = dst[t];
     }
+  };
+  request_slots(tid);
+  const float w_in = A.q_w[(size_t)qi * HI + min(tid, HI - 1)];
+  const float scale_in = A.q_scale ? A.q_scale[(size_t)qi * HI + min(tid, HI - 1)] : 0.f;
+  const bool rotary = A.q_scale != nullptr && A.fin.pairing >= 0;
+  const long pos = !rotary ? 0 : A.pos_q ? A.pos_q[qi] : qi / A.fin.batch;
+  const uint4 q_in = *(const uint4*)(qrow + min(tid, HI * 8 - 1) * 16);
+  __builtin_amdgcn_sched_barrier(0);
+  int last = -1;
+  for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {   // ids first: the transfers of key rows want nothing else
+    if (t0 != tid) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) kv[i] = A.k_scale[(v[i] >= 0 && v[i] < A.Sk) ? v[i] : 0];
+      for (int i = 0; i < 4; i++) v[i] = ids[min(t0 + i * THREADS, K - 1)];
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int t = t0 + i * THREADS;
+      const bool ok = v[i] >= 0 && v[i] < A.Sk;
       if (t < K) {
-        const bool ok = v[i] >= 0 && v[i] < A.Sk;
-        const float a = ok ? gv[i] * kv[i] : 0.f;
-        const unsigned short hi = f32_to_bf16_bits(a);
         idx_s[t] = ok ? v[i] : 0;
-        a_s[t] = a;
-        ahl_s[(t >> 2) * 8 + (t & 3)] = hi;
-        ahl_s[(t >> 2) * 8 + 4 + (t & 3)] = f32_to_bf16_bits(a - bf16_bits_to_f32(hi));
-        dst_s[t] = (ok && d[i] >= 0) ? d[i] : A.dummy_row;
         if (ok) last = t;
       }
     }
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) last = max(last, __shfl_xor(last, o, 64));
+  __syncthreads();                                  // *last_s has been set
   if (lane == 0) atomicMax(last_s, last);
-  DSA_WAIT_VMCNT(0);
+  if (tid < HI) {
+    w_s[tid] = w_in;
+    scale_s[tid] = scale_in;
+  }
+  if (tid < HI * 8) *(uint4*)(qs + (tid >> 3) * D + (((tid & 7) ^ slot_xor(tid >> 3)) << 4)) = q_in;
+  DSA_WAIT_VMCNT(0);                                // every load so far: what is in flight below are the transfers and the scales
   __syncthreads();
   const int ntile = (*last_s + TK) / TK;            // tiles behind the last valid slot have nothing to add
 
@@ -274,6 +298,30 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int c = 0; c < 4; c++) dma16(lb + c * 1024, (lds_read<unsigned>(ia + c * 32) << 7) | (g_off ^ (unsigned)((c & 1) * 64)), A.k8);
   };
   for (int n = 0; n < STAGES - 1 && n < ntile; n++) issue(n, n);
+  __builtin_amdgcn_sched_barrier(0);
+  // factors and destination rows of the slots and the token's angles, while the first key rows are on their way
+  const float cs_in = rotary && tid < 128 ? table_entry(tid < 64 ? A.fin.cos_t : A.fin.sin_t, A.fin.cs_f32, pos * 64 + (tid & 63)) : 0.f;
+  for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {
+    if (K > 4 * THREADS) request_slots(t0);
+    float kv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) kv[i] = A.k_scale[(v[i] >= 0 && v[i] < A.Sk) ? v[i] : 0];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int t = t0 + i * THREADS;
+      if (t < K) {
+        const bool ok = v[i] >= 0 && v[i] < A.Sk;
+        const float a = ok ? gv[i] * kv[i] : 0.f;
+        const unsigned short hi = f32_to_bf16_bits(a);
+        a_s[t] = a;
+        ahl_s[(t >> 2) * 8 + (t & 3)] = hi;
+        ahl_s[(t >> 2) * 8 + 4 + (t & 3)] = f32_to_bf16_bits(a - bf16_bits_to_f32(hi));
+        dst_s[t] = (ok && d[i] >= 0) ? d[i] : A.dummy_row;
+      }
+    }
+  }
+  if (tid < 128) cs_s[tid] = cs_in;
+  __syncthreads();
   auto key_rows = [&](unsigned stage_off, i32x8 (&bk)[2]) {
 #pragma unroll
     for (int s = 0; s < 2; s++) {
@@ -509,9 +557,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
 
   // ---- sums over the four slot groups, in a fixed order ----------------------------------------------
-  float w_row[NHT];          // (the weights' place in LDS is overwritten)
-#pragma unroll
-  for (int it = 0; it < NHT; it++) w_row[it] = A.q_w[(size_t)qi * HI + 32 * it + (tid >> 4)];
   __syncthreads();
   const int sub = tid & 15;
 #pragma unroll
@@ -524,12 +569,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
       for (int k = 0; k < 4; k++) p[k] = *(const f32x4*)(red + ((size_t)k * HI + h) * RED_STRIDE + 8 * sub + 4 * x);
 #pragma unroll
-      for (int e = 0; e < 4; e++) v[4 * x + e] = ((p[0][e] + p[1][e]) + (p[2][e] + p[3][e])) * w_row[it];
+      for (int e = 0; e < 4; e++) v[4 * x + e] = ((p[0][e] + p[1][e]) + (p[2][e] + p[3][e])) * w_s[h];
     }
     if (A.q_scale == nullptr) {
       store_row(v, A.d_q8, 1, (size_t)qi * HI + h, D, sub);
     } else {
-      finish_row(v, sub, A.q_scale[(size_t)qi * HI + h], A.fin, A.pos_q, qi);
+      finish_row(v, sub, scale_s[h], A.fin, nullptr, qi, cs_s);
       if (h < A.heads) store_row(v, A.d_q, A.q_f32, (size_t)qi * A.heads + h, A.dim, sub);
     }
   }
@@ -538,7 +583,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     if (A.q_scale == nullptr) {
       A.d_qw[(size_t)qi * HI + tid] = s;
     } else if (tid < A.heads) {
-      const float y = s * A.q_scale[(size_t)qi * HI + tid] * A.w_scale;
+      const float y = s * scale_s[tid] * A.w_scale;
       if (A.w_f32) ((float*)A.d_w)[(size_t)qi * A.heads + tid] = y;
       else ((unsigned short*)A.d_w)[(size_t)qi * A.heads + tid] = f32_to_bf16_bits(y);
     }
@@ -631,7 +676,7 @@ __global__ __launch_bounds__(256) void indexer_key_finish_kernel(const KeyArgs A
     const f32x4 p0 = *(const f32x4*)(A.d_k8 + (size_t)row * D + 8 * sub), p1 = *(const f32x4*)(A.d_k8 + (size_t)row * D + 8 * sub + 4);
 #pragma unroll
     for (int i = 0; i < 4; i++) { v[i] = p0[i]; v[4 + i] = p1[i]; }
-    finish_row(v, sub, A.k_scale[row], A.fin, A.positions, row);
+    finish_row(v, sub, A.k_scale[row], A.fin, A.positions, row, nullptr);
     if (A.k_in) {
       const uint4 raw = *(const uint4*)(A.k_in + (size_t)row * D + 8 * sub);
       const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
