@@ -1287,12 +1287,16 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // that follows.  The constants are measured times in us, random rows.  A round among others, FULL: the rows of all its queries come in
 // together, and the gathers of 256 workgroups share the fabric.  A single or last round, LAST: IDLE on an empty chip, and nearly that
 // while it is half empty, hence the square.  Modes 3 and 4 by whether workgroups share a compute unit; where few do, what they take
-// with keys that lie far apart.
+// with keys that lie far apart.  Those of single rounds and of the ranges are fitted to every form and number of ranges timed at 1300
+// sizes (1 - 1200 queries, 32 - 128 heads, 192 - 8192 slots, keys of one long sequence and of a sequence per query): the form that
+// the estimate picks takes 0.6 % more than the best one in the mean, 10 % at most (1.2 and 23 % with constants from a dozen sizes).  us,
+// before and after: 61 queries x 64 heads x 1024 slots 31.4 (one range) and 28.9 (two), 121 x 32 x 1024 42.7 and 37.9, 80 x 128 x 2048 83
+// (mode 1) and 73 (mode 0 in two ranges), 40 x 64 x 768 25.5 and 22.3 (three ranges), 250 x 64 x 512 35 (mode 1) and 31 (mode 3).
 // 2048 slots, 128 heads: one query 86 us in mode 0 and 15 as 64 workgroups of mode 2 in 16 ranges; 48 queries 90 in mode 0 and
 // 47 in mode 1 of two ranges; 128 queries 100 and 82 (mode 1), 160 queries 100 and 148, 600 queries 334 and 392.  64 heads: 256 queries
 // 94 us in mode 3 and 83 in mode 1, 300 queries 123 and 140, 3000 817 and 900; 513 - 738 queries, one
 // round of mode 3's 512 places and a short second one, are as fast in mode 1 (600 queries 218 and 216, with 65536 keys 243 and 256) and take it.
-// Mode 0 in ranges: up to 2048 slots it is the best form for 65 - 76 queries only (70 queries 65 us, mode 1 73); lists beyond what
+// Mode 0 in ranges: of up to 2048 slots for some 43 - 101 queries (70 queries 65 us, mode 1 73); lists beyond what
 // modes 1 and 2 hold (3840) have it up to some hundred queries: 100 queries x 4096 slots 121 us and 152 in mode 1 of two ranges, x 8192
 // 215 and 285 (303 in mode 0 undivided), 300 x 4096 357 and 391 (381).
 // 32 heads: 257 queries 78 us in mode 4 and 112 in mode 2, 800 queries 175 and 236.  4000 queries of 128 heads: 256 slots 440 us in
@@ -1300,10 +1304,10 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
 // mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
-  constexpr float REDO = 4.6f, COMBINE = 4.0f, COMBINE_RANGE = 0.25f, SHARED_RANGE = 0.12f, COMBINE_BYTES_PER_US = 6e6f;
-  constexpr float FIXED_IDLE = 6.0f, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
-  constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.6f, 1.3f, 2.7f, 2.2f};
-  constexpr float PAIR_LAST[3] = {3.65f, 2.15f, 1.65f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.3f, 2.05f};
+  constexpr float REDO = 4.6f, COMBINE = 2.37f, COMBINE_RANGE = 0.22f, SHARED_RANGE = 0.1f, COMBINE_BYTES_PER_US = 6.2e6f;
+  constexpr float FIXED_IDLE[5] = {4.91f, 5.86f, 4.51f, 5.57f, 3.8f}, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
+  constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.68f, 1.31f, 2.82f, 1.78f};
+  constexpr float PAIR_LAST[3] = {3.65f, 2.24f, 1.75f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.41f, 1.42f};
   constexpr int HEADS[5] = {128, 64, 32, 64, 32}, SLOTS[5] = {256, 256, 256, 512, 512};
   if (K <= 2 * BI) return {3, (H + HEADS[3] - 1) / HEADS[3], 1, K};
   const int pairs = K / (2 * BI);
@@ -1323,7 +1327,7 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const float pair = mode < 3      ? PAIR_IDLE[mode] + rest * rest * (PAIR_LAST[mode] - PAIR_IDLE[mode])
                          : rest > 0.5f ? PAIR_SHARED[mode] + 2.0f * (rest - 0.5f) * (PAIR_FULL[mode] - PAIR_SHARED[mode])
                                        : PAIR_IDLE[mode];
-      const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE;
+      const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE[mode];
       float t = (float)rounds * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += fixed + per * pair;
       t += ksplit == 1 ? (mode >= 2 ? 0.0f : REDO)
