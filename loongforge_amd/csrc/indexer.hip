@@ -9,11 +9,20 @@
 // sub-tile a wave issues, per group of 32 heads, two v_mfma_f32_32x32x64_f8f6f4 (A = the query's fp8
 // rows, held in registers for the whole sweep; B = key rows from LDS).  The accumulator layout puts
 // one key per lane and 16 heads per register file column, so the weighted ReLU-sum over heads is 2
-// VALU ops per element inside a lane plus one exchange between the two half-waves.  Per sub-tile
-// that is 4 MFMAs of 64 cycles against about 77 VALU issues of 4 cycles: the VALU port is the busier
-// of the two, and the matrix pipe of one wave overlaps the epilogue of the others, not its own -
-// hence the small register footprint and the high occupancy.  HBM is far from binding (q8 / k8 are
-// read once, logits written once).
+// VALU ops per element inside a lane plus one exchange between the two half-waves, which serves two
+// sub-tiles at a time.
+//
+// Per sub-tile of 64 heads that is 4 MFMAs of 64 cycles beside some 76 VALU issues of 4: both ports are
+// nearly equally busy, so a wave interleaves the products of one head group with the sums of the one
+// before, half a group at a time.  Left to the waves of a SIMD to overlap each other's phases, with masked stores that
+// every tile waited for and the windows read one after the other by each wave: 8192 queries x 64 heads 505 000
+// cycles (MFMA busy 52 %, both ports at once 34 %) and 300 us; as it is now 455 000 (58 and 44 %) and 275, at
+// the 1.7 GHz that the part's power leaves both.  us, before and after: 1500 queries behind 6692 keys 95.5
+// and 90, 3000 behind 5000 161 and 151, 2077 in four documents 18.2 and 16.5, 61 behind 20 000 18.0 and 16.2,
+// 48 unrelated windows of 7000 14.5 and 13.5; 32 heads, 5000 behind 500 82 and 80.5, 50 x 4 windows of 2500 8.5 and
+// 7.8.  HBM is far from binding (q8 / k8 are read once, logits written once).
+#include <type_traits>
+
 #include "dsa_common.h"
 
 namespace {
@@ -22,6 +31,7 @@ constexpr int D = 128;          // indexer head dim (bytes per fp8 row)
 constexpr int BK = 128;         // keys per LDS tile
 constexpr int TILE_BYTES = BK * D;
 constexpr int QB = 8;           // queries per workgroup
+constexpr unsigned NOWHERE = 0x40000000u;   // a store offset behind any row, also when added twice
 
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
@@ -47,27 +57,34 @@ __global__ void fill_neg_inf_kernel(float* __restrict__ p, long rows, long ld, i
     p[(e / width) * ld + (e % width)] = -INFINITY;
 }
 
-// sum of x over the two half-waves (lanes l and l ^ 32), in every lane.  v_permlane32_swap
-// exchanges the upper half of its first operand with the lower half of its second: afterwards one
-// register holds the lower-half values in both halves and the other the upper-half values.  (Written
-// as inline assembly: given the same value for both operands the compiler's builtin is folded as if
-// both results were equal.)
-__device__ __forceinline__ float add_halves(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-  return a + b;
+// Sums over the two half-waves (lanes l and l ^ 32): that of x in the lower half, that of y in the upper one.
+// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second: afterwards one
+// register holds the lower-half values and the other the upper-half values.  (Written as inline assembly: given the same
+// value for both operands the compiler's builtin is folded as if both results were equal.)
+__device__ __forceinline__ float add_pair(float x, float y) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+  return x + y;
+}
+__device__ __forceinline__ float add_halves(float x) { return add_pair(x, x); }
+
+__device__ __forceinline__ f32x16 mfma_fp8(const i32x8& a, const i32x8& b, const f32x16& acc) {
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, 0, 0, 0, 0, 0, 0);
+}
+
+// weighted ReLU-sum of heads [E, E + 8) of the 16 that a lane holds of a head group
+template <int E>
+__device__ __forceinline__ float weigh(const f32x16& acc, const float (&wq)[16], float sum) {
+#pragma unroll
+  for (int e = E; e < E + 8; e++) sum = fmaf(wq[e], relu1(acc[e]), sum);
+  return sum;
 }
 
 // 32 heads x 32 keys of fp8 products into the weighted ReLU-sum of a lane's key
 __device__ __forceinline__ float head_sum(const i32x8 (&aq)[2], const i32x8 (&bk)[2], const float (&wq)[16], float sum) {
-  f32x16 acc;
-#pragma unroll
-  for (int e = 0; e < 16; e++) acc[e] = 0.f;
-  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[0], bk[0], acc, 0, 0, 0, 127, 0, 127);
-  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[1], bk[1], acc, 0, 0, 0, 127, 0, 127);
-#pragma unroll
-  for (int e = 0; e < 16; e++) sum = fmaf(wq[e], relu1(acc[e]), sum);
-  return sum;
+  f32x16 acc = {};
+  acc = mfma_fp8(aq[0], bk[0], acc);
+  acc = mfma_fp8(aq[1], bk[1], acc);
+  return weigh<8>(acc, wq, weigh<0>(acc, wq, sum));
 }
 
 // a query's fp8 rows as the A operand, and the weights of the 16 heads a lane sees per head group
@@ -98,7 +115,8 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
     const unsigned char* __restrict__ q8, const float* __restrict__ q_w, const unsigned char* __restrict__ k8,
     const float* __restrict__ k_scale, const int* __restrict__ ks, const int* __restrict__ ke,
     int S, int Sk, int width, float* __restrict__ logits, long ld, int q_begin, int q_count, int parts) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * TILE_BYTES + 2 * BK * 4];
+  // two tiles of rows, two of scales, and so much more that the reads behind a tile's last row stay inside
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * TILE_BYTES + 32 * D];
   constexpr int NWAVE = QB;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: window tests below become scalar branches
@@ -107,24 +125,24 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
   const int blk = nblk - 1 - (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;            // longest windows first
   const int qb0 = q_begin + blk * QB;
   const int q_end = q_begin + q_count;
-  // end of the window that starts at lo: no key has a column beyond the row's (absolute columns: Sk is at most the width)
-  auto window_end = [&](int i, int lo) {
-    const int hi = min(ke[i], Sk);
-    return RELATIVE && hi - lo > width ? lo + width : hi;
-  };
+  // The windows of the block's queries, one per lane, from one pair of loads: [first key, end), where no key has a column beyond
+  // the row's (absolute columns: Sk is at most the width).
+  const int n_q = min(QB, q_end - qb0);
+  const int w_first = ks[qb0 + min(lane & (QB - 1), n_q - 1)], w_start = max(w_first, 0);
+  int w_end = min(ke[qb0 + min(lane & (QB - 1), n_q - 1)], Sk);
+  if (RELATIVE && w_end - w_start > width) w_end = w_start + width;
+  auto start_of = [&](int t) { return __builtin_amdgcn_readlane(w_start, t); };
+  auto end_of = [&](int t) { return __builtin_amdgcn_readlane(w_end, t); };
 
   // window union of the block
   int jlo = 0x7fffffff, jhi = 0, total = 0;
+#pragma unroll
   for (int t = 0; t < QB; t++) {
-    const int i = qb0 + t;
-    if (i < q_end) {
-      const int lo = max(ks[i], 0), hi = window_end(i, lo);
-      jlo = min(jlo, ks[i]);
-      jhi = max(jhi, hi);
-      total += (max(hi - lo, 0) + 31) / 32;
-    }
+    const int lo = start_of(t), hi = end_of(t);
+    jlo = min(jlo, lo);
+    jhi = max(jhi, hi);
+    total += t < n_q ? (max(hi - lo, 0) + 31) / 32 : 0;
   }
-  jlo = max(jlo, 0);
 
   if (2 * total < 3 * ((jhi - jlo + 31) / 32)) {
     // Unrelated windows (the sequences of a batch, or a single query): a key tile in LDS would serve one wave.  The
@@ -134,8 +152,8 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
     const int a = (int)((long)total * my / (parts * NWAVE)), b = (int)((long)total * (my + 1) / (parts * NWAVE));
     int before = 0;
 #pragma unroll 1
-    for (int i = qb0; i < min(qb0 + QB, q_end); i++) {
-      const int w_lo = max(ks[i], 0), w_hi = window_end(i, w_lo), n = (max(w_hi - w_lo, 0) + 31) / 32;
+    for (int i = qb0; i < qb0 + n_q; i++) {
+      const int w_lo = start_of(i - qb0), w_hi = end_of(i - qb0), n = (max(w_hi - w_lo, 0) + 31) / 32;
       const int u_lo = max(a - before, 0), u_hi = min(b - before, n);
       before += n;
       if (u_lo >= u_hi) continue;
@@ -173,10 +191,32 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
   // this wave's query
   const int i_q = qb0 + wave;
   const bool live = i_q < q_end;
-  const int qi = live ? i_q : -1;
-  const int qks = live ? max(ks[i_q], 0) : 0;
-  const int qke = live ? window_end(i_q, qks) : 0;
-  const int wlo = live ? qks : 0x7fffffff, whi = live ? qke : 0;     // the wave's window
+  const int qks = live ? start_of(wave) : 0, qke = live ? end_of(wave) : 0;
+
+  // this part's share of the window union, in sub-tiles of 32 keys: [s_lo, s_hi), and the wave's own of them [u_lo, u_hi)
+  const int s_first = jlo / 32, s_all = max((jhi + 31) / 32 - s_first, 0);
+  const int s_lo = s_first + (int)((long)s_all * part / parts), s_hi = s_first + (int)((long)s_all * (part + 1) / parts);
+  const int u_lo = max(qks / 32, s_lo), u_hi = qke > qks ? min((qke + 31) / 32, s_hi) : 0;
+  const int n_tiles = (s_hi - s_lo + BK / 32 - 1) / (BK / 32);
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  auto issue = [&](int t) {
+    int me = tid;
+    asm volatile("" : "+v"(me));                              // no registers for what one tile in four sub-tiles needs
+    const int gkey = me >> 3, gsub = me & 7;                  // 8 NWAVE key rows per DMA instruction
+    const int first = 32 * s_lo + t * BK;
+    const unsigned lb = lds0 + (unsigned)((t & 1) * TILE_BYTES + wave * 1024);
+#pragma unroll
+    for (int c = 0; c < BK / (8 * NWAVE); c++) {
+      const int key = c * 8 * NWAVE + gkey;
+      const int row = min(first + key, Sk - 1);
+      dma16(lb + c * 1024 * NWAVE, (unsigned)row * D + (unsigned)((gsub ^ swz(key)) * 16), k8);
+    }
+    if (wave < BK / 64) {   // the tile's per-key scales
+      const unsigned sb = lds0 + (unsigned)(2 * TILE_BYTES + (t & 1) * BK * 4 + wave * 256);
+      dma4(sb, (unsigned)min(first + me, Sk - 1) * 4u, k_scale);
+    }
+  };
+  if (n_tiles > 0) issue(0);
   i32x8 aq[NHT][2];
   float wq[NHT][16];
   load_query(q8, q_w, live ? i_q : qb0, r, g, aq, wq);
@@ -186,62 +226,122 @@ __global__ __launch_bounds__(64 * QB, NHT == 1 ? 6 : 4) void indexer_logits_kern
 #pragma unroll
     for (int s = 0; s < 2; s++) asm volatile("" : "+v"(aq[t][s]));
 
-  // this part's share of the window union's key tiles: [t_lo, t_hi)
-  const int t_first = jlo / BK, t_all = max((jhi + BK - 1) / BK - t_first, 0);
-  const int t_lo = t_first + (int)((long)t_all * part / parts), t_hi = t_first + (int)((long)t_all * (part + 1) / parts);
-  const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  const int gkey = tid >> 3, gsub = tid & 7;                  // 8 NWAVE key rows per DMA instruction
-  auto issue = [&](int t) {
-    const unsigned lb = lds0 + (unsigned)((t & 1) * TILE_BYTES + wave * 1024);
+  // B operand of a sub-tile: key row r, bytes [64s + 32g, +32) = 16-byte slots 4s+2g, 4s+2g+1.  Few registers are left: what
+  // an address is made of passes through empty assembly, so that it is made where it is used and not carried.
+  const unsigned b_off = (unsigned)(r * D + (((2 * g) ^ swz(r)) << 4));
+  struct KeyAddr { unsigned at[2][2]; };
+  auto key_addr = [&](unsigned base) {
+    asm volatile("" : "+s"(base));
+    KeyAddr k;
 #pragma unroll
-    for (int c = 0; c < BK / (8 * NWAVE); c++) {
-      const int key = c * 8 * NWAVE + gkey;
-      const int row = min(t * BK + key, Sk - 1);
-      dma16(lb + c * 1024 * NWAVE, (unsigned)row * D + (unsigned)((gsub ^ swz(key)) * 16), k8);
-    }
-    if (wave < BK / 64) {   // the tile's per-key scales
-      const unsigned sb = lds0 + (unsigned)(2 * TILE_BYTES + (t & 1) * BK * 4 + wave * 256);
-      dma4(sb, (unsigned)min(t * BK + wave * 64 + lane, Sk - 1) * 4u, k_scale);
-    }
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int x = 0; x < 2; x++) k.at[s][x] = (b_off ^ (unsigned)(64 * s + 16 * x)) + base;
+    return k;
   };
-  // B operand of sub-tile c: key row 32c + r, bytes [64s + 32g, +32) = 16-byte slots 4s+2g, 4s+2g+1
-  unsigned b_off[2][2];
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int x = 0; x < 2; x++) b_off[s][x] = (unsigned)(r * D + (((4 * s + 2 * g + x) ^ swz(r)) << 4));
+  auto read_keys = [&](const KeyAddr& k, int s, int off) {
+    const i32x4 lo = *(const i32x4*)(smem + k.at[s][0] + off);
+    const i32x4 hi = *(const i32x4*)(smem + k.at[s][1] + off);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  const unsigned lane4 = 4u * (unsigned)lane;
+  auto scale_of = [&](unsigned base) {
+    asm volatile("" : "+s"(base));
+    return *(const float*)(smem + 2 * TILE_BYTES + (lane4 + base));
+  };
+  // A row's stores go through a descriptor of exactly its window, counted from its first key: keys in front of it (a huge
+  // offset) and keys behind it are dropped by the bounds check, with neither compares nor masks.  Every pair of sub-tiles so
+  // issues exactly one store, which is what lets the wait in front of the barrier leave them in flight.
+  const __amdgpu_buffer_rsrc_t row_out = __builtin_amdgcn_make_buffer_rsrc(
+      logits + (size_t)((live ? i_q : qb0) - q_begin) * ld + (RELATIVE ? 0 : qks), 0, 4 * max(qke - qks, 0), 0x00027000);
+  auto store = [&](float v, unsigned at, bool lower) {         // lower: of the lower half-wave only
+    asm volatile("" : "+s"(at));
+    unsigned o = lane4;
+    if (lower) {
+      asm volatile("" : "+v"(o));
+      o |= (o & 128u) << 23;
+      static_assert(NOWHERE == 128u << 23, "");
+    }
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), row_out, (int)(o + at), 0, 0);
+  };
 
-  if (t_lo < t_hi) issue(t_lo);
-  for (int t = t_lo; t < t_hi; t++) {
-    DSA_WAIT_VMCNT(0);
-    __syncthreads();
-    if (t + 1 < t_hi) issue(t + 1);
-    const unsigned char* tb = smem + (t & 1) * TILE_BYTES;
-    const float* ksc_s = (const float*)(smem + 2 * TILE_BYTES) + (t & 1) * BK;
+  // What the next sub-tile's products overlap: the second head group's products of the last one (acc1) and the first group's sum.
+  f32x16 acc1 = {};
+  float sum1 = 0.f;
+  // the pair of sub-tiles it belongs to: the first one's sum, the scales, the place
+  float sum_a = 0.f, ksc1 = 0.f;
+  unsigned out1 = NOWHERE;
+
+  bool steady = false;
+  unsigned kb = 0, sb = 0;                                     // where a tile's rows and scales lie
 #pragma unroll 1
-    for (int c = 0; c < BK / 32; c++) {
-      const int j0 = t * BK + c * 32;
-      if (j0 >= whi || j0 + 32 <= wlo) continue;               // scalar: nothing of this wave's windows here
-      const int j = j0 + r;
-      const unsigned char* cb = tb + c * 32 * D;
-      i32x8 bk[2];
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        const i32x4 lo = *(const i32x4*)(cb + b_off[s][0]);
-        const i32x4 hi = *(const i32x4*)(cb + b_off[s][1]);
-        bk[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  for (int t = 0; t < n_tiles; t++, kb ^= TILE_BYTES, sb ^= BK * 4) {
+    if (steady) DSA_WAIT_VMCNT(BK / (32 * NHT));                      // the tile's rows, not the stores behind them
+    else DSA_WAIT_VMCNT(0);
+    __syncthreads();
+    if (t + 1 < n_tiles) issue(t + 1);
+    const int first = s_lo + t * (BK / 32);
+    const int c_lo = max(u_lo - first, 0), c_hi = min(u_hi - first, BK / 32);
+    steady = c_hi - c_lo == BK / 32;
+    if (c_lo >= c_hi) continue;
+    const unsigned ob = 128u * (unsigned)first - 4u * (unsigned)qks;
+    int c = c_lo;
+    const KeyAddr ka = key_addr(kb + c * 32 * D);
+    i32x8 bk0 = read_keys(ka, 0, 0), bk1 = read_keys(ka, 1, 0);
+    if constexpr (NHT == 2) {
+      // One sub-tile: each product of 64 cycles is followed by half a head group's weighted sums, which take as long to issue, of a
+      // product that ended before; a wave alone keeps both ports busy.  B: the second one of a pair.
+      auto sub_tile = [&](const KeyAddr& k, auto b) {
+        constexpr bool B = decltype(b)::value;
+        f32x16 acc0 = {};
+        acc0 = mfma_fp8(aq[0][0], bk0, acc0);
+        __builtin_amdgcn_sched_barrier(0);
+        sum1 = weigh<0>(acc1, wq[1], sum1);
+        __builtin_amdgcn_sched_barrier(0);
+        acc0 = mfma_fp8(aq[0][1], bk1, acc0);
+        __builtin_amdgcn_sched_barrier(0);
+        sum1 = weigh<8>(acc1, wq[1], sum1);
+        if constexpr (B) sum_a = sum1;
+        else store(add_pair(sum_a, sum1) * ksc1, out1, false);
+        __builtin_amdgcn_sched_barrier(0);
+        acc1 = f32x16{};
+        acc1 = mfma_fp8(aq[1][0], bk0, acc1);
+        __builtin_amdgcn_sched_barrier(0);
+        bk0 = read_keys(k, 0, (B ? 2 : 1) * 32 * D);
+        if constexpr (!B) ksc1 = scale_of(sb + c * 128);
+        sum1 = weigh<0>(acc0, wq[0], 0.f);
+        __builtin_amdgcn_sched_barrier(0);
+        acc1 = mfma_fp8(aq[1][1], bk1, acc1);
+        __builtin_amdgcn_sched_barrier(0);
+        bk1 = read_keys(k, 1, (B ? 2 : 1) * 32 * D);
+        sum1 = weigh<8>(acc0, wq[0], sum1);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll 1
+      for (; c < c_hi; c += 2) {
+        const KeyAddr k = key_addr(kb + c * 32 * D);
+        sub_tile(k, std::false_type{});
+        out1 = ob + c * 128u;
+        if (c + 1 < c_hi) sub_tile(k, std::true_type{});
+        else {                                                 // a last one without a partner: nothing of it stays open
+          sum1 = weigh<8>(acc1, wq[1], weigh<0>(acc1, wq[1], sum1));
+          store(add_pair(sum1, sum1) * ksc1, out1, true);
+          out1 = NOWHERE;
+        }
       }
-      const float ksc = ksc_s[c * 32 + r];
-      float sum = 0.f;
-#pragma unroll
-      for (int tt = 0; tt < NHT; tt++) sum = head_sum(aq[tt], bk, wq[tt], sum);
-      sum = add_halves(sum) * ksc;
-      if (g == 0 && j >= qks && j < qke) {
-        const int col = RELATIVE ? j - qks : j;
-        logits[(size_t)(qi - q_begin) * ld + col] = sum;
+    } else {
+#pragma unroll 1
+      for (; c < c_hi; c++) {
+        const i32x8 bk[2] = {bk0, bk1};
+        const float sum = head_sum(aq[0], bk, wq[0], 0.f);
+        const KeyAddr kn = key_addr(kb + min(c + 1, BK / 32 - 1) * 32 * D);
+        bk0 = read_keys(kn, 0, 0);
+        bk1 = read_keys(kn, 1, 0);
+        store(add_halves(sum) * scale_of(sb + c * 128), ob + c * 128u, true);
       }
     }
   }
+  if constexpr (NHT == 2) store(add_pair(sum_a, weigh<8>(acc1, wq[1], weigh<0>(acc1, wq[1], sum1))) * ksc1, out1, false);
 }
 
 }  // namespace

@@ -366,6 +366,35 @@ def test_logits_of_few_queries_and_unrelated_windows(gpu, Hi):
 
 
 @pytest.mark.parametrize("relative", [False, True])
+@pytest.mark.parametrize("Hi", [32, 64])
+def test_logits_at_the_edges_of_tiles(gpu, Hi, relative):
+    """Windows that begin and end around the sub-tiles of 32 keys, their pairs and the tiles of 128, eight related ones to a
+    block, in few blocks (cut into parts) and in many; nothing outside a window is written."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(Hi)
+    edges = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 159, 161]
+    rows = [(lo, 300 + hi) for lo in edges[::2] for hi in edges[1::2]] + [(lo, lo + n) for n in (1, 32, 33, 64, 65, 96, 128, 160) for lo in edges[::2]]
+    sk = 461
+    for copies in (1, 9):
+        ks, ke = (torch.tensor(x, dtype=torch.int32).repeat(copies) for x in zip(*rows))
+        S = ks.numel()
+        q = torch.randn(S, Hi, 128, generator=g).to(torch.float8_e4m3fn)
+        k = torch.randn(sk, 128, generator=g).to(torch.float8_e4m3fn)
+        w, sc = torch.randn(S, Hi, generator=g), torch.rand(sk, generator=g)
+        got = ops.indexer_logits(q.to(gpu), w.to(gpu), k.to(gpu), sc.to(gpu), ks.to(gpu), ke.to(gpu), relative=relative).cpu()
+        want = O.indexer_logits(q, w, k, sc, ks, ke, dtype=torch.float64)
+        # 128 exact products and Hi weighted terms in sums of 32 bits: an ulp each of the sum of the magnitudes
+        dot = torch.einsum("ihd,jd->ihj", q.double().abs(), k.double().abs())
+        bound = (128 + Hi) * 2.0 ** -24 * torch.einsum("ih,ihj->ij", w.double().abs(), dot) * sc.double()
+        for i in range(S):
+            lo, hi = int(ks[i]), int(ke[i])
+            row = got[i, :hi - lo] if relative else got[i, lo:hi]
+            assert ((row - want[i, lo:hi]).abs() <= bound[i, lo:hi]).all(), (copies, i, lo, hi)
+            assert int(torch.isfinite(got[i]).sum()) == hi - lo, (copies, i)
+
+
+@pytest.mark.parametrize("relative", [False, True])
 @pytest.mark.parametrize("S", [3, 300])                  # unrelated and shared windows
 def test_logits_in_rows_narrower_than_the_windows(gpu, relative, S):
     """Keys that have no column in the row are left out, and nothing is written behind it."""
