@@ -550,6 +550,32 @@ def test_backward_of_joint_queries_keeps_nonfinite_values_apart(gpu, H, S, where
         assert (~torch.isfinite(dkv[touched])).any(1).all() and torch.equal(dkv[~touched], dkv0.float().cpu()[~touched])
 
 
+@pytest.mark.parametrize("H", [32, 128])
+def test_backward_of_keys_with_few_and_many_rows(gpu, H):
+    """Keys with numbers of rows around one row per thread group (7) and one batch of loads (56), and with none, in any
+    neighbourhood."""
+    from loongforge_amd import ops
+
+    counts = [0, 1, 6, 7, 0, 0, 0, 0, 8, 55, 56, 57, 111, 112, 113, 180, 168, 0, 63, 5, 0]
+    S, K, skv = 180, 64, len(counts)
+    inp = O.make_mla_inputs(S, H, K, seed=H, skv=skv, q_start=skv)
+    idx = torch.full((S, K), -1, dtype=torch.int32)
+    for i in range(S):
+        mine = [j for j, c in enumerate(counts) if i < c]
+        idx[i, :len(mine)] = torch.tensor(mine, dtype=torch.int32)
+    q, kv, do, ids = inp.q.to(gpu), inp.kv.to(gpu), inp.dout.to(gpu), idx.to(gpu)
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, skv, inp.sm_scale)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, skv, inp.sm_scale)
+    # Against the same rounding points (bf16 P, dS and rows), within the bound that assert_mla_grads derives for them: one step of the
+    # bf16 grid at the largest row that enters.  (Its further limits against plain fp32 are for selections of many keys; with a
+    # dozen P is of order 0.1 and so are the errors that its rounding to bf16 puts into sums of 180 rows.)
+    _, ref, _, largest = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, idx, inp.dout, skv, inp.sm_scale, 512, out=out.cpu(), lse=lse.cpu(),
+                                                          dtype=torch.float64, round_rows_bf16=True, return_abs_sum=True)
+    dkv = dkv.float().cpu()
+    assert ((dkv - ref).abs() <= 2e-2 + 1e-2 * ref.abs() + 2.0 ** -7 * largest).all()
+    assert (dkv[torch.tensor(counts) == 0] == 0).all()
+
+
 def test_backward_does_not_depend_on_the_slot_order(gpu):
     """The backward walks each query's ids in ascending key order whatever order they arrive in, so
     permuting the slots (independently per query) and scattering unused slots between the used ones
