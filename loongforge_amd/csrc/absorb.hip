@@ -19,9 +19,9 @@
 // bytes per lane, next block requested before this block's MFMAs).  With C^T in the accumulators a lane
 // owns one output row; four column tiles go through an 8 KB strip per wave, so that a store instruction
 // writes four 256-byte row segments instead of 32 of 32 bytes.
-// Few rows (absorb_few_kernel): one wave per (head, 64 columns) on the query side, two per (head, 32
-// columns) on the output side read their weight rows straight into registers and walk the row blocks:
-// more waves, no trip of the weights through LDS.
+// Few rows (absorb_few_kernel): one wave per (head, 64 columns) on the query side, two or four per (head,
+// 32 or 64 columns) on the output side read their weight rows straight into registers and walk the row
+// blocks: more waves, no trip of the weights through LDS.
 #include <algorithm>
 
 #include "mla_tile.h"
@@ -184,21 +184,25 @@ __device__ __forceinline__ void rotate_block(const AbsorbArgs& p, int blk, int h
       rope::store_quad<PAIRING>(rope::rotate<false>(x[i], t[i]), p.pe_dst + (size_t)s[i] * p.c_tok + (size_t)h * p.c_head, q, EMB);
 }
 
-// One workgroup per (head, column tiles) and range of row blocks, plus one per head for the rotary part.  Query side: one wave
-// and two 32-column tiles, so that it fills whole 128-byte lines of the output (us, one / two / four tiles: 48 rows x 128 heads
-// 13.1 / 11.1 / 11.6; waves in workgroups of their own: 1 row 4.8, in pairs 5.5, in fours 7.1).  Output side (K = 512): two
-// waves share a tile, half of the sum each: half the registers (the next rows are requested before these rows' products) and
-// twice the waves; the halves meet in LDS, the two waves storing every other block.
-template <int K> constexpr int FEW_SHARE = K == 512 ? 2 : 1;
-template <int K> constexpr int FEW_COLS = K == 512 ? 1 : 2;
-template <int K, int N>
-__global__ __launch_bounds__(64 * FEW_SHARE<K>, 2) void absorb_few_kernel(AbsorbArgs p) {
-  constexpr int SHARE = FEW_SHARE<K>, KS = K / 16 / SHARE, COLS = FEW_COLS<K>, NT = N / (32 * COLS);
-  __shared__ f32x4 box[SHARE == 1 ? 1 : 2 * 4 * 64];         // [block % 2][4][lane]
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+// One workgroup per (head, COLS * 32 columns) and range of row blocks, plus one per head for the rotary part.  SHARE waves share the
+// sum over k (K = 512), each a part of it: fewer registers (the next rows are requested before these rows' products) and more
+// waves; the parts meet in LDS, every wave adding up and storing its share of the block.
+// 16x16x32 products: four lanes read 64 consecutive bytes of a row, and with the weight rows of a tile in the order 8 kg + i,
+// 8 kg + 4 + i a lane owns eight consecutive columns of two tiles and four lanes store 64 consecutive bytes (32x32x16: 32 bytes
+// either way).  The workgroups of a head sit on one XCD (where the heads divide evenly), so that its L2 fetches the head's rows and
+// weights once.  Bound by what the caches deliver and by the round trips of a launch.  us, 32x32x16 products of two tiles and heads
+// over all XCDs before / now, cold caches, query side: 48 rows x 128 heads 10.5 / 9.2, 200 x 32 9.5 / 8.5, 61 x 64 7.0 / 6.7, 90 x 128
+// 16.0 / 13.2; output side: 48 x 128 9.8 / 8.6, 200 x 32 8.9 / 8.3, 61 x 64 7.0 / 6.3, 120 x 64 9.7 / 8.5.
+template <int K, int N, int SHARE, int COLS>
+__global__ __launch_bounds__(64 * SHARE, 2) void absorb_few_kernel(AbsorbArgs p) {
+  constexpr int KS = K / 32 / SHARE, NT = N / (32 * COLS), MINE = 2 * COLS / SHARE;        // k-steps; column groups; a wave's units of
+  static_assert(SHARE == 1 || MINE == 1);                                                   // (16 rows, 32 columns) to store: all, or one
+  __shared__ f32x4 box[SHARE == 1 ? 1 : 2 * SHARE * (SHARE - 1) * 2 * 64];                  // [block % 2][unit][other waves][2][lane]
+  const int lane = threadIdx.x & 63, m = lane & 15, kg = lane >> 4;
   const int part = SHARE == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int per = p.pe_src ? NT + 1 : NT;
-  const int h = (int)blockIdx.x / per, nt = (int)blockIdx.x % per;
+  const int per = p.pe_src ? NT + 1 : NT, bx = (int)blockIdx.x;
+  const bool xcd = p.H % 8 == 0;
+  const int h = xcd ? 8 * ((bx >> 3) / per) + (bx & 7) : bx / per, nt = (xcd ? bx >> 3 : bx) % per;
   const int nblk = (p.S + 31) / 32;
   const int b_lo = (int)((long)nblk * blockIdx.y / gridDim.y), b_hi = (int)((long)nblk * (blockIdx.y + 1) / gridDim.y);
   if (nt == NT) {
@@ -211,88 +215,103 @@ __global__ __launch_bounds__(64 * FEW_SHARE<K>, 2) void absorb_few_kernel(Absorb
     }
     return;
   }
-  bf16x8 wv[COLS][KS], cur[KS], nxt[KS];
+  bf16x8 wv[2 * COLS][KS], cur[2][KS], nxt[2][KS];
 #pragma unroll
-  for (int c = 0; c < COLS; c++) {
-    const bf16x8* wp = (const bf16x8*)(p.w + ((size_t)h * N + 32 * (COLS * nt + c) + r) * K) + 2 * KS * part + g;
+  for (int c = 0; c < 2 * COLS; c++) {
+    const int n = 32 * (COLS * nt + (c >> 1)) + 8 * (m >> 2) + 4 * (c & 1) + (m & 3);
+    const bf16x8* wp = (const bf16x8*)(p.w + ((size_t)h * N + n) * K) + 4 * KS * part + kg;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) wv[c][ks] = wp[2 * ks];
+    for (int ks = 0; ks < KS; ks++) wv[c][ks] = wp[4 * ks];
   }
-  auto load_rows = [&](int blk, bf16x8 (&t)[KS]) {
-    const bf16x8* ap = (const bf16x8*)(p.a + (size_t)min(32 * blk + r, p.S - 1) * p.a_tok + (size_t)h * p.a_head) + 2 * KS * part + g;
+  auto load_rows = [&](int blk, bf16x8 (&t)[2][KS]) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) t[ks] = ap[2 * ks];
+    for (int rt = 0; rt < 2; rt++) {
+      const bf16x8* ap = (const bf16x8*)(p.a + (size_t)min(32 * blk + 16 * rt + m, p.S - 1) * p.a_tok + (size_t)h * p.a_head) + 4 * KS * part + kg;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) t[rt][ks] = ap[4 * ks];
+    }
   };
   load_rows(b_lo, cur);
 #pragma unroll 1
   for (int blk = b_lo; blk < b_hi; blk++) {
     if (blk + 1 < b_hi) load_rows(blk + 1, nxt);
     __builtin_amdgcn_sched_barrier(0);       // all loads in flight before the first product
+    f32x4 acc[2][2 * COLS];
 #pragma unroll
-    for (int c = 0; c < COLS; c++) {
-      f32x16 acc;
+    for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[e] = 0.f;
+      for (int c = 0; c < 2 * COLS; c++) acc[rt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[c][ks], cur[ks], acc, 0, 0, 0);
-      bool mine = true;
-      if (SHARE == 2) {
-        // one barrier per block: a box is written again two blocks on, behind the barrier that follows its reading
-        f32x4* b = box + (blk & 1) * 256 + lane;
-        mine = part == (blk & 1);
-        if (!mine) {
+    for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) b[j * 64] = f32x4{acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
+      for (int c = 0; c < 2 * COLS; c++)
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[c][ks], cur[rt][ks], acc[rt][c], 0, 0, 0);
+    if (SHARE > 1) {
+      // one barrier per block: a box is written again two blocks on, behind the barrier that follows its reading
+      f32x4* b = box + (blk & 1) * (SHARE * (SHARE - 1) * 2 * 64) + lane;
+#pragma unroll
+      for (int u = 0; u < SHARE; u++)
+        if (u != part) {
+#pragma unroll
+          for (int x = 0; x < 2; x++) b[((u * (SHARE - 1) + (part < u ? part : part - 1)) * 2 + x) * 64] = acc[u / COLS][2 * (u % COLS) + x];
         }
-        __syncthreads();
-        if (mine) {
+      __syncthreads();
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const f32x4 o = b[j * 64];
+      for (int u = 0; u < SHARE; u++)
+        if (u == part) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[4 * j + e] += o[e];
-          }
+          for (int o = 0; o < SHARE - 1; o++)
+#pragma unroll
+            for (int x = 0; x < 2; x++) acc[u / COLS][2 * (u % COLS) + x] += b[((u * (SHARE - 1) + o) * 2 + x) * 64];
         }
-      }
-      if (mine) {
-        uint4 o[2];
-        acc_row_to_16B(acc, 1.0f, o);        // every lane takes part; rows past the end are not stored
-        const int s = 32 * blk + r;
-        if (s < p.S) {
-          unsigned short* out = (unsigned short*)p.c + (size_t)s * p.c_tok + (size_t)h * p.c_head + 32 * (COLS * nt + c) + 8 * g;
-          *(uint4*)out = o[0];
-          *(uint4*)(out + 16) = o[1];
-        }
-      }
     }
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) cur[ks] = nxt[ks];
+    for (int u = 0; u < 2 * COLS; u++) {
+      if (SHARE > 1 && u != part) continue;
+      const int rt = u / COLS, c = 2 * (u % COLS), s = 32 * blk + 16 * rt + m;
+      const f32x4 lo = acc[rt][c], hi = acc[rt][c + 1];
+      if (s < p.S)
+        *(uint4*)((unsigned short*)p.c + (size_t)s * p.c_tok + (size_t)h * p.c_head + 32 * COLS * nt + 16 * c + 8 * kg) =
+            make_uint4(cvt_pk_bf16(lo[0], lo[1]), cvt_pk_bf16(lo[2], lo[3]), cvt_pk_bf16(hi[0], hi[1]), cvt_pk_bf16(hi[2], hi[3]));
+    }
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) cur[rt][ks] = nxt[rt][ks];
   }
 }
 
-// Up to this many (row, head) pairs the weights are better re-read by the waves than brought through LDS once per head: there the
-// other kernel is one workgroup per head that mostly waits for its weights.  us, this kernel against the other, query side with
-// rotary part / output side: 128 heads x 1 row 4.8 / 4.9 against 12.5 / 9.5, x 64 rows 12.5 / 10.7 against 15.8 / 11.3, x 100
-// 17.0 / 14.2 against 17.1 / 12.1; 64 heads x 100 11.0 / 8.1 against 14.0 / 10.4, x 200 16.6 / 13.3 against 16.6 / 12.6;
-// 32 heads x 200 10.2 / 8.6 against 15.4 / 10.9, x 300 13.1 / 11.2 against 17.1 / 11.0.
-template <int K> constexpr int FEW_ROW_HEADS = K == 512 ? 8192 : 12288;
-// Row ranges until there are so many workgroups.  The query side's share of the weights is read in one round trip, so every
-// row block has its own waves; the output side's is not (48 rows x 128 heads 11.4 us with the weights read by both blocks'
-// waves, 9.0 in one range).
-template <int K> constexpr int FEW_GROUPS = K == 512 ? 512 : 1 << 16;
+// Row ranges: `full` workgroups, or twice as many with more than three row blocks for every two of them; more read the weights too often.
+// us, output side with 256 / 512 workgroups: 200 rows x 32 heads 7.6 / 8.6, 48 x 128 8.2 / 9.0, 400 x 32 11.1 / 10.8; query side with up to
+// 1200 / 2400: 200 x 32 8.5 / 9.2, 250 x 64 15.9 / 15.2.
+template <int K, int N, int SHARE, int COLS>
+void launch_few(const AbsorbArgs& p, int full, hipStream_t st) {
+  const int groups = p.H * (N / (32 * COLS) + (p.pe_src ? 1 : 0)), nblk = (p.S + 31) / 32, many = 2 * full / groups;
+  const int ranges = 2 * nblk > 3 * many ? many : std::min(full / groups, nblk);
+  absorb_few_kernel<K, N, SHARE, COLS><<<dim3(groups, std::max(1, ranges)), dim3(64 * SHARE), 0, st>>>(p);
+}
 
+// Up to `few` (row, head) pairs the weights are better re-read by the waves than brought through LDS once per head: there the other
+// kernel is one workgroup per head that mostly waits for its weights.  us, cold caches, this kernel against the other, query side with
+// rotary part / output side: 128 heads x 1 row 5.7 / 5.7 against 14.3 / 11.1, x 100 14.2 / 11.6 against 17.9 / 13.3, x 160 18.7 / 14.4
+// against 20.7 / 16.2, x 200 22.3 / 16.9 against 21.3 / 16.4; 64 heads x 250 15.1 / 11.5 against 20.8 / 13.0, x 400 21.0 / 16.4 against
+// 20.8 / 16.4; 32 heads x 640 17.8 / 14.9 against 20.6 / 14.1.  The other kernel's workgroups walk whole steps: two of them
+// are worse than half as many row blocks here (output side, 128 heads x 300 20.6 against 25.5, 32 heads x 1400 21.7 against 26.1).
+// Output side: four waves and 64 columns a workgroup where those fill the chip (61 rows x 64 heads 6.0 and 6.8 as two waves and 32
+// columns), two and 32 where they do not (16 x 64 5.5 and 4.7, 33 x 32 6.0 and 4.8).
 template <int K, int N>
 int launch(const AbsorbArgs& p, hipStream_t st) {
-  if ((long)p.S * p.H <= FEW_ROW_HEADS<K>) {
-    const int groups = p.H * (N / (32 * FEW_COLS<K>) + (p.pe_src ? 1 : 0));
-    const int ranges = std::max(1, std::min(FEW_GROUPS<K> / groups, (p.S + 31) / 32));
-    absorb_few_kernel<K, N><<<dim3(groups, ranges), dim3(64 * FEW_SHARE<K>), 0, st>>>(p);
-    return 0;
-  }
   constexpr int WAVES = K == 128 ? 8 : 4;    // rows of 1 KB in registers twice: four waves
   const int nblk = (p.S + 32 * WAVES - 1) / (32 * WAVES);
-  int splits = (256 + p.H - 1) / p.H;        // one workgroup per compute unit: its LDS holds one weight matrix
-  if (splits > nblk) splits = nblk;
+  const int splits = std::min((256 + p.H - 1) / p.H, nblk);        // one workgroup per compute unit: its LDS holds one weight matrix
+  const long few = K == 128 ? 22528 : nblk <= splits ? 18432 : 49152;
+  if ((long)p.S * p.H <= few) {
+    if constexpr (K == 128) launch_few<K, N, 1, 2>(p, 1200, st);
+    else if (p.H * (N / 64) * ((p.S + 31) / 32) >= 240) launch_few<K, N, 4, 2>(p, 256, st);
+    else launch_few<K, N, 2, 1>(p, 512, st);
+    return 0;
+  }
   const size_t smem = (size_t)K * N * 2 + 32768;
   auto kern = K == 128 && p.pe_src ? absorb_kernel<K, N, WAVES, K == 128> : absorb_kernel<K, N, WAVES, false>;
   if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) return -2;

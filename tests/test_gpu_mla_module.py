@@ -61,6 +61,14 @@ def test_absorb_of_few_and_many_rows(gpu, S, H, k, n):
     assert (c[:, :, n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("S,H", [(32, 120), (31, 119), (61, 64), (113, 40), (97, 128), (257, 64), (352, 64), (353, 64), (384, 128), (18433, 1)])
+@pytest.mark.parametrize("k,n", [(128, 512), (512, 128)])
+def test_absorb_of_few_rows_by_number_of_waves_and_ranges(gpu, S, H, k, n):
+    """Both sides of the rules for two and four waves a workgroup, for ranges of row blocks and for the kernel of many rows; heads that
+    do and do not divide over the XCDs."""
+    test_absorb_of_few_and_many_rows(gpu, S, H, k, n)
+
+
 @pytest.mark.parametrize("S,H", [(1, 3), (33, 16), (64, 2), (65, 5), (300, 128), (777, 1)])
 @pytest.mark.parametrize("pairing,dtype", [(0, torch.bfloat16), (1, torch.float32)])
 def test_absorb_and_rope_in_one_kernel(gpu, S, H, pairing, dtype):
