@@ -84,6 +84,20 @@ __device__ __forceinline__ void acc_row_to_16B(const f32x16& acc, float scale, u
   o[0] = make_uint4(pc[0][0], pc[0][1], pc[1][0], pc[1][1]);
   o[1] = make_uint4(pc[2][0], pc[2][1], pc[3][0], pc[3][1]);
 }
+// Order of work for kernels whose workgroups own a compute unit each: workgroup i -> position among n queries in order of decreasing length.
+// Taken strictly in that order the 256 workgroups of the first round have the same length, stay in step from round to round, and all
+// read a query's operands at the same time, when nothing else uses the memory, and compute at the same time, when the memory idles.  So
+// the first `round` workgroups take every so-many-th of the last `ramp` positions, where a causal window grows from nothing to its
+// full length, and those from there on find them out of step; the others follow in order, the shortest again at the end.
+__device__ __forceinline__ int spread_start(int i, int n, int round, int ramp) {
+  const int tail = min(n, max(ramp, 2 * round)), step = tail / round;
+  if (step < 2) return i;
+  if (i < round) return n - tail + i * step;
+  const int j = i - round - (n - tail);                // >= 0: among the tail's positions that are left
+  if (j < 0) return i - round;
+  if (j >= round * (step - 1)) return n - tail + round + j;
+  return n - tail + j + j / (step - 1) + 1;
+}
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding).
 #define DSA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 0xf) | (((n) >> 4) << 14)) | (0x7 << 4) | (0xf << 8))
 

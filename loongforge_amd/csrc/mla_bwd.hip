@@ -1040,15 +1040,22 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-// The query of workgroup i, from the last one on; with groups of G in G turns over the groups with one query of each, so that the
+// The query of workgroup i, from the last one on (RAMP > 0: but for the first 256, spread over the last RAMP * K); with groups of G in G turns over the groups with one query of each, so that the
 // workgroups that do joint units follow one another.  Neighbouring workgroups go to different XCDs: with the groups' queries side by side
 // every G-th workgroup did the work, on 8 / G of the XCDs (3072 x 32 heads x 640 slots: scores and rows 865 us instead of 296).
-template <int G>
-__device__ __forceinline__ int query_of(int i, int cnt) {
+// RAMP: scores and rows read 410 KB per query or unit in front of 8 to 64 tiles of matrix work.  us, in strict order / first round spread over
+// K / over 4 K queries: 5000 x 128 heads, window and compressed keys 1932 / 1922 / 1770, 3072 x 64 heads of these 590 / 591 / 556, 2077 x
+// 512 x 64 heads 304 / 302 / 291, 1300 x 512 x 128 432 / 389 / 415, 8192 x 2048 x 128 8967 / 8906 / 8865, long documents of few slots
+// and 9000 x 2048 x 64 the same; two rounds spread 6 % slower than one.  dQ, whose set-up is small, does not gain.
+constexpr int PDS_RAMP = 4;
+template <int G, int RAMP>
+__device__ __forceinline__ int query_of(int i, int cnt, int K) {
   const int groups = cnt / G, rest = cnt - groups * G;
-  if (G == 1 || i < rest) return cnt - 1 - i;
+  if (i < rest) return cnt - 1 - i;
   const int turn = (i - rest) / groups;
-  return (groups - 1 - (i - rest - turn * groups)) * G + turn;
+  int p = i - rest - turn * groups;
+  if (RAMP > 0) p = spread_start(p, groups, 256, RAMP * K / G);
+  return (groups - 1 - p) * G + turn;
 }
 
 // G: queries of a group that may be a joint unit (4 / HG), or 1.  units: padded slot counts of the groups' units, 0 where the queries
@@ -1060,7 +1067,7 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, const int* __restrict__ units,
     size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int ql = query_of<G>((int)blockIdx.x, cnt);
+  const int ql = query_of<G, PDS_RAMP>((int)blockIdx.x, cnt, K);
   // (two copies of every body: each copy meets the same barriers)
   if constexpr (HG == 4 || G > 1) {            // 128 heads: of the query or of a unit
     const int slots = G > 1 ? units[ql / G] : K;
@@ -1091,7 +1098,7 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
   if (rs.first) {
-    const int ql = query_of<G>(rs.i, cnt);
+    const int ql = query_of<G, 0>(rs.i, cnt, K);
     const int* list = ids + (size_t)ql * K;
     __bf16* dq_rows = dq + (size_t)(q0 + ql) * H * DQK;
     const unsigned char* own = pds + (size_t)(ql / G) * group_pds;

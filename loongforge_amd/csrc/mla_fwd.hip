@@ -814,8 +814,10 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
 template <bool SPLIT, int POUT>
 __global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int u = (int)blockIdx.x;             // longest prefixes first
-  const int qi = a.S - 1 - (SPLIT ? u / a.ksplit : u), sp = SPLIT ? u % a.ksplit : 0;
+  // Longest prefixes first, but for the first round.  us, in strict order / spread over K / over 4 K queries: with logits 1300 x 512 slots 223 /
+  // 199 / 211, 5000 x 1024 in five documents 928 / 893 / 900, 8192 x 2048 4006 / 3949 / 3973; without them the same within 1 %.
+  const int u = (int)blockIdx.x;
+  const int qi = a.S - 1 - (SPLIT ? u / a.ksplit : spread_start(u, a.S, 256, a.K)), sp = SPLIT ? u % a.ksplit : 0;
   if (threadIdx.x < 256) wide_body<true, SPLIT, POUT>(a, qi, sp, smem);
   else wide_body<false, SPLIT, POUT>(a, qi, sp, smem);
 }

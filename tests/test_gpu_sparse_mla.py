@@ -387,6 +387,22 @@ def test_backward_of_many_heads_in_one_pass(gpu, S, H, K, q_start):
     test_backward_of_few_heads(gpu, H, S, K, q_start, None)
 
 
+@pytest.mark.parametrize("S,H,K", [(511, 128, 64), (512, 96, 64), (770, 128, 64), (1301, 128, 192)])
+def test_every_query_of_several_rounds_is_worked_on(gpu, S, H, K):
+    """The first 256 workgroups take queries from the whole range, the others what is left: each query once, whatever the sizes."""
+    from loongforge_amd import ops
+
+    inp = O.make_mla_inputs(S, H, K, seed=S)
+    q, kv, ids, do = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu)
+    torch.full((3 * S, H, 576), float("nan"), dtype=torch.bfloat16, device=gpu)        # (what is left unwritten is likely to show)
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, 0, inp.sm_scale)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, 0, inp.sm_scale)
+    ro, rl, _ = O.sparse_mla_fwd(inp.q, inp.kv, inp.idx, 0, inp.sm_scale, 512)
+    assert_close(out, ro, "out")
+    assert (lse.cpu() - rl).abs().max().item() < 1e-4
+    assert_mla_grads(dq, dkv, inp.q, inp.kv, inp.idx, inp.dout, 0, inp.sm_scale, name="rounds", out=out, lse=lse)
+
+
 def _overlapping_ids(S, K, skv, turn, far, seed):
     """Causal ids of queries at positions skv - S + i: K of the K + K / 8 keys behind a place that moves by a key every ``turn``
     queries (0: never), and for every ``far``-th run of 16 queries ids at random, which neighbours hardly share."""
@@ -465,6 +481,7 @@ def test_backward_of_joint_queries(gpu, H, S, K, skv, turn, far):
     (32, 1100, 2048, 2900, False),    # nearly the longest list
     (32, 1537, 192, 1537, True),      # from one key on
     (32, 1540, 256, 6000, False),     # little in common: no units
+    (32, 2103, 128, 2103, True),      # more than two rounds of groups
 ])
 def test_backward_of_joint_queries_is_that_of_wider_queries(gpu, H, S, K, skv, causal):
     """The same gradients as through the kernels for 128 heads with heads of zeros beside the queries' own, in one sweep and in
