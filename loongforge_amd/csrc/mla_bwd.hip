@@ -535,9 +535,13 @@ __device__ __forceinline__ void pds_rows_body(
 // other columns of dO by rows (wave w: heads 16 w ..) and by columns (wave w: columns 64 w ..).
 // That leaves room for one tile and one buffer of P and dS, so a step has two halves with a barrier each: S, dP -> P, dS of the
 // tile; then the transfer of the next tile starts and the rows are multiplied and stored under it.
-// 7700 cycles a step at 8192 queries x 2048 slots x 128 heads, 4352 of them in the matrix pipe (46 % busy; a pass costs 75 000
-// more for its set-up, 557 KB through LDS): the 816 LDS reads, 36 KB of transfers and 37 KB of stores of a step share the way
-// between the registers and LDS or cache, and hold each other up: LDS reads slow down by half while a tile arrives.  8.7 ms where
+// The set-up of a query is one round trip to memory: ids, Q, dO and O are requested together (410 KB), dO goes on to LDS from the
+// registers that its sums with O had it in, and the first tile travels meanwhile.  (ids behind the operands, dO read twice and the first tile
+// behind all that were four: 12000 queries of three documents x 256 slots 2692 us and 2455 now, 5000 x 1024 1898 and 1816, 5000 of
+// window and compressed keys 1786 and 1743, 2077 x 512 x 64 heads 291 and 286, 8192 x 2048 8.89 ms and 8.81.  The first 32 of every
+// 64 columns read again from the L2 instead of kept, which saves 32 registers on the way: 1 - 5 % slower.)
+// 7700 cycles a step at 8192 queries x 2048 slots x 128 heads, 4352 of them in the matrix pipe (46 % busy): the 816 LDS reads,
+// 36 KB of transfers and 37 KB of stores of a step share the way between the registers and LDS or cache, and hold each other up: LDS reads slow down by half while a tile arrives.  8.7 ms where
 // the two passes took 4.15 + 5.55, with 8 KB less to write and 16 KB less to read per tile.  Slower than this form, though each
 // has fewer LDS reads: 32x32x16 products for the rows (644, stores of 32 bytes in 32 rows), all column tiles at once (704, the
 // stores of a step together at its end), and waves 0-3 for P, dS beside waves 4-7 for the rows, with the next tile's first groups
@@ -596,8 +600,18 @@ __device__ __forceinline__ void pds_rows_wide_body(
   // Rows of Q and dO travel to LDS in groups of 128 bytes of all 128 rows, chunk c of row r in slot c ^ (r & 7).  Wave w moves rows
   // 8 w .. 8 w + 7 and 64 + 8 w ..; heads beyond H repeat the last one (their P and dS are zero).
   const unsigned char* q_rows = (const unsigned char*)uniform_ptr(q);
-  const unsigned char* do_rows = (const unsigned char*)uniform_ptr(dout);
   const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
+  // The ids are requested first, then Q, O and dO: one round trip to memory.
+  constexpr int NV = G > 1 ? UNIT_SLOTS / PDS_THREADS : 4;
+  int v[NV], pad = 0;
+  if constexpr (G > 1) {
+    pad = ids[0];
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = ids[min(tid + PDS_THREADS * i, K - 1)];
+  } else {
+    request_ids(ids, 0, K, v);
+  }
+  __builtin_amdgcn_sched_barrier(0);
   auto group_base = [](int p) { return p < 4 ? p * 16384 : p < 8 ? WIDE_TILE + (p - 4) * 16384 : WIDE_ROT; };
   {
     const int l = fresh_lane();
@@ -608,14 +622,15 @@ __device__ __forceinline__ void pds_rows_wide_body(
       for (int p = 0; p < 9; p++) dma16(lb + rb * 8192 + group_base(p), src + p * 128, q_rows);
     }
   }
-  bf16x8 doreg[VS / 2];                        // dO, the odd 32 columns
+  const int m = lane & 15, kg = lane >> 4;
+  const int h = wave * 16 + m;
+  const bool head_ok = h < H;
+  const size_t hrow = min(h, H - 1);
+  int ntiles = NT;
+  bf16x8 dkeep[VS / 2], doreg[VS / 2];         // dO, the even and the odd 32 columns
   unsigned bad_do = 0;                         // G > 1: which of the wave's heads have values in dO that are not finite
   auto of_heads = [](unsigned long long b) { return (unsigned)((b | b >> 16 | b >> 32 | b >> 48) & 0xffffu); };   // lanes (m, kg) -> heads m
   {
-    const int m = lane & 15, kg = lane >> 4;
-    const int h = wave * 16 + m;
-    const bool head_ok = h < H;
-    const size_t hrow = head_ok ? h : 0;
     const bf16x8* op = (const bf16x8*)(out + hrow * DV) + kg;
     const bf16x8* dp = (const bf16x8*)(dout + hrow * DV) + kg;
     bf16x8 o[VS], d[VS];
@@ -623,6 +638,16 @@ __device__ __forceinline__ void pds_rows_wide_body(
     for (int ks = 0; ks < VS; ks++) { d[ks] = dp[4 * ks]; o[ks] = op[4 * ks]; }
     const float lse_h = lse[hrow];
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (G > 1) {
+      // slots behind the last key repeat the first one, for none of the queries
+#pragma unroll
+      for (int i = 0; i < NV; i++) {
+        const int t = tid + PDS_THREADS * i;
+        if (t < K) idx_s[t] = v[i] < 0 ? pad & UNIT_KEY : v[i];
+      }
+    } else {
+      ntiles = stage_requested_ids(v, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
+    }
     float part = 0.f;                          // delta = rowsum(O . dO)
 #pragma unroll
     for (int ks = 0; ks < VS; ks++) {
@@ -631,6 +656,8 @@ __device__ __forceinline__ void pds_rows_wide_body(
       if (ks & 1) {
         doreg[ks >> 1] = d[ks];
         asm volatile("" : "+a"(doreg[ks >> 1]));
+      } else {
+        dkeep[ks >> 1] = d[ks];
       }
     }
     part += __shfl_xor(part, 16, 64);
@@ -641,10 +668,6 @@ __device__ __forceinline__ void pds_rows_wide_body(
     }
     if (G > 1) bad_do = of_heads(__ballot(!(fabsf(part) < INFINITY)));
   }
-  int ntiles = NT;
-  // (the helper is written for four waves; the other four repeat part of its work with equal results)
-  if constexpr (G > 1) stage_unit(ids, K, idx_s);
-  else ntiles = stage_ids(ids, 0, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();
@@ -709,46 +732,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
         else asm volatile("" : "+v"(xq[c][ks]));
       }
   }
-  __syncthreads();                             // dO takes the place of Q's first groups
-  // dO: pair j of 64 columns, its first 32 of either to stay, the second 32 to pass through
-  {
-    const int l = fresh_lane(), sw = (l & 7) ^ (l >> 3);
-#pragma unroll
-    for (int rb = 0; rb < 2; rb++) {
-      const unsigned src = (unsigned)min(64 * rb + 8 * wave + (l >> 3), H - 1) * (DV * 2) + (sw >> 2) * 128 + (sw & 3) * 16;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        dma16(lb + rb * 8192 + j * 16384, src + j * 256, do_rows);
-        dma16(lb + rb * 8192 + WIDE_TILE + j * 16384, src + j * 256 + 64, do_rows);
-      }
-    }
-  }
-  DSA_WAIT_VMCNT(0);
-  __syncthreads();
-  if constexpr (G > 1) {
-    if (bad_do) {
-      const int l = fresh_lane();
-#pragma unroll 1
-      for (int j = 0; j < 8; j++)
-#pragma unroll 1
-        for (int c = l; c < 128; c += 64) drop_nonfinite(smem + (j < 4 ? 0 : WIDE_TILE) + (j & 3) * 16384 + 2048 * wave + c * 16);
-    }
-    __syncthreads();
-  }
-  {
-    const int l = fresh_lane();
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        xo[c][ks] = tr_pair(smem + WIDE_TILE + (wave >> 1) * 16384 + ks * 4096 + tr_off(l, 4 * (wave & 1) + 2 * c));
-        asm volatile("" : "+v"(xo[c][ks]));
-      }
-  }
-  __syncthreads();
-
-  const int ln = fresh_lane();
-  const int lm = ln & 15, lk = ln >> 4, lg = ln >> 5;
+  __syncthreads();                             // Q is in registers: its place is free for the first tile and for dO
   // transfers of a tile: waves 0-3 take groups 0-4, waves 4-7 groups 5-8; wave 7 the tile's destination rows
   const int grp0 = hh * 5;
   const unsigned tile_lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(WIDE_TILE + (wave & 3) * 1024 + grp0 * GRP_BYTES));
@@ -763,6 +747,41 @@ __device__ __forceinline__ void pds_rows_wide_body(
     if (wave == 7) dma16(lds0 + (unsigned)((unsigned char*)dst_s - smem) + (n & 1) * 1024, (unsigned)l * 16, dst + tile * BI);
   };
   issue(0);
+  // dO from the registers: of every 64 columns first the second 32, for the column operands, then the first 32, to stay.  Chunk c of a row
+  // of group j (columns 128 j + 64 (c / 4) + 8 (c % 4) .., of the first or second 32) lies in slot c ^ (row & 7).
+  auto put_do = [&](const bf16x8 (&x)[VS / 2]) {
+    const int l = fresh_lane();
+    unsigned char* row = smem + (wave * 16 + (l & 15)) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int half = 0; half < 2; half++) *(bf16x8*)(row + j * 16384 + (((4 * half + (l >> 4)) ^ (l & 7)) << 4)) = x[2 * j + half];
+    if constexpr (G > 1) {
+      if (bad_do) {                            // the wave's own rows
+#pragma unroll 1
+        for (int j = 0; j < 4; j++)
+#pragma unroll 1
+          for (int c = l; c < 128; c += 64) drop_nonfinite(smem + j * 16384 + 2048 * wave + c * 16);
+      }
+    }
+  };
+  put_do(doreg);
+  __syncthreads();
+  {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) {
+        xo[c][ks] = tr_pair(smem + (wave >> 1) * 16384 + ks * 4096 + tr_off(l, 4 * (wave & 1) + 2 * c));
+        asm volatile("" : "+v"(xo[c][ks]));
+      }
+  }
+  __syncthreads();
+  put_do(dkeep);
+
+  const int ln = fresh_lane();
+  const int lm = ln & 15, lk = ln >> 4, lg = ln >> 5;
 
   // accumulator i of a lane is head 16 wave + 4 lk + i, for key 16 kt + lm
   unsigned boff[2], loff[2];                   // row operands of even and odd 32 columns: of a key, of the lane's head
