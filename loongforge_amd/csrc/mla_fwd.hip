@@ -247,9 +247,15 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   int* tlist = (int*)(tmask + NT);
   int* ntile_s = tlist + NT;
 
-  // ---- Q of the workgroup's heads, requested before the ids are staged so that both come back in one round trip
-  // to memory: 32-head blocks in the tiles' layout, where tiles 2 and 3 will lie.  (mla_fwd_wide_kernel gains nothing from
-  // this: its queries come in rounds of 256 and their rows at the rate of the memory, 3.33 ms either way.) ----------
+  // ---- The ids and Q of the workgroup's heads, requested together so that both come back in one round trip to memory: Q as
+  // 32-head blocks in the tiles' layout, where tiles 2 and 3 will lie.  The ids first, so that the list is made and the first tiles start
+  // while Q arrives: 200 queries x 32 heads x 512 slots 27.5 -> 26.2 us.  A range of a query is short, its Q comes with it, and there Q
+  // goes first (61 queries x 64 heads in two ranges 24.9 us, 25.3 the other way).  (Q through LDS gains nothing in mla_fwd_wide_kernel:
+  // its queries come in rounds of 256 and their rows at the rate of the memory, 3.33 ms either way.) ----------
+  const int* const ids = a.ids + (size_t)qi * K + k0;
+  int first[8];
+  if (!SPLIT) request_first_ids(ids, 0, KL, first);
+  __builtin_amdgcn_sched_barrier(0);
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   const int h = hb * 32 + r;
   const bool head_ok = h < H;
@@ -259,7 +265,8 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- stage the ids, mark valid slots, list the tiles that have any ---------------------
-  const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, qpos, idx_s, tmask, tlist, ntile_s);
+  if (SPLIT) request_first_ids(ids, 0, KL, first);
+  const int ntiles = stage_from_first_ids(first, ids, 0, KL, a.Skv, qpos, idx_s, tmask, tlist, ntile_s);
   const int nsteps = (ntiles + 1) / 2;
 
   // slots of tiles that are never visited still need their -inf in p_out
@@ -554,6 +561,10 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
   int* tlist = (int*)(tmask + NT);
   float* const inv_s = (float*)pbuf;         // after the last tile
 
+  const int* const ids = a.ids + (size_t)qi * K + k0;
+  int first[8];
+  if (!SPLIT) request_first_ids(ids, 0, KL, first);
+  __builtin_amdgcn_sched_barrier(0);
   const int h = 32 * w + r;                  // of the scores
   const bool head_ok = h < H;                // the same for all lanes of a wave
   bf16x8 qreg[SCORES ? KSTEPS : 1];
@@ -563,7 +574,8 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
     for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
     __builtin_amdgcn_sched_barrier(0);
   }
-  const int ntiles = stage_ids(a.ids + (size_t)qi * K + k0, 0, KL, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  if (SPLIT) request_first_ids(ids, 0, KL, first);
+  const int ntiles = stage_from_first_ids(first, ids, 0, KL, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
   if constexpr (SCORES) {
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
@@ -848,13 +860,17 @@ static_assert(TILE_BYTES + 8192 * 4 + 8192 / BI * 8 + 16 <= HALF_LDS, "a tile an
 __device__ __forceinline__ int swz16(int r) { return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | (r & 1); }
 
 // stage_ids without the ids: the masks and the list of the tiles that have a valid slot
-__device__ __forceinline__ int stage_masks(const int* __restrict__ ids, int K, unsigned limit, unsigned* tmask, int* tlist, int* ntile_s) {
+// (v: the first eight loads of a thread, requested ahead of the operands as in request_first_ids: 2077 queries x 512 slots x 64 heads with
+// logits 145 -> 142 us)
+__device__ __forceinline__ void request_mask_ids(const int* __restrict__ ids, int K, int t0, int (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 64) + (int)(threadIdx.x & 63)];    // (under its condition each would be waited for by itself)
+}
+__device__ __forceinline__ int stage_masks(int (&v)[8], const int* __restrict__ ids, int K, unsigned limit, unsigned* tmask, int* tlist, int* ntile_s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int NT = K / BI;
   for (int t0 = wave * 64; t0 < K; t0 += 8 * 256) {          // eight loads in flight
-    int v[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 64) + lane];    // (under its condition each would be waited for by itself)
+    if (t0 >= 8 * 256) request_mask_ids(ids, K, t0, v);
     asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -908,6 +924,10 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
 
   const int h = 32 * HB * hg + 16 * hw + m;  // of the scores
   const bool head_ok = 32 * HB * hg + 16 * hw < H;           // the same for all lanes of a wave
+  const int* const row_ids = a.ids + (size_t)qi * K;
+  int first[8];
+  request_mask_ids(row_ids, K, w * 64, first);
+  __builtin_amdgcn_sched_barrier(0);
   bf16x8 qreg[KS];
   {
     const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : m)) * DQK) + kg;
@@ -915,8 +935,7 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
     for (int ks = 0; ks < KS; ks++) qreg[ks] = qp[4 * ks];
   }
   __builtin_amdgcn_sched_barrier(0);
-  const int* const row_ids = a.ids + (size_t)qi * K;
-  const int ntiles = stage_masks(row_ids, K, limit, tmask, tlist, tlist + NT);
+  const int ntiles = stage_masks(first, row_ids, K, limit, tmask, tlist, tlist + NT);
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qreg[ks]));
 

@@ -42,17 +42,26 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
   return (const T*)(((unsigned long long)hi << 32) | lo);
 }
 
+// stage_ids in two steps: the first 2048 ids requested ahead of a query's operands.  Loads come back in order: ids requested behind the operands
+// arrive only after them, and the tiles, which wait for the ids, start on their way only then.
+__device__ __forceinline__ void request_first_ids(const int* __restrict__ ids, int qi, int K, int (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min((int)threadIdx.x + i * 256, K - 1)];
+}
+
 // Stages the K ids of query qi in LDS (invalid slots become -1), builds the 32-bit validity mask
 // of every tile and the ordered list of tiles with at least one valid slot.  Returns the number
 // of such tiles.  Ends with a barrier.  K % 64 == 0.
-__device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, int K, int Skv, int qpos,
-                                         int* idx_s, unsigned* tmask, int* tlist, int* ntile_s) {
+__device__ __forceinline__ int stage_from_first_ids(int (&v)[8], const int* __restrict__ ids, int qi, int K, int Skv, int qpos,
+                                                    int* idx_s, unsigned* tmask, int* tlist, int* ntile_s) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int NT = K / BI;
   for (int t0 = tid; t0 < K; t0 += 8 * 256) {     // eight loads in flight per thread
-    int v[8];
+    if (t0 >= 8 * 256) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(t0 + i * 256, K - 1)];
+      for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(t0 + i * 256, K - 1)];
+    }
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const bool ok = (v[i] >= 0) && (v[i] < Skv) && (v[i] <= qpos);
@@ -80,6 +89,13 @@ __device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, in
   }
   __syncthreads();
   return *ntile_s;
+}
+
+__device__ __forceinline__ int stage_ids(const int* __restrict__ ids, int qi, int K, int Skv, int qpos,
+                                         int* idx_s, unsigned* tmask, int* tlist, int* ntile_s) {
+  int v[8];
+  request_first_ids(ids, qi, K, v);
+  return stage_from_first_ids(v, ids, qi, K, Skv, qpos, idx_s, tmask, tlist, ntile_s);
 }
 
 // stage_ids for 512 threads and at most 2048 slots, in two steps: the ids are requested before the operands of a query, so that
