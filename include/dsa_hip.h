@@ -210,6 +210,11 @@ int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const floa
 int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, int chunk_offset, int32_t* ks, int32_t* ke,
                        int32_t* total, void* stream);
 /*
+ * Windows of the queries [offset, offset + S) of one sequence over its compressed keys, `ratio` tokens to a key: ks[i] = 0, ke[i] =
+ * (offset + i + 1) / ratio, at least 1 and at most `keys`.
+ */
+int dsa_indexer_compressed_window(int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream);
+/*
  * Position of packed token t + offset inside its own sequence, t in [0, tokens) (0 past the last sequence).
  */
 int dsa_thd_positions(const void* cu, int cu_i64, int ncu, int tokens, int64_t offset, int32_t* positions, void* stream);

@@ -124,41 +124,50 @@ class CSAIndexerKernelFunction(torch.autograd.Function):
         softmax_scale = dim ** -0.5
         head_p = 32 if head <= 32 else 64
 
-        q = _pad_to(index_q.squeeze(1).to(torch.bfloat16), head_p, 1).contiguous()
-        k = index_k.squeeze(1).to(torch.bfloat16).contiguous()
-        w = _pad_to(weights.squeeze(1).float(), head_p, 1)
-        q_fp8, q_scale, weight_scaled = ops.quant_rowwise_e4m3_weights(q, w, softmax_scale)
-        k_fp8, k_scale = ops.quant_rowwise_e4m3(k)
-
-        row = torch.arange(sq, dtype=torch.int, device=device)
-        if packed_seq_params is not None:
-            cu_q = packed_seq_params.cu_seqlens_q_padded
-            if cu_q is None:
-                cu_q = packed_seq_params.cu_seqlens_q
-            cu_kv = packed_seq_params.cu_seqlens_kv_padded
-            if cu_kv is None:
-                cu_kv = packed_seq_params.cu_seqlens_kv
-            cu_q, cu_kv = cu_q.to(device).int(), cu_kv.to(device).int()
-            seg = _segment_of_row(cu_q, sq)
-            k_start = cu_kv[seg]
-            visible = torch.div(row - cu_q[seg] + 1, compress_ratio, rounding_mode="floor")
-            visible = torch.minimum(visible, (cu_kv[1:] - cu_kv[:-1])[seg])
-            visible = torch.where(row < cu_q[-1], visible, torch.zeros_like(visible))
-            k_end = k_start + visible
-            effective_topk = min(index_topk, int(packed_seq_params.max_seqlen_kv))
+        whole = None
+        if packed_seq_params is None and sk > 0 and type(sq_offset) is int and type(compress_ratio) is int and 0 < compress_ratio < 2 ** 31:
+            # quantisers, windows, logits and top-k in one native call (one launch for the windows instead of five)
+            whole = ops.indexer_forward(index_q.squeeze(1), index_k.squeeze(1), weights.squeeze(1), False, softmax_scale, None, sq_offset,
+                                        min(index_topk, sk), True, ratio=compress_ratio)
+        if whole is not None:
+            index_score_topk, topk_indices, q_fp8, q_scale, weight_scaled, k_fp8, k_scale, _ = whole
+            global_ids = topk_indices
         else:
-            k_start = torch.zeros(sq, dtype=torch.int, device=device)
-            k_end = torch.div(row + (sq_offset + 1), compress_ratio, rounding_mode="floor").clamp(min=1, max=sk)
-            effective_topk = min(index_topk, sk)
+            q = _pad_to(index_q.squeeze(1).to(torch.bfloat16), head_p, 1).contiguous()
+            k = index_k.squeeze(1).to(torch.bfloat16).contiguous()
+            w = _pad_to(weights.squeeze(1).float(), head_p, 1)
+            q_fp8, q_scale, weight_scaled = ops.quant_rowwise_e4m3_weights(q, w, softmax_scale)
+            k_fp8, k_scale = ops.quant_rowwise_e4m3(k)
 
-        # the reference asks for unsorted output, i.e. any slot order will do: the descending-score path of the
-        # top-k kernel is its fast one
-        index_score_topk, global_ids = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start.int(),
-                                                        k_end.int(), effective_topk, True)
-        if packed_seq_params is not None:
-            topk_indices = torch.where(global_ids >= 0, global_ids - k_start.unsqueeze(1), global_ids)
-        else:
-            topk_indices = global_ids
+            row = torch.arange(sq, dtype=torch.int, device=device)
+            if packed_seq_params is not None:
+                cu_q = packed_seq_params.cu_seqlens_q_padded
+                if cu_q is None:
+                    cu_q = packed_seq_params.cu_seqlens_q
+                cu_kv = packed_seq_params.cu_seqlens_kv_padded
+                if cu_kv is None:
+                    cu_kv = packed_seq_params.cu_seqlens_kv
+                cu_q, cu_kv = cu_q.to(device).int(), cu_kv.to(device).int()
+                seg = _segment_of_row(cu_q, sq)
+                k_start = cu_kv[seg]
+                visible = torch.div(row - cu_q[seg] + 1, compress_ratio, rounding_mode="floor")
+                visible = torch.minimum(visible, (cu_kv[1:] - cu_kv[:-1])[seg])
+                visible = torch.where(row < cu_q[-1], visible, torch.zeros_like(visible))
+                k_end = k_start + visible
+                effective_topk = min(index_topk, int(packed_seq_params.max_seqlen_kv))
+            else:
+                k_start = torch.zeros(sq, dtype=torch.int, device=device)
+                k_end = torch.div(row + (sq_offset + 1), compress_ratio, rounding_mode="floor").clamp(min=1, max=sk)
+                effective_topk = min(index_topk, sk)
+
+            # the reference asks for unsorted output, i.e. any slot order will do: the descending-score path of the
+            # top-k kernel is its fast one
+            index_score_topk, global_ids = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start.int(),
+                                                            k_end.int(), effective_topk, True)
+            if packed_seq_params is not None:
+                topk_indices = torch.where(global_ids >= 0, global_ids - k_start.unsqueeze(1), global_ids)
+            else:
+                topk_indices = global_ids
         ctx.softmax_scale = softmax_scale
         ctx.head = head
         ctx.in_dtypes = (index_q.dtype, index_k.dtype, weights.dtype)

@@ -399,16 +399,17 @@ def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offse
 
 
 def indexer_forward(index_q, index_k, weights, rotate: bool, factor: float, cu_seqlens, chunk_offset: int, K: int, sorted: bool, front=None,
-                    ln_weight=None, ln_bias=None):
+                    ln_weight=None, ln_bias=None, ratio: int = 0):
     """Quantisers (with ``front``, an ``IndexerFrontEnd``, behind the front end), :func:`indexer_window` and :func:`indexer_topk` of bf16
     ``index_q [S, 32 or 64, 128]`` and ``index_k [Sk, 128]`` in one native call: (scores, ids, q8, q_scale, scaled weights, k8,
-    k_scale, check or None); None for other arguments and for calls that are not eager ones on ordinary tensors."""
+    k_scale, check or None); None for other arguments and for calls that are not eager ones on ordinary tensors.  ``ratio`` > 0: one
+    sequence, query ``i`` sees the first ``(chunk_offset + i + 1) // ratio`` keys, at least one."""
     if torch.compiler.is_compiling():
         return None
     f = front
     return _native().indexer_forward(index_q, index_k, weights, bool(rotate), float(factor), cu_seqlens, int(chunk_offset), int(K), bool(sorted),
                                      f and f.cos, f and f.sin, f.pairing if f else -1, f and f.positions_q, f and f.positions_k,
-                                     f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0)
+                                     f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0, int(ratio))
 
 
 # --------------------------------------------------------------------------------------------

@@ -69,6 +69,41 @@ def test_csa_indexer_single_sequence(gpu, sq, ratio, topk, offset, heads):
     _check_backward(q, k, wt, sc, ids.cpu(), aux, seed=13)
 
 
+@pytest.mark.parametrize("sq,ratio,sk,topk,offset,heads,dtype", [
+    (257, 4, 64, 32, 0, 64, torch.bfloat16),
+    (300, 4, 128, 512, 212, 32, torch.bfloat16),      # a chunk behind others; fewer keys than slots
+    (200, 7, 20, 64, 5, 64, torch.float32),           # weights of another type; windows that end before the keys do and behind them
+    (5, 128, 3, 2, 0, 32, torch.bfloat16),            # no query has a whole key
+    (1, 1, 1, 1, 0, 64, torch.bfloat16),
+])
+def test_csa_indexer_in_one_call_is_that_of_separate_calls(gpu, monkeypatch, sq, ratio, sk, topk, offset, heads, dtype):
+    """Scores, ids and gradients bit for bit, on contiguous tensors and on strided ones."""
+    from loongforge_amd import ops
+    from loongforge_amd.csa_kernels import CSAIndexerKernel
+
+    g = torch.Generator().manual_seed(sq)
+    q = torch.randn(sq, 2, heads, 128, generator=g).bfloat16().to(gpu)[:, :1]
+    k = torch.randn(sk, 2, 128, generator=g).bfloat16().to(gpu)[:, 1:]
+    w = torch.randn(sq, 1, heads, generator=g).to(dtype).to(gpu)
+    whole, taken = ops.indexer_forward, []
+
+    def run(forward):
+        monkeypatch.setattr(ops, "indexer_forward", forward)
+        args = [t.detach().requires_grad_(True) for t in (q, k, w)]
+        scores, ids = CSAIndexerKernel(ratio)(*args, topk, offset)
+        d = torch.where(ids >= 0, torch.arange(scores.numel(), device=gpu).view(scores.shape) % 7 - 3.0, 0.0)
+        return [scores.detach(), ids, *torch.autograd.grad(scores, args, d)]
+
+    def counted(*a, **kw):
+        taken.append(whole(*a, **kw))
+        return taken[-1]
+
+    got, want = run(counted), run(lambda *a, **kw: None)
+    assert taken[0] is not None
+    for x, y in zip(got, want):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+
+
 def test_csa_indexer_packed_returns_segment_local_ids(gpu):
     from loongforge_amd.csa_kernels import CSAIndexerKernel
     from loongforge_amd.megatron_compat import PackedSeqParams
