@@ -210,10 +210,14 @@ int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const floa
 int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, int chunk_offset, int32_t* ks, int32_t* ke,
                        int32_t* total, void* stream);
 /*
- * Windows of the queries [offset, offset + S) of one sequence over its compressed keys, `ratio` tokens to a key: ks[i] = 0, ke[i] =
- * (offset + i + 1) / ratio, at least 1 and at most `keys`.
+ * What the indexer's logits wait for, in one launch: dsa_quant_rowwise_e4m3_weights of the query rows q (weights fp32, or bf16 if
+ * weights_bf16), the same quantiser of the key rows k, both behind the Hadamard rotation if rotate, and the windows of S queries
+ * [offset, offset + S) of one sequence: ks[i] = 0, ke[i] = offset + i + 1, or over compressed keys, ratio > 0 tokens to a key,
+ * ke[i] = (offset + i + 1) / ratio, at least 1 and at most `keys`.  Rows of 128 bf16 values.
  */
-int dsa_indexer_compressed_window(int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream);
+int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void* k, int64_t k_rows, int rotate, void* q8, float* q_scale, void* k8,
+                            float* k_scale, float eps, int pow2, const void* weights, int weights_bf16, float factor,
+                            float* weight_scaled, int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream);
 /*
  * Position of packed token t + offset inside its own sequence, t in [0, tokens) (0 past the last sequence).
  */

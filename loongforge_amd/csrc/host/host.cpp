@@ -444,15 +444,6 @@ Window key_windows(const OptTensor& cu_, int64_t S, int64_t chunk_offset, const 
   return {window, std::move(check)};
 }
 
-// Of one sequence over compressed keys, `ratio` tokens to a key
-Window compressed_windows(int64_t S, int64_t offset, int64_t ratio, int64_t keys, const Tensor& like) {
-  Call call(like);
-  Tensor window = make({2, S}, at::kInt, like);
-  run("dsa_indexer_compressed_window", dsa_indexer_compressed_window, (int)S, offset, (int)ratio, (int)keys, out_ptr<int32_t>(window),
-      out_ptr<int32_t>(window) + S, call.stream);
-  return {window, std::make_unique<WindowCheck>()};
-}
-
 py::tuple indexer_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, const Tensor& like) {
   Window w = key_windows(cu, S, chunk_offset, like);
   return py::make_tuple(w.bounds.select(0, 0), w.bounds.select(0, 1), std::move(w.check));
@@ -460,8 +451,9 @@ py::tuple indexer_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, c
 
 // The indexer's forward in one call: quantisers (behind the front end if there are rotary tables, else behind the rotation if
 // asked for), key windows, logits and top-k.  Five calls from Python cost 35 - 40 us of host time, more than the kernels of a few
-// queries take.  ratio > 0: the windows are those over compressed keys.  None for shapes and types that need padding or conversion first.  -> (scores, ids, q8, q_scale, scaled weights,
-// k8, k_scale, check or None): check.wait() belongs behind it, as with indexer_window.
+// queries take.  ratio > 0: the windows are those over compressed keys.  None for shapes and types that need padding or conversion
+// first.  -> (scores, ids, q8, q_scale, scaled weights, k8, k_scale, check or None): check.wait() belongs behind it, as with
+// indexer_window.
 py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weights, bool rotate, double factor, const OptTensor& cu,
                            int64_t chunk_offset, int64_t K, bool sort, const OptTensor& cos, const OptTensor& sin, int64_t pairing,
                            const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& ln_weight,
@@ -469,23 +461,32 @@ py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weigh
   if (!plain(q, k, weights, cu, cos, sin, positions_q, positions_k, ln_weight, ln_bias)) return py::none();
   if (!q.is_cuda() || q.dim() != 3 || k.dim() != 2 || q.size(2) != 128 || k.size(1) != 128 || (q.size(1) != 32 && q.size(1) != 64) ||
       q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || weights.sizes() != q.sizes().slice(0, 2)) return py::none();
-  using Three = std::tuple<Tensor, Tensor, Tensor>;
   using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
   Tensor q8, q_scale, scaled, k8, k_scale, rows;
+  Window w;
   if (cos) {
     std::tie(q8, q_scale, rows, scaled) = py::cast<Four>(indexer_front(q, q.size(1), {}, {}, 0.0, cos, sin, pairing, positions_q, batch, rotate,
                                                                        weights, factor, true, false, 1e-12, true, false));
     std::tie(k8, k_scale, rows, rows) = py::cast<Four>(indexer_front(k, 1, ln_weight, ln_bias, ln_eps, cos, sin, pairing, positions_k, batch, rotate,
                                                                      {}, 1.0, true, false, 1e-12, true, false));
   } else {
-    std::tie(q8, q_scale, scaled) = py::cast<Three>(quant_weights(q, weights, factor, rotate, 1e-12, true, false));
-    if (rotate) std::tie(k8, k_scale, rows) = py::cast<Three>(rotate_quant(k, 1e-12, true, true, false, false));
-    else std::tie(k8, k_scale) = py::cast<std::pair<Tensor, Tensor>>(quant_rowwise(k, 1e-12, true, false));
+    need_gpus(q, k, weights);
+    const Tensor qc = q.contiguous(), kc = k.contiguous();
+    const Tensor wc = weights.scalar_type() == at::kBFloat16 ? weights.contiguous() : f32(weights);
+    const int64_t S = q.size(0);
+    Call call(qc);
+    q8 = make(qc.sizes(), at::kFloat8_e4m3fn, qc); q_scale = make(weights.sizes(), at::kFloat, qc); scaled = make(weights.sizes(), at::kFloat, qc);
+    k8 = make(kc.sizes(), at::kFloat8_e4m3fn, kc); k_scale = make({kc.size(0)}, at::kFloat, kc);
+    w.bounds = make({2, S}, at::kInt, qc);
+    run("dsa_indexer_inputs_e4m3", dsa_indexer_inputs_e4m3, qc.const_data_ptr(), qc.numel() / 128, kc.const_data_ptr(), kc.size(0), rotate,
+        out_ptr<void>(q8), out_ptr<float>(q_scale), out_ptr<void>(k8), out_ptr<float>(k_scale), 1e-12f, 1, wc.const_data_ptr(),
+        wc.scalar_type() == at::kBFloat16, (float)factor, out_ptr<float>(scaled), cu ? 0 : (int)S, chunk_offset, (int)ratio, (int)kc.size(0),
+        out_ptr<int32_t>(w.bounds), out_ptr<int32_t>(w.bounds) + S, call.stream);
   }
-  Window w = ratio ? compressed_windows(q.size(0), chunk_offset, ratio, k.size(0), q8) : key_windows(cu, q.size(0), chunk_offset, q8);
+  if (cu || cos) w = key_windows(cu, q.size(0), chunk_offset, q8);
   const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
       indexer_topk(q8, scaled, k8, k_scale, w.bounds.select(0, 0), w.bounds.select(0, 1), K, sort, false));
-  return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale, w.check->done ? py::cast(std::move(w.check)) : py::none());
+  return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale, w.check && w.check->done ? py::cast(std::move(w.check)) : py::none());
 }
 
 py::object thd_positions(const Tensor& cu_, int64_t tokens, int64_t offset) {

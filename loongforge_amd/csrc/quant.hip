@@ -13,12 +13,20 @@ __device__ __forceinline__ float wave_max16(float v) {   // max over the 16 lane
   return v;
 }
 
+// A weight per row: fp32, or bf16 as it came
+struct F32Weight { const float* p; __device__ float operator[](int64_t i) const { return p[i]; } };
+struct AnyWeight {
+  const void* p;
+  bool bf16;
+  __device__ float operator[](int64_t i) const { return bf16 ? bf16_bits_to_f32(((const unsigned short*)p)[i]) : ((const float*)p)[i]; }
+};
+
 // cols == 128: 16 lanes per row, 4 rows per wave, 16 rows per 256-thread block.
-__global__ __launch_bounds__(256) void quant128_kernel(const uint4* __restrict__ x, uint2* __restrict__ x8,
-                                                       float* __restrict__ scale_inv, int64_t rows,
-                                                       float eps, int pow2, const float* __restrict__ w_in,
-                                                       float w_factor, float* __restrict__ w_scaled) {
-  int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+template <class W>
+__device__ __forceinline__ void quant128_rows(unsigned block, const uint4* __restrict__ x, uint2* __restrict__ x8,
+                                              float* __restrict__ scale_inv, int64_t rows, float eps, int pow2, W w_in, float w_factor,
+                                              float* __restrict__ w_scaled) {
+  int64_t row = (int64_t)block * 16 + (threadIdx.x >> 4);
   int sub = threadIdx.x & 15;
   bool live = row < rows;
   uint4 raw = live ? x[row * 16 + sub] : make_uint4(0, 0, 0, 0);
@@ -54,17 +62,23 @@ __global__ __launch_bounds__(256) void quant128_kernel(const uint4* __restrict__
   }
 }
 
+__global__ __launch_bounds__(256) void quant128_kernel(const uint4* __restrict__ x, uint2* __restrict__ x8,
+                                                       float* __restrict__ scale_inv, int64_t rows,
+                                                       float eps, int pow2, const float* __restrict__ w_in,
+                                                       float w_factor, float* __restrict__ w_scaled) {
+  quant128_rows(blockIdx.x, x, x8, scale_inv, rows, eps, pow2, F32Weight{w_in}, w_factor, w_scaled);
+}
+
 // Hadamard rotation of a 128-element row (Sylvester order, scaled by 128^-0.5, rounded to bf16 as the
 // unfused sequence "fp32 product with the Hadamard matrix -> bf16" does) followed by the same
 // quantiser.  The butterfly runs over the 7 index bits: 3 inside a lane's 8 elements, 4 across the
 // 16 lanes of a row.  Either output may be absent (x8 == nullptr: rotation only; y == nullptr:
 // quantised payload only).
-__global__ __launch_bounds__(256) void rotate_quant128_kernel(const uint4* __restrict__ x, uint2* __restrict__ x8,
-                                                              float* __restrict__ scale_inv, uint4* __restrict__ y,
-                                                              int64_t rows, float eps, int pow2,
-                                                              const float* __restrict__ w_in, float w_factor,
-                                                              float* __restrict__ w_scaled) {
-  int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+template <class W>
+__device__ __forceinline__ void rotate_quant128_rows(unsigned block, const uint4* __restrict__ x, uint2* __restrict__ x8,
+                                                     float* __restrict__ scale_inv, uint4* __restrict__ y, int64_t rows, float eps, int pow2,
+                                                     W w_in, float w_factor, float* __restrict__ w_scaled) {
+  int64_t row = (int64_t)block * 16 + (threadIdx.x >> 4);
   int sub = threadIdx.x & 15;
   bool live = row < rows;
   uint4 raw = live ? x[row * 16 + sub] : make_uint4(0, 0, 0, 0);
@@ -121,6 +135,50 @@ __global__ __launch_bounds__(256) void rotate_quant128_kernel(const uint4* __res
   }
 }
 
+__global__ __launch_bounds__(256) void rotate_quant128_kernel(const uint4* __restrict__ x, uint2* __restrict__ x8,
+                                                              float* __restrict__ scale_inv, uint4* __restrict__ y,
+                                                              int64_t rows, float eps, int pow2,
+                                                              const float* __restrict__ w_in, float w_factor,
+                                                              float* __restrict__ w_scaled) {
+  rotate_quant128_rows(blockIdx.x, x, x8, scale_inv, y, rows, eps, pow2, F32Weight{w_in}, w_factor, w_scaled);
+}
+
+// What the indexer's logits wait for, side by side in one launch: the quantised queries with their weights, the quantised keys, and the
+// windows of one sequence.  Each part alone fills a fraction of the chip for a chunk of a prompt, and takes its 3 - 5 us behind the
+// other two.  The whole pass, us, as three launches and as one: chunks of a few dozen tokens 76.5 and 68.8, 61 tokens x 64 heads behind
+// 20 000 82.2 and 78.0, 1500 behind 6692 1014 and 1010, 3072 queries over compressed keys, forward and backward, 1567 and 1564.
+struct InputArgs {
+  const uint4 *q, *k;
+  uint2 *q8, *k8;
+  float *q_scale, *k_scale;
+  int64_t q_rows, k_rows;
+  AnyWeight w_in;
+  float w_factor;
+  float* w_scaled;
+  unsigned q_blocks, k_blocks;
+  float eps;
+  int pow2;
+  int S, ratio, keys;
+  long long offset;
+  int *ks, *ke;
+};
+template <bool ROTATE>
+__global__ __launch_bounds__(256) void indexer_inputs_kernel(const InputArgs a) {
+  const unsigned b = blockIdx.x;
+  if (b < a.q_blocks) {
+    if (ROTATE) rotate_quant128_rows(b, a.q, a.q8, a.q_scale, nullptr, a.q_rows, a.eps, a.pow2, a.w_in, a.w_factor, a.w_scaled);
+    else quant128_rows(b, a.q, a.q8, a.q_scale, a.q_rows, a.eps, a.pow2, a.w_in, a.w_factor, a.w_scaled);
+  } else if (b < a.q_blocks + a.k_blocks) {
+    if (ROTATE) rotate_quant128_rows(b - a.q_blocks, a.k, a.k8, a.k_scale, nullptr, a.k_rows, a.eps, a.pow2, F32Weight{nullptr}, 0.f, nullptr);
+    else quant128_rows(b - a.q_blocks, a.k, a.k8, a.k_scale, a.k_rows, a.eps, a.pow2, F32Weight{nullptr}, 0.f, nullptr);
+  } else {
+    const int i = (int)(b - a.q_blocks - a.k_blocks) * 256 + (int)threadIdx.x;
+    if (i >= a.S) return;
+    const long long end = a.offset + i + 1;
+    a.ks[i] = 0;
+    a.ke[i] = (int)(a.ratio ? min(max(end / a.ratio, 1ll), (long long)a.keys) : end);
+  }
+}
 
 // The quantiser over rows that are padded on the way: token t's heads_in rows of dim_in elements become heads_out rows of 128,
 // zeros in between (as if the bf16 tensor had been padded first: zero rows get the scale of the epsilon floor, and the
@@ -327,6 +385,25 @@ extern "C" int dsa_rotate_quant_e4m3(const void* x, int64_t rows, int cols, void
   rotate_quant128_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(
       (const uint4*)x, (uint2*)x8, scale_inv, (uint4*)y, rows, eps, pow2, nullptr, 0.f, nullptr);
   DSA_CHECK_LAUNCH("dsa_rotate_quant_e4m3");
+  return DSA_OK;
+}
+
+extern "C" int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void* k, int64_t k_rows, int rotate, void* q8, float* q_scale, void* k8,
+                                       float* k_scale, float eps, int pow2, const void* weights, int weights_bf16, float factor,
+                                       float* weight_scaled, int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream) {
+  DSA_REQUIRE(q_rows >= 0 && k_rows >= 0 && S >= 0 && ratio >= 0 && keys >= 0, "dsa_indexer_inputs_e4m3: bad sizes");
+  DSA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)q8 % 8) == 0 && ((uintptr_t)k8 % 8) == 0,
+              "dsa_indexer_inputs_e4m3: misaligned pointer");
+  DSA_REQUIRE(q_rows == 0 || (q && q8 && q_scale && weights && weight_scaled), "dsa_indexer_inputs_e4m3: null pointer");
+  DSA_REQUIRE((k_rows == 0 || (k && k8 && k_scale)) && (S == 0 || (ks && ke)), "dsa_indexer_inputs_e4m3: null pointer");
+  const int64_t q_blocks = (q_rows + 15) / 16, k_blocks = (k_rows + 15) / 16, blocks = q_blocks + k_blocks + dsa_cdiv(S, 256);
+  DSA_REQUIRE(blocks < (1ll << 31), "dsa_indexer_inputs_e4m3: too many rows");
+  if (blocks == 0) return DSA_OK;
+  const InputArgs a{(const uint4*)q, (const uint4*)k, (uint2*)q8, (uint2*)k8, q_scale, k_scale, q_rows, k_rows, {weights, weights_bf16 != 0}, factor,
+                    weight_scaled, (unsigned)q_blocks, (unsigned)k_blocks, eps, pow2, S, ratio, keys, offset, ks, ke};
+  if (rotate) indexer_inputs_kernel<true><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
+  else indexer_inputs_kernel<false><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
+  DSA_CHECK_LAUNCH("dsa_indexer_inputs_e4m3");
   return DSA_OK;
 }
 

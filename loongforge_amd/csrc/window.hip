@@ -38,14 +38,6 @@ __global__ __launch_bounds__(256) void window_kernel(const T* __restrict__ cu, i
   ke[i] = end;
 }
 
-__global__ __launch_bounds__(256) void compressed_window_kernel(int S, long long offset, int ratio, int keys, int* __restrict__ ks,
-                                                                int* __restrict__ ke) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= S) return;
-  ks[i] = 0;
-  ke[i] = (int)min(max((offset + i + 1) / ratio, 1ll), (long long)keys);
-}
-
 template <typename T>
 __global__ void positions_kernel(const T* __restrict__ cu, int ncu, int tokens, long long offset, int* __restrict__ pos) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -65,14 +57,6 @@ extern "C" int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, in
   if (cu_i64) window_kernel<long long><<<grid, 256, 0, (hipStream_t)stream>>>((const long long*)cu, ncu, S, chunk_offset, ks, ke, total);
   else window_kernel<int><<<grid, 256, 0, (hipStream_t)stream>>>((const int*)cu, ncu, S, chunk_offset, ks, ke, total);
   DSA_CHECK_LAUNCH("indexer_window");
-  return DSA_OK;
-}
-
-extern "C" int dsa_indexer_compressed_window(int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream) {
-  DSA_REQUIRE(S >= 0 && ratio > 0 && keys >= 0, "indexer_compressed_window: bad sizes");
-  if (S == 0) return DSA_OK;
-  compressed_window_kernel<<<dim3(dsa_cdiv(S, 256)), 256, 0, (hipStream_t)stream>>>(S, offset, ratio, keys, ks, ke);
-  DSA_CHECK_LAUNCH("indexer_compressed_window");
   return DSA_OK;
 }
 

@@ -490,3 +490,32 @@ def test_native_host_layer_equals_the_registered_ops(gpu):
         ops.topk(logits.double(), 4)
     with pytest.raises(ValueError, match="dsa_topk"):
         ops.topk(logits, 0)
+
+
+@pytest.mark.parametrize("S,Sk,heads,rotate,bf16_weights,offset,ratio", [
+    (1, 1, 32, True, False, 0, 0),
+    (61, 300, 64, True, True, 239, 0),
+    (255, 257, 32, False, True, 2, 0),               # windows and rows that end inside a workgroup
+    (257, 64, 64, False, False, 0, 4),
+    (512, 40, 32, True, True, 100, 15),              # windows beyond the last compressed key are cut there
+    (9, 2, 64, False, True, 0, 1000),                # no query has a whole compressed key
+])
+def test_indexer_inputs_in_one_launch_are_those_of_separate_launches(gpu, S, Sk, heads, rotate, bf16_weights, offset, ratio):
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(S)
+    q = torch.randn(S, heads, 128, generator=g).bfloat16().to(gpu)
+    k = torch.randn(Sk, 128, generator=g).bfloat16().to(gpu)
+    w = torch.randn(S, heads, generator=g).to(torch.bfloat16 if bf16_weights else torch.float32).to(gpu)
+    K = min(64, Sk)
+    got = ops.indexer_forward(q, k, w, rotate, 0.1, None, offset, K, True, ratio=ratio)
+    q8, q_scale, scaled = ops.quant_rowwise_e4m3_weights(q, w.float(), 0.1, rotate)
+    k8, k_scale = (ops.rotate_quant_e4m3 if rotate else ops.quant_rowwise_e4m3)(k)
+    end = torch.arange(S, device=gpu, dtype=torch.int32) + offset + 1
+    if ratio:
+        end = torch.div(end, ratio, rounding_mode="floor").clamp(min=1, max=Sk)
+    scores, ids = ops.indexer_topk(q8, scaled, k8, k_scale, torch.zeros_like(end), end, K, True)
+    for x, y in zip(got, (scores, ids, q8, q_scale, scaled, k8, k_scale)):
+        x, y = (t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t for t in (x, y))
+        assert x.dtype == y.dtype and torch.equal(x, y)
+    assert got[7] is None
