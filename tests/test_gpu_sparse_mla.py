@@ -429,7 +429,7 @@ def _joint_groups(ids, H):
         rows = [r[r >= 0] for r in ids[g * G:(g + 1) * G]]
         tiles = (len(torch.unique(torch.cat(rows))) + 31) // 32
         one_by_one = sum(int((226 if H == 64 else 140) * apart) + int((50 if H == 64 else 48) * apart) * ((len(r) + 31) // 32) for r in rows if len(r))
-        joint += 0 < 32 * tiles <= 3072 and int(420 * wide) + int(66 * wide) * tiles <= one_by_one
+        joint += 64 < 32 * tiles <= 3072 and int(420 * wide) + int(66 * wide) * tiles <= one_by_one
     return joint, full
 
 
