@@ -16,6 +16,7 @@
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
 #include <algorithm>
+#include <type_traits>
 
 #include "mla_tile.h"
 #include "order.h"
@@ -28,6 +29,7 @@ using namespace mla;
 constexpr int pds_kind_bytes(int HG) { return HG * 2048; }
 inline int head_groups(int H) { return H <= 32 ? 1 : H <= 64 ? 2 : 4; }
 constexpr int ROW_BYTES = DQK * 2;           // one pair row of the dKV buffer
+constexpr int EXP_BYTES = 16;                // its exponents where rows may be those of joint units: see below
 constexpr int PDS_THREADS = 512;
 
 // Joint units.  With 64 or 32 heads, 2 or 4 consecutive queries may be worked as one query of 128 heads: their rows of Q, dO, O, lse and
@@ -42,6 +44,14 @@ constexpr int PDS_THREADS = 512;
 // 1010 / 507 / 506; 2077 x 512 at random, 64 heads (0.73) 827 / 775 / 736, 32 heads (0.48) 683 / 512 / 494; 4000 x 512, 64 heads (0.83)
 // 1557 / 1619 / 1504, 32 heads (0.63) 1301 / 1178 / 1145; 8000 x 256, 64 heads (0.94) 1970 / 2189 / 1969; 3000 x 2048, 32 heads (0.28)
 // 2483 / 1105 / 1113.
+//
+// A unit's row stands for 2 or 4 rows, so it is held in more bits than they: 11 instead of 8 significant ones, fp16 with a power of
+// two for every 64 columns (16 of the rotary part), chosen so that the largest of them lies in [2^14, 2^15).  Values down to 2^-29 of that
+// one have all 11 bits.  The power's fp32 exponent is one of EXP_BYTES bytes per row: groups 0 - 7 the 64-column groups, 8 - 11 the
+// rotary ones; 0 marks a bf16 row, one of a query by itself.  In bf16 the rows' rounding error would be that of the rows it stands for only
+// where those are independent, and grows with what neighbouring queries have in common: rms over 256 queries x 256 of 288 slots, rows per query 1,
+// unit in bf16 / fp16: correlation 0 of Q and dO 1.00 / 0.13, 0.9 1.27 / 0.16 (64 heads) and 1.68 / 0.21 (32 heads), 0.99 1.36 / 0.17 and 1.88 /
+// 0.24.
 constexpr int unit_queries(int HG) { return 4 / HG; }
 constexpr int UNIT_SLOTS = 3072;             // what the lists in LDS behind the operands of 128 heads have room for
 constexpr int UNIT_KEY = 0xffffff;
@@ -270,11 +280,11 @@ static_assert(64 * (DQK + DV) * 2 <= FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH +
 __host__ __device__ inline size_t fused_lds_bytes(int K) {
   return (size_t)FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT + ids_lds_bytes(K) + 512 + (size_t)K * 4;
 }
-template <int hh, int HG>                    // HG: groups of 32 heads, 2 or 1
+template <int hh, int HG, bool MARK>         // HG: groups of 32 heads, 2 or 1; MARK: the rows have exponents
 __device__ __forceinline__ void pds_rows_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, unsigned char* __restrict__ exps,
     int q0, int ql, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
   constexpr int H = 32 * HG, KS = DQK / 32, VS = DV / 32, STAGES = FUSED_STAGES;
   constexpr int DO_ACC = 12;                   // steps of dO in accumulation registers, beside all of Q: 120
@@ -326,7 +336,10 @@ __device__ __forceinline__ void pds_rows_body(
   const int ntiles = stage_requested_ids(slot_id, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
 #pragma unroll
   for (int i = 0; i < 4; i++)                  // invalid slots land in a scratch row: the store count stays fixed
-    if (tid + 512 * i < K) dst_s[tid + 512 * i] = slot_row[i] >= 0 ? slot_row[i] : dummy_row;
+    if (tid + 512 * i < K) {
+      dst_s[tid + 512 * i] = slot_row[i] >= 0 ? slot_row[i] : dummy_row;
+      if (MARK && slot_row[i] >= 0) *(uint4*)(exps + (size_t)slot_row[i] * EXP_BYTES) = make_uint4(0u, 0u, 0u, 0u);
+    }
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();
@@ -552,8 +565,33 @@ constexpr int WIDE_XCH = WIDE_TILE + TILE_BYTES;
 constexpr int WIDE_LISTS = 128 * DQK * 2;              // Q of the query fits in front of the lists before the rest is there
 static_assert(WIDE_XCH + 2 * pds_kind_bytes(4) <= WIDE_LISTS && WIDE_TILE + 65536 <= WIDE_LISTS, "the lists lie behind everything else");
 inline size_t wide_lds_bytes(int K) { return (size_t)WIDE_LISTS + ids_lds_bytes(K) + 1024 + 2048; }
-inline size_t unit_lds_bytes(int slots) { return (size_t)WIDE_LISTS + (size_t)slots * 4 + 1024 + 2048; }
-static_assert(WIDE_LISTS + UNIT_SLOTS * 4 + 1024 + 2048 <= 160 * 1024, "the list of a joint unit");
+__host__ __device__ constexpr size_t unit_lds_bytes(int slots) { return (size_t)WIDE_LISTS + (size_t)slots * 4 + 1024 + 2048 + BI * EXP_BYTES; }
+static_assert(unit_lds_bytes(UNIT_SLOTS) <= 160 * 1024, "the list of a joint unit");
+
+// Exponent of the power of two that a group of columns of a unit's row is divided by.  group_max: the largest magnitude over the 16 values of
+// every lane with the same lane % 16; values that are not finite do not count, they stay what they are in fp16.
+template <int N>
+__device__ __forceinline__ float group_max(const f32x4 (&x)[N]) {
+  float most = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(x[i][e]), "v"(x[i][e + 1]));      // (NaN does not count)
+  if (__any(most == INFINITY)) {
+    most = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) most = fabsf(x[i][e]) < INFINITY ? fmaxf(most, fabsf(x[i][e])) : most;
+  }
+  float other = most;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(most), "+v"(other));
+  most = other = fmaxf(most, other);
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(most), "+v"(other));
+  return fmaxf(most, other);
+}
+__device__ __forceinline__ int group_exponent(float most) { return max((int)(__builtin_bit_cast(unsigned, most) >> 23) - 14, 1); }
+__device__ __forceinline__ float group_scale(int exponent) { return __builtin_bit_cast(float, (unsigned)(254 - exponent) << 23); }
 
 // Zero where a bf16 value is not finite (exponent all ones), in 16 bytes of LDS
 __device__ __forceinline__ void drop_nonfinite(unsigned char* p) {
@@ -575,7 +613,7 @@ template <int hh, int G>
 __device__ __forceinline__ void pds_rows_wide_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, unsigned char* __restrict__ exps,
     int H, int Skv, int K, int qpos, float sm_scale, int dummy_row, unsigned char* smem) {
   constexpr int VS = DV / 32;
   constexpr int XQ_ACC = 7;                    // column operands of Q in accumulation registers, beside all row operands: 124
@@ -589,6 +627,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
   int* ntile_s = tlist + NT;
   float* stat_s = G > 1 ? (float*)(idx_s + K) : (float*)(ntile_s + 4);       // [2][128]: lse * log2(e), delta
   int* dst_s = (int*)(stat_s + 256);           // [2][256]: destination rows from the tile's first slot on
+  unsigned char* exp_s = (unsigned char*)(dst_s + 512);                      // G > 1: [32][EXP_BYTES], exponents of the tile's rows
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   // Registers are short: what depends on the lane is worked out anew for every part.
   auto fresh_lane = []() {
@@ -886,23 +925,45 @@ __device__ __forceinline__ void pds_rows_wide_body(
       }
       asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
       unsigned char* row = rows + (size_t)(drow >= 0 ? drow : dummy_row) * ROW_BYTES;       // invalid slots: a scratch row
+      float scale = 1.f;
+      auto pack = [&](float a, float b) { return G > 1 ? cvt_pk_f16(a * scale, b * scale) : cvt_pk_bf16(a, b); };
+      auto choose = [&](float most, int group) {               // G > 1: the power of two of a group of columns
+        const int exponent = group_exponent(most), l = fresh_lane();
+        if (l < 16) exp_s[(16 * kt + l) * EXP_BYTES + group] = (unsigned char)exponent;
+        scale = group_scale(exponent);
+      };
+      if (G > 1) choose(group_max(acc), wave);
 #pragma unroll
       for (int pr = 0; pr < 2; pr++) {
         unsigned w0[2], w1[2];
 #pragma unroll
         for (int e = 0; e < 2; e++) {
-          w0[e] = cvt_pk_bf16(acc[2 * pr][2 * e], acc[2 * pr][2 * e + 1]);
-          w1[e] = cvt_pk_bf16(acc[2 * pr + 1][2 * e], acc[2 * pr + 1][2 * e + 1]);
+          w0[e] = pack(acc[2 * pr][2 * e], acc[2 * pr][2 * e + 1]);
+          w1[e] = pack(acc[2 * pr + 1][2 * e], acc[2 * pr + 1][2 * e + 1]);
           swap_halves(w0[e], w1[e]);
         }
         *(uint4*)(row + pr * 64 + coloff) = make_uint4(w0[0], w0[1], w1[0], w1[1]);
       }
       if (kt == hh) {
         mfma16_done(rot);
-        *(uint2*)(row + rotoff) = make_uint2(cvt_pk_bf16(rot[0], rot[1]), cvt_pk_bf16(rot[2], rot[3]));
+        if constexpr (G > 1) {
+          const f32x4 r1[1] = {rot};
+          choose(group_max(r1), 8 + (wave & 3));
+        }
+        *(uint2*)(row + rotoff) = make_uint2(pack(rot[0], rot[1]), pack(rot[2], rot[3]));
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+
+  // exponents of the rows of tile n: 512 bytes by one wave, ahead of the next transfers (that tile's destination rows are in LDS until then)
+  auto put_exponents = [&](int n) {
+    const int l = fresh_lane();
+    if (wave == 7 && l < BI) {
+      const int drow = dst_s[(n & 1) * 256 + l];
+      *(uint4*)(exps + (size_t)(drow >= 0 ? drow : dummy_row) * EXP_BYTES) = *(const uint4*)(exp_s + l * EXP_BYTES);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
 
 #pragma clang loop unroll(disable)
@@ -911,11 +972,16 @@ __device__ __forceinline__ void pds_rows_wide_body(
     // behind the tile's transfers: the five row stores of the tile before
     if (n > 0) { DSA_WAIT_VMCNT(5); } else { DSA_WAIT_VMCNT(0); }
     __syncthreads();
+    if (G > 1 && n > 0) put_exponents(n - 1);
     phase_pds(n);
     __syncthreads();
     if (n + 1 < ntiles) issue(n + 1);
     __builtin_amdgcn_sched_barrier(0);
     phase_rows(n);
+  }
+  if (G > 1) {
+    __syncthreads();
+    put_exponents(ntiles - 1);
   }
 }
 
@@ -946,7 +1012,9 @@ constexpr int RED_KEYS = 4;                  // consecutive keys per workgroup
 // combined.  (One key per workgroup left the per-key latencies - segment bounds, first loads, barrier, combine -
 // exposed once a key has few rows per launch: with the queries of 32768 tokens walked in four chunks the launch
 // took 27.1 ms against 18.9 ms for one sweep; per key the sums and their order are the same as before.)
-__device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ rows, const int* __restrict__ start,
+// SCALED: rows may be those of joint units; a chunk's exponent is loaded beside it.
+template <bool SCALED>
+__device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
                                             float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int key0, int n_keys,
                                             int accumulate, const int* __restrict__ dup_flag, unsigned char* smem) {
   float* part = (float*)smem;                  // [RED_KEYS][RED_GROUPS][DQK]
@@ -973,31 +1041,61 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
     // Always RED_FLIGHT loads, whatever is left (behind the rows the last one again, which `add` leaves out): only so can the
     // waits for one batch leave the next one's loads in flight.
     const unsigned lane_off = (unsigned)(grp * ROW_BYTES + ch * 16);
-    auto load = [&](uint4 (&v)[RED_FLIGHT], const Place& p) {
+    const unsigned lane_exp = (unsigned)(grp * EXP_BYTES + (ch < DV / 8 ? ch >> 3 : 8 + ((ch - DV / 8) >> 1)));
+    struct Batch { uint4 v[RED_FLIGHT]; unsigned e[RED_FLIGHT]; };
+    auto load = [&](Batch& t, const Place& p) {
       const int b = p.k < nk ? p.b : bounds_end - 1, n = (p.k < nk ? p.s1 : bounds_end) - b;
       const unsigned last = (unsigned)((n - 1) * ROW_BYTES + ch * 16);
       const unsigned char* base = rows + (size_t)b * ROW_BYTES;
 #pragma unroll
-      for (int u = 0; u < RED_FLIGHT; u++) v[u] = row_load16(base + min((unsigned)(u * RED_GROUPS * ROW_BYTES) + lane_off, last));
-    };
-    float acc[8] = {};
-    auto add1 = [&](const uint4& x) {
-      const unsigned w[4] = {x.x, x.y, x.z, x.w};
+      for (int u = 0; u < RED_FLIGHT; u++) t.v[u] = row_load16(base + min((unsigned)(u * RED_GROUPS * ROW_BYTES) + lane_off, last));
+      if constexpr (SCALED) {
+        const unsigned end = (unsigned)((n - 1) * EXP_BYTES) + lane_exp % EXP_BYTES;
+        const unsigned char* base_e = exps + (size_t)b * EXP_BYTES;
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        acc[2 * e] += __builtin_bit_cast(float, w[e] << 16);
-        acc[2 * e + 1] += __builtin_bit_cast(float, w[e] & 0xffff0000u);
+        for (int u = 0; u < RED_FLIGHT; u++) t.e[u] = base_e[min((unsigned)(u * RED_GROUPS * EXP_BYTES) + lane_exp, end)];
       }
     };
-    auto add = [&](const uint4 (&v)[RED_FLIGHT], const Place& p) {
+    float acc[8] = {};
+    // FORM 0: bf16 rows; 1: fp16 with a power of two; 2: either
+    auto add1 = [&](const uint4& x, unsigned exponent, auto form) {
+      constexpr int FORM = decltype(form)::value;
+      const unsigned w[4] = {x.x, x.y, x.z, x.w};
+      const bool half = FORM == 1 || (FORM == 2 && exponent != 0u);
+      const float scale = half ? __builtin_bit_cast(float, exponent << 23) : 1.f;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float b0 = __builtin_bit_cast(float, w[e] << 16), b1 = __builtin_bit_cast(float, w[e] & 0xffff0000u);
+        if constexpr (FORM == 0) {
+          acc[2 * e] += b0;
+          acc[2 * e + 1] += b1;
+        } else {
+          const f16x2_t h = __builtin_bit_cast(f16x2_t, w[e]);
+          acc[2 * e] = fmaf(half ? (float)h[0] : b0, scale, acc[2 * e]);
+          acc[2 * e + 1] = fmaf(half ? (float)h[1] : b1, scale, acc[2 * e + 1]);
+        }
+      }
+    };
+    auto add_as = [&](const Batch& t, const Place& p, auto form) {
       const int n = p.s1 - p.b;
       if (n >= RED_BATCH) {
 #pragma unroll
-        for (int u = 0; u < RED_FLIGHT; u++) add1(v[u]);
+        for (int u = 0; u < RED_FLIGHT; u++) add1(t.v[u], t.e[u], form);
       } else {
 #pragma unroll
         for (int u = 0; u < RED_FLIGHT; u++)
-          if (u * RED_GROUPS + grp < n) add1(v[u]);
+          if (u * RED_GROUPS + grp < n) add1(t.v[u], t.e[u], form);
+      }
+    };
+    auto add = [&](const Batch& t, const Place& p) {
+      if constexpr (SCALED) {
+        unsigned least = t.e[0];
+#pragma unroll
+        for (int u = 1; u < RED_FLIGHT; u++) least = min(least, t.e[u]);
+        if (__any(least == 0u)) add_as(t, p, std::integral_constant<int, 2>{});
+        else add_as(t, p, std::integral_constant<int, 1>{});
+      } else {
+        add_as(t, p, std::integral_constant<int, 0>{});
       }
     };
     auto put = [&](int k, int k_end) {                         // the sums of key k, and of keys without rows behind it
@@ -1009,7 +1107,7 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
         }
       }
     };
-    uint4 va[RED_FLIGHT], vb[RED_FLIGHT];
+    Batch va, vb;
     Place p = settle({0, __builtin_amdgcn_readlane(bounds, 0), __builtin_amdgcn_readlane(bounds, 1)});
     put(0, p.k);
     if (p.k < nk) load(va, p);
@@ -1083,8 +1181,8 @@ template <int HG, int G>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, const int* __restrict__ units,
-    size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, unsigned char* __restrict__ exps,
+    const int* __restrict__ units, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int ql = query_of<G, PDS_RAMP>((int)blockIdx.x, cnt, K);
   // (two copies of every body: each copy meets the same barriers)
@@ -1096,15 +1194,15 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
       unsigned char* unit = pds + (size_t)(ql / G) * group_pds;
       const __bf16 *q_rows = q + hrow * DQK, *out_rows = out + hrow * DV, *do_rows = dout + hrow * DV;
       const int *list = ids + (size_t)ql * K, *drow = dst + (size_t)ql * K;
-      if (threadIdx.x < 256) pds_rows_wide_body<0, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
-      else pds_rows_wide_body<1, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
+      if (threadIdx.x < 256) pds_rows_wide_body<0, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, exps, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
+      else pds_rows_wide_body<1, G>(q_rows, kv, list, out_rows, do_rows, lse + hrow, unit, drow, rows, exps, G > 1 ? 128 : H, Skv, slots, q_start + q0 + ql, sm_scale, dummy_row, smem);
       return;
     }
   }
   if constexpr (HG <= 2) {
     unsigned char* own = pds + (size_t)(ql / G) * group_pds + (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
-    if (threadIdx.x < 256) pds_rows_body<0, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-    else pds_rows_body<1, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    if (threadIdx.x < 256) pds_rows_body<0, HG, (G > 1)>(q, kv, ids, out, dout, lse, own, dst, rows, exps, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_body<1, HG, (G > 1)>(q, kv, ids, out, dout, lse, own, dst, rows, exps, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
   }
 }
 
@@ -1112,8 +1210,8 @@ template <int HG, int G>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
     __bf16* __restrict__ dq, const int* __restrict__ units, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
-    const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const int* __restrict__ start, float* __restrict__ dkv_acc,
-    unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
+    const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
+    float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
   if (rs.first) {
@@ -1135,7 +1233,7 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     // from the last key (compressed keys behind a sliding window)
     const int groups = (n_keys + RED_KEYS - 1) / RED_KEYS;
     const bool forward = 2 * (long long)start[n_keys / 2] >= start[n_keys];
-    reduce_body(rows, start, dkv_acc, dkv, (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS, n_keys, accumulate, dup_flag, smem);
+    reduce_body<(G > 1)>(rows, exps, start, dkv_acc, dkv, (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS, n_keys, accumulate, dup_flag, smem);
   }
 }
 
@@ -1165,7 +1263,7 @@ struct BwdPlan {
   int chunk;            // queries per pass over the buffers
   int G;                // queries of a group that may be a unit, or 1
   int W;                // bitmap words per key
-  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_bad, off_dst, off_sorted, off_pds, off_rows, off_acc, total;
+  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_bad, off_dst, off_sorted, off_pds, off_rows, off_exps, off_acc, total;
 };
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1187,6 +1285,7 @@ BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_pds = o; o = align_up(o + (size_t)((chunk + G - 1) / G) * group_pds_bytes(HG, G, K));
   p.off_rows = o; o = align_up(o + ((size_t)chunk * K + 1) * ROW_BYTES);
+  p.off_exps = o; o = align_up(o + (G > 1 ? ((size_t)chunk * K + 1) * EXP_BYTES : 0));
   p.off_acc = o; o = align_up(o + (size_t)Skv * DQK * 4);
   p.total = o;
   return p;
@@ -1257,6 +1356,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   int* sorted = (int*)(ws + p.off_sorted);
   unsigned char* pds = ws + p.off_pds;
   unsigned char* rows = ws + p.off_rows;
+  unsigned char* exps = ws + p.off_exps;       // (units)
   float* acc = (float*)(ws + p.off_acc);
 
   const int HG = head_groups(H);
@@ -1309,13 +1409,13 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
     pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smem_rows, st>>>(
-        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, units, group_pds, q0, cnt, H, Skv, K,
+        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, exps, units, group_pds, q0, cnt, H, Skv, K,
         q_start, sm_scale, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
     dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, units, group_pds, q0, cnt, H, Skv,
-                                                                   K, q_start, dup_flag, rows, start, acc,
+                                                                   K, q_start, dup_flag, rows, exps, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");
     DSA_MARK(3);

@@ -475,6 +475,34 @@ def test_backward_of_joint_queries(gpu, H, S, K, skv, turn, far):
     assert torch.isnan(dq3.float()).all() and torch.isnan(dkv3.float()).all()
 
 
+@pytest.mark.parametrize("H,S,K,skv", [(64, 512, 128, 300), (32, 800, 128, 300), (32, 768, 64, 200)])
+@pytest.mark.parametrize("alike,steep", [(0.0, 1.0), (0.9, 1.0), (0.99, 1.0), (0.9, 2.0)])
+def test_backward_of_joint_queries_is_no_less_accurate_than_one_by_one(gpu, H, S, K, skv, alike, steep):
+    """Neighbouring queries with most of their keys, and of their values (``alike``: correlation of Q and dO), in common: dKV is no
+    further from bf16 P and dS with unrounded rows than the sums of one bf16 row per query are, the result's own rounding on
+    both sides."""
+    from loongforge_amd import ops
+
+    inp = O.make_mla_inputs(S, H, K, seed=S + H, skv=skv, q_start=skv)
+    g = torch.Generator().manual_seed(S)
+    mix = lambda t: (alike ** 0.5 * torch.randn((S + 7) // 8, 1, *t.shape[1:], generator=g).expand(-1, 8, -1, -1).flatten(0, 1)[:S]    # noqa: E731
+                     + (1 - alike) ** 0.5 * torch.randn(t.shape, generator=g)).to(torch.bfloat16)
+    inp.q, inp.dout = mix(inp.q), mix(inp.dout)
+    pool = torch.stack([torch.randperm(skv, generator=g)[:K + K // 8] for _ in range((S + 7) // 8)])
+    inp.idx = torch.stack([pool[i // 8][torch.randperm(K + K // 8, generator=g)[:K]] for i in range(S)]).int()
+    assert _joint_groups(inp.idx, H)[0] > S * H // 128 // 2
+    q, kv, idx, do, sm = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu), steep * inp.sm_scale
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, skv, sm)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, skv, sm)
+    kw = dict(out=out.cpu(), lse=lse.cpu(), dtype=torch.float64)
+    dq_b, ref = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, inp.idx, inp.dout, skv, sm, 512, **kw)
+    _, rows = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, inp.idx, inp.dout, skv, sm, 512, round_rows_bf16=True, **kw)
+    assert_close(dq, dq_b, "dQ")
+    off, one_by_one = dkv.cpu().double() - ref, rows.to(torch.bfloat16).double() - ref
+    assert off.norm() <= one_by_one.norm()
+    assert off.abs().max() <= 1.1 * one_by_one.abs().max()                 # (the largest of many roundings, of other values)
+
+
 @pytest.mark.parametrize("H,S,K,skv,causal", [
     (64, 700, 2048, 4076, False),     # unions beyond the longest list of a unit, and within it
     (64, 1030, 512, 1200, True),
