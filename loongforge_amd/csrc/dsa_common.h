@@ -51,10 +51,6 @@ __device__ __forceinline__ unsigned cvt_pk_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
 }
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ unsigned cvt_pk_f16(float lo, float hi) {
-  const f32x2_t v = {lo, hi};
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, f16x2_t));
-}
 // The value of lane ^ m (m = 1, 2, 4 or 8, a constant after unrolling) by moves inside rows of 16 lanes, which must all be
 // active: vector instructions that the consumer mostly absorbs, where a shuffle is a trip through LDS.
 __device__ __forceinline__ float xor16(float x, int m) {

@@ -47,11 +47,12 @@ constexpr int PDS_THREADS = 512;
 //
 // A unit's row stands for 2 or 4 rows, so it is held in more bits than they: 11 instead of 8 significant ones, fp16 with a power of
 // two for every 64 columns (16 of the rotary part), chosen so that the largest of them lies in [2^14, 2^15).  Values down to 2^-29 of that
-// one have all 11 bits.  The power's fp32 exponent is one of EXP_BYTES bytes per row: groups 0 - 7 the 64-column groups, 8 - 11 the
+// one have all 11 bits.  Its fp32 exponent is one of EXP_BYTES bytes per row: groups 0 - 7 the 64-column groups, 8 - 11 the
 // rotary ones; 0 marks a bf16 row, one of a query by itself.  In bf16 the rows' rounding error would be that of the rows it stands for only
 // where those are independent, and grows with what neighbouring queries have in common: rms over 256 queries x 256 of 288 slots, rows per query 1,
 // unit in bf16 / fp16: correlation 0 of Q and dO 1.00 / 0.13, 0.9 1.27 / 0.16 (64 heads) and 1.68 / 0.21 (32 heads), 0.99 1.36 / 0.17 and 1.88 /
-// 0.24.
+// 0.24.  What it takes, bf16 / fp16: scores and rows 530 / 575 us at 3072 queries x 640 slots x 64 heads and 276 / 299 at 2077 x 512 (maxima 16
+// of the 45, the rest products with the power and the exponents' way through LDS), dQ and the sums 308 / 317 and 179 / 185.
 constexpr int unit_queries(int HG) { return 4 / HG; }
 constexpr int UNIT_SLOTS = 3072;             // what the lists in LDS behind the operands of 128 heads have room for
 constexpr int UNIT_KEY = 0xffffff;
@@ -568,30 +569,37 @@ inline size_t wide_lds_bytes(int K) { return (size_t)WIDE_LISTS + ids_lds_bytes(
 __host__ __device__ constexpr size_t unit_lds_bytes(int slots) { return (size_t)WIDE_LISTS + (size_t)slots * 4 + 1024 + 2048 + BI * EXP_BYTES; }
 static_assert(unit_lds_bytes(UNIT_SLOTS) <= 160 * 1024, "the list of a joint unit");
 
-// Exponent of the power of two that a group of columns of a unit's row is divided by.  group_max: the largest magnitude over the 16 values of
-// every lane with the same lane % 16; values that are not finite do not count, they stay what they are in fp16.
+// Largest magnitude over the values of every lane with the same lane % 16, as bits, and at least 2^-112 (below that the scale stays as it
+// is).  Values that are not finite do not count: they are what they are in fp16.
 template <int N>
-__device__ __forceinline__ float group_max(const f32x4 (&x)[N]) {
-  float most = 0.f;
+__device__ __forceinline__ unsigned group_max(const f32x4 (&x)[N]) {
+  constexpr float LEAST = 0x1p-112f;
+  float most = LEAST;
 #pragma unroll
   for (int i = 0; i < N; i++)
 #pragma unroll
-    for (int e = 0; e < 4; e += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(x[i][e]), "v"(x[i][e + 1]));      // (NaN does not count)
+    for (int e = 0; e < 4; e += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(x[i][e]), "v"(x[i][e + 1]));      // (passes over NaN)
   if (__any(most == INFINITY)) {
-    most = 0.f;
+    most = LEAST;
 #pragma unroll
     for (int i = 0; i < N; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) most = fabsf(x[i][e]) < INFINITY ? fmaxf(most, fabsf(x[i][e])) : most;
   }
   float other = most;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(most), "+v"(other));
-  most = other = fmaxf(most, other);
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(most), "+v"(other));
-  return fmaxf(most, other);
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1\n\tv_max_f32 %0, %0, %1\n\tv_mov_b32 %1, %0\n\ts_nop 1\n\t"
+               "v_permlane16_swap_b32 %0, %1\n\ts_nop 1\n\tv_max_f32 %0, %0, %1" : "+v"(most), "+v"(other));
+  return __builtin_bit_cast(unsigned, most);
 }
-__device__ __forceinline__ int group_exponent(float most) { return max((int)(__builtin_bit_cast(unsigned, most) >> 23) - 14, 1); }
-__device__ __forceinline__ float group_scale(int exponent) { return __builtin_bit_cast(float, (unsigned)(254 - exponent) << 23); }
+// 2^(14 - k) for a largest magnitude of 2^k .. 2^(k + 1), whose exponent bits are kept with the row
+__device__ __forceinline__ float group_scale(unsigned most) { return __builtin_bit_cast(float, (268u << 23) - (most & 0x7f800000u)); }
+// (a scale, b scale) in fp16, product and rounding in one instruction each
+__device__ __forceinline__ unsigned scaled_pk_f16(float a, float b, float scale) {
+  unsigned r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(scale));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(b), "v"(scale));
+  return r;
+}
 
 // Zero where a bf16 value is not finite (exponent all ones), in 16 bytes of LDS
 __device__ __forceinline__ void drop_nonfinite(unsigned char* p) {
@@ -870,7 +878,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
       // (G > 1: the query of the wave's heads is wave * G / 8)
-      const bool valid = G > 1 ? (idx_s[n * BI + 16 * kt + lm] >> (24 + wave * G / 8)) & 1 : (mask >> (16 * kt + lm)) & 1u;
+      const bool valid = G > 1 ? (idx_s[n * BI + 16 * kt + (fresh_lane() & 15)] >> (24 + wave * G / 8)) & 1 : (mask >> (16 * kt + lm)) & 1u;
       float pf[4], df[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -893,10 +901,11 @@ __device__ __forceinline__ void pds_rows_wide_body(
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
+  auto put_exponent = [&](unsigned most, int row, int group) { exp_s[(row + (fresh_lane() & 15)) * EXP_BYTES + group] = (unsigned char)(most >> 23); };
   auto phase_rows = [&](int n) {
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      const int drow = dst_s[(n & 1) * 256 + 16 * kt + lm];
+      const int drow = dst_s[(n & 1) * 256 + 16 * kt + (G > 1 ? fresh_lane() & 15 : lm)];
       f32x4 acc[4], rot;
       bf16x8 cf[2], x[2];                      // coefficients of step k = 0 .. 3: dS . Q, 4 .. 7: P . dO; column operands from LDS
       auto coef = [&](int k) { return *(const bf16x8*)(xch + k * 2048 + kt * 256 + coff); };
@@ -926,13 +935,12 @@ __device__ __forceinline__ void pds_rows_wide_body(
       asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
       unsigned char* row = rows + (size_t)(drow >= 0 ? drow : dummy_row) * ROW_BYTES;       // invalid slots: a scratch row
       float scale = 1.f;
-      auto pack = [&](float a, float b) { return G > 1 ? cvt_pk_f16(a * scale, b * scale) : cvt_pk_bf16(a, b); };
-      auto choose = [&](float most, int group) {               // G > 1: the power of two of a group of columns
-        const int exponent = group_exponent(most), l = fresh_lane();
-        if (l < 16) exp_s[(16 * kt + l) * EXP_BYTES + group] = (unsigned char)exponent;
-        scale = group_scale(exponent);
-      };
-      if (G > 1) choose(group_max(acc), wave);
+      auto pack = [&](float a, float b) { return G > 1 ? scaled_pk_f16(a, b, scale) : cvt_pk_bf16(a, b); };
+      if constexpr (G > 1) {
+        const unsigned most = group_max(acc);
+        scale = group_scale(most);
+        put_exponent(most, 16 * kt, wave);
+      }
 #pragma unroll
       for (int pr = 0; pr < 2; pr++) {
         unsigned w0[2], w1[2];
@@ -948,7 +956,9 @@ __device__ __forceinline__ void pds_rows_wide_body(
         mfma16_done(rot);
         if constexpr (G > 1) {
           const f32x4 r1[1] = {rot};
-          choose(group_max(r1), 8 + (wave & 3));
+          const unsigned most = group_max(r1);
+          scale = group_scale(most);
+          put_exponent(most, 16 * kt, 8 + (wave & 3));
         }
         *(uint2*)(row + rotoff) = make_uint2(pack(rot[0], rot[1]), pack(rot[2], rot[3]));
       }
@@ -1062,7 +1072,7 @@ __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ ro
       constexpr int FORM = decltype(form)::value;
       const unsigned w[4] = {x.x, x.y, x.z, x.w};
       const bool half = FORM == 1 || (FORM == 2 && exponent != 0u);
-      const float scale = half ? __builtin_bit_cast(float, exponent << 23) : 1.f;
+      const float scale = half ? __builtin_bit_cast(float, (exponent - 14u) << 23) : 1.f;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float b0 = __builtin_bit_cast(float, w[e] << 16), b1 = __builtin_bit_cast(float, w[e] & 0xffff0000u);

@@ -595,6 +595,30 @@ def test_backward_of_joint_queries_keeps_nonfinite_values_apart(gpu, H, S, where
         assert (~torch.isfinite(dkv[touched])).any(1).all() and torch.equal(dkv[~touched], dkv0.float().cpu()[~touched])
 
 
+@pytest.mark.parametrize("H,S", [(64, 520), (32, 800)])
+def test_backward_of_joint_queries_with_a_column_that_overflows(gpu, H, S):
+    """A sum over the heads beyond the range of fp32 in one column of a pair row leaves the row's other columns as they are."""
+    from loongforge_amd import ops
+
+    K, skv, bad, col = 128, 700, 101, 77
+    inp = O.make_mla_inputs(S, H, K, seed=S, skv=skv, q_start=skv)
+    idx = _overlapping_ids(S, K, skv + S, 0, 0, 5)
+    assert _joint_groups(idx, H)[0] > S * H // 128 // 2
+    key = int(idx[bad, 3])
+    q, kv, do, ids, sm = inp.q.to(gpu), inp.kv.to(gpu), inp.dout.to(gpu), idx.to(gpu), inp.sm_scale
+    kv[:, col] = 0                             # (else dP and delta overflow as well)
+    kv[key] *= 4
+    q[bad] = kv[key]                           # every head's probability is on this key
+    do[bad, :, col] = 0
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, skv, sm)
+    dq0, dkv0 = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, skv, sm)
+    do[bad, :, col] = 3e38
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, skv, sm)
+    assert torch.isposinf(dkv[key, col])
+    rest = torch.arange(576, device=gpu) != col
+    assert torch.isfinite(dkv0.float()).all() and torch.equal(dq, dq0) and torch.equal(dkv[:, rest], dkv0[:, rest])
+
+
 @pytest.mark.parametrize("H", [32, 128])
 def test_backward_of_keys_with_few_and_many_rows(gpu, H):
     """Keys with numbers of rows around one row per thread group (7) and one batch of loads (56), and with none, in any
