@@ -299,7 +299,9 @@ int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges
  * natural-log lse.  P and dS enter the matrix products as bf16 (as in the reference's kernel); the
  * contribution of one (query, key) pair to dKV - a row of 576 values, summed over all heads in
  * fp32 - is rounded to bf16 once, and the rows of a key are then summed in fp32 in a fixed order
- * (bit-reproducible, no float atomics); dKV is returned as bf16.  The ids of one query must be
+ * (bit-reproducible, no float atomics); dKV is returned as bf16.  With 32 or 64 heads 4 or 2 consecutive queries
+ * that share enough of their keys are worked as one: one row then stands for the key's pairs with all of them, summed in fp32 and
+ * rounded once, to 11 significant bits (fp16 with a power of two per 64 columns).  The ids of one query must be
  * distinct (any top-k is): a row with a repeated valid id makes the call return dq and dkv filled
  * with NaN rather than sums that miss a term.  Replaces flash_mla_bwd.flash_mla_sparse_bwd /
  * sparse_mla_bwd_interface as called at dsa_fused_kernels.py:2086-2110
@@ -309,7 +311,9 @@ int dsa_sparse_mla_fwd_form(int S, int H, int K, int with_workspace, int* ranges
  * sweep (22 GiB at S = Skv = 8192, K = 2048; 89 GiB at 32768 tokens).  Any size from
  * dsa_sparse_mla_bwd_workspace_bytes_min on is accepted: with less than the full size the queries are walked in
  * chunks (the largest of S, S/2, S/4, ... that fits, at least 64), a few per cent slower per extra chunk; the
- * chunking follows from the sizes alone, and dKV is bit-reproducible for a given workspace size.
+ * chunking follows from the sizes alone, and dKV is bit-reproducible for a given workspace size.  dQ does not depend on
+ * the workspace; with 32 or 64 heads its last bits, as those of dKV, depend on the number of queries in the call and on the
+ * queries beside a query, which decide what is worked as one.
  */
 size_t dsa_sparse_mla_bwd_workspace_bytes(int S, int H, int Skv, int K);
 size_t dsa_sparse_mla_bwd_workspace_bytes_min(int S, int H, int Skv, int K);

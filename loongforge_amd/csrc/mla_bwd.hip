@@ -1270,16 +1270,25 @@ __global__ void poison_bf16_kernel(unsigned short* __restrict__ p, size_t n, con
 bool use_units(int HG, int S, int Skv) { return HG < 4 && S >= 192 * unit_queries(HG) && order::unit_lists_fit(unit_queries(HG), Skv); }
 
 struct BwdPlan {
-  int chunk;            // queries per pass over the buffers
-  int G;                // queries of a group that may be a unit, or 1
+  int chunk;            // queries per pass over the buffers, a multiple of G
+  int G;                // queries of a group that may be a unit, or 1: from the whole call, so that a query's dQ does not depend on the chunks
   int W;                // bitmap words per key
   size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_bad, off_dst, off_sorted, off_pds, off_rows, off_exps, off_acc, total;
 };
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
+int group_queries(int S, int H, int Skv) {
+  const int HG = head_groups(H);
+  return use_units(HG, S, Skv) ? unit_queries(HG) : 1;
+}
+
+// For S queries in groups of G, `chunk` of them at a time
+BwdPlan layout_plan(int S, int G, int chunk, int H, int Skv, int K) {
   BwdPlan p;
+  const int HG = head_groups(H);
+  p.G = G;
+  chunk = (chunk + G - 1) / G * G;
   p.chunk = chunk;
   p.W = (chunk + 31) / 32;
   size_t o = 0;
@@ -1288,12 +1297,11 @@ BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
   p.off_count = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_start = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_flag = o; o = align_up(o + 4);
-  const int HG = head_groups(H), G = p.G = use_units(HG, chunk, Skv) ? unit_queries(HG) : 1;
-  p.off_units = o; o = align_up(o + (size_t)(chunk + G - 1) / G * 4);
+  p.off_units = o; o = align_up(o + (G > 1 ? (size_t)((S + G - 1) / G) * 4 : 0));
   p.off_bad = o; o = align_up(o + (size_t)((Skv + 31) / 32) * 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
-  p.off_pds = o; o = align_up(o + (size_t)((chunk + G - 1) / G) * group_pds_bytes(HG, G, K));
+  p.off_pds = o; o = align_up(o + (size_t)(chunk / G) * group_pds_bytes(HG, G, K));
   p.off_rows = o; o = align_up(o + ((size_t)chunk * K + 1) * ROW_BYTES);
   p.off_exps = o; o = align_up(o + (G > 1 ? ((size_t)chunk * K + 1) * EXP_BYTES : 0));
   p.off_acc = o; o = align_up(o + (size_t)Skv * DQK * 4);
@@ -1302,15 +1310,18 @@ BwdPlan layout_plan(int chunk, int H, int Skv, int K) {
 }
 
 // Largest chunk of queries (all of them if possible, else repeated halving, at least 64) whose
-// buffers fit the budget.
+// buffers fit the budget; without units if those of the smallest chunk do not.
 BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
-  int chunk = S;
-  BwdPlan p = layout_plan(chunk, H, Skv, K);
-  while (p.total > budget && chunk > 64) {
-    chunk = (chunk + 1) / 2;
-    p = layout_plan(chunk, H, Skv, K);
+  BwdPlan p;
+  for (int G = group_queries(S, H, Skv);; G = 1) {
+    int chunk = S;
+    p = layout_plan(S, G, chunk, H, Skv, K);
+    while (p.total > budget && chunk > 64) {
+      chunk = (chunk + 1) / 2;
+      p = layout_plan(S, G, chunk, H, Skv, K);
+    }
+    if (p.total <= budget || G == 1) return p;
   }
-  return p;
 }
 
 // What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, fitted to
@@ -1335,7 +1346,7 @@ extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes(int S, int H, int Skv, int 
 
 extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes_min(int S, int H, int Skv, int K) {
   if (S <= 0 || Skv <= 0 || K <= 0) return 0;
-  return layout_plan(S < 64 ? S : 64, H, Skv, K).total;
+  return layout_plan(S, group_queries(S, H, Skv), S < 64 ? S : 64, H, Skv, K).total;
 }
 
 static int bwd_impl(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
@@ -1355,7 +1366,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   BwdPlan p = make_plan(S > 0 ? S : 1, H, Skv, K, workspace_bytes);
   if (p.total > workspace_bytes || workspace == nullptr)
     DSA_FAIL(DSA_ERR_WORKSPACE, "dsa_sparse_mla_bwd: workspace of %zu bytes is too small (need at least %zu)",
-             workspace_bytes, make_plan(64, H, Skv, K, 1).total);
+             workspace_bytes, layout_plan(S, 1, S < 64 ? S : 64, H, Skv, K).total);
   unsigned char* ws = (unsigned char*)workspace;
   unsigned* bitmap = (unsigned*)(ws + p.off_bitmap);
   unsigned* prefix = (unsigned*)(ws + p.off_prefix);
@@ -1413,18 +1424,18 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
     const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     DSA_MARK(0);
-    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units, unit_slots(HG, K), unit_cost(HG, p.chunk));
+    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S));
     else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
     pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smem_rows, st>>>(
-        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, exps, units, group_pds, q0, cnt, H, Skv, K,
+        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, exps, units + q0 / G, group_pds, q0, cnt, H, Skv, K,
         q_start, sm_scale, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, units, group_pds, q0, cnt, H, Skv,
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, units + q0 / G, group_pds, q0, cnt, H, Skv,
                                                                    K, q_start, dup_flag, rows, exps, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");

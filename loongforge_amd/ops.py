@@ -489,7 +489,7 @@ ATTN_DIST_QK_MAX_SLOTS = 4096
 def _bwd_workspace(full_bytes: int, device):
     """Workspace of the sparse-MLA backward: ``full_bytes`` lets it take all queries in one sweep (22 GiB at 8k
     tokens, top-k 2048; 89 GiB at 32k); given less, the library walks the queries in chunks.  The size handed to
-    the library - and with it the chunking, on which the last bits of dKV depend - follows from the shapes and
+    the library - and with it the chunking, on which the last bits of dKV depend (those of dQ do not) - follows from the shapes and
     from ``DSA_BWD_WORKSPACE_GIB`` (default 48) alone, never from what happens to be free or from earlier calls.
     The buffer is kept per device and reused by later calls on the same stream (held until :func:`release_bwd_workspace`;
     ``DSA_BWD_WORKSPACE_CACHE=0`` keeps none).  A call on another stream, which may overlap, lets go of it - the allocator

@@ -551,6 +551,37 @@ def test_backward_of_joint_queries_is_that_of_wider_queries(gpu, H, S, K, skv, c
     assert (a - b).norm() <= 5e-3 * b.norm()
 
 
+@pytest.mark.parametrize("H,S", [(64, 700), (32, 1103)])
+def test_dq_of_joint_queries_does_not_depend_on_the_workspace(gpu, H, S):
+    """Which queries are worked as one follows from the whole call and not from the chunks that a smaller workspace allows: the same
+    bits of dQ in one sweep, in two, in chunks of 64 or less, and dKV to the order of its sums.  Less than the smallest documented
+    workspace is still taken if it holds 64 queries one by one."""
+    from loongforge_amd import _lib, ops
+
+    K, skv = 192, 1200
+    inp = O.make_mla_inputs(S, H, K, seed=S, skv=skv, q_start=skv)
+    inp.idx = _overlapping_ids(S, K, skv + S, 0, 3, S)
+    joint, groups = _joint_groups(inp.idx, H)
+    assert groups // 4 < joint < groups
+    q, kv, idx, do, sm = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu), inp.sm_scale
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, skv, sm)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, idx, lse, skv, sm)
+    lib = _lib.load()
+    least, one_by_one = lib.dsa_sparse_mla_bwd_workspace_bytes_min(S, H, skv, K), lib.dsa_sparse_mla_bwd_workspace_bytes(64, H, skv, K)
+    assert one_by_one <= least
+    for nbytes in (lib.dsa_sparse_mla_bwd_workspace_bytes((S + 3) // 2, H, skv, K) + 2 ** 20, least, one_by_one):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+        dq2, dkv2 = torch.empty_like(q), torch.empty_like(kv)
+        rc = lib.dsa_sparse_mla_bwd(q.data_ptr(), kv.data_ptr(), out.data_ptr(), do.data_ptr(), idx.data_ptr(), lse.data_ptr(), S, H, skv, K,
+                                    skv, sm, 512, dq2.data_ptr(), dkv2.data_ptr(), ws.data_ptr(), nbytes,
+                                    torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.dsa_last_error()
+        assert torch.equal(dq, dq2) or nbytes < least
+        a, b = dkv2.float(), dkv.float()
+        assert (a - b).norm() <= 3e-3 * b.norm()
+        assert_close(dq2, dq, "dQ")
+
+
 @pytest.mark.parametrize("H,S", [(64, 520), (32, 800)])
 @pytest.mark.parametrize("where,value", [("dout", float("nan")), ("dout", float("inf")), ("q", float("nan")), ("q_rope", float("inf")),
                                          ("kv", float("nan"))])
