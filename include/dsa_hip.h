@@ -321,6 +321,13 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const void* out, const voi
                        const int32_t* ids, const float* lse, int S, int H, int Skv, int K,
                        int q_start, float sm_scale, int d_v, void* dq, void* dkv,
                        void* workspace, size_t workspace_bytes, void* stream);
+/*
+ * How the backward goes about a call of these sizes and this workspace, for tests and measurements: how many consecutive queries
+ * make a group that may be worked as one query (1: none).  If more than one, *units_offset is where in its workspace the call leaves
+ * an int32 for every group, ceil(S / group) of them: the slots of the group worked as one, in whole tiles of 32, or 0 for queries one by
+ * one.  -1 for sizes that the backward does not take.
+ */
+int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t workspace_bytes, size_t* units_offset);
 
 /*
  * KL loss of the indexer's scores against the attention distribution, and its gradient, per query row:

@@ -1349,6 +1349,14 @@ extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes_min(int S, int H, int Skv, 
   return layout_plan(S, group_queries(S, H, Skv), S < 64 ? S : 64, H, Skv, K).total;
 }
 
+extern "C" int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t workspace_bytes, size_t* units_offset) {
+  if (S <= 0 || Skv <= 0 || Skv > order::MAX_KEYS || H <= 0 || H > 128 || H % 32 || K <= 0 || K % 64 || K > 2048) return -1;
+  const BwdPlan p = make_plan(S, H, Skv, K, workspace_bytes);
+  if (p.total > workspace_bytes) return -1;
+  if (units_offset) *units_offset = p.off_units;
+  return p.G;
+}
+
 static int bwd_impl(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
                     const float* lse, int S, int H, int Skv, int K, int q_start, float sm_scale, int d_v,
                     void* dq, void* dkv, void* workspace, size_t workspace_bytes, void* stream, float* pass_ms) {

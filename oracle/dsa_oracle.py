@@ -277,9 +277,20 @@ def sparse_mla_bwd(q, kv, idx, dout, q_start=0, sm_scale=None, d_v=512, dtype=to
     return qd.grad, kvd.grad
 
 
+def round_unit_rows(rows: torch.Tensor) -> torch.Tensor:
+    """``rows [n, 576]`` in fp16 with a power of two for every 64 columns (16 from column 512 on) that brings the largest magnitude among
+    them to [2**14, 2**15)."""
+    out = torch.empty_like(rows)
+    for lo, hi in [(64 * i, 64 * i + 64) for i in range(8)] + [(512 + 16 * i, 528 + 16 * i) for i in range(4)]:
+        x = rows[:, lo:hi]
+        scale = torch.exp2(14 - torch.floor(torch.log2(x.abs().amax(1, keepdim=True).clamp_min(2.0 ** -112))))
+        out[:, lo:hi] = (x * scale).to(torch.float16).to(rows.dtype) / scale
+    return out
+
+
 def sparse_mla_bwd_kernel_rounding(q, kv, idx, dout, q_start=0, sm_scale=None, d_v=512, out=None, lse=None,
                                    round_p_ds_bf16=True, round_rows_bf16=False, return_abs_sum=False, chunk=32,
-                                   attn_sink=None, dtype=torch.float32):
+                                   attn_sink=None, dtype=torch.float32, units=None):
     """dQ, dKV by the closed form of the reference's backward kernel, with that kernel's rounding
     points (ops/tilelang_ops/sparse_mla_bwd.py): every product accumulates in fp32 from bf16
     operands; ``P = exp(S*scale - lse)`` (:192-193) and ``dS = P*(dP - Delta)*scale`` (:197-199,
@@ -296,6 +307,9 @@ def sparse_mla_bwd_kernel_rounding(q, kv, idx, dout, q_start=0, sm_scale=None, d
     ``2**-9 * A`` bounds what that rounding can change (round-to-nearest bf16 moves a value by at
     most 2**-9 of its size), and ``2**-7 * M`` is one step of the bf16 grid at the largest row, i.e.
     what two evaluations differ by when that row lands on either side of a rounding boundary.
+    ``units = (G, joint)``: for every group of ``G`` consecutive queries whether it is worked as one query; the rows of such
+    a group are summed per key and rounded together, to fp16 with a power of two per 64 columns (:func:`round_unit_rows`), a
+    grid eight times finer than bf16, so they count an eighth in ``A`` and ``M``.
     Written with device-agnostic tensor ops, so a test may evaluate it on tensors that live on
     the GPU when the full benchmark sizes are too slow for the host (it stays a torch fp32
     evaluation of the same lines either way).  ``attn_sink`` only enters through ``lse`` (the sink
@@ -335,6 +349,21 @@ def sparse_mla_bwd_kernel_rounding(q, kv, idx, dout, q_start=0, sm_scale=None, d
         dq[s:e] = torch.einsum("mhk,mkd->mhd", ds_b, kvg)
         contrib = torch.einsum("mhk,mhd->mkd", ds_b, qf[s:e])
         contrib[..., :d_v] += torch.einsum("mhk,mhd->mkd", p_b, dof[s:e])
+        if units is not None:
+            for g in range(-(-s // units[0]), -(-e // units[0])):
+                a, b = g * units[0] - s, (g + 1) * units[0] - s
+                if not units[1][g]:
+                    continue
+                assert b <= e - s, "groups do not straddle chunks"
+                keys, place = torch.unique(safe[s:e][a:b][valid[s:e][a:b]], return_inverse=True)
+                rows = torch.zeros(len(keys), dqk, device=q.device, dtype=dtype).index_add_(0, place, contrib[a:b][valid[s:e][a:b]])
+                if round_rows_bf16:
+                    rows = round_unit_rows(rows)
+                dkv[keys] += rows
+                if return_abs_sum:
+                    abs_sum[keys] += rows.abs() / 8
+                    abs_max[keys] = torch.maximum(abs_max[keys], rows.abs() / 8)
+                contrib[a:b] = 0
         if round_rows_bf16:
             contrib = contrib.to(torch.bfloat16).to(dtype)
         dkv.index_add_(0, safe[s:e].reshape(-1), contrib.reshape(-1, dqk))   # invalid slots add zeros to row 0

@@ -18,6 +18,31 @@ def mla_form(S, H, K, with_workspace=True):
     return _lib.load().dsa_sparse_mla_fwd_form(S, H, K, int(with_workspace), ctypes.addressof(ranges)), ranges.value
 
 
+def mla_bwd_with_groups(q, kv, out, dout, idx, lse, q_start, sm_scale, nbytes=None):
+    """(dq, dkv, G, joint): the backward through the C ABI with ``nbytes`` of workspace (default: all that it can use), and for every
+    group of ``G`` consecutive queries whether the call worked it as one query, as the call left it in its workspace."""
+    import ctypes
+
+    from loongforge_amd import _lib
+
+    lib = _lib.load()
+    (S, H, _), skv, K = q.shape, kv.shape[0], idx.shape[1]
+    nbytes = nbytes or lib.dsa_sparse_mla_bwd_workspace_bytes(S, H, skv, K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+    rc = lib.dsa_sparse_mla_bwd(q.data_ptr(), kv.data_ptr(), out.data_ptr(), dout.data_ptr(), idx.data_ptr(), lse.data_ptr(), S, H, skv, K,
+                                q_start, sm_scale, 512, dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), nbytes,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.dsa_last_error()
+    at = ctypes.c_size_t(0)
+    G = lib.dsa_sparse_mla_bwd_groups(S, H, skv, K, nbytes, ctypes.addressof(at))
+    assert G >= 1
+    joint = [False] * S
+    if G > 1:
+        joint = (ws[at.value:at.value + (S + G - 1) // G * 4].view(torch.int32) > 0).tolist()
+    return dq, dkv, G, joint
+
+
 def assert_close(got, ref, name, atol=2e-2, rtol=1e-2):
     """|got - ref| <= atol + rtol * |ref| for every element (the tolerance the path is specified
     with: max-abs 2e-2, relative 1e-2 against an fp32 reference)."""

@@ -110,3 +110,26 @@ def test_bench_refuses_more_than_one_gpu():
                          timeout=120)
     assert res.returncode != 0
     assert "one GPU" in (res.stdout + res.stderr)
+
+
+def test_groups_of_the_sparse_mla_backward():
+    """Queries of 64 and 32 heads may be worked in groups of 2 and 4, from so many queries on, in every workspace from the smallest
+    documented one on; queries of more heads and sizes that the backward does not take are not."""
+    from loongforge_amd import _lib
+
+    lib = _lib.load()
+    at = ctypes.c_size_t(0)
+    for H, G in ((64, 2), (32, 4)):
+        for S in (192 * G, 1000, 1003):
+            full, least = lib.dsa_sparse_mla_bwd_workspace_bytes(S, H, 500, 128), lib.dsa_sparse_mla_bwd_workspace_bytes_min(S, H, 500, 128)
+            for nbytes in (full, (full + least) // 2, least):
+                assert lib.dsa_sparse_mla_bwd_groups(S, H, 500, 128, nbytes, ctypes.addressof(at)) == G
+                assert 0 < at.value and at.value % 256 == 0 and at.value + (S + G - 1) // G * 4 <= nbytes
+        one_by_one = lib.dsa_sparse_mla_bwd_workspace_bytes(64, H, 500, 128)          # (less than `least`, and taken all the same)
+        assert one_by_one < lib.dsa_sparse_mla_bwd_workspace_bytes_min(1024, H, 500, 128)
+        assert lib.dsa_sparse_mla_bwd_groups(1024, H, 500, 128, one_by_one, None) == 1
+        assert lib.dsa_sparse_mla_bwd_groups(192 * G - 1, H, 500, 128, full, None) == 1
+    assert lib.dsa_sparse_mla_bwd_groups(1000, 128, 500, 128, 2 ** 40, None) == 1
+    for S, H, Skv, K, nbytes in ((0, 64, 500, 128, 2 ** 40), (1000, 48, 500, 128, 2 ** 40), (1000, 64, 500, 100, 2 ** 40), (1000, 64, 0, 128, 2 ** 40),
+                                 (1000, 64, 500, 2112, 2 ** 40), (1000, 64, 500, 128, 1 << 20)):
+        assert lib.dsa_sparse_mla_bwd_groups(S, H, Skv, K, nbytes, None) == -1
