@@ -48,7 +48,9 @@ constexpr int PDS_THREADS = 512;
 // A unit's row stands for 2 or 4 rows, so it is held in more bits than they: 11 instead of 8 significant ones, fp16 with a power of
 // two for every 64 columns (16 of the rotary part), chosen so that the largest of them lies in [2^14, 2^15).  Values down to 2^-29 of that
 // one have all 11 bits.  Its fp32 exponent is one of EXP_BYTES bytes per row: groups 0 - 7 the 64-column groups, 8 - 11 the
-// rotary ones; 0 marks a bf16 row, one of a query by itself.  In bf16 the rows' rounding error would be that of the rows it stands for only
+// rotary ones; 0 marks a bf16 row, one of a query by itself: all of them are 0 before the rows are written, and where a call has no unit
+// they are neither cleared nor read (marked row by row instead: scores and rows of 3000 x 2048 of 32768 keys, no units, 2867 -> 3234 us).
+// In bf16 the rows' rounding error would be that of the rows it stands for only
 // where those are independent, and grows with what neighbouring queries have in common: rms over 256 queries x 256 of 288 slots, rows per query 1,
 // unit in bf16 / fp16: correlation 0 of Q and dO 1.00 / 0.13, 0.9 1.27 / 0.16 (64 heads) and 1.68 / 0.21 (32 heads), 0.99 1.36 / 0.17 and 1.88 /
 // 0.24.  What it takes, bf16 / fp16: scores and rows 530 / 575 us at 3072 queries x 640 slots x 64 heads and 276 / 299 at 2077 x 512 (maxima 16
@@ -281,11 +283,11 @@ static_assert(64 * (DQK + DV) * 2 <= FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH +
 __host__ __device__ inline size_t fused_lds_bytes(int K) {
   return (size_t)FUSED_STAGES * TILE_BYTES + 2 * FUSED_XCH + FUSED_ROT + ids_lds_bytes(K) + 512 + (size_t)K * 4;
 }
-template <int hh, int HG, bool MARK>         // HG: groups of 32 heads, 2 or 1; MARK: the rows have exponents
+template <int hh, int HG>                    // HG: groups of 32 heads, 2 or 1
 __device__ __forceinline__ void pds_rows_body(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
-    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, unsigned char* __restrict__ exps,
+    unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows,
     int q0, int ql, int Skv, int K, int q_start, float sm_scale, int dummy_row, unsigned char* smem) {
   constexpr int H = 32 * HG, KS = DQK / 32, VS = DV / 32, STAGES = FUSED_STAGES;
   constexpr int DO_ACC = 12;                   // steps of dO in accumulation registers, beside all of Q: 120
@@ -337,10 +339,7 @@ __device__ __forceinline__ void pds_rows_body(
   const int ntiles = stage_requested_ids(slot_id, K, Skv, q_start + qi, idx_s, tmask, tlist, ntile_s);
 #pragma unroll
   for (int i = 0; i < 4; i++)                  // invalid slots land in a scratch row: the store count stays fixed
-    if (tid + 512 * i < K) {
-      dst_s[tid + 512 * i] = slot_row[i] >= 0 ? slot_row[i] : dummy_row;
-      if (MARK && slot_row[i] >= 0) *(uint4*)(exps + (size_t)slot_row[i] * EXP_BYTES) = make_uint4(0u, 0u, 0u, 0u);
-    }
+    if (tid + 512 * i < K) dst_s[tid + 512 * i] = slot_row[i] >= 0 ? slot_row[i] : dummy_row;
   DSA_WAIT_VMCNT(0);
   if (ntiles == 0) return;
   __syncthreads();
@@ -1211,8 +1210,8 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
   }
   if constexpr (HG <= 2) {
     unsigned char* own = pds + (size_t)(ql / G) * group_pds + (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
-    if (threadIdx.x < 256) pds_rows_body<0, HG, (G > 1)>(q, kv, ids, out, dout, lse, own, dst, rows, exps, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
-    else pds_rows_body<1, HG, (G > 1)>(q, kv, ids, out, dout, lse, own, dst, rows, exps, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    if (threadIdx.x < 256) pds_rows_body<0, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
+    else pds_rows_body<1, HG>(q, kv, ids, out, dout, lse, own, dst, rows, q0, ql, Skv, K, q_start, sm_scale, dummy_row, smem);
   }
 }
 
@@ -1243,7 +1242,9 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     // from the last key (compressed keys behind a sliding window)
     const int groups = (n_keys + RED_KEYS - 1) / RED_KEYS;
     const bool forward = 2 * (long long)start[n_keys / 2] >= start[n_keys];
-    reduce_body<(G > 1)>(rows, exps, start, dkv_acc, dkv, (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS, n_keys, accumulate, dup_flag, smem);
+    const int key0 = (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS;
+    if (G > 1 && dup_flag[1]) reduce_body<true>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+    else reduce_body<false>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
   }
 }
 
@@ -1296,7 +1297,7 @@ BwdPlan layout_plan(int S, int G, int chunk, int H, int Skv, int K) {
   p.off_prefix = o; o = align_up(o + order::prefix_words(chunk, Skv) * 4);
   p.off_count = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_start = o; o = align_up(o + (size_t)(Skv + 1) * 4);
-  p.off_flag = o; o = align_up(o + 4);
+  p.off_flag = o; o = align_up(o + 8);
   p.off_units = o; o = align_up(o + (G > 1 ? (size_t)((S + G - 1) / G) * 4 : 0));
   p.off_bad = o; o = align_up(o + (size_t)((Skv + 31) / 32) * 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
@@ -1380,7 +1381,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   unsigned* prefix = (unsigned*)(ws + p.off_prefix);
   int* count = (int*)(ws + p.off_count);
   int* start = (int*)(ws + p.off_start);
-  int* dup_flag = (int*)(ws + p.off_flag);
+  int* dup_flag = (int*)(ws + p.off_flag);     // [2]: a query has a repeated id; some queries are worked as one
   int* dstp = (int*)(ws + p.off_dst);
   int* sorted = (int*)(ws + p.off_sorted);
   unsigned char* pds = ws + p.off_pds;
@@ -1432,7 +1433,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
     const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     DSA_MARK(0);
-    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S));
+    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S), (uint4*)exps);
     else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql

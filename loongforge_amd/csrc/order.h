@@ -75,14 +75,14 @@ static __global__ __launch_bounds__(256) void qmap_kernel(const int* __restrict_
 }
 
 // ---- groups of G consecutive queries that may be worked as one unit ----
-// bad[w] bit b  <=>  row 32 w + b of kv (row16 pieces of 16 bytes, bf16) holds a value that is not finite.  Also clears the flag of
-// repeated ids.
+// bad[w] bit b  <=>  row 32 w + b of kv (row16 pieces of 16 bytes, bf16) holds a value that is not finite.  Also clears the flags
+// of repeated ids and of units.
 static __global__ __launch_bounds__(256) void kv_check_kernel(const uint4* __restrict__ kv, int Skv, int row16, unsigned* __restrict__ bad,
-                                                              int* __restrict__ dup_flag) {
+                                                              int* __restrict__ flags) {
   __shared__ unsigned word;
   if (threadIdx.x == 0) {
     word = 0u;
-    if (blockIdx.x == 0) *dup_flag = 0;
+    if (blockIdx.x == 0) flags[0] = flags[1] = 0;
   }
   __syncthreads();
   const int n = min(32, Skv - 32 * (int)blockIdx.x) * row16;
@@ -114,7 +114,7 @@ struct UnitCost { int unit_fixed, unit_tile, fixed, tile; };
 // themselves the two differ by more than a step of the largest row (by 7e-3 more; from 65 keys on they stay 9e-3 within it).
 constexpr int UNIT_FEW = 64;
 
-// qmap_kernel for a group of G queries per workgroup.  units[group] = slots of the unit, a multiple of 32, or 0 for single queries.  A
+// qmap_kernel for a group of G queries per workgroup.  dup_flag[1]: there is a unit.  units[group] = slots of the unit, a multiple of 32, or 0 for single queries.  A
 // unit has the bits of all its queries in its first one's row of qmap, so that it counts as one query in everything behind; its
 // list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query at the end, up to
 // UNIT_FEW or more than max_slots keys, keys with values that are not finite (a product over the slots would carry them to the queries that do not have
@@ -192,7 +192,10 @@ static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __rest
     apart += n[j] ? cost.fixed + cost.tile * ((n[j] + 31) / 32) : 0;
   }
   const bool unit = nq == G && keys > UNIT_FEW && 32 * tiles <= max_slots && total[NC - 1] >> 16 == 0u && cost.unit_fixed + cost.unit_tile * tiles <= apart;
-  if (tid == 0) units[blockIdx.x] = unit ? 32 * tiles : 0;
+  if (tid == 0) {
+    units[blockIdx.x] = unit ? 32 * tiles : 0;
+    if (unit) dup_flag[1] = 1;
+  }
   for (int w = w0; w < w1; w++) {
     if (unit) {
       pre[w] = inc[NC - 1] & 0xffffu;
@@ -261,10 +264,19 @@ static __global__ __launch_bounds__(256) void bm_transpose_kernel(const unsigned
 }
 
 // prefix[w][key] = number of set bits of the key in words < w; count[key] = total.  A workgroup takes 64 keys; its 16 waves
-// count a part of the words each, then write the prefixes of that part.
+// count a part of the words each, then write the prefixes of that part.  Workgroups behind those clear `marks` (n_marks of 16 bytes)
+// if there is a unit: the counting leaves most of the chip idle.
 static __global__ __launch_bounds__(1024) void bm_prefix_kernel(const unsigned* __restrict__ bitmap, unsigned* __restrict__ prefix,
-                                                                int* __restrict__ count, int Skv, int W) {
+                                                                int* __restrict__ count, int Skv, int W, const int* __restrict__ flags,
+                                                                uint4* __restrict__ marks, size_t n_marks) {
   __shared__ int part[16][64];
+  const int counting = (Skv + 63) / 64;
+  if ((int)blockIdx.x >= counting) {
+    if (flags[1])
+      for (size_t e = (size_t)((int)blockIdx.x - counting) * 1024 + threadIdx.x; e < n_marks; e += (size_t)(gridDim.x - counting) * 1024)
+        marks[e] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
   const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
   const int key = min(blockIdx.x * 64 + lane, (unsigned)Skv - 1u);
   const bool live = blockIdx.x * 64 + lane < (unsigned)Skv;
@@ -382,11 +394,13 @@ inline bool sorted_list_fits(int Skv, int K) {
 // dup_flag: one int the caller has cleared (clear_flag) before the first block of queries of a call.
 inline void clear_flag(int* dup_flag, hipStream_t st) { zero_u32_kernel<<<dim3(1), dim3(64), 0, st>>>((unsigned*)dup_flag, 1); }
 inline void build_ranks(const int* lists, int row0, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
-                        int* count, int* start, int* dst, int W, const int* units, int G, hipStream_t st) {
+                        int* count, int* start, int* dst, int W, const int* units, int G, hipStream_t st, const int* flags = nullptr,
+                        uint4* marks = nullptr, size_t n_marks = 0) {
   const int Wk = (Skv + 31) / 32;
   // every word of the bitmap is written (zeros beyond the last query), so no clearing pass is needed
   bm_transpose_kernel<<<dim3((W + 7) / 8, Wk), dim3(256), 0, st>>>(prefix, cnt, Skv, Wk, bitmap, W);
-  bm_prefix_kernel<<<dim3((Skv + 63) / 64), dim3(1024), 0, st>>>(bitmap, prefix, count, Skv, W);
+  const int clearing = (int)((n_marks + 4095) / 4096 < 512 ? (n_marks + 4095) / 4096 : 512);
+  bm_prefix_kernel<<<dim3((Skv + 63) / 64 + clearing), dim3(1024), 0, st>>>(bitmap, prefix, count, Skv, W, flags, marks, n_marks);
   key_scan_kernel<<<dim3(1), dim3(1024), 0, st>>>(count, start, Skv);
   const int range = Skv < RANK_KEYS ? Skv : RANK_KEYS;
   if (range * 8 > 48 * 1024) (void)dsa_reserve_lds((const void*)rank_kernel, (size_t)range * 8);
@@ -405,16 +419,17 @@ inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, 
 }
 // LDS of qmap_unit_kernel
 inline bool unit_lists_fit(int G, int Skv) { return (size_t)((Skv + 31) / 32) * 4 * (G + G / 2) <= (size_t)150 * 1024; }
-// build with the sorted lists, for groups of G (2 or 4) queries that may be units
+// build with the sorted lists, for groups of G (2 or 4) queries that may be units; 16 bytes of `marks` for every row (cnt K at most) are
+// cleared if there are any
 inline void build_units(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix, int* count, int* start,
                         int* dst, int W, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
-                        UnitCost cost) {
+                        UnitCost cost, uint4* marks) {
   const int Wk = (Skv + 31) / 32;
   const size_t lds = (size_t)Wk * 4 * (G + G / 2);
   auto kernel = G == 2 ? qmap_unit_kernel<2> : qmap_unit_kernel<4>;
   if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)kernel, lds);
   kernel<<<dim3((cnt + G - 1) / G), dim3(512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
-  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st);
+  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st, dup_flag, marks, (size_t)cnt * K);
 }
 
 }  // namespace order
