@@ -108,16 +108,10 @@ static __global__ __launch_bounds__(256) void kv_check_kernel(const uint4* __res
 // What a group costs as one unit and as single queries: a fixed part and a part per 32 slots each
 struct UnitCost { int unit_fixed, unit_tile, fixed, tile; };
 
-// Up to this many keys queries stay by themselves: their lists take next to nothing, and where so few share the probability the rows of the pairs are
-// large.  A unit's row is rounded to bf16 once where its queries' rows are rounded each: no larger an error in all (rms 2.06e-3 either way
-// over 2048 queries x 512 slots at random, largest 0.113 and 0.100), but on the key that the first queries of a sequence have to
-// themselves the two differ by more than a step of the largest row (by 7e-3 more; from 65 keys on they stay 9e-3 within it).
-constexpr int UNIT_FEW = 64;
-
 // qmap_kernel for a group of G queries per workgroup.  dup_flag[1]: there is a unit.  units[group] = slots of the unit, a multiple of 32, or 0 for single queries.  A
 // unit has the bits of all its queries in its first one's row of qmap, so that it counts as one query in everything behind; its
-// list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query at the end, up to
-// UNIT_FEW or more than max_slots keys, keys with values that are not finite (a product over the slots would carry them to the queries that do not have
+// list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query at the end, without a key
+// or with more than max_slots, keys with values that are not finite (a product over the slots would carry them to the queries that do not have
 // them), and what costs less query by query.
 template <int G>
 static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __restrict__ ids, int q0, int cnt, int K, int Skv, int q_start,
@@ -191,7 +185,7 @@ static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __rest
     n[j] = (int)(total[j / 2] >> (16 * (j & 1)) & 0xffffu);
     apart += n[j] ? cost.fixed + cost.tile * ((n[j] + 31) / 32) : 0;
   }
-  const bool unit = nq == G && keys > UNIT_FEW && 32 * tiles <= max_slots && total[NC - 1] >> 16 == 0u && cost.unit_fixed + cost.unit_tile * tiles <= apart;
+  const bool unit = nq == G && keys > 0 && 32 * tiles <= max_slots && total[NC - 1] >> 16 == 0u && cost.unit_fixed + cost.unit_tile * tiles <= apart;
   if (tid == 0) {
     units[blockIdx.x] = unit ? 32 * tiles : 0;
     if (unit) dup_flag[1] = 1;

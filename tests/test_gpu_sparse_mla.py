@@ -467,7 +467,8 @@ def test_backward_of_joint_queries(gpu, H, S, K, skv, turn, far):
     assert torch.isnan(dq3.float()).all() and torch.isnan(dkv3.float()).all()
 
 
-@pytest.mark.parametrize("H,S,K,skv", [(64, 512, 128, 300), (64, 1024, 64, 72), (32, 800, 128, 300), (32, 768, 64, 200)])
+@pytest.mark.parametrize("H,S,K,skv", [(64, 512, 128, 300), (64, 1024, 64, 72), (64, 520, 64, 64), (32, 800, 128, 300), (32, 768, 64, 200),
+                                       (32, 800, 64, 64)])
 @pytest.mark.parametrize("alike,steep", [(0.0, 1.0), (0.9, 1.0), (0.99, 1.0), (0.9, 2.0)])
 def test_backward_of_joint_queries_is_no_less_accurate_than_one_by_one(gpu, H, S, K, skv, alike, steep):
     """Neighbouring queries with most of their keys, and of their values (``alike``: correlation of Q and dO), in common: dKV is no
@@ -480,8 +481,9 @@ def test_backward_of_joint_queries_is_no_less_accurate_than_one_by_one(gpu, H, S
     mix = lambda t: (alike ** 0.5 * torch.randn((S + 7) // 8, 1, *t.shape[1:], generator=g).expand(-1, 8, -1, -1).flatten(0, 1)[:S]    # noqa: E731
                      + (1 - alike) ** 0.5 * torch.randn(t.shape, generator=g)).to(torch.bfloat16)
     inp.q, inp.dout = mix(inp.q), mix(inp.dout)
-    pool = torch.stack([torch.randperm(skv, generator=g)[:K + K // 8] for _ in range((S + 7) // 8)])
-    inp.idx = torch.stack([pool[i // 8][torch.randperm(K + K // 8, generator=g)[:K]] for i in range(S)]).int()
+    some = min(K + K // 8, skv)
+    pool = torch.stack([torch.randperm(skv, generator=g)[:some] for _ in range((S + 7) // 8)])
+    inp.idx = torch.stack([pool[i // 8][torch.randperm(some, generator=g)[:K]] for i in range(S)]).int()
     q, kv, idx, do, sm = inp.q.to(gpu), inp.kv.to(gpu), inp.idx.to(gpu), inp.dout.to(gpu), steep * inp.sm_scale
     out, lse, _ = ops.sparse_mla_fwd(q, kv, idx, skv, sm)
     dq, dkv, G, joint = mla_bwd_with_groups(q, kv, out, do, idx, lse, skv, sm)
