@@ -1013,8 +1013,12 @@ __device__ __forceinline__ uint4 row_load16(const void* p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 constexpr int RED_GROUPS = 7;
-constexpr int RED_FLIGHT = 8;                // row pieces a thread loads at a time; it sums one such batch while the next is on its way
-constexpr int RED_BATCH = RED_FLIGHT * RED_GROUPS;
+// Row pieces a thread loads at a time; it sums one such batch while the next is on its way.  A batch never holds rows of two keys, so what a key
+// lacks of it is loaded in vain: batches of 2 where there are few rows per key.  Whole backward, us, batches of 2 / 4 / 8 / one of 16 at a
+// time and single loads: 2000 queries x 512 slots of 131072 keys (8 rows per key) 128 heads 1865 / 1962 / 2257 / 2049, 64 heads
+// 1704 / 1805 / 2101 / 1772; 8000 x 256 of 131072 (16) x 64 heads 3269 / 3273 / 3608 / 3339, of 32768 (62) 2247 / 2247 / 2281 / 2484, of
+// 8000 (256) 2025 / 1988 / 2020 / 1938; with 128 heads 2568 / 2559 / 2577 / 2765.
+constexpr int RED_FLIGHT = 4, RED_FLIGHT_FEW = 2, RED_FEW_ROWS = 24;
 constexpr int RED_KEYS = 4;                  // consecutive keys per workgroup
 // A workgroup sums RED_KEYS consecutive keys (their rows follow one another in the buffer): every thread walks its
 // share of the first key's rows, then of the next one's, without a barrier in between; one barrier, then the seven partial sums of each key are
@@ -1022,10 +1026,11 @@ constexpr int RED_KEYS = 4;                  // consecutive keys per workgroup
 // exposed once a key has few rows per launch: with the queries of 32768 tokens walked in four chunks the launch
 // took 27.1 ms against 18.9 ms for one sweep; per key the sums and their order are the same as before.)
 // SCALED: rows may be those of joint units; a chunk's exponent is loaded beside it.
-template <bool SCALED>
+template <bool SCALED, int RED_FLIGHT>
 __device__ __forceinline__ void reduce_body(const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
                                             float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int key0, int n_keys,
                                             int accumulate, const int* __restrict__ dup_flag, unsigned char* smem) {
+  constexpr int RED_BATCH = RED_FLIGHT * RED_GROUPS;
   float* part = (float*)smem;                  // [RED_KEYS][RED_GROUPS][DQK]
   const int tid = threadIdx.x;
   const int ch = tid % 72, grp = tid / 72;
@@ -1243,8 +1248,14 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const int groups = (n_keys + RED_KEYS - 1) / RED_KEYS;
     const bool forward = 2 * (long long)start[n_keys / 2] >= start[n_keys];
     const int key0 = (forward ? rs.i : groups - 1 - rs.i) * RED_KEYS;
-    if (G > 1 && dup_flag[1]) reduce_body<true>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
-    else reduce_body<false>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+    const bool few = start[n_keys] < RED_FEW_ROWS * (long long)n_keys;
+    if (G > 1 && dup_flag[1]) {
+      if (few) reduce_body<true, RED_FLIGHT_FEW>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+      else reduce_body<true, RED_FLIGHT>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+    } else {
+      if (few) reduce_body<false, RED_FLIGHT_FEW>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+      else reduce_body<false, RED_FLIGHT>(rows, exps, start, dkv_acc, dkv, key0, n_keys, accumulate, dup_flag, smem);
+    }
   }
 }
 
