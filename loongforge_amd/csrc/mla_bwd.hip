@@ -53,8 +53,8 @@ constexpr int PDS_THREADS = 512;
 // In bf16 the rows' rounding error would be that of the rows it stands for only
 // where those are independent, and grows with what neighbouring queries have in common: rms over 256 queries x 256 of 288 slots, rows per query 1,
 // unit in bf16 / fp16: correlation 0 of Q and dO 1.00 / 0.13, 0.9 1.27 / 0.16 (64 heads) and 1.68 / 0.21 (32 heads), 0.99 1.36 / 0.17 and 1.88 /
-// 0.24.  What it takes, bf16 / fp16: scores and rows 530 / 575 us at 3072 queries x 640 slots x 64 heads and 276 / 299 at 2077 x 512 (maxima 16
-// of the 45, the rest products with the power and the exponents' way through LDS), dQ and the sums 308 / 317 and 179 / 185.
+// 0.24.  What it takes, bf16 / fp16: scores and rows 521 / 562 us at 3072 queries x 640 slots x 64 heads and 276 / 297 at 2077 x 512 (maxima 22
+// of the 41, products with the power 10, the exponents' way through LDS 8), dQ and the sums 308 / 314 and 180 / 176.
 constexpr int unit_queries(int HG) { return 4 / HG; }
 constexpr int UNIT_SLOTS = 3072;             // what the lists in LDS behind the operands of 128 heads have room for
 constexpr int UNIT_KEY = 0xffffff;
@@ -592,12 +592,11 @@ __device__ __forceinline__ unsigned group_max(const f32x4 (&x)[N]) {
 }
 // 2^(14 - k) for a largest magnitude of 2^k .. 2^(k + 1), whose exponent bits are kept with the row
 __device__ __forceinline__ float group_scale(unsigned most) { return __builtin_bit_cast(float, (268u << 23) - (most & 0x7f800000u)); }
-// (a scale, b scale) in fp16, product and rounding in one instruction each
+// (a scale, b scale) in fp16.  (v_fma_mixlo_f16 / mixhi, a product and its rounding in one, are no faster than these three: scores and rows
+// of 3072 queries x 640 slots 566 and 562 us.)
 __device__ __forceinline__ unsigned scaled_pk_f16(float a, float b, float scale) {
-  unsigned r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(scale));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(b), "v"(scale));
-  return r;
+  const f32x2_t v = {a * scale, b * scale};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, f16x2_t));
 }
 
 // Zero where a bf16 value is not finite (exponent all ones), in 16 bytes of LDS
@@ -1278,8 +1277,12 @@ __global__ void poison_bf16_kernel(unsigned short* __restrict__ p, size_t n, con
 // host side
 // ---------------------------------------------------------------------------------------------
 // Units pay from 192 groups on, where their lists fit.  Below, too many of the 256 compute units are left without one: 150 pairs of queries
-// 82 us by themselves and 85 joint, 75 groups of four 72 and 82, and looking for them costs 2 - 8 us.
-bool use_units(int HG, int S, int Skv) { return HG < 4 && S >= 192 * unit_queries(HG) && order::unit_lists_fit(unit_queries(HG), Skv); }
+// 82 us by themselves and 85 joint, 75 groups of four 72 and 82.  Looking for them where there are none costs the difference of
+// qmap_unit_kernel and qmap_kernel and the look at the keys: 6 + 5 us at 8000 queries x 256 slots of 8000 keys (whole backward 1990), 4 + 8 at
+// 3000 x 2048 of 32768 (4950), -4 + 23 at 2000 x 512 of 131072 (1580).
+bool use_units(int HG, int S, int Skv, int K) {
+  return HG < 4 && S >= 192 * unit_queries(HG) && order::unit_lists_lds(unit_queries(HG), Skv, K) <= (size_t)150 * 1024;
+}
 
 struct BwdPlan {
   int chunk;            // queries per pass over the buffers, a multiple of G
@@ -1290,9 +1293,9 @@ struct BwdPlan {
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-int group_queries(int S, int H, int Skv) {
+int group_queries(int S, int H, int Skv, int K) {
   const int HG = head_groups(H);
-  return use_units(HG, S, Skv) ? unit_queries(HG) : 1;
+  return use_units(HG, S, Skv, K) ? unit_queries(HG) : 1;
 }
 
 // For S queries in groups of G, `chunk` of them at a time
@@ -1325,7 +1328,7 @@ BwdPlan layout_plan(int S, int G, int chunk, int H, int Skv, int K) {
 // buffers fit the budget; without units if those of the smallest chunk do not.
 BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
   BwdPlan p;
-  for (int G = group_queries(S, H, Skv);; G = 1) {
+  for (int G = group_queries(S, H, Skv, K);; G = 1) {
     int chunk = S;
     p = layout_plan(S, G, chunk, H, Skv, K);
     while (p.total > budget && chunk > 64) {
@@ -1358,7 +1361,7 @@ extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes(int S, int H, int Skv, int 
 
 extern "C" size_t dsa_sparse_mla_bwd_workspace_bytes_min(int S, int H, int Skv, int K) {
   if (S <= 0 || Skv <= 0 || K <= 0) return 0;
-  return layout_plan(S, group_queries(S, H, Skv), S < 64 ? S : 64, H, Skv, K).total;
+  return layout_plan(S, group_queries(S, H, Skv, K), S < 64 ? S : 64, H, Skv, K).total;
 }
 
 extern "C" int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t workspace_bytes, size_t* units_offset) {

@@ -108,58 +108,89 @@ static __global__ __launch_bounds__(256) void kv_check_kernel(const uint4* __res
 // What a group costs as one unit and as single queries: a fixed part and a part per 32 slots each
 struct UnitCost { int unit_fixed, unit_tile, fixed, tile; };
 
-// qmap_kernel for a group of G queries per workgroup.  dup_flag[1]: there is a unit.  units[group] = slots of the unit, a multiple of 32, or 0 for single queries.  A
-// unit has the bits of all its queries in its first one's row of qmap, so that it counts as one query in everything behind; its
-// list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query at the end, without a key
-// or with more than max_slots, keys with values that are not finite (a product over the slots would carry them to the queries that do not have
-// them), and what costs less query by query.
-template <int G>
-static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __restrict__ ids, int q0, int cnt, int K, int Skv, int q_start,
+// Words of a key bitmap in LDS: whole 16-byte pieces
+__host__ __device__ inline int unit_words(int n) { return (n + 3) / 4 * 4; }
+// qmap_kernel for a group of G queries per workgroup.  dup_flag[1]: there is a unit.  units[group] = slots of the unit, a multiple of 32,
+// or 0 for single queries.  A unit has the bits of all its queries in its first one's row of qmap, so that it counts as one query in
+// everything behind; its list (G K places from the first query's on) holds key | queries << 24.  Not a unit: groups that lack a query
+// at the end, without a key or with more than max_slots, keys with values that are not finite (a product over the slots would carry
+// them to the queries that do not have them), and what costs less query by query.
+// Like qmap_kernel it goes over the words of the key bitmap, four at a time, and over the ids; it is bound by latency, LDS traffic and the
+// workgroups that the LDS leaves room for.  us, with the lists made by a walk over all keys / as they are; qmap_kernel, for queries by
+// themselves: 8000 queries x 256 slots of 8000 keys in pairs 43 / 22; 16, of 131072 312 / 68; 100; 3000 x 2048 of 32768 48 / 22; 18; in fours
+// 8000 x 256 of 32768 69 / 22; 21, 2000 x 512 of 131072 144 / 27; 31.
+template <int G, int BL>
+static __global__ __launch_bounds__(BL) void qmap_unit_kernel(const int* __restrict__ ids, int q0, int cnt, int K, int Skv, int q_start,
                                                                unsigned* __restrict__ qmap, int Wk, int* __restrict__ sorted,
                                                                int* __restrict__ dup_flag, const unsigned* __restrict__ bad,
                                                                int* __restrict__ units, int max_slots, UnitCost cost) {
-  extern __shared__ unsigned qbits[];        // [G][Wk] bits, [G / 2][Wk] prefix counts, 16 bits each
-  __shared__ unsigned wave_tot[G / 2 + 1][8];
+  extern __shared__ __attribute__((aligned(16))) unsigned qbits[];      // [G][WL] bits, [G / 2][WL] prefix counts, 16 bits each, [G][K] list
+  __shared__ unsigned wave_tot[G / 2 + 1][BL / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ql0 = blockIdx.x * G, nq = min(G, cnt - ql0);
-  unsigned* pre = qbits + G * Wk;
-  for (int w = tid; w < G * Wk; w += 512) qbits[w] = 0u;
-  __syncthreads();
+  const int ql0 = blockIdx.x * G, nq = min(G, cnt - ql0), n_ids = nq * K;
+  const int WL = unit_words(Wk);
+  unsigned* pre = qbits + G * WL;
+  int* list = (int*)(pre + G / 2 * WL);
   const int* src = ids + (size_t)(q0 + ql0) * K;
-  for (int t0 = tid; t0 < nq * K; t0 += 8 * 512) {
-    int v[8];
+  // f(id, query) for every valid id, the first 8 of a thread requested ahead
+  int v[8];
+  auto request = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = t0 + i * 512 < nq * K ? src[t0 + i * 512] : -1;
+    for (int i = 0; i < 8; i++) v[i] = src[min(t0 + i * BL, n_ids - 1)];
+  };
+  auto each_id = [&](bool have, auto f) {
+    for (int t0 = tid; t0 < n_ids; t0 += 8 * BL) {
+      if (!have || t0 >= 8 * BL) request(t0);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int j = __builtin_amdgcn_readfirstlane((t0 + i * 512) / K);        // (K is a multiple of 64: the same for a wave)
-      if (v[i] >= 0 && v[i] < Skv && v[i] <= q_start + q0 + ql0 + j) {
-        const unsigned bit = 1u << (v[i] & 31);
-        if (atomicOr(&qbits[j * Wk + (v[i] >> 5)], bit) & bit) *dup_flag = 1;
+      for (int i = 0; i < 8; i++) {
+        const int t = t0 + i * BL, j = __builtin_amdgcn_readfirstlane(t / K);        // (K is a multiple of 64: the same for a wave)
+        if (t < n_ids && v[i] >= 0 && v[i] < Skv && v[i] <= q_start + q0 + ql0 + j) f(v[i], j);
       }
     }
-  }
-  __syncthreads();
-  const int per = (Wk + 511) / 512, w0 = tid * per, w1 = min(w0 + per, Wk);
-  auto any = [&](int w) {
-    unsigned b = qbits[w];
-#pragma unroll
-    for (int j = 1; j < G; j++) b |= qbits[j * Wk + w];
-    return b;
   };
+  request(tid);
+  for (int w = 4 * tid; w < G * WL; w += 4 * BL) *(uint4*)(qbits + w) = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  each_id(true, [&](int id, int j) {
+    const unsigned bit = 1u << (id & 31);
+    if (atomicOr(&qbits[j * WL + (id >> 5)], bit) & bit) *dup_flag = 1;
+  });
+  __syncthreads();
   // one scan over the threads: the queries' counts in pairs (a query has at most 2048 keys), then the union's beside the number of
   // threads that saw a key with values that are not finite
+  const int per = unit_words((Wk + BL - 1) / BL), w0 = min(tid * per, WL), w1 = min(w0 + per, WL);
   constexpr int NC = G / 2 + 1;
   unsigned mine[NC], inc[NC], total[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) mine[c] = 0u;
-  for (int w = w0; w < w1; w++) {
+  bool sees_bad = false;
+  struct Words { unsigned own[G][4], any[4]; };
+  auto words = [&](int w) {                  // of four neighbouring words: the queries' bits and their union
+    Words x;
 #pragma unroll
-    for (int j = 0; j < G; j++) mine[j / 2] += (unsigned)__popc(qbits[j * Wk + w]) << (16 * (j & 1));
-    const unsigned b = any(w);
-    mine[NC - 1] += __popc(b);
-    if (b & bad[w]) mine[NC - 1] |= 0x10000u;
+    for (int j = 0; j < G; j++) {
+      const uint4 b = *(const uint4*)(qbits + j * WL + w);
+      const unsigned y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        x.own[j][i] = y[i];
+        x.any[i] = j ? x.any[i] | y[i] : y[i];
+      }
+    }
+    return x;
+  };
+  for (int w = w0; w < w1; w += 4) {
+    const Words x = words(w);
+    const uint4 b = *(const uint4*)(bad + w);
+    sees_bad |= ((x.any[0] & b.x) | (x.any[1] & b.y) | (x.any[2] & b.z) | (x.any[3] & b.w)) != 0u;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+      for (int j = 0; j < G; j++) mine[j / 2] += (unsigned)__popc(x.own[j][i]) << (16 * (j & 1));
+      mine[NC - 1] += __popc(x.any[i]);
+    }
   }
+  if (sees_bad) mine[NC - 1] |= 0x10000u;
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     inc[c] = mine[c];
@@ -173,7 +204,7 @@ static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __rest
     inc[c] -= mine[c];
     total[c] = 0u;
 #pragma unroll
-    for (int w = 0; w < 8; w++) {
+    for (int w = 0; w < BL / 64; w++) {
       if (w < wave) inc[c] += wave_tot[c][w];
       total[c] += wave_tot[c][w];
     }
@@ -190,50 +221,65 @@ static __global__ __launch_bounds__(512) void qmap_unit_kernel(const int* __rest
     units[blockIdx.x] = unit ? 32 * tiles : 0;
     if (unit) dup_flag[1] = 1;
   }
-  for (int w = w0; w < w1; w++) {
-    if (unit) {
-      pre[w] = inc[NC - 1] & 0xffffu;
-      inc[NC - 1] += __popc(any(w));
-    } else {
+  inc[NC - 1] &= 0xffffu;
+  for (int w = w0; w < w1; w += 4) {
+    const Words x = words(w);
+    unsigned p[NC - 1][4];
 #pragma unroll
-      for (int c = 0; c < NC - 1; c++) {
-        pre[c * Wk + w] = inc[c];
-        inc[c] += (unsigned)__popc(qbits[2 * c * Wk + w]) + ((unsigned)__popc(qbits[(2 * c + 1) * Wk + w]) << 16);
+    for (int i = 0; i < 4; i++) {
+      if (unit) {
+        p[0][i] = inc[NC - 1];
+        inc[NC - 1] += __popc(x.any[i]);
+      } else {
+#pragma unroll
+        for (int c = 0; c < NC - 1; c++) {
+          p[c][i] = inc[c];
+          inc[c] += (unsigned)__popc(x.own[2 * c][i]) + ((unsigned)__popc(x.own[2 * c + 1][i]) << 16);
+        }
       }
     }
+#pragma unroll
+    for (int c = 0; c < NC - 1; c++)
+      if (!unit || c == 0) *(uint4*)(pre + c * WL + w) = make_uint4(p[c][0], p[c][1], p[c][2], p[c][3]);
   }
+  auto any = [&](int w) {
+    unsigned b = qbits[w];
+#pragma unroll
+    for (int j = 1; j < G; j++) b |= qbits[j * WL + w];
+    return b;
+  };
   for (int j = 0; j < nq; j++)
-    for (int w = tid; w < Wk; w += 512) qmap[(size_t)(ql0 + j) * Wk + w] = !unit ? qbits[j * Wk + w] : j == 0 ? any(w) : 0u;
+    for (int w = tid; w < Wk; w += BL) qmap[(size_t)(ql0 + j) * Wk + w] = !unit ? qbits[j * WL + w] : j == 0 ? any(w) : 0u;
   __syncthreads();
-  // the lists, ascending: a thread per key, whose place is the number of set bits below it
-  int* row = sorted + (size_t)ql0 * K;
-  for (int k = tid; k < 32 * Wk; k += 512) {
-    const int w = k >> 5, b = k & 31;
+  // the lists, ascending: an id's place is the number of set bits below it (an id of several queries of a unit is put there by each)
+  each_id(n_ids <= 8 * BL, [&](int id, int j) {
+    const int w = id >> 5, b = id & 31;
     const unsigned below = (1u << b) - 1u;
-    unsigned own[G], bits = 0u;
-    int v = k;
-#pragma unroll
-    for (int j = 0; j < G; j++) {
-      own[j] = qbits[j * Wk + w];
-      bits |= own[j];
-      v |= (int)(own[j] >> b & 1u) << (24 + j);
-    }
     if (unit) {
-      if (bits >> b & 1u) row[pre[w] + __popc(bits & below)] = v;
-    } else {
+      unsigned bits = 0u;
+      int entry = id;
 #pragma unroll
-      for (int j = 0; j < G; j++)
-        if (own[j] >> b & 1u) row[j * K + (int)(pre[(j / 2) * Wk + w] >> (16 * (j & 1)) & 0xffffu) + __popc(own[j] & below)] = k;
+      for (int k = 0; k < G; k++) {
+        const unsigned own = qbits[k * WL + w];
+        bits |= own;
+        entry |= (int)(own >> b & 1u) << (24 + k);
+      }
+      list[pre[w] + __popc(bits & below)] = entry;
+    } else {
+      list[j * K + (int)(pre[(j >> 1) * WL + w] >> (16 * (j & 1)) & 0xffffu) + __popc(qbits[j * WL + w] & below)] = id;
     }
-  }
+  });
   if (unit) {
-    for (int t = keys + tid; t < G * K; t += 512) row[t] = -1;
+    for (int t = keys + tid; t < n_ids; t += BL) list[t] = -1;
   } else {
 #pragma unroll
     for (int j = 0; j < G; j++)
       if (j < nq)
-        for (int t = n[j] + tid; t < K; t += 512) row[j * K + t] = -1;
+        for (int t = n[j] + tid; t < K; t += BL) list[j * K + t] = -1;
   }
+  __syncthreads();
+  int* row = sorted + (size_t)ql0 * K;
+  for (int t = 4 * tid; t < n_ids; t += 4 * BL) *(int4*)(row + t) = *(const int4*)(list + t);
 }
 
 // grid (ceil(cnt / 256), Wk); workgroup = 4 waves = 256 queries of one key word
@@ -412,17 +458,18 @@ inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, 
   build_ranks(sorted ? sorted : ids, sorted ? 0 : q0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, nullptr, 1, st);
 }
 // LDS of qmap_unit_kernel
-inline bool unit_lists_fit(int G, int Skv) { return (size_t)((Skv + 31) / 32) * 4 * (G + G / 2) <= (size_t)150 * 1024; }
+inline size_t unit_lists_lds(int G, int Skv, int K) { return (size_t)unit_words((Skv + 31) / 32) * 4 * (G + G / 2) + (size_t)G * K * 4; }
 // build with the sorted lists, for groups of G (2 or 4) queries that may be units; 16 bytes of `marks` for every row (cnt K at most) are
 // cleared if there are any
 inline void build_units(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix, int* count, int* start,
                         int* dst, int W, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
                         UnitCost cost, uint4* marks) {
   const int Wk = (Skv + 31) / 32;
-  const size_t lds = (size_t)Wk * 4 * (G + G / 2);
-  auto kernel = G == 2 ? qmap_unit_kernel<2> : qmap_unit_kernel<4>;
+  const size_t lds = unit_lists_lds(G, Skv, K);
+  const bool small = G * K <= 2048 && Wk <= 1024;      // (one round of ids for 256 threads, and then twice the workgroups on a compute unit)
+  auto kernel = G == 2 ? (small ? qmap_unit_kernel<2, 256> : qmap_unit_kernel<2, 512>) : small ? qmap_unit_kernel<4, 256> : qmap_unit_kernel<4, 512>;
   if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)kernel, lds);
-  kernel<<<dim3((cnt + G - 1) / G), dim3(512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
+  kernel<<<dim3((cnt + G - 1) / G), dim3(small ? 256 : 512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
   build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st, dup_flag, marks, (size_t)cnt * K);
 }
 
