@@ -436,8 +436,8 @@ def _assert_rounded_rows(dkv, inp, units, q_start, sm, out, lse):
     (64, 515, 128, 900, 1, 0),        # pairs of queries as one, one query left over
     (64, 520, 192, 1400, 1, 3),       # both kinds of groups
     (64, 513, 128, 520, 2, 0),        # lists that begin short
-    (64, 402, 192, 40_000, 1, 3),     # long key arrays
-    (32, 800, 64, 33_000, 2, 2),
+    (64, 520, 192, 40_000, 1, 3),     # long key arrays
+    (32, 1030, 64, 33_000, 2, 2),
     (32, 768, 64, 1100, 1, 0),        # four queries as one
     (32, 771, 64, 1500, 1, 2),        # three queries left over, both kinds
 ])
