@@ -16,6 +16,7 @@
 // an exclusive scan over keys: integer work only, so the order - and with it every fp32 sum - is
 // identical from run to run.  No floating-point atomics anywhere.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "mla_tile.h"
@@ -1339,15 +1340,16 @@ BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
   }
 }
 
-// What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, fitted to
-// whole backward passes of 1000 - 8000 queries with 8 - 47 tiles (by themselves 62.8 us at 8 tiles, 98.5 at 15, 236 at 42 of 64 heads, 52 /
-// 81 / 216 of 32; units 135 at 15, 200 at 25, 337 at 46).  Units come in rounds of 256 like queries, G times as few: of up to
-// G x 256 queries there is only one.
+// What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, and how much more
+// where the last round of 256 is not full: half of what it lacks, spread over all.  Fitted to whole backward passes of 800 - 6000 queries
+// x 64 - 2048 slots with unions of 1.0 - 3.9 lists, all joint and all by themselves (328 pairs of times): what the prices pick takes 0.1 - 0.2 %
+// more than the better one in the mean, 5 % at most.  us, joint / by themselves, 64 heads: 1100 x 512 547 / 489 (union 24 tiles), 461 /
+// 571 (16), 2077 x 512 962 / 918 (24), 801 / 1031 (16); 32 heads: 1100 x 512 533 / 392 (44), 318 / 426 (23), 3072 x 512 1073 / 1024 (44),
+// 807 / 1076 (28).
 order::UnitCost unit_cost(int HG, int S) {       // (HG 1 or 2)
-  const int G = unit_queries(HG), CUS = 256;
-  const float unit = std::max(1.0f, (float)(G * CUS) / S), apart = std::max(1.0f, (float)CUS / S);
-  const float fixed = HG == 2 ? 226.f : 140.f, tile = HG == 2 ? 50.f : 48.f;
-  return {(int)(420.f * unit), (int)(66.f * unit), (int)(fixed * apart), (int)(tile * apart)};
+  auto waste = [](float rounds) { return rounds < 1.f ? 1.f / rounds : 1.f + 0.5f * (std::ceil(rounds) - rounds) / rounds; };
+  const float unit = waste((float)S / (256 * unit_queries(HG))), apart = waste((float)S / 256);
+  return {(int)((HG == 2 ? 280.f : 460.f) * unit), (int)(70.f * unit), (int)(180.f * apart), (int)((HG == 2 ? 50.f : 48.f) * apart)};
 }
 
 constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;

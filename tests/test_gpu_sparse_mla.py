@@ -500,12 +500,12 @@ def test_backward_of_joint_queries_is_no_less_accurate_than_one_by_one(gpu, H, S
 
 
 @pytest.mark.parametrize("H,S,K,skv,causal", [
-    (64, 700, 2048, 4076, False),     # unions beyond the longest list of a unit, and within it
+    (64, 700, 2048, 2300, False),
+    (32, 1100, 2048, 3110, False),    # unions beyond the longest list of a unit, and within it
     (64, 1030, 512, 1200, True),
-    (32, 1100, 2048, 2900, False),    # nearly the longest list
     (32, 1537, 192, 1537, True),      # from one key on
     (32, 1540, 256, 6000, False),     # little in common: no units
-    (32, 2103, 128, 2103, True),      # more than two rounds of groups
+    (32, 2103, 128, 400, False),      # more than two rounds of groups
 ])
 def test_backward_of_joint_queries_is_that_of_wider_queries(gpu, H, S, K, skv, causal):
     """The same gradients as through the kernels for 128 heads with heads of zeros beside the queries' own, in one sweep and in
