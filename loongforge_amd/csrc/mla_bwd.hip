@@ -1171,8 +1171,9 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-// The query of workgroup i, from the last one on (RAMP > 0: but for the first 256, spread over the last RAMP * K); with groups of G in G turns over the groups with one query of each, so that the
-// workgroups that do joint units follow one another.  Neighbouring workgroups go to different XCDs: with the groups' queries side by side
+// The query of workgroup i: from the last query on, but for the first 256 workgroups if RAMP > 0, which spread over the last RAMP * K.
+// Groups of G queries are gone over in G turns, one query of each group at a time, so that the workgroups that do joint units (a
+// group's first query) follow one another: neighbouring workgroups go to different XCDs, and with the groups' queries side by side
 // every G-th workgroup did the work, on 8 / G of the XCDs (3072 x 32 heads x 640 slots: scores and rows 865 us instead of 296).
 // RAMP: scores and rows read 410 KB per query or unit in front of 8 to 64 tiles of matrix work.  us, in strict order / first round spread over
 // K / over 4 K queries: 5000 x 128 heads, window and compressed keys 1932 / 1922 / 1770, 3072 x 64 heads of these 590 / 591 / 556, 2077 x

@@ -366,8 +366,8 @@ static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __rest
 
 // dst[ql][slot] = row of the pair in key-sorted order (-1 for invalid slots).  A workgroup takes the 32 queries of a word, or
 // a part of them (blockIdx.y) where there are few words, and has the word's bits and first rows of `range` keys at a time in
-// LDS, where the lookups by id go (units: ids are the lists of qmap_unit_kernel, and a unit's pairs are its first query's): from memory they were two dependent random reads of 4 bytes per pair (8192 queries x
-// 2048 slots: 0.165 ms; 32768 x 2048: 1.29 ms).
+// LDS, where the lookups by id go: from memory they were two dependent random reads of 4 bytes per pair (8192 queries x 2048 slots
+// 0.165 ms; 32768 x 2048 1.29 ms).  With `units` the ids are the lists of qmap_unit_kernel, and the pairs of a unit are its first query's.
 static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict__ ids, int row0, int q0, int cnt, int K, int Skv, int q_start,
                                                            const unsigned* __restrict__ bitmap, const unsigned* __restrict__ prefix,
                                                            const int* __restrict__ start, int range, int* __restrict__ dst,

@@ -195,7 +195,7 @@ constexpr int LIN_MAX_BIN = 256;             // largest segment ranked by pairwi
 // starts written over the counts.  False when a bin is too crowded for the ranking step.
 template <int BL>
 __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff, int& tbin, int& above, int& c) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x;
   constexpr int PER = HBINS / BL;
   int* found = scratch + 3 * NWAVES<BL>;
   int cnt[PER], local = 0;

@@ -552,8 +552,9 @@ class DSAttentionFused(MegatronModule):
         # The logits of the selected slots are needed for one thing only, the head-averaged attention
         # distribution the indexer is trained towards (dsa_fused.py:903-929 of the reference asks the
         # kernel for p_out [sq, n, topk] and reduces it with triton_attn_dist).  Here the attention call
-        # returns that distribution itself, recomputed from q, kv and lse, and only when the loss will
-        # be formed: no [sq, n, topk] tensor exists (4.3 GB at 8k tokens, 17 GB at 32k).
+        # returns that distribution itself, and only when the loss will be formed: the logits pass through a
+        # buffer of at most DSA_P_OUT_BUDGET_GIB (default 6) GiB, so at 8k tokens all of them (4.3 GB)
+        # and at 32k (17 GB) a block of queries at a time.
         need_loss = self.training and torch.is_grad_enabled() and not self.skip_topk
         res = self.sparse_attention(
             chunk_query,

@@ -81,9 +81,9 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
     slot.  As in the reference it is only accepted together with ``return_p_out`` (:2971-2974).
     ``dist_heads`` > 0 (not in the reference) returns, instead of the logits, what the training path
     makes of them: the head-averaged attention distribution over the slots, mean over the first
-    ``dist_heads`` heads (dsa_fused.py:915-929): reduced from the logits when those are a small passing
-    allocation (at most DSA_P_OUT_BUDGET_GIB, default 6, GiB), recomputed from q, kv and lse otherwise, so
-    that no large [sq, n, topk] tensor is ever allocated.
+    ``dist_heads`` heads (dsa_fused.py:915-929): reduced from the logits, which pass through a buffer of all queries, or
+    of a block of them at a time, of at most DSA_P_OUT_BUDGET_GIB (default 6) GiB; recomputed from q, kv and lse
+    where that does not hold the logits of 64 queries (of all, if there are fewer).
     """
 
     @staticmethod

@@ -415,20 +415,6 @@ def indexer_forward(index_q, index_k, weights, rotate: bool, factor: float, cu_s
 # --------------------------------------------------------------------------------------------
 # sparse MLA
 # --------------------------------------------------------------------------------------------
-def _check_mla(q, kv, ids):
-    _need_gpu(q, kv, ids)
-    if q.ndim != 3 or kv.ndim != 2 or ids.ndim != 2:
-        raise ValueError("sparse MLA expects q [S,H,576], kv [Skv,576], ids [S,K]")
-    if q.dtype != torch.bfloat16 or kv.dtype != torch.bfloat16:
-        raise ValueError("sparse MLA expects bf16 q and kv")
-    if q.shape[-1] != 576 or kv.shape[-1] != 576:
-        raise ValueError("you should assign dim otherwise: d_qk must be 576 (512 latent + 64 rope)")
-    if ids.shape[0] != q.shape[0]:
-        raise ValueError("ids and q disagree on the number of queries")
-    if ids.shape[1] % 64 != 0:
-        raise ValueError("top-k must be padded to a multiple of 64 (pad ids with -1)")
-
-
 @torch.library.custom_op("dsa::sparse_mla_fwd", mutates_args=())
 def _mla_fwd_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, q_start: int, sm_scale: float, d_v: int,
                 p_out_mode: int, attn_sink: Optional[torch.Tensor] = None,
