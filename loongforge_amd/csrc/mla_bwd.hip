@@ -708,7 +708,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
     }
     part += __shfl_xor(part, 16, 64);
     part += __shfl_xor(part, 32, 64);
-    if (kg == 0) {
+    if (G > 1 ? fresh_lane() < 16 : kg == 0) {
       stat_s[h] = head_ok ? lse_h * LOG2E : INFINITY;
       stat_s[128 + h] = head_ok ? part : 0.f;
     }
@@ -1171,40 +1171,45 @@ __device__ __forceinline__ RoleSlot role_slot(int b, int nX, int nY) {
   return {true, b - y0};
 }
 
-// The query of workgroup i: from the last query on, but for the first 256 workgroups if RAMP > 0, which spread over the last RAMP * K.
-// Groups of G queries are gone over in G turns, one query of each group at a time, so that the workgroups that do joint units (a
-// group's first query) follow one another: neighbouring workgroups go to different XCDs, and with the groups' queries side by side
-// every G-th workgroup did the work, on 8 / G of the XCDs (3072 x 32 heads x 640 slots: scores and rows 865 us instead of 296).
+// What workgroup i does: a query, and the tiles of its unit if it is the first one of a unit; query -1: nothing.  From the last query on, but for the
+// first 256 workgroups if RAMP > 0, which spread over the last RAMP * K.  Where some queries are worked jointly they follow the
+// work list, so that what has nothing to do comes at the end: a workgroup goes to the XCD, and there to the shader engine, that its number
+// says, and waits for a place there.  (With one workgroup per query, those of a unit's other queries returning at once and eight in a row,
+// G - 1 of G engines were idle: scores and rows of 4001 x 32 heads of window and compressed keys 1290 us instead of 410.)  The list has units and
+// queries by themselves apart: 3000 x 512 of 2000 keys x 32 heads, a third of the groups units, whole backward 1217 us with both kinds mixed,
+// 1158 in turns over the groups' queries, 1033 as it is; 1069 all joint, 989 all by themselves.
 // RAMP: scores and rows read 410 KB per query or unit in front of 8 to 64 tiles of matrix work.  us, in strict order / first round spread over
 // K / over 4 K queries: 5000 x 128 heads, window and compressed keys 1932 / 1922 / 1770, 3072 x 64 heads of these 590 / 591 / 556, 2077 x
 // 512 x 64 heads 304 / 302 / 291, 1300 x 512 x 128 432 / 389 / 415, 8192 x 2048 x 128 8967 / 8906 / 8865, long documents of few slots
 // and 9000 x 2048 x 64 the same; two rounds spread 6 % slower than one.  dQ, whose set-up is small, does not gain.
 constexpr int PDS_RAMP = 4;
+struct Work { int query, tiles; };
 template <int G, int RAMP>
-__device__ __forceinline__ int query_of(int i, int cnt, int K) {
-  const int groups = cnt / G, rest = cnt - groups * G;
-  if (i < rest) return cnt - 1 - i;
-  const int turn = (i - rest) / groups;
-  int p = i - rest - turn * groups;
-  if (RAMP > 0) p = spread_start(p, groups, 256, RAMP * K / G);
-  return (groups - 1 - p) * G + turn;
+__device__ __forceinline__ Work work_of(int i, int cnt, int K, const int* __restrict__ work, bool joint) {
+  if (G == 1 || !joint) return {cnt - 1 - (RAMP > 0 ? spread_start(i, cnt, 256, RAMP * K) : i), 0};
+  const int n = __builtin_amdgcn_readfirstlane(work[0]), first = __builtin_amdgcn_readfirstlane(work[1]);
+  if (i >= n) return {-1, 0};
+  const int place = RAMP == 0 ? i : i < first ? spread_start(i, first, 256, RAMP * K / G) : first + spread_start(i - first, n - first, 256, RAMP * K / G);
+  const int item = __builtin_amdgcn_readfirstlane(work[2 + place]);
+  return {item >> 8, item & 255};
 }
 
-// G: queries of a group that may be a joint unit (4 / HG), or 1.  units: padded slot counts of the groups' units, 0 where the queries
-// are by themselves.
+// G: queries of a group that may be a joint unit (4 / HG), or 1
 template <int HG, int G>
 __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ ids,
     const __bf16* __restrict__ out, const __bf16* __restrict__ dout, const float* __restrict__ lse,
     unsigned char* __restrict__ pds, const int* __restrict__ dst, unsigned char* __restrict__ rows, unsigned char* __restrict__ exps,
-    const int* __restrict__ units, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start, float sm_scale, int dummy_row) {
+    const int* __restrict__ work, const int* __restrict__ flags, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
+    float sm_scale, int dummy_row) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int ql = query_of<G, PDS_RAMP>((int)blockIdx.x, cnt, K);
+  const Work w = work_of<G, PDS_RAMP>((int)blockIdx.x, cnt, K, work, G > 1 && flags[1]);
+  const int ql = w.query;
+  if (G > 1 && ql < 0) return;
   // (two copies of every body: each copy meets the same barriers)
   if constexpr (HG == 4 || G > 1) {            // 128 heads: of the query or of a unit
-    const int slots = G > 1 ? units[ql / G] : K;
+    const int slots = G > 1 ? 32 * w.tiles : K;
     if (slots > 0) {
-      if (G > 1 && ql % G) return;
       const size_t hrow = (size_t)(q0 + ql) * H;
       unsigned char* unit = pds + (size_t)(ql / G) * group_pds;
       const __bf16 *q_rows = q + hrow * DQK, *out_rows = out + hrow * DV, *do_rows = dout + hrow * DV;
@@ -1224,20 +1229,21 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
 template <int HG, int G>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, const int* __restrict__ units, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
+    __bf16* __restrict__ dq, const int* __restrict__ work, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
     const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
     float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const RoleSlot rs = role_slot((int)blockIdx.x, cnt, (n_keys + RED_KEYS - 1) / RED_KEYS);
   if (rs.first) {
-    const int ql = query_of<G, 0>(rs.i, cnt, K);
+    const Work w = work_of<G, 0>(rs.i, cnt, K, work, G > 1 && dup_flag[1]);
+    const int ql = w.query;
+    if (G > 1 && ql < 0) return;
     const int* list = ids + (size_t)ql * K;
     __bf16* dq_rows = dq + (size_t)(q0 + ql) * H * DQK;
     const unsigned char* own = pds + (size_t)(ql / G) * group_pds;
     if constexpr (G > 1) {
-      const int slots = units[ql / G];
-      if (slots > 0) {
-        if (ql % G == 0) dq_body<3, 4, true>(kv, list, own, dq_rows, 128, Skv, slots, 0, dup_flag, smem);
+      if (w.tiles > 0) {
+        dq_body<3, 4, true>(kv, list, own, dq_rows, 128, Skv, 32 * w.tiles, 0, dup_flag, smem);
         return;
       }
       own += (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
@@ -1290,7 +1296,7 @@ struct BwdPlan {
   int chunk;            // queries per pass over the buffers, a multiple of G
   int G;                // queries of a group that may be a unit, or 1: from the whole call, so that a query's dQ does not depend on the chunks
   int W;                // bitmap words per key
-  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_bad, off_dst, off_sorted, off_pds, off_rows, off_exps, off_acc, total;
+  size_t off_bitmap, off_prefix, off_count, off_start, off_flag, off_units, off_work, off_bad, off_dst, off_sorted, off_pds, off_rows, off_exps, off_acc, total;
 };
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1315,6 +1321,7 @@ BwdPlan layout_plan(int S, int G, int chunk, int H, int Skv, int K) {
   p.off_start = o; o = align_up(o + (size_t)(Skv + 1) * 4);
   p.off_flag = o; o = align_up(o + 8);
   p.off_units = o; o = align_up(o + (G > 1 ? (size_t)((S + G - 1) / G) * 4 : 0));
+  p.off_work = o; o = align_up(o + (G > 1 ? ((size_t)chunk + 2) * 4 : 0));
   p.off_bad = o; o = align_up(o + (size_t)((Skv + 31) / 32) * 4);
   p.off_dst = o; o = align_up(o + (size_t)chunk * K * 4);
   p.off_sorted = o; o = align_up(o + (size_t)chunk * K * 4);
@@ -1341,16 +1348,19 @@ BwdPlan make_plan(int S, int H, int Skv, int K, size_t budget) {
   }
 }
 
-// What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, and how much more
-// where the last round of 256 is not full: half of what it lacks, spread over all.  Fitted to whole backward passes of 800 - 6000 queries
-// x 64 - 2048 slots with unions of 1.0 - 3.9 lists, all joint and all by themselves (328 pairs of times): what the prices pick takes 0.1 - 0.2 %
-// more than the better one in the mean, 5 % at most.  us, joint / by themselves, 64 heads: 1100 x 512 547 / 489 (union 24 tiles), 461 /
-// 571 (16), 2077 x 512 962 / 918 (24), 801 / 1031 (16); 32 heads: 1100 x 512 533 / 392 (44), 318 / 426 (23), 3072 x 512 1073 / 1024 (44),
-// 807 / 1076 (28).
+// What a unit and a query by itself take of a compute unit (scores and rows, dQ and its share of the sums), tenths of us, and, where the units
+// are up to three rounds of 256, how much more because the last round is not full: a part of what it lacks, spread over all (in more
+// rounds, queries of other lengths fill it).  Fitted to whole backward passes of 800 - 8000 queries of one length x 64 - 2048 slots with
+// unions of 1.0 - 3.9 lists, all joint and all by themselves (331 pairs of times): what the prices pick takes 0.2 (64 heads) and 0.1 % more
+// than the better one in the mean, 6 and 9 % at most.  us, joint / by themselves, 64 heads: 1100 x 512 547 / 489 (union 24 tiles), 461 / 571 (16),
+// 2077 x 512 962 / 918 (24), 801 / 1031 (16); 32 heads: 1100 x 512 533 / 392 (44), 318 / 426 (23), 3072 x 512 1073 / 1024 (44), 807 / 1076 (28),
+// 8000 x 256 1770 / 1612 (26).  Near the border the two cost the same, and calls of both kinds a few per cent more.
 order::UnitCost unit_cost(int HG, int S) {       // (HG 1 or 2)
-  auto waste = [](float rounds) { return rounds < 1.f ? 1.f / rounds : 1.f + 0.5f * (std::ceil(rounds) - rounds) / rounds; };
-  const float unit = waste((float)S / (256 * unit_queries(HG))), apart = waste((float)S / 256);
-  return {(int)((HG == 2 ? 280.f : 460.f) * unit), (int)(70.f * unit), (int)(180.f * apart), (int)((HG == 2 ? 50.f : 48.f) * apart)};
+  const float rounds = (float)S / (256 * unit_queries(HG)), part = rounds < 3.f ? (HG == 2 ? 0.3f : 0.4f) : 0.f;
+  auto waste = [part](float n) { return n < 1.f ? 1.f / n : 1.f + part * (std::ceil(n) - n) / n; };
+  const float unit = waste(rounds), apart = waste((float)S / 256);
+  return {(int)((HG == 2 ? 310.f : 420.f) * unit), (int)((HG == 2 ? 70.f : 78.f) * unit), (int)((HG == 2 ? 200.f : 180.f) * apart),
+          (int)((HG == 2 ? 50.f : 48.f) * apart)};
 }
 
 constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;
@@ -1415,6 +1425,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   const int G = p.G;
   const size_t group_pds = group_pds_bytes(HG, G, K);
   int* units = (int*)(ws + p.off_units);
+  int* work = (int*)(ws + p.off_work);
   unsigned* bad = (unsigned*)(ws + p.off_bad);
   const size_t reduce_lds = (size_t)RED_KEYS * RED_GROUPS * DQK * 4;
   size_t smem_dq = (size_t)3 * (TILE_BYTES + pds_kind_bytes(HG)) + ids_lds_bytes(K);
@@ -1450,18 +1461,18 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
     const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     DSA_MARK(0);
-    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S), (uint4*)exps);
+    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S), (uint4*)exps, work);
     else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);
     pds_rows_kernel<<<dim3(cnt), dim3(PDS_THREADS), smem_rows, st>>>(
-        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, exps, units + q0 / G, group_pds, q0, cnt, H, Skv, K,
-        q_start, sm_scale, p.chunk * K);
+        (const __bf16*)q, (const __bf16*)kv, sids, (const __bf16*)out, (const __bf16*)dout, lse, pds, dstp, rows, exps, work, dup_flag, group_pds, q0, cnt, H, Skv,
+        K, q_start, sm_scale, p.chunk * K);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, units + q0 / G, group_pds, q0, cnt, H, Skv,
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, work, group_pds, q0, cnt, H, Skv,
                                                                    K, q_start, dup_flag, rows, exps, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");

@@ -339,16 +339,17 @@ static __global__ __launch_bounds__(1024) void bm_prefix_kernel(const unsigned* 
   }
 }
 
-// start[key] = exclusive prefix sum of count (single workgroup; Skv is at most a few 10^5)
-static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __restrict__ count, int* __restrict__ start, int Skv) {
+// Exclusive prefix sums of value(k), k in [0, n), by one workgroup: put(k, sum, value) for each; returns the total.
+template <class Value, class Put>
+__device__ __forceinline__ int scan_block(int n_values, Value value, Put put) {
   __shared__ int wsum[16];
   __shared__ int carry_s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid == 0) carry_s = 0;
   __syncthreads();
-  for (int base = 0; base < Skv; base += 1024) {
+  for (int base = 0; base < n_values; base += 1024) {
     const int k = base + tid;
-    const int c = k < Skv ? count[k] : 0;
+    const int c = k < n_values ? value(k) : 0;
     int inc = c;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { int n = __shfl_up(inc, o, 64); if (lane >= o) inc += n; }
@@ -356,12 +357,45 @@ static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __rest
     __syncthreads();
     int before = carry_s;
     for (int w = 0; w < wave; w++) before += wsum[w];
-    if (k < Skv) start[k] = before + inc - c;
+    if (k < n_values) put(k, before + inc - c, c);
     __syncthreads();
     if (tid == 1023) carry_s = before + inc;
     __syncthreads();
   }
-  if (tid == 0) start[Skv] = carry_s;
+  return carry_s;
+}
+
+// What there is to do where some groups of G queries are units: work[2 ..] = first query << 8 | tiles of 32 slots for the units, query << 8
+// for the queries by themselves, both from the last query on; work[0] entries in all, work[1] those of the kind that comes first, which
+// is the rarer one (a few long queries behind everything else would end alone).  The two kinds apart, because a workgroup that does the
+// one and its neighbour that does the other displace each other's code from the instruction cache that they share.
+struct WorkList { const int* units; int cnt, G; int* work; };
+
+// start[key] = exclusive prefix sum of count (one workgroup; Skv is at most a few 10^5).  A second workgroup makes the work list.
+static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __restrict__ count, int* __restrict__ start, int Skv, WorkList list) {
+  if (blockIdx.x == 0) {
+    const int total = scan_block(Skv, [&](int k) { return count[k]; }, [&](int k, int sum, int) { start[k] = sum; });
+    if (threadIdx.x == 0) start[Skv] = total;
+  } else {
+    const int G = list.G, groups = (list.cnt + G - 1) / G;
+    auto tiles = [&](int k) { return list.units[groups - 1 - k] / 32; };
+    auto unit = [&](int k) { return tiles(k) ? 1 : 0; };
+    auto apart = [&](int k) { return tiles(k) ? 0 : min(G, list.cnt - (groups - 1 - k) * G); };
+    const int n_units = scan_block(groups, unit, [](int, int, int) {}), n_apart = list.cnt - G * n_units;
+    const bool units_first = n_units <= n_apart;
+    __syncthreads();
+    scan_block(groups, unit, [&](int k, int sum, int n) {
+      if (n) list.work[2 + (units_first ? 0 : n_apart) + sum] = ((groups - 1 - k) * G) << 8 | tiles(k);
+    });
+    __syncthreads();
+    scan_block(groups, apart, [&](int k, int sum, int n) {
+      for (int j = 0; j < n; j++) list.work[2 + (units_first ? n_units : 0) + sum + j] = ((groups - 1 - k) * G + n - 1 - j) << 8;
+    });
+    if (threadIdx.x == 0) {
+      list.work[0] = n_units + n_apart;
+      list.work[1] = min(n_units, n_apart);
+    }
+  }
 }
 
 // dst[ql][slot] = row of the pair in key-sorted order (-1 for invalid slots).  A workgroup takes the 32 queries of a word, or
@@ -435,13 +469,13 @@ inline bool sorted_list_fits(int Skv, int K) {
 inline void clear_flag(int* dup_flag, hipStream_t st) { zero_u32_kernel<<<dim3(1), dim3(64), 0, st>>>((unsigned*)dup_flag, 1); }
 inline void build_ranks(const int* lists, int row0, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
                         int* count, int* start, int* dst, int W, const int* units, int G, hipStream_t st, const int* flags = nullptr,
-                        uint4* marks = nullptr, size_t n_marks = 0) {
+                        uint4* marks = nullptr, size_t n_marks = 0, int* work = nullptr) {
   const int Wk = (Skv + 31) / 32;
   // every word of the bitmap is written (zeros beyond the last query), so no clearing pass is needed
   bm_transpose_kernel<<<dim3((W + 7) / 8, Wk), dim3(256), 0, st>>>(prefix, cnt, Skv, Wk, bitmap, W);
   const int clearing = (int)((n_marks + 4095) / 4096 < 512 ? (n_marks + 4095) / 4096 : 512);
   bm_prefix_kernel<<<dim3((Skv + 63) / 64 + clearing), dim3(1024), 0, st>>>(bitmap, prefix, count, Skv, W, flags, marks, n_marks);
-  key_scan_kernel<<<dim3(1), dim3(1024), 0, st>>>(count, start, Skv);
+  key_scan_kernel<<<dim3(units ? 2 : 1), dim3(1024), 0, st>>>(count, start, Skv, WorkList{units, cnt, G, work});
   const int range = Skv < RANK_KEYS ? Skv : RANK_KEYS;
   if (range * 8 > 48 * 1024) (void)dsa_reserve_lds((const void*)rank_kernel, (size_t)range * 8);
   const int words = (cnt + 31) / 32, parts = words >= 256 ? 1 : words >= 128 ? 2 : words >= 64 ? 4 : 8;
@@ -460,17 +494,17 @@ inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, 
 // LDS of qmap_unit_kernel
 inline size_t unit_lists_lds(int G, int Skv, int K) { return (size_t)unit_words((Skv + 31) / 32) * 4 * (G + G / 2) + (size_t)G * K * 4; }
 // build with the sorted lists, for groups of G (2 or 4) queries that may be units; 16 bytes of `marks` for every row (cnt K at most) are
-// cleared if there are any
+// cleared if there are any.  work: cnt + 2 ints
 inline void build_units(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix, int* count, int* start,
                         int* dst, int W, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
-                        UnitCost cost, uint4* marks) {
+                        UnitCost cost, uint4* marks, int* work) {
   const int Wk = (Skv + 31) / 32;
   const size_t lds = unit_lists_lds(G, Skv, K);
   const bool small = G * K <= 2048 && Wk <= 1024;      // (one round of ids for 256 threads, and then twice the workgroups on a compute unit)
   auto kernel = G == 2 ? (small ? qmap_unit_kernel<2, 256> : qmap_unit_kernel<2, 512>) : small ? qmap_unit_kernel<4, 256> : qmap_unit_kernel<4, 512>;
   if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)kernel, lds);
   kernel<<<dim3((cnt + G - 1) / G), dim3(small ? 256 : 512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
-  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st, dup_flag, marks, (size_t)cnt * K);
+  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st, dup_flag, marks, (size_t)cnt * K, work);
 }
 
 }  // namespace order
