@@ -16,8 +16,9 @@
 // nearly equally busy, so a wave interleaves the products of one head group with the sums of the one
 // before, half a group at a time.  Left to the waves of a SIMD to overlap each other's phases, with masked stores that
 // every tile waited for and the windows read one after the other by each wave: 8192 queries x 64 heads 505 000
-// cycles (MFMA busy 52 %, both ports at once 34 %) and 300 us; as it is now 455 000 (58 and 44 %) and 275, at
-// the 1.7 GHz that the part's power leaves both.  us, before and after: 1500 queries behind 6692 keys 95.5
+// cycles (MFMA busy 52 %, both ports at once 34 %) and, launched by itself again and again, 300 us; as it is now 455 000 (58 and
+// 44 %) and 275, at the 1.7 GHz that the part's power leaves both then.  Inside the pass of a prompt of 8192 257 and 247,
+// of 1500 behind 6692 keys 100 and 96.  us, by itself, before and after: 1500 queries behind 6692 keys 95.5
 // and 90, 3000 behind 5000 161 and 151, 2077 in four documents 18.2 and 16.5, 61 behind 20 000 18.0 and 16.2,
 // 48 unrelated windows of 7000 14.5 and 13.5; 32 heads, 5000 behind 500 82 and 80.5, 50 x 4 windows of 2500 8.5 and
 // 7.8.  HBM is far from binding (q8 / k8 are read once, logits written once).

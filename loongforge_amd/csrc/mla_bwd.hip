@@ -37,24 +37,24 @@ constexpr int PDS_THREADS = 512;
 // dQ follow one another in memory just like that.  The unit's slots are the union of the queries' keys, ascending; an entry carries
 // in bits 24 .. 27 which of the queries have it (UNIT_KEY masks the key), and P and dS are zero for the heads of the others.  One
 // pair row then stands for the key's pairs with all of them, and a key tile is gathered once.  order::qmap_unit_kernel decides
-// for every group; `units` holds its padded slot count, or 0 where the queries stay by themselves.
+// for every group; `units` holds its padded slot count, or 0 where the queries stay by themselves, and the work list (order::WorkList) what there
+// is to do.
 // Why: the backward of few heads is bound by its pair rows, 1152 bytes written and read whatever the heads, and neighbouring queries share
 // keys - a sliding window all but one, a selection of K out of L at least K / L of them.  The matrix work of the heads that have not
 // selected a slot is wasted, which the pipes have room for.  Whole backward, us, by themselves / joint / as the rule takes them (u:
-// union over sum of the lists): 3072 queries x 640 slots, window and compressed keys, 64 heads (u 0.54) 1219 / 937 / 933, 32 heads (0.27)
-// 1010 / 507 / 506; 2077 x 512 at random, 64 heads (0.73) 827 / 775 / 736, 32 heads (0.48) 683 / 512 / 494; 4000 x 512, 64 heads (0.83)
-// 1557 / 1619 / 1504, 32 heads (0.63) 1301 / 1178 / 1145; 8000 x 256, 64 heads (0.94) 1970 / 2189 / 1969; 3000 x 2048, 32 heads (0.28)
-// 2483 / 1105 / 1113.
+// union over sum of the lists): 3072 queries x 640 slots, window and compressed keys, 64 heads (u 0.54) 1138 / 904 / 903, 32 heads (0.27)
+// 959 / 519 / 517; 2077 x 512 at random, 64 heads (0.73) 740 / 751 / 736, 32 heads (0.48) 617 / 509 / 519; 4000 x 512, 64 heads (0.83)
+// 1482 / 1612 / 1486, 32 heads (0.63) 1229 / 1211 / 1128; 8000 x 256, 64 heads (0.94) 1889 / 2138 / 1831; 3000 x 2048, 32 heads (0.28)
+// 2338 / 1167 / 1170.
 //
 // A unit's row stands for 2 or 4 rows, so it is held in more bits than they: 11 instead of 8 significant ones, fp16 with a power of
 // two for every 64 columns (16 of the rotary part), chosen so that the largest of them lies in [2^14, 2^15).  Values down to 2^-29 of that
 // one have all 11 bits.  Its fp32 exponent is one of EXP_BYTES bytes per row: groups 0 - 7 the 64-column groups, 8 - 11 the
 // rotary ones; 0 marks a bf16 row, one of a query by itself: all of them are 0 before the rows are written, and where a call has no unit
 // they are neither cleared nor read (marked row by row instead: scores and rows of 3000 x 2048 of 32768 keys, no units, 2867 -> 3234 us).
-// In bf16 the rows' rounding error would be that of the rows it stands for only
-// where those are independent, and grows with what neighbouring queries have in common: rms over 256 queries x 256 of 288 slots, rows per query 1,
-// unit in bf16 / fp16: correlation 0 of Q and dO 1.00 / 0.13, 0.9 1.27 / 0.16 (64 heads) and 1.68 / 0.21 (32 heads), 0.99 1.36 / 0.17 and 1.88 /
-// 0.24.  What it takes, bf16 / fp16: scores and rows 521 / 562 us at 3072 queries x 640 slots x 64 heads and 276 / 297 at 2077 x 512 (maxima 22
+// In bf16 the rounding error would be that of the rows it stands for only where those are independent, and grows with what neighbouring
+// queries have in common.  Its rms, emulated, over 256 queries x 256 of 288 slots, with rows per query 1, with units in bf16 / fp16: correlation 0
+// of Q and dO 1.00 / 0.13; 0.9 1.27 / 0.16 (64 heads), 1.68 / 0.21 (32 heads); 0.99 1.36 / 0.17, 1.88 / 0.24.  What it takes, bf16 / fp16: scores and rows 521 / 562 us at 3072 queries x 640 slots x 64 heads and 276 / 297 at 2077 x 512 (maxima 22
 // of the 41, products with the power 10, the exponents' way through LDS 8), dQ and the sums 308 / 314 and 180 / 176.
 constexpr int unit_queries(int HG) { return 4 / HG; }
 constexpr int UNIT_SLOTS = 3072;             // what the lists in LDS behind the operands of 128 heads have room for
@@ -1002,9 +1002,9 @@ __device__ __forceinline__ void pds_rows_wide_body(
 // depends only on the segment, never on scheduling.  Pure streaming reads of 1152-byte rows, RED_FLIGHT to
 // twice that of them in flight per thread: a batch is loaded while the one before is summed, over the borders of keys, and
 // always as a whole.  (One batch of 16 at a time, with a key's last rows loaded one by one, each behind the sum of the one
-// before: with the dQ role beside it 1024 queries x 256 slots of 16 heads 60 us and 52 now, 2077 x 512 of 64 heads 205 and 181, 3072 x
-// 640 341 and 309; 8192 x 2048 of 128 heads, where the rows of a key fill many batches and the caches' gathers bound the
-// launch, 4.50 ms either way.  Batches of 12 and 16: the same within 3 %.)
+// before: with the dQ role beside it 1024 queries x 256 slots of 16 heads 60 us and 52 in batches of 8, 2077 x 512 of 64 heads 205 and
+// 181, 3072 x 640 341 and 309; 8192 x 2048 of 128 heads, where the rows of a key fill many batches and the caches' gathers bound the
+// launch, 4.50 ms either way.)
 // The rows are read once: a non-temporal load keeps them from displacing other lines in the caches
 // (a streaming read of this size runs at 6.8 TB/s with it against 6.1 TB/s without).
 typedef unsigned u32x4_nt __attribute__((ext_vector_type(4)));
