@@ -611,6 +611,30 @@ def test_backward_of_joint_queries_keeps_nonfinite_values_apart(gpu, H, S, where
 
 
 @pytest.mark.parametrize("H,S", [(64, 520), (32, 800)])
+@pytest.mark.parametrize("factor", [2.0 ** -12, 2.0 ** -20])
+def test_backward_of_joint_queries_with_columns_of_unlike_size(gpu, H, S, factor):
+    """Every other column of Q, dO and the keys smaller: those columns of dKV share their power of two with the large ones and are no
+    less accurate for it than one bf16 row per query makes them."""
+    from loongforge_amd import ops
+
+    K, skv = 128, 700
+    inp = O.make_mla_inputs(S, H, K, seed=S, skv=skv, q_start=skv)
+    inp.idx = _overlapping_ids(S, K, skv + S, 0, 0, 5)
+    for t in (inp.q, inp.kv, inp.dout):
+        t[..., 1::2] *= factor
+    q, kv, do, ids, sm = inp.q.to(gpu), inp.kv.to(gpu), inp.dout.to(gpu), inp.idx.to(gpu), inp.sm_scale
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, skv, sm)
+    _, dkv, G, joint = mla_bwd_with_groups(q, kv, out, do, ids, lse, skv, sm)
+    assert sum(joint) > len(joint) // 2
+    kw = dict(out=out.cpu(), lse=lse.cpu(), dtype=torch.float64)
+    _, ref = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, inp.idx, inp.dout, skv, sm, 512, **kw)
+    _, rows = O.sparse_mla_bwd_kernel_rounding(inp.q, inp.kv, inp.idx, inp.dout, skv, sm, 512, round_rows_bf16=True, **kw)
+    off, one_by_one = dkv.cpu().double() - ref, rows.to(torch.bfloat16).double() - ref
+    for c in (slice(0, None, 2), slice(1, None, 2)):
+        assert off[:, c].norm() <= one_by_one[:, c].norm()
+
+
+@pytest.mark.parametrize("H,S", [(64, 520), (32, 800)])
 def test_backward_of_joint_queries_with_a_column_that_overflows(gpu, H, S):
     """A sum over the heads beyond the range of fp32 in one column of a pair row leaves the row's other columns as they are."""
     from loongforge_amd import ops

@@ -322,3 +322,30 @@ def test_random_index_generator_is_causal_unique_and_padded():
     v = idx >= 0
     assert ((idx >= ks[:, None]) | ~v).all() and ((idx < ke[:, None]) | ~v).all()
     assert torch.equal(v.sum(-1), torch.minimum(ke - ks, torch.tensor(8)))
+
+
+def test_rows_of_joint_queries():
+    """The rows of a group worked as one are those of its queries, summed per key: without rounding the same dKV, with it within a step of
+    11 bits of every unit's row; :func:`round_unit_rows` against fp16 with the scale worked out value by value."""
+    S, H, K, skv, G = 38, 4, 16, 24, 4
+    g = torch.Generator().manual_seed(3)
+    q, do, kv = (torch.randn(*s, generator=g).to(torch.bfloat16) for s in ((S, H, 576), (S, H, 512), (skv, 576)))
+    idx = torch.stack([torch.randperm(skv, generator=g)[:K] for _ in range(S)]).int()
+    idx[5, 3:] = -1
+    joint = [i % 3 != 1 for i in range(S // G)] + [False]
+    kw = dict(q_start=skv, sm_scale=192 ** -0.5, dtype=torch.float64)
+    dq0, dkv0 = O.sparse_mla_bwd_kernel_rounding(q, kv, idx, do, **kw)
+    dq1, dkv1, _, most = O.sparse_mla_bwd_kernel_rounding(q, kv, idx, do, units=(G, joint), return_abs_sum=True, **kw)
+    assert torch.equal(dq0, dq1) and torch.allclose(dkv0, dkv1, rtol=1e-12, atol=1e-12)
+    _, dkv2 = O.sparse_mla_bwd_kernel_rounding(q, kv, idx, do, units=(G, [True] * (S // G) + [False]), round_rows_bf16=True, **kw)
+    _, rows = O.sparse_mla_bwd_kernel_rounding(q, kv, idx, do, round_rows_bf16=True, **kw)
+    assert 0 < (dkv2 - dkv0).norm() < 0.5 * (rows - dkv0).norm()
+    x = torch.randn(7, 576, generator=g, dtype=torch.float64) * torch.logspace(-9, 9, 7, dtype=torch.float64)[:, None]
+    x[2] = 0
+    y = O.round_unit_rows(x)
+    assert (y[2] == 0).all() and ((y - x).abs() <= 2.0 ** -11 * x.abs() + 2.0 ** -39 * x.abs().amax(1, keepdim=True)).all()
+    top = x[3, 512:528].abs().max().item()
+    k = -200
+    while 2.0 ** (k + 1) <= top:
+        k += 1
+    assert torch.equal(y[3, 512:528], (x[3, 512:528] * 2.0 ** (14 - k)).to(torch.float16).double() * 2.0 ** (k - 14))
