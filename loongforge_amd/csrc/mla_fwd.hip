@@ -142,7 +142,6 @@ __device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned
   *(uint4*)p = o[0];
   *(uint4*)(p + 16) = o[1];
 }
-
 // One 32-head block of a query relative to the true maximum of every head, all slots, one tile at a time: every
 // wave computes S^T of the block and sums its own value column tile dt.  For the marked blocks only: simple, and
 // light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.
@@ -250,8 +249,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   // ---- The ids and Q of the workgroup's heads, requested together so that both come back in one round trip to memory: Q as
   // 32-head blocks in the tiles' layout, where tiles 2 and 3 will lie.  The ids first, so that the list is made and the first tiles start
   // while Q arrives: 200 queries x 32 heads x 512 slots 27.5 -> 26.2 us.  A range of a query is short, its Q comes with it, and there Q
-  // goes first (61 queries x 64 heads in two ranges 24.9 us, 25.3 the other way).  (Q through LDS gains nothing in mla_fwd_wide_kernel:
-  // its queries come in rounds of 256 and their rows at the rate of the memory, 3.33 ms either way.) ----------
+  // goes first (61 queries x 64 heads in two ranges 24.9 us, 25.3 the other way). ----------
   const int* const ids = a.ids + (size_t)qi * K + k0;
   int first[8];
   if (!SPLIT) request_first_ids(ids, 0, KL, first);
@@ -542,11 +540,22 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
 // and the arriving tile) is close behind.  Forward 3.70 -> 3.33 ms, with the logits 4.39 -> 3.97; 1500 queries behind
 // a long prefix 809 -> 715 us.  Transfers spread over the products instead of first in the step: products
 // 2550 cycles (a transfer holds the wave, and the operand reads behind it); wave priorities: no difference.
+//
+// Set-up: the scores' waves bring the first 5 of 9 column groups of Q by whole lines through LDS, where tiles 1 and 2 and P will be, and
+// load the rest in the operands' layout, which takes 32 bytes of each of 32 rows and keeps the address path busy for four times as long a
+// byte; meanwhile the other waves make the list of tiles and start tile 0.  With all of Q in the operands' layout and the list made by all
+// waves, i.e. behind the issue of those loads, the first scores of a query started 16 800 cycles after it, now 11 600, of 198 000 in all at
+// 8192 queries x 2048 slots.  The forward there is held by the power it takes (2.40 ms with zeros for data, at full clock), so that
+// cycles saved are time saved in part: 3.41 -> 3.36 ms on one card, 3.51 -> 3.49 on another; 96 queries in ranges 72.3 -> 70.8 us, 1300 x
+// 512 with logits 239.0 -> 234.7, 600 x 128 heads 327 -> 323, 600 x 96 heads, whose fourth wave has nothing to load, 319 -> 308.  Output rows
+// by whole lines through LDS as well: no difference (one wave of a SIMD rounds 13 of its 16 blocks, which takes as long as the stores did).
 // ---------------------------------------------------------------------------------------------
 constexpr int WIDE_RING = 3;                 // tiles: the values of n, the scores of n + 1, the transfers of n + 2
 constexpr int P_BYTES = 4 * 2 * 1024;        // P of a tile, [32-head block][16 keys][lane] of 16 bytes
 constexpr int WIDE_LDS = WIDE_RING * TILE_BYTES + 2 * P_BYTES;
 constexpr int Q_ACC = 18;                    // k-steps of the Q slice in accumulation registers
+constexpr int Q_GROUPS = 5;                  // 128-byte groups of the rows of Q that pass through LDS, behind tile 0
+static_assert(TILE_BYTES + 4 * Q_GROUPS * GRP_BYTES <= WIDE_LDS, "Q lies where tiles 1 and 2 and P will be");
 
 template <bool SCORES, bool SPLIT, int POUT>
 __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsigned char* smem) {
@@ -562,21 +571,44 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
   float* const inv_s = (float*)pbuf;         // after the last tile
 
   const int* const ids = a.ids + (size_t)qi * K + k0;
-  int first[8];
-  if (!SPLIT) request_first_ids(ids, 0, KL, first);
-  __builtin_amdgcn_sched_barrier(0);
   const int h = 32 * w + r;                  // of the scores
   const bool head_ok = h < H;                // the same for all lanes of a wave
+  const unsigned row0 = (unsigned)(r * 128 + ((g ^ swz(r)) << 4));       // chunk 2 j + g of a group: row0 ^ 32 j
   bf16x8 qreg[SCORES ? KSTEPS : 1];
+  const unsigned q_lds = (unsigned)(uintptr_t)smem + TILE_BYTES + w * Q_GROUPS * GRP_BYTES;
+  int first[8];
   if constexpr (SCORES) {
-    const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + (head_ok ? h : 0)) * DQK) + g;
+    const unsigned char* const base = (const unsigned char*)uniform_ptr(a.q + ((size_t)qi * H + 32 * w) * DQK);
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < 4 && head_ok; i++) { // rows 8 i .. of the wave's heads
+      const int row = 8 * i + (lane >> 3);
+      const unsigned src = (unsigned)(row * (DQK * 2) + ((lane & 7) ^ swz(row)) * 16);
+#pragma unroll
+      for (int p = 0; p < Q_GROUPS; p++) dma16(__builtin_amdgcn_readfirstlane(q_lds + p * GRP_BYTES + i * 1024), src + p * 128, base);
+    }
+  } else {
+    request_first_ids(ids, 0, KL, first, threadIdx.x & 255);
+    stage_requested(first, ids, KL, a.Skv, a.q_start + qi, idx_s, tmask, threadIdx.x & 255);
   }
-  if (SPLIT) request_first_ids(ids, 0, KL, first);
-  const int ntiles = stage_from_first_ids(first, ids, 0, KL, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  __syncthreads();
+  if (!SCORES && w == 0) list_tiles(NT, tmask, tlist, tlist + NT);
+  __syncthreads();
+  const int ntiles = tlist[NT];
   if constexpr (SCORES) {
+    if (head_ok) {
+      const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * H + h) * DQK) + g;
+#pragma unroll
+      for (int ks = 4 * Q_GROUPS; ks < KSTEPS; ks++) qreg[ks] = qp[2 * ks];
+      __builtin_amdgcn_sched_barrier(0);
+      DSA_WAIT_VMCNT(KSTEPS - 4 * Q_GROUPS); // the wave's own rows are in LDS
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < 4 * Q_GROUPS; ks++)
+        qreg[ks] = *LDS_PTR(const bf16x8, (uintptr_t)(((q_lds + row0) ^ (32 * (ks & 3))) + (ks >> 2) * GRP_BYTES));
+    } else {                                 // 96 heads: nothing of this wave's scores is used
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++) qreg[ks] = bf16x8{};
+    }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
       if (ks < Q_ACC) asm volatile("" : "+a"(qreg[ks]));
@@ -584,7 +616,6 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
     }
   }
   if constexpr (SCORES) {
-    const unsigned row0 = (unsigned)(r * 128 + ((g ^ swz(r)) << 4));     // chunk 2 j + g of a group: row0 ^ 32 j
     const int tile0 = k0 / BI, p_skip = a.p_skip;
     // slots of tiles that are never visited still need their -inf in p_out
     // (p_out holds the slots from p_skip on: its rows are K - p_skip wide)
@@ -683,7 +714,7 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
 #pragma unroll
         for (int hb = 0; hb < 3; hb++) mfma_a_vv(o[hb], v[s], pr[s][hb]);
     };
-    __syncthreads();                         // tile 0 has landed
+    __syncthreads();                         // tile 0 has landed, Q is in registers
     int slot = -1;                           // of tile n
     if (ntiles > 0) {
       int tile_v = tlist[0];
@@ -748,13 +779,12 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
       asm volatile("" : "+v"(ov[hb]));
     }
     asm volatile("" : "+v"(o3));
-#pragma unroll
-    for (int n = 0; n < WIDE_RING; n++)
-      if (n < ntiles) gather(n, n);
-    if (ntiles >= 3) { DSA_WAIT_VMCNT(18); }
-    else if (ntiles == 2) { DSA_WAIT_VMCNT(9); }
-    else { DSA_WAIT_VMCNT(0); }
+    if (ntiles > 0) gather(0, 0);
+    DSA_WAIT_VMCNT(0);
     __syncthreads();
+#pragma unroll
+    for (int n = 1; n < WIDE_RING; n++)
+      if (n < ntiles) gather(n, n);
     if (ntiles > 0) {
       if (ntiles >= 3) { DSA_WAIT_VMCNT(9); }
       else { DSA_WAIT_VMCNT(0); }

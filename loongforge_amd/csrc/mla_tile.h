@@ -44,9 +44,47 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 
 // stage_ids in two steps: the first 2048 ids requested ahead of a query's operands.  Loads come back in order: ids requested behind the operands
 // arrive only after them, and the tiles, which wait for the ids, start on their way only then.
-__device__ __forceinline__ void request_first_ids(const int* __restrict__ ids, int qi, int K, int (&v)[8]) {
+__device__ __forceinline__ void request_first_ids(const int* __restrict__ ids, int qi, int K, int (&v)[8], int tid) {
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min((int)threadIdx.x + i * 256, K - 1)];
+  for (int i = 0; i < 8; i++) v[i] = ids[(size_t)qi * K + min(tid + i * 256, K - 1)];
+}
+__device__ __forceinline__ void request_first_ids(const int* __restrict__ ids, int qi, int K, int (&v)[8]) {
+  request_first_ids(ids, qi, K, v, (int)threadIdx.x);
+}
+
+// The rest of stage_ids in two steps with a barrier behind each, by four waves of a workgroup (tid: 0 .. 255 among them): ids and masks ...
+__device__ __forceinline__ void stage_requested(int (&v)[8], const int* __restrict__ ids, int K, int Skv, int qpos, int* idx_s,
+                                                unsigned* tmask, int tid) {
+  for (int t0 = tid; t0 < K; t0 += 8 * 256) {     // eight loads in flight per thread
+    if (t0 >= 8 * 256) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = ids[min(t0 + i * 256, K - 1)];
+    }
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int t = t0 + i * 256;            // 64 consecutive slots per wave: the masks of two tiles
+      const bool ok = (v[i] >= 0) && (v[i] < Skv) && (v[i] <= qpos);
+      const unsigned long long b = __ballot(ok);
+      if (t < K) {
+        idx_s[t] = ok ? v[i] : -1;
+        if ((tid & 63) == 0) { tmask[t / BI] = (unsigned)b; tmask[t / BI + 1] = (unsigned)(b >> 32); }
+      }
+    }
+  }
+}
+// ... and the list of tiles, by one wave
+__device__ __forceinline__ void list_tiles(int NT, const unsigned* tmask, int* tlist, int* ntile_s) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int t0 = 0; t0 < NT; t0 += 64) {
+    const int t = t0 + lane;
+    const bool nz = t < NT && tmask[t] != 0u;
+    const unsigned long long b = __ballot(nz);
+    if (nz) tlist[base + __popcll(b & ((1ull << lane) - 1ull))] = t;
+    base += __popcll(b);
+  }
+  if (lane == 0) *ntile_s = base;
 }
 
 // Stages the K ids of query qi in LDS (invalid slots become -1), builds the 32-bit validity mask
