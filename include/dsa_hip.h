@@ -200,6 +200,14 @@ int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const floa
                       const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps, int heads,
                       int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32, float* d_ln_w,
                       float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream);
+/* The same for queries that see at most `span` neighbouring keys each (0: not known): it decides how d_k is summed, not what it is. */
+size_t dsa_indexer_grads_span_workspace_bytes(int S, int Hi, int Sk, int K, int span);
+int dsa_indexer_grads_span(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
+                           const int32_t* ids, int S, int Hi, int Sk, int K, int span, const float* q_scale, float w_scale, int rotate,
+                           const void* cos, const void* sin, int tables_f32, int pairing, const int32_t* positions_q,
+                           const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps, int heads,
+                           int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32, float* d_ln_w,
+                           float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Windows of the causal queries [chunk_offset, chunk_offset + S) over packed sequences, cu[ncu] (i32, or i64 if cu_i64)

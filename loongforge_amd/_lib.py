@@ -31,6 +31,9 @@ SIGNATURES = {
     "dsa_indexer_grads_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "dsa_indexer_grads": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _f, _i, _vp, _vp, _i, _i, _vp, _vp, _i, _vp, _vp,
                                _f, _i, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _vp, _vp, _sz, _vp]),
+    "dsa_indexer_grads_span_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "dsa_indexer_grads_span": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _f, _i, _vp, _vp, _i, _i, _vp, _vp, _i, _vp,
+                                    _vp, _f, _i, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _vp, _vp, _sz, _vp]),
     "dsa_quant_padded_e4m3": (_i, [_vp, _i64, _i, _i, _i, _vp, _vp, _f, _i, _vp, _i, _f, _vp, _vp]),
     "dsa_rotary_tables": (_i, [_vp, _i, _i, _f, _i, _vp, _vp, _vp]),
     "dsa_rope_steps": (_i, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _f, _i, _i, _i64, _i, _i, _i, _vp]),

@@ -15,7 +15,7 @@ import torch
 from torch import Tensor
 
 from . import ops
-from .dsa_fused_kernels import _pad_to
+from .dsa_fused_kernels import _known_span, _pad_to
 from .megatron_compat import PackedSeqParams
 
 
@@ -170,6 +170,7 @@ class CSAIndexerKernelFunction(torch.autograd.Function):
                 topk_indices = global_ids
         ctx.softmax_scale = softmax_scale
         ctx.head = head
+        ctx.span = _known_span(packed_seq_params)
         ctx.in_dtypes = (index_q.dtype, index_k.dtype, weights.dtype)
         ctx.save_for_backward(q_fp8, k_fp8, q_scale, k_scale, weight_scaled, global_ids)
         ctx.mark_non_differentiable(topk_indices)
@@ -183,7 +184,7 @@ class CSAIndexerKernelFunction(torch.autograd.Function):
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, global_ids = ctx.saved_tensors
         # padding slots (id -1) are constants of the forward: their upstream gradient (often NaN) is dropped by the kernel
         d_q, d_k, d_weights, _, _ = ops.indexer_grads(grad_score, q_fp8, k_fp8, k_scale, weight_scaled, global_ids, q_scale,
-                                                      ctx.softmax_scale, ctx.head, 128, ctx.in_dtypes)
+                                                      ctx.softmax_scale, ctx.head, 128, ctx.in_dtypes, span=ctx.span)
         return d_q.unsqueeze(1), d_k.unsqueeze(1), d_weights.unsqueeze(1), None, None, None, None
 
 

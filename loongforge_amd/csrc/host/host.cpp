@@ -350,7 +350,7 @@ py::object indexer_bwd(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, c
 py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, const Tensor& k_scale_, const Tensor& q_w_, const Tensor& ids_,
                         const Tensor& q_scale_, double w_scale, bool rotate, const OptTensor& cos_, const OptTensor& sin_, int64_t pairing,
                         const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& k_in, const OptTensor& ln_w_,
-                        double ln_eps, int64_t heads, int64_t dim, at::ScalarType q_type, at::ScalarType k_type, at::ScalarType w_type) {
+                        double ln_eps, int64_t heads, int64_t dim, int64_t span, at::ScalarType q_type, at::ScalarType k_type, at::ScalarType w_type) {
   need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_, q_scale_, cos_, sin_, positions_q, positions_k, k_in, ln_w_);
   const int64_t S = q8_.size(0), Hi = q8_.size(1), Sk = k8_.size(0);
   REQUIRE(ids_.dim() == 2 && g_.sizes() == ids_.sizes() && ids_.size(0) == S && q_scale_.numel() == S * Hi,
@@ -375,12 +375,12 @@ py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, 
   Call call(q8);
   auto out_type = [](at::ScalarType t) { return t == at::kBFloat16 ? t : at::kFloat; };
   Tensor d_q = make({S, heads, dim}, out_type(q_type), q8), d_k = make({Sk, dim}, out_type(k_type), q8), d_w = make({S, heads}, out_type(w_type), q8);
-  const size_t nbytes = dsa_indexer_grads_workspace_bytes((int)S, (int)Hi, (int)Sk, (int)ids.size(1));
+  const size_t nbytes = dsa_indexer_grads_span_workspace_bytes((int)S, (int)Hi, (int)Sk, (int)ids.size(1), (int)span);
   Tensor ws = make({(int64_t)std::max<size_t>(nbytes, 256)}, at::kByte, q8);
   auto is_f32 = [](const Tensor& t) { return (int)(t.scalar_type() == at::kFloat); };
-  run("dsa_indexer_grads", dsa_indexer_grads, (const float*)g.const_data_ptr(), q8.const_data_ptr(), k8.const_data_ptr(),
+  run("dsa_indexer_grads", dsa_indexer_grads_span, (const float*)g.const_data_ptr(), q8.const_data_ptr(), k8.const_data_ptr(),
       (const float*)k_scale.const_data_ptr(), (const float*)q_w.const_data_ptr(), (const int32_t*)ids.const_data_ptr(), (int)S, (int)Hi, (int)Sk,
-      (int)ids.size(1), (const float*)q_scale.const_data_ptr(), (float)w_scale, (int)rotate, ptr(cos), ptr(sin), cos ? is_f32(*cos) : 0,
+      (int)ids.size(1), (int)span, (const float*)q_scale.const_data_ptr(), (float)w_scale, (int)rotate, ptr(cos), ptr(sin), cos ? is_f32(*cos) : 0,
       (int)pairing, (const int32_t*)ptr(pos_q), (const int32_t*)ptr(pos_k), (int)batch, ptr(k_in), (const float*)ptr(ln_w), (float)ln_eps,
       (int)heads, (int)dim, d_q.data_ptr(), is_f32(d_q), d_k.data_ptr(), is_f32(d_k), d_w.data_ptr(), is_f32(d_w),
       k_in ? (float*)d_ln_w.data_ptr() : nullptr, k_in ? (float*)d_ln_b.data_ptr() : nullptr, ws.data_ptr(), nbytes, call.stream);

@@ -27,11 +27,12 @@
 // reads and 40 writes per wave and tile.)  Rows written in slot order instead of scattered: the same; non-temporal: 2.9 ms.
 #include "dsa_common.h"
 #include "order.h"
+#include <type_traits>
 
 namespace {
 
 constexpr int D = 128;
-constexpr int TK = 128;                 // slots per tile
+constexpr int TK = 128;                 // slots per tile of the waves that share them (a list's length is a multiple of it)
 constexpr int WAVE_BYTES = 32 * D;      // fp8 key rows of a wave's share of a tile
 constexpr int THREADS = 512;
 constexpr int RED_STRIDE = 132;         // floats per head row of the cross-wave reduction buffers
@@ -61,6 +62,39 @@ template <typename T>
 __device__ __forceinline__ T lds_read(unsigned addr) { return *(__attribute__((address_space(3))) const T*)(uintptr_t)addr; }
 __device__ __forceinline__ i32x2 read_tr8(unsigned addr) {
   return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) i32x2*)(uintptr_t)addr);
+}
+
+// The (q_w Q)^T operand of d-tile dt and k-step kk: lane = d row 32 dt + r, heads 16 kk + 4 g .. and 16 kk + 8 + 4 g .. (the order in
+// which an accumulator of scores holds them); the query's fp8 rows lie in LDS with their chunks at c ^ slot_xor(row).
+__device__ __forceinline__ uint4 weighted_query(unsigned q_lds, const float* w_s, int lane, int dt, int kk) {
+  const int g = lane >> 5, blk = lane >> 4, ii = lane & 15;
+  const f32x4 w0 = *(const f32x4*)(w_s + 16 * kk + 4 * g), w1 = *(const f32x4*)(w_s + 16 * kk + 8 + 4 * g);
+  const int row = 16 * kk + 8 * (ii >> 3) + 4 * g + ((ii >> 1) & 3);
+  const bf16x8 x = fp8_to_bf16(read_tr8(q_lds + row * D + (((2 * dt + (blk & 1)) ^ slot_xor(row)) << 4) + 8 * (ii & 1)));
+  unsigned pk[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const f32x4& w = e < 2 ? w0 : w1;
+    pk[e] = cvt_pk_bf16((float)x[2 * e] * w[(2 * e) & 3], (float)x[2 * e + 1] * w[(2 * e + 1) & 3]);
+  }
+  return make_uint4(pk[0], pk[1], pk[2], pk[3]);
+}
+// The mask [r > 0] of an accumulator of scores (times 2^20: at least 4 where positive, r is a multiple of 2^-18) as the bf16 operand of
+// the next product, each entry 0 or 2^-7: the half-precision 1.0 read as bf16, a conversion and a packed clamp for two.
+template <int NHT>
+__device__ __forceinline__ void score_masks(const f32x16 (&acc)[NHT], bf16x8 (&mk)[2 * NHT]) {
+#pragma unroll
+  for (int t = 0; t < NHT; t++)
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      unsigned pk[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        pk[e] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(acc[t][8 * s + 2 * e], acc[t][8 * s + 2 * e + 1]));
+        asm("v_pk_max_f16 %0, %0, %0 clamp" : "+v"(pk[e]));
+      }
+      mk[2 * t + s] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+    }
 }
 
 // ---- what follows the sums: from payload gradients to gradients of the projections' outputs ------------------
@@ -165,7 +199,7 @@ struct BwdArgs {
   const int* ids;
   const int* dst;
   unsigned short* rows;
-  int q0, cnt, Sk, K, dummy_row;
+  int q0, cnt, Sk, K, dummy_row;         // (dst, rows, dummy_row: only where the workgroups write rows)
   // plain payload gradients (q_scale null) ...
   float* d_q8;                           // [S, HI, 128]
   float* d_qw;                           // [S, HI]
@@ -186,34 +220,39 @@ int bwd_stages(int K) { return K <= 2048 ? 3 : 2; }
 // What a workgroup needs to the end lies behind both the loop's arrays and the reduction buffers that take their place: weights [64],
 // scales [64], cosines and sines [2][64], last slot.
 constexpr size_t KEPT_BYTES = 4 * 64 * 4 + 64;
-__host__ __device__ constexpr size_t kept_offset(int HI, int stages, int K) {
-  const size_t loop = (size_t)stages * 8 * WAVE_BYTES + (size_t)HI * D + (size_t)K * 16;
-  const size_t red = (size_t)4 * HI * RED_STRIDE * 4 + 4 * 64 * 4;
+__host__ __device__ constexpr size_t kept_offset(int HI, int stages, int K, bool rows) {
+  const size_t loop = (size_t)stages * (rows ? 8 : 4) * WAVE_BYTES + (size_t)HI * D + (size_t)K * (rows ? 16 : 12);
+  const size_t red = (size_t)4 * (rows ? HI : 32) * RED_STRIDE * 4 + 4 * 64 * 4;
   return loop > red ? loop : red;
 }
-size_t bwd_lds_bytes(int HI, int K) { return kept_offset(HI, bwd_stages(K), K) + KEPT_BYTES; }
+size_t bwd_lds_bytes(int HI, int stages, int K, bool rows) { return kept_offset(HI, stages, K, rows) + KEPT_BYTES; }
 
 // The waves share nothing inside the loop: each brings the 32 key rows of its slots into a ring of its own and there is no
 // barrier, so that one wave's vector work runs under the matrix work of the other wave of its SIMD.  The loop is bound by
 // vector issue, hence one role per wave (both products in every wave, a half of d or of the heads each, doubles the masks
 // and the operand conversions: 1.5 ms at the size above), a mask of 2^-7 (the half-precision 1.0 read as bf16, made by a
 // conversion and a packed clamp for two elements) and slot offsets in the instructions.
-template <int NHT, int STAGES>   // head tiles of 32
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void indexer_bwd_kernel(const BwdArgs A) {
+//
+// ROWS = false: d_k8 is the work of the kernels by key tiles (below).  Four waves sum d_q8 then, in half of a compute unit's LDS (two
+// tiles in a ring): one query's set-up and final sums pass under another's loop.
+template <int NHT, int STAGES, bool ROWS>   // head tiles of 32
+__global__ __launch_bounds__(ROWS ? THREADS : THREADS / 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void indexer_bwd_kernel(const BwdArgs A) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int HI = 32 * NHT;
+  constexpr int NT = ROWS ? THREADS : THREADS / 2, WAVES = NT / 64;
+  constexpr int PT = 4 * THREADS / NT;              // slots per thread and round trip
   // [8 waves][STAGES][WAVE_BYTES] fp8 key rows | q8 [HI][128] | a_s [K] f32 | ahl_s [K / 4][4 hi, 4 lo] bf16 | idx_s [K] | dst_s [K] ||
   // w_s [64] | scale_s [64] | cs_s [2][64] | last_s
-  unsigned char* qs = smem + 8 * STAGES * WAVE_BYTES;
+  unsigned char* qs = smem + WAVES * STAGES * WAVE_BYTES;
   const int K = A.K;
   float* a_s = (float*)(qs + HI * D);
   unsigned short* ahl_s = (unsigned short*)(a_s + K);
   int* idx_s = (int*)(ahl_s + 2 * K);
   int* dst_s = idx_s + K;
-  float* w_s = (float*)(smem + kept_offset(HI, STAGES, K));
+  float* w_s = (float*)(smem + kept_offset(HI, STAGES, K, ROWS));
   float *scale_s = w_s + 64, *cs_s = w_s + 128;
   int* last_s = (int*)(w_s + 256);
-  float* dw_red = (float*)smem;                     // [4][64], then red [4][HI][RED_STRIDE], reuse the front at the end
+  float* dw_red = (float*)smem;                     // [4][64], then red [4][HI or 32][RED_STRIDE], reuse the front at the end
   float* red = dw_red + 4 * 64;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -228,16 +267,16 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const unsigned char* qrow = A.q8 + (size_t)qi * HI * D;
   const int* ids = A.ids + (size_t)qi * K;
   const float* gsc = A.gsc + (size_t)qi * K;
-  const int* dst = A.dst + (size_t)ql * K;
-  int v[4], d[4];
-  float gv[4];
-  auto request_slots = [&](int t0) {                // four slots per thread with all their loads in flight
+  const int* dst = ROWS ? A.dst + (size_t)ql * K : nullptr;
+  int v[PT], d[PT];
+  float gv[PT];
+  auto request_slots = [&](int t0) {                // a thread's slots with all their loads in flight
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int t = min(t0 + i * THREADS, K - 1);
+    for (int i = 0; i < PT; i++) {
+      const int t = min(t0 + i * NT, K - 1);
       v[i] = ids[t];
       gv[i] = gsc[t];
-      d[i] = dst[t];
+      if (ROWS) d[i] = dst[t];
     }
   };
   request_slots(tid);
@@ -246,19 +285,22 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const bool rotary = A.q_scale != nullptr && A.fin.pairing >= 0;
   const long pos = !rotary ? 0 : A.pos_q ? A.pos_q[qi] : qi / A.fin.batch;
   const uint4 q_in = *(const uint4*)(qrow + min(tid, HI * 8 - 1) * 16);
+  const uint4 q_in2 = *(const uint4*)(qrow + min(tid + NT, HI * 8 - 1) * 16);
+  // Where the key of a slot that counts for nothing is read (its factor is 0): the first slot's key, which the query has selected
+  const int spare = (unsigned)ids[0] < (unsigned)A.Sk ? ids[0] : 0;
   __builtin_amdgcn_sched_barrier(0);
   int last = -1;
   for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {   // ids first: the transfers of key rows want nothing else
     if (t0 != tid) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = ids[min(t0 + i * THREADS, K - 1)];
+      for (int i = 0; i < PT; i++) v[i] = ids[min(t0 + i * NT, K - 1)];
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int t = t0 + i * THREADS;
+    for (int i = 0; i < PT; i++) {
+      const int t = t0 + i * NT;
       const bool ok = v[i] >= 0 && v[i] < A.Sk;
       if (t < K) {
-        idx_s[t] = ok ? v[i] : 0;
+        idx_s[t] = ok ? v[i] : spare;
         if (ok) last = t;
       }
     }
@@ -271,7 +313,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     w_s[tid] = w_in;
     scale_s[tid] = scale_in;
   }
-  if (tid < HI * 8) *(uint4*)(qs + (tid >> 3) * D + (((tid & 7) ^ slot_xor(tid >> 3)) << 4)) = q_in;
+  auto keep_query = [&](int c, const uint4& q) {
+    if (c < HI * 8) *(uint4*)(qs + (c >> 3) * D + (((c & 7) ^ slot_xor(c >> 3)) << 4)) = q;
+  };
+  keep_query(tid, q_in);
+  if (NT < HI * 8) keep_query(tid + NT, q_in2);
   DSA_WAIT_VMCNT(0);                                // every load so far: what is in flight below are the transfers and the scales
   __syncthreads();
   const int ntile = (*last_s + TK) / TK;            // tiles behind the last valid slot have nothing to add
@@ -303,12 +349,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const float cs_in = rotary && tid < 128 ? table_entry(tid < 64 ? A.fin.cos_t : A.fin.sin_t, A.fin.cs_f32, pos * 64 + (tid & 63)) : 0.f;
   for (int t0 = tid; t0 < K; t0 += 4 * THREADS) {
     if (K > 4 * THREADS) request_slots(t0);
-    float kv[4];
+    float kv[PT];
 #pragma unroll
-    for (int i = 0; i < 4; i++) kv[i] = A.k_scale[(v[i] >= 0 && v[i] < A.Sk) ? v[i] : 0];
+    for (int i = 0; i < PT; i++) kv[i] = A.k_scale[(v[i] >= 0 && v[i] < A.Sk) ? v[i] : 0];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int t = t0 + i * THREADS;
+    for (int i = 0; i < PT; i++) {
+      const int t = t0 + i * NT;
       if (t < K) {
         const bool ok = v[i] >= 0 && v[i] < A.Sk;
         const float a = ok ? gv[i] * kv[i] : 0.f;
@@ -316,7 +362,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         a_s[t] = a;
         ahl_s[(t >> 2) * 8 + (t & 3)] = hi;
         ahl_s[(t >> 2) * 8 + 4 + (t & 3)] = f32_to_bf16_bits(a - bf16_bits_to_f32(hi));
-        dst_s[t] = (ok && d[i] >= 0) ? d[i] : A.dummy_row;
+        if (ROWS) dst_s[t] = (ok && d[i] >= 0) ? d[i] : A.dummy_row;
       }
     }
   }
@@ -345,26 +391,50 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   };
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-  if (wave < 4) {
+  auto leave_sums = [&](int head, const f32x16 (&acc)[4]) {       // this wave's sums of 32 heads, to rows head .. of its part of red
+    constexpr int PER = ROWS ? HI : 32;
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) {
+      float* rp = red + ((size_t)kg * PER + head + r) * RED_STRIDE + 32 * dt + 4 * g;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        *(f32x4*)(rp + 8 * j) = f32x4{acc[dt][4 * j], acc[dt][4 * j + 1], acc[dt][4 * j + 2], acc[dt][4 * j + 3]};
+    }
+  };
+  // ---- sums of 32 heads over the four slot groups, in a fixed order, and what follows them ------------------
+  const int sub = tid & 15;
+  auto finish_heads = [&](int it, int head) {
+    constexpr int PER = ROWS ? HI : 32;
+#pragma unroll
+    for (int hh = 0; hh < 32; hh += NT / 16) {
+      const int h = 32 * it + hh + (tid >> 4);
+      float v[8];
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        f32x4 p[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) p[k] = *(const f32x4*)(red + ((size_t)k * PER + head + hh + (tid >> 4)) * RED_STRIDE + 8 * sub + 4 * x);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[4 * x + e] = ((p[0][e] + p[1][e]) + (p[2][e] + p[3][e])) * w_s[h];
+      }
+      if (A.q_scale == nullptr) {
+        store_row(v, A.d_q8, 1, (size_t)qi * HI + h, D, sub);
+      } else {
+        finish_row(v, sub, scale_s[h], A.fin, nullptr, qi, cs_s);
+        if (h < A.heads) store_row(v, A.d_q, A.q_f32, (size_t)qi * A.heads + h, A.dim, sub);
+      }
+    }
+  };
+
+  if (ROWS && wave < 4) {
     // ======== rows of d_k8 ============================================================================
     // (q_w Q)^T operands: lane = d row 32 dt + r, 8 heads of k-step kk = 2 t + s in accumulator order
     bf16x8 qt[4][2 * NHT];
 #pragma unroll
-    for (int kk = 0; kk < 2 * NHT; kk++) {
-      const f32x4 w0 = *(const f32x4*)(w_s + 16 * kk + 4 * g), w1 = *(const f32x4*)(w_s + 16 * kk + 8 + 4 * g);
-      const int row = 16 * kk + tr_row;
+    for (int kk = 0; kk < 2 * NHT; kk++)
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) {
-        const bf16x8 x = fp8_to_bf16(read_tr8(lds0 + (unsigned)(qs - smem) + row * D + (((2 * dt + (blk & 1)) ^ slot_xor(row)) << 4) + 8 * (ii & 1)));
-        unsigned pk[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const f32x4& w = e < 2 ? w0 : w1;
-          pk[e] = cvt_pk_bf16((float)x[2 * e] * w[(2 * e) & 3], (float)x[2 * e + 1] * w[(2 * e + 1) & 3]);
-        }
-        qt[dt][kk] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
-      }
-    }
+      for (int dt = 0; dt < 4; dt++)
+        qt[dt][kk] = __builtin_bit_cast(bf16x8, weighted_query(lds0 + (unsigned)(qs - smem), w_s, lane, dt, kk));
     query_rows();
     unsigned short* const rows = A.rows + 8 * g;
     const unsigned slot_off = (unsigned)(32 * kg + r) * 4;
@@ -400,18 +470,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const float a_n = a;
         unsigned short* const rowp = rows + (size_t)row * D;
         bf16x8 mk[2 * NHT];
-#pragma unroll
-        for (int t = 0; t < NHT; t++)
-#pragma unroll
-          for (int s = 0; s < 2; s++) {
-            unsigned pk[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              pk[e] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(acc[t][8 * s + 2 * e], acc[t][8 * s + 2 * e + 1]));
-              asm("v_pk_max_f16 %0, %0, %0 clamp" : "+v"(pk[e]));
-            }
-            mk[2 * t + s] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
-          }
+        score_masks<NHT>(acc, mk);
         f32x16 racc[2];
 #pragma unroll
         for (int dt = 0; dt < 5; dt++) {       // the products of a d-tile run while the one before it is rounded and stored
@@ -546,37 +605,25 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int t = 0; t < NHT; t++) {
       const float v = dw[t] + __shfl_xor(dw[t], 32, 64);
       if (g == 0) dw_red[kg * 64 + 32 * t + r] = v;
+    }
+    if (ROWS) {
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) {
-        float* rp = red + ((size_t)kg * HI + 32 * t + r) * RED_STRIDE + 32 * dt + 4 * g;
+      for (int t = 0; t < NHT; t++) leave_sums(32 * t, dq_acc[t]);
+    } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          *(f32x4*)(rp + 8 * j) = f32x4{dq_acc[t][dt][4 * j], dq_acc[t][dt][4 * j + 1], dq_acc[t][dt][4 * j + 2], dq_acc[t][dt][4 * j + 3]};
+      for (int t = 0; t < NHT; t++) {
+        if (t) __syncthreads();
+        leave_sums(0, dq_acc[t]);
+        __syncthreads();
+        finish_heads(t, 0);
       }
     }
   }
 
-  // ---- sums over the four slot groups, in a fixed order ----------------------------------------------
-  __syncthreads();
-  const int sub = tid & 15;
+  if (ROWS) {
+    __syncthreads();
 #pragma unroll
-  for (int it = 0; it < NHT; it++) {
-    const int h = 32 * it + (tid >> 4);
-    float v[8];
-#pragma unroll
-    for (int x = 0; x < 2; x++) {
-      f32x4 p[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) p[k] = *(const f32x4*)(red + ((size_t)k * HI + h) * RED_STRIDE + 8 * sub + 4 * x);
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[4 * x + e] = ((p[0][e] + p[1][e]) + (p[2][e] + p[3][e])) * w_s[h];
-    }
-    if (A.q_scale == nullptr) {
-      store_row(v, A.d_q8, 1, (size_t)qi * HI + h, D, sub);
-    } else {
-      finish_row(v, sub, scale_s[h], A.fin, nullptr, qi, cs_s);
-      if (h < A.heads) store_row(v, A.d_q, A.q_f32, (size_t)qi * A.heads + h, A.dim, sub);
-    }
+    for (int it = 0; it < NHT; it++) finish_heads(it, 32 * it);
   }
   if (tid < HI) {
     const float s = (dw_red[tid] + dw_red[64 + tid]) + (dw_red[128 + tid] + dw_red[192 + tid]);
@@ -636,6 +683,341 @@ __global__ __launch_bounds__(16 * RED_GROUPS) void indexer_reduce_kernel(const u
     if (accumulate) s += *p;
     if (*dup_flag) s = __builtin_nanf("");       // a query row held a repeated id: no sum that misses a term
     *p = s;
+  }
+}
+
+// ======== d_k8 by key tiles ==========================================================================
+// Where a good part of the keys that the queries see is selected, a row per pair through memory (256 bytes written and read, the
+// key-sorted order, the sums) costs more than the products with every key of the range: a workgroup then owns 256 keys and a
+// chunk of queries, its sums stay in registers, and the pair factors a (0 for a pair that is not selected) come from a dense array.
+//   scatter   per query: the factors of its 256-key tiles that hold a selected key, which tiles these are, and the operands of both
+//             products in the layout of the matrix instructions
+//   keys      per (chunk of queries, 256 keys): d_k8 over the chunk's queries that touch the tile, in ascending order
+//   reduce    per key: the chunks' sums in a fixed order
+// The sums are fp32 throughout (a row of a pair is not rounded to bf16).
+constexpr int KT = 256;                 // keys per tile
+constexpr int PIECE_TILES = 16;         // tiles whose factors are scattered in LDS at a time; their marks are one word
+constexpr unsigned UNSELECTED = 0x80000000u;       // -0: adds nothing, and is told from a selected pair's factor 0
+constexpr int QUERY_BAD = 1, QUERY_DUP = 2;
+
+__host__ __device__ constexpr int operand_bytes(int NHT) { return NHT * 12 * 1024; }   // fp8 rows 4 KB, (q_w Q)^T 8 KB per head tile
+
+struct DenseArgs {
+  const float* gsc;
+  const unsigned char* q8;
+  const unsigned char* k8;
+  const float* k_scale;
+  const float* q_w;
+  const int* ids;
+  int q0, cnt, Sk, K;
+  int tiles, words, chunk, chunks;      // key tiles, words of marks per query, queries per chunk
+  float* factors;                       // [cnt][tiles][KT], written where marked
+  unsigned* marks;                      // [cnt][words]
+  int* state;                           // [cnt]
+  unsigned char* ops;                   // [cnt][operand_bytes]
+  float* part;                          // [chunks][tiles][KT][D], written where used
+  int* used;                            // [chunks][tiles]: queries summed; negative: a query of the chunk repeats an id
+};
+
+// Bound by what it writes: at 8192 queries x 2048 slots x 64 heads 200 MB of operands and up to 268 MB of factors.
+template <int NHT>
+__global__ __launch_bounds__(256) void indexer_scatter_kernel(const DenseArgs A) {
+  constexpr int HI = 32 * NHT, SLOTS = 16;          // K <= 4096
+  constexpr unsigned EMPTY = 0xffffffffu;
+  __shared__ __attribute__((aligned(16))) unsigned row[PIECE_TILES * KT];
+  __shared__ __attribute__((aligned(1024))) unsigned char qs[HI * D];
+  __shared__ __attribute__((aligned(16))) float w_s[HI];
+  __shared__ int lo_s, hi_s, flags_s;
+  __shared__ unsigned marks_s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ql = blockIdx.x, qi = A.q0 + ql;
+  if (tid == 0) { lo_s = 0x7fffffff; hi_s = -1; flags_s = 0; marks_s = 0; }
+  const int* ids = A.ids + (size_t)qi * A.K;
+  const float* gsc = A.gsc + (size_t)qi * A.K;
+  int id[SLOTS];
+  unsigned a[SLOTS];
+#pragma unroll
+  for (int i = 0; i < SLOTS; i++) {
+    const int t = tid + 256 * i;
+    id[i] = t < A.K ? ids[t] : -1;
+    a[i] = t < A.K ? __builtin_bit_cast(unsigned, gsc[t]) : 0u;
+  }
+  for (int c = tid; c < HI * 8; c += 256) *(uint4*)(qs + (c >> 3) * D + (((c & 7) ^ slot_xor(c >> 3)) << 4)) = *(const uint4*)(A.q8 + (size_t)qi * HI * D + c * 16);
+  if (tid < HI) w_s[tid] = A.q_w[(size_t)qi * HI + tid];
+  int lo = 0x7fffffff, hi = -1;
+#pragma unroll
+  for (int i = 0; i < SLOTS; i++) {
+    if (id[i] >= A.Sk) id[i] = -1;
+    if (id[i] >= 0) {
+      float f = __builtin_bit_cast(float, a[i]) * A.k_scale[id[i]];
+      a[i] = __builtin_bit_cast(unsigned, f);
+      if (a[i] == EMPTY) a[i] = 0x7fc00000u;        // a NaN all the same
+      if (a[i] == UNSELECTED) a[i] = 0u;
+      lo = min(lo, id[i]);
+      hi = max(hi, id[i]);
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  __syncthreads();
+  if (lane == 0) {
+    atomicMin(&lo_s, lo);
+    atomicMax(&hi_s, hi);
+  }
+  // ---- operands ------------------------------------------------------------------------------------
+  unsigned char* ops = A.ops + (size_t)ql * operand_bytes(NHT) + lane * 16;
+  const unsigned q_lds = (unsigned)(uintptr_t)qs;
+  const int r = lane & 31, g = lane >> 5;
+  for (int b = wave; b < 4 * NHT; b += 4) {         // block (t, s, x): bytes [64 s + 32 g + 16 x, + 16) of head 32 t + r
+    const int t = b >> 2, s = (b >> 1) & 1, x = b & 1;
+    *(uint4*)(ops + b * 1024) = *(const uint4*)(qs + (32 * t + r) * D + (((4 * s + 2 * g + x) ^ slot_xor(r)) << 4));
+  }
+  bool bad = false;
+  for (int b = wave; b < 8 * NHT; b += 4) {         // block (dt, kk)
+    const uint4 v = weighted_query(q_lds, w_s, lane, b / (2 * NHT), b % (2 * NHT));
+    const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) bad |= (w[e] & 0x7f80u) == 0x7f80u || (w[e] & 0x7f800000u) == 0x7f800000u;
+    *(uint4*)(ops + (4 * NHT + b) * 1024) = v;
+  }
+  // ---- factors, a piece of the keys at a time ----------------------------------------------------------
+  __syncthreads();
+  const int first = hi_s < 0 ? A.words : lo_s / (PIECE_TILES * KT), behind = hi_s < 0 ? 0 : hi_s / (PIECE_TILES * KT) + 1;
+  bool dup = false;
+  for (int p = 0; p < A.words; p++) {
+    if (p < first || p >= behind) {
+      if (tid == 0) A.marks[(size_t)ql * A.words + p] = 0u;
+      continue;
+    }
+    const int nt = min(PIECE_TILES, A.tiles - p * PIECE_TILES);
+    for (int c = tid; c < nt * (KT / 4); c += 256) *(uint4*)(row + 4 * c) = make_uint4(EMPTY, EMPTY, EMPTY, EMPTY);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SLOTS; i++)
+      if (id[i] >= 0 && id[i] / (PIECE_TILES * KT) == p) dup |= atomicExch(row + id[i] % (PIECE_TILES * KT), a[i]) != EMPTY;
+    __syncthreads();
+    float* out = A.factors + ((size_t)ql * A.tiles + p * PIECE_TILES) * KT + 4 * lane;
+    unsigned marks = 0;
+    for (int t = wave; t < nt; t += 4) {
+      uint4 v = *(const uint4*)(row + t * KT + 4 * lane);
+      const bool any = v.x != EMPTY || v.y != EMPTY || v.z != EMPTY || v.w != EMPTY;
+      if (__ballot(any) == 0) continue;
+      marks |= 1u << t;
+      v.x = v.x == EMPTY ? UNSELECTED : v.x;
+      v.y = v.y == EMPTY ? UNSELECTED : v.y;
+      v.z = v.z == EMPTY ? UNSELECTED : v.z;
+      v.w = v.w == EMPTY ? UNSELECTED : v.w;
+      *(uint4*)(out + t * KT) = v;
+    }
+    if (lane == 0 && marks) atomicOr(&marks_s, marks);
+    __syncthreads();
+    if (tid == 0) {
+      A.marks[(size_t)ql * A.words + p] = marks_s;
+      marks_s = 0;
+    }
+  }
+  if (bad || dup) atomicOr(&flags_s, (bad ? QUERY_BAD : 0) | (dup ? QUERY_DUP : 0));
+  __syncthreads();
+  if (tid == 0) A.state[ql] = flags_s;
+}
+
+__device__ __forceinline__ void dma4(unsigned lds_base, unsigned goff, const void* gbase) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
+}
+
+// One workgroup of eight waves, 32 keys a wave: scores of the query's heads with the wave's keys on the columns, their masks, the rows
+// of the keys, times the pairs' factors into the sums.  Two queries a step; their operands and factors come into a ring of three steps
+// by transfers that the waves share out.
+constexpr int KEYS_STAGES = 3;
+constexpr int MAX_CHUNK = 128;
+template <int NHT> constexpr size_t keys_lds_bytes() { return (size_t)KEYS_STAGES * (2 * operand_bytes(NHT) + 8 * 256) + (MAX_CHUNK + 4) * 4; }
+
+template <int NHT>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void indexer_keys_kernel(const DenseArgs A) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  constexpr int OPS = operand_bytes(NHT), STAGE = 2 * OPS + 8 * 256;
+  constexpr int PER = OPS / 4096 + 1;               // transfers of a wave per step
+  int* list = (int*)(smem + KEYS_STAGES * STAGE);   // [MAX_CHUNK] queries; their number; whether an operand of the chunk is not finite
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, g = lane >> 5;
+  // chunk c is an XCD's (c mod 8): the workgroups that read the same queries' operands at the same time share an L2
+  const int c = ((int)blockIdx.x >> 3) / A.tiles * 8 + ((int)blockIdx.x & 7), tile = ((int)blockIdx.x >> 3) % A.tiles;
+  if (c >= A.chunks) return;
+  if (wave == 0) {
+    int n = 0;
+    bool dup = false, bad = false;
+    for (int h = 0; h < A.chunk; h += 64) {
+      const int i = h + lane, q = c * A.chunk + i;
+      const bool in = i < A.chunk && q < A.cnt;
+      const int st = in ? A.state[q] : 0;
+      const bool live = in && ((A.marks[(size_t)q * A.words + tile / PIECE_TILES] >> (tile % PIECE_TILES)) & 1u);
+      const unsigned long long m = __ballot(live);
+      if (live) list[n + __popcll(m & ((1ull << lane) - 1))] = q;
+      n += __popcll(m);
+      dup |= __ballot(st & QUERY_DUP) != 0;
+      bad |= __ballot(st & QUERY_BAD) != 0;
+    }
+    if (lane == 0) {
+      list[MAX_CHUNK] = n;
+      list[MAX_CHUNK + 1] = bad;
+      A.used[(size_t)c * A.tiles + tile] = dup ? -1 : n;
+    }
+  }
+  __syncthreads();
+  const int n = __builtin_amdgcn_readfirstlane(list[MAX_CHUNK]);
+  const bool bad = __builtin_amdgcn_readfirstlane(list[MAX_CHUNK + 1]) != 0;
+  if (n == 0) return;
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  const float* fbase = A.factors + ((size_t)c * A.chunk * A.tiles + tile) * KT + 32 * wave;
+  int qa, qb;                                       // the two queries of the step that is requested next
+  auto look_up = [&](int step) {
+    qa = list[min(2 * step, n - 1)];
+    qb = list[min(2 * step + 1, n - 1)];
+  };
+  auto issue = [&](int slot) {
+    const int a = __builtin_amdgcn_readfirstlane(qa), b = __builtin_amdgcn_readfirstlane(qb);
+    const unsigned base = lds0 + (unsigned)(slot * STAGE);
+    const unsigned char* src = A.ops + (size_t)(wave < 4 ? a : b) * OPS + (wave & 3) * (OPS / 4);
+    const unsigned dst = base + (unsigned)((wave >> 2) * OPS + (wave & 3) * (OPS / 4));
+#pragma unroll
+    for (int i = 0; i < PER - 1; i++) dma16(dst + i * 1024, (unsigned)(lane * 16 + i * 1024), src);
+    dma4(base + (unsigned)(2 * OPS + wave * 256), (unsigned)(((lane < 32 ? a : b) - c * A.chunk) * A.tiles * (KT * 4) + r * 4), fbase);
+  };
+  // key row of the lane, bytes [64 s + 32 g, + 32)
+  i32x8 bk[2];
+  {
+    const unsigned char* kp = A.k8 + (size_t)min(tile * KT + 32 * wave + r, A.Sk - 1) * D + 32 * g;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const i32x4 lo = *(const i32x4*)(kp + 64 * s), hi = *(const i32x4*)(kp + 64 * s + 16);
+      bk[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  }
+  DSA_WAIT_VMCNT(0);                                // from here on only the transfers count
+  asm volatile("" : "+v"(bk[0]), "+v"(bk[1]) :: "memory");
+  const int steps = (n + 1) >> 1;
+  look_up(0);
+  issue(0);
+  look_up(1);
+  if (steps > 1) issue(1);
+  look_up(2);
+  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  f32x16 sum[4], acc[NHT], racc[2];
+  bf16x8 mk[2 * NHT], qt[2][2 * NHT];
+#pragma unroll
+  for (int dt = 0; dt < 4; dt++) sum[dt] = zero;
+  auto read_query = [&](int t, unsigned ob, i32x8 (&aq)[2]) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const i32x4 lo = lds_read<i32x4>(ob + (4 * t + 2 * s) * 1024), hi = lds_read<i32x4>(ob + (4 * t + 2 * s + 1) * 1024);
+      aq[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  auto scores = [&](int t, const i32x8 (&aq)[2]) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aq[s], bk[s], s ? acc[t] : zero, 0, 0, 0, 147, 0, 127);
+  };
+  auto read_weighted = [&](int dt, unsigned ob) {
+#pragma unroll
+    for (int kk = 0; kk < 2 * NHT; kk++) qt[dt & 1][kk] = lds_read<bf16x8>(ob + (4 * NHT + dt * 2 * NHT + kk) * 1024);
+  };
+  if (steps > 1) { DSA_WAIT_VMCNT(PER); } else { DSA_WAIT_VMCNT(0); }
+  asm volatile("s_barrier" ::: "memory");
+  unsigned ob = lds0 + (unsigned)(lane * 16);       // operands of the query in hand
+#pragma unroll
+  for (int t = 0; t < NHT; t++) {
+    i32x8 aq[2];
+    read_query(t, ob, aq);
+    scores(t, aq);
+  }
+  score_masks<NHT>(acc, mk);
+  read_weighted(0, ob);
+  // Scores and masks of the query behind the one in hand are made under the products of the latter (behind the last one: of what lies
+  // in the ring, unused).  FINITE: every operand of the chunk is; otherwise infinities and NaN stay with the keys that the query selected.
+  auto sweep = [&](auto finite) {
+    constexpr bool FINITE = decltype(finite)::value;
+    int slot = 0;
+    for (int step = 0; step < steps; step++) {
+      const int next_slot = slot + 1 < KEYS_STAGES ? slot + 1 : 0;
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        if (x == 1 && 2 * step + 1 >= n) break;
+        if (x == 1 || 2 * step + 1 >= n) {          // the last query of the step: the next step's operands from here on
+          // its transfers have landed, and every read of the step before this one has come back: its slot is filled next
+          DSA_WAIT_VMCNT(0);
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          if (step + 2 < steps) issue(slot >= 1 ? slot - 1 : KEYS_STAGES - 1);
+          look_up(step + 3);
+        }
+        const unsigned on = x == 0 ? ob + OPS : lds0 + (unsigned)(next_slot * STAGE + lane * 16);
+        const float a = lds_read<float>(lds0 + (unsigned)(slot * STAGE + 2 * OPS + wave * 256 + x * 128 + r * 4));
+        const float a128 = a * 128.f;               // (the masks' entries are 2^-7)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < 5; dt++) {            // the products of a d-tile run while the one before it is added
+          constexpr int STEP = 16 / (2 * NHT);
+          i32x8 aq[2];
+          if (dt < 4) read_weighted((dt + 1) & 3, dt < 3 ? ob : on);
+          if (dt < NHT) read_query(dt, on, aq);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = 0; kk < 2 * NHT; kk++) {
+            if (dt < 4) racc[dt & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt[dt & 1][kk], mk[kk], kk ? racc[dt & 1] : zero, 0, 0, 0);
+            if (dt > 0) {
+#pragma unroll
+              for (int e = STEP * kk; e < STEP * (kk + 1); e++) {
+                float v = racc[(dt - 1) & 1][e];
+                if (!FINITE) v = __builtin_bit_cast(unsigned, a) == UNSELECTED ? 0.f : v;
+                sum[dt - 1][e] = fmaf(a128, v, sum[dt - 1][e]);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (dt < NHT) scores(dt, aq);
+          if (dt == 3) score_masks<NHT>(acc, mk);   // (the masks in hand have had their last use)
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        ob = on;
+      }
+      slot = next_slot;
+    }
+  };
+  if (bad) sweep(std::false_type()); else sweep(std::true_type());
+  float* out = A.part + (((size_t)c * A.tiles + tile) * KT + 32 * wave + r) * D + 4 * g;
+#pragma unroll
+  for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      *(f32x4*)(out + 32 * dt + 8 * j) = f32x4{sum[dt][4 * j], sum[dt][4 * j + 1], sum[dt][4 * j + 2], sum[dt][4 * j + 3]};
+}
+
+// d_k8[key] (+)= the sums of the chunks that hold the key: 8 groups of 32 threads, chunk c in group c mod 8, the groups in a fixed order.
+__global__ __launch_bounds__(256) void indexer_chunk_sum_kernel(const float* __restrict__ part, const int* __restrict__ used, int chunks, int tiles,
+                                                                float* __restrict__ d_k8, int accumulate) {
+  __shared__ f32x4 part_s[8][32];
+  const int key = blockIdx.x, tile = key / KT, col = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  bool dup = false;
+#pragma unroll 4
+  for (int c = grp; c < chunks; c += 8) {
+    const int n = used[(size_t)c * tiles + tile];
+    dup |= n < 0;
+    if (n > 0) acc += *(const f32x4*)(part + (((size_t)c * tiles + tile) * KT + key % KT) * D + 4 * col);
+  }
+  part_s[grp][col] = acc;
+  dup = __syncthreads_or(dup);
+  if (grp == 0) {
+    f32x4 s = ((part_s[0][col] + part_s[1][col]) + (part_s[2][col] + part_s[3][col])) +
+              ((part_s[4][col] + part_s[5][col]) + (part_s[6][col] + part_s[7][col]));
+    float* p = d_k8 + (size_t)key * D + 4 * col;
+    if (accumulate) s += *(const f32x4*)p;
+    if (dup) s = f32x4{1.f, 1.f, 1.f, 1.f} * __builtin_nanf("");        // a query row held a repeated id: no sum that misses a term
+    *(f32x4*)p = s;
   }
 }
 
@@ -766,13 +1148,70 @@ Plan make_plan(int S, int Sk, int K, size_t budget) {
 }
 constexpr size_t DEFAULT_BUDGET = (size_t)16 << 30;
 
+struct DensePlan {
+  int queries, tiles, words, chunk, chunks;          // queries of a sweep; key tiles; words of marks; queries of a chunk; chunks of a sweep
+  size_t off_factors, off_marks, off_state, off_ops, off_part, off_used, total;
+};
+DensePlan dense_layout(int queries, int Hi, int Sk, int seen) {
+  DensePlan p;
+  p.queries = queries;
+  p.tiles = dsa_cdiv(Sk, KT);
+  p.words = dsa_cdiv(p.tiles, PIECE_TILES);
+  // Queries of a chunk: rounds of 256 workgroups of 7 us and 1.2 us a query (0.65 with one head tile), against 128 KB of sums written and
+  // read per workgroup.  Under a causal window a query sees half of `seen` in the mean, and half of a tile besides.  (Chunks of
+  // 16 / 32 / 64 / 128, us of the whole call: 1000 queries x 256 slots 73 / 83 / 114 / 177, taken 16; 3072 x 512 of 768 keys
+  // 158 / 143 / 170 / 231, 32; 8192 x 2048 1786 / 1505 / 1366 / 1369, 128.)
+  float best = INFINITY;
+  for (int chunk : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96, MAX_CHUNK}) {
+    const float live = dsa_cdiv(queries, chunk) * (seen / (2.f * KT) + 0.5f);
+    const float us = (live <= 160 ? 1.f : live / 256 + 0.6f) * (7 + chunk * (Hi <= 32 ? 0.65f : 1.2f)) + live * 0.058f;
+    if (us < best) {
+      best = us;
+      p.chunk = chunk;
+    }
+  }
+  p.chunks = dsa_cdiv(queries, p.chunk);
+  size_t o = 0;
+  p.off_factors = o; o = align_up(o + (size_t)queries * p.tiles * KT * 4);
+  p.off_marks = o; o = align_up(o + (size_t)queries * p.words * 4);
+  p.off_state = o; o = align_up(o + (size_t)queries * 4);
+  p.off_ops = o; o = align_up(o + (size_t)queries * operand_bytes(Hi / 32));
+  p.off_part = o; o = align_up(o + (size_t)p.chunks * p.tiles * KT * D * 4);
+  p.off_used = o; o = align_up(o + (size_t)p.chunks * p.tiles * 4);
+  p.total = o;
+  return p;
+}
+DensePlan dense_plan(int S, int Hi, int Sk, int span, size_t budget) {
+  const int seen = span > 0 && span < Sk ? span : Sk;
+  int queries = S;
+  DensePlan p = dense_layout(queries, Hi, Sk, seen);
+  while (p.total > budget && queries > 64) {
+    queries = (queries + 1) / 2;
+    p = dense_layout(queries, Hi, Sk, seen);
+  }
+  return p;
+}
+// Whether d_k8 is summed by key tiles, by prices in ns a query (fitted to 20 shapes of 300-32 768 queries, 256-2048 slots): the products with
+// a key that the query sees 0.0225, a pair with a row of its own 0.11 against 0.031 for its part in d_q8 alone, the key-sorted order
+// 11 more than the scattered factors; 10 us a call for the longer chain.  Whole call, rows / key tiles in us: 8192 queries x 2048 slots of a
+// causal window 2070 / 1640, 12 000 x 2048 2800 / 2520, x 1024 1540 / 2190, x 256 673 / 1918, in five documents x 512 942 / 899; 3072 x 512 of
+// 768 compressed keys 246 / 185; 500 x 512 of 6000 keys 71 / 126.  span: the most keys that a query sees, 0 if not known.
+bool by_key_tiles(int S, int Sk, int K, int span) {
+  const float seen = span > 0 && span < Sk ? span : Sk, queries = S > 0 ? S : 1;
+  const float visible = queries < seen ? seen - 0.5f * queries : 0.5f * seen;       // the window of the last queries, or one that grows from nothing
+  const float selected = queries < seen ? fminf(K, visible) : K < seen ? K - 0.5f * K * K / seen : visible;
+  return 0.0225f * (visible + 0.8f * KT) + 10000.f / queries < 11.f + 0.079f * selected;
+}
+
 }  // namespace
 
-extern "C" size_t dsa_indexer_bwd_workspace_bytes(int S, int Hi, int Sk, int K) {
-  (void)Hi;
+static size_t bwd_workspace(int S, int Hi, int Sk, int K, int span) {
   if (S <= 0 || Sk <= 0 || K <= 0) return 0;
+  if (by_key_tiles(S, Sk, K, span)) return dense_plan(S, Hi <= 32 ? 32 : 64, Sk, span, DEFAULT_BUDGET).total;
   return make_plan(S, Sk, K, DEFAULT_BUDGET).total;
 }
+
+extern "C" size_t dsa_indexer_bwd_workspace_bytes(int S, int Hi, int Sk, int K) { return bwd_workspace(S, Hi, Sk, K, 0); }
 
 namespace {
 
@@ -783,7 +1222,52 @@ struct KeyFinish {
   float* d_ln_b;
 };
 
-int run_bwd(const char* name, BwdArgs A, int S, int Hi, float* d_k8, const KeyFinish* kf, void* workspace, size_t workspace_bytes, void* stream) {
+int finish_keys(const char* name, const KeyFinish* kf, int Sk, hipStream_t st) {
+  if (!kf) return DSA_OK;
+  const int blocks = dsa_cdiv(Sk, 16) < KEY_BLOCKS ? dsa_cdiv(Sk, 16) : KEY_BLOCKS;
+  indexer_key_finish_kernel<<<dim3(blocks), dim3(256), 0, st>>>(kf->key);
+  if (kf->key.k_in) indexer_ln_sum_kernel<<<dim3(4), dim3(256), 0, st>>>(kf->key.part, blocks, kf->d_ln_w, kf->d_ln_b);
+  DSA_CHECK_LAUNCH("indexer_bwd(keys)");
+  return DSA_OK;
+}
+
+int run_by_key_tiles(const char* name, BwdArgs A, const DensePlan& p, int S, int Hi, float* d_k8, const KeyFinish* kf, unsigned char* ws, hipStream_t st) {
+  const int Sk = A.Sk, K = A.K;
+  DenseArgs d = {};
+  d.gsc = A.gsc; d.q8 = A.q8; d.k8 = A.k8; d.k_scale = A.k_scale; d.q_w = A.q_w; d.ids = A.ids;
+  d.Sk = Sk; d.K = K;
+  d.tiles = p.tiles; d.words = p.words; d.chunk = p.chunk;
+  d.factors = (float*)(ws + p.off_factors);
+  d.marks = (unsigned*)(ws + p.off_marks);
+  d.state = (int*)(ws + p.off_state);
+  d.ops = ws + p.off_ops;
+  d.part = (float*)(ws + p.off_part);
+  d.used = (int*)(ws + p.off_used);
+  const size_t smem = bwd_lds_bytes(Hi, 2, K, false), smem_keys = Hi == 32 ? keys_lds_bytes<1>() : keys_lds_bytes<2>();
+  auto scatter = Hi == 32 ? indexer_scatter_kernel<1> : indexer_scatter_kernel<2>;
+  auto keys = Hi == 32 ? indexer_keys_kernel<1> : indexer_keys_kernel<2>;
+  auto queries = Hi == 32 ? indexer_bwd_kernel<1, 2, false> : indexer_bwd_kernel<2, 2, false>;
+  if (dsa_reserve_lds((const void*)queries, smem) != hipSuccess || dsa_reserve_lds((const void*)keys, smem_keys) != hipSuccess)
+    DSA_FAIL(DSA_ERR_LAUNCH, "%s: cannot reserve LDS", name);
+  for (int q0 = 0; q0 < S; q0 += p.queries) {
+    d.q0 = A.q0 = q0;
+    d.cnt = A.cnt = S - q0 < p.queries ? S - q0 : p.queries;
+    d.chunks = dsa_cdiv(d.cnt, p.chunk);
+    scatter<<<dim3(d.cnt), dim3(256), 0, st>>>(d);
+    DSA_CHECK_LAUNCH("indexer_bwd(factors)");
+    queries<<<dim3(d.cnt), dim3(THREADS / 2), smem, st>>>(A);
+    DSA_CHECK_LAUNCH("indexer_bwd");
+    keys<<<dim3(dsa_cdiv(d.chunks, 8) * 8 * p.tiles), dim3(THREADS), smem_keys, st>>>(d);
+    DSA_CHECK_LAUNCH("indexer_bwd(key tiles)");
+    indexer_chunk_sum_kernel<<<dim3(Sk), dim3(256), 0, st>>>(d.part, d.used, d.chunks, d.tiles, d_k8, q0 > 0);
+    DSA_CHECK_LAUNCH("indexer_bwd(chunk sums)");
+  }
+  if (S == 0) order::zero_u32_kernel<<<dim3(256), dim3(256), 0, st>>>((unsigned*)d_k8, (size_t)Sk * D);
+  return finish_keys(name, kf, Sk, st);
+}
+
+int run_bwd(const char* name, BwdArgs A, int S, int Hi, int span, float* d_k8, const KeyFinish* kf, void* workspace, size_t workspace_bytes,
+            void* stream) {
   const int Sk = A.Sk, K = A.K;
   DSA_REQUIRE(Hi == 32 || Hi == 64, "%s: head count must be 32 or 64, got %d", name, Hi);
   DSA_REQUIRE(S >= 0 && Sk > 0, "%s: bad sizes S=%d Sk=%d", name, S, Sk);
@@ -794,6 +1278,10 @@ int run_bwd(const char* name, BwdArgs A, int S, int Hi, float* d_k8, const KeyFi
               ((uintptr_t)A.d_q8 % 16) == 0 && ((uintptr_t)A.d_q % 16) == 0 && ((uintptr_t)d_k8 % 16) == 0 && ((uintptr_t)workspace % 256) == 0,
               "%s: misaligned pointer", name);
   hipStream_t st = (hipStream_t)stream;
+  if (workspace != nullptr && by_key_tiles(S, Sk, K, span)) {
+    const DensePlan p = dense_plan(S > 0 ? S : 1, Hi, Sk, span, workspace_bytes);
+    if (p.total <= workspace_bytes) return run_by_key_tiles(name, A, p, S, Hi, d_k8, kf, (unsigned char*)workspace, st);
+  }
   Plan p = make_plan(S > 0 ? S : 1, Sk, K, workspace_bytes);
   if (p.total > workspace_bytes || workspace == nullptr)
     DSA_FAIL(DSA_ERR_WORKSPACE, "%s: workspace of %zu bytes is too small (need at least %zu)", name, workspace_bytes, layout_plan(64, Sk, K).total);
@@ -807,9 +1295,9 @@ int run_bwd(const char* name, BwdArgs A, int S, int Hi, float* d_k8, const KeyFi
   A.dst = dstp;
   A.rows = (unsigned short*)(ws + p.off_rows);
   A.dummy_row = p.chunk * K;
-  const size_t smem = bwd_lds_bytes(Hi, K);
-  auto kern = bwd_stages(K) == 3 ? (Hi == 32 ? indexer_bwd_kernel<1, 3> : indexer_bwd_kernel<2, 3>)
-                                 : (Hi == 32 ? indexer_bwd_kernel<1, 2> : indexer_bwd_kernel<2, 2>);
+  const size_t smem = bwd_lds_bytes(Hi, bwd_stages(K), K, true);
+  auto kern = bwd_stages(K) == 3 ? (Hi == 32 ? indexer_bwd_kernel<1, 3, true> : indexer_bwd_kernel<2, 3, true>)
+                                 : (Hi == 32 ? indexer_bwd_kernel<1, 2, true> : indexer_bwd_kernel<2, 2, true>);
   if (dsa_reserve_lds((const void*)kern, smem) != hipSuccess) DSA_FAIL(DSA_ERR_LAUNCH, "%s: cannot reserve LDS", name);
   bool first = true;
   order::clear_flag(dup_flag, st);
@@ -826,13 +1314,7 @@ int run_bwd(const char* name, BwdArgs A, int S, int Hi, float* d_k8, const KeyFi
     first = false;
   }
   if (S == 0) order::zero_u32_kernel<<<dim3(256), dim3(256), 0, st>>>((unsigned*)d_k8, (size_t)Sk * D);
-  if (kf) {
-    const int blocks = dsa_cdiv(Sk, 16) < KEY_BLOCKS ? dsa_cdiv(Sk, 16) : KEY_BLOCKS;
-    indexer_key_finish_kernel<<<dim3(blocks), dim3(256), 0, st>>>(kf->key);
-    if (kf->key.k_in) indexer_ln_sum_kernel<<<dim3(4), dim3(256), 0, st>>>(kf->key.part, blocks, kf->d_ln_w, kf->d_ln_b);
-    DSA_CHECK_LAUNCH("indexer_bwd(keys)");
-  }
-  return DSA_OK;
+  return finish_keys(name, kf, Sk, st);
 }
 
 size_t grads_extra_bytes(int Sk) { return align_up((size_t)Sk * D * 4) + align_up((size_t)KEY_BLOCKS * 2 * D * 4); }
@@ -845,13 +1327,14 @@ extern "C" int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, c
   BwdArgs A = {};
   A.gsc = g; A.q8 = (const unsigned char*)q8; A.k8 = (const unsigned char*)k8; A.k_scale = k_scale; A.q_w = q_w; A.ids = ids;
   A.Sk = Sk; A.K = K; A.d_q8 = d_q8; A.d_qw = d_qw;
-  return run_bwd("dsa_indexer_bwd", A, S, Hi, d_k8, nullptr, workspace, workspace_bytes, stream);
+  return run_bwd("dsa_indexer_bwd", A, S, Hi, 0, d_k8, nullptr, workspace, workspace_bytes, stream);
 }
 
-extern "C" size_t dsa_indexer_grads_workspace_bytes(int S, int Hi, int Sk, int K) {
+extern "C" size_t dsa_indexer_grads_span_workspace_bytes(int S, int Hi, int Sk, int K, int span) {
   if (Sk <= 0 || K <= 0) return 0;
-  return dsa_indexer_bwd_workspace_bytes(S > 0 ? S : 1, Hi, Sk, K) + grads_extra_bytes(Sk);
+  return bwd_workspace(S > 0 ? S : 1, Hi, Sk, K, span) + grads_extra_bytes(Sk);
 }
+extern "C" size_t dsa_indexer_grads_workspace_bytes(int S, int Hi, int Sk, int K) { return dsa_indexer_grads_span_workspace_bytes(S, Hi, Sk, K, 0); }
 
 extern "C" int dsa_indexer_grads(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
                                  const int32_t* ids, int S, int Hi, int Sk, int K, const float* q_scale, float w_scale, int rotate,
@@ -859,6 +1342,17 @@ extern "C" int dsa_indexer_grads(const float* g, const void* q8, const void* k8,
                                  const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps,
                                  int heads, int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32,
                                  float* d_ln_w, float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream) {
+  return dsa_indexer_grads_span(g, q8, k8, k_scale, q_w, ids, S, Hi, Sk, K, 0, q_scale, w_scale, rotate, cos, sin, tables_f32, pairing,
+                                positions_q, positions_k, batch, k_in, ln_w, ln_eps, heads, dim, d_q, q_f32, d_k, k_f32, d_w, w_f32, d_ln_w,
+                                d_ln_b, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsa_indexer_grads_span(const float* g, const void* q8, const void* k8, const float* k_scale, const float* q_w,
+                                      const int32_t* ids, int S, int Hi, int Sk, int K, int span, const float* q_scale, float w_scale, int rotate,
+                                      const void* cos, const void* sin, int tables_f32, int pairing, const int32_t* positions_q,
+                                      const int32_t* positions_k, int batch, const void* k_in, const float* ln_w, float ln_eps,
+                                      int heads, int dim, void* d_q, int q_f32, void* d_k, int k_f32, void* d_w, int w_f32,
+                                      float* d_ln_w, float* d_ln_b, void* workspace, size_t workspace_bytes, void* stream) {
   DSA_REQUIRE(heads > 0 && heads <= Hi && dim > 0 && dim <= D, "dsa_indexer_grads: %d heads of %d channels do not fit %d x %d", heads, dim, Hi, D);
   DSA_REQUIRE(q_scale != nullptr, "dsa_indexer_grads: q_scale is missing");
   DSA_REQUIRE(pairing < 0 || (cos != nullptr && sin != nullptr && pairing <= 1 && batch > 0), "dsa_indexer_grads: bad rotary arguments");
@@ -879,5 +1373,5 @@ extern "C" int dsa_indexer_grads(const float* g, const void* q8, const void* k8,
   kf.key = KeyArgs{d_k8, k_scale, Sk, A.fin, positions_k, (const unsigned short*)k_in, ln_w, ln_eps, d_k, k_f32, dim,
                    (float*)((unsigned char*)workspace + align_up((size_t)Sk * D * 4))};
   kf.d_ln_w = d_ln_w; kf.d_ln_b = d_ln_b;
-  return run_bwd("dsa_indexer_grads", A, S, Hi, d_k8, &kf, (unsigned char*)workspace + extra, workspace_bytes - extra, stream);
+  return run_bwd("dsa_indexer_grads", A, S, Hi, span, d_k8, &kf, (unsigned char*)workspace + extra, workspace_bytes - extra, stream);
 }

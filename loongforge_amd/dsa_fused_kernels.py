@@ -243,6 +243,12 @@ def _pad_to(x: Tensor, size: int, dim: int) -> Tensor:
     return torch.nn.functional.pad(x, pad)
 
 
+def _known_span(packed_seq_params) -> int:
+    """The most keys that a query sees, 0 where the host does not know it."""
+    longest = getattr(packed_seq_params, "max_seqlen_kv", None)
+    return longest if isinstance(longest, int) else 0
+
+
 class DSAIndexerKernelFunction(torch.autograd.Function):
     """fp8 lightning indexer: quantise -> windowed logits -> top-k, with the sparse backward.
 
@@ -320,6 +326,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
         ctx.softmax_scale = softmax_scale
         ctx.rotate = rotate
         ctx.index_topk = index_topk
+        ctx.span = _known_span(packed_seq_params)
         ctx.shape = (head, dim)
         ctx.in_dtypes = (index_q.dtype, index_k.dtype, weights.dtype)
         ctx.front = front
@@ -339,7 +346,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
         k_in, ln_w, ln_b = ctx.front_saved if ctx.front is not None else (None, None, None)
         d_q, d_k, d_weights, d_ln_w, d_ln_b = ops.indexer_grads(
             grad_score, q_fp8, k_fp8, k_scale, weight_scaled, topk_indices, q_scale, ctx.softmax_scale, head, dim, ctx.in_dtypes,
-            ctx.rotate, ctx.front, k_in, ln_w)
+            ctx.rotate, ctx.front, k_in, ln_w, ctx.span)
         if ctx.front is not None:
             d_ln_w, d_ln_b = d_ln_w.to(ln_w.dtype), d_ln_b.to(ln_b.dtype)
         return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b

@@ -347,18 +347,19 @@ def indexer_bwd(g, q8, k8, k_scale, q_w, ids):
 
 
 def indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale: float, heads: int, dim: int, dtypes, rotate: bool = False,
-                  front=None, k_in=None, ln_weight=None):
+                  front=None, k_in=None, ln_weight=None, span: int = 0):
     """:func:`indexer_bwd` carried on to the outputs of the projections: ``(d_q [S, heads, dim], d_k [Sk, dim], d_weights
     [S, heads], d_ln_weight, d_ln_bias)`` in ``dtypes`` (of q, k, weights), the last two fp32 or None.  Unscaled (rows on the
     quantiser's epsilon floor, loongforge/models/foundation/deepseek_v4/deepseek_v4_csa.py:1525-1541, get zero), back
     through the Hadamard rotation if ``rotate``, and with ``front`` (an ``IndexerFrontEnd``) through the rotary embedding
-    and the LayerNorm of the keys (input ``k_in``, weight ``ln_weight``)."""
+    and the LayerNorm of the keys (input ``k_in``, weight ``ln_weight``).  ``span``: the most neighbouring keys that a query
+    sees, 0 if that is not known; it decides how the keys' gradients are summed, not what they are."""
     f = front
     if f is None and not ordinary(g, q8, k8, k_scale, q_w, ids, q_scale):
         return _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, rotate)
     return _native().indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, float(w_scale), bool(rotate), f and f.cos, f and f.sin,
                                    f.pairing if f else -1, f and f.positions_q, f and f.positions_k, f.batch if f else 1,
-                                   k_in, ln_weight, f.k_norm_eps if f else 0.0, int(heads), int(dim), *dtypes)
+                                   k_in, ln_weight, f.k_norm_eps if f else 0.0, int(heads), int(dim), int(span), *dtypes)
 
 
 def _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, rotate):

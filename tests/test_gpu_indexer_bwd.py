@@ -210,3 +210,77 @@ def test_key_sums_over_many_keys(gpu, S, Sk, K):
     assert (dq.cpu() - rq).abs().max() <= 1e-4 * rq.abs().max() and (dw.cpu() - rw).abs().max() <= 1e-4 * rw.abs().max()
     # pair rows are bf16, from head factors w q in bf16
     assert ((dk.cpu() - rk).abs() <= 2e-2 * rk_abs[:, None] + 1e-3).all()
+
+
+def _pairs(S, Sk, K, Hi, seed, full):
+    """Inputs of a backward whose queries select about `full` of K slots, no gate within accumulation noise of zero."""
+    gen = torch.Generator().manual_seed(seed)
+    q8 = torch.randn(S, Hi, 128, generator=gen).to(torch.float8_e4m3fn)
+    k8 = torch.randn(Sk, 128, generator=gen).to(torch.float8_e4m3fn)
+    ksc, w, g = torch.rand(Sk, generator=gen) + 0.5, torch.randn(S, Hi, generator=gen), torch.randn(S, K, generator=gen)
+    ids = torch.full((S, K), -1, dtype=torch.int32)
+    n = min(K, Sk)
+    ids[:, :n] = torch.rand(S, Sk, generator=gen).topk(n, dim=1).indices.int()
+    ids[torch.rand(S, K, generator=gen) > full] = -1
+    ids[S // 3] = -1
+    k = k8.double()[ids.clamp(min=0).long()]
+    r = q8.double() @ k.transpose(1, 2)
+    noise = r.abs() <= 2.0 ** -16 * (q8.double().abs() @ k.abs().transpose(1, 2))
+    g[noise.any(1)] = 0.0
+    return g, q8, k8, ksc, w, ids, r, k
+
+
+def _grads(gpu, g, q8, k8, ksc, w, ids, span):
+    from loongforge_amd import ops
+
+    S, Hi = w.shape
+    t = [x.to(gpu) for x in (g, q8, k8, ksc, w, ids)]
+    d_q, d_k, d_w, _, _ = ops.indexer_grads(*t, torch.ones(S, Hi, device=gpu), 1.0, Hi, 128, [torch.float32] * 3, span=span)
+    return d_q.cpu().double(), d_k.cpu().double() * ksc.double()[:, None], d_w.cpu().double()
+
+
+# From 1600 queries on a span of one key makes the products with whole key tiles the cheaper way whatever the sizes.
+@pytest.mark.parametrize("S,Sk,K,Hi,full", [
+    (1600, 1, 128, 32, 0.9),
+    (1601, 255, 128, 64, 0.5),           # one tile, a key short
+    (1663, 257, 256, 32, 1.0),           # one key in the second tile
+    (1605, 513, 384, 64, 0.01),          # tiles that few queries touch
+    (1600, 4097, 128, 64, 1.0),          # one key in the second piece of factors
+    (1700, 9000, 256, 32, 0.3),
+])
+def test_key_gradients_by_key_tiles(gpu, S, Sk, K, Hi, full):
+    g, q8, k8, ksc, w, ids, r, k = _pairs(S, Sk, K, Hi, S + Sk, full)
+    live = ids >= 0
+    a = torch.where(live, g.double() * ksc.double()[ids.clamp(min=0).long()], torch.zeros(()).double())
+    m = (r > 0).double()
+    wq = w.double()[:, :, None] * q8.double()
+    rk, rk_abs = torch.zeros(Sk, 128).double(), torch.zeros(Sk, 128).double()
+    flat = ids.clamp(min=0).long().flatten()
+    rk.index_add_(0, flat, (a[:, :, None] * (m.transpose(1, 2) @ wq)).flatten(0, 1))
+    rk_abs.index_add_(0, flat, (a.abs()[:, :, None] * (m.transpose(1, 2) @ wq.abs())).flatten(0, 1))
+    rq = w.double()[:, :, None] * ((a[:, None, :] * m) @ k)
+    rw = (a[:, None, :] * r.clamp(min=0)).sum(2)
+    d_q, d_k, d_w = _grads(gpu, g, q8, k8, ksc, w, ids, 1)
+    assert (d_q - rq).abs().max() <= 1e-4 * rq.abs().max() and (d_w - rw).abs().max() <= 1e-4 * rw.abs().max()
+    # w q is rounded to bf16 (half a step: 2^-9); everything behind it is 32-bit sums of at most 64 S terms
+    assert ((d_k - rk).abs() <= (2.0 ** -9 + 1e-5) * rk_abs + 1e-30).all()
+    again = _grads(gpu, g, q8, k8, ksc, w, ids, 1)
+    assert torch.equal(d_q, again[0]) and torch.equal(d_k, again[1]) and torch.equal(d_w, again[2])
+
+
+def test_key_gradients_by_key_tiles_of_values_that_are_not_finite(gpu):
+    """An infinite weight or factor, a NaN: the keys that the query selected get them, no others do - as with a row per pair."""
+    g, q8, k8, ksc, w, ids, _, _ = _pairs(1600, 4500, 128, 64, 3, 1.0)
+    w[17, 5], w[900, 0], g[1200, 3], g[1300, 4] = float("inf"), float("nan"), float("inf"), float("nan")
+    g[900, 7] = g[17, 9] = 0.0
+    rows, tiles = _grads(gpu, g, q8, k8, ksc, w, ids, 0), _grads(gpu, g, q8, k8, ksc, w, ids, 1)
+    for a, b in zip(rows, tiles):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b)) and not torch.isfinite(a).all()
+    fin = torch.isfinite(rows[1])
+    assert fin.any() and (rows[1] - tiles[1])[fin].norm() <= 1e-2 * rows[1][fin].norm()
+
+
+def test_key_gradients_by_key_tiles_with_a_repeated_id(gpu):
+    g, q8, k8, ksc, w, ids, _, _ = _pairs(1600, 4500, 128, 32, 4, 1.0)
+    ids[1599, 100] = ids[1599, 3]
+    assert torch.isnan(_grads(gpu, g, q8, k8, ksc, w, ids, 1)[1]).all()
