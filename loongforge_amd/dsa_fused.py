@@ -25,7 +25,7 @@ from typing import Optional, Tuple, Union
 import torch
 import torch.nn.functional as F
 
-from .dsa_fused_kernels import DSADotProductAttention, DSAIndexerKernel, triton_attn_dist
+from .dsa_fused_kernels import DSADotProductAttention, DSAIndexerKernel, _takes_checks, triton_attn_dist
 from .megatron_compat import (
     AttnMaskType,
     DSAIndexerLossAutoScaler,
@@ -408,8 +408,10 @@ class DSAIndexerFused(MegatronModule):
                                positions_k=pos_k, batch=1 if packed_seq_params is not None else x.shape[1],
                                k_norm_eps=float(k_norm.eps))
 
-    def forward(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None):
-        """-> ``(index_score_topk [s, topk], topk_indices [s, topk])`` (dsa_fused.py:640-703)."""
+    def forward(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None, checks: Optional[list] = None):
+        """-> ``(index_score_topk [s, topk], topk_indices [s, topk])`` (dsa_fused.py:640-703).  ``checks``: as with
+        ``DSAIndexerKernel``."""
+        late = {"checks": checks} if checks is not None and _takes_checks(self.indexer_kernel, DSAIndexerKernel) else {}
         chunkpipe = getattr(self.config, "enable_chunkpipe", False)
         rotate = getattr(self.config, "dsa_indexer_rotate_activation", True)
         front = self._fused_front_end(x, packed_seq_params)
@@ -426,7 +428,7 @@ class DSAIndexerFused(MegatronModule):
             return self.indexer_kernel(
                 q.contiguous(), k.squeeze(1).contiguous(), weights.squeeze(1).contiguous(), self.index_topk,
                 chunk_offset=self.pg_collection.tp.rank() * q.size(0), packed_seq_params=packed_seq_params,
-                rotate=bool(rotate), front=front, k_norm_weight=self.k_norm.weight, k_norm_bias=self.k_norm.bias)
+                rotate=bool(rotate), front=front, k_norm_weight=self.k_norm.weight, k_norm_bias=self.k_norm.bias, **late)
         # (with chunkpipe the cached keys are the rotated ones, so the rotation stays outside the kernel)
         fuse = (rotate and self.index_head_dim == 128
                 and x.is_cuda and not chunkpipe and getattr(self.indexer_kernel, "supports_fused_rotate", False))
@@ -450,6 +452,7 @@ class DSAIndexerFused(MegatronModule):
             chunk_offset=kv_offset,
             packed_seq_params=packed_seq_params,
             **({"rotate": True} if fuse else {}),
+            **late,
         )
 
 
@@ -516,6 +519,7 @@ class DSAttentionFused(MegatronModule):
         """query ``[sq, b, h, 576]`` (or ``[t, h, 576]`` packed), key ``[skv, b, 576]`` -> ``[b, sq, h, 512]``
         (``[t, h, 512]`` packed), with the indexer loss attached in training mode."""
         sq = query.size(0)
+        checks = []
         topk_holder = (
             get_dsa_index_share_topk_holder(packed_seq_params, index_share_carrier, self.skip_topk,
                                             self.layer_number, self.source_layer)
@@ -534,9 +538,10 @@ class DSAttentionFused(MegatronModule):
         else:
             x = x.detach()
             qr = qr.detach()
-            index_scores, topk_indices = self.indexer(x, qr, packed_seq_params=packed_seq_params)
-        if topk_holder is not None and not self.skip_topk:
-            topk_holder[self.layer_number] = topk_indices
+            # That the packed sequences hold every query is only known on the device.  The host does not wait for it behind the
+            # indexer, with 30 us of kernels in front of the device, but behind the attention and the loss.
+            late = {"checks": checks} if packed_seq_params is not None and _takes_checks(self.indexer, DSAIndexerFused) else {}
+            index_scores, topk_indices = self.indexer(x, qr, packed_seq_params=packed_seq_params, **late)
 
         chunk_query = query
         if self.num_attention_heads < self.num_attention_heads_padded:
@@ -576,6 +581,11 @@ class DSAttentionFused(MegatronModule):
             # softmax, F.kl_div(log(pred + 1e-10), target + 1e-10, "sum") and their backward in one kernel
             from . import ops
             loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10)
+        for check in checks:
+            check.wait()
+        if topk_holder is not None and not self.skip_topk:
+            topk_holder[self.layer_number] = topk_indices
+        if need_loss:
             indexer_loss = loss * (indexer_loss_coeff / sq) if sq else indexer_loss_coeff * loss / sq      # (one launch each way)
             if indexer_loss_coeff > 0:
                 DSAIndexerLossLoggingHelperFused.save_loss_to_tracker(

@@ -243,6 +243,11 @@ def _pad_to(x: Tensor, size: int, dim: int) -> Tensor:
     return torch.nn.functional.pad(x, pad)
 
 
+def _takes_checks(module, cls) -> bool:
+    """Whether ``module``'s forward is that of ``cls``, with its ``checks`` argument, and not a subclass's or a patched one."""
+    return getattr(getattr(module, "forward", None), "__func__", None) is cls.forward
+
+
 def _known_span(packed_seq_params) -> int:
     """The most keys that a query sees, 0 where the host does not know it."""
     longest = getattr(packed_seq_params, "max_seqlen_kv", None)
@@ -263,7 +268,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, index_q: Tensor, index_k: Tensor, weights: Tensor, index_topk: int, chunk_offset: int,
                 packed_seq_params: Optional[PackedSeqParams], rotate: bool = False, front: Optional["IndexerFrontEnd"] = None,
-                k_norm_weight: Optional[Tensor] = None, k_norm_bias: Optional[Tensor] = None):
+                k_norm_weight: Optional[Tensor] = None, k_norm_bias: Optional[Tensor] = None, checks: Optional[list] = None):
         assert index_q.ndim == 3 and index_k.ndim == 2 and weights.ndim == 2
         seq_q, head, dim = index_q.size()
         seq_k, _dim = index_k.size()
@@ -294,8 +299,6 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
         if whole is not None:
             index_score_topk, topk_indices, q_fp8, q_scale, weight_scaled, k_fp8, k_scale, covered = whole
             k_p = index_k.contiguous()
-            if covered is not None:
-                covered.wait()
         elif front is None and not rotate and (head != head_p or dim != 128) and ops.ordinary(index_q, index_k, weights):
             q_fp8, q_scale, weight_scaled = ops.quant_padded_e4m3(index_q, head_p, weights, softmax_scale)
             k_fp8, k_scale, _ = ops.quant_padded_e4m3(index_k.unsqueeze(1), 1)
@@ -322,7 +325,11 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
         if topk_indices is None:
             k_start, k_end, covered = ops.indexer_window(cu, seq_q, chunk_offset, q_fp8)
             index_score_topk, topk_indices = ops.indexer_topk(q_fp8, weight_scaled, k_fp8, k_scale, k_start, k_end, index_topk, sort)
-            covered.wait()
+        if covered is not None:
+            if checks is None:
+                covered.wait()
+            else:
+                checks.append(covered)
         ctx.softmax_scale = softmax_scale
         ctx.rotate = rotate
         ctx.index_topk = index_topk
@@ -340,7 +347,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_score, grad_topk):
         if grad_score is None:
-            return (None,) * 10
+            return (None,) * 11
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, topk_indices = ctx.saved_tensors
         head, dim = ctx.shape
         k_in, ln_w, ln_b = ctx.front_saved if ctx.front is not None else (None, None, None)
@@ -349,7 +356,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
             ctx.rotate, ctx.front, k_in, ln_w, ctx.span)
         if ctx.front is not None:
             d_ln_w, d_ln_b = d_ln_w.to(ln_w.dtype), d_ln_b.to(ln_b.dtype)
-        return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b
+        return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b, None
 
 
 @dataclass
@@ -378,12 +385,14 @@ class DSAIndexerKernel(torch.nn.Module):
     supports_fused_front_end = True
 
     def forward(self, index_q, index_k, weights, index_topk, chunk_offset, packed_seq_params, rotate=False,
-                front=None, k_norm_weight=None, k_norm_bias=None):
+                front=None, k_norm_weight=None, k_norm_bias=None, checks=None):
         """``front`` (an extension, :class:`IndexerFrontEnd`): ``index_q`` / ``index_k`` are the outputs of the
         projections and the key LayerNorm (``k_norm_weight``, ``k_norm_bias``), the rotary embedding and the rotation
-        run inside the quantiser kernels."""
+        run inside the quantiser kernels.  ``checks`` (an extension): a list that takes what is left to be checked on the
+        device (that the packed sequences hold every query) instead of waiting for it here; the caller calls ``wait()`` of its
+        entries once it has launched the work that it can launch."""
         return _apply(DSAIndexerKernelFunction, (index_q, index_k, weights, k_norm_weight, k_norm_bias), index_q, index_k, weights,
-                      index_topk, chunk_offset, packed_seq_params, rotate, front, k_norm_weight, k_norm_bias)
+                      index_topk, chunk_offset, packed_seq_params, rotate, front, k_norm_weight, k_norm_bias, checks)
 
 
 # ---------------------------------------------------------------------------------------------------

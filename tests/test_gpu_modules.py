@@ -198,6 +198,51 @@ def test_indexer_front_end_with_fused_rope_matches_the_torch_rope(gpu):
         fused.zero_grad()
 
 
+@pytest.mark.parametrize("patched,training", [(False, True), (False, False), (True, True)])
+def test_packed_sequences_that_do_not_hold_every_query_are_refused_by_the_module(gpu, patched, training):
+    """The check that is left to the device is waited for behind the attention, and still before the module returns, counts a loss
+    or publishes ids; an indexer whose forward is not the module's own waits itself."""
+    from loongforge_amd import dsa_fused
+    from loongforge_amd.megatron_compat import AttnMaskType, ModuleSpec, PackedSeqParams
+
+    S, H, Hi, Di, K, hid, qlr = 200, 32, 32, 128, 64, 96, 48
+    cfg = _cfg(num_attention_heads=H, hidden_size=hid, q_lora_rank=qlr, dsa_indexer_n_heads=Hi,
+               dsa_indexer_head_dim=Di, dsa_indexer_topk=K, dsa_indexer_loss_coeff=1.0, rope_type="rope",
+               rotary_percent=1.0, rotary_base=10000, init_method=None, layernorm_epsilon=1e-5,
+               dsa_indexer_rotate_activation=True, enable_chunkpipe=False, dsa_indexer_topk_freq=2,
+               dsa_indexer_skip_topk_offset=0, num_layers=2)
+    sub = dsa_fused.DSAttentionFusedSubmodules(indexer=ModuleSpec(
+        module=dsa_fused.DSAIndexerFused,
+        submodules=dsa_fused.DSAIndexerFusedSubmodules(linear_wq_b=_Linear, linear_wk=_Linear, k_norm=_Norm,
+                                                       linear_weights_proj=_Linear)))
+    torch.manual_seed(5)
+    mod = dsa_fused.DSAttentionFused(cfg, sub, layer_number=1, attn_mask_type=AttnMaskType.causal, attention_type="self",
+                                     k_channels=192)
+    for p in mod.parameters():
+        if p.ndim == 2:
+            torch.nn.init.normal_(p, std=p.shape[1] ** -0.5)
+    mod = mod.to(gpu).train(training)
+    if patched:
+        own = mod.indexer.forward
+        mod.indexer.forward = lambda x, qr, packed_seq_params=None: own(x, qr, packed_seq_params)
+    q, k = (torch.randn(*s, device=gpu, dtype=torch.bfloat16) for s in ((S, H, 576), (S, 576)))
+    x, qr = (torch.randn(S, n, device=gpu, dtype=torch.bfloat16) for n in (hid, qlr))
+
+    def call(ends):
+        cu = torch.tensor([0] + ends, dtype=torch.int32, device=gpu)
+        packed = PackedSeqParams(qkv_format="thd", cu_seqlens_q=cu, cu_seqlens_kv=cu, max_seqlen_q=S, max_seqlen_kv=S)
+        return mod(q, k, None, None, x=x, qr=qr, attn_mask_type=AttnMaskType.causal, packed_seq_params=packed, index_share_carrier=carrier)
+
+    tracker = dsa_fused.DSAIndexerLossLoggingHelperFused.tracker
+    carrier = SimpleNamespace()
+    tracker.clear()
+    with pytest.raises(ValueError, match="inconsistent shapes"):
+        call([90, S - 1])
+    assert not tracker and not getattr(carrier, "dsa_topk_holder", {})
+    carrier = SimpleNamespace()
+    assert torch.isfinite(call([90, S]).float()).all() and set(carrier.dsa_topk_holder) == {1}
+
+
 def test_index_share_second_layer_reuses_the_first_layers_topk(gpu):
     """dsa_indexer_topk_freq = 2 (dsa_fused.py:752-778, :839-878 of the reference): layer 1 owns an indexer
     and publishes its top-k ids in the carrier, layer 2 owns none and attends over layer 1's ids; only
