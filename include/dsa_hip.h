@@ -186,7 +186,7 @@ int dsa_indexer_bwd(const float* g, const void* q8, const void* k8, const float*
 
 /*
  * The same together with the way from the payload gradients back to the outputs of the projections: per row / scale
- * (rows on the quantiser's epsilon floor get 0), [Hadamard rotation], [bf16, transposed rotary embedding of the first 64
+ * (rows on the quantiser's epsilon floor get 0), [Hadamard rotation; rotate = 2 with dim = 64: of the 64 channels], [bf16, transposed rotary embedding of the first 64
  * channels: cos / sin [positions, 64], `pairing` as dsa_rope_rows or -1; the position of a query / key row is positions_q /
  * positions_k[row], or row / batch where that is NULL], for keys [LayerNorm backward with input k_in [Sk,128] bf16, weight
  * ln_w, into d_ln_w, d_ln_b [128]]; d_w = d_qw * q_scale * w_scale.  q8, q_w are padded to Hi heads and 128 channels:
@@ -226,6 +226,14 @@ int dsa_indexer_window(const void* cu, int cu_i64, int ncu, int S, int chunk_off
 int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void* k, int64_t k_rows, int rotate, void* q8, float* q_scale, void* k8,
                             float* k_scale, float eps, int pow2, const void* weights, int weights_bf16, float factor,
                             float* weight_scaled, int S, int64_t offset, int ratio, int keys, int32_t* ks, int32_t* ke, void* stream);
+/*
+ * The same for heads of 64 channels, all of them rotary, of bf16 q [S,heads,64] and k [keys,64]: rotary embedding (cos / sin bf16
+ * [positions,64], row i of queries and keys at position i, split pairs, every product and the sum rounded to bf16), Hadamard rotation
+ * of the 64, and dsa_quant_padded_e4m3 to heads_out heads and rows of 128; windows of one sequence (ratio 0).
+ */
+int dsa_indexer_narrow_e4m3(const void* q, int S, int heads, int heads_out, const void* k, int keys, const void* cos, const void* sin,
+                            int positions, void* q8, float* q_scale, void* k8, float* k_scale, const void* weights, int weights_bf16,
+                            float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke, void* stream);
 /*
  * Position of packed token t + offset inside its own sequence, t in [0, tokens) (0 past the last sequence).
  */

@@ -348,7 +348,7 @@ py::object indexer_bwd(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, c
 }
 
 py::tuple indexer_grads(const Tensor& g_, const Tensor& q8_, const Tensor& k8_, const Tensor& k_scale_, const Tensor& q_w_, const Tensor& ids_,
-                        const Tensor& q_scale_, double w_scale, bool rotate, const OptTensor& cos_, const OptTensor& sin_, int64_t pairing,
+                        const Tensor& q_scale_, double w_scale, int64_t rotate, const OptTensor& cos_, const OptTensor& sin_, int64_t pairing,
                         const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& k_in, const OptTensor& ln_w_,
                         double ln_eps, int64_t heads, int64_t dim, int64_t span, at::ScalarType q_type, at::ScalarType k_type, at::ScalarType w_type) {
   need_gpus(g_, q8_, k8_, k_scale_, q_w_, ids_, q_scale_, cos_, sin_, positions_q, positions_k, k_in, ln_w_);
@@ -487,6 +487,35 @@ py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weigh
   const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
       indexer_topk(q8, scaled, k8, k_scale, w.bounds.select(0, 0), w.bounds.select(0, 1), K, sort, false));
   return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale, w.check && w.check->done ? py::cast(std::move(w.check)) : py::none());
+}
+
+// indexer_forward for heads of 64 rotary channels behind their projections (q [S, heads, 64], k [Sk, 64] behind its norm; cos, sin bf16
+// [positions, 64]), padded on the way to 32 or 64 heads of 128 channels, one sequence.  -> (scores, ids, q8, q_scale, scaled
+// weights, k8, k_scale); None for other arguments.
+py::object indexer_forward_narrow(const Tensor& q, const Tensor& k, const Tensor& weights, const Tensor& cos, const Tensor& sin, double factor,
+                                  int64_t chunk_offset, int64_t K, bool sort) {
+  if (!plain(q, k, weights, cos, sin) || !q.is_cuda() || q.dim() != 3 || k.dim() != 2 || q.size(2) != 64 || k.size(1) != 64 || q.size(1) < 1 ||
+      q.size(1) > 64 || q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || weights.sizes() != q.sizes().slice(0, 2) ||
+      cos.scalar_type() != at::kBFloat16 || sin.scalar_type() != at::kBFloat16 || cos.numel() != sin.numel() || cos.numel() % 64) return py::none();
+  need_gpus(q, k, weights, cos, sin);
+  const int64_t S = q.size(0), heads = q.size(1), heads_out = heads <= 32 ? 32 : 64, Sk = k.size(0), positions = cos.numel() / 64;
+  if (positions < std::max(S, Sk)) return py::none();
+  auto lined = [](const Tensor& t) {           // a view may start inside a 16-byte piece
+    const Tensor x = t.contiguous();
+    return (uintptr_t)x.const_data_ptr() % 16 ? x.clone() : x;
+  };
+  const Tensor qc = lined(q), kc = lined(k), c = lined(cos), s = lined(sin);
+  const Tensor wc = weights.scalar_type() == at::kBFloat16 ? weights.contiguous() : f32(weights);
+  Call call(qc);
+  Tensor q8 = make({S, heads_out, 128}, at::kFloat8_e4m3fn, qc), q_scale = make({S, heads_out}, at::kFloat, qc), scaled = at::empty_like(q_scale);
+  Tensor k8 = make({Sk, 128}, at::kFloat8_e4m3fn, qc), k_scale = make({Sk}, at::kFloat, qc), bounds = make({2, S}, at::kInt, qc);
+  run("dsa_indexer_narrow_e4m3", dsa_indexer_narrow_e4m3, qc.const_data_ptr(), (int)S, (int)heads, (int)heads_out, kc.const_data_ptr(), (int)Sk,
+      c.const_data_ptr(), s.const_data_ptr(), (int)positions, out_ptr<void>(q8), out_ptr<float>(q_scale), out_ptr<void>(k8), out_ptr<float>(k_scale),
+      wc.const_data_ptr(), wc.scalar_type() == at::kBFloat16, (float)factor, out_ptr<float>(scaled), chunk_offset, out_ptr<int32_t>(bounds),
+      out_ptr<int32_t>(bounds) + S, call.stream);
+  const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
+      indexer_topk(q8, scaled, k8, k_scale, bounds.select(0, 0), bounds.select(0, 1), K, sort, false));
+  return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale);
 }
 
 py::object thd_positions(const Tensor& cu_, int64_t tokens, int64_t offset) {
@@ -764,6 +793,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(kl_loss);
   DEF(indexer_window);
   DEF(indexer_forward);
+  DEF(indexer_forward_narrow);
   DEF(thd_positions);
   DEF(absorb_into);
   DEF(absorb);

@@ -104,7 +104,7 @@ __device__ __forceinline__ void score_masks(const f32x16 (&acc)[NHT], bf16x8 (&m
 // rotation (its own transpose), bf16, transposed rotary embedding of the first 64 elements - the steps of the front
 // end backwards, rounding where the separate operations round.
 struct RowFinish {
-  int rotate;
+  int rotate;                            // 0 none, 1 of all 128 elements, 2 of the leading 64 (heads of 64 channels)
   const void* cos_t;
   const void* sin_t;
   int cs_f32, pairing, batch;            // pairing -1: no rotary part
@@ -127,14 +127,22 @@ __device__ __forceinline__ void finish_row(float (&v)[8], int sub, float scale_i
       for (int i = 0; i < 8; i++)
         if (!(i & m)) { const float a = v[i], b = v[i | m]; v[i] = a + b; v[i | m] = a - b; }
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1)
+    for (int m = 1; m < 8; m <<= 1)
 #pragma unroll
       for (int i = 0; i < 8; i++) {
         const float o = xor16(v[i], m);
         v[i] = (sub & m) ? o - v[i] : v[i] + o;
       }
+    if (f.rotate == 1) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] *= 0.08838834764831845f;
+      for (int i = 0; i < 8; i++) {
+        const float o = xor16(v[i], 8);
+        v[i] = (sub & 8) ? o - v[i] : v[i] + o;
+      }
+    }
+    const float norm = f.rotate == 1 ? 0.08838834764831845f : 0.125f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] *= norm;
   }
   if (f.pairing >= 0) {
 #pragma clang fp contract(off)
@@ -1373,7 +1381,7 @@ extern "C" int dsa_indexer_grads_span(const float* g, const void* q8, const void
   A.gsc = g; A.q8 = (const unsigned char*)q8; A.k8 = (const unsigned char*)k8; A.k_scale = k_scale; A.q_w = q_w; A.ids = ids;
   A.Sk = Sk; A.K = K;
   A.q_scale = q_scale; A.w_scale = w_scale;
-  A.fin = RowFinish{rotate, cos, sin, tables_f32, pairing, batch};
+  A.fin = RowFinish{rotate == 2 && dim == 64 ? 2 : rotate != 0, cos, sin, tables_f32, pairing, batch};
   A.pos_q = positions_q; A.heads = heads; A.dim = dim;
   A.d_q = d_q; A.q_f32 = q_f32; A.d_w = d_w; A.w_f32 = w_f32;
   KeyFinish kf = {};

@@ -225,6 +225,109 @@ __global__ __launch_bounds__(256) void quant_padded_kernel(const unsigned short*
   }
 }
 
+// The front end of 64-channel heads, all of them rotary, as quant_padded_kernel's rows of 128: rotary embedding (split pairs, every
+// product and the sum rounded to bf16, as the separate operations of rope_steps_kernel round), Hadamard rotation of 64 elements
+// (hadamard_kernel<64>), quantiser; keys (one head, behind their norm) and the windows of one sequence beside the queries in one
+// launch.  Six launches of 3 - 6 us, and four nodes of the graph each way, became this one, which 1024 tokens x 4 heads leave bound
+// by its launch; the payloads are the same bits.
+struct NarrowArgs {
+  const uint4 *q, *k;                      // [S, heads, 64], [keys, 64]
+  const uint4 *cos_t, *sin_t;              // [>= S, keys][64], bf16
+  int heads, heads_out;
+  int64_t q_rows, k_rows;                  // q_rows = S heads_out
+  uint2 *q8, *k8;
+  float *q_scale, *k_scale;
+  AnyWeight w_in;
+  float w_factor;
+  float* w_scaled;
+  unsigned q_blocks, k_blocks;
+  int S;
+  long long offset;
+  int *ks, *ke;
+};
+__global__ __launch_bounds__(256) void indexer_narrow_kernel(const NarrowArgs a) {
+#pragma clang fp contract(off)
+  if (blockIdx.x >= a.q_blocks + a.k_blocks) {
+    const int i = (int)(blockIdx.x - a.q_blocks - a.k_blocks) * 256 + (int)threadIdx.x;
+    if (i >= a.S) return;
+    a.ks[i] = 0;
+    a.ke[i] = (int)(a.offset + i + 1);
+    return;
+  }
+  const bool keys = blockIdx.x >= a.q_blocks;
+  const int64_t row = (int64_t)(blockIdx.x - (keys ? a.q_blocks : 0)) * 16 + (threadIdx.x >> 4);
+  const int sub = threadIdx.x & 15;
+  if (row >= (keys ? a.k_rows : a.q_rows)) return;         // (the 16 lanes of a row leave together)
+  const unsigned tok = keys ? (unsigned)row : (unsigned)row / (unsigned)a.heads_out, h = keys ? 0 : (unsigned)row % (unsigned)a.heads_out;
+  const bool real = keys || (int)h < a.heads;
+  float v[8], c[8], s[8];
+  auto load8 = [&](const uint4* p, int64_t i, float (&o)[8]) {
+    const uint4 raw = real && sub < 8 ? p[i] : make_uint4(0, 0, 0, 0);
+    const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      o[2 * e] = __builtin_bit_cast(float, w[e] << 16);
+      o[2 * e + 1] = __builtin_bit_cast(float, w[e] & 0xffff0000u);
+    }
+  };
+  load8(keys ? a.k : a.q, keys ? row * 8 + sub : ((int64_t)tok * a.heads + h) * 8 + sub, v);
+  load8(a.cos_t, (int64_t)tok * 8 + sub, c);
+  load8(a.sin_t, (int64_t)tok * 8 + sub, s);
+  auto round_bf16 = [](float (&t)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const unsigned u = cvt_pk_bf16(t[i], t[i + 1]);
+      t[i] = __builtin_bit_cast(float, u << 16);
+      t[i + 1] = __builtin_bit_cast(float, u & 0xffff0000u);
+    }
+  };
+  float o[8];                              // element e of lane s pairs with element e of lane s ^ 4
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    o[i] = xor16(v[i], 4);
+    o[i] = (sub < 4 ? -o[i] : o[i]) * s[i];
+    v[i] = v[i] * c[i];
+  }
+  round_bf16(v);
+  round_bf16(o);
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = v[i] + o[i];
+  round_bf16(v);
+#pragma unroll
+  for (int m = 1; m < 8; m <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      if (!(i & m)) { const float x = v[i], y = v[i | m]; v[i] = x + y; v[i | m] = x - y; }
+#pragma unroll
+  for (int m = 1; m < 8; m <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float x = xor16(v[i], m);
+      v[i] = (sub & m) ? x - v[i] : v[i] + x;
+    }
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = v[i] * 0.125f;
+  round_bf16(v);
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
+  amax = fmaxf(wave_max16(amax), 1e-12f);
+  const float scale = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, 448.0f / amax) & 0xff800000u);
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = fminf(fmaxf(v[i] * scale, -448.0f), 448.0f);
+  int lo = 0, hi = 0;
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], lo, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], hi, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
+  (keys ? a.k8 : a.q8)[row * 16 + sub] = make_uint2((unsigned)lo, (unsigned)hi);
+  if (sub == 0) {
+    const float si = 1.0f / scale;
+    (keys ? a.k_scale : a.q_scale)[row] = si;
+    if (!keys) a.w_scaled[row] = ((real ? a.w_in[(int64_t)tok * a.heads + h] : 0.f) * si) * a.w_factor;
+  }
+}
+
 // The indexer front end behind its projections, one pass over a 128-element row:
 //   LN    (key rows)  y = ((x - mean) * rstd) * gamma + beta, statistics in fp32, rounded to bf16
 //   ROPE              rotation of the leading 64 elements by the row's position (pairs adjacent or split,
@@ -404,6 +507,26 @@ extern "C" int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void
   if (rotate) indexer_inputs_kernel<true><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
   else indexer_inputs_kernel<false><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
   DSA_CHECK_LAUNCH("dsa_indexer_inputs_e4m3");
+  return DSA_OK;
+}
+
+extern "C" int dsa_indexer_narrow_e4m3(const void* q, int S, int heads, int heads_out, const void* k, int keys, const void* cos, const void* sin,
+                                       int positions, void* q8, float* q_scale, void* k8, float* k_scale, const void* weights, int weights_bf16,
+                                       float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke, void* stream) {
+  DSA_REQUIRE(S >= 0 && keys >= 0 && heads > 0 && heads <= heads_out && heads_out <= 64, "dsa_indexer_narrow_e4m3: bad sizes");
+  DSA_REQUIRE(positions >= S && positions >= keys, "dsa_indexer_narrow_e4m3: cos / sin tables are shorter than the sequence");
+  DSA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)cos % 16) == 0 && ((uintptr_t)sin % 16) == 0 &&
+              ((uintptr_t)q8 % 8) == 0 && ((uintptr_t)k8 % 8) == 0, "dsa_indexer_narrow_e4m3: misaligned pointer");
+  DSA_REQUIRE((S == 0 && keys == 0) || (cos && sin), "dsa_indexer_narrow_e4m3: null pointer");
+  DSA_REQUIRE(S == 0 || (q && q8 && q_scale && weights && weight_scaled && ks && ke), "dsa_indexer_narrow_e4m3: null pointer");
+  DSA_REQUIRE(keys == 0 || (k && k8 && k_scale), "dsa_indexer_narrow_e4m3: null pointer");
+  const int64_t q_rows = (int64_t)S * heads_out, q_blocks = (q_rows + 15) / 16, k_blocks = (keys + 15) / 16, blocks = q_blocks + k_blocks + dsa_cdiv(S, 256);
+  DSA_REQUIRE(q_rows < (1ll << 31), "dsa_indexer_narrow_e4m3: too many rows");
+  if (blocks == 0) return DSA_OK;
+  const NarrowArgs a{(const uint4*)q, (const uint4*)k, (const uint4*)cos, (const uint4*)sin, heads, heads_out, q_rows, keys, (uint2*)q8, (uint2*)k8,
+                     q_scale, k_scale, {weights, weights_bf16 != 0}, factor, weight_scaled, (unsigned)q_blocks, (unsigned)k_blocks, S, offset, ks, ke};
+  indexer_narrow_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
+  DSA_CHECK_LAUNCH("dsa_indexer_narrow_e4m3");
   return DSA_OK;
 }
 

@@ -25,6 +25,7 @@ from typing import Optional, Tuple, Union
 import torch
 import torch.nn.functional as F
 
+from . import megatron_compat as _compat
 from .dsa_fused_kernels import DSADotProductAttention, DSAIndexerKernel, _takes_checks, triton_attn_dist
 from .megatron_compat import (
     AttnMaskType,
@@ -321,10 +322,20 @@ class DSAIndexerFused(MegatronModule):
                                     mscale=mscale, cp_group=self.pg_collection.cp)
         return x_pe if all_rotary else torch.cat([x_pe, x[..., self.qk_pos_emb_head_dim:]], dim=-1)
 
+    def _projections(self, x, qr):
+        """q ``[s, (b,) h, d]``, k behind its norm and weights, before the rotary embedding."""
+        x, qr = x.detach(), qr.detach()
+        q, _ = self.linear_wq_b(qr)
+        q = q.view(*q.size()[:-1], self.index_n_heads, self.index_head_dim)
+        k, _ = self.linear_wk(x)
+        weights, _ = self.linear_weights_proj(x)
+        return q, self.k_norm(k), weights * self.index_n_heads ** -0.5
+
     def get_query_key_weight_tensors(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None,
-                                     defer_rotation: bool = False):
+                                     defer_rotation: bool = False, projected=None):
         """q ``[s, (b,) h, d]``, k ``[s, (b,) d]``, weights ``[s, (b,) h]`` (dsa_fused.py:490-638).
-        ``defer_rotation`` leaves the Hadamard rotation to the caller (the indexer kernel fuses it)."""
+        ``defer_rotation`` leaves the Hadamard rotation to the caller (the indexer kernel fuses it); ``projected``: what
+        ``_projections`` returned, where the caller has called it."""
         x = x.detach()
         qr = qr.detach()
         rotary_seq_len = self.rotary_pos_emb.get_rotary_seq_len(None, None, x, self.config, packed_seq_params)
@@ -350,12 +361,8 @@ class DSAIndexerFused(MegatronModule):
         else:
             cu_seqlens_q = cu_seqlens_kv = None
 
-        q, _ = self.linear_wq_b(qr)
-        q = q.view(*q.size()[:-1], self.index_n_heads, self.index_head_dim)
+        q, k, weights = self._projections(x, qr) if projected is None else projected
         q = self._apply_rope(q, rotary_pos_emb, mscale, cu_seqlens_q, cos, sin)
-
-        k, _ = self.linear_wk(x)
-        k = self.k_norm(k)
         if packed_seq_params is None:
             k = k.unsqueeze(-2)
             k = self._apply_rope(k, rotary_pos_emb, mscale, cu_seqlens_kv, cos, sin)
@@ -372,9 +379,6 @@ class DSAIndexerFused(MegatronModule):
             # this chunk's own key gradient (dsa_fused.py:606-622)
             pos, last = self._chunk_position()[1], self.num_chunks_per_seq - 1
             k.register_hook(lambda g: g if pos == last else g + self._chunk_slab.grads.pop(pos))
-
-        weights, _ = self.linear_weights_proj(x)
-        weights = weights * self.index_n_heads ** -0.5
         return q, k, weights
 
     def _fused_front_end(self, x, packed_seq_params):
@@ -408,6 +412,25 @@ class DSAIndexerFused(MegatronModule):
                                positions_k=pos_k, batch=1 if packed_seq_params is not None else x.shape[1],
                                k_norm_eps=float(k_norm.eps))
 
+    def _narrow_tables(self, x, packed_seq_params):
+        """bf16 ``(cos, sin)`` for :class:`DSAIndexerKernel`'s ``rotary_tables``, or None: heads of 64 channels that are rotary
+        throughout (split pairs) and rotated, one unpacked sequence on the device, no fused rotary path and no chunkpipe (its key
+        cache holds finished keys), and this file's own steps between the projections and the kernel."""
+        cfg = self.config
+        if not (self.index_head_dim == 64 == self.qk_pos_emb_head_dim and self.index_n_heads <= 64 and x.is_cuda and x.dtype == torch.bfloat16
+                and x.ndim == 3 and x.shape[1] == 1 and packed_seq_params is None and not getattr(cfg, "apply_rope_fusion", False)
+                and getattr(cfg, "dsa_indexer_rotate_activation", True) and not getattr(cfg, "dsa_indexer_rope_interleaved", False)
+                and not getattr(cfg, "enable_chunkpipe", False) and type(self.rotary_pos_emb) is RotaryEmbedding
+                and RotaryEmbedding is _compat.RotaryEmbedding and apply_rotary_pos_emb is _compat.apply_rotary_pos_emb
+                and _takes_checks(self.indexer_kernel, DSAIndexerKernel)
+                and all(getattr(getattr(self, name), "__func__", None) is getattr(DSAIndexerFused, name)
+                        for name in ("_apply_rope", "get_query_key_weight_tensors"))):
+            return None
+        from . import ops
+
+        tables = self.rotary_pos_emb.get_cached_cos_sin(x.shape[0], dtype=torch.bfloat16) if ops.ordinary(x) else None
+        return tables if tables is not None and tables[0].shape[-1] == 64 and ops.ordinary(*tables) else None
+
     def forward(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None, checks: Optional[list] = None):
         """-> ``(index_score_topk [s, topk], topk_indices [s, topk])`` (dsa_fused.py:640-703).  ``checks``: as with
         ``DSAIndexerKernel``."""
@@ -429,11 +452,21 @@ class DSAIndexerFused(MegatronModule):
                 q.contiguous(), k.squeeze(1).contiguous(), weights.squeeze(1).contiguous(), self.index_topk,
                 chunk_offset=self.pg_collection.tp.rank() * q.size(0), packed_seq_params=packed_seq_params,
                 rotate=bool(rotate), front=front, k_norm_weight=self.k_norm.weight, k_norm_bias=self.k_norm.bias, **late)
+        tables, projected = self._narrow_tables(x, packed_seq_params), None
+        if tables is not None:
+            from . import ops
+
+            projected = q, k, weights = self._projections(x, qr)
+            if q.dtype == k.dtype == torch.bfloat16 and ops.ordinary(q, k, weights):
+                return self.indexer_kernel(q.squeeze(1), k.squeeze(1), weights.squeeze(1), self.index_topk,
+                                           chunk_offset=self.pg_collection.tp.rank() * q.size(0), packed_seq_params=None,
+                                           rotary_tables=tables, **late)
         # (with chunkpipe the cached keys are the rotated ones, so the rotation stays outside the kernel)
         fuse = (rotate and self.index_head_dim == 128
                 and x.is_cuda and not chunkpipe and getattr(self.indexer_kernel, "supports_fused_rotate", False))
         indexer_query, indexer_key, indexer_weights = self.get_query_key_weight_tensors(x, qr, packed_seq_params,
-                                                                                        defer_rotation=fuse)
+                                                                                        defer_rotation=fuse,
+                                                                                        **({} if projected is None else {"projected": projected}))
         if packed_seq_params is None:
             indexer_query = indexer_query.squeeze(1).contiguous()
         indexer_key = indexer_key.squeeze(1).contiguous()

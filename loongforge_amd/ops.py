@@ -347,14 +347,20 @@ def indexer_bwd(g, q8, k8, k_scale, q_w, ids):
 
 
 def indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale: float, heads: int, dim: int, dtypes, rotate: bool = False,
-                  front=None, k_in=None, ln_weight=None, span: int = 0):
+                  front=None, k_in=None, ln_weight=None, span: int = 0, narrow=None):
     """:func:`indexer_bwd` carried on to the outputs of the projections: ``(d_q [S, heads, dim], d_k [Sk, dim], d_weights
     [S, heads], d_ln_weight, d_ln_bias)`` in ``dtypes`` (of q, k, weights), the last two fp32 or None.  Unscaled (rows on the
     quantiser's epsilon floor, loongforge/models/foundation/deepseek_v4/deepseek_v4_csa.py:1525-1541, get zero), back
     through the Hadamard rotation if ``rotate``, and with ``front`` (an ``IndexerFrontEnd``) through the rotary embedding
     and the LayerNorm of the keys (input ``k_in``, weight ``ln_weight``).  ``span``: the most neighbouring keys that a query
-    sees, 0 if that is not known; it decides how the keys' gradients are summed, not what they are."""
+    sees, 0 if that is not known; it decides how the keys' gradients are summed, not what they are.  ``narrow``: the
+    ``(cos, sin)`` of :func:`indexer_forward_narrow`."""
     f = front
+    if narrow is not None:
+        if not ordinary(g, q8, k8, k_scale, q_w, ids, q_scale, *narrow):
+            return _indexer_grads_narrow(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, *narrow)
+        return _native().indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, float(w_scale), 2, *narrow, ROPE_SPLIT, None, None, 1, None, None,
+                                       0.0, int(heads), int(dim), int(span), *dtypes)
     if f is None and not ordinary(g, q8, k8, k_scale, q_w, ids, q_scale):
         return _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, rotate)
     return _native().indexer_grads(g, q8, k8, k_scale, q_w, ids, q_scale, float(w_scale), bool(rotate), f and f.cos, f and f.sin,
@@ -374,6 +380,23 @@ def _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, head
         h = _hadamard(128, d_q.device, torch.float32)
         d_q, d_k = (d_q @ h) * 128 ** -0.5, (d_k @ h) * 128 ** -0.5
     return d_q[:, :heads, :dim].to(dtypes[0]), d_k[:, :dim].to(dtypes[1]), d_w[:, :heads].to(dtypes[2]), None, None
+
+
+def _indexer_grads_narrow(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim, dtypes, cos, sin):
+    """:func:`indexer_grads` of :func:`indexer_forward_narrow` as tensor operations, for traced and batched tensors."""
+    from .dsa_fused import _hadamard
+
+    d_q, d_k, d_w, _, _ = _indexer_grads_composed(g, q8, k8, k_scale, q_w, ids, q_scale, w_scale, heads, dim,
+                                                  (torch.float32, torch.float32, dtypes[2]), False)
+
+    def back(d, dtype, c, s):
+        d = ((d @ _hadamard(dim, d.device, torch.float32)) * dim ** -0.5).to(torch.bfloat16)
+        u, half = d.float() * s, dim // 2
+        return (d.float() * c + torch.cat((u[..., half:], -u[..., :half]), dim=-1)).to(dtype)
+
+    c, s = cos.reshape(-1, dim).float(), sin.reshape(-1, dim).float()
+    S, Sk = q8.shape[0], k8.shape[0]
+    return back(d_q, dtypes[0], c[:S, None], s[:S, None]), back(d_k, dtypes[1], c[:Sk], s[:Sk]), d_w, None, None
 
 
 class _Unchecked:
@@ -411,6 +434,14 @@ def indexer_forward(index_q, index_k, weights, rotate: bool, factor: float, cu_s
     return _native().indexer_forward(index_q, index_k, weights, bool(rotate), float(factor), cu_seqlens, int(chunk_offset), int(K), bool(sorted),
                                      f and f.cos, f and f.sin, f.pairing if f else -1, f and f.positions_q, f and f.positions_k,
                                      f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0, int(ratio))
+
+
+def indexer_forward_narrow(index_q, index_k, weights, cos, sin, factor: float, chunk_offset: int, K: int, sorted: bool):
+    """:func:`indexer_forward` over one sequence for bf16 ``index_q [S, <= 64, 64]`` and ``index_k [Sk, 64]`` that still need their
+    rotary embedding (bf16 ``cos`` / ``sin [positions, .., 64]``, every channel rotary, split pairs, rounded like
+    :func:`rope_steps`) and their Hadamard rotation: (scores, ids, q8, q_scale, scaled weights, k8, k_scale), padded to
+    32 or 64 heads of 128; None for arguments it does not take."""
+    return _native().indexer_forward_narrow(index_q, index_k, weights, cos, sin, float(factor), int(chunk_offset), int(K), bool(sorted))
 
 
 # --------------------------------------------------------------------------------------------

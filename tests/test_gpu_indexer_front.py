@@ -315,3 +315,78 @@ def test_separate_operations_under_transforms(gpu, interleaved):
         torch.testing.assert_close(tangent, f(v), **near)
     odd = rnd(4 * 64 + 1)[1:].view(4, 64)
     assert torch.equal(rotate_activation(odd), rotate_activation(odd.clone()))
+
+
+@pytest.mark.parametrize("S,Sk,heads,bf16_weights", [(1, 1, 1, True), (15, 15, 4, True), (17, 17, 32, False), (257, 300, 33, True), (1030, 1030, 64, False)])
+def test_narrow_heads_in_one_kernel_are_those_of_the_separate_kernels(gpu, S, Sk, heads, bf16_weights):
+    """Rotary embedding in rounded steps, rotation, padded quantisers and windows of 64-channel heads: the same bits in one launch, also
+    for views that do not start on 16 bytes or do not lie in order; finished gradients against the same steps in 32 bits, each rounded
+    to bf16 once (2^-8 relative each)."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(S + heads)
+    K, factor, offset = 64, 64 ** -0.5, Sk - S
+    q = torch.randn(S * heads * 64 + 1, generator=g).to(gpu, torch.bfloat16)[1:].view(S, heads, 64)
+    k = torch.randn(64, Sk, generator=g).to(gpu, torch.bfloat16).t()
+    w = torch.randn(S, heads, generator=g).to(gpu, torch.bfloat16 if bf16_weights else torch.float32)
+    q[S // 2] = 0.0
+    inv_freq = (10000.0 ** (-torch.arange(0, 64, 2, dtype=torch.float32) / 64)).to(gpu)
+    angles = ops.rotary_angles(inv_freq, Sk)
+    cos, sin = ops.rotary_cos_sin(inv_freq, Sk, 0.0, torch.bfloat16)
+    scores, ids, q8, q_scale, scaled, k8, k_scale = ops.indexer_forward_narrow(q, k, w, cos, sin, factor, offset, K, True)
+    qr = ops.hadamard(ops.rope_steps(q.contiguous(), angles))
+    kr = ops.hadamard(ops.rope_steps(k.contiguous().unsqueeze(1), angles))
+    want_q = ops.quant_padded_e4m3(qr, 32 if heads <= 32 else 64, w, factor)
+    want_k = ops.quant_padded_e4m3(kr, 1)
+    for a, b in zip((q8.view(torch.uint8), q_scale, scaled, k8.view(torch.uint8), k_scale),
+                    (want_q[0].view(torch.uint8), want_q[1], want_q[2], want_k[0].squeeze(1).view(torch.uint8), want_k[1].squeeze(1))):
+        assert torch.equal(a, b)
+    ks, ke, _ = ops.indexer_window(None, S, offset, q8)
+    want = ops.indexer_topk(q8, scaled, k8, k_scale, ks, ke, K)
+    assert torch.equal(scores, want[0]) and torch.equal(ids, want[1])
+    grad = torch.randn(S, K, generator=g).to(gpu) * (ids >= 0)
+    args = (grad, q8, k8, k_scale, scaled, ids, q_scale, factor, heads, 64)
+    got = ops.indexer_grads(*args, (torch.float32,) * 3, narrow=[cos, sin])
+    ref = ops._indexer_grads_narrow(*args, (torch.float32,) * 3, cos, sin)
+    for a, b in zip(got[:3], ref[:3]):
+        assert a.shape == b.shape
+        assert (a - b).norm().item() <= 2.0 ** -7 * b.norm().item() + 1e-12
+    assert ops.indexer_forward_narrow(q, k, w, cos[:Sk - 1], sin[:Sk - 1], factor, offset, K, True) is None
+
+
+@pytest.mark.parametrize("S,heads", [(1, 4), (129, 4), (1024, 40)])
+def test_indexer_module_of_narrow_heads_in_one_kernel(gpu, S, heads):
+    """DSAIndexerFused with 64-channel heads: the same scores and ids as with the separate operations, gradients of its
+    projections and its norm within the bf16 roundings that the one kernel leaves out."""
+    from types import SimpleNamespace
+
+    from loongforge_amd import dsa_fused
+
+    hid, qlr, K = 96, 48, 64
+    cfg = SimpleNamespace(qk_pos_emb_head_dim=64, apply_rope_fusion=False, hidden_size=hid, q_lora_rank=qlr, dsa_indexer_n_heads=heads,
+                          dsa_indexer_head_dim=64, dsa_indexer_topk=K, rope_type="rope", rotary_percent=1.0, rotary_base=10000, init_method=None,
+                          layernorm_epsilon=1e-5, dsa_indexer_rotate_activation=True, enable_chunkpipe=False)
+    sub = dsa_fused.DSAIndexerFusedSubmodules(linear_wq_b=_Linear, linear_wk=_Linear, k_norm=_Norm, linear_weights_proj=_Linear)
+    torch.manual_seed(5)
+    mod = dsa_fused.DSAIndexerFused(cfg, sub)
+    for p in mod.parameters():
+        if p.ndim == 2:
+            torch.nn.init.normal_(p, std=p.shape[1] ** -0.5)
+    mod = mod.to(gpu)
+    g = torch.Generator().manual_seed(6)
+    x, qr = torch.randn(S, 1, hid, generator=g).to(gpu, torch.bfloat16), torch.randn(S, 1, qlr, generator=g).to(gpu, torch.bfloat16)
+    grad = torch.randn(S, K, generator=g).to(gpu)
+
+    def passes():
+        scores, ids = mod(x, qr)
+        return scores.detach(), ids, torch.autograd.grad(scores, list(mod.parameters()), grad * (ids >= 0))
+
+    assert mod._narrow_tables(x, None) is not None
+    narrow = passes()
+    mod._apply_rope = lambda *a: dsa_fused.DSAIndexerFused._apply_rope(mod, *a)        # not the class's own: the separate operations
+    assert mod._narrow_tables(x, None) is None
+    apart = passes()
+    assert torch.equal(narrow[0], apart[0]) and torch.equal(narrow[1], apart[1])
+    for a, b in zip(narrow[2], apart[2]):
+        # three bf16 roundings each way, and the one of the result
+        assert (a - b).float().norm().item() <= 2.0 ** -6 * b.float().norm().item() + 1e-6
