@@ -337,6 +337,13 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const void* out, const voi
                        const int32_t* ids, const float* lse, int S, int H, int Skv, int K,
                        int q_start, float sm_scale, int d_v, void* dq, void* dkv,
                        void* workspace, size_t workspace_bytes, void* stream);
+/* The same where only the first dq_heads heads are real: dq is [S, dq_heads, 576]. */
+int dsa_sparse_mla_bwd_heads(const void* q, const void* kv, const void* out, const void* dout,
+                             const int32_t* ids, const float* lse, int S, int H, int dq_heads, int Skv, int K,
+                             int q_start, float sm_scale, int d_v, void* dq, void* dkv,
+                             void* workspace, size_t workspace_bytes, void* stream);
+/* src [tokens, heads, row_bytes] -> dst [tokens, heads_out, row_bytes], zeros behind the heads (rows of a multiple of 16 bytes). */
+int dsa_pad_heads(const void* src, int tokens, int heads, int heads_out, int row_bytes, void* dst, void* stream);
 /*
  * How the backward goes about a call of these sizes and this workspace, for tests and measurements: how many consecutive queries
  * make a group that may be worked as one query (1: none).  If more than one, *units_offset is where in its workspace the call leaves

@@ -591,22 +591,41 @@ py::object mla_fwd_dist(const Tensor& q_, const Tensor& kv_, const Tensor& ids_,
   return py::make_tuple(out, lse, dist);
 }
 
+// bf16 [S, h, width] -> [S, heads, width] with zeros behind
+Tensor with_zero_heads(const Tensor& x_, int64_t heads) {
+  Tensor x = x_.contiguous();
+  if ((uintptr_t)x.const_data_ptr() % 16) x = x.clone();        // a view that starts inside a 16-byte piece
+  Call call(x);
+  Tensor y = make({x.size(0), heads, x.size(2)}, at::kBFloat16, x);
+  run("dsa_pad_heads", dsa_pad_heads, x.const_data_ptr(), (int)x.size(0), (int)x.size(1), (int)heads, (int)x.size(2) * 2, out_ptr<void>(y), call.stream);
+  return y;
+}
+py::object pad_heads(const Tensor& x, int64_t heads) {
+  if (!plain(x) || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || x.dim() != 3 || x.size(2) % 8 || x.size(2) > 32768 || x.size(1) < 1 ||
+      x.size(1) > heads || heads > 1024 || x.size(2) < 1) return py::none();
+  need_gpus(x);
+  return py::cast(with_zero_heads(x, heads));
+}
+
 py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, const Tensor& dout_, const Tensor& ids_, const Tensor& lse_,
-                   int64_t q_start, double sm_scale, int64_t d_v, const py::function& workspace, bool force) {
+                   int64_t q_start, double sm_scale, int64_t d_v, int64_t heads, const py::function& workspace, bool force) {
   PLAIN_OR_NONE(q_, kv_, out_, dout_, ids_, lse_);
   mla_shape(q_, kv_, ids_);
   need_gpus(q_, out_, dout_, lse_);
   const Tensor q = q_.contiguous(), kv = kv_.contiguous(), ids = i32(ids_), out = out_.contiguous(), lse = f32(lse_);
-  const Tensor dout = dout_.to(at::kBFloat16).contiguous();
   const int64_t S = q.size(0), H = q.size(1), K = ids.size(1), Skv = kv.size(0);
+  const bool some = heads > 0 && heads < H;          // only the first heads are real: dout has theirs, and dq
+  REQUIRE(!some || dout_.sizes() == at::IntArrayRef({S, heads, d_v}), "sparse_mla_bwd: dout must be [S,heads,d_v]");
+  Tensor dout = dout_.to(at::kBFloat16).contiguous();
+  if (some) dout = with_zero_heads(dout, H);
   REQUIRE(out.sizes() == at::IntArrayRef({S, H, d_v}) && dout.sizes() == out.sizes() && lse.sizes() == at::IntArrayRef({S, H}),
           "sparse_mla_bwd: out/dout must be [S,H,d_v] and lse [S,H]");
-  Tensor dq = at::empty_like(q), dkv = at::empty_like(kv);
+  Tensor dq = some ? make({S, heads, 576}, at::kBFloat16, q) : at::empty_like(q), dkv = at::empty_like(kv);
   const size_t full = dsa_sparse_mla_bwd_workspace_bytes((int)S, (int)H, (int)Skv, (int)K);
   const auto [ws, nbytes] = py::cast<std::pair<Tensor, size_t>>(workspace(full, q.device()));
   Call call(q);
-  run("dsa_sparse_mla_bwd", dsa_sparse_mla_bwd, q.const_data_ptr(), kv.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
-      (const int32_t*)ids.const_data_ptr(), (const float*)lse.const_data_ptr(), (int)S, (int)H, (int)Skv, (int)K, (int)q_start, (float)sm_scale,
+  run("dsa_sparse_mla_bwd", dsa_sparse_mla_bwd_heads, q.const_data_ptr(), kv.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
+      (const int32_t*)ids.const_data_ptr(), (const float*)lse.const_data_ptr(), (int)S, (int)H, (int)(some ? heads : H), (int)Skv, (int)K, (int)q_start, (float)sm_scale,
       (int)d_v, dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), nbytes, call.stream);
   return py::make_tuple(dq, dkv);
 }
@@ -788,6 +807,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(indexer_grads);
   DEF(mla_fwd);
   DEF(mla_fwd_dist);
+  DEF(pad_heads);
   DEF(mla_bwd);
   DEF(attn_dist);
   DEF(kl_loss);

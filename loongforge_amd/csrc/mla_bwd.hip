@@ -91,11 +91,12 @@ __device__ __forceinline__ void stage_unit(const int* __restrict__ list, int n, 
 // With up to 64 heads a wave owns its 3 d-tiles for head group hp only; with up to 32, for one k-step (16 keys) of the only
 // head group, and the two k-steps' sums are added at the end.
 constexpr int DQ_THREADS = 768;
-// ids, pds, dq: the query's (UNIT: the joint unit's) slots, dS tiles and rows of dQ; qpos: its position
+// ids, pds, dq: the query's (UNIT: the joint unit's) slots, dS tiles and rows of dQ; qpos: its position; of every `per` heads the first
+// `real` have a row in dq
 template <int STAGES, int HG, bool UNIT>
 __device__ __forceinline__ void dq_body(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, int H, int Skv, int K, int qpos, const int* __restrict__ dup_flag,
+    __bf16* __restrict__ dq, int H, int per, int real, int Skv, int K, int qpos, const int* __restrict__ dup_flag,
     unsigned char* smem) {
   constexpr int STAGE_BYTES = TILE_BYTES + pds_kind_bytes(HG);
   constexpr int NJ = HG == 4 ? 2 : 1;          // head groups of a wave
@@ -251,12 +252,15 @@ __device__ __forceinline__ void dq_body(
     const int dt = 3 * dg + u / NJ;
     const int h = (hg0 + u % NJ) * 32 + r;
     if (h < H) {                               // the same for all lanes of a wave (H is a multiple of 32)
-      unsigned short* op = (unsigned short*)dq + (size_t)h * DQK + 32 * dt + 8 * g;
+      const int query = UNIT ? h / per : 0, own = UNIT ? h % per : h;
+      unsigned short* op = (unsigned short*)dq + (size_t)(query * real + own) * DQK + 32 * dt + 8 * g;
       uint4 o[2];
       acc_row_to_16B(acc[u], 1.0f, o);
       if (poison) o[0] = o[1] = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
-      *(uint4*)op = o[0];
-      *(uint4*)(op + 16) = o[1];
+      if (own < real) {
+        *(uint4*)op = o[0];
+        *(uint4*)(op + 16) = o[1];
+      }
     }
   }
 }
@@ -1229,7 +1233,7 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
 template <int HG, int G>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, const int* __restrict__ work, size_t group_pds, int q0, int cnt, int H, int Skv, int K, int q_start,
+    __bf16* __restrict__ dq, const int* __restrict__ work, size_t group_pds, int q0, int cnt, int H, int real, int Skv, int K, int q_start,
     const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
     float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -1239,16 +1243,16 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const int ql = w.query;
     if (G > 1 && ql < 0) return;
     const int* list = ids + (size_t)ql * K;
-    __bf16* dq_rows = dq + (size_t)(q0 + ql) * H * DQK;
+    __bf16* dq_rows = dq + (size_t)(q0 + ql) * real * DQK;
     const unsigned char* own = pds + (size_t)(ql / G) * group_pds;
     if constexpr (G > 1) {
       if (w.tiles > 0) {
-        dq_body<3, 4, true>(kv, list, own, dq_rows, 128, Skv, 32 * w.tiles, 0, dup_flag, smem);
+        dq_body<3, 4, true>(kv, list, own, dq_rows, 128, 128 / G, real, Skv, 32 * w.tiles, 0, dup_flag, smem);
         return;
       }
       own += (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
     }
-    dq_body<3, HG, false>(kv, list, own, dq_rows, H, Skv, K, q_start + q0 + ql, dup_flag, smem);
+    dq_body<3, HG, false>(kv, list, own, dq_rows, H, H, real, Skv, K, q_start + q0 + ql, dup_flag, smem);
   } else {
     // longest work first: from the first key on where the first half of the keys has most of the rows (causal windows), else
     // from the last key (compressed keys behind a sliding window)
@@ -1386,11 +1390,12 @@ extern "C" int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t wo
 }
 
 static int bwd_impl(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
-                    const float* lse, int S, int H, int Skv, int K, int q_start, float sm_scale, int d_v,
+                    const float* lse, int S, int H, int dq_heads, int Skv, int K, int q_start, float sm_scale, int d_v,
                     void* dq, void* dkv, void* workspace, size_t workspace_bytes, void* stream, float* pass_ms) {
   DSA_REQUIRE(d_v == DV, "dsa_sparse_mla_bwd: only d_v = 512 (d_qk = 576) is supported, got d_v = %d", d_v);
   DSA_REQUIRE(S >= 0 && Skv > 0, "dsa_sparse_mla_bwd: bad sequence sizes S=%d Skv=%d", S, Skv);
   DSA_REQUIRE(H > 0 && H <= 128 && H % 32 == 0, "dsa_sparse_mla_bwd: head count must be 32, 64, 96 or 128, got %d", H);
+  DSA_REQUIRE(dq_heads > 0 && dq_heads <= H, "dsa_sparse_mla_bwd: gradients of %d heads of %d", dq_heads, H);
   DSA_REQUIRE(K > 0 && K % 64 == 0 && K <= 2048, "dsa_sparse_mla_bwd: top-k must be a multiple of 64 up to 2048, got %d", K);
   DSA_REQUIRE((size_t)Skv * DQK * 2 <= 0xffffffffull, "dsa_sparse_mla_bwd: kv larger than 4 GiB is not supported");
   DSA_REQUIRE(Skv <= order::MAX_KEYS, "dsa_sparse_mla_bwd: at most %d keys are supported, got %d", order::MAX_KEYS, Skv);
@@ -1472,7 +1477,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, work, group_pds, q0, cnt, H, Skv,
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, work, group_pds, q0, cnt, H, dq_heads, Skv,
                                                                    K, q_start, dup_flag, rows, exps, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");
@@ -1488,7 +1493,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   }
   if (S == 0 || S > p.chunk) cast_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>(acc, (unsigned short*)dkv, (size_t)Skv * DQK, dup_flag);
   if (S > p.chunk)      // more than one chunk: the flag may have come up after earlier chunks wrote their dQ
-    poison_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>((unsigned short*)dq, (size_t)S * H * DQK, dup_flag);
+    poison_bf16_kernel<<<dim3(2048), dim3(256), 0, st>>>((unsigned short*)dq, (size_t)S * dq_heads * DQK, dup_flag);
   DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(cast)");
   if (pass_ms) for (int i = 0; i < 4; i++) hipEventDestroy(ev[i]);
 #undef DSA_MARK
@@ -1498,7 +1503,14 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
 extern "C" int dsa_sparse_mla_bwd(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
                                   const float* lse, int S, int H, int Skv, int K, int q_start, float sm_scale, int d_v,
                                   void* dq, void* dkv, void* workspace, size_t workspace_bytes, void* stream) {
-  return bwd_impl(q, kv, out, dout, ids, lse, S, H, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
+  return bwd_impl(q, kv, out, dout, ids, lse, S, H, H, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
+                  stream, nullptr);
+}
+
+extern "C" int dsa_sparse_mla_bwd_heads(const void* q, const void* kv, const void* out, const void* dout, const int32_t* ids,
+                                        const float* lse, int S, int H, int dq_heads, int Skv, int K, int q_start, float sm_scale, int d_v,
+                                        void* dq, void* dkv, void* workspace, size_t workspace_bytes, void* stream) {
+  return bwd_impl(q, kv, out, dout, ids, lse, S, H, dq_heads, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
                   stream, nullptr);
 }
 
@@ -1508,7 +1520,7 @@ extern "C" int dsa_sparse_mla_bwd_profile(const void* q, const void* kv, const v
                                           float sm_scale, int d_v, void* dq, void* dkv, void* workspace,
                                           size_t workspace_bytes, void* stream, float* pass_ms) {
   DSA_REQUIRE(pass_ms != nullptr, "dsa_sparse_mla_bwd_profile: pass_ms must point at 3 floats");
-  return bwd_impl(q, kv, out, dout, ids, lse, S, H, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
+  return bwd_impl(q, kv, out, dout, ids, lse, S, H, H, Skv, K, q_start, sm_scale, d_v, dq, dkv, workspace, workspace_bytes,
                   stream, pass_ms);
 }
 #endif

@@ -577,7 +577,10 @@ class DSAttentionFused(MegatronModule):
             index_scores, topk_indices = self.indexer(x, qr, packed_seq_params=packed_seq_params, **late)
 
         chunk_query = query
-        if self.num_attention_heads < self.num_attention_heads_padded:
+        padded, inside = self.num_attention_heads < self.num_attention_heads_padded, {}
+        if padded and query.size(-2) == self.num_attention_heads and _takes_checks(self.sparse_attention, DSADotProductAttention):
+            padded, inside = False, {"padded_heads": self.num_attention_heads_padded}       # inside the attention: fewer launches and nodes
+        if padded:
             pad_size = self.num_attention_heads_padded - self.num_attention_heads
             chunk_query = F.pad(chunk_query, [0, 0, 0, pad_size])
         offset = self.pg_collection.tp.rank() * chunk_query.size(0)
@@ -603,9 +606,10 @@ class DSAttentionFused(MegatronModule):
             packed_seq_params=packed_seq_params,
             attn_sink=self.attn_sink,
             return_attn_dist=self.num_attention_heads if need_loss else 0,
+            **inside,
         )
         output, main_attn_probs = res if need_loss else (res, None)
-        if self.num_attention_heads < self.num_attention_heads_padded:
+        if padded:
             output = output[..., : self.num_attention_heads, :]
 
         if need_loss:

@@ -84,12 +84,14 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
     ``dist_heads`` heads (dsa_fused.py:915-929): reduced from the logits, which pass through a buffer of all queries, or
     of a block of them at a time, of at most DSA_P_OUT_BUDGET_GIB (default 6) GiB; recomputed from q, kv and lse
     where that does not hold the logits of 64 queries (of all, if there are fewer).
+    ``padded_heads`` (not in the reference): the kernels work on that many heads, zeros behind those of ``q``; outputs and
+    gradients are those of ``q``'s heads.
     """
 
     @staticmethod
     def forward(ctx, q, kv, indices, chunk_offset=0, sm_scale=None, d_v=512, return_p_out=False,
                 packed_seq_params=None, topk_length=None, attn_sink=None, window_size=0, fast_mode=False,
-                dist_heads=0):
+                dist_heads=0, padded_heads=0):
         window_size = int(window_size or 0)
         if dist_heads and (return_p_out or window_size):
             raise ValueError("dist_heads replaces return_p_out and does not take a window_size")
@@ -98,7 +100,9 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
         if window_size % 32:
             raise NotImplementedError("window_size must be a multiple of 32, got %d" % window_size)
         # q [sq, n, d]; kv [skv, 1, d]; indices [sq, 1, topk]
-        sq = q.size(0)
+        sq, heads = q.size(0), q.size(1)
+        if padded_heads > heads:
+            q = ops.pad_heads(q, padded_heads)
         kv2 = kv.reshape(kv.shape[0], kv.shape[-1])
         ids = indices.reshape(sq, indices.shape[-1])
         if topk_length is not None:
@@ -129,7 +133,8 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
         ctx.sm_scale = sm_scale
         ctx.chunk_offset = chunk_offset
         ctx.d_v = d_v
-        out = out.unsqueeze(0)
+        ctx.heads = heads
+        out = out[:, :heads].unsqueeze(0)
         if return_p_out:
             ctx.mark_non_differentiable(p_out)
             return out, p_out
@@ -143,12 +148,12 @@ class DSADotProductAttentionFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out, grad_p_out=None):
         if grad_out is None:
-            return (None,) * 13
+            return (None,) * 14
         q, kv, ids, out, lse = ctx.saved_tensors
         grad_out = grad_out.squeeze(0).contiguous()
         kv2 = kv.reshape(kv.shape[0], kv.shape[-1])
-        grad_q, grad_kv = ops.sparse_mla_bwd(q, kv2, out, grad_out, ids, lse, ctx.chunk_offset, ctx.sm_scale, ctx.d_v)
-        return (grad_q, grad_kv.reshape(kv.shape), None, None, None, None, None, None, None, None, None, None, None)
+        grad_q, grad_kv = ops.sparse_mla_bwd(q, kv2, out, grad_out, ids, lse, ctx.chunk_offset, ctx.sm_scale, ctx.d_v, ctx.heads)
+        return (grad_q, grad_kv.reshape(kv.shape), None, None, None, None, None, None, None, None, None, None, None, None)
 
 
 class DSADotProductAttention(MegatronModule):
@@ -164,9 +169,10 @@ class DSADotProductAttention(MegatronModule):
                 attn_mask_type: AttnMaskType = None, attention_bias: Tensor = None,
                 packed_seq_params: PackedSeqParams = None, return_p_out: bool = False, window_size: int = 0,
                 topk_length: Optional[Tensor] = None, attn_sink: Optional[Tensor] = None,
-                return_attn_dist: int = 0):
+                return_attn_dist: int = 0, padded_heads: int = 0):
         # return_attn_dist = n > 0 (not in the reference's signature): also return the attention
         # distribution averaged over the first n heads, [sq, topk] fp32, without materialising p_out
+        # padded_heads (not in the reference's signature): see the function; without p_out, which would have them all
         if attn_mask_type is None:
             attn_mask_type = AttnMaskType.causal
         assert attn_mask_type in (AttnMaskType.causal, AttnMaskType.padding_causal), (
@@ -213,11 +219,11 @@ class DSADotProductAttention(MegatronModule):
 
         res = _apply(DSADotProductAttentionFunction, (query, kv, indices, topk_length, attn_sink), query, kv, indices, chunk_offset,
                      self.softmax_scale, d_v, return_p_out, packed_seq_params, topk_length, attn_sink, window_size, True,
-                     int(return_attn_dist))
+                     int(return_attn_dist), 0 if return_p_out else int(padded_heads))
         core_attn_out, p_out = (res if (return_p_out or return_attn_dist) else (res, None))
         if qkv_format == "thd":
-            core_attn_out = core_attn_out.squeeze(0).contiguous()
-        else:
+            core_attn_out = core_attn_out.squeeze(0)
+        if core_attn_out.size(-2) >= padded_heads:       # (the leading ones of the padded heads stay where they are)
             core_attn_out = core_attn_out.contiguous()
         if return_p_out:
             return core_attn_out, p_out

@@ -547,7 +547,7 @@ def release_bwd_workspace(device=None):
 @torch.library.custom_op("dsa::sparse_mla_bwd", mutates_args=())
 def _mla_bwd_op(q: torch.Tensor, kv: torch.Tensor, out: torch.Tensor, dout: torch.Tensor, ids: torch.Tensor,
                 lse: torch.Tensor, q_start: int, sm_scale: float, d_v: int) -> Tuple[torch.Tensor, torch.Tensor]:
-    return _native().mla_bwd(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v, _bwd_workspace, True)
+    return _native().mla_bwd(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v, 0, _bwd_workspace, True)
 
 
 @_mla_bwd_op.register_fake
@@ -555,16 +555,26 @@ def _(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v):
     return torch.empty_like(q), torch.empty_like(kv)
 
 
-def _mla_bwd(*args):
+def _mla_bwd(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v, heads):
     if not torch.compiler.is_compiling():
-        res = _native().mla_bwd(*args, _bwd_workspace, False)
+        res = _native().mla_bwd(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v, heads, _bwd_workspace, False)
         if res is not None:
             return res
-    return _mla_bwd_op(*args)
+    if not 0 < heads < q.shape[1]:
+        return _mla_bwd_op(q, kv, out, dout, ids, lse, q_start, sm_scale, d_v)
+    dq, dkv = _mla_bwd_op(q, kv, out, pad_heads(dout, q.shape[1]), ids, lse, q_start, sm_scale, d_v)
+    return dq[:, :heads].contiguous(), dkv
 
 
-def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optional[float] = None, d_v: int = 512):
-    """(dq, dkv) in bf16; dkv is accumulated in a fixed order (bit-reproducible).
+def pad_heads(x, heads: int):
+    """``x [S, h, width]`` with zero heads behind its own, ``heads`` in all."""
+    padded = None if torch.compiler.is_compiling() else _native().pad_heads(x, int(heads))
+    return torch.nn.functional.pad(x, (0, 0, 0, heads - x.shape[1])) if padded is None else padded
+
+
+def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optional[float] = None, d_v: int = 512, heads: int = 0):
+    """(dq, dkv) in bf16; dkv is accumulated in a fixed order (bit-reproducible).  ``heads`` > 0: only that many leading heads of ``q``
+    are real and the rest padding; ``dout`` has the real ones, and so has dq.
 
     The kernels take up to 2048 slots per query.  Longer lists are walked 2048 slots at a time: with the
     softmax statistics (``lse``) and ``out`` of the whole list given, the gradients are sums over the slots, so the
@@ -573,13 +583,13 @@ def sparse_mla_bwd(q, kv, out, dout, ids, lse, q_start: int = 0, sm_scale: Optio
         sm_scale = q.shape[-1] ** -0.5
     K = ids.shape[1]
     if K <= BWD_MAX_SLOTS:
-        return _mla_bwd(q, kv, out, dout, ids, lse, int(q_start), float(sm_scale), int(d_v))
+        return _mla_bwd(q, kv, out, dout, ids, lse, int(q_start), float(sm_scale), int(d_v), int(heads))
     dq32 = dkv32 = None
     for k0 in range(0, K, BWD_MAX_SLOTS):
         part = ids[:, k0:k0 + BWD_MAX_SLOTS]
         if part.shape[1] % 64:
             part = torch.nn.functional.pad(part, (0, 64 - part.shape[1] % 64), value=-1)
-        dq, dkv = _mla_bwd(q, kv, out, dout, part.contiguous(), lse, int(q_start), float(sm_scale), int(d_v))
+        dq, dkv = _mla_bwd(q, kv, out, dout, part.contiguous(), lse, int(q_start), float(sm_scale), int(d_v), int(heads))
         dq32 = dq.float() if dq32 is None else dq32.add_(dq)
         dkv32 = dkv.float() if dkv32 is None else dkv32.add_(dkv)
     return dq32.to(torch.bfloat16), dkv32.to(torch.bfloat16)

@@ -448,3 +448,36 @@ def test_calls_that_are_not_eager_take_the_functions(gpu):
     seen = []
     torch.func.vmap(lambda x: (seen.append(ops.indexer_forward(x, k, w, True, 1.0, None, 0, 64, True)), x)[1])(torch.stack([q.detach(), q.detach()]))
     assert seen == [None]
+
+
+@pytest.mark.parametrize("heads,S,packed", [(16, 1, False), (16, 900, False), (40, 450, True), (100, 130, False), (1, 70, True)])
+def test_heads_are_padded_inside_the_attention(gpu, heads, S, packed):
+    """Head counts that are no multiple of 32: the same bits as with the query padded and the output cut outside the attention, forward and
+    gradients, where queries are worked as one (900 x 16 and 450 x 40 heads) and where not."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import DSADotProductAttention
+    from loongforge_amd.megatron_compat import PackedSeqParams
+
+    g = torch.Generator().manual_seed(heads)
+    K, total = 128, (heads + 31) // 32 * 32
+    attn = DSADotProductAttention(_cfg(num_attention_heads=heads), softmax_scale=192 ** -0.5)
+    lead = (S,) if packed else (S, 1)
+    q = torch.randn(*lead, heads, 576, generator=g).to(gpu, torch.bfloat16).requires_grad_(True)
+    kv = torch.randn(*lead, 576, generator=g).to(gpu, torch.bfloat16).requires_grad_(True)
+    # neighbouring queries share their keys, so that joint units pay
+    seen = [torch.randperm(max(i, 1), generator=g)[:K].tolist() for i in range(0, S, 8)]
+    ids = torch.tensor([(seen[i // 8] + [-1] * K)[:K] for i in range(S)], dtype=torch.int32, device=gpu)
+    psp = PackedSeqParams(qkv_format="thd") if packed else None
+    dout = torch.randn(*((S,) if packed else (1, S)), heads, 512, generator=g).to(gpu, torch.bfloat16)
+    inside, dist = attn(q, kv, ids.unsqueeze(0), 0, packed_seq_params=psp, return_attn_dist=heads, padded_heads=total)
+    got = torch.autograd.grad(inside, [q, kv], dout)
+    outside, dist2 = attn(torch.nn.functional.pad(q, (0, 0, 0, total - heads)), kv, ids.unsqueeze(0), 0, packed_seq_params=psp, return_attn_dist=heads)
+    outside = outside[..., :heads, :]
+    want = torch.autograd.grad(outside, [q, kv], dout)
+    assert inside.shape == outside.shape and torch.equal(inside, outside) and torch.equal(dist, dist2)
+    assert got[0].shape == q.shape and got[0].is_contiguous() and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    with pytest.raises(ValueError):
+        attn(q, kv, ids.unsqueeze(0), 0, packed_seq_params=psp)                       # still refused without the padding
+    x = q.detach().reshape(-1)[4:4 + S // 2 * heads * 576].view(-1, heads, 576)       # starts inside a 16-byte piece
+    if x.numel():
+        assert torch.equal(ops.pad_heads(x, total), torch.nn.functional.pad(x, (0, 0, 0, total - heads)))
