@@ -229,11 +229,21 @@ int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void* k, int64_
 /*
  * The same for heads of 64 channels, all of them rotary, of bf16 q [S,heads,64] and k [keys,64]: rotary embedding (cos / sin bf16
  * [positions,64], row i of queries and keys at position i, split pairs, every product and the sum rounded to bf16), Hadamard rotation
- * of the 64, and dsa_quant_padded_e4m3 to heads_out heads and rows of 128; windows of one sequence (ratio 0).
+ * of the 64, and dsa_quant_padded_e4m3 to heads_out heads and rows of 128; windows of one sequence (ratio 0).  Weights count
+ * times weights_scale, bf16 ones rounded to bf16 behind it.
  */
 int dsa_indexer_narrow_e4m3(const void* q, int S, int heads, int heads_out, const void* k, int keys, const void* cos, const void* sin,
                             int positions, void* q8, float* q_scale, void* k8, float* k_scale, const void* weights, int weights_bf16,
-                            float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke, void* stream);
+                            float weights_scale, float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke, void* stream);
+/*
+ * dsa_indexer_front_e4m3 of the query rows q [S,heads,128] with their weights (as above) and of the key rows k [keys,128] behind their
+ * LayerNorm, and dsa_indexer_window, in one launch; power-of-two scales, pairing 0 or 1.
+ */
+int dsa_indexer_fronts_e4m3(const void* q, int S, int heads, const void* k, int keys, const float* ln_weight, const float* ln_bias, float ln_eps,
+                            const void* cos, const void* sin, int cos_sin_f32, int pairing, const int32_t* positions_q,
+                            const int32_t* positions_k, int batch, int rotate, void* q8, float* q_scale, void* k8, float* k_scale,
+                            const void* weights, int weights_bf16, float weights_scale, float factor, float* weight_scaled, const void* cu,
+                            int cu_i64, int ncu, int chunk_offset, int32_t* ks, int32_t* ke, int32_t* total, void* stream);
 /*
  * Position of packed token t + offset inside its own sequence, t in [0, tokens) (0 past the last sequence).
  */

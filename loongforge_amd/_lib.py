@@ -40,7 +40,9 @@ SIGNATURES = {
     "dsa_hadamard": (_i, [_vp, _vp, _i64, _i, _vp]),
     "dsa_indexer_window": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "dsa_indexer_inputs_e4m3": (_i, [_vp, _i64, _vp, _i64, _i, _vp, _vp, _vp, _vp, _f, _i, _vp, _i, _f, _vp, _i, _i64, _i, _i, _vp, _vp, _vp]),
-    "dsa_indexer_narrow_e4m3": (_i, [_vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _f, _vp, _i64, _vp, _vp, _vp]),
+    "dsa_indexer_narrow_e4m3": (_i, [_vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp, _i64, _vp, _vp, _vp]),
+    "dsa_indexer_fronts_e4m3": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp, _f, _vp, _vp, _i, _i, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp,
+                                     _vp, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "dsa_thd_positions": (_i, [_vp, _i, _i, _i, _i64, _vp, _vp]),
     "dsa_sparse_mla_fwd": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp]),
     "dsa_sparse_mla_fwd_ex": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _i, _vp]),

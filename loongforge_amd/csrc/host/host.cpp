@@ -151,6 +151,28 @@ py::object quant_weights(const Tensor& x_, const Tensor& weights_, double factor
   return py::make_tuple(x8, scale_inv, scaled);
 }
 
+struct FrontTables { Tensor cos, sin; OptTensor positions; };
+FrontTables front_tables(const OptTensor& cos, const OptTensor& sin, const OptTensor& positions, int64_t batch, int64_t tokens) {
+  REQUIRE(batch > 0, "indexer_front_e4m3: batch must be positive, got ", batch);       // (divided by below)
+  REQUIRE(cos && sin && cos->scalar_type() == sin->scalar_type() &&
+          (cos->scalar_type() == at::kFloat || cos->scalar_type() == at::kBFloat16),
+          "indexer_front_e4m3: cos / sin must both be fp32 or bf16 tables");
+  REQUIRE(cos->size(-1) == 64 && sin->size(-1) == 64 && cos->numel() == sin->numel(),
+          "indexer_front_e4m3: cos / sin rows must have 64 entries");
+  FrontTables t{cos->contiguous(), sin->contiguous(), {}};
+  if (positions) {
+    t.positions = i32(*positions);
+    REQUIRE(t.positions->numel() == tokens, "indexer_front_e4m3: one position per token expected");
+  } else {
+    REQUIRE((tokens + batch - 1) / batch <= t.cos.numel() / 64, "indexer_front_e4m3: cos / sin tables are shorter than the sequence");
+  }
+  return t;
+}
+std::pair<Tensor, Tensor> front_norm(const Tensor& weight, const Tensor& bias) {
+  REQUIRE(weight.numel() == 128 && bias.numel() == 128, "indexer_front_e4m3: LayerNorm weight and bias must have 128 entries");
+  return {f32(weight), f32(bias)};
+}
+
 py::object indexer_front(const Tensor& x_, int64_t rows_per_token, const OptTensor& ln_weight_, const OptTensor& ln_bias_, double ln_eps,
                          const OptTensor& cos_, const OptTensor& sin_, int64_t pairing, const OptTensor& positions_, int64_t batch,
                          bool rotate, const OptTensor& weights_, double factor, bool want_payload, bool want_rows, double eps, bool pow2,
@@ -168,26 +190,11 @@ py::object indexer_front(const Tensor& x_, int64_t rows_per_token, const OptTens
   int tables_f32 = 0;
   OptTensor cos, sin, positions, ln_weight, ln_bias, weights;
   if (pairing >= 0) {
-    REQUIRE(cos_ && sin_ && cos_->scalar_type() == sin_->scalar_type() &&
-            (cos_->scalar_type() == at::kFloat || cos_->scalar_type() == at::kBFloat16),
-            "indexer_front_e4m3: cos / sin must both be fp32 or bf16 tables");
-    REQUIRE(cos_->size(-1) == 64 && sin_->size(-1) == 64 && cos_->numel() == sin_->numel(),
-            "indexer_front_e4m3: cos / sin rows must have 64 entries");
-    cos = cos_->contiguous();
-    sin = sin_->contiguous();
-    tables_f32 = cos->scalar_type() == at::kFloat;
-    if (positions_) {
-      positions = i32(*positions_);
-      REQUIRE(positions->numel() == tokens, "indexer_front_e4m3: one position per token expected");
-    } else {
-      REQUIRE((tokens + batch - 1) / batch <= cos->numel() / 64, "indexer_front_e4m3: cos / sin tables are shorter than the sequence");
-    }
+    FrontTables t = front_tables(cos_, sin_, positions_, batch, tokens);
+    tables_f32 = t.cos.scalar_type() == at::kFloat;
+    cos = t.cos; sin = t.sin; positions = t.positions;
   }
-  if (ln_weight_) {
-    ln_weight = f32(*ln_weight_);
-    ln_bias = f32(*ln_bias_);
-    REQUIRE(ln_weight->numel() == 128 && ln_bias->numel() == 128, "indexer_front_e4m3: LayerNorm weight and bias must have 128 entries");
-  }
+  if (ln_weight_) std::tie(ln_weight, ln_bias) = front_norm(*ln_weight_, *ln_bias_);
   if (weights_) {
     REQUIRE(want_payload && weights_->numel() == rows, "indexer_front_e4m3: one weight per row expected, together with the payload");
     weights = f32(*weights_);
@@ -397,6 +404,11 @@ struct WindowCheck {
   hipEvent_t done = nullptr;
   WindowCheck() = default;
   WindowCheck(const WindowCheck&) = delete;
+  int32_t* pinned() const { return need ? (int32_t*)total.data_ptr() : nullptr; }
+  void launched(const Call& call) {
+    if (need && (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess || hipEventRecord(done, (hipStream_t)call.stream) != hipSuccess))
+      throw std::runtime_error("indexer window: no event");
+  }
   ~WindowCheck() { if (done) { (void)hipEventSynchronize(done); (void)hipEventDestroy(done); } }
   void wait() {
     if (!done) return;
@@ -420,28 +432,30 @@ Tensor seqlens(const Tensor& cu, const c10::Device& device) {
 
 struct Window { Tensor bounds; std::unique_ptr<WindowCheck> check; };      // [2, S]: first key, key behind the last
 
+// The tensors that a kernel fills with the windows; check->pinned() goes to it, check->launched() comes behind it.
+Window pending_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, const Tensor& like, const Call& call) {
+  Window w{make({2, S}, at::kInt, like), std::make_unique<WindowCheck>()};
+  if (cu && S > 0) {
+    hipStreamCaptureStatus capturing;
+    if (hipStreamIsCapturing((hipStream_t)call.stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
+      w.check->total = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+      w.check->need = chunk_offset + S;
+    }
+  }
+  return w;
+}
+
 Window key_windows(const OptTensor& cu_, int64_t S, int64_t chunk_offset, const Tensor& like) {
   need_gpus(like);
   OptTensor cu;
   if (cu_) cu = seqlens(*cu_, like.device());
   REQUIRE(!cu || S == 0 || cu->numel() > 1, "indexer: inconsistent shapes (no packed sequence)");
   Call call(like);
-  Tensor window = make({2, S}, at::kInt, like);
-  auto check = std::make_unique<WindowCheck>();
-  if (cu && S > 0) {
-    hipStreamCaptureStatus capturing;
-    if (hipStreamIsCapturing((hipStream_t)call.stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
-      check->total = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-      check->need = chunk_offset + S;
-    }
-  }
+  Window w = pending_window(cu, S, chunk_offset, like, call);
   run("dsa_indexer_window", dsa_indexer_window, cu ? ptr(cu) : nullptr, cu && cu->scalar_type() == at::kLong, cu ? (int)cu->numel() : 0, (int)S,
-      (int)chunk_offset, out_ptr<int32_t>(window), out_ptr<int32_t>(window) + S,
-      check->need ? (int32_t*)check->total.data_ptr() : nullptr, call.stream);
-  if (check->need && (hipEventCreateWithFlags(&check->done, hipEventDisableTiming) != hipSuccess ||
-                      hipEventRecord(check->done, (hipStream_t)call.stream) != hipSuccess))
-    throw std::runtime_error("indexer window: no event");
-  return {window, std::move(check)};
+      (int)chunk_offset, out_ptr<int32_t>(w.bounds), out_ptr<int32_t>(w.bounds) + S, w.check->pinned(), call.stream);
+  w.check->launched(call);
+  return w;
 }
 
 py::tuple indexer_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, const Tensor& like) {
@@ -457,18 +471,35 @@ py::tuple indexer_window(const OptTensor& cu, int64_t S, int64_t chunk_offset, c
 py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weights, bool rotate, double factor, const OptTensor& cu,
                            int64_t chunk_offset, int64_t K, bool sort, const OptTensor& cos, const OptTensor& sin, int64_t pairing,
                            const OptTensor& positions_q, const OptTensor& positions_k, int64_t batch, const OptTensor& ln_weight,
-                           const OptTensor& ln_bias, double ln_eps, int64_t ratio) {
+                           const OptTensor& ln_bias, double ln_eps, int64_t ratio, double weights_scale) {
   if (!plain(q, k, weights, cu, cos, sin, positions_q, positions_k, ln_weight, ln_bias)) return py::none();
   if (!q.is_cuda() || q.dim() != 3 || k.dim() != 2 || q.size(2) != 128 || k.size(1) != 128 || (q.size(1) != 32 && q.size(1) != 64) ||
       q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || weights.sizes() != q.sizes().slice(0, 2)) return py::none();
-  using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
-  Tensor q8, q_scale, scaled, k8, k_scale, rows;
+  if (cos ? !ln_weight || !ln_bias || pairing < 0 : weights_scale != 1.0) return py::none();
+  Tensor q8, q_scale, scaled, k8, k_scale;
   Window w;
   if (cos) {
-    std::tie(q8, q_scale, rows, scaled) = py::cast<Four>(indexer_front(q, q.size(1), {}, {}, 0.0, cos, sin, pairing, positions_q, batch, rotate,
-                                                                       weights, factor, true, false, 1e-12, true, false));
-    std::tie(k8, k_scale, rows, rows) = py::cast<Four>(indexer_front(k, 1, ln_weight, ln_bias, ln_eps, cos, sin, pairing, positions_k, batch, rotate,
-                                                                     {}, 1.0, true, false, 1e-12, true, false));
+    need_gpus(q, k, weights, cos, sin, positions_q, positions_k, ln_weight, ln_bias);
+    const int64_t S = q.size(0), Sk = k.size(0);
+    const Tensor qc = q.contiguous(), kc = k.contiguous();
+    const Tensor wc = weights.scalar_type() == at::kBFloat16 ? weights.contiguous() : f32(weights);
+    const FrontTables tq = front_tables(cos, sin, positions_q, batch, S), tk = front_tables(cos, sin, positions_k, batch, Sk);
+    const auto [lw, lb] = front_norm(*ln_weight, *ln_bias);
+    OptTensor lens;
+    if (cu) lens = seqlens(*cu, q.device());
+    REQUIRE(!lens || S == 0 || lens->numel() > 1, "indexer: inconsistent shapes (no packed sequence)");
+    Call call(qc);
+    q8 = make(qc.sizes(), at::kFloat8_e4m3fn, qc); q_scale = make(weights.sizes(), at::kFloat, qc); scaled = make(weights.sizes(), at::kFloat, qc);
+    k8 = make(kc.sizes(), at::kFloat8_e4m3fn, kc); k_scale = make({Sk}, at::kFloat, kc);
+    w = pending_window(lens, S, chunk_offset, qc, call);
+    run("dsa_indexer_fronts_e4m3", dsa_indexer_fronts_e4m3, qc.const_data_ptr(), (int)S, (int)q.size(1), kc.const_data_ptr(), (int)Sk,
+        (const float*)lw.const_data_ptr(), (const float*)lb.const_data_ptr(), (float)ln_eps, tq.cos.const_data_ptr(), tq.sin.const_data_ptr(),
+        (int)(tq.cos.scalar_type() == at::kFloat), (int)pairing, (const int32_t*)ptr(tq.positions), (const int32_t*)ptr(tk.positions), (int)batch, (int)rotate,
+        out_ptr<void>(q8), out_ptr<float>(q_scale), out_ptr<void>(k8), out_ptr<float>(k_scale), wc.const_data_ptr(),
+        (int)(wc.scalar_type() == at::kBFloat16), (float)weights_scale, (float)factor, out_ptr<float>(scaled), lens ? ptr(lens) : nullptr,
+        (int)(lens && lens->scalar_type() == at::kLong), lens ? (int)lens->numel() : 0, (int)chunk_offset, out_ptr<int32_t>(w.bounds),
+        out_ptr<int32_t>(w.bounds) + S, w.check->pinned(), call.stream);
+    w.check->launched(call);
   } else {
     need_gpus(q, k, weights);
     const Tensor qc = q.contiguous(), kc = k.contiguous();
@@ -483,7 +514,7 @@ py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weigh
         wc.scalar_type() == at::kBFloat16, (float)factor, out_ptr<float>(scaled), cu ? 0 : (int)S, chunk_offset, (int)ratio, (int)kc.size(0),
         out_ptr<int32_t>(w.bounds), out_ptr<int32_t>(w.bounds) + S, call.stream);
   }
-  if (cu || cos) w = key_windows(cu, q.size(0), chunk_offset, q8);
+  if (cu && !cos) w = key_windows(cu, q.size(0), chunk_offset, q8);
   const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
       indexer_topk(q8, scaled, k8, k_scale, w.bounds.select(0, 0), w.bounds.select(0, 1), K, sort, false));
   return py::make_tuple(scores, ids, q8, q_scale, scaled, k8, k_scale, w.check && w.check->done ? py::cast(std::move(w.check)) : py::none());
@@ -492,8 +523,8 @@ py::object indexer_forward(const Tensor& q, const Tensor& k, const Tensor& weigh
 // indexer_forward for heads of 64 rotary channels behind their projections (q [S, heads, 64], k [Sk, 64] behind its norm; cos, sin bf16
 // [positions, 64]), padded on the way to 32 or 64 heads of 128 channels, one sequence.  -> (scores, ids, q8, q_scale, scaled
 // weights, k8, k_scale); None for other arguments.
-py::object indexer_forward_narrow(const Tensor& q, const Tensor& k, const Tensor& weights, const Tensor& cos, const Tensor& sin, double factor,
-                                  int64_t chunk_offset, int64_t K, bool sort) {
+py::object indexer_forward_narrow(const Tensor& q, const Tensor& k, const Tensor& weights, const Tensor& cos, const Tensor& sin,
+                                  double weights_scale, double factor, int64_t chunk_offset, int64_t K, bool sort) {
   if (!plain(q, k, weights, cos, sin) || !q.is_cuda() || q.dim() != 3 || k.dim() != 2 || q.size(2) != 64 || k.size(1) != 64 || q.size(1) < 1 ||
       q.size(1) > 64 || q.scalar_type() != at::kBFloat16 || k.scalar_type() != at::kBFloat16 || weights.sizes() != q.sizes().slice(0, 2) ||
       cos.scalar_type() != at::kBFloat16 || sin.scalar_type() != at::kBFloat16 || cos.numel() != sin.numel() || cos.numel() % 64) return py::none();
@@ -511,7 +542,7 @@ py::object indexer_forward_narrow(const Tensor& q, const Tensor& k, const Tensor
   Tensor k8 = make({Sk, 128}, at::kFloat8_e4m3fn, qc), k_scale = make({Sk}, at::kFloat, qc), bounds = make({2, S}, at::kInt, qc);
   run("dsa_indexer_narrow_e4m3", dsa_indexer_narrow_e4m3, qc.const_data_ptr(), (int)S, (int)heads, (int)heads_out, kc.const_data_ptr(), (int)Sk,
       c.const_data_ptr(), s.const_data_ptr(), (int)positions, out_ptr<void>(q8), out_ptr<float>(q_scale), out_ptr<void>(k8), out_ptr<float>(k_scale),
-      wc.const_data_ptr(), wc.scalar_type() == at::kBFloat16, (float)factor, out_ptr<float>(scaled), chunk_offset, out_ptr<int32_t>(bounds),
+      wc.const_data_ptr(), wc.scalar_type() == at::kBFloat16, (float)weights_scale, (float)factor, out_ptr<float>(scaled), chunk_offset, out_ptr<int32_t>(bounds),
       out_ptr<int32_t>(bounds) + S, call.stream);
   const auto [scores, ids] = py::cast<std::pair<Tensor, Tensor>>(
       indexer_topk(q8, scaled, k8, k_scale, bounds.select(0, 0), bounds.select(0, 1), K, sort, false));

@@ -1,7 +1,7 @@
 // Row-wise e4m3 quantiser (one power-of-two scale per 128-element row).
 // HBM-bound: reads 2 B and writes 1 B per element plus 4 B per row; one 64-lane wave per row
 // group, each lane handling 8 consecutive elements (16-byte loads, 8-byte stores).
-#include "dsa_common.h"
+#include "window.h"
 
 namespace {
 
@@ -13,12 +13,15 @@ __device__ __forceinline__ float wave_max16(float v) {   // max over the 16 lane
   return v;
 }
 
-// A weight per row: fp32, or bf16 as it came
+// A weight per row: fp32, or bf16 as it came; AnyWeight times `scale`, rounded to its own type as a tensor operation would
 struct F32Weight { const float* p; __device__ float operator[](int64_t i) const { return p[i]; } };
 struct AnyWeight {
   const void* p;
   bool bf16;
-  __device__ float operator[](int64_t i) const { return bf16 ? bf16_bits_to_f32(((const unsigned short*)p)[i]) : ((const float*)p)[i]; }
+  float scale;
+  __device__ float operator[](int64_t i) const {
+    return bf16 ? bf16_bits_to_f32(f32_to_bf16_bits(bf16_bits_to_f32(((const unsigned short*)p)[i]) * scale)) : ((const float*)p)[i] * scale;
+  }
 };
 
 // cols == 128: 16 lanes per row, 4 rows per wave, 16 rows per 256-thread block.
@@ -336,15 +339,15 @@ __global__ __launch_bounds__(256) void indexer_narrow_kernel(const NarrowArgs a)
 //   quantiser         power-of-two scale, e4m3 payload, optionally weights * scale_inv * factor
 // Every stage rounds where the separate operations round, so the payload is that of the unfused sequence.
 // Sums run in a fixed order (a lane's 8 elements in sequence, then the 16 lanes of a row by xor 1, 2, 4, 8).
-template <bool LN, int PAIRING>   // PAIRING: -1 no rotary part, 0 adjacent pairs, 1 split pairs (i, i + 32)
-__global__ __launch_bounds__(256) void indexer_front128_kernel(
-    const uint4* __restrict__ x, int64_t rows, int rows_per_token, const float* __restrict__ ln_w,
+template <bool LN, int PAIRING, class W>   // PAIRING: -1 no rotary part, 0 adjacent pairs, 1 split pairs (i, i + 32)
+__device__ __forceinline__ void front128_rows(
+    unsigned block, const uint4* __restrict__ x, int64_t rows, int rows_per_token, const float* __restrict__ ln_w,
     const float* __restrict__ ln_b, float ln_eps, const void* __restrict__ cos_t, const void* __restrict__ sin_t,
     int cs_f32, const int* __restrict__ positions, int batch, int rotate, uint2* __restrict__ x8,
-    float* __restrict__ scale_inv, uint4* __restrict__ y, float eps, int pow2, const float* __restrict__ w_in,
+    float* __restrict__ scale_inv, uint4* __restrict__ y, float eps, int pow2, W w_in,
     float w_factor, float* __restrict__ w_scaled) {
 #pragma clang fp contract(off)
-  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int64_t row = (int64_t)block * 16 + (threadIdx.x >> 4);
   const int sub = threadIdx.x & 15;
   const bool live = row < rows;
   const uint4 raw = live ? x[row * 16 + sub] : make_uint4(0, 0, 0, 0);
@@ -472,6 +475,55 @@ __global__ __launch_bounds__(256) void indexer_front128_kernel(
   }
 }
 
+template <bool LN, int PAIRING>
+__global__ __launch_bounds__(256) void indexer_front128_kernel(
+    const uint4* __restrict__ x, int64_t rows, int rows_per_token, const float* __restrict__ ln_w,
+    const float* __restrict__ ln_b, float ln_eps, const void* __restrict__ cos_t, const void* __restrict__ sin_t,
+    int cs_f32, const int* __restrict__ positions, int batch, int rotate, uint2* __restrict__ x8,
+    float* __restrict__ scale_inv, uint4* __restrict__ y, float eps, int pow2, const float* __restrict__ w_in,
+    float w_factor, float* __restrict__ w_scaled) {
+  front128_rows<LN, PAIRING>(blockIdx.x, x, rows, rows_per_token, ln_w, ln_b, ln_eps, cos_t, sin_t, cs_f32, positions, batch, rotate, x8, scale_inv,
+                             y, eps, pow2, F32Weight{w_in}, w_factor, w_scaled);
+}
+
+// Both sides' front end and the windows in one launch: the keys first (LayerNorm: the longest chain), then the queries' heads, then the
+// windows, of packed sequences too.  With the head weights scaled on the way it takes the place of five launches of 3 - 6 us beside
+// the queries' own, and of the scaling's node.
+struct FrontArgs {
+  const uint4 *q, *k;
+  int64_t q_rows, k_rows;
+  int heads;
+  const float *ln_w, *ln_b;
+  float ln_eps;
+  const void *cos_t, *sin_t;
+  int cs_f32;
+  const int *pos_q, *pos_k;
+  int batch, rotate;
+  uint2 *q8, *k8;
+  float *q_scale, *k_scale;
+  AnyWeight w_in;
+  float w_factor;
+  float* w_scaled;
+  unsigned k_blocks, q_blocks;
+  const void* cu;
+  int cu_i64, ncu, S, chunk_offset;
+  int *ks, *ke, *total;
+};
+template <int PAIRING>
+__global__ __launch_bounds__(256) void indexer_fronts_kernel(const FrontArgs a) {
+  const unsigned b = blockIdx.x;
+  if (b < a.k_blocks)
+    front128_rows<true, PAIRING>(b, a.k, a.k_rows, 1, a.ln_w, a.ln_b, a.ln_eps, a.cos_t, a.sin_t, a.cs_f32, a.pos_k, a.batch, a.rotate, a.k8, a.k_scale,
+                                 nullptr, 1e-12f, 1, F32Weight{nullptr}, 0.f, nullptr);
+  else if (b < a.k_blocks + a.q_blocks)
+    front128_rows<false, PAIRING>(b - a.k_blocks, a.q, a.q_rows, a.heads, nullptr, nullptr, 0.f, a.cos_t, a.sin_t, a.cs_f32, a.pos_q, a.batch, a.rotate,
+                                  a.q8, a.q_scale, nullptr, 1e-12f, 1, a.w_in, a.w_factor, a.w_scaled);
+  else if (a.cu_i64)
+    window_part((int)(b - a.k_blocks - a.q_blocks), (const long long*)a.cu, a.ncu, a.S, a.chunk_offset, a.ks, a.ke, a.total);
+  else
+    window_part((int)(b - a.k_blocks - a.q_blocks), (const int*)a.cu, a.ncu, a.S, a.chunk_offset, a.ks, a.ke, a.total);
+}
+
 }  // namespace
 
 extern "C" int dsa_rotate_quant_e4m3(const void* x, int64_t rows, int cols, void* x8, float* scale_inv, void* y,
@@ -502,7 +554,7 @@ extern "C" int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void
   const int64_t q_blocks = (q_rows + 15) / 16, k_blocks = (k_rows + 15) / 16, blocks = q_blocks + k_blocks + dsa_cdiv(S, 256);
   DSA_REQUIRE(blocks < (1ll << 31), "dsa_indexer_inputs_e4m3: too many rows");
   if (blocks == 0) return DSA_OK;
-  const InputArgs a{(const uint4*)q, (const uint4*)k, (uint2*)q8, (uint2*)k8, q_scale, k_scale, q_rows, k_rows, {weights, weights_bf16 != 0}, factor,
+  const InputArgs a{(const uint4*)q, (const uint4*)k, (uint2*)q8, (uint2*)k8, q_scale, k_scale, q_rows, k_rows, {weights, weights_bf16 != 0, 1.0f}, factor,
                     weight_scaled, (unsigned)q_blocks, (unsigned)k_blocks, eps, pow2, S, ratio, keys, offset, ks, ke};
   if (rotate) indexer_inputs_kernel<true><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
   else indexer_inputs_kernel<false><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
@@ -512,7 +564,8 @@ extern "C" int dsa_indexer_inputs_e4m3(const void* q, int64_t q_rows, const void
 
 extern "C" int dsa_indexer_narrow_e4m3(const void* q, int S, int heads, int heads_out, const void* k, int keys, const void* cos, const void* sin,
                                        int positions, void* q8, float* q_scale, void* k8, float* k_scale, const void* weights, int weights_bf16,
-                                       float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke, void* stream) {
+                                       float weights_scale, float factor, float* weight_scaled, int64_t offset, int32_t* ks, int32_t* ke,
+                                       void* stream) {
   DSA_REQUIRE(S >= 0 && keys >= 0 && heads > 0 && heads <= heads_out && heads_out <= 64, "dsa_indexer_narrow_e4m3: bad sizes");
   DSA_REQUIRE(positions >= S && positions >= keys, "dsa_indexer_narrow_e4m3: cos / sin tables are shorter than the sequence");
   DSA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)cos % 16) == 0 && ((uintptr_t)sin % 16) == 0 &&
@@ -524,7 +577,7 @@ extern "C" int dsa_indexer_narrow_e4m3(const void* q, int S, int heads, int head
   DSA_REQUIRE(q_rows < (1ll << 31), "dsa_indexer_narrow_e4m3: too many rows");
   if (blocks == 0) return DSA_OK;
   const NarrowArgs a{(const uint4*)q, (const uint4*)k, (const uint4*)cos, (const uint4*)sin, heads, heads_out, q_rows, keys, (uint2*)q8, (uint2*)k8,
-                     q_scale, k_scale, {weights, weights_bf16 != 0}, factor, weight_scaled, (unsigned)q_blocks, (unsigned)k_blocks, S, offset, ks, ke};
+                     q_scale, k_scale, {weights, weights_bf16 != 0, weights_scale}, factor, weight_scaled, (unsigned)q_blocks, (unsigned)k_blocks, S, offset, ks, ke};
   indexer_narrow_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(a);
   DSA_CHECK_LAUNCH("dsa_indexer_narrow_e4m3");
   return DSA_OK;
@@ -611,5 +664,31 @@ extern "C" int dsa_indexer_front_e4m3(const void* x, int64_t rows, int cols, int
   }
 #undef DSA_FRONT_LAUNCH
   DSA_CHECK_LAUNCH("dsa_indexer_front_e4m3");
+  return DSA_OK;
+}
+
+extern "C" int dsa_indexer_fronts_e4m3(const void* q, int S, int heads, const void* k, int keys, const float* ln_weight, const float* ln_bias, float ln_eps,
+                                       const void* cos, const void* sin, int cos_sin_f32, int pairing, const int32_t* positions_q,
+                                       const int32_t* positions_k, int batch, int rotate, void* q8, float* q_scale, void* k8, float* k_scale,
+                                       const void* weights, int weights_bf16, float weights_scale, float factor, float* weight_scaled,
+                                       const void* cu, int cu_i64, int ncu, int chunk_offset, int32_t* ks, int32_t* ke, int32_t* total, void* stream) {
+  DSA_REQUIRE(S >= 0 && keys >= 0 && heads > 0 && batch > 0 && ncu >= 0, "dsa_indexer_fronts_e4m3: bad sizes");
+  DSA_REQUIRE(pairing == 0 || pairing == 1, "dsa_indexer_fronts_e4m3: pairing must be 0 or 1");
+  DSA_REQUIRE(cos != nullptr && sin != nullptr && ln_weight != nullptr && ln_bias != nullptr && (cu != nullptr || ncu == 0),
+              "dsa_indexer_fronts_e4m3: null pointer");
+  DSA_REQUIRE(S == 0 || (q && q8 && q_scale && weights && weight_scaled && ks && ke), "dsa_indexer_fronts_e4m3: null pointer");
+  DSA_REQUIRE(keys == 0 || (k && k8 && k_scale), "dsa_indexer_fronts_e4m3: null pointer");
+  DSA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)q8 % 8) == 0 && ((uintptr_t)k8 % 8) == 0 &&
+              ((uintptr_t)ln_weight % 16) == 0 && ((uintptr_t)ln_bias % 16) == 0 && ((uintptr_t)cos % 16) == 0 &&
+              ((uintptr_t)sin % 16) == 0, "dsa_indexer_fronts_e4m3: misaligned pointer");
+  const int64_t q_rows = (int64_t)S * heads, q_blocks = (q_rows + 15) / 16, k_blocks = (keys + 15) / 16;
+  DSA_REQUIRE(q_rows < (1ll << 32), "dsa_indexer_fronts_e4m3: too many rows");
+  const FrontArgs a{(const uint4*)q, (const uint4*)k, q_rows, keys, heads, ln_weight, ln_bias, ln_eps, cos, sin, cos_sin_f32, positions_q, positions_k, batch,
+                    rotate, (uint2*)q8, (uint2*)k8, q_scale, k_scale, {weights, weights_bf16 != 0, weights_scale}, factor, weight_scaled,
+                    (unsigned)k_blocks, (unsigned)q_blocks, cu, cu_i64, ncu, S, chunk_offset, ks, ke, total};
+  const dim3 grid((unsigned)(k_blocks + q_blocks + dsa_cdiv(S > 0 ? S : 1, 256)));
+  if (pairing == 0) indexer_fronts_kernel<0><<<grid, dim3(256), 0, (hipStream_t)stream>>>(a);
+  else indexer_fronts_kernel<1><<<grid, dim3(256), 0, (hipStream_t)stream>>>(a);
+  DSA_CHECK_LAUNCH("dsa_indexer_fronts_e4m3");
   return DSA_OK;
 }

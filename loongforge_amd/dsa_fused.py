@@ -322,14 +322,21 @@ class DSAIndexerFused(MegatronModule):
                                     mscale=mscale, cp_group=self.pg_collection.cp)
         return x_pe if all_rotary else torch.cat([x_pe, x[..., self.qk_pos_emb_head_dim:]], dim=-1)
 
+    def _weights_scale(self, weights):
+        """The head weights times ``heads ** -0.5``, or as they are with the ``weights_scale`` that tells the kernel to."""
+        scale = self.index_n_heads ** -0.5
+        if weights.dtype == torch.bfloat16 and weights.is_cuda and _takes_checks(self.indexer_kernel, DSAIndexerKernel):
+            return weights, {"weights_scale": scale}
+        return weights * scale, {}
+
     def _projections(self, x, qr):
-        """q ``[s, (b,) h, d]``, k behind its norm and weights, before the rotary embedding."""
+        """q ``[s, (b,) h, d]``, k behind its norm and the weights without their scale, before the rotary embedding."""
         x, qr = x.detach(), qr.detach()
         q, _ = self.linear_wq_b(qr)
         q = q.view(*q.size()[:-1], self.index_n_heads, self.index_head_dim)
         k, _ = self.linear_wk(x)
         weights, _ = self.linear_weights_proj(x)
-        return q, self.k_norm(k), weights * self.index_n_heads ** -0.5
+        return q, self.k_norm(k), weights
 
     def get_query_key_weight_tensors(self, x, qr, packed_seq_params: Optional[PackedSeqParams] = None,
                                      defer_rotation: bool = False, projected=None):
@@ -379,7 +386,7 @@ class DSAIndexerFused(MegatronModule):
             # this chunk's own key gradient (dsa_fused.py:606-622)
             pos, last = self._chunk_position()[1], self.num_chunks_per_seq - 1
             k.register_hook(lambda g: g if pos == last else g + self._chunk_slab.grads.pop(pos))
-        return q, k, weights
+        return q, k, weights * self.index_n_heads ** -0.5
 
     def _fused_front_end(self, x, packed_seq_params):
         """An :class:`IndexerFrontEnd` when key LayerNorm, rotary embedding and rotation can run inside the indexer
@@ -407,7 +414,7 @@ class DSAIndexerFused(MegatronModule):
             cu_k = packed_seq_params.cu_seqlens_kv if cu_k is None else cu_k
             cp = self.pg_collection.cp
             pos_q = _token_positions(cu_q, x.shape[0], cp.rank(), cp.size())
-            pos_k = _token_positions(cu_k, x.shape[0], cp.rank(), cp.size())
+            pos_k = pos_q if cu_k is cu_q else _token_positions(cu_k, x.shape[0], cp.rank(), cp.size())
         return IndexerFrontEnd(cos=cos.reshape(-1, 64), sin=sin.reshape(-1, 64), pairing=ops.ROPE_SPLIT, positions_q=pos_q,
                                positions_k=pos_k, batch=1 if packed_seq_params is not None else x.shape[1],
                                k_norm_eps=float(k_norm.eps))
@@ -445,22 +452,23 @@ class DSAIndexerFused(MegatronModule):
             q = q.view(*q.size()[:-1], self.index_n_heads, self.index_head_dim)
             k, _ = self.linear_wk(x)
             weights, _ = self.linear_weights_proj(x)
-            weights = weights * self.index_n_heads ** -0.5
+            weights, scale = self._weights_scale(weights)
             if packed_seq_params is None:
                 q = q.squeeze(1)
             return self.indexer_kernel(
                 q.contiguous(), k.squeeze(1).contiguous(), weights.squeeze(1).contiguous(), self.index_topk,
                 chunk_offset=self.pg_collection.tp.rank() * q.size(0), packed_seq_params=packed_seq_params,
-                rotate=bool(rotate), front=front, k_norm_weight=self.k_norm.weight, k_norm_bias=self.k_norm.bias, **late)
+                rotate=bool(rotate), front=front, k_norm_weight=self.k_norm.weight, k_norm_bias=self.k_norm.bias, **scale, **late)
         tables, projected = self._narrow_tables(x, packed_seq_params), None
         if tables is not None:
             from . import ops
 
             projected = q, k, weights = self._projections(x, qr)
             if q.dtype == k.dtype == torch.bfloat16 and ops.ordinary(q, k, weights):
+                weights, scale = self._weights_scale(weights)
                 return self.indexer_kernel(q.squeeze(1), k.squeeze(1), weights.squeeze(1), self.index_topk,
                                            chunk_offset=self.pg_collection.tp.rank() * q.size(0), packed_seq_params=None,
-                                           rotary_tables=tables, **late)
+                                           rotary_tables=tables, **scale, **late)
         # (with chunkpipe the cached keys are the rotated ones, so the rotation stays outside the kernel)
         fuse = (rotate and self.index_head_dim == 128
                 and x.is_cuda and not chunkpipe and getattr(self.indexer_kernel, "supports_fused_rotate", False))

@@ -275,7 +275,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
     def forward(ctx, index_q: Tensor, index_k: Tensor, weights: Tensor, index_topk: int, chunk_offset: int,
                 packed_seq_params: Optional[PackedSeqParams], rotate: bool = False, front: Optional["IndexerFrontEnd"] = None,
                 k_norm_weight: Optional[Tensor] = None, k_norm_bias: Optional[Tensor] = None, checks: Optional[list] = None,
-                cos: Optional[Tensor] = None, sin: Optional[Tensor] = None):
+                cos: Optional[Tensor] = None, sin: Optional[Tensor] = None, weights_scale: float = 1.0):
         assert index_q.ndim == 3 and index_k.ndim == 2 and weights.ndim == 2
         seq_q, head, dim = index_q.size()
         seq_k, _dim = index_k.size()
@@ -303,9 +303,11 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
         k_p = topk_indices = covered = None
         whole = None if cos is not None else ops.indexer_forward(
             index_q, index_k, weights, rotate, softmax_scale, cu, chunk_offset, index_topk, sort, front,
-            k_norm_weight if front is not None else None, k_norm_bias if front is not None else None)
+            k_norm_weight if front is not None else None, k_norm_bias if front is not None else None, weights_scale=weights_scale)
+        if whole is None and cos is None and weights_scale != 1.0:
+            weights = weights * weights_scale
         if cos is not None:
-            narrow = ops.indexer_forward_narrow(index_q, index_k, weights, cos, sin, softmax_scale, chunk_offset, index_topk, sort)
+            narrow = ops.indexer_forward_narrow(index_q, index_k, weights, cos, sin, softmax_scale, chunk_offset, index_topk, sort, weights_scale)
             if narrow is None:
                 raise ValueError("the rotary tables of narrow heads take ordinary bf16 device tensors with heads of 64 channels")
             index_score_topk, topk_indices, q_fp8, q_scale, weight_scaled, k_fp8, k_scale = narrow
@@ -343,7 +345,7 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
                 covered.wait()
             else:
                 checks.append(covered)
-        ctx.softmax_scale = softmax_scale
+        ctx.weights_factor = softmax_scale * weights_scale
         ctx.rotate = rotate
         ctx.index_topk = index_topk
         ctx.span = _known_span(packed_seq_params)
@@ -360,16 +362,16 @@ class DSAIndexerKernelFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_score, grad_topk):
         if grad_score is None:
-            return (None,) * 13
+            return (None,) * 14
         q_fp8, k_fp8, q_scale, k_scale, weight_scaled, topk_indices, *narrow = ctx.saved_tensors
         head, dim = ctx.shape
         k_in, ln_w, ln_b = ctx.front_saved if ctx.front is not None else (None, None, None)
         d_q, d_k, d_weights, d_ln_w, d_ln_b = ops.indexer_grads(
-            grad_score, q_fp8, k_fp8, k_scale, weight_scaled, topk_indices, q_scale, ctx.softmax_scale, head, dim, ctx.in_dtypes,
+            grad_score, q_fp8, k_fp8, k_scale, weight_scaled, topk_indices, q_scale, ctx.weights_factor, head, dim, ctx.in_dtypes,
             ctx.rotate, ctx.front, k_in, ln_w, ctx.span, narrow or None)
         if ctx.front is not None:
             d_ln_w, d_ln_b = d_ln_w.to(ln_w.dtype), d_ln_b.to(ln_b.dtype)
-        return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b, None, None, None
+        return d_q, d_k, d_weights, None, None, None, None, None, d_ln_w, d_ln_b, None, None, None, None
 
 
 @dataclass
@@ -398,19 +400,21 @@ class DSAIndexerKernel(torch.nn.Module):
     supports_fused_front_end = True
 
     def forward(self, index_q, index_k, weights, index_topk, chunk_offset, packed_seq_params, rotate=False,
-                front=None, k_norm_weight=None, k_norm_bias=None, checks=None, rotary_tables=None):
+                front=None, k_norm_weight=None, k_norm_bias=None, checks=None, rotary_tables=None,
+                weights_scale=1.0):
         """``front`` (an extension, :class:`IndexerFrontEnd`): ``index_q`` / ``index_k`` are the outputs of the
         projections and the key LayerNorm (``k_norm_weight``, ``k_norm_bias``), the rotary embedding and the rotation
         run inside the quantiser kernels.  ``checks`` (an extension): a list that takes what is left to be checked on the
         device (that the packed sequences hold every query) instead of waiting for it here; the caller calls ``wait()`` of its
         entries once it has launched the work that it can launch.  ``rotary_tables`` (an extension): bf16 ``(cos, sin)`` of one
         sequence's positions for 64-channel heads that are rotary throughout; rotary embedding, rotation and padding run inside the
-        quantiser kernel."""
+        quantiser kernel.  ``weights_scale`` (an extension): ``weights`` count times this, rounded to their type."""
         cos, sin = rotary_tables if rotary_tables is not None else (None, None)
         if cos is not None and (rotate or front is not None or packed_seq_params is not None):
             raise ValueError("rotary_tables comes with the rotation, without a front end and for one sequence")
         return _apply(DSAIndexerKernelFunction, (index_q, index_k, weights, k_norm_weight, k_norm_bias), index_q, index_k, weights,
-                      index_topk, chunk_offset, packed_seq_params, rotate, front, k_norm_weight, k_norm_bias, checks, cos, sin)
+                      index_topk, chunk_offset, packed_seq_params, rotate, front, k_norm_weight, k_norm_bias, checks, cos, sin,
+                      float(weights_scale))
 
 
 # ---------------------------------------------------------------------------------------------------

@@ -423,25 +423,28 @@ def indexer_window(cu_seqlens: Optional[torch.Tensor], queries: int, chunk_offse
 
 
 def indexer_forward(index_q, index_k, weights, rotate: bool, factor: float, cu_seqlens, chunk_offset: int, K: int, sorted: bool, front=None,
-                    ln_weight=None, ln_bias=None, ratio: int = 0):
+                    ln_weight=None, ln_bias=None, ratio: int = 0, weights_scale: float = 1.0):
     """Quantisers (with ``front``, an ``IndexerFrontEnd``, behind the front end), :func:`indexer_window` and :func:`indexer_topk` of bf16
     ``index_q [S, 32 or 64, 128]`` and ``index_k [Sk, 128]`` in one native call: (scores, ids, q8, q_scale, scaled weights, k8,
     k_scale, check or None); None for other arguments and for calls that are not eager ones on ordinary tensors.  ``ratio`` > 0: one
-    sequence, query ``i`` sees the first ``(chunk_offset + i + 1) // ratio`` keys, at least one."""
+    sequence, query ``i`` sees the first ``(chunk_offset + i + 1) // ratio`` keys, at least one.  ``weights_scale`` (with ``front``): the
+    weights count times this, rounded to their type."""
     if torch.compiler.is_compiling():
         return None
     f = front
     return _native().indexer_forward(index_q, index_k, weights, bool(rotate), float(factor), cu_seqlens, int(chunk_offset), int(K), bool(sorted),
                                      f and f.cos, f and f.sin, f.pairing if f else -1, f and f.positions_q, f and f.positions_k,
-                                     f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0, int(ratio))
+                                     f.batch if f else 1, ln_weight, ln_bias, f.k_norm_eps if f else 0.0, int(ratio), float(weights_scale))
 
 
-def indexer_forward_narrow(index_q, index_k, weights, cos, sin, factor: float, chunk_offset: int, K: int, sorted: bool):
+def indexer_forward_narrow(index_q, index_k, weights, cos, sin, factor: float, chunk_offset: int, K: int, sorted: bool,
+                           weights_scale: float = 1.0):
     """:func:`indexer_forward` over one sequence for bf16 ``index_q [S, <= 64, 64]`` and ``index_k [Sk, 64]`` that still need their
     rotary embedding (bf16 ``cos`` / ``sin [positions, .., 64]``, every channel rotary, split pairs, rounded like
     :func:`rope_steps`) and their Hadamard rotation: (scores, ids, q8, q_scale, scaled weights, k8, k_scale), padded to
     32 or 64 heads of 128; None for arguments it does not take."""
-    return _native().indexer_forward_narrow(index_q, index_k, weights, cos, sin, float(factor), int(chunk_offset), int(K), bool(sorted))
+    return _native().indexer_forward_narrow(index_q, index_k, weights, cos, sin, float(weights_scale), float(factor), int(chunk_offset), int(K),
+                                            bool(sorted))
 
 
 # --------------------------------------------------------------------------------------------

@@ -390,3 +390,45 @@ def test_indexer_module_of_narrow_heads_in_one_kernel(gpu, S, heads):
     for a, b in zip(narrow[2], apart[2]):
         # three bf16 roundings each way, and the one of the result
         assert (a - b).float().norm().item() <= 2.0 ** -6 * b.float().norm().item() + 1e-6
+
+
+@pytest.mark.parametrize("S,heads,pairing,packed,bf16_weights,rotate", [
+    (1, 32, R.SPLIT, False, True, True), (17, 64, R.ADJACENT, False, False, True), (300, 32, R.SPLIT, True, True, True),
+    (515, 64, R.SPLIT, "int64", True, False), (257, 64, R.ADJACENT, True, False, False)])
+def test_both_fronts_and_the_windows_in_one_launch_are_those_of_separate_launches(gpu, S, heads, pairing, packed, bf16_weights, rotate):
+    """Payloads, scales, head weights (scaled and rounded to their type on the way) and selection bit for bit; a table, a
+    packed batch or an alignment that the separate kernels refuse is refused."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import IndexerFrontEnd
+
+    g = torch.Generator().manual_seed(S)
+    q = torch.randn(S, heads, 128, generator=g).to(gpu, torch.bfloat16)
+    k = torch.randn(S, 128, generator=g).to(gpu, torch.bfloat16)
+    w = torch.randn(S, heads, generator=g).to(gpu, torch.bfloat16 if bf16_weights else torch.float32)
+    lw, lb = torch.randn(128, generator=g).to(gpu), torch.randn(128, generator=g).to(gpu)
+    cos, sin = (t.to(gpu) for t in R.rope_tables(S, 64, dtype=torch.bfloat16))
+    cu = pos = None
+    if packed:
+        cu = torch.tensor([0, S // 3, S // 3, S // 3 + 1, S], dtype=torch.int64 if packed == "int64" else torch.int32, device=gpu)
+        pos = ops.thd_positions(cu, S)
+    front = IndexerFrontEnd(cos=cos, sin=sin, pairing=pairing, positions_q=pos, positions_k=pos, batch=1, k_norm_eps=1e-6)
+    scale, factor, K = heads ** -0.5, 128 ** -0.5, 64
+    scores, ids, q8, q_scale, scaled, k8, k_scale, check = ops.indexer_forward(q, k, w, rotate, factor, cu, 0, K, True, front, lw, lb, weights_scale=scale)
+    assert (check is not None) == bool(packed)
+    if check is not None:
+        check.wait()
+    want_q = ops.indexer_front_e4m3(q, heads, None, None, 0.0, cos, sin, pairing, pos, 1, rotate, (w * scale).float(), factor)
+    want_k = ops.indexer_front_e4m3(k, 1, lw, lb, 1e-6, cos, sin, pairing, pos, 1, rotate)
+    for a, b in ((q8, want_q[0]), (k8, want_k[0])):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert torch.equal(q_scale, want_q[1]) and torch.equal(scaled, want_q[3]) and torch.equal(k_scale, want_k[1])
+    ks, ke, _ = ops.indexer_window(cu, S, 0, q8)
+    want = ops.indexer_topk(q8, scaled, k8, k_scale, ks, ke, K)
+    assert torch.equal(scores, want[0]) and torch.equal(ids, want[1])
+    if packed:
+        short = ops.indexer_forward(q, k, w, rotate, factor, cu[:-1], 0, K, True, front, lw, lb)[-1]
+        with pytest.raises(ValueError, match="inconsistent shapes"):
+            short.wait()
+    else:
+        with pytest.raises(ValueError, match="shorter than the sequence"):
+            ops.indexer_forward(q, k, w, rotate, factor, None, 0, K, True, IndexerFrontEnd(cos=cos[1:], sin=sin[1:], pairing=pairing), lw, lb)
