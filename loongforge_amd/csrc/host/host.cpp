@@ -687,6 +687,24 @@ py::object kl_loss(const Tensor& scores_, const Tensor& target_, double eps, boo
   return py::make_tuple(row_loss, grad);
 }
 
+// The loss of all rows times factor, and its gradient behind kl_loss: grad * g * factor.  None for what the kernels do not take.
+py::object kl_total(const Tensor& row_loss, double factor) {
+  if (!plain(row_loss) || !row_loss.is_cuda() || row_loss.scalar_type() != at::kFloat || row_loss.dim() != 1 || !row_loss.is_contiguous()) return py::none();
+  Call call(row_loss);
+  Tensor total = make({}, at::kFloat, row_loss);
+  run("dsa_indexer_kl_total", dsa_indexer_kl_total, (const float*)ptr(row_loss), (int)row_loss.numel(), (float)factor, (float*)total.data_ptr(), call.stream);
+  return py::cast(total);
+}
+
+py::object kl_scale(const Tensor& grad, const Tensor& g, double factor) {
+  if (!plain(grad, g) || !grad.is_cuda() || !g.is_cuda() || g.device() != grad.device() || grad.scalar_type() != at::kFloat || g.scalar_type() != at::kFloat || g.numel() != 1 ||
+      !grad.is_contiguous() || (uintptr_t)grad.const_data_ptr() % 16) return py::none();
+  Call call(grad);
+  Tensor y = at::empty_like(grad);
+  run("dsa_indexer_kl_scale", dsa_indexer_kl_scale, (const float*)ptr(grad), (const float*)ptr(g), (float)factor, out_ptr<float>(y), grad.numel(), call.stream);
+  return py::cast(y);
+}
+
 // ---- absorption and rotary kernels (write into their arguments) ---------------------------------------
 void need_bf16(const Tensor& a, const Tensor& b, const Tensor& c) {
   REQUIRE(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && c.scalar_type() == at::kBFloat16,
@@ -842,6 +860,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(mla_bwd);
   DEF(attn_dist);
   DEF(kl_loss);
+  DEF(kl_total);
+  DEF(kl_scale);
   DEF(indexer_window);
   DEF(indexer_forward);
   DEF(indexer_forward_narrow);

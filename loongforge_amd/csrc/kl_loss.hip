@@ -79,7 +79,56 @@ __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict_
   if (tid == 0) row_loss[row] = loss;
 }
 
+// *out = factor * sum of the rows' losses, in a fixed order.  One launch for the sum and the scaling behind it (5 us each).
+__global__ __launch_bounds__(1024) void kl_total_kernel(const float* __restrict__ row_loss, int S, float factor, float* __restrict__ out) {
+  __shared__ float part[16];
+  float s = 0.f;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < S; i += 1024) s += row_loss[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  s = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) s += part[i];
+  *out = s * factor;
+}
+
+// y = x * (*g * factor): the loss's gradient carried on to the scores, bound by memory.
+__global__ __launch_bounds__(256) void kl_scale_kernel(const f32x4* __restrict__ x, const float* __restrict__ g, float factor, f32x4* __restrict__ y, int64_t n) {
+  const float f = *g * factor;
+  const int64_t n4 = n / 4, i0 = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+  f32x4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (i0 + 256 * i < n4) v[i] = x[i0 + 256 * i];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (i0 + 256 * i < n4) y[i0 + 256 * i] = v[i] * f;
+  if (blockIdx.x == 0 && (int64_t)threadIdx.x < n % 4) ((float*)y)[4 * n4 + threadIdx.x] = ((const float*)x)[4 * n4 + threadIdx.x] * f;
+}
+
 }  // namespace
+
+extern "C" int dsa_indexer_kl_total(const float* row_loss, int S, float factor, float* out, void* stream) {
+  DSA_REQUIRE(S >= 0 && out != nullptr && (S == 0 || row_loss != nullptr), "dsa_indexer_kl_total: bad arguments");
+  kl_total_kernel<<<dim3(1), dim3(1024), 0, (hipStream_t)stream>>>(row_loss, S, factor, out);
+  DSA_CHECK_LAUNCH("dsa_indexer_kl_total");
+  return DSA_OK;
+}
+
+extern "C" int dsa_indexer_kl_scale(const float* grad, const float* g, float factor, float* out, int64_t n, void* stream) {
+  DSA_REQUIRE(n >= 0 && (n == 0 || (grad && g && out)), "dsa_indexer_kl_scale: bad arguments");
+  DSA_REQUIRE(((uintptr_t)grad % 16) == 0 && ((uintptr_t)out % 16) == 0, "dsa_indexer_kl_scale: misaligned pointer");
+  if (n == 0) return DSA_OK;
+  const int64_t blocks = (n / 4 + 1024) / 1024;
+  DSA_REQUIRE(blocks < (1ll << 31), "dsa_indexer_kl_scale: too many elements");
+  kl_scale_kernel<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>((const f32x4*)grad, g, factor, (f32x4*)out, n);
+  DSA_CHECK_LAUNCH("dsa_indexer_kl_scale");
+  return DSA_OK;
+}
 
 extern "C" int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S, int K,
                                    float eps, float* row_loss, float* grad, void* stream) {

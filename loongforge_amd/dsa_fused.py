@@ -625,13 +625,15 @@ class DSAttentionFused(MegatronModule):
             main_attn_probs = main_attn_probs[:, : index_scores.shape[-1]]
             # softmax, F.kl_div(log(pred + 1e-10), target + 1e-10, "sum") and their backward in one kernel
             from . import ops
-            loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10)
+            scaled = bool(sq) and isinstance(indexer_loss_coeff, (int, float))       # (one launch each way with the loss itself)
+            indexer_loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10, indexer_loss_coeff / sq if scaled else 1.0)
         for check in checks:
             check.wait()
         if topk_holder is not None and not self.skip_topk:
             topk_holder[self.layer_number] = topk_indices
         if need_loss:
-            indexer_loss = loss * (indexer_loss_coeff / sq) if sq else indexer_loss_coeff * loss / sq      # (one launch each way)
+            if not scaled:
+                indexer_loss = indexer_loss * (indexer_loss_coeff / sq) if sq else indexer_loss_coeff * indexer_loss / sq
             if indexer_loss_coeff > 0:
                 DSAIndexerLossLoggingHelperFused.save_loss_to_tracker(
                     loss=indexer_loss,

@@ -684,22 +684,26 @@ class _IndexerKLLoss(torch.autograd.Function):
     """The loss and its gradient come out of the same kernel; backward only scales what forward kept."""
 
     @staticmethod
-    def forward(ctx, scores, target, eps):
+    def forward(ctx, scores, target, eps, factor):
         row_loss, grad = _direct("kl_loss", _kl_loss_op, scores.detach(), target.detach(), eps)
         ctx.save_for_backward(grad)
-        ctx.in_dtype = scores.dtype
-        return row_loss.sum()
+        ctx.in_dtype, ctx.factor = scores.dtype, factor
+        total = None if torch.compiler.is_compiling() else _native().kl_total(row_loss, factor)
+        return row_loss.sum() * factor if total is None else total
 
     @staticmethod
     def backward(ctx, g):
         (grad,) = ctx.saved_tensors
-        return (grad * g).to(ctx.in_dtype), None, None
+        scaled = None
+        if not torch.is_grad_enabled() and not torch.compiler.is_compiling() and ordinary(grad, g):
+            scaled = _native().kl_scale(grad, g, ctx.factor)
+        return (grad * (g * ctx.factor) if scaled is None else scaled).to(ctx.in_dtype), None, None, None
 
 
-def indexer_kl_loss(scores: torch.Tensor, target: torch.Tensor, eps: float = 1e-10) -> torch.Tensor:
+def indexer_kl_loss(scores: torch.Tensor, target: torch.Tensor, eps: float = 1e-10, factor: float = 1.0) -> torch.Tensor:
     """``F.kl_div((softmax(scores, -1) + eps).log(), target + eps, reduction="sum")`` as one kernel
-    (dsa_fused.py:931-937 of the reference); differentiable in ``scores``, the target is a constant."""
-    return _IndexerKLLoss.apply(scores, target, float(eps))
+    (dsa_fused.py:931-937 of the reference), times ``factor``; differentiable in ``scores``, the target is a constant."""
+    return _IndexerKLLoss.apply(scores, target, float(eps), float(factor))
 
 
 def _rows_view(t: torch.Tensor, what: str):

@@ -69,3 +69,23 @@ def test_kl_loss_equals_f_kl_div_and_vanishes_for_equal_distributions(gpu):
     wide = torch.cat([tg, torch.zeros(64, 64)], -1).to(gpu)
     got3 = ops.indexer_kl_loss(sc.to(gpu), wide[:, :512])
     assert got3.item() == got.item()
+
+
+@pytest.mark.parametrize("S,K", [(1, 1), (3, 65), (1025, 64), (5000, 131)])
+def test_scaled_sum_and_its_gradient(gpu, S, K):
+    """The loss times a factor and its gradient in a launch each: the sum within S half-ulps of 64 bits, the gradient's bits those of the
+    product with (g * factor); with a graph of the backward the tensor operations."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(S)
+    scores = torch.randn(S, K, generator=g).to(gpu).requires_grad_(True)
+    target = torch.softmax(torch.randn(S, K, generator=g), -1).to(gpu)
+    rows, grad = ops._kl_loss_op(scores.detach(), target, 1e-10)
+    up = torch.tensor(1.7, device=gpu)
+    loss = ops.indexer_kl_loss(scores, target, 1e-10, 0.37)
+    want = rows.double().sum().item() * 0.37
+    assert loss.shape == () and abs(loss.item() - want) <= (S + 1) * 2.0 ** -24 * rows.double().abs().sum().item() * 0.37 + 1e-12
+    (got,) = torch.autograd.grad(loss, scores, up, retain_graph=True)
+    assert torch.equal(got, grad * (up * 0.37))
+    (again,) = torch.autograd.grad(loss, scores, up, create_graph=True)
+    assert torch.equal(again, got)
