@@ -68,10 +68,10 @@ struct FwdArgs {
 // The softmax of a head is taken relative to a reference point, the maximum of the first tile, so the
 // O^T accumulators are never rescaled (a rescaling branch in the loop, even one never taken, costs the
 // register allocator hundreds of spills).  Where a later tile exceeds it by more than 2^64 (exp2 then nears
-// the end of fp32) the wave marks its heads - a NaN with a payload in lse, or in the statistics of its
-// slot range - and the kernel that follows does them again relative to the true row maximum.  In modes 3 and 4, and in mode
-// 2 with all slots in one workgroup, where the waves' registers have room for it, the workgroup does so itself: the kernel that
-// follows takes 4.5 us also when nothing is marked.
+// the end of fp32) the wave marks its heads and they are done again relative to the true row maximum: by the workgroup itself behind its
+// output, when its accumulators are free, or where the slots are in ranges by the kernel that sums those (the mark is a NaN with a
+// payload in the range's statistics).  A kernel for it behind the ones with all slots in one workgroup took 4.5 us also when nothing
+// was marked.
 constexpr float REDO_ABOVE = 64.0f, REDO_TERM = 0x1p64f;
 constexpr unsigned REDO_MARK = 0x7fc0d5a0u;
 __device__ __forceinline__ bool is_marked(float x) { return __builtin_bit_cast(unsigned, x) == REDO_MARK; }
@@ -144,17 +144,31 @@ __device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned
 }
 // One 32-head block of a query relative to the true maximum of every head, all slots, one tile at a time: every
 // wave computes S^T of the block and sums its own value column tile dt.  For the marked blocks only: simple, and
-// light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.
-__device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int dt, f32x16& acc, float& m, float& l) {
+// light on registers and LDS (one tile, the ids) so that the kernels that carry it stay small.  tid: the thread's number among 256; a
+// second half of 512 threads stages and gathers the same again.
+template <bool COUNTED>                      // tid is counted anew; else it is threadIdx.x, of 256
+__device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int dt, f32x16& acc, float& m, float& l, int tid) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int lane = tid & 63, r = lane & 31, g = lane >> 5;
   const int NT = a.K / BI;
   int* idx_s = (int*)(smem + TILE_BYTES);
   unsigned* tmask = (unsigned*)(idx_s + a.K);
   int* tlist = (int*)(tmask + NT);
   __syncthreads();
-  const int ntiles = stage_ids(a.ids, qi, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
-  const LaneOffsets lo = lane_offsets();
+  int ntiles;
+  if constexpr (COUNTED) {
+    const int* const ids = a.ids + (size_t)qi * a.K;
+    int first[8];
+    request_first_ids(ids, 0, a.K, first, tid);
+    stage_requested(first, ids, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tid);
+    __syncthreads();
+    if (tid < 64) list_tiles(NT, tmask, tlist, tlist + NT, tid);
+    __syncthreads();
+    ntiles = tlist[NT];
+  } else {
+    ntiles = stage_ids(a.ids, qi, a.K, a.Skv, a.q_start + qi, idx_s, tmask, tlist, tlist + NT);
+  }
+  const LaneOffsets lo = lane_offsets(tid);
   const bf16x8* qp = (const bf16x8*)(a.q + ((size_t)qi * a.H + hb * 32 + r) * DQK) + g;
   const float c2 = a.sm_scale * LOG2E;
   unsigned v_off[2][2];                      // the wave's value columns: lo.tr_off[s][t][dt & 1]
@@ -171,7 +185,7 @@ __device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int
   for (int step = 0; step < 2 * ntiles; step++) {            // first sweep: the maximum; second: the sums
     const int tile = tlist[step < ntiles ? step : step - ntiles];
     __syncthreads();
-    gather_tile(a.kv, idx_s, tile, (unsigned)(uintptr_t)smem);
+    gather_tile(a.kv, idx_s, tile, (unsigned)(uintptr_t)smem, tid);
     DSA_WAIT_VMCNT(0);
     __syncthreads();
     f32x16 sacc;
@@ -201,13 +215,34 @@ __device__ __forceinline__ void redo_block(const FwdArgs& a, int qi, int hb, int
   l += __shfl_xor(l, 32, 64);
 }
 
-__device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, int dt, const f32x16& acc, float m, float l) {
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+__device__ __forceinline__ void write_block(const FwdArgs& a, int qi, int hb, int dt, const f32x16& acc, float m, float l, int tid) {
+  const int lane = tid & 63, r = lane & 31, g = lane >> 5;
   const int h = hb * 32 + r;
   const Final fin = finish_head(m, l, a.sink ? a.sink + h : nullptr);
   if (dt == 0 && g == 0) a.lse[(size_t)qi * a.H + h] = fin.lse;
   store_out(acc, fin.inv, (unsigned short*)a.out + ((size_t)qi * a.H + h) * DV + 32 * dt + 8 * g);
 }
+
+// The marked ones (bit hb) of a query's head blocks again, by all WAVES waves of the workgroup.
+template <int WAVES>
+__device__ __forceinline__ void redo_marked(const FwdArgs& a, int qi, unsigned marked, int wave, int lane) {
+  const int tid = (wave & 3) * 64 + lane;
+#pragma unroll 1
+  while (marked) {
+    const int hb = __builtin_ctz(marked);
+    marked &= marked - 1;
+#pragma unroll 1
+    for (int dt = wave; dt < DTILES; dt += WAVES) {
+      f32x16 acc;
+      float m, l;
+      redo_block<true>(a, qi, hb, dt, acc, m, l, tid);
+      write_block(a, qi, hb, dt, acc, m, l, tid);
+    }
+  }
+}
+
+// The lane counted anew, for what follows the loop over the tiles to hold no register through it.
+__device__ __forceinline__ int lane_again() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
 // Workgroup -> (unit, head group), a unit being a query, or a slot range of one.  The head groups of a unit gather the same rows:
 // they sit eight workgroups apart, i.e. on the same XCD and its L2.  So do `span` neighbouring units: the drafted tokens of a
@@ -227,7 +262,6 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   const int r = lane & 31, g = lane >> 5;
   const int stream = wave >> 1, sub = wave & 1;
   const int S = a.S, H = a.H, K = a.K, p_skip = a.p_skip;
-
   const int units = S * (SPLIT ? a.ksplit : 1);              // longest prefixes first, range by range
   int hg;
   const int u = unit_of(a, (int)blockIdx.x, hg);
@@ -444,7 +478,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   // ---- two streams: the second one's sums reach the first through the (now free) tile ring, scaled to the
   // common reference point; the first one's waves finish --------------------------------------------------
   __syncthreads();                         // the last tiles and the id arrays have been read
-  static_assert(2 * NDT * 4096 + 1024 <= RING, "the hand-over fits the tile ring");
+  static_assert(2 * NDT * 4096 + 1024 + 8 <= RING, "the hand-over fits the tile ring");
   float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the two waves' boxes
   if (g == 0) {
     ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
@@ -458,8 +492,8 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     for (int dt = wave; dt < DTILES; dt += 4) {
       f32x16 acc;
       float m, l;
-      redo_block(a, qi, hb, dt, acc, m, l);
-      write_block(a, qi, hb, dt, acc, m, l);
+      redo_block<false>(a, qi, hb, dt, acc, m, l, tid);
+      write_block(a, qi, hb, dt, acc, m, l, tid);
     }
     return;
   }
@@ -478,8 +512,10 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
         box[(dt * 4 + j) * 64] = v;
       }
   }
+  unsigned* const marked_s = (unsigned*)(ml + 256);        // mode 1: the head blocks to be done again
+  if (MODE == 1 && !SPLIT && stream == 1 && lane == 0) marked_s[sub] = again && head_ok;
   __syncthreads();
-  if (stream == 1) return;
+  if (stream == 1 && (MODE == 2 || SPLIT)) return;
   const float mine = f;
   auto merged = [&](int dt) {                // column tile dt of the wave's heads, both streams
     f32x16 t;
@@ -491,20 +527,17 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
     return t;
   };
-  if (!head_ok) return;                      // the same for all lanes of a wave
-  const bool stats = g == 0 && (MODE != 2 || sub == 0);
-  float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
-  if (again) {
-    if (stats) {
-      if (SPLIT) part_ml[0] = __builtin_bit_cast(float, REDO_MARK);
-      else a.lse[(size_t)qi * H + h] = __builtin_bit_cast(float, REDO_MARK);
-    }
-    return;
-  }
 
   // ---- epilogue: the wave's column tiles, normalised to out[i,h,:] with lse[i,h], or as they are to the workspace ----
+  const bool stats = g == 0 && (MODE != 2 || sub == 0);
   const int dt0 = MODE == 2 ? sub * NDT : 0;
   if (SPLIT) {
+    if (!head_ok) return;                    // the same for all lanes of a wave
+    float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
+    if (again) {
+      if (stats) part_ml[0] = __builtin_bit_cast(float, REDO_MARK);
+      return;
+    }
     if (stats) { part_ml[0] = m_ref; part_ml[1] = l_tot; }
     f32x4* po = a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt0) * 256 + lane;
 #pragma unroll
@@ -514,13 +547,19 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
     return;
   }
-  const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
-  if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
-  unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
+  if (head_ok && !again && stream == 0) {
+    const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
+    if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
+    unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
 #pragma unroll
-  for (int dt = 0; dt < NDT; dt++) {
-    store_out(merged(dt), fin.inv, op + 32 * dt);
-    __builtin_amdgcn_sched_barrier(0);
+    for (int dt = 0; dt < NDT; dt++) {
+      store_out(merged(dt), fin.inv, op + 32 * dt);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (MODE == 1) {
+    const unsigned marked = __builtin_amdgcn_readfirstlane(marked_s[0] | (marked_s[1] << 1));
+    if (marked) redo_marked<4>(a, qi, marked << (2 * hg), wave, lane_again());
   }
 }
 
@@ -557,8 +596,9 @@ constexpr int Q_ACC = 18;                    // k-steps of the Q slice in accumu
 constexpr int Q_GROUPS = 5;                  // 128-byte groups of the rows of Q that pass through LDS, behind tile 0
 static_assert(TILE_BYTES + 4 * Q_GROUPS * GRP_BYTES <= WIDE_LDS, "Q lies where tiles 1 and 2 and P will be");
 
+// -> the head blocks to be done again (bit hb) and, where there are any, 16 times the wave's number
 template <bool SCORES, bool SPLIT, int POUT>
-__device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsigned char* smem) {
+__device__ __forceinline__ unsigned wide_body(const FwdArgs& a, int qi, int sp, unsigned char* smem) {
   const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
   const int H = a.H, K = a.K;
@@ -569,6 +609,11 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
   unsigned* tmask = (unsigned*)(idx_s + KL);
   int* tlist = (int*)(tmask + NT);
   float* const inv_s = (float*)pbuf;         // after the last tile
+  unsigned* const marked_s = (unsigned*)(inv_s + 128);
+  unsigned marked = 0;
+  auto marked_blocks = [&] {
+    return (unsigned)__builtin_amdgcn_readfirstlane(marked_s[0] | (marked_s[1] << 1) | (marked_s[2] << 2) | (marked_s[3] << 3));
+  };
 
   const int* const ids = a.ids + (size_t)qi * K + k0;
   const int h = 32 * w + r;                  // of the scores
@@ -591,7 +636,7 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
     stage_requested(first, ids, KL, a.Skv, a.q_start + qi, idx_s, tmask, threadIdx.x & 255);
   }
   __syncthreads();
-  if (!SCORES && w == 0) list_tiles(NT, tmask, tlist, tlist + NT);
+  if (!SCORES && w == 0) list_tiles(NT, tmask, tlist, tlist + NT, (int)threadIdx.x);
   __syncthreads();
   const int ntiles = tlist[NT];
   if constexpr (SCORES) {
@@ -745,14 +790,16 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
       }
     } else {
       const Final fin = finish_head(m_ref, l_tot, a.sink && head_ok ? a.sink + h : nullptr);
-      if (head_ok && g == 0) a.lse[(size_t)qi * H + h] = again ? __builtin_bit_cast(float, REDO_MARK) : fin.lse;
+      if (head_ok && g == 0 && !again) a.lse[(size_t)qi * H + h] = fin.lse;
       if (g == 0) inv_s[h] = fin.inv;
+      if (lane == 0) marked_s[w] = again && head_ok;
     }
     __syncthreads();
+    if (!SPLIT) marked = marked_blocks();
 #pragma unroll
     for (int hb = 0; hb < 3; hb++) {
       mfma_done_a(o[hb]);
-      if (32 * hb < H) {
+      if (32 * hb < H && !((marked >> hb) & 1)) {
         const int dt = 4 * w + 3;
         if (SPLIT) store_partial(o[hb], a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt) * 256 + lane);
         else store_out(o[hb], inv_s[32 * hb + r], (unsigned short*)a.out + ((size_t)qi * H + 32 * hb + r) * DV + 32 * dt + 8 * g);
@@ -832,8 +879,9 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
       }
     }
     __syncthreads();                         // the heads' factors
+    if (!SPLIT) marked = marked_blocks();
     auto store = [&](const f32x16& t, int hb, int i) {
-      if (32 * hb >= H) return;
+      if (32 * hb >= H || ((marked >> hb) & 1)) return;
       const int dt = 4 * w + i;
       if (SPLIT) store_partial(t, a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt) * 256 + lane);
       else store_out(t, inv_s[32 * hb + r], (unsigned short*)a.out + ((size_t)qi * H + 32 * hb + r) * DV + 32 * dt + 8 * g);
@@ -851,6 +899,7 @@ __device__ __forceinline__ void wide_body(const FwdArgs& a, int qi, int sp, unsi
     mfma_done_v(o3);
     store(o3, 3, 3);
   }
+  return marked ? marked | (unsigned)(w + (SCORES ? 0 : 4)) << 4 : 0;
 }
 
 template <bool SPLIT, int POUT>
@@ -860,8 +909,10 @@ __global__ __launch_bounds__(512, 2) void mla_fwd_wide_kernel(FwdArgs a) {
   // 199 / 211, 5000 x 1024 in five documents 928 / 893 / 900, 8192 x 2048 4006 / 3949 / 3973; without them the same within 1 %.
   const int u = (int)blockIdx.x;
   const int qi = a.S - 1 - (SPLIT ? u / a.ksplit : spread_start(u, a.S, 256, a.K)), sp = SPLIT ? u % a.ksplit : 0;
-  if (threadIdx.x < 256) wide_body<true, SPLIT, POUT>(a, qi, sp, smem);
-  else wide_body<false, SPLIT, POUT>(a, qi, sp, smem);
+  unsigned marked;
+  if (threadIdx.x < 256) marked = wide_body<true, SPLIT, POUT>(a, qi, sp, smem);
+  else marked = wide_body<false, SPLIT, POUT>(a, qi, sp, smem);
+  if (!SPLIT && marked) redo_marked<8>(a, qi, marked & 15, marked >> 4, lane_again());
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1202,37 +1253,11 @@ __global__ __launch_bounds__(256, 2) void mla_fwd_half_kernel(FwdArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  for (int hb = 0; hb < HB; hb++) {          // here and not in a kernel behind this one: that takes 4.5 us also when nothing is marked
-    if (32 * (HB * hg + hb) >= H || !again[hb]) continue;
-#pragma unroll 1
-    for (int dt = w; dt < DTILES; dt += 4) {
-      f32x16 acc;
-      float m1, l1;
-      redo_block(a, qi, HB * hg + hb, dt, acc, m1, l1);
-      write_block(a, qi, HB * hg + hb, dt, acc, m1, l1);
-    }
-  }
-}
-
-// Modes 0 and 1, ksplit = 1: workgroup b looks at the marks of queries 32b .. 32b + 31 with one load per lane and head block and
-// redoes the marked blocks; a launch in which nothing is marked costs a few microseconds.
-__global__ __launch_bounds__(256) void mla_fwd_redo_kernel(FwdArgs a) {
-  const int wave = threadIdx.x >> 6;
-  const int qc = (int)blockIdx.x * 32 + (int)(threadIdx.x & 31);
-  for (int hb = 0; hb < a.H / 32; hb++) {
-    unsigned todo = (unsigned)__ballot(qc < a.S && is_marked(a.lse[(size_t)(qc < a.S ? qc : 0) * a.H + hb * 32]));
-    __syncthreads();                         // every wave reads the same marks before any of them is rewritten
-    while (todo) {
-      const int qi = (int)blockIdx.x * 32 + __builtin_ctz(todo);
-      todo &= todo - 1;
-      for (int dt = wave; dt < DTILES; dt += 4) {
-        f32x16 acc;
-        float m, l;
-        redo_block(a, qi, hb, dt, acc, m, l);
-        write_block(a, qi, hb, dt, acc, m, l);
-      }
-    }
-  }
+  unsigned marked = 0;
+#pragma unroll
+  for (int hb = 0; hb < HB; hb++)
+    if (32 * (HB * hg + hb) < H && again[hb]) marked |= 1u << (HB * hg + hb);
+  if (marked) redo_marked<4>(a, qi, marked, w, lane_again());
 }
 
 // Sum of the ksplit partial results of a query, reading the accumulator layout in which they were stored (1 KB per
@@ -1274,7 +1299,7 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
 #pragma unroll
   for (int e = 0; e < 16; e++) acc[e] = 0.f;
   if (__ballot(again) != 0ull) {
-    redo_block(a, qi, hb, dt, acc, m, l);
+    redo_block<false>(a, qi, hb, dt, acc, m, l, (int)threadIdx.x);
     if (SHARED && wave != 0) return;         // all waves have the same block
   } else {
     for (int s = s0; s < ns; s += AHEAD * s_step) {
@@ -1314,7 +1339,7 @@ __global__ __launch_bounds__(256) void mla_fwd_combine_kernel(FwdArgs a) {
       }
     }
   }
-  write_block(a, qi, hb, dt, acc, m, l);
+  write_block(a, qi, hb, dt, acc, m, l, (int)threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1352,10 +1377,13 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // 215 and 285 (303 in mode 0 undivided), 300 x 4096 357 and 391 (381).
 // 32 heads: 257 queries 78 us in mode 4 and 112 in mode 2, 800 queries 175 and 236.  4000 queries of 128 heads: 256 slots 440 us in
 // mode 0 and 390 in mode 3, 640 slots 760 and 800 (150 queries x 256 slots 28.6 and 31.2).
+// WHOLE: what modes 0 and 1 take beyond the fit with all slots in one workgroup, more with few pairs (250 queries x 64 heads x 256 slots
+// 27.5 us in mode 1 and 23.7 in mode 3, 89 x 128 x 256 22.8 and 21.2; 94 x 128 x 2048 82.6 in mode 1 and 87.6 in two ranges of mode 0).
+// Blocks done again inside them and not by a kernel behind: 168 x 64 x 512 35.2 -> 32.2 us, 108 x 128 x 1024 52.7 -> 50.6.
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
 // mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
-  constexpr float REDO = 4.6f, COMBINE = 2.37f, COMBINE_RANGE = 0.22f, SHARED_RANGE = 0.1f, COMBINE_BYTES_PER_US = 6.2e6f;
+  constexpr float WHOLE = 1.8f, WHOLE_FEW = 4.6f, COMBINE = 2.37f, COMBINE_RANGE = 0.22f, SHARED_RANGE = 0.1f, COMBINE_BYTES_PER_US = 6.2e6f;
   constexpr float FIXED_IDLE[5] = {4.91f, 5.86f, 4.51f, 5.57f, 3.8f}, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
   constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.68f, 1.31f, 2.82f, 1.78f};
   constexpr float PAIR_LAST[3] = {3.65f, 2.24f, 1.75f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.41f, 1.42f};
@@ -1381,7 +1409,7 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       const float fixed = mode >= 3 && rest > 0.5f ? FIXED_FULL[mode] : FIXED_IDLE[mode];
       float t = (float)rounds * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += fixed + per * pair;
-      t += ksplit == 1 ? (mode >= 2 ? 0.0f : REDO)
+      t += ksplit == 1 ? (mode >= 2 ? 0.0f : pairs <= 8 ? WHOLE_FEW : WHOLE)
                        : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
       if (wgs >= 4096) break;                // more ranges only add rounds
@@ -1429,10 +1457,9 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, bool shared, hipStream_t st) {
 #undef DSA_FWD_LAUNCH
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
-  if (MODE >= 2 && !SPLIT) return 0;
-  if (dsa_reserve_lds(SPLIT ? (const void*)combine : (const void*)mla_fwd_redo_kernel, tail) != hipSuccess) return -2;
-  if (SPLIT) combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), 256, tail, st>>>(a);
-  else mla_fwd_redo_kernel<<<dim3((a.S + 31) / 32), 256, tail, st>>>(a);
+  if (!SPLIT) return 0;
+  if (dsa_reserve_lds((const void*)combine, tail) != hipSuccess) return -2;
+  combine<<<dim3(a.S * (a.H / 32) * (shared ? DTILES : DTILES / 4)), 256, tail, st>>>(a);
   return 0;
 }
 

@@ -74,8 +74,8 @@ __device__ __forceinline__ void stage_requested(int (&v)[8], const int* __restri
   }
 }
 // ... and the list of tiles, by one wave
-__device__ __forceinline__ void list_tiles(int NT, const unsigned* tmask, int* tlist, int* ntile_s) {
-  const int lane = threadIdx.x & 63;
+__device__ __forceinline__ void list_tiles(int NT, const unsigned* tmask, int* tlist, int* ntile_s, int tid) {
+  const int lane = tid & 63;
   int base = 0;
   for (int t0 = 0; t0 < NT; t0 += 64) {
     const int t = t0 + lane;
@@ -172,8 +172,8 @@ __device__ __forceinline__ int stage_requested_ids(int (&v)[4], int K, int Skv, 
 __host__ __device__ inline size_t ids_lds_bytes(int K) { return (size_t)K * 4 + (size_t)(K / BI) * 8 + 16; }
 
 // Gather of one tile: thread (key = tid/8, sub = tid%8) moves slot `sub` of each of the 9 groups.
-__device__ __forceinline__ void gather_tile(const void* kv, const int* idx_s, int tile, unsigned lds_tile_base) {
-  const int tid = threadIdx.x, wave = tid >> 6;
+__device__ __forceinline__ void gather_tile(const void* kv, const int* idx_s, int tile, unsigned lds_tile_base, int tid) {
+  const int wave = tid >> 6;
   const int gkey = tid >> 3, gsub = tid & 7;
   int kid = idx_s[tile * BI + gkey];
   kid = kid < 0 ? 0 : kid;
@@ -181,6 +181,10 @@ __device__ __forceinline__ void gather_tile(const void* kv, const int* idx_s, in
   const unsigned lb = __builtin_amdgcn_readfirstlane(lds_tile_base + (unsigned)(wave * 1024));
 #pragma unroll
   for (int grp = 0; grp < 9; grp++) dma16(lb + grp * GRP_BYTES, goff + grp * 128, kv);
+}
+
+__device__ __forceinline__ void gather_tile(const void* kv, const int* idx_s, int tile, unsigned lds_tile_base) {
+  gather_tile(kv, idx_s, tile, lds_tile_base, (int)threadIdx.x);
 }
 
 // 32 consecutive rows of an array, in the layout of a tile: thread (row = tid / 8, sub = tid % 8).  Every transfer moves whole
@@ -205,9 +209,9 @@ struct LaneOffsets {
   unsigned row_off[4];
   unsigned tr_off[2][2][2];
 };
-__device__ __forceinline__ LaneOffsets lane_offsets() {
+__device__ __forceinline__ LaneOffsets lane_offsets(int tid) {
   LaneOffsets o;
-  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int lane = tid & 63, r = lane & 31, g = lane >> 5;
 #pragma unroll
   for (int j = 0; j < 4; j++) o.row_off[j] = (unsigned)(r * 128 + (((2 * j + g) ^ swz(r)) << 4));
   const int blk = lane >> 4, ii = lane & 15;
@@ -223,6 +227,8 @@ __device__ __forceinline__ LaneOffsets lane_offsets() {
     }
   return o;
 }
+
+__device__ __forceinline__ LaneOffsets lane_offsets() { return lane_offsets((int)threadIdx.x); }
 
 // ---------------------------------------------------------------------------------------------
 // MFMA through inline asm with explicit register files ("v" architectural, "a" accumulation).

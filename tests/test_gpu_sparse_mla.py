@@ -235,6 +235,8 @@ def test_forward_shares_a_query_among_workgroups(gpu, S, H, K, q_start, skv):
     (260, 128, 192, 0, None),         # up to six tiles, fewer than the ring in the early rows; a second round of workgroups
     (170, 96, 320, 400, 500),         # the fourth 32-head block is not there
     (300, 128, 768, 0, None),         # from one tile in the early rows to 24
+    (110, 128, 512, 900, None),       # two tiles at a time by 64 heads, without ranges: the blocks done again are the second group's
+    (110, 96, 512, 900, None),
     (48, 96, 2048, 3000, None),       # in ranges of slots, by 64 heads
     (88, 96, 2048, 3000, None),       # in ranges, in two roles
     (70, 128, 2048, 0, 2100),         # the same; ranges without a tile in the early rows
