@@ -591,8 +591,14 @@ class ApplyMLARotaryEmbAbsorbKV(torch.autograd.Function):
         dk3 = dk.contiguous().view(-1, nheads, emb_dim + k_dim)
         T = dk3.shape[0]
         d_kv = dk3.new_empty(T, nheads, k_dim)
-        ops.rope_rows(None, None, None, None, 0, 0, main_src=dk3[:, :, :k_dim], main_dst=d_kv)
-        d_emb = ops.rope_headsum_inverse(dk3[:, :, k_dim:], cos, sin, out_pairing, positions, batch).view(T, 1, emb_dim)
+        if nheads == 1 and emb_dim <= 256 and emb_dim & (emb_dim - 1) == 0:
+            # the absorbed key has one head: nothing to sum, and both parts go in one launch (4096 tokens 4.7 + 5.0 -> 4.9 us)
+            d_emb = dk3.new_empty(T, 1, emb_dim)
+            ops.rope_rows(dk3[:, :, k_dim:], d_emb, cos, sin, out_pairing, ops.ROPE_ADJACENT, True, positions, batch,
+                          main_src=dk3[:, :, :k_dim], main_dst=d_kv)
+        else:
+            ops.rope_rows(None, None, None, None, 0, 0, main_src=dk3[:, :, :k_dim], main_dst=d_kv)
+            d_emb = ops.rope_headsum_inverse(dk3[:, :, k_dim:], cos, sin, out_pairing, positions, batch).view(T, 1, emb_dim)
         if max_seqlen is not None:
             d_kv = d_kv.view(max_seqlen, batch, nheads, k_dim)
             d_emb = d_emb.view(max_seqlen, batch, 1, emb_dim)

@@ -123,3 +123,25 @@ def test_argument_errors_of_the_rope_entry(gpu):
         ops.rope_rows(x[:, :, 8:], x[:, :, 8:], cos, cos, 0, 0)
     with pytest.raises(ValueError):
         ops.rope_rows(x.float(), x.float(), cos, cos, 0, 0)
+
+
+@pytest.mark.parametrize("inter", [False, True])
+@pytest.mark.parametrize("s,b,kd,thd", [(1, 1, 512, False), (37, 2, 512, False), (75, 1, 512, True), (70, 1, 128, True), (4099, 1, 512, False)])
+def test_gradient_of_a_key_of_one_head(gpu, inter, s, b, kd, thd):
+    """Both parts in one launch: bit for bit the copy and the sum over heads, which has one term."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import fused_apply_mla_rope_for_absorb_kv
+
+    T, emb = s * b, 64
+    cos, sin = (t.to(gpu) for t in _tables(max(T, 90), emb, inter, BF if inter else torch.float32, True))
+    cu = torch.tensor([0, 5, T], dtype=torch.int32, device=gpu) if thd else None
+    kv = _rand(*((s, 1, kd) if thd else (s, b, 1, kd)), seed=1).to(gpu).requires_grad_(True)
+    ke = _rand(*((s, 1, emb) if thd else (s, b, 1, emb)), seed=2).to(gpu).requires_grad_(True)
+    key = fused_apply_mla_rope_for_absorb_kv(kv, ke, cos, sin, emb, kd, cu, 0, 1, inter)
+    g = _rand(*key.shape, seed=3).to(gpu)
+    dkv, demb = torch.autograd.grad(key, [kv, ke], g)
+    assert dkv.shape == kv.shape and demb.shape == ke.shape and torch.equal(dkv, g[..., :kd])
+    pos = ops.thd_positions(cu, T) if thd else None
+    pairing = ops.ROPE_ADJACENT if inter else ops.ROPE_SPLIT
+    want = ops.rope_headsum_inverse(g.view(T, 1, kd + emb)[:, :, kd:], cos, sin, pairing, pos, b)
+    assert torch.equal(demb.view(T, emb), want)
