@@ -205,6 +205,145 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
     target[i * K + t] = ((acc_s[t] + acc_s[K + t]) + (acc_s[2 * K + t] + acc_s[3 * K + t])) * invh;
 }
 
+// Up to 512 slots: a wave works four heads at a time (up to 256 slots eight, two of them side by side in its half-waves), whose maxima
+// and sums are reduced together: two steps leave each row of 16 lanes with one head, four more finish all four, where six for each head
+// by itself cost as much as the exponentials.  The sums' reciprocals are divided once for four heads.  Issue-bound like the kernel above.
+// A lane of a half-wave owns 8 consecutive slots.
+// us, that kernel and this: 2077 queries x 64 heads x 512 slots 31.9 and 28.1, 8192 x 128 x 512 195 and 182 (5.9 TB/s), 7951 x 32 x 256
+// 42.4 and 26.0, 1192 x 64 x 256 17.9 and 10.8, 2077 x 64 x 128 26.5 and 12.8, 1024 x 16 x 256 7 and 7.
+__device__ __forceinline__ void trade_halves(float& x, float& y) {       // the upper half-wave of x against the lower one of y
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+}
+__device__ __forceinline__ void trade_rows(float& x, float& y) {         // rows of 16 lanes 1 and 3 of x against rows 0 and 2 of y
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+}
+// f over the lanes of a wave (HALVES: of each half-wave) for v[0 .. 3]; v[j] comes back in every lane that it is over.
+template <bool HALVES, class F, class G>
+__device__ __forceinline__ void fold4(float (&v)[4], F f, G last) {
+  float a, b;
+  if (!HALVES) {                             // row 2 i + k of 16 lanes ends with head 2 k + i
+    trade_halves(v[0], v[1]);
+    a = f(v[0], v[1]);                       // the lower half-wave has head 0, the upper one head 1
+    trade_halves(v[2], v[3]);
+    b = f(v[2], v[3]);
+    trade_rows(a, b);
+    a = f(a, b);
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) a = f(a, xor16(a, m));
+    a = last(a);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      v[j] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 32 * (j & 1) + 16 * (j >> 1)));
+  } else {                                   // rows 0 and 2 end with v[0] (v[2]) of the half-wave, rows 1 and 3 with v[1] (v[3])
+    trade_rows(v[0], v[1]);
+    a = f(v[0], v[1]);
+    trade_rows(v[2], v[3]);
+    b = f(v[2], v[3]);
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) { a = f(a, xor16(a, m)); b = f(b, xor16(b, m)); }
+    a = last(a);
+    b = last(b);
+    v[0] = v[1] = a;
+    trade_rows(v[0], v[1]);                  // v[0]: rows 0, 0, 2, 2; v[1]: rows 1, 1, 3, 3
+    v[2] = v[3] = b;
+    trade_rows(v[2], v[3]);
+  }
+}
+
+template <bool HALVES, bool STREAMED, bool LIVE>
+__global__ __launch_bounds__(256) void attn_dist_few_kernel(const unsigned short* __restrict__ p_out, int H, int K, int64_t ld_s, int64_t ld_h, float c2,
+                                                            float* __restrict__ target, const int* __restrict__ ids, int Skv, int q_start) {
+  extern __shared__ float acc_s[];           // [4 waves][2 half-waves if HALVES][K]
+  constexpr int SIDE = HALVES ? 2 : 1;       // heads side by side
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, side = HALVES ? lane >> 5 : 0;
+  const int t = 8 * (HALVES ? lane & 31 : lane);
+  const int64_t i = blockIdx.x;
+  bool has = t < K;
+  if constexpr (LIVE) {
+    const int last = (int)min((int64_t)Skv - 1, (int64_t)q_start + i);
+    const int at = min(t, K - 8);
+    const int4 a = *(const int4*)(ids + i * K + at), b = *(const int4*)(ids + i * K + at + 4);
+    const int id[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    bool any = false;
+#pragma unroll
+    for (int e = 0; e < 8; e++) any |= id[e] >= 0 && id[e] <= last;
+    const unsigned long long m = __ballot(any && t < K);
+    has = (m >> (lane & ~3)) & 0xfull;       // four lanes share a tile
+  }
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc[e] = 0.f;
+  struct Raw { uint4 x[4]; };
+  auto fetch = [&](int h0, Raw& r) {         // heads h0 + SIDE j + side; those beyond the last one as the last one, without weight
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const i32x4* at = (const i32x4*)(p_out + i * ld_s + min(h0 + SIDE * j + side, H - 1) * ld_h + t);
+      if (has) r.x[j] = __builtin_bit_cast(uint4, STREAMED ? __builtin_nontemporal_load(at) : *at);
+    }
+  };
+  auto heads = [&](int h0, const Raw& r) {
+    float z[4][8], m[4], s[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const unsigned w[4] = {r.x[j].x, r.x[j].y, r.x[j].z, r.x[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        z[j][2 * e] = __builtin_bit_cast(float, w[e] << 16);
+        z[j][2 * e + 1] = __builtin_bit_cast(float, w[e] & 0xffff0000u);
+      }
+      m[j] = z[j][0];
+#pragma unroll
+      for (int e = 1; e < 8; e++) m[j] = fmaxf(m[j], z[j][e]);
+    }
+    fold4<HALVES>(m, [](float x, float y) { return fmaxf(x, y); }, [](float x) { return x; });
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float off = -m[j] * c2;          // (a head with no valid slot contributes nothing below)
+      s[j] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) { z[j][e] = __builtin_amdgcn_exp2f(fmaf(z[j][e], c2, off)); s[j] += z[j][e]; }
+    }
+    fold4<HALVES>(s, [](float x, float y) { return x + y; }, [](float x) { return 1.0f / x; });
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const bool in = h0 + SIDE * j + side < H && m[j] != -INFINITY;
+      if (__ballot(!in) == 0ull) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += z[j][e] * s[j];
+      } else if (in) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += z[j][e] * s[j];
+      }
+    }
+  };
+  Raw r0, r1;
+#pragma unroll
+  for (int j = 0; j < 4; j++) r0.x[j] = r1.x[j] = make_uint4(0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u);      // -inf where nothing is read
+  constexpr int STEP = 4 * SIDE;             // heads of a wave at a time
+  fetch(STEP * wave, r0);
+  for (int h = STEP * wave; h < H; h += 8 * STEP) {
+    fetch(h + 4 * STEP, r1);
+    heads(h, r0);
+    if (h + 4 * STEP < H) {
+      fetch(h + 8 * STEP, r0);
+      heads(h + 4 * STEP, r1);
+    }
+  }
+  if (t < K) {
+    float* const own = acc_s + (wave * SIDE + side) * K + t;
+    *(f32x4*)own = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    *(f32x4*)(own + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+  }
+  __syncthreads();
+  const float invh = 1.0f / (float)H;
+  for (int t = threadIdx.x; t < K; t += 256) {
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4 * SIDE; k++) sum += acc_s[k * K + t];
+    target[i * K + t] = sum * invh;
+  }
+}
+
 // ids: null, or those whose dead tiles have no logits
 template <bool F32>
 int launch(const void* p_out, int S, int H, int K, int64_t ld_s, int64_t ld_h, float sm_scale, float* target, const int* ids, int Skv,
@@ -215,6 +354,21 @@ int launch(const void* p_out, int S, int H, int K, int64_t ld_s, int64_t ld_h, f
   if (vec) {
     const int nc = (K + 511) / 512;
     const bool streamed = (int64_t)S * H * K * (F32 ? 4 : 2) > (256ll << 20);
+    if constexpr (!F32) {
+      if (nc == 1 && H >= 8) {               // fewer heads: a wave's four would be one and its copies
+        const bool halves = K <= 256;
+        if (halves) smem *= 2;
+#define DSA_FEW_LAUNCH(HV, STR, LIVE) \
+        attn_dist_few_kernel<HV, STR, LIVE><<<dim3(S), dim3(256), smem, st>>>((const unsigned short*)p_out, H, K, ld_s, ld_h, c2, target, ids, Skv, q_start)
+#define DSA_FEW_CASE(HV) \
+        if (ids) { if (streamed) DSA_FEW_LAUNCH(HV, true, true); else DSA_FEW_LAUNCH(HV, false, true); } \
+        else if (streamed) DSA_FEW_LAUNCH(HV, true, false); else DSA_FEW_LAUNCH(HV, false, false)
+        if (halves) { DSA_FEW_CASE(true); } else { DSA_FEW_CASE(false); }
+#undef DSA_FEW_CASE
+#undef DSA_FEW_LAUNCH
+        return 0;
+      }
+    }
 #define DSA_ADV_LAUNCH(N, STR, LIVE) \
     attn_dist_vec_kernel<F32, N, STR, LIVE><<<dim3(S), dim3(256), smem, st>>>(p_out, H, K, ld_s, ld_h, c2, target, ids, Skv, q_start)
 #define DSA_ADV_CASE(N) \

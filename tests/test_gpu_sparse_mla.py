@@ -1058,3 +1058,36 @@ def test_recomputed_distribution_refuses_host_tensors(gpu):
     for host in range(4):
         with pytest.raises(RuntimeError, match="HIP device"):
             ops.attn_dist_qk(*[t if i == host else t.to(gpu) for i, t in enumerate(args)], 0, 0.1)
+
+
+@pytest.mark.parametrize("H", [7, 8, 9, 33, 64, 128])
+@pytest.mark.parametrize("K", [8, 64, 200, 256, 264, 512])
+def test_attn_dist_of_short_lists(gpu, H, K):
+    """Rows of up to 512 slots, four heads of a wave together and up to 256 slots two side by side: against 64 bits, with heads and slots of
+    -inf, a head far above the others, strided rows; NaN and +inf reach their query alone."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(H * K)
+    S, scale = 37, 192 ** -0.5
+    wide = (torch.randn(S, H + 2, K + 8, generator=g) * 30).to(torch.bfloat16)
+    p = wide[:, 1:H + 1, :K]
+    p[torch.rand(S, H, K, generator=g) < 0.2] = -float("inf")
+    p[3, : H // 2] = -float("inf")
+    p[4] = -float("inf")
+    p[5, :, K // 2:] = -float("inf")
+    p[6, H - 1] *= 100
+    pd = wide.to(gpu)[:, 1:H + 1, :K]
+    got = ops.attn_dist(pd.contiguous(), scale)
+    z = p.double() * scale
+    ref = torch.nan_to_num(torch.softmax(z, -1), 0.0).sum(1) / H        # a head without a slot adds nothing
+    # a term's exponent and product in 32 bits, sums of K and H of them
+    assert (got.double().cpu() - ref).abs().max().item() <= 2.0 ** -23 * (8 + 64)
+    assert ((got.double().cpu() - ref).abs() <= 2e-5 * ref + 1e-30).all()
+    assert (got[4] == 0).all()
+    bad = pd.contiguous().clone()
+    bad[7, H - 1, K - 1] = float("nan")
+    bad[8, 0, 0] = float("inf")
+    mixed = ops.attn_dist(bad, scale)
+    keep = torch.ones(S, dtype=torch.bool)
+    keep[7:9] = False
+    assert torch.equal(mixed[keep.to(gpu)], got[keep.to(gpu)]) and torch.isnan(mixed[7]).any() and torch.isnan(mixed[8]).any()
