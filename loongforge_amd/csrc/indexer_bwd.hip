@@ -1039,7 +1039,8 @@ __global__ __launch_bounds__(256) void indexer_chunk_sum_kernel(const float* __r
 // Gradients of the keys' projection from the summed payload gradients: the same steps as for the queries, then back
 // through the LayerNorm (fp32).  16 lanes per row; a workgroup takes every gridDim-th group of 16 rows and leaves its
 // share of the LayerNorm's parameter gradients in part[block][2][128] (summed in block order by the next kernel).
-// Bound by its launch (8192 keys: 6 MB).
+// Bound by its chain of loads, 4 us a group of rows; up to 512 workgroups, one group each up to 8192 keys (with 128 of them 2077 keys
+// 11.6 and now 7.6 us, 6710 keys 22.3 and 8.9; the parameters' sums behind it by 16 groups of threads for 4).
 struct KeyArgs {
   const float* d_k8;
   const float* k_scale;
@@ -1052,7 +1053,7 @@ struct KeyArgs {
   void* d_k; int k_f32, dim;
   float* part;
 };
-constexpr int KEY_BLOCKS = 128;
+constexpr int KEY_BLOCKS = 512;
 
 __device__ __forceinline__ float sum16(float v) {
 #pragma unroll
@@ -1116,18 +1117,20 @@ __global__ __launch_bounds__(256) void indexer_key_finish_kernel(const KeyArgs A
   A.part[(size_t)blockIdx.x * 2 * D + threadIdx.x] = s;
 }
 
-__global__ __launch_bounds__(256) void indexer_ln_sum_kernel(const float* __restrict__ part, int blocks, float* __restrict__ d_w,
-                                                             float* __restrict__ d_b) {
-  __shared__ float red_s[4][64];
+constexpr int LN_GROUPS = 16;
+__global__ __launch_bounds__(64 * LN_GROUPS) void indexer_ln_sum_kernel(const float* __restrict__ part, int blocks, float* __restrict__ d_w,
+                                                                        float* __restrict__ d_b) {
+  __shared__ float red_s[LN_GROUPS][64];
   const int c = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;      // column of [2][128]
   float s = 0.f;
 #pragma unroll 8
-  for (int b = grp; b < blocks; b += 4) s += part[(size_t)b * 2 * D + c];
+  for (int b = grp; b < blocks; b += LN_GROUPS) s += part[(size_t)b * 2 * D + c];
   red_s[grp][threadIdx.x & 63] = s;
   __syncthreads();
   if (grp == 0) {
-    const int t = threadIdx.x;
-    s = (red_s[0][t] + red_s[1][t]) + (red_s[2][t] + red_s[3][t]);
+    s = 0.f;
+#pragma unroll
+    for (int k = 0; k < LN_GROUPS; k++) s += red_s[k][threadIdx.x];
     if (c < D) d_w[c] = s; else d_b[c - D] = s;
   }
 }
@@ -1241,7 +1244,7 @@ int finish_keys(const char* name, const KeyFinish* kf, int Sk, hipStream_t st) {
   if (!kf) return DSA_OK;
   const int blocks = dsa_cdiv(Sk, 16) < KEY_BLOCKS ? dsa_cdiv(Sk, 16) : KEY_BLOCKS;
   indexer_key_finish_kernel<<<dim3(blocks), dim3(256), 0, st>>>(kf->key);
-  if (kf->key.k_in) indexer_ln_sum_kernel<<<dim3(4), dim3(256), 0, st>>>(kf->key.part, blocks, kf->d_ln_w, kf->d_ln_b);
+  if (kf->key.k_in) indexer_ln_sum_kernel<<<dim3(4), dim3(64 * LN_GROUPS), 0, st>>>(kf->key.part, blocks, kf->d_ln_w, kf->d_ln_b);
   DSA_CHECK_LAUNCH("indexer_bwd(keys)");
   return DSA_OK;
 }
