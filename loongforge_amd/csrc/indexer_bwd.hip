@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(256) void indexer_chunk_sum_kernel(const float* __r
 // through the LayerNorm (fp32).  16 lanes per row; a workgroup takes every gridDim-th group of 16 rows and leaves its
 // share of the LayerNorm's parameter gradients in part[block][2][128] (summed in block order by the next kernel).
 // Bound by its chain of loads, 4 us a group of rows; up to 512 workgroups, one group each up to 8192 keys (with 128 of them 2077 keys
-// 11.6 and now 7.6 us, 6710 keys 22.3 and 8.9; the parameters' sums behind it by 16 groups of threads for 4).
+// 11.6 and now 7.9 us, 8192 keys 22.3 and 9.7; the parameters' sums behind it by 16 groups of threads for 4).
 struct KeyArgs {
   const float* d_k8;
   const float* k_scale;

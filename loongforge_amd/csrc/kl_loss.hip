@@ -33,34 +33,50 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* scratch) {
   b = (scratch[4] + scratch[5]) + (scratch[6] + scratch[7]);
 }
 
-template <int NE>   // slots per thread: K <= NE * BLOCK
-__global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict__ scores, int64_t ld_s,
-                                                        const float* __restrict__ target, int64_t ld_t, int K, float eps,
-                                                        float* __restrict__ row_loss, float* __restrict__ grad) {
-  __shared__ float scratch[8];
-  const int tid = threadIdx.x;
-  const int64_t row = blockIdx.x;
+// Sums over the threads that share a row: a workgroup, or a wave by itself.
+struct BlockRow {
+  float* scratch;
+  __device__ float max(float v) const { return block_max(v, scratch); }
+  __device__ void sum2(float& a, float& b) const { block_sum2(a, b, scratch); }
+};
+struct WaveRow {
+  __device__ float max(float v) const {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, o > 8 ? __shfl_xor(v, o, 64) : xor16(v, o));
+    return v;
+  }
+  __device__ void sum2(float& a, float& b) const {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { a += o > 8 ? __shfl_xor(a, o, 64) : xor16(a, o); b += o > 8 ? __shfl_xor(b, o, 64) : xor16(b, o); }
+  }
+};
+
+// thread tid of the NT that share a row has its slots tid, tid + NT, ..: K <= NE * NT
+template <int NE, int NT, class Row>
+__device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, const float* __restrict__ scores, int64_t ld_s,
+                                       const float* __restrict__ target, int64_t ld_t, int K, float eps, float* __restrict__ row_loss,
+                                       float* __restrict__ grad) {
   const float* sp = scores + row * ld_s;
   const float* tp = target + row * ld_t;
   float s[NE], u[NE];
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < NE; i++) {
-    const int t = tid + BLOCK * i;
+    const int t = tid + NT * i;
     s[i] = t < K ? sp[t] : -INFINITY;
     u[i] = (t < K ? tp[t] : 0.f) + eps;
     mx = fmaxf(mx, s[i]);
   }
-  mx = block_max(mx, scratch);
+  mx = over.max(mx);
   float z = 0.f, unused = 0.f;
 #pragma unroll
   for (int i = 0; i < NE; i++) { s[i] = expf(s[i] - mx); z += s[i]; }     // a row of -inf only: NaN, as torch.softmax
-  block_sum2(z, unused, scratch);
+  over.sum2(z, unused);
   const float inv = 1.0f / z;
   float loss = 0.f, inner = 0.f;
 #pragma unroll
   for (int i = 0; i < NE; i++) {
-    const int t = tid + BLOCK * i;
+    const int t = tid + NT * i;
     const float p = s[i] * inv;
     const float w = u[i] / (p + eps);
     if (t < K) {
@@ -70,13 +86,33 @@ __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict_
     s[i] = p;
     u[i] = w;
   }
-  block_sum2(loss, inner, scratch);
+  over.sum2(loss, inner);
 #pragma unroll
   for (int i = 0; i < NE; i++) {
-    const int t = tid + BLOCK * i;
+    const int t = tid + NT * i;
     if (t < K) grad[row * K + t] = s[i] * (inner - u[i]);
   }
   if (tid == 0) row_loss[row] = loss;
+}
+
+template <int NE>
+__global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict__ scores, int64_t ld_s,
+                                                        const float* __restrict__ target, int64_t ld_t, int K, float eps,
+                                                        float* __restrict__ row_loss, float* __restrict__ grad) {
+  __shared__ float scratch[8];
+  kl_row<NE, BLOCK>(BlockRow{scratch}, threadIdx.x, blockIdx.x, scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+}
+
+// Up to 512 slots: a row to a wave.  A workgroup to a row spent its time in three reductions with barriers and on eight slots a thread of
+// which one or two were there (7951 x 256 slots 30.4 us and 7.6 so, 2077 x 512 11.3 and 6.1, 300 x 256 4.8 and 3.3; beyond, four
+// slots a thread where that is enough: 4000 x 1024 18.8 and 13.8).
+template <int NE>
+__global__ __launch_bounds__(BLOCK) void kl_loss_wave_kernel(const float* __restrict__ scores, int64_t ld_s, const float* __restrict__ target,
+                                                             int64_t ld_t, int S, int K, float eps, float* __restrict__ row_loss,
+                                                             float* __restrict__ grad) {
+  const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6));
+  if (row >= S) return;
+  kl_row<NE, 64>(WaveRow{}, threadIdx.x & 63, row, scores, ld_s, target, ld_t, K, eps, row_loss, grad);
 }
 
 // *out = factor * sum of the rows' losses, in a fixed order.  One launch for the sum and the scaling behind it (5 us each).
@@ -137,7 +173,11 @@ extern "C" int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const floa
               (long long)ld_t, K);
   if (S == 0) return DSA_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (K <= 8 * BLOCK) kl_loss_kernel<8><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+  const dim3 waves(dsa_cdiv(S, BLOCK / 64));
+  if (K <= 256) kl_loss_wave_kernel<4><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, row_loss, grad);
+  else if (K <= 512) kl_loss_wave_kernel<8><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, row_loss, grad);
+  else if (K <= 4 * BLOCK) kl_loss_kernel<4><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+  else if (K <= 8 * BLOCK) kl_loss_kernel<8><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
   else kl_loss_kernel<32><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
   DSA_CHECK_LAUNCH("dsa_indexer_kl_loss");
   return DSA_OK;

@@ -26,7 +26,10 @@ def _case(S, K, seed, pad_from=None, target_kind="dist"):
 
 
 @pytest.mark.parametrize("S,K,padded,kind", [(37, 64, False, "dist"), (130, 2048, True, "dist"), (9, 200, True, "dist"),
-                                             (5, 4096, False, "onehot"), (3, 8192, True, "dist"), (1, 1, False, "dist")])
+                                             (5, 4096, False, "onehot"), (3, 8192, True, "dist"), (1, 1, False, "dist"),
+                                             # a row to a wave up to 512 slots, four slots a thread up to 1024
+                                             (6, 256, True, "dist"), (7, 257, False, "onehot"), (5, 512, True, "dist"),
+                                             (9, 513, True, "dist"), (5, 1024, True, "dist"), (6, 1025, True, "dist")])
 def test_kl_loss_and_gradient_match_the_oracle(gpu, S, K, padded, kind):
     from loongforge_amd import ops
 
