@@ -209,8 +209,8 @@ __global__ __launch_bounds__(256) void attn_dist_vec_kernel(const void* __restri
 // and sums are reduced together: two steps leave each row of 16 lanes with one head, four more finish all four, where six for each head
 // by itself cost as much as the exponentials.  The sums' reciprocals are divided once for four heads.  Issue-bound like the kernel above.
 // A lane of a half-wave owns 8 consecutive slots.
-// us, that kernel and this: 2077 queries x 64 heads x 512 slots 31.9 and 28.1, 8192 x 128 x 512 195 and 182 (5.9 TB/s), 7951 x 32 x 256
-// 42.4 and 26.0, 1192 x 64 x 256 17.9 and 10.8, 2077 x 64 x 128 26.5 and 12.8, 1024 x 16 x 256 7 and 7.
+// us, that kernel and this: 2077 queries x 64 heads x 512 slots 31.9 and 28.0, 8192 x 128 x 512 195 and 182 (5.9 TB/s), 7951 x 32 x 256
+// 42.4 and 26.9, 1192 x 64 x 256 17.9 and 10.9, 2077 x 64 x 128 26.5 and 12.8, 1024 x 16 x 256 7 and 7.
 __device__ __forceinline__ void trade_halves(float& x, float& y) {       // the upper half-wave of x against the lower one of y
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
 }
@@ -337,10 +337,13 @@ __global__ __launch_bounds__(256) void attn_dist_few_kernel(const unsigned short
   __syncthreads();
   const float invh = 1.0f / (float)H;
   for (int t = threadIdx.x; t < K; t += 256) {
-    float sum = 0.f;
+    float part[SIDE];
 #pragma unroll
-    for (int k = 0; k < 4 * SIDE; k++) sum += acc_s[k * K + t];
-    target[i * K + t] = sum * invh;
+    for (int k = 0; k < SIDE; k++) {
+      const float* const a = acc_s + 4 * k * K + t;
+      part[k] = (a[0] + a[K]) + (a[2 * K] + a[3 * K]);
+    }
+    target[i * K + t] = (HALVES ? part[0] + part[SIDE - 1] : part[0]) * invh;
   }
 }
 

@@ -51,6 +51,15 @@ struct WaveRow {
   }
 };
 
+// Sum of a thread's four or eight values in pairs, for a wave that has a row by itself to round no more than a workgroup's 256 threads
+template <int N>
+__device__ __forceinline__ float pairs_sum(const float (&v)[N]) {
+  static_assert(N == 4 || N == 8);
+  const float a = (v[0] + v[1]) + (v[2] + v[3]);
+  if constexpr (N == 8) return a + ((v[4] + v[5]) + (v[6] + v[7]));
+  return a;
+}
+
 // thread tid of the NT that share a row has its slots tid, tid + NT, ..: K <= NE * NT
 template <int NE, int NT, class Row>
 __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, const float* __restrict__ scores, int64_t ld_s,
@@ -68,23 +77,35 @@ __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, co
     mx = fmaxf(mx, s[i]);
   }
   mx = over.max(mx);
+  constexpr bool WAVE = NT == 64;
   float z = 0.f, unused = 0.f;
 #pragma unroll
-  for (int i = 0; i < NE; i++) { s[i] = expf(s[i] - mx); z += s[i]; }     // a row of -inf only: NaN, as torch.softmax
+  for (int i = 0; i < NE; i++) {                                          // a row of -inf only: NaN, as torch.softmax
+    s[i] = expf(s[i] - mx);
+    if (!WAVE) z += s[i];
+  }
+  if constexpr (WAVE) z = pairs_sum(s);
   over.sum2(z, unused);
   const float inv = 1.0f / z;
-  float loss = 0.f, inner = 0.f;
+  float loss = 0.f, inner = 0.f, l[WAVE ? NE : 1], n[WAVE ? NE : 1];
 #pragma unroll
   for (int i = 0; i < NE; i++) {
     const int t = tid + NT * i;
     const float p = s[i] * inv;
     const float w = u[i] / (p + eps);
-    if (t < K) {
+    if constexpr (WAVE) {
+      l[i] = t < K ? u[i] * (logf(u[i]) - logf(p + eps)) : 0.f;
+      n[i] = t < K ? w * p : 0.f;
+    } else if (t < K) {
       loss += u[i] * (logf(u[i]) - logf(p + eps));
       inner += w * p;
     }
     s[i] = p;
     u[i] = w;
+  }
+  if constexpr (WAVE) {
+    loss = pairs_sum(l);
+    inner = pairs_sum(n);
   }
   over.sum2(loss, inner);
 #pragma unroll
