@@ -1213,19 +1213,21 @@ DensePlan dense_plan(int S, int Hi, int Sk, int span, size_t budget) {
 // a key that the query sees 0.0225, a pair with a row of its own 0.11 against 0.031 for its part in d_q8 alone, the key-sorted order
 // 11 more than the scattered factors; 10 us a call for the longer chain.  Whole call, rows / key tiles in us: 8192 queries x 2048 slots of a
 // causal window 2070 / 1640, 12 000 x 2048 2800 / 2520, x 1024 1540 / 2190, x 256 673 / 1918, in five documents x 512 942 / 899; 3072 x 512 of
-// 768 compressed keys 246 / 185; 500 x 512 of 6000 keys 71 / 126.  span: the most keys that a query sees, 0 if not known.
-bool by_key_tiles(int S, int Sk, int K, int span) {
+// 768 compressed keys 246 / 185; 500 x 512 of 6000 keys 71 / 126.  32 heads: 0.017 (half the products, the same
+// lists; causal window, rows / key tiles: 4000 x 512 300 / 258, 6000 x 512 454 / 452, 9000 x 512 675 / 836, x 1024 1049 / 898, 12 000 x 1024
+// 1414 / 1426, 3000 x 256 143 / 169).  span: the most keys that a query sees, 0 if not known.
+bool by_key_tiles(int S, int Hi, int Sk, int K, int span) {
   const float seen = span > 0 && span < Sk ? span : Sk, queries = S > 0 ? S : 1;
   const float visible = queries < seen ? seen - 0.5f * queries : 0.5f * seen;       // the window of the last queries, or one that grows from nothing
   const float selected = queries < seen ? fminf(K, visible) : K < seen ? K - 0.5f * K * K / seen : visible;
-  return 0.0225f * (visible + 0.8f * KT) + 10000.f / queries < 11.f + 0.079f * selected;
+  return (Hi <= 32 ? 0.017f : 0.0225f) * (visible + 0.8f * KT) + 10000.f / queries < 11.f + 0.079f * selected;
 }
 
 }  // namespace
 
 static size_t bwd_workspace(int S, int Hi, int Sk, int K, int span) {
   if (S <= 0 || Sk <= 0 || K <= 0) return 0;
-  if (by_key_tiles(S, Sk, K, span)) return dense_plan(S, Hi <= 32 ? 32 : 64, Sk, span, DEFAULT_BUDGET).total;
+  if (by_key_tiles(S, Hi, Sk, K, span)) return dense_plan(S, Hi <= 32 ? 32 : 64, Sk, span, DEFAULT_BUDGET).total;
   return make_plan(S, Sk, K, DEFAULT_BUDGET).total;
 }
 
@@ -1296,7 +1298,7 @@ int run_bwd(const char* name, BwdArgs A, int S, int Hi, int span, float* d_k8, c
               ((uintptr_t)A.d_q8 % 16) == 0 && ((uintptr_t)A.d_q % 16) == 0 && ((uintptr_t)d_k8 % 16) == 0 && ((uintptr_t)workspace % 256) == 0,
               "%s: misaligned pointer", name);
   hipStream_t st = (hipStream_t)stream;
-  if (workspace != nullptr && by_key_tiles(S, Sk, K, span)) {
+  if (workspace != nullptr && by_key_tiles(S, Hi, Sk, K, span)) {
     const DensePlan p = dense_plan(S > 0 ? S : 1, Hi, Sk, span, workspace_bytes);
     if (p.total <= workspace_bytes) return run_by_key_tiles(name, A, p, S, Hi, d_k8, kf, (unsigned char*)workspace, st);
   }

@@ -284,3 +284,13 @@ def test_key_gradients_by_key_tiles_with_a_repeated_id(gpu):
     g, q8, k8, ksc, w, ids, _, _ = _pairs(1600, 4500, 128, 32, 4, 1.0)
     ids[1599, 100] = ids[1599, 3]
     assert torch.isnan(_grads(gpu, g, q8, k8, ksc, w, ids, 1)[1]).all()
+
+
+@pytest.mark.parametrize("Hi", [32, 64])
+def test_key_gradients_where_the_number_of_heads_decides(gpu, Hi):
+    """900 visible keys: whole key tiles for 32 heads, rows for 64, whose sums are the same bits with and without a span."""
+    g, q8, k8, ksc, w, ids, _, _ = _pairs(1600, 4500, 128, Hi, 5, 1.0)
+    rows, chosen = _grads(gpu, g, q8, k8, ksc, w, ids, 0), _grads(gpu, g, q8, k8, ksc, w, ids, 900)
+    for a, b in zip(rows, chosen):
+        assert (a - b).norm() <= 1e-2 * a.norm()       # the rows' bf16 pairs, as in the comparisons above
+    assert torch.equal(rows[1], chosen[1]) == (Hi == 64)
