@@ -25,6 +25,8 @@
 // instructions per wave on two tiles and are then bound by the gather.  A query's heads may also be spread over several
 // workgroups, and its slots over `ksplit` of them (few queries: one workgroup per query would leave most of the 256
 // compute units idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
+#include <type_traits>
+
 #include "mla_tile.h"
 
 // attn_dist.hip
@@ -474,16 +476,26 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   bool again = __ballot(overflow) != 0ull;   // the same for all lanes of a wave
 
-  f32x4* box = (f32x4*)(smem + (size_t)sub * NDT * 4096) + lane;
-  // ---- two streams: the second one's sums reach the first through the (now free) tile ring, scaled to the
-  // common reference point; the first one's waves finish --------------------------------------------------
+  // ---- two streams: their sums are merged through the (now free) tile ring, scaled to the common reference point.  Each stream's
+  // wave sends the other's half of the column tiles and finishes its own, so that all four waves store: with the second stream's
+  // sums all sent to the first, two waves stored the 131 KB of 64 heads while two had ended. ---------------------------------
   __syncthreads();                         // the last tiles and the id arrays have been read
   static_assert(2 * NDT * 4096 + 1024 + 8 <= RING, "the hand-over fits the tile ring");
-  float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the two waves' boxes
+  float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the waves' boxes
   if (g == 0) {
     ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
     ml[((stream * 2 + sub) * 32 + r) * 2 + 1] = l_tot;
   }
+  constexpr int HALF = NDT / 2;
+  auto box_of = [&](int to) { return (f32x4*)(smem + (size_t)((to * 2 + sub) * HALF) * 4096) + lane; };
+  auto send = [&](auto first, int to) {
+    f32x4* const box = box_of(to);
+#pragma unroll
+    for (int i = 0; i < HALF; i++) store_partial(oacc[decltype(first)::value + i], box + i * 256);
+  };
+  if (stream == 0) send(std::integral_constant<int, HALF>{}, 1);
+  else send(std::integral_constant<int, 0>{}, 0);
+  unsigned* const marked_s = (unsigned*)(ml + 256);        // mode 1: the head blocks to be done again
   __syncthreads();
   const float m_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2], l_o = ml[(((stream ^ 1) * 2 + sub) * 32 + r) * 2 + 1];
   again |= is_marked(m_o);
@@ -497,40 +509,39 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
     return;
   }
+  // the first stream's terms first on both sides: a head's denominator has the same bits in both of its waves
   const float nm = fmaxf(m_ref, m_o);
-  const float f = __builtin_amdgcn_exp2f(m_ref - nm);
-  l_tot = l_tot * f + l_o * __builtin_amdgcn_exp2f(m_o - nm);
+  const float f_own = __builtin_amdgcn_exp2f(m_ref - nm), f_other = __builtin_amdgcn_exp2f(m_o - nm);
+  const float f0 = stream == 0 ? f_own : f_other, f1 = stream == 0 ? f_other : f_own;
+  l_tot = fmaf(stream == 0 ? l_tot : l_o, f0, (stream == 0 ? l_o : l_tot) * f1);
   m_ref = nm;
-  if (stream == 1) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        f32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = oacc[dt][4 * j + e] * f;
-        box[(dt * 4 + j) * 64] = v;
-      }
-  }
-  unsigned* const marked_s = (unsigned*)(ml + 256);        // mode 1: the head blocks to be done again
-  if (MODE == 1 && !SPLIT && stream == 1 && lane == 0) marked_s[sub] = again && head_ok;
-  __syncthreads();
-  if (stream == 1 && (MODE == 2 || SPLIT)) return;
-  const float mine = f;
-  auto merged = [&](int dt) {                // column tile dt of the wave's heads, both streams
-    f32x16 t;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const f32x4 v = box[(dt * 4 + j) * 64];
-#pragma unroll
-      for (int e = 0; e < 4; e++) t[4 * j + e] = fmaf(oacc[dt][4 * j + e], mine, v[e]);
-    }
-    return t;
-  };
 
   // ---- epilogue: the wave's column tiles, normalised to out[i,h,:] with lse[i,h], or as they are to the workspace ----
-  const bool stats = g == 0 && (MODE != 2 || sub == 0);
+  const bool stats = stream == 0 && g == 0 && (MODE != 2 || sub == 0);
   const int dt0 = MODE == 2 ? sub * NDT : 0;
+  auto finish = [&](auto first, auto write) {              // column tiles `first` .. of the wave's, both streams
+    constexpr int FIRST = decltype(first)::value;
+    const f32x4* const box = box_of(FIRST == 0 ? 0 : 1);
+#pragma unroll
+    for (int i = 0; i < HALF; i++) {
+      f32x16 t;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const f32x4 v = box[(i * 4 + j) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float own = oacc[FIRST + i][4 * j + e];
+          t[4 * j + e] = FIRST == 0 ? fmaf(own, f0, v[e] * f1) : fmaf(v[e], f0, own * f1);
+        }
+      }
+      write(t, FIRST + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto finish_mine = [&](auto write) {
+    if (stream == 0) finish(std::integral_constant<int, 0>{}, write);
+    else finish(std::integral_constant<int, HALF>{}, write);
+  };
   if (SPLIT) {
     if (!head_ok) return;                    // the same for all lanes of a wave
     float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
@@ -540,24 +551,18 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     }
     if (stats) { part_ml[0] = m_ref; part_ml[1] = l_tot; }
     f32x4* po = a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt0) * 256 + lane;
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++) {
-      store_partial(merged(dt), po + dt * 256);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    finish_mine([&](const f32x16& t, int dt) { store_partial(t, po + dt * 256); });
     return;
   }
-  if (head_ok && !again && stream == 0) {
+  if (head_ok && !again) {
     const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
     if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
     unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++) {
-      store_out(merged(dt), fin.inv, op + 32 * dt);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    finish_mine([&](const f32x16& t, int dt) { store_out(t, fin.inv, op + 32 * dt); });
   }
   if (MODE == 1) {
+    if (stream == 1 && lane == 0) marked_s[sub] = again && head_ok;
+    __syncthreads();
     const unsigned marked = __builtin_amdgcn_readfirstlane(marked_s[0] | (marked_s[1] << 1));
     if (marked) redo_marked<4>(a, qi, marked << (2 * hg), wave, lane_again());
   }
