@@ -184,6 +184,7 @@ __device__ __forceinline__ void bitonic_regs(float* outv, int* outi, unsigned lo
 // not depend on the order in which the atomics land.  Returns false without writing anything when
 // the row is unsuitable (no spread, or a crowded bin): the caller then takes the general path.
 constexpr int LIN_SPARE = 960;               // extra buffer entries for the threshold bin's surplus
+constexpr int LIN_PAD = 4;                   // and behind the last element: what the ranking reads at a time
 constexpr int REG_ROW = 8192 + 4 * 256;      // longest row (plus alignment slack) the register variant holds
 constexpr int REG_ROW_BIG = 32768 + 4 * 256; // the same for the variant with twice the registers
 constexpr int REG_ROW_WIDE = 9 * 4 * 1024;   // the same for the 1024-thread variant
@@ -193,10 +194,11 @@ constexpr int LIN_MAX_BIN = 256;             // largest segment ranked by pairwi
 
 // Threshold bin of a filled histogram (thread t owns bins [PER t, PER t + PER)), then the segment
 // starts written over the counts.  False when a bin is too crowded for the ranking step.
-template <int BL>
+template <int BL, int BINS>
 __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff, int& tbin, int& above, int& c) {
   const int tid = threadIdx.x;
-  constexpr int PER = HBINS / BL;
+  constexpr int PER = BINS / BL;
+  static_assert(PER % 4 == 0, "a thread's bins go by 16 bytes");
   int* found = scratch + 3 * NWAVES<BL>;
   int cnt[PER], local = 0;
 #pragma unroll
@@ -234,22 +236,52 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
   return !found[3] && c <= LIN_SPARE;
 }
 
-// Final position of every scattered element: hist[b] is the end of segment b by now.
+// Final position of every scattered element: hist[b] is the end of segment b by now.  The elements of later segments come behind it
+// and so do the LIN_PAD entries behind the last one, so that counting may run past the end of its segment: four entries at a time for
+// two elements of a thread together, as often as the longest segment of the wave asks for.  (One entry at a time in a loop of every
+// lane's own length is a chain of LDS trips.  us, then / now, with the number of bins by the row's length below: top-k 2048, 8192 causal
+// rows 102 / 95, 1500 rows of 7500 33.0 / 30.5, 8192 of 2048 84 / 76; top-k 512, 4000 rows of 1000 29.0 / 21.8, 2077 of up to 692
+// 15.6 / 12.6; up to 256 rows the same.)
 template <int BL, class BinOf>
 __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const int* hist, int filled, int keff, int K,
                                          int base_id, BinOf bin_of, float* sv, int* si) {
   const int tid = threadIdx.x;
-  for (int p = tid; p < filled; p += BL) {
-    const unsigned long long key = obuf[p];
-    const float v = sort_key_score(key);
-    const int b = bin_of(v);
-    const int start = b > 0 ? hist[b - 1] : 0, end = hist[b];
-    int rank = 0;
-    for (int j = start; j < end; j++) rank += obuf[j] < key;
-    const int pos = start + rank;
-    if (pos < keff) { sv[pos] = v; si[pos] = base_id + (int)(unsigned)key; }
+  constexpr int PAIR = 2;
+  for (int p0 = tid; p0 < filled; p0 += PAIR * BL) {
+    unsigned long long key[PAIR];
+    float v[PAIR];
+    int start[PAIR], end[PAIR], rank[PAIR];
+#pragma unroll
+    for (int u = 0; u < PAIR; u++) key[u] = obuf[min(p0 + u * BL, filled)];
+#pragma unroll
+    for (int u = 0; u < PAIR; u++) {
+      v[u] = sort_key_score(key[u]);
+      const bool in = p0 + u * BL < filled;
+      const int b = in ? bin_of(v[u]) : 0;
+      start[u] = in ? (b > 0 ? hist[b - 1] : 0) : filled;
+      end[u] = in ? hist[b] : filled;
+      rank[u] = 0;
+    }
+    int longest = max(end[0] - start[0], end[1] - start[1]);
+    for (int j = 0; __any(j < longest); j += LIN_PAD) {
+#pragma unroll
+      for (int u = 0; u < PAIR; u++) {
+        const unsigned long long* o = obuf + min(start[u] + j, filled);
+#pragma unroll
+        for (int i = 0; i < LIN_PAD; i++) rank[u] += o[i] < key[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PAIR; u++) {
+      const int pos = start[u] + rank[u];
+      if (pos < keff && p0 + u * BL < filled) { sv[pos] = v[u]; si[pos] = base_id + (int)(unsigned)key[u]; }
+    }
   }
   for (int t = keff + tid; t < K; t += BL) { sv[t] = -INFINITY; si[t] = -1; }
+}
+// The entries behind the last scattered one: behind everything.
+__device__ __forceinline__ void lin_pad(unsigned long long* obuf, int filled) {
+  if (threadIdx.x < LIN_PAD) obuf[filled + threadIdx.x] = ~0ull;
 }
 
 // The same for rows of at most 4 NV BL elements, with the row held in registers instead of
@@ -319,14 +351,14 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
 // x in [mn, mx]), and chunks wholly inside the row need no position tests.  Returns 1 when the row is
 // done, 0 when it is unsuitable (no spread, a crowded bin), -1 when it holds a non-finite value (the
 // caller then runs the tolerant form below on the same registers).
-template <int BL, int NV>
+template <int BL, int NV, int BINS>
 __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int off, int m, int K, int base_id, int* hist,
                                                   int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr int CH = 4 * BL;
   const int nch = (m + CH - 1) / CH;                        // chunks that hold any of the row
   auto chunk_full = [&](int i) { return (i > 0 || off == 0) && CH * (i + 1) <= m; };   // the same for all threads
-  for (int b = tid; b < HBINS; b += BL) hist[b] = 0;
+  for (int b = tid; b < BINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
   float mn = INFINITY, mx = -INFINITY;
   bool nan = false;
 #pragma unroll
@@ -357,7 +389,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   const float span = mx - mn;
   if (!(span > 0.f) || !(span < INFINITY)) return 0;
   const int keff = min(K, m - off);
-  const float scale = ((float)HBINS - 0.5f) / span;
+  const float scale = ((float)BINS - 0.5f) / span;
   auto bin_of = [&](float x) { return (int)((mx - x) * scale); };
 #pragma unroll
   for (int i = 0; i < NV; i++) {
@@ -374,7 +406,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   }
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return 0;
+  if (!lin_threshold<BL, BINS>(hist, scratch, keff, tbin, above, c)) return 0;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     if (i >= nch) continue;
@@ -387,6 +419,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
         if (b <= tbin) obuf[atomicAdd(&hist[b], 1)] = sort_key(v[i][j], p + j - off);
       }
   }
+  lin_pad(obuf, above + c);
   __syncthreads();
   lin_rank<BL>(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
   return 1;
@@ -394,11 +427,11 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
 
 // The tolerant form: values that are not finite (-inf marks a column that cannot be selected) are skipped
 // one by one.
-template <int BL, int NV>
+template <int BL, int NV, int BINS>
 __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], int off, int K, int base_id, int* hist,
                                                      int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int b = tid; b < HBINS; b += BL) hist[b] = 0;
+  for (int b = tid; b < BINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
   float mn = INFINITY, mx = -INFINITY;
   int nfin = 0;
 #pragma unroll
@@ -416,8 +449,8 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
   const float span = mx - mn;
   if (!(span > 0.f) || !(span < INFINITY)) return false;
   const int keff = min(K, nfin);
-  const float scale = ((float)HBINS - 0.5f) / span;
-  auto bin_of = [&](float x) { return min(HBINS - 1, (int)((mx - x) * scale)); };
+  const float scale = ((float)BINS - 0.5f) / span;
+  auto bin_of = [&](float x) { return min(BINS - 1, (int)((mx - x) * scale)); };
 #pragma unroll
   for (int i = 0; i < NV; i++)
 #pragma unroll
@@ -425,7 +458,7 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
       if (fabsf(v[i][j]) < INFINITY) atomicAdd(&hist[bin_of(v[i][j])], 1);
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return false;
+  if (!lin_threshold<BL, BINS>(hist, scratch, keff, tbin, above, c)) return false;
 #pragma unroll
   for (int i = 0; i < NV; i++)
 #pragma unroll
@@ -434,21 +467,24 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
         const int b = bin_of(v[i][j]);
         if (b <= tbin) obuf[atomicAdd(&hist[b], 1)] = sort_key(v[i][j], 4 * (tid + BL * i) + j - off);
       }
+  lin_pad(obuf, above + c);
   __syncthreads();
   lin_rank<BL>(obuf, hist, above + c, keff, K, base_id, bin_of, sv, si);
   return true;
 }
 
+// BINS: as many as the registers have elements, up to HBINS: clearing and scanning 4096 of them is most of the work of a short row.
 template <int BL, int NV>
 __device__ __forceinline__ bool linear_select_sort_regs(const float* __restrict__ src, int n, int K, int base_id,
                                                         int* hist, int* scratch, unsigned long long* obuf, float* sv, int* si) {
+  constexpr int BINS = 4 * NV * BL < HBINS ? 4 * NV * BL : HBINS;
   float v[NV][4];
   int off, m;
   load_row_regs<BL, NV>(src, n, v, off, m);
-  const int r = select_regs_finite<BL, NV>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
+  const int r = select_regs_finite<BL, NV, BINS>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
   if (r >= 0) return r == 1;
   __syncthreads();
-  return select_regs_tolerant<BL, NV>(v, off, K, base_id, hist, scratch, obuf, sv, si);
+  return select_regs_tolerant<BL, NV, BINS>(v, off, K, base_id, hist, scratch, obuf, sv, si);
 }
 
 // LEAN 0: unsorted output, the row staged in LDS where it fits.  1, 2, 3: sorted output, rows held in registers.  1: rows of up
@@ -471,7 +507,7 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
   int* scratch = hist + HBINS;                     // SCRATCH<BL>
   float* outv = (float*)(scratch + SCRATCH<BL>);   // Kp2
   int* outi = (int*)(outv + Kp2);                  // Kp2
-  unsigned* keys = (unsigned*)(outi + Kp2 + 2 * LIN_SPARE);   // width (STAGED only); the gap extends the (score, id) buffer
+  unsigned* keys = (unsigned*)(outi + Kp2 + 2 * (LIN_SPARE + LIN_PAD));   // width (STAGED only); the gap extends the (score, id) buffer
   const int tid = threadIdx.x;
   const long row = blockIdx.x;
   const int cb = max(row_begin ? row_begin[row] : 0, 0);
@@ -492,7 +528,8 @@ __global__ __launch_bounds__(BL, LEAN == 1 ? 4 : LEAN == 2 ? 2 : LEAN == 3 ? 4 :
     if (LEAN == 1 && n + 3 <= REG_ROW) {
       bool done;
       unsigned long long* obuf = (unsigned long long*)outv;
-      if (n + 3 <= 8 * BL) done = linear_select_sort_regs<BL, 2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      if (n + 3 <= 4 * BL) done = linear_select_sort_regs<BL, 1>(src, n, K, base_id, hist, scratch, obuf, sv, si);
+      else if (n + 3 <= 8 * BL) done = linear_select_sort_regs<BL, 2>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       else if (n + 3 <= 16 * BL) done = linear_select_sort_regs<BL, 4>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       else done = linear_select_sort_regs<BL, REG_ROW / (4 * BL)>(src, n, K, base_id, hist, scratch, obuf, sv, si);
       if (done) return;
@@ -666,7 +703,7 @@ int dsa_topk_launch(const float* logits, int S, int64_t ld, const int32_t* row_b
   if (S == 0) return DSA_OK;
   int Kp2 = 1;
   while (Kp2 < K) Kp2 <<= 1;
-  const size_t buffers = (size_t)HBINS * 4 + (size_t)Kp2 * 8 + (size_t)LIN_SPARE * 8;
+  const size_t buffers = (size_t)HBINS * 4 + (size_t)Kp2 * 8 + (size_t)(LIN_SPARE + LIN_PAD) * 8;
   const size_t fixed = buffers + SCRATCH<256> * 4, wide = buffers + SCRATCH<1024> * 4;
   const size_t staged = fixed + (size_t)width * 4;
   // Sorted rows that fit a register variant need no staging buffer: rows of up to REG_ROW elements go to the

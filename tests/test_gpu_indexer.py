@@ -208,6 +208,33 @@ def test_topk_on_full_width_rows_at_every_alignment(gpu):
         assert torch.equal(sc.cpu(), torch.gather(x.cpu(), 1, ref))
 
 
+@pytest.mark.parametrize("copies", [1, 80])             # at most 256 rows: 1024 threads a row; more: 256
+@pytest.mark.parametrize("n,K", [(1021, 64), (1022, 1000), (2045, 64), (2046, 2048), (4090, 2048), (8189, 512)])
+def test_topk_segments_of_equal_values(gpu, copies, n, K):
+    """Bins that hold 1 .. 256 elements, and a bin at the K-th place with as many as the buffer has room for and one more: each
+    element's place among its bin's, on both sides of the lengths at which the number of bins changes."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(n + K)
+    rows = []
+    for run in (1, 3, 4, 5, 8, 255, 256, 257, 959, 960, 961):
+        x = torch.rand(n, generator=g)
+        at = torch.randperm(n, generator=g)
+        run = min(run, n - 2)
+        first = min(max(K - run // 2, 0), n - run)                  # the K-th largest value lies in the run, or the run at the end
+        order = torch.argsort(-x, stable=True)
+        x[order[first: first + run]] = x[order[first]].item()
+        x[at[:4]] = x[at[0]].item()
+        rows.append(x)
+    x = torch.stack(rows).repeat(copies, 1)
+    sc, ids = ops.topk(x.to(gpu), K)
+    ref = torch.sort(-x, stable=True, dim=-1).indices[:, :K]
+    kk = min(n, K)
+    assert torch.equal(ids.cpu().long()[:, :kk], ref[:, :kk])
+    assert torch.equal(sc.cpu()[:, :kk], torch.gather(x, 1, ref)[:, :kk])
+    assert (ids.cpu()[:, kk:] == -1).all()
+
+
 def test_fused_rotation_and_quantiser(gpu):
     """rotate_quant_e4m3 against the unfused sequence rotate_activation -> quantiser: the rotated bf16
     values agree to one bf16 step (the fp32 sums are taken in a different order), payload and scale
