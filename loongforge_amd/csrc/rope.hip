@@ -60,11 +60,14 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RopeArgs a) {
 // 4096 tokens x 128 heads 379 / 383 -> 216 / 228 (5.6 TB/s), 700 x 128 63 / 62 -> 30 / 30, 8192 x 32 183 / 177 -> 108 / 109,
 // 60 x 128 33 / 33 -> 4.7 / 5.1.  Tiles of 1, 2, 4 or 8 tokens measured within 2 %, of 32 tokens 5 % slower.
 constexpr int MLA_MAIN = 512, MLA_EMB = 64, TILE_ROWS = 32, TOK_LOG2 = 1;
-// Non-temporal loads where the rows exceed the memory-side cache (4096 x 128: 216 against 227 us); below it the data may
-// still be there from the kernel that wrote it (700 x 128: 34 against 30 us).
+// Where the rows read and written exceed the memory-side cache, loads and stores of the main parts are non-temporal (STREAMED): both parts
+// are whole lines, used once.  us, forward and backward of query and key: 4096 tokens x 128 heads 469 with plain ones, 462 with such loads,
+// 446 with such stores, 420 with both (5.8 TB/s); 8192 x 64 466 -> 431, 1500 x 128 190 -> 167, 2600 x 64 167 -> 140 - 156.  Below that size
+// the data may still be there from the kernel that wrote it, or for the one that reads it (700 x 128, forward: 34 against 30 us with such
+// loads).  It is a template's argument because of a choice at run time the compiler makes one plain load or store.
 constexpr long CACHE_BYTES = 256l << 20;
-template <int IN, int OUT, bool INVERSE>
-__global__ __launch_bounds__(256) void rope_mla_rows_kernel(RopeArgs a, int tok_log2, int head_tiles, bool streamed) {
+template <int IN, int OUT, bool INVERSE, bool STREAMED>
+__global__ __launch_bounds__(256) void rope_mla_rows_kernel(RopeArgs a, int tok_log2, int head_tiles) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tok0 = ((int)blockIdx.x / head_tiles) << tok_log2;
   const int head0 = ((int)blockIdx.x % head_tiles) * (TILE_ROWS >> tok_log2);
@@ -82,7 +85,7 @@ __global__ __launch_bounds__(256) void rope_mla_rows_kernel(RopeArgs a, int tok_
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const i32x4* src = (const i32x4*)at(a.main_src, a.ms_tok, a.ms_head, wave * 8 + i) + lane;
-    if (streamed) v[i] = __builtin_nontemporal_load(src);
+    if constexpr (STREAMED) v[i] = __builtin_nontemporal_load(src);
     else v[i] = *src;
   }
   const Quad x = load_quad<IN>(at(a.pe_src, a.ps_tok, a.ps_head, pe_row), q, MLA_EMB);
@@ -90,8 +93,11 @@ __global__ __launch_bounds__(256) void rope_mla_rows_kernel(RopeArgs a, int tok_
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < 8; i++)
-    if (there(wave * 8 + i))
-      *((i32x4*)(a.main_dst + (long)token(wave * 8 + i) * a.md_tok + (long)head(wave * 8 + i) * a.md_head) + lane) = v[i];
+    if (there(wave * 8 + i)) {
+      i32x4* dst = (i32x4*)(a.main_dst + (long)token(wave * 8 + i) * a.md_tok + (long)head(wave * 8 + i) * a.md_head) + lane;
+      if constexpr (STREAMED) __builtin_nontemporal_store(v[i], dst);
+      else *dst = v[i];
+    }
   if (there(pe_row))
     store_quad<OUT>(rotate<INVERSE>(x, tables), a.pe_dst + (long)token(pe_row) * a.pd_tok + (long)head(pe_row) * a.pd_head, q, MLA_EMB);
 }
@@ -188,7 +194,8 @@ extern "C" int dsa_rope_rows(const void* main_src, int64_t ms_tok, int64_t ms_he
   const bool streamed = (long)tokens * heads * (MLA_MAIN + MLA_EMB) * 4 > CACHE_BYTES;
   const dim3 grid(mla ? (unsigned)tiles : tokens < (1 << 20) ? tokens : (1 << 20));
 #define DSA_ROPE(IN, OUT, INV) do { \
-    if (mla) rope_mla_rows_kernel<IN, OUT, INV><<<grid, block, 0, st>>>(a, tok_log2, head_tiles, streamed); \
+    if (mla && streamed) rope_mla_rows_kernel<IN, OUT, INV, true><<<grid, block, 0, st>>>(a, tok_log2, head_tiles); \
+    else if (mla) rope_mla_rows_kernel<IN, OUT, INV, false><<<grid, block, 0, st>>>(a, tok_log2, head_tiles); \
     else rope_rows_kernel<IN, OUT, INV><<<grid, block, 0, st>>>(a); \
   } while (0)
   switch (sel) {

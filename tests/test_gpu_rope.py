@@ -169,3 +169,25 @@ def test_tables_shorter_than_the_sequence_are_refused(gpu):
                     call()
     with pytest.raises(ValueError):
         ops.rope_headsum_inverse(x, cos, sin, 0, torch.zeros(T - 1, device=gpu, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("inter", [False, True])
+@pytest.mark.parametrize("tokens", [910, 911])          # x 128 heads: read and written 256 MiB less 64 KB, and 224 KB more
+def test_rows_beyond_the_caches_are_those_of_their_parts(gpu, tokens, inter):
+    """The rows that pass by the caches have the bits of parts of them that do not (which the tests above compare with the oracle)."""
+    from loongforge_amd.dsa_fused_kernels import fused_rope_permute_cat
+
+    g = torch.Generator(device=gpu).manual_seed(tokens)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=BF)      # noqa: E731
+    cos, sin = (t.to(gpu) for t in _tables(tokens, 64, inter, torch.float32, True))
+    qc, pe, grad = rnd(128, tokens, 512), rnd(tokens, 1, 128, 64), rnd(tokens, 1, 128, 576)
+
+    def both(rows):
+        a, b = qc[:, rows].contiguous().requires_grad_(True), pe[rows].clone().requires_grad_(True)
+        out = fused_rope_permute_cat(a, b, cos[rows].contiguous(), sin[rows].contiguous(), rotary_interleaved=inter)
+        return (out.detach(), *torch.autograd.grad(out, (a, b), grad[rows].contiguous()))
+
+    out, d_qc, d_pe = both(slice(None))
+    for rows in (slice(0, 301), slice(301, tokens)):
+        part = both(rows)
+        assert torch.equal(out[rows], part[0]) and torch.equal(d_qc[:, rows], part[1]) and torch.equal(d_pe[rows], part[2])
