@@ -276,3 +276,22 @@ def test_chunkpipe_through_the_mla_module_matches_the_whole_sequence(gpu, fusion
     assert not chunked.micro_batch_to_cache_chunk_map
     with pytest.raises(RuntimeError):
         whole.concat_cached_chunk_key_value_dsa(x)
+
+
+@pytest.mark.parametrize("heads,rows", [(128, 2730), (128, 2731), (64, 6557)])      # 512 MiB read and written: from 2731 x 128 (query), 6554 x 64 (output)
+def test_absorption_beyond_the_caches_is_that_of_its_parts(gpu, heads, rows):
+    """The rows that pass by the caches have the bits of parts of them that do not."""
+    from loongforge_amd.dsa_fused_kernels import absorb_attention_output, fused_absorb_rope_query
+
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=torch.bfloat16)      # noqa: E731
+    q_up, w_uk_t, w_uv = rnd(rows, heads, 192), rnd(heads, 512, 128), rnd(heads, 128, 512)
+    cos, sin = (f(torch.rand(rows, 64, generator=g, device=gpu) * 6.28).to(torch.bfloat16).view(rows, 1, 1, 64) for f in (torch.cos, torch.sin))
+    with torch.no_grad():
+        for inter in (False, True):
+            whole = fused_absorb_rope_query(q_up, w_uk_t, cos, sin, rotary_interleaved=inter)
+            out = absorb_attention_output(whole[..., :512].contiguous(), w_uv)
+            for part in (slice(0, 1001), slice(1001, rows)):
+                query = fused_absorb_rope_query(q_up[part], w_uk_t, cos[part].contiguous(), sin[part].contiguous(), rotary_interleaved=inter)
+                assert torch.equal(query, whole[part])
+                assert torch.equal(absorb_attention_output(query[..., :512].contiguous(), w_uv), out[part])
