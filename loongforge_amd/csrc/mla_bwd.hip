@@ -93,10 +93,11 @@ __device__ __forceinline__ void stage_unit(const int* __restrict__ list, int n, 
 constexpr int DQ_THREADS = 768;
 // ids, pds, dq: the query's (UNIT: the joint unit's) slots, dS tiles and rows of dQ; qpos: its position; of every `per` heads the first
 // `real` have a row in dq
+// once: dS is read with the non-temporal hint
 template <int STAGES, int HG, bool UNIT>
 __device__ __forceinline__ void dq_body(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, int H, int per, int real, int Skv, int K, int qpos, const int* __restrict__ dup_flag,
+    __bf16* __restrict__ dq, int H, int per, int real, int Skv, int K, int qpos, const int* __restrict__ dup_flag, bool once,
     unsigned char* smem) {
   constexpr int STAGE_BYTES = TILE_BYTES + pds_kind_bytes(HG);
   constexpr int NJ = HG == 4 ? 2 : 1;          // head groups of a wave
@@ -163,7 +164,10 @@ __device__ __forceinline__ void dq_body(
   // step 0 .. 2: the wave's three groups of the key rows; step 3: its part of the dS block (waves 0 .. DS_WAVES - 1)
   auto issue_step = [&](int j) {
     if (j < 3) dma16(t_lb + 3 * j * GRP_BYTES, t_goff + 3 * j * 128, kv);
-    else if (wave < DS_WAVES) dma16(t_lbd, ds_src, t_src);
+    else if (wave < DS_WAVES) {
+      if (once) dma16_once(t_lbd, ds_src, t_src);
+      else dma16(t_lbd, ds_src, t_src);
+    }
   };
 
   const int hg0 = HG == 4 ? 2 * hp : HG == 2 ? hp : 0;
@@ -327,9 +331,9 @@ __device__ __forceinline__ void pds_rows_body(
     const unsigned lb = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * 1024u);
     const unsigned row = (unsigned)(8 * wave + (lane >> 3)), col = (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
 #pragma unroll
-    for (int k = 0; k < 9; k++) dma16(lb + k * 8192, row * (DQK * 2) + col + k * 128, q_rows);
+    for (int k = 0; k < 9; k++) dma16_once(lb + k * 8192, row * (DQK * 2) + col + k * 128, q_rows);
 #pragma unroll
-    for (int k = 0; k < 8; k++) dma16(lb + (9 + k) * 8192, row * (DV * 2) + col + k * 128, do_rows);
+    for (int k = 0; k < 8; k++) dma16_once(lb + (9 + k) * 8192, row * (DV * 2) + col + k * 128, do_rows);
   }
   const int h = hw * 16 + m;
   const size_t hrow = (size_t)qi * H + h;
@@ -669,7 +673,7 @@ __device__ __forceinline__ void pds_rows_wide_body(
     for (int rb = 0; rb < 2; rb++) {
       const unsigned src = (unsigned)min(64 * rb + 8 * wave + (l >> 3), H - 1) * (DQK * 2) + ((l & 7) ^ (l >> 3)) * 16;
 #pragma unroll
-      for (int p = 0; p < 9; p++) dma16(lb + rb * 8192 + group_base(p), src + p * 128, q_rows);
+      for (int p = 0; p < 9; p++) dma16_once(lb + rb * 8192 + group_base(p), src + p * 128, q_rows);
     }
   }
   const int m = lane & 15, kg = lane >> 4;
@@ -900,7 +904,9 @@ __device__ __forceinline__ void pds_rows_wide_body(
     const uint4 d16 = make_uint4(dw[0][0], dw[0][1], dw[1][0], dw[1][1]);
     *(uint4*)(xch + chunk) = d16;
     *(uint4*)(xch + pds_kind_bytes(4) + chunk) = make_uint4(pw[0][0], pw[0][1], pw[1][0], pw[1][1]);
-    *(uint4*)(pds + (size_t)tile * pds_kind_bytes(4) + chunk) = d16;
+    i32x4* const d_out = (i32x4*)(pds + (size_t)tile * pds_kind_bytes(4) + chunk);
+    if constexpr (G == 1) __builtin_nontemporal_store(__builtin_bit_cast(i32x4, d16), d_out);
+    else *d_out = __builtin_bit_cast(i32x4, d16);
     __builtin_amdgcn_sched_barrier(0);
   };
   // the rows of tile n
@@ -1233,7 +1239,7 @@ __global__ __launch_bounds__(PDS_THREADS, 1) void bwd_pds_rows_kernel(
 template <int HG, int G>
 __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const __bf16* __restrict__ kv, const int* __restrict__ ids, const unsigned char* __restrict__ pds,
-    __bf16* __restrict__ dq, const int* __restrict__ work, size_t group_pds, int q0, int cnt, int H, int real, int Skv, int K, int q_start,
+    __bf16* __restrict__ dq, const int* __restrict__ work, size_t group_pds, int ds_once, int q0, int cnt, int H, int real, int Skv, int K, int q_start,
     const int* __restrict__ dup_flag, const unsigned char* __restrict__ rows, const unsigned char* __restrict__ exps, const int* __restrict__ start,
     float* __restrict__ dkv_acc, unsigned short* __restrict__ dkv, int n_keys, int accumulate) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -1247,12 +1253,12 @@ __global__ __launch_bounds__(DQ_THREADS, 1) void bwd_dq_reduce_kernel(
     const unsigned char* own = pds + (size_t)(ql / G) * group_pds;
     if constexpr (G > 1) {
       if (w.tiles > 0) {
-        dq_body<3, 4, true>(kv, list, own, dq_rows, 128, 128 / G, real, Skv, 32 * w.tiles, 0, dup_flag, smem);
+        dq_body<3, 4, true>(kv, list, own, dq_rows, 128, 128 / G, real, Skv, 32 * w.tiles, 0, dup_flag, ds_once, smem);
         return;
       }
       own += (size_t)(ql % G) * (K / BI) * pds_kind_bytes(HG);
     }
-    dq_body<3, HG, false>(kv, list, own, dq_rows, H, H, real, Skv, K, q_start + q0 + ql, dup_flag, smem);
+    dq_body<3, HG, false>(kv, list, own, dq_rows, H, H, real, Skv, K, q_start + q0 + ql, dup_flag, HG == 4 || ds_once, smem);
   } else {
     // longest work first: from the first key on where the first half of the keys has most of the rows (causal windows), else
     // from the last key (compressed keys behind a sliding window)
@@ -1368,6 +1374,14 @@ order::UnitCost unit_cost(int HG, int S) {       // (HG 1 or 2)
 }
 
 constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;
+// What is read or written once passes by the L2, whose key rows the workgroups of an XCD share: Q (with up to 64 heads dO too: the other
+// loads of the set-up take lines by parts) and, with 128 heads, dS both ways.  Up to 64 heads dS is read so up to this size (of queries by
+// themselves); beyond, where it no longer lies in the memory-side cache, that is the slower way.  Whole backward, us, plain / Q (and dO) / dS read
+// so besides: 64 heads 10000 x 512 slots 4021 / 3864 / 3842 (655 MB), 1000 x 2048 1479 / 1473 / 1388 (262 MB), 6000 x 1024 3929 / 3900 / 3913 (786 MB),
+// 3000 x 2048 4227 / 4216 / 4267 beside plain Q (786 MB), 2077 x 512 741 / 726 / 707; 32 heads 3000 x 2048 3912 / 3895 / 3833 (393 MB), 6000 x 1024
+// 2902 / 2863 / 2894 (393 MB).  128 heads, plain / Q / dS written so / read so: 8192 x 2048 12 968 / 12 883 / 12 835 / 13 002 against 13 028, 400 x
+// 2048 833 / 828 / 822 / 809, 1500 x 1024 1501 / 1490 / 1491 / 1465; units write dS as before (1024 x 256 x 32 heads 175 and 180).
+constexpr size_t DS_ONCE_BYTES = (size_t)384 << 20;
 
 }  // namespace
 
@@ -1477,7 +1491,8 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(P, dS, dKV rows)");
     DSA_MARK(2);
     // dQ of every query beside the sums of every key.
-    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, work, group_pds, q0, cnt, H, dq_heads, Skv,
+    const int ds_once = (size_t)cnt * (K / BI) * pds_kind_bytes(HG) <= DS_ONCE_BYTES;
+    dq_reduce_kernel<<<dim3(cnt + (Skv + RED_KEYS - 1) / RED_KEYS), dim3(DQ_THREADS), smem_dq, st>>>((const __bf16*)kv, sids, pds, (__bf16*)dq, work, group_pds, ds_once, q0, cnt, H, dq_heads, Skv,
                                                                    K, q_start, dup_flag, rows, exps, start, acc,
                                                                    S <= p.chunk ? (unsigned short*)dkv : nullptr, Skv, first ? 0 : 1);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(dQ | dKV reduce)");

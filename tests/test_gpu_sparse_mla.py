@@ -802,6 +802,25 @@ def test_sink_survives_the_exact_pass(gpu):
     assert ((lse.cpu() - rl).abs() / rl.abs().clamp_min(1)).max().item() < 1e-3
 
 
+@pytest.mark.parametrize("S,H,K", [(3073, 32, 2048), (1537, 64, 2048)])          # dS of the sweep 384 MiB and 128 or 256 KiB more
+def test_backward_on_both_sides_of_the_way_that_ds_is_read(gpu, monkeypatch, S, H, K):
+    """One sweep whose dS is just above the size from which it is read through the caches, against sweeps of less: the same dQ."""
+    from loongforge_amd import _lib, ops
+
+    g = torch.Generator(device=gpu).manual_seed(S)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=torch.bfloat16)      # noqa: E731
+    q, kv, do = rnd(S, H, 576), rnd(S + 500, 576), rnd(S, H, 512)
+    ids = ops.topk(torch.randn(S, S + 500, generator=g, device=gpu), K)[1]
+    out, lse, _ = ops.sparse_mla_fwd(q, kv, ids, S + 500)
+    dq, dkv = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, S + 500)
+    half = _lib.load().dsa_sparse_mla_bwd_workspace_bytes((S + 1) // 2 + 4, H, S + 500, K)
+    monkeypatch.setenv("DSA_BWD_WORKSPACE_GIB", repr(half / 2 ** 30))
+    dq2, dkv2 = ops.sparse_mla_bwd(q, kv, out, do, ids, lse, S + 500)
+    ops.release_bwd_workspace()
+    assert torch.equal(dq, dq2) and torch.isfinite(dq.float()).all()
+    assert (dkv.float() - dkv2.float()).abs().max().item() <= 2 * 2.0 ** -8 * dkv.float().abs().max().item()
+
+
 def test_backward_chunked_workspace_through_the_c_abi(gpu):
     """A workspace too small for all queries at once makes the library walk the queries in chunks;
     the result must not change."""
