@@ -375,6 +375,9 @@ int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t workspace_byt
  */
 int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S,
                         int K, float eps, float* row_loss, float* grad, void* stream);
+/* The same with every gradient times factor, rounded once more: what dsa_indexer_kl_scale makes of it with *g = 1. */
+int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S,
+                               int K, float eps, float factor, float* row_loss, float* grad, void* stream);
 /* *out = factor * the sum of row_loss [S]; and out = grad * (*g * factor), n elements: the two ways through the scaled sum of the rows. */
 int dsa_indexer_kl_total(const float* row_loss, int S, float factor, float* out, void* stream);
 int dsa_indexer_kl_scale(const float* grad, const float* g, float factor, float* out, int64_t n, void* stream);

@@ -91,7 +91,7 @@ def _compile_host(force):
 def _link_host(obj):
     from torch.utils.cpp_extension import library_paths
 
-    libs = ["-l" + n for n in ("dsa_hip", "c10", "c10_hip", "torch", "torch_cpu", "torch_python", "amdhip64")]
+    libs = ["-l" + n for n in ("dsa_hip", "c10", "c10_hip", "torch", "torch_cpu", "torch_hip", "torch_python", "amdhip64")]
     res = subprocess.run([os.environ.get("CXX", "g++"), "-shared", "-o", HOST_LIB, obj, "-L" + PKG]
                          + ["-L" + p for p in library_paths()] + ["-L/opt/rocm/lib"] + libs + ["-Wl,-rpath,$ORIGIN"],
                          capture_output=True, text=True)

@@ -7,6 +7,7 @@
 // functional tensor, a traced or transformed call, or one whose gradient is being recorded): the caller then goes
 // through the registered custom op, whose implementation calls back here with force = true.
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -98,7 +99,11 @@ struct Call {
 
 Tensor f32(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
 Tensor i32(const Tensor& t) { return t.to(at::kInt).contiguous(); }
-Tensor make(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) { return at::empty(shape, like.options().dtype(type)); }
+// (past the dispatcher: 0.5 us and not 0.8 a tensor, of which a training pass of a layer makes fifty)
+Tensor make(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) {
+  if (!like.is_cuda()) return at::empty(shape, like.options().dtype(type));
+  return at::detail::empty_cuda(shape, type, like.device(), std::nullopt);
+}
 at::ScalarType payload_type(bool raw) { return raw ? at::kByte : at::kFloat8_e4m3fn; }
 const void* ptr(const OptTensor& t) { return t && t->numel() ? t->const_data_ptr() : nullptr; }
 template <class P> P* out_ptr(const Tensor& t) { return t.numel() ? (P*)t.data_ptr() : nullptr; }
@@ -653,8 +658,10 @@ py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, cons
           "sparse_mla_bwd: out/dout must be [S,H,d_v] and lse [S,H]");
   Tensor dq = some ? make({S, heads, 576}, at::kBFloat16, q) : at::empty_like(q), dkv = at::empty_like(kv);
   const size_t full = dsa_sparse_mla_bwd_workspace_bytes((int)S, (int)H, (int)Skv, (int)K);
-  const auto [ws, nbytes] = py::cast<std::pair<Tensor, size_t>>(workspace(full, q.device()));
   Call call(q);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)call.stream, &status) != hipSuccess) status = hipStreamCaptureStatusActive;
+  const auto [ws, nbytes] = py::cast<std::pair<Tensor, size_t>>(workspace(full, q.device(), (size_t)call.stream, status != hipStreamCaptureStatusNone));
   run("dsa_sparse_mla_bwd", dsa_sparse_mla_bwd_heads, q.const_data_ptr(), kv.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
       (const int32_t*)ids.const_data_ptr(), (const float*)lse.const_data_ptr(), (int)S, (int)H, (int)(some ? heads : H), (int)Skv, (int)K, (int)q_start, (float)sm_scale,
       (int)d_v, dq.data_ptr(), dkv.data_ptr(), ws.data_ptr(), nbytes, call.stream);
@@ -673,8 +680,7 @@ py::object attn_dist(const Tensor& p_, double sm_scale, bool force) {
   return py::cast(target);
 }
 
-py::object kl_loss(const Tensor& scores_, const Tensor& target_, double eps, bool force) {
-  PLAIN_OR_NONE(scores_, target_);
+std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, double eps, double factor) {
   need_gpus(scores_, target_);
   REQUIRE(scores_.dim() == 2 && target_.sizes() == scores_.sizes(), "indexer_kl_loss expects scores and target of one shape [S, K]");
   const int64_t S = scores_.size(0), K = scores_.size(1);
@@ -683,17 +689,31 @@ py::object kl_loss(const Tensor& scores_, const Tensor& target_, double eps, boo
   if (target.stride(1) != 1) target = target.contiguous();
   Call call(scores);
   Tensor row_loss = make({S}, at::kFloat, scores), grad = make({S, K}, at::kFloat, scores);
-  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, (const float*)target.const_data_ptr(), S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
+  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss_scaled, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, (const float*)target.const_data_ptr(), S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float)factor, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
+  return {row_loss, grad};
+}
+
+py::object kl_loss(const Tensor& scores, const Tensor& target, double eps, bool force) {
+  PLAIN_OR_NONE(scores, target);
+  const auto [row_loss, grad] = kl_rows(scores, target, eps, 1.0);
   return py::make_tuple(row_loss, grad);
 }
 
 // The loss of all rows times factor, and its gradient behind kl_loss: grad * g * factor.  None for what the kernels do not take.
-py::object kl_total(const Tensor& row_loss, double factor) {
-  if (!plain(row_loss) || !row_loss.is_cuda() || row_loss.scalar_type() != at::kFloat || row_loss.dim() != 1 || !row_loss.is_contiguous()) return py::none();
+Tensor rows_total(const Tensor& row_loss, double factor) {
   Call call(row_loss);
   Tensor total = make({}, at::kFloat, row_loss);
   run("dsa_indexer_kl_total", dsa_indexer_kl_total, (const float*)ptr(row_loss), (int)row_loss.numel(), (float)factor, (float*)total.data_ptr(), call.stream);
-  return py::cast(total);
+  return total;
+}
+py::object kl_total(const Tensor& row_loss, double factor) {
+  if (!plain(row_loss) || !row_loss.is_cuda() || row_loss.scalar_type() != at::kFloat || row_loss.dim() != 1 || !row_loss.is_contiguous()) return py::none();
+  return py::cast(rows_total(row_loss, factor));
+}
+// Both, the gradient times factor: (loss of all rows times factor, its gradient).
+py::object kl_loss_total(const Tensor& scores, const Tensor& target, double eps, double factor) {
+  const auto [row_loss, grad] = kl_rows(scores, target, eps, factor);
+  return py::make_tuple(rows_total(row_loss, factor), grad);
 }
 
 py::object kl_scale(const Tensor& grad, const Tensor& g, double factor) {
@@ -863,6 +883,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(attn_dist);
   DEF(kl_loss);
   DEF(kl_total);
+  DEF(kl_loss_total);
   DEF(kl_scale);
   DEF(indexer_window);
   DEF(indexer_forward);

@@ -63,7 +63,7 @@ __device__ __forceinline__ float pairs_sum(const float (&v)[N]) {
 // thread tid of the NT that share a row has its slots tid, tid + NT, ..: K <= NE * NT
 template <int NE, int NT, class Row>
 __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, const float* __restrict__ scores, int64_t ld_s,
-                                       const float* __restrict__ target, int64_t ld_t, int K, float eps, float* __restrict__ row_loss,
+                                       const float* __restrict__ target, int64_t ld_t, int K, float eps, float factor, float* __restrict__ row_loss,
                                        float* __restrict__ grad) {
   const float* sp = scores + row * ld_s;
   const float* tp = target + row * ld_t;
@@ -111,17 +111,17 @@ __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, co
 #pragma unroll
   for (int i = 0; i < NE; i++) {
     const int t = tid + NT * i;
-    if (t < K) grad[row * K + t] = s[i] * (inner - u[i]);
+    if (t < K) grad[row * K + t] = (s[i] * (inner - u[i])) * factor;
   }
   if (tid == 0) row_loss[row] = loss;
 }
 
 template <int NE>
 __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict__ scores, int64_t ld_s,
-                                                        const float* __restrict__ target, int64_t ld_t, int K, float eps,
+                                                        const float* __restrict__ target, int64_t ld_t, int K, float eps, float factor,
                                                         float* __restrict__ row_loss, float* __restrict__ grad) {
   __shared__ float scratch[8];
-  kl_row<NE, BLOCK>(BlockRow{scratch}, threadIdx.x, blockIdx.x, scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+  kl_row<NE, BLOCK>(BlockRow{scratch}, threadIdx.x, blockIdx.x, scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
 }
 
 // Up to 512 slots: a row to a wave.  A workgroup to a row spent its time in three reductions with barriers and on eight slots a thread of
@@ -129,11 +129,11 @@ __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict_
 // slots a thread where that is enough: 4000 x 1024 18.8 and 13.8).
 template <int NE>
 __global__ __launch_bounds__(BLOCK) void kl_loss_wave_kernel(const float* __restrict__ scores, int64_t ld_s, const float* __restrict__ target,
-                                                             int64_t ld_t, int S, int K, float eps, float* __restrict__ row_loss,
+                                                             int64_t ld_t, int S, int K, float eps, float factor, float* __restrict__ row_loss,
                                                              float* __restrict__ grad) {
   const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6));
   if (row >= S) return;
-  kl_row<NE, 64>(WaveRow{}, threadIdx.x & 63, row, scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+  kl_row<NE, 64>(WaveRow{}, threadIdx.x & 63, row, scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
 }
 
 // *out = factor * sum of the rows' losses, in a fixed order and 64 bits, so that the result is rounded and not the sums on the way.  One
@@ -196,17 +196,22 @@ extern "C" int dsa_indexer_kl_scale(const float* grad, const float* g, float fac
 
 extern "C" int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S, int K,
                                    float eps, float* row_loss, float* grad, void* stream) {
+  return dsa_indexer_kl_loss_scaled(scores, ld_s, target, ld_t, S, K, eps, 1.0f, row_loss, grad, stream);
+}
+
+extern "C" int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S, int K,
+                                          float eps, float factor, float* row_loss, float* grad, void* stream) {
   DSA_REQUIRE(S >= 0 && K > 0 && K <= 32 * BLOCK, "dsa_indexer_kl_loss: K must lie in [1, %d], got %d", 32 * BLOCK, K);
   DSA_REQUIRE(ld_s >= K && ld_t >= K, "dsa_indexer_kl_loss: row strides %lld / %lld below K = %d", (long long)ld_s,
               (long long)ld_t, K);
   if (S == 0) return DSA_OK;
   hipStream_t st = (hipStream_t)stream;
   const dim3 waves(dsa_cdiv(S, BLOCK / 64));
-  if (K <= 256) kl_loss_wave_kernel<4><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, row_loss, grad);
-  else if (K <= 512) kl_loss_wave_kernel<8><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, row_loss, grad);
-  else if (K <= 4 * BLOCK) kl_loss_kernel<4><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
-  else if (K <= 8 * BLOCK) kl_loss_kernel<8><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
-  else kl_loss_kernel<32><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, row_loss, grad);
+  if (K <= 256) kl_loss_wave_kernel<4><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
+  else if (K <= 512) kl_loss_wave_kernel<8><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
+  else if (K <= 4 * BLOCK) kl_loss_kernel<4><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+  else if (K <= 8 * BLOCK) kl_loss_kernel<8><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+  else kl_loss_kernel<32><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
   DSA_CHECK_LAUNCH("dsa_indexer_kl_loss");
   return DSA_OK;
 }

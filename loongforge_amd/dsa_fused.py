@@ -497,7 +497,12 @@ class DSAIndexerFused(MegatronModule):
         )
 
 
+def _scaler_steps(scaler):
+    return [scaler] + [getattr(scaler, name, None) for name in ("forward", "backward", "apply")]
+
+
 _INDEXER_FORWARD = DSAIndexerFused.forward
+_OWN_SCALER = _scaler_steps(DSAIndexerLossAutoScaler)
 _OWN_STEPS = [RotaryEmbedding, apply_rotary_pos_emb, rotate_activation, RotaryEmbedding.forward, DSAIndexerFused._apply_rope,
               DSAIndexerFused.get_query_key_weight_tensors]
 
@@ -631,7 +636,12 @@ class DSAttentionFused(MegatronModule):
             # softmax, F.kl_div(log(pred + 1e-10), target + 1e-10, "sum") and their backward in one kernel
             from . import ops
             scaled = bool(sq) and isinstance(indexer_loss_coeff, (int, float))       # (one launch each way with the loss itself)
-            indexer_loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10, indexer_loss_coeff / sq if scaled else 1.0)
+            attached = scaled and _scaler_steps(DSAIndexerLossAutoScaler) == _OWN_SCALER and ops.ordinary(output, index_scores, main_attn_probs)
+            if attached:
+                output, indexer_loss = ops.attached_indexer_kl_loss(output, index_scores, main_attn_probs, 1e-10, indexer_loss_coeff / sq,
+                                                                    DSAIndexerLossAutoScaler)
+            else:
+                indexer_loss = ops.indexer_kl_loss(index_scores, main_attn_probs, 1e-10, indexer_loss_coeff / sq if scaled else 1.0)
         for check in checks:
             check.wait()
         if topk_holder is not None and not self.skip_topk:
@@ -645,5 +655,6 @@ class DSAttentionFused(MegatronModule):
                     layer_number=self.layer_number,
                     num_layers=self.config.num_layers + getattr(self.config, "mtp_num_layers", 0),
                 )
-            output = DSAIndexerLossAutoScaler.apply(output, indexer_loss)
+            if not attached:
+                output = DSAIndexerLossAutoScaler.apply(output, indexer_loss)
         return output

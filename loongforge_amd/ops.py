@@ -507,7 +507,7 @@ BWD_MAX_SLOTS = 2048      # slots per query the backward kernels take in one cal
 ATTN_DIST_QK_MAX_SLOTS = 4096
 
 
-def _bwd_workspace(full_bytes: int, device):
+def _bwd_workspace(full_bytes: int, device, stream: Optional[int] = None, capturing: bool = False):
     """Workspace of the sparse-MLA backward: ``full_bytes`` lets it take all queries in one sweep (22 GiB at 8k
     tokens, top-k 2048; 89 GiB at 32k); given less, the library walks the queries in chunks.  The size handed to
     the library - and with it the chunking, on which the last bits of dKV depend (those of dQ do not) - follows from the shapes and
@@ -515,12 +515,13 @@ def _bwd_workspace(full_bytes: int, device):
     The buffer is kept per device and reused by later calls on the same stream (held until :func:`release_bwd_workspace`;
     ``DSA_BWD_WORKSPACE_CACHE=0`` keeps none).  A call on another stream, which may overlap, lets go of it - the allocator
     hands it out again behind the work of its own stream only - and allocates one there.  A graph that is being captured gets
-    one of its own, which lives as long as the graph."""
+    one of its own, which lives as long as the graph.  ``stream`` (and whether it is ``capturing``): from a caller that knows it."""
     want = max(int(full_bytes), 256)
     cap = os.environ.get("DSA_BWD_WORKSPACE_GIB", "48")
     want = min(want, max(int(float(cap) * 2 ** 30), 256))
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    capturing, stream = torch.cuda.is_current_stream_capturing(), torch.cuda.current_stream(device).cuda_stream
+    if stream is None:
+        capturing, stream = torch.cuda.is_current_stream_capturing(), torch.cuda.current_stream(device).cuda_stream
     if not capturing:
         kept = _BWD_WS.get(idx)
         if kept is not None and kept.numel() >= want and kept.stream == stream:
@@ -704,6 +705,40 @@ def indexer_kl_loss(scores: torch.Tensor, target: torch.Tensor, eps: float = 1e-
     """``F.kl_div((softmax(scores, -1) + eps).log(), target + eps, reduction="sum")`` as one kernel
     (dsa_fused.py:931-937 of the reference), times ``factor``; differentiable in ``scores``, the target is a constant."""
     return _IndexerKLLoss.apply(scores, target, float(eps), float(factor))
+
+
+class _AttachedKLLoss(torch.autograd.Function):
+    """:class:`_IndexerKLLoss` and the auto-scaler that feeds its backward, in one node: the gradient of the scores is made, times
+    ``factor``, with the loss, and goes out as it is while no loss scale is set (two nodes, a fill and a pass over the scores' gradient
+    less)."""
+
+    @staticmethod
+    def forward(ctx, output, scores, target, eps, factor, scaler):
+        loss, grad = _native().kl_loss_total(scores.detach(), target.detach(), eps, factor)
+        ctx.save_for_backward(grad)
+        ctx.in_dtype, ctx.scaler = scores.dtype, scaler
+        ctx.mark_non_differentiable(loss)
+        ctx.set_materialize_grads(False)
+        return output, loss
+
+    @staticmethod
+    def backward(ctx, grad_output, _):
+        d_scores, scale = None, ctx.scaler.main_loss_backward_scale
+        if ctx.needs_input_grad[1]:
+            (d_scores,) = ctx.saved_tensors
+            if scale is not None:
+                g, scaled = scale.to(d_scores.device).to(torch.float32), None
+                if not torch.is_grad_enabled() and not torch.compiler.is_compiling() and ordinary(d_scores, g):
+                    scaled = _native().kl_scale(d_scores, g, 1.0)
+                d_scores = d_scores * g.reshape(()) if scaled is None else scaled
+            d_scores = d_scores.to(ctx.in_dtype)
+        return grad_output, d_scores, None, None, None, None
+
+
+def attached_indexer_kl_loss(output, scores: torch.Tensor, target: torch.Tensor, eps: float, factor: float, scaler):
+    """``(output, loss)``: the loss of :func:`indexer_kl_loss`, detached, and ``output`` with it attached as ``scaler`` (the class
+    with the loss's ``main_loss_backward_scale``) attaches an auxiliary loss; for :func:`ordinary` tensors."""
+    return _AttachedKLLoss.apply(output, scores, target, float(eps), float(factor), scaler)
 
 
 def _rows_view(t: torch.Tensor, what: str):

@@ -483,6 +483,66 @@ def test_heads_are_padded_inside_the_attention(gpu, heads, S, packed):
         assert torch.equal(ops.pad_heads(x, total), torch.nn.functional.pad(x, (0, 0, 0, total - heads)))
 
 
+@pytest.mark.parametrize("scale", [None, 4.0, "one element"])
+def test_loss_attached_in_one_node_is_that_of_the_two(gpu, scale, monkeypatch):
+    """The indexer's loss with its attachment in one node: the bits of the loss function and the auto-scaler by themselves, for no loss scale
+    and for one (a power of two: it is applied behind the loss's factor there and before it here), in a second backward pass, with
+    saved tensors on their way through a hook and where the indexer needs no gradient."""
+    from loongforge_amd import dsa_fused, megatron_compat, ops
+    from loongforge_amd.megatron_compat import AttnMaskType, ModuleSpec
+
+    S, H, hid, qlr = 300, 32, 96, 48
+    cfg = _cfg(num_attention_heads=H, hidden_size=hid, q_lora_rank=qlr, dsa_indexer_n_heads=32, dsa_indexer_head_dim=128, dsa_indexer_topk=128,
+               dsa_indexer_loss_coeff=1.5, rope_type="rope", rotary_percent=1.0, rotary_base=10000, init_method=None, layernorm_epsilon=1e-5,
+               dsa_indexer_rotate_activation=True, enable_chunkpipe=False, apply_rope_fusion=True)
+    sub = dsa_fused.DSAttentionFusedSubmodules(indexer=ModuleSpec(
+        module=dsa_fused.DSAIndexerFused,
+        submodules=dsa_fused.DSAIndexerFusedSubmodules(linear_wq_b=_Linear, linear_wk=_Linear, k_norm=_Norm, linear_weights_proj=_Linear)))
+    torch.manual_seed(0)
+    mod = dsa_fused.DSAttentionFused(cfg, sub, layer_number=1, attn_mask_type=AttnMaskType.causal, attention_type="self", k_channels=192)
+    for p in mod.parameters():
+        if p.ndim == 2:
+            torch.nn.init.normal_(p, std=p.shape[1] ** -0.5)
+    mod = mod.to(gpu).train()
+    g = torch.Generator(device=gpu).manual_seed(0)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=torch.bfloat16)      # noqa: E731
+    query, key, x, qr, dout = rnd(S, 1, H, 576).requires_grad_(True), rnd(S, 1, 576).requires_grad_(True), rnd(S, 1, hid), rnd(S, 1, qlr), rnd(1, S, H, 512)
+    value = None if scale is None else torch.tensor(4.0, device=gpu) if scale == 4.0 else torch.tensor(4.0)
+
+    class Subclass(megatron_compat.DSAIndexerLossAutoScaler):        # no longer the class itself: the two nodes
+        pass
+
+    calls = []
+    attach = ops.attached_indexer_kl_loss
+    monkeypatch.setattr(ops, "attached_indexer_kl_loss", lambda *a: (calls.append(1), attach(*a))[1])
+    monkeypatch.setattr(megatron_compat.DSAIndexerLossAutoScaler, "main_loss_backward_scale", value)
+
+    def run():
+        inputs = [query, key] + [p for p in mod.parameters() if p.requires_grad]
+        out = mod(query, key, None, None, x=x, qr=qr, attn_mask_type=AttnMaskType.causal)
+        first = torch.autograd.grad(out, inputs, dout, retain_graph=True, allow_unused=True)
+        again = torch.autograd.grad(out, inputs, dout, allow_unused=True)
+        assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(first, again))
+        return [out.detach(), dsa_fused.DSAIndexerLossLoggingHelperFused.tracker[1], *first]
+
+    def same(a, b):
+        assert len(a) == len(b) and all((u is None and v is None) or torch.equal(u, v) for u, v in zip(a, b))
+
+    one = run()
+    assert calls == [1]
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.clone())[1], lambda t: t):
+        same(run(), one)
+    assert (S, 128) in packed
+    with monkeypatch.context() as m:
+        m.setattr(dsa_fused, "DSAIndexerLossAutoScaler", Subclass)
+        same(run(), one)
+    assert len(calls) == 2
+    mod.indexer.requires_grad_(False)
+    frozen = run()
+    same(frozen, one[:4])
+
+
 @pytest.mark.parametrize("heads,sinks", [(16, 16), (16, 4), (48, 48), (40, 64)])
 def test_attention_sinks_of_padded_heads(gpu, heads, sinks):
     """A sink for every head, or one for several neighbouring ones, goes with the heads of the query and not with the padded ones; one that
