@@ -24,7 +24,10 @@
 // Modes 1 and 2 are mla_fwd_kernel: four waves of up to 512 registers, one per SIMD.  They spend 68 / 52 matrix
 // instructions per wave on two tiles and are then bound by the gather.  A query's heads may also be spread over several
 // workgroups, and its slots over `ksplit` of them (few queries: one workgroup per query would leave most of the 256
-// compute units idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together.
+// compute units idle); those write unnormalised fp32 sums that mla_fwd_combine_kernel puts together, or, of two ranges in
+// modes 1 and 2, the second of their workgroups.
+#include <atomic>
+#include <chrono>
 #include <type_traits>
 
 #include "mla_tile.h"
@@ -65,6 +68,7 @@ struct FwdArgs {
   int n_hg, ksplit, k_loc;                   // head groups per query, slot ranges per query, slots of a range
   int span;                                  // modes 1 - 4: neighbouring queries (ranges) on one XCD
   f32x4* part_o; float* part_ml;             // ksplit > 1: sums [S][ksplit][H/32][16][4][64] x 4, (m, l) [S][ksplit][H][2]
+  unsigned long long *turn, token;           // two ranges that meet by themselves: [S][n_hg], else null; the call's number
 };
 
 // The softmax of a head is taken relative to a reference point, the maximum of the first tile, so the
@@ -136,6 +140,14 @@ __device__ __forceinline__ void store_partial(const f32x16& t, f32x4* p) {
   for (int j = 0; j < 4; j++) {
     const f32x4 v = {t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]};
     p[j * 64] = v;
+  }
+}
+// The same in device scope: written through, for a workgroup on another XCD to read
+__device__ __forceinline__ void store_partial_through(const f32x16& t, f32x4* p) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const f32x4 v = {t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]};
+    asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p + j * 64), "v"(v) : "memory");
   }
 }
 __device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned short* p) {   // all lanes of the wave
@@ -480,7 +492,7 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
   // wave sends the other's half of the column tiles and finishes its own, so that all four waves store: with the second stream's
   // sums all sent to the first, two waves stored the 131 KB of 64 heads while two had ended. ---------------------------------
   __syncthreads();                         // the last tiles and the id arrays have been read
-  static_assert(2 * NDT * 4096 + 1024 + 8 <= RING, "the hand-over fits the tile ring");
+  static_assert(2 * NDT * 4096 + 1024 + 16 <= RING, "the hand-over fits the tile ring");
   float* ml = (float*)(smem + 2 * NDT * 4096);             // [stream][sub][32][2], behind the waves' boxes
   if (g == 0) {
     ml[((stream * 2 + sub) * 32 + r) * 2] = again ? __builtin_bit_cast(float, REDO_MARK) : m_ref;
@@ -543,19 +555,88 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
     else finish(std::integral_constant<int, HALF>{}, write);
   };
   if (SPLIT) {
-    if (!head_ok) return;                    // the same for all lanes of a wave
-    float* const part_ml = a.part_ml + (((size_t)qi * a.ksplit + sp) * H + h) * 2;
-    if (again) {
-      if (stats) part_ml[0] = __builtin_bit_cast(float, REDO_MARK);
+    if (!head_ok && !a.turn) return;         // the same for all lanes of a wave
+    const size_t range_ml = (size_t)H * 2, range_o = (size_t)(H / 32) * DTILES * 256;
+    float* const part_ml = a.part_ml + ((size_t)qi * a.ksplit * H + h) * 2;
+    f32x4* const po = a.part_o + (((size_t)qi * a.ksplit * (H / 32) + hb) * DTILES + dt0) * 256 + lane;
+    if (head_ok) {
+      if (stats) {
+        __hip_atomic_store(part_ml + sp * range_ml, again ? __builtin_bit_cast(float, REDO_MARK) : m_ref, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(part_ml + sp * range_ml + 1, l_tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (!again) finish_mine([&](const f32x16& t, int dt) {
+        if (a.turn) store_partial_through(t, po + sp * range_o + dt * 256);
+        else store_partial(t, po + sp * range_o + dt * 256);
+      });
+    }
+    if (!a.turn) return;
+    // Two ranges: the workgroup that is second to have its sums in memory puts both together.  Whatever the word of the pair held, it
+    // holds the call's number once the first has been there.
+    unsigned* const second_s = marked_s + 2;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (a barrier alone does not wait for other waves' stores)
+    __syncthreads();
+    if (tid == 0) {
+      unsigned long long* const word = a.turn + (size_t)qi * a.n_hg + hg;
+      const bool second = __hip_atomic_exchange(word, a.token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.token;
+      if (second) *word = 0;                 // (the number comes again where a captured launch is replayed)
+      *second_s = second;
+    }
+    __syncthreads();
+    if (!__builtin_amdgcn_readfirstlane(*second_s)) return;
+    asm volatile("" ::: "memory");
+    if (head_ok) {
+      const float m_x = __hip_atomic_load(part_ml + (sp ^ 1) * range_ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const float l_x = __hip_atomic_load(part_ml + (sp ^ 1) * range_ml + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      again |= is_marked(m_x);               // the same for all heads of a block
+      if (!again) {
+        const f32x4* const px = po + (sp ^ 1) * range_o;
+        const float top = fmaxf(m_ref, m_x), e_own = __builtin_amdgcn_exp2f(m_ref - top), e_x = __builtin_amdgcn_exp2f(m_x - top);
+        // the first range's terms first, as mla_fwd_combine_kernel has them
+        const Final fin = finish_head(top, sp == 0 ? fmaf(l_x, e_x, l_tot * e_own) : fmaf(l_tot, e_own, l_x * e_x), a.sink ? a.sink + h : nullptr);
+        if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
+        unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
+        constexpr int AHEAD = MODE == 1 ? 2 : 4;     // column tiles of the other range on their way
+        f32x4 x[AHEAD][4];
+        const int first_dt = stream == 0 ? 0 : HALF;
+        auto request = [&](int i) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const unsigned long long* p8 = (const unsigned long long*)(px + (first_dt + i) * 256 + j * 64);
+            const unsigned long long lo = __hip_atomic_load(p8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), hi = __hip_atomic_load(p8 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+            x[i % AHEAD][j] = __builtin_bit_cast(f32x4, (u64x2{lo, hi}));
+          }
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) request(i);
+        finish_mine([&](const f32x16& t, int dt) {
+          const int i = dt % HALF;
+          f32x16 o;
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const float own = t[4 * j + e], y = x[i % AHEAD][j][e];
+              o[4 * j + e] = sp == 0 ? fmaf(y, e_x, own * e_own) : fmaf(own, e_own, y * e_x);
+            }
+          if (i + AHEAD < HALF) request(i + AHEAD);
+          store_out(o, fin.inv, op + 32 * dt);
+        });
+      }
+    }
+    if (MODE == 2) {
+      if (again) {
+#pragma unroll 1
+        for (int dt = wave; dt < DTILES; dt += 4) {
+          f32x16 acc;
+          float m, l;
+          redo_block<false>(a, qi, hb, dt, acc, m, l, tid);
+          write_block(a, qi, hb, dt, acc, m, l, tid);
+        }
+      }
       return;
     }
-    if (stats) { part_ml[0] = m_ref; part_ml[1] = l_tot; }
-    f32x4* po = a.part_o + ((((size_t)qi * a.ksplit + sp) * (H / 32) + hb) * DTILES + dt0) * 256 + lane;
-    finish_mine([&](const f32x16& t, int dt) { store_partial(t, po + dt * 256); });
-    return;
-  }
-  if (head_ok && !again) {
-    const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
+  } else if (head_ok && !again) {    const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
     if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
     unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
     finish_mine([&](const f32x16& t, int dt) { store_out(t, fin.inv, op + 32 * dt); });
@@ -1353,6 +1434,13 @@ int max_slots(int mode) {                    // slots of a range whose id arrays
 constexpr int SHARE_RANGES = 4, SHARE_BLOCKS = 16;
 bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES && (long)S * (H / 32) <= SHARE_BLOCKS; }
 
+// Two ranges of modes 1 and 2 meet by themselves: both workgroups write their sums, through to where every XCD sees them, and the one
+// that is second puts its own, which it still has, beside the other's.  That is one launch less, and half of the sums are read.  us, with
+// mla_fwd_combine_kernel behind / so: 48 queries x 128 heads x 2048 slots 52.5 / 49.4, 61 x 64 x 1024 29.6 / 27.8, 121 x 32 x 1024 28.6 / 26.0, 30 x
+// 128 x 1024 28.4 / 27.0.  With fences for the whole device around plain stores and loads 37 for the second of these (each writes back, or
+// drops, an XCD's whole L2), with such stores and a fence before plain loads 33.
+bool ranges_meet(int mode, int ksplit) { return ksplit == 2 && (mode == 1 || mode == 2); }
+
 // The mode and the number of slot ranges with the least estimated time: rounds of workgroups over the 256 compute
 // units (512 places in modes 3 and 4), each a fixed part (Q rows, ids, first tile, epilogue) plus its pairs of tiles, plus the kernel
 // that follows.  The constants are measured times in us, random rows.  A round among others, FULL: the rows of all its queries come in
@@ -1378,7 +1466,7 @@ bool combine_shares(int S, int H, int ksplit) { return ksplit >= SHARE_RANGES &&
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
 // mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.
 FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
-  constexpr float WHOLE = 1.8f, WHOLE_FEW = 4.6f, COMBINE = 2.37f, COMBINE_RANGE = 0.22f, SHARED_RANGE = 0.1f, COMBINE_BYTES_PER_US = 6.2e6f;
+  constexpr float WHOLE = 1.8f, WHOLE_FEW = 4.6f, COMBINE = 2.37f, COMBINE_RANGE = 0.22f, SHARED_RANGE = 0.1f, COMBINE_BYTES_PER_US = 6.2e6f, MEET_BYTES = 0.62f;
   constexpr float FIXED_IDLE[5] = {4.91f, 5.86f, 4.51f, 5.57f, 3.8f}, FIXED_FULL[5] = {14.5f, 10.5f, 6.8f, 9.0f, 8.5f};
   constexpr float PAIR_FULL[5] = {3.36f, 2.1f, 1.8f, 4.05f, 2.8f}, PAIR_IDLE[5] = {2.35f, 1.68f, 1.31f, 2.82f, 1.78f};
   constexpr float PAIR_LAST[3] = {3.65f, 2.24f, 1.75f}, PAIR_SHARED[5] = {0.f, 0.f, 0.f, 3.41f, 1.42f};
@@ -1405,7 +1493,8 @@ FwdPlan plan_fwd(int S, int H, int K, bool may_split) {
       float t = (float)rounds * (FIXED_FULL[mode] + per * PAIR_FULL[mode]);
       if (rest > 0.0f) t += fixed + per * pair;
       t += ksplit == 1 ? (mode >= 2 ? 0.0f : pairs <= 8 ? WHOLE_FEW : WHOLE)
-                       : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit + (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
+                       : COMBINE + (combine_shares(S, H, ksplit) ? SHARED_RANGE : COMBINE_RANGE) * ksplit +
+                             (ranges_meet(mode, ksplit) ? MEET_BYTES : 1.0f) * (float)S * ksplit * H * (2 * DV * 4) / COMBINE_BYTES_PER_US;
       if (t < best_t) { best_t = t; best = {mode, n_hg, ksplit, 64 * per}; }
       if (wgs >= 4096) break;                // more ranges only add rounds
     }
@@ -1423,7 +1512,16 @@ int unit_span(const FwdPlan& p, int S) {
 }
 
 size_t part_bytes(const FwdPlan& p, int S, int H) {
-  return p.ksplit > 1 ? (size_t)S * p.ksplit * H * (DV * 4 + 8) + 256 : 0;
+  if (p.ksplit == 1) return 0;
+  return (size_t)S * p.ksplit * H * (DV * 4 + 8) + 256 + (ranges_meet(p.mode, p.ksplit) ? (size_t)S * p.n_hg * 8 : 0);
+}
+
+// A number that no other call of the process has, and that what lies in uninitialised memory does not hold but by a chance of 2^-64.
+unsigned long long call_number() {
+  static std::atomic<unsigned long long> next{(unsigned long long)std::chrono::system_clock::now().time_since_epoch().count() << 20};
+  unsigned long long x = next.fetch_add(1, std::memory_order_relaxed);
+  x = (x ^ x >> 31) * 0x9e3779b97f4a7c15ull;           // (one to one)
+  return x ? x : call_number();
 }
 
 template <int MODE, bool SPLIT, int POUT>
@@ -1451,6 +1549,7 @@ int launch_fwd(const FwdArgs& a, int p_out_f32, bool shared, hipStream_t st) {
   else DSA_FWD_LAUNCH(2);
 #undef DSA_FWD_LAUNCH
   const size_t tail = (size_t)TILE_BYTES + ids_lds_bytes(a.K);           // one tile and the ids, for blocks done again
+  if (a.turn) return 0;
   auto combine = shared ? mla_fwd_combine_kernel<true> : mla_fwd_combine_kernel<false>;
   if (!SPLIT) return 0;
   if (dsa_reserve_lds((const void*)combine, tail) != hipSuccess) return -2;
@@ -1481,7 +1580,11 @@ int fwd_impl(const void* q, const void* kv, const int32_t* ids, int S_all, int S
   if (part_bytes(p, S, H) > workspace_bytes || (p.ksplit > 1 && workspace == nullptr)) p = plan_fwd(S_all, H, K, false);
   FwdArgs a{(const __bf16*)q, (const __bf16*)kv, ids, (__bf16*)out, lse, p_out, S, H, Skv, K, q_start, sm_scale, attn_sink,
             p_out ? p_out_skip : 0, p_all, p.n_hg, p.ksplit, p.k_loc, unit_span(p, S), (f32x4*)workspace,
-            (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4)};
+            (float*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * DV * 4), nullptr, 0};
+  if (ranges_meet(p.mode, p.ksplit)) {
+    a.turn = (unsigned long long*)((unsigned char*)workspace + (size_t)S * p.ksplit * H * (DV * 4 + 8));
+    a.token = call_number();
+  }
   int rc;
   const bool split = p.ksplit > 1, shared = combine_shares(S_all, H, p.ksplit);
   if (p.mode == 0) rc = split ? launch_fwd<0, true>(a, p_out_f32, shared, st) : launch_fwd<0, false>(a, p_out_f32, shared, st);

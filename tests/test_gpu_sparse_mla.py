@@ -321,6 +321,59 @@ def test_forward_of_long_lists_in_every_form_for_many_queries(gpu, form, ranges,
                 assert torch.equal(p.to(torch.bfloat16), p16)
 
 
+@pytest.mark.parametrize("form,S,H,K", [(2, 128, 32, 1024), (2, 61, 64, 1024), (2, 40, 96, 1024), (1, 115, 64, 2048), (1, 61, 96, 2048), (1, 55, 128, 2048)])
+def test_two_ranges_of_slots_that_meet(gpu, form, S, H, K):
+    """Two ranges whose second workgroup puts both together: keys that beat all before them by far more than 2^64 in the first range, in
+    the second, in both; rows with nothing in one range or in either; sinks; whatever the workspace held; replays of a captured call."""
+    from loongforge_amd import _lib, ops
+
+    assert mla_form(S, H, K) == (form, 2)
+    lib, skv, g = _lib.load(), K + 900, torch.Generator().manual_seed(S + H)
+    q, kv = (torch.randn(*shape, generator=g).to(torch.bfloat16) for shape in ((S, H, 576), (skv, 576)))
+    idx = torch.stack([torch.randperm(skv - 4, generator=g)[:K] for _ in range(S)]).int()
+    idx[3] = -1
+    idx[4, :K // 2] = -1
+    idx[5, K // 2:] = -1
+    for n, (row, slots) in enumerate([(6, [K // 2 - 1]), (7, [K - 1]), (8, [K // 2 - 1, K - 1])]):
+        idx[row, slots[-1]] = skv - 1 - n
+        idx[row, slots[0]] = skv - 1 - n if len(slots) == 1 else skv - 4
+        kv[skv - 1 - n] = (q[row, H - 1].float() * 40.0).to(torch.bfloat16)
+    kv[skv - 4] = kv[skv - 3] * 1.5
+    rows, sm = list(range(12)) + [S - 1], 192 ** -0.5
+    qg, kvg, ig = q.to(gpu), kv.to(gpu), idx.to(gpu)
+    for sk in (None, torch.linspace(-2, 2, H)):
+        sg = None if sk is None else sk.to(gpu)
+        out, lse, _ = ops.sparse_mla_fwd(qg, kvg, ig, skv, sm, attn_sink=sg)
+        ref = [O.sparse_mla_fwd(q[i:i + 1], kv, idx[i:i + 1], skv, sm, 512, attn_sink=sk) for i in rows]
+        ro, rl = (torch.cat(x) for x in list(zip(*ref))[:2])
+        assert_close(out[rows], ro, "out", atol=4e-2)
+        got, fin = lse[rows].cpu(), torch.isfinite(rl)
+        assert torch.equal(torch.isposinf(got), ~fin) and ((got - rl)[fin].abs() / rl[fin].abs().clamp_min(1)).max().item() < 1e-3
+        nbytes = lib.dsa_sparse_mla_fwd_workspace_bytes(S, H, skv, K)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+        for fill in (0, 255, 85, None, None):
+            if fill is not None:
+                ws.fill_(fill)
+            o2, l2 = torch.full_like(out, 7.0), torch.full_like(lse, 7.0)
+            rc = lib.dsa_sparse_mla_fwd_ws(qg.data_ptr(), kvg.data_ptr(), ig.data_ptr(), S, H, skv, K, skv, sm, 512, o2.data_ptr(), l2.data_ptr(),
+                                           None, 0, None if sg is None else sg.data_ptr(), 0, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.dsa_last_error()
+            assert torch.equal(o2, out) and torch.equal(l2, lse)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    plain = ops.sparse_mla_fwd(qg, kvg, ig, skv, sm)[0]
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        ops.sparse_mla_fwd(qg, kvg, ig, skv, sm)
+    torch.cuda.current_stream().wait_stream(stream)
+    with torch.cuda.graph(graph):
+        captured = ops.sparse_mla_fwd(qg, kvg, ig, skv, sm)[0]
+    for _ in range(4):
+        captured.zero_()
+        graph.replay()
+        assert torch.equal(captured, plain)
+        assert torch.equal(ops.sparse_mla_fwd(qg, kvg, ig, skv, sm)[0], plain)
+
+
 def test_forward_slot_permutation_invariance(gpu):
     inp = O.make_mla_inputs(100, 128, 128, seed=7)
     out1, lse1, _ = _run_fwd(inp, gpu)
