@@ -1345,7 +1345,7 @@ int run_bwd(const char* name, BwdArgs A, int S, int Hi, int span, float* d_k8, c
     A.q0 = q0;
     A.cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     // every id inside [0, Sk) counts: the causal window was already applied when the ids were selected
-    order::build(A.ids, q0, A.cnt, K, Sk, 0x3fffffff, bitmap, prefix, count, start, dstp, p.W, st, dup_flag);
+    order::build(A.ids, q0, A.cnt, K, Sk, 0x3fffffff, bitmap, prefix, count, start, dstp, p.W, order::Room{A.rows, p.total - p.off_rows}, st, dup_flag);
     DSA_CHECK_LAUNCH("indexer_bwd(order)");
     kern<<<dim3(A.cnt), dim3(THREADS), smem, st>>>(A);
     DSA_CHECK_LAUNCH("indexer_bwd");

@@ -1434,6 +1434,7 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   unsigned char* rows = ws + p.off_rows;
   unsigned char* exps = ws + p.off_exps;       // (units)
   float* acc = (float*)(ws + p.off_acc);
+  const order::Room room{pds, p.off_exps - p.off_pds};       // (the sweep before has read them when the next order is made)
 
   const int HG = head_groups(H);
   // The passes are free to choose their slot order (P, dS and the dKV rows never leave the workspace): they walk each query's valid
@@ -1480,8 +1481,8 @@ static int bwd_impl(const void* q, const void* kv, const void* out, const void* 
   for (int q0 = 0; q0 < S; q0 += p.chunk) {
     const int cnt = S - q0 < p.chunk ? S - q0 : p.chunk;
     DSA_MARK(0);
-    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S), (uint4*)exps, work);
-    else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, st, dup_flag, sort_ids ? sorted : nullptr);
+    if (G > 1) order::build_units(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, room, st, dup_flag, sorted, G, bad, units + q0 / G, unit_slots(HG, K), unit_cost(HG, S), (uint4*)exps, work);
+    else order::build(ids, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dstp, p.W, room, st, dup_flag, sort_ids ? sorted : nullptr);
     DSA_CHECK_LAUNCH("dsa_sparse_mla_bwd(order)");
     const int* sids = sort_ids ? sorted : ids + (size_t)q0 * K;      // row ql belongs to query q0 + ql
     DSA_MARK(1);

@@ -1462,6 +1462,10 @@ bool ranges_meet(int mode, int ksplit) { return ksplit == 2 && (mode == 1 || mod
 // mode 0 and 390 in mode 3, 640 slots 760 and 800 (150 queries x 256 slots 28.6 and 31.2).
 // WHOLE: what modes 0 and 1 take beyond the fit with all slots in one workgroup, more with few pairs (250 queries x 64 heads x 256 slots
 // 27.5 us in mode 1 and 23.7 in mode 3, 89 x 128 x 256 22.8 and 21.2; 94 x 128 x 2048 82.6 in mode 1 and 87.6 in two ranges of mode 0).
+// MEET_BYTES: what two ranges that meet (modes 1 and 2) take of the time for the sums' bytes, of which half are not read back; the wait of one
+// workgroup for the other takes the place of the launch.  251 random sizes of 32 - 128 heads, 1 - 256 queries, 128 - 2048 slots: 0.975 of the time
+// with a kernel behind all ranges in the mean, 0.89 to 1.025; with nothing but the bytes for them small calls split where they should not
+// (up to 1.27).
 // Blocks done again inside them and not by a kernel behind: 168 x 64 x 512 35.2 -> 32.2 us, 108 x 128 x 1024 52.7 -> 50.6.
 // One pair of tiles is always mode 3, so that a query has the same bits whatever heads stand beside it: 4000 queries of 128 heads 320 us in
 // mode 0 and 278, 1800 of 64 heads 90 and 64, 2 of 32 11.0 and 10.4.

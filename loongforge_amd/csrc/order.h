@@ -7,6 +7,8 @@
 // repeated id (the bit it sets is set already) and raises *dup_flag; the callers' last kernels then
 // fill their outputs with NaN instead of returning sums that silently miss a term.
 #pragma once
+#include <type_traits>
+
 #include "dsa_common.h"
 
 namespace order {
@@ -18,9 +20,7 @@ static __global__ void zero_u32_kernel(unsigned* __restrict__ p, size_t n) {
 // bitmap[w][key] bit b  <=>  local query 32w + b selects key (keys contiguous: the kernels behind it read it along the keys).
 // Built without global atomics, in two steps.  (1) One workgroup per query sets the query's bits
 // over the keys in LDS and writes them out as one row of qmap[query][key / 32] (Wk words).
-// (2) A transpose of the bit matrix: a wave loads the words of 64 consecutive queries for one key
-// word and turns bit b of all lanes into the 64-bit mask of key 32*kw + b with one ballot; the
-// masks of 4 such query groups are combined through LDS so that 32 keys of a word row are written at a time.
+// (2) A transpose of the bit matrix: a wave loads the words of 64 consecutive queries for 64 keys and turns them in its registers.
 static __global__ __launch_bounds__(256) void qmap_kernel(const int* __restrict__ ids, int q0, int cnt, int K, int Skv,
                                                           int q_start, unsigned* __restrict__ qmap, int Wk,
                                                           int* __restrict__ sorted, int* __restrict__ dup_flag) {
@@ -282,87 +282,38 @@ static __global__ __launch_bounds__(BL) void qmap_unit_kernel(const int* __restr
   for (int t = 4 * tid; t < n_ids; t += 4 * BL) *(int4*)(row + t) = *(const int4*)(list + t);
 }
 
-// grid (ceil(cnt / 256), Wk); workgroup = 4 waves = 256 queries of one key word
-static __global__ __launch_bounds__(256) void bm_transpose_kernel(const unsigned* __restrict__ qmap, int cnt, int Skv, int Wk,
-                                                                  unsigned* __restrict__ bitmap, int W) {
-  __shared__ unsigned long long mask_s[32][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kw = blockIdx.y;
-  const int ql = blockIdx.x * 256 + threadIdx.x;
-  const unsigned word = ql < cnt ? qmap[(size_t)ql * Wk + kw] : 0u;
-#pragma unroll
-  for (int b = 0; b < 32; b++) {
-    const unsigned long long m = __ballot((word >> b) & 1u);
-    if (lane == b) mask_s[b][wave] = m;
-  }
-  __syncthreads();
-  // thread t: 32-bit piece t / 32 of the 256 queries of this workgroup, key bit t % 32
-  const int piece = threadIdx.x >> 5, b = threadIdx.x & 31;
-  const int key = kw * 32 + b;
-  const int w = blockIdx.x * 8 + piece;
-  if (key < Skv && w < W) bitmap[(size_t)w * Skv + key] = ((const unsigned*)&mask_s[b][0])[piece];
+// A 64 x 64 bit matrix across a wave, lane = row with columns 0 - 31 in `lo` and 32 - 63 in `hi`, becomes its transpose.
+__device__ __forceinline__ void transpose64(unsigned& lo, unsigned& hi, int lane) {
+  // the off-diagonal quarters: the upper half-wave's lo against the lower one's hi
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
+  // then bit o of lane and column for o = 16 .. 1: half of the bits are the partner's, from o columns to the right or left
+  auto step = [&](auto o_c, unsigned m) {
+    constexpr int o = decltype(o_c)::value;
+    const bool up = lane & o;
+    const unsigned take = up ? m : ~m, by = up ? o : 32 - o;
+    auto swap = [&](unsigned& x) {
+      const unsigned y = (unsigned)__builtin_amdgcn_ds_swizzle((int)x, o << 10 | 0x1f);
+      x = (x & ~take) | (__builtin_amdgcn_alignbit(y, y, by) & take);
+    };
+    swap(lo);
+    swap(hi);
+  };
+  step(std::integral_constant<int, 16>{}, 0x0000ffffu);
+  step(std::integral_constant<int, 8>{}, 0x00ff00ffu);
+  step(std::integral_constant<int, 4>{}, 0x0f0f0f0fu);
+  step(std::integral_constant<int, 2>{}, 0x33333333u);
+  step(std::integral_constant<int, 1>{}, 0x55555555u);
 }
 
-// prefix[w][key] = number of set bits of the key in words < w; count[key] = total.  A workgroup takes 64 keys; its 16 waves
-// count a part of the words each, then write the prefixes of that part.  Workgroups behind those clear `marks` (n_marks of 16 bytes)
-// if there is a unit: the counting leaves most of the chip idle.
-static __global__ __launch_bounds__(1024) void bm_prefix_kernel(const unsigned* __restrict__ bitmap, unsigned* __restrict__ prefix,
-                                                                int* __restrict__ count, int Skv, int W, const int* __restrict__ flags,
-                                                                uint4* __restrict__ marks, size_t n_marks) {
-  __shared__ int part[16][64];
-  const int counting = (Skv + 63) / 64;
-  if ((int)blockIdx.x >= counting) {
-    if (flags[1])
-      for (size_t e = (size_t)((int)blockIdx.x - counting) * 1024 + threadIdx.x; e < n_marks; e += (size_t)(gridDim.x - counting) * 1024)
-        marks[e] = make_uint4(0u, 0u, 0u, 0u);
-    return;
-  }
-  const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
-  const int key = min(blockIdx.x * 64 + lane, (unsigned)Skv - 1u);
-  const bool live = blockIdx.x * 64 + lane < (unsigned)Skv;
-  const int per = (W + 15) / 16;
-  const int w0 = seg * per, w1 = min(w0 + per, W);
-  int n = 0;
-#pragma unroll 8
-  for (int w = w0; w < w1; w++) n += __popc(bitmap[(size_t)w * Skv + key]);
-  part[seg][lane] = n;
-  __syncthreads();
-  int run = 0;
-  for (int s = 0; s < seg; s++) run += part[s][lane];
-  if (live) {
-#pragma unroll 8
-    for (int w = w0; w < w1; w++) {
-      prefix[(size_t)w * Skv + key] = (unsigned)run;
-      run += __popc(bitmap[(size_t)w * Skv + key]);
-    }
-    if (seg == 15) count[key] = run;
-  }
-}
-
-// Exclusive prefix sums of value(k), k in [0, n), by one workgroup: put(k, sum, value) for each; returns the total.
-template <class Value, class Put>
-__device__ __forceinline__ int scan_block(int n_values, Value value, Put put) {
-  __shared__ int wsum[16];
-  __shared__ int carry_s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (int base = 0; base < n_values; base += 1024) {
-    const int k = base + tid;
-    const int c = k < n_values ? value(k) : 0;
-    int inc = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { int n = __shfl_up(inc, o, 64); if (lane >= o) inc += n; }
-    if (lane == 63) wsum[wave] = inc;
-    __syncthreads();
-    int before = carry_s;
-    for (int w = 0; w < wave; w++) before += wsum[w];
-    if (k < n_values) put(k, before + inc - c, c);
-    __syncthreads();
-    if (tid == 1023) carry_s = before + inc;
-    __syncthreads();
-  }
-  return carry_s;
+// inclusive sums over the lanes of a wave, within the vector unit (rows of 16 lanes, then their ends to the rows behind them)
+__device__ __forceinline__ int wave_sums(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);       // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast 15, into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast 31, into rows 2 and 3
+  return x;
 }
 
 // What there is to do where some groups of G queries are units: work[2 ..] = first query << 8 | tiles of 32 slots for the units, query << 8
@@ -371,53 +322,203 @@ __device__ __forceinline__ int scan_block(int n_values, Value value, Put put) {
 // one and its neighbour that does the other displace each other's code from the instruction cache that they share.
 struct WorkList { const int* units; int cnt, G; int* work; };
 
-// start[key] = exclusive prefix sum of count (one workgroup; Skv is at most a few 10^5).  A second workgroup makes the work list.
-static __global__ __launch_bounds__(1024) void key_scan_kernel(const int* __restrict__ count, int* __restrict__ start, int Skv, WorkList list) {
-  if (blockIdx.x == 0) {
-    const int total = scan_block(Skv, [&](int k) { return count[k]; }, [&](int k, int sum, int) { start[k] = sum; });
-    if (threadIdx.x == 0) start[Skv] = total;
-  } else {
-    const int G = list.G, groups = (list.cnt + G - 1) / G;
-    auto tiles = [&](int k) { return list.units[groups - 1 - k] / 32; };
-    auto unit = [&](int k) { return tiles(k) ? 1 : 0; };
-    auto apart = [&](int k) { return tiles(k) ? 0 : min(G, list.cnt - (groups - 1 - k) * G); };
-    const int n_units = scan_block(groups, unit, [](int, int, int) {}), n_apart = list.cnt - G * n_units;
-    const bool units_first = n_units <= n_apart;
-    __syncthreads();
-    scan_block(groups, unit, [&](int k, int sum, int n) {
-      if (n) list.work[2 + (units_first ? 0 : n_apart) + sum] = ((groups - 1 - k) * G) << 8 | tiles(k);
-    });
-    __syncthreads();
-    scan_block(groups, apart, [&](int k, int sum, int n) {
-      for (int j = 0; j < n; j++) list.work[2 + (units_first ? n_units : 0) + sum + j] = ((groups - 1 - k) * G + n - 1 - j) << 8;
-    });
-    if (threadIdx.x == 0) {
-      list.work[0] = n_units + n_apart;
-      list.work[1] = min(n_units, n_apart);
-    }
+// One workgroup of 1024 threads, each with a run of the groups, which it counts and then, from the counts of those before it, writes.
+__device__ __forceinline__ void make_work_list(const WorkList& list) {
+  __shared__ int wave_units[16], wave_apart[16];
+  const int G = list.G, groups = (list.cnt + G - 1) / G, per = (groups + 1023) / 1024;
+  const int k0 = min((int)threadIdx.x * per, groups), k1 = min(k0 + per, groups);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int units = 0, apart = 0;
+  for (int k = k0; k < k1; k++) {
+    if (list.units[groups - 1 - k] / 32) units++;
+    else apart += min(G, list.cnt - (groups - 1 - k) * G);
+  }
+  int at_u = wave_sums(units), at_a = wave_sums(apart);
+  if (lane == 63) { wave_units[wave] = at_u; wave_apart[wave] = at_a; }
+  __syncthreads();
+  at_u -= units;
+  at_a -= apart;
+  int n_units = 0, n_apart = 0;
+  for (int w = 0; w < 16; w++) {
+    if (w < wave) { at_u += wave_units[w]; at_a += wave_apart[w]; }
+    n_units += wave_units[w];
+    n_apart += wave_apart[w];
+  }
+  const bool units_first = n_units <= n_apart;
+  int* to_u = list.work + 2 + (units_first ? 0 : n_apart) + at_u;
+  int* to_a = list.work + 2 + (units_first ? n_units : 0) + at_a;
+  for (int k = k0; k < k1; k++) {
+    const int g = groups - 1 - k, tiles = list.units[g] / 32;
+    if (tiles) *to_u++ = (g * G) << 8 | tiles;
+    else for (int j = min(G, list.cnt - g * G) - 1; j >= 0; j--) *to_a++ = (g * G + j) << 8;
+  }
+  if (threadIdx.x == 0) {
+    list.work[0] = n_units + n_apart;
+    list.work[1] = min(n_units, n_apart);
   }
 }
 
+// A share of the clearing of `marks` (n_marks of 16 bytes), which are read if there is a unit: it goes beside kernels that leave most of
+// the chip idle.
+struct Marks { const int* flags; uint4* at; size_t n; int blocks; };
+__device__ __forceinline__ void clear_marks(const Marks& m, int block) {
+  if (m.flags[1])
+    for (size_t e = (size_t)block * 1024 + threadIdx.x; e < m.n; e += (size_t)m.blocks * 1024) m.at[e] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// BITS: bitmap from qmap.  COUNTS: prefix[w][key] = number of set bits of the key in words < w; count[key] = total.  A workgroup takes 64
+// keys; its 16 waves turn and count a part of the queries each, 64 at a time, then write the prefixes of that part.  Others clear marks,
+// and a last one makes the work list, if there is one.  Both at once where
+// qmap does not lie in the prefixes' place.  An XCD has a run of keys, and so its L2 the 128-byte lines of qmap that 16 workgroups share.
+template <bool BITS, bool COUNTS>
+static __global__ __launch_bounds__(1024) void key_bits_kernel(const unsigned* qmap, int cnt, int Skv, int Wk, unsigned* bitmap,
+                                                               unsigned* prefix, int* __restrict__ count, int W, int per_xcd, WorkList list, Marks marks) {
+  __shared__ int part[16][64];
+  const int beside = (int)blockIdx.x - 8 * per_xcd, kb = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+  if (beside >= 0) {
+    if (beside < marks.blocks) clear_marks(marks, beside);
+    else make_work_list(list);
+    return;
+  }
+  if (64 * kb >= Skv) return;
+  const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int key = kb * 64 + lane, kw = 2 * kb;
+  const bool live = key < Skv;
+  unsigned* bits = bitmap + min(key, Skv - 1);
+  const int pairs = (W + 1) / 2, per = (pairs + 15) / 16;
+  const int p0 = min(seg * per, pairs), p1 = min(p0 + per, pairs), w1 = min(2 * p1, W);
+  unsigned lo[4], hi[4];
+  int n = 0;
+  if (BITS) {
+    for (int p = p0; p < p1; p += 4) {
+      const unsigned* src = qmap + (size_t)(64 * p + lane) * Wk + kw;
+      const int left = cnt - 64 * p - lane;             // queries from the lane's first on
+      if (Wk & 1) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const bool in = p + i < p1 && 64 * i < left;
+          lo[i] = in ? src[(size_t)64 * i * Wk] : 0u;
+          hi[i] = in && kw + 1 < Wk ? src[(size_t)64 * i * Wk + 1] : 0u;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const uint2 v = p + i < p1 && 64 * i < left ? *(const uint2*)(src + (size_t)64 * i * Wk) : make_uint2(0u, 0u);
+          lo[i] = v.x;
+          hi[i] = v.y;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (p + i >= p1) break;
+        transpose64(lo[i], hi[i], lane);
+        const int w = 2 * (p + i);
+        if (live) {
+          bits[(size_t)w * Skv] = lo[i];
+          if (w + 1 < W) bits[(size_t)(w + 1) * Skv] = hi[i];        // (else of queries beyond the last: none)
+        }
+        n += __popc(lo[i]) + __popc(hi[i]);
+      }
+    }
+  } else {
+#pragma unroll 8
+    for (int w = 2 * p0; w < w1; w++) n += __popc(bits[(size_t)w * Skv]);
+  }
+  if (!COUNTS) return;
+  part[seg][lane] = n;
+  __syncthreads();
+  int run = 0;
+  for (int s = 0; s < seg; s++) run += part[s][lane];
+  if (!live) return;
+  if (BITS && per <= 4) {                               // (all in registers)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int w = 2 * (p0 + i);
+      if (w >= w1) break;
+      prefix[(size_t)w * Skv + key] = (unsigned)run;
+      run += __popc(lo[i]);
+      if (w + 1 < w1) prefix[(size_t)(w + 1) * Skv + key] = (unsigned)run;
+      run += __popc(hi[i]);
+    }
+  } else {
+    for (int w0 = 2 * p0; w0 < w1; w0 += 8) {
+      unsigned b[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) b[i] = bits[(size_t)min(w0 + i, w1 - 1) * Skv];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        if (w0 + i >= w1) break;
+        prefix[(size_t)(w0 + i) * Skv + key] = (unsigned)run;
+        run += __popc(b[i]);
+      }
+    }
+  }
+  if (seg == 15) count[key] = run;
+}
+
+// Keys whose bits and first rows the last kernel holds in LDS at a time
+constexpr int RANK_KEYS = 16384;
 // dst[ql][slot] = row of the pair in key-sorted order (-1 for invalid slots).  A workgroup takes the 32 queries of a word, or
 // a part of them (blockIdx.y) where there are few words, and has the word's bits and first rows of `range` keys at a time in
 // LDS, where the lookups by id go: from memory they were two dependent random reads of 4 bytes per pair (8192 queries x 2048 slots
-// 0.165 ms; 32768 x 2048 1.29 ms).  With `units` the ids are the lists of qmap_unit_kernel, and the pairs of a unit are its first query's.
+// 0.165 ms; 32768 x 2048 1.29 ms).  With `units` the ids are the lists of qmap_unit_kernel, and the pairs of a unit are its first
+// query's; workgroups behind the others clear marks.
+// start[key], the exclusive prefix sums of count, every workgroup works out for itself under the loads of the bits (two barriers a range)
+// and one writes: in a kernel of its own between this one and the counts it was a launch of one workgroup.
 static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict__ ids, int row0, int q0, int cnt, int K, int Skv, int q_start,
                                                            const unsigned* __restrict__ bitmap, const unsigned* __restrict__ prefix,
-                                                           const int* __restrict__ start, int range, int* __restrict__ dst,
-                                                           const int* __restrict__ units, int G) {
+                                                           const int* __restrict__ count, int* __restrict__ start, int range,
+                                                           int* __restrict__ dst, int words, const int* __restrict__ units, int G, Marks marks) {
   extern __shared__ uint2 tab[];             // {first row of the word's queries, bits}
-  const int w = blockIdx.x, share = 32 / gridDim.y;
+  constexpr int ROUNDS = RANK_KEYS / 1024;
+  __shared__ int sums[16 * ROUNDS + 1];      // counts of 64 keys, then of all keys before them; of all keys up to the range's end
+  const int w = blockIdx.x;
+  if (w >= words) { clear_marks(marks, (w - words) * (int)gridDim.y + (int)blockIdx.y); return; }
+  const bool writes = w == 0 && blockIdx.y == 0;
+  const int share = 32 / gridDim.y;
   const int q_lo = 32 * w + blockIdx.y * share, q_hi = min(q_lo + share, cnt);
   const int sub = threadIdx.x >> 8, lane = threadIdx.x & 255;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wl = threadIdx.x & 63;
+  int before = 0;                            // pairs of the ranges before
   for (int k0 = 0; k0 < Skv; k0 += range) {
-    const int nk = min(range, Skv - k0);
+    const int nk = min(range, Skv - k0), rounds = (nk + 1023) / 1024;
     if (k0) __syncthreads();
-    for (int k = threadIdx.x; k < nk; k += 1024) {
-      const size_t e = (size_t)w * Skv + k0 + k;
-      tab[k] = make_uint2((unsigned)start[k0 + k] + prefix[e], bitmap[e]);
+    for (int r0 = 0; r0 < rounds; r0 += 4) {
+      int c[4], inc[4];
+      uint2 e[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int k = min(1024 * (r0 + i) + (int)threadIdx.x, nk - 1);
+        c[i] = count[k0 + k];
+        e[i] = make_uint2(prefix[(size_t)w * Skv + k0 + k], bitmap[(size_t)w * Skv + k0 + k]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        c[i] = 1024 * (r0 + i) + (int)threadIdx.x < nk ? c[i] : 0;
+        inc[i] = wave_sums(c[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int k = 1024 * (r0 + i) + threadIdx.x;
+        if (k < nk) tab[k] = make_uint2(e[i].x + (unsigned)(inc[i] - c[i]), e[i].y);
+        if (wl == 63 && r0 + i < rounds) sums[16 * (r0 + i) + wave] = inc[i];
+      }
     }
     __syncthreads();
+    if (wave == 0) {
+      int c[4], all = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) { c[i] = 4 * wl + i < 16 * rounds ? sums[4 * wl + i] : 0; all += c[i]; }
+      int sum = before + wave_sums(all) - all;
+#pragma unroll
+      for (int i = 0; i < 4; i++) { if (4 * wl + i < 16 * rounds) sums[4 * wl + i] = sum; sum += c[i]; }
+      if (wl == 63) sums[16 * ROUNDS] = sum;
+    }
+    static_assert(16 * ROUNDS == 4 * 64, "one wave has the sums of a range");
+    __syncthreads();
+    before = sums[16 * ROUNDS];
+    if (writes)                              // (the first word has no queries before it)
+      for (int k = threadIdx.x; k < nk; k += 1024) start[k0 + k] = (int)tab[k].x + sums[k >> 6];
     for (int ql = q_lo + sub; ql < q_hi; ql += 4) {
       const int owner = units && units[ql / G] ? ql / G * G : ql;
       const unsigned below = (1u << (owner & 31)) - 1u;
@@ -435,7 +536,7 @@ static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict
           const int k = id - k0;
           if (ok && k >= 0 && k < nk) {
             const uint2 e = tab[k];
-            dst[(size_t)ql * K + t0 + i * 256] = (int)e.x + __popc(e.y & below);
+            dst[(size_t)ql * K + t0 + i * 256] = (int)e.x + sums[k >> 6] + __popc(e.y & below);
           } else if (!ok && k0 == 0) {
             dst[(size_t)ql * K + t0 + i * 256] = -1;
           }
@@ -443,68 +544,81 @@ static __global__ __launch_bounds__(1024) void rank_kernel(const int* __restrict
       }
     }
   }
+  if (writes && threadIdx.x == 0) start[Skv] = before;
 }
 
-// Launches the five kernels above for queries [q0, q0 + cnt).  A slot counts when its id v is in
+// Launches the kernels above for queries [q0, q0 + cnt).  A slot counts when its id v is in
 // [0, Skv) and v <= q_start + (query index); pass a huge q_start to accept every id in range.
 // With `sorted` ([cnt][K] ints) the first kernel also writes every query's valid ids in ascending
 // order (-1 after them) and dst refers to the slots of that list: a caller that is free to choose
 // its slot order uses the list instead of ids, which makes concurrently running queries gather
 // neighbouring key rows at the same time (the rows then hit in the L2 of the XCD).
-// The prefix buffer doubles as the scratch of step (1) (cnt * ceil(Skv / 32) words; it is rewritten by
-// the prefix pass afterwards): size it with prefix_words().
+// qmap (cnt * ceil(Skv / 32) words) lies in `room`, memory of the caller that is free until the order is made, where that is large enough:
+// then one kernel makes the bitmap and counts.  Else it lies in the prefix buffer, which the prefixes are written over afterwards: size that
+// with prefix_words().
+struct Room { void* at; size_t bytes; };
+inline unsigned* qmap_place(const Room& room, unsigned* prefix, int cnt, int Wk) {
+  return (size_t)cnt * Wk * 4 <= room.bytes ? (unsigned*)room.at : prefix;
+}
 inline size_t prefix_words(int chunk, int Skv) {
   const size_t W = (size_t)(chunk + 31) / 32, Wk = (size_t)(Skv + 31) / 32;
   return (size_t)Skv * W > (size_t)chunk * Wk ? (size_t)Skv * W : (size_t)chunk * Wk;
 }
 // The first kernel keeps one bit per key in LDS: the largest key count the builder takes
 constexpr int MAX_KEYS = 150 * 1024 * 8;
-// Keys whose bits and first rows the last kernel holds in LDS at a time
-constexpr int RANK_KEYS = 16384;
 // LDS of the first kernel with the sorted list: bitmap and prefix counts over all keys plus the list
 inline bool sorted_list_fits(int Skv, int K) {
   return (size_t)((Skv + 31) / 32) * 8 + (size_t)K * 4 <= (size_t)150 * 1024;
 }
 // dup_flag: one int the caller has cleared (clear_flag) before the first block of queries of a call.
 inline void clear_flag(int* dup_flag, hipStream_t st) { zero_u32_kernel<<<dim3(1), dim3(64), 0, st>>>((unsigned*)dup_flag, 1); }
-inline void build_ranks(const int* lists, int row0, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
-                        int* count, int* start, int* dst, int W, const int* units, int G, hipStream_t st, const int* flags = nullptr,
-                        uint4* marks = nullptr, size_t n_marks = 0, int* work = nullptr) {
-  const int Wk = (Skv + 31) / 32;
+inline void build_ranks(const int* lists, int row0, int q0, int cnt, int K, int Skv, int q_start, const unsigned* qmap, unsigned* bitmap,
+                        unsigned* prefix, int* count, int* start, int* dst, int W, WorkList list, hipStream_t st, const int* flags = nullptr,
+                        uint4* marks = nullptr, size_t n_marks = 0) {
+  // Two kernels; they are short, so their number and the trips to memory in each are what they cost.  us in kernels as four (bits, counts,
+  // one workgroup's scan, rows) / as two, a launch each besides: 2077 queries x 512 slots in pairs 26.3 / 21.5, 3072 x 640 32.1 / 23.9, 8192 x 2048
+  // by themselves 72 / 52.  (The work list, in one pass over the groups instead of three, beside the counts or the rows: the same.)
+  const int Wk = (Skv + 31) / 32, per_xcd = ((Skv + 63) / 64 + 7) / 8;
   // every word of the bitmap is written (zeros beyond the last query), so no clearing pass is needed
-  bm_transpose_kernel<<<dim3((W + 7) / 8, Wk), dim3(256), 0, st>>>(prefix, cnt, Skv, Wk, bitmap, W);
-  const int clearing = (int)((n_marks + 4095) / 4096 < 512 ? (n_marks + 4095) / 4096 : 512);
-  bm_prefix_kernel<<<dim3((Skv + 63) / 64 + clearing), dim3(1024), 0, st>>>(bitmap, prefix, count, Skv, W, flags, marks, n_marks);
-  key_scan_kernel<<<dim3(units ? 2 : 1), dim3(1024), 0, st>>>(count, start, Skv, WorkList{units, cnt, G, work});
+  const int words = (cnt + 31) / 32, parts = words >= 256 ? 1 : words >= 128 ? 2 : words >= 64 ? 4 : 8;
+  const size_t half = n_marks / 2, rest = n_marks - half, each = (rest + 4095) / 4096 < 256 ? (rest + 4095) / 4096 : 256;
+  const Marks first{flags, marks, half, (int)each}, second{flags, marks + half, rest, (int)(each + parts - 1) / parts * parts};
+  if (qmap != prefix) {
+    key_bits_kernel<true, true><<<dim3(8 * per_xcd + first.blocks + (list.units ? 1 : 0)), dim3(1024), 0, st>>>(qmap, cnt, Skv, Wk, bitmap, prefix, count, W, per_xcd, list, first);
+  } else {
+    key_bits_kernel<true, false><<<dim3(8 * per_xcd), dim3(1024), 0, st>>>(qmap, cnt, Skv, Wk, bitmap, prefix, count, W, per_xcd, list, first);
+    key_bits_kernel<false, true><<<dim3(8 * per_xcd + first.blocks + (list.units ? 1 : 0)), dim3(1024), 0, st>>>(qmap, cnt, Skv, Wk, bitmap, prefix, count, W, per_xcd, list, first);
+  }
   const int range = Skv < RANK_KEYS ? Skv : RANK_KEYS;
   if (range * 8 > 48 * 1024) (void)dsa_reserve_lds((const void*)rank_kernel, (size_t)range * 8);
-  const int words = (cnt + 31) / 32, parts = words >= 256 ? 1 : words >= 128 ? 2 : words >= 64 ? 4 : 8;
-  rank_kernel<<<dim3(words, parts), dim3(1024), (size_t)range * 8, st>>>(lists, row0, q0, cnt, K, Skv, q_start, bitmap, prefix, start, range, dst,
-                                                                         units, G);
+  rank_kernel<<<dim3(words + second.blocks / parts, parts), dim3(1024), (size_t)range * 8, st>>>(
+      lists, row0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, range, dst, words, list.units, list.G, second);
 }
 inline void build(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix,
-                  int* count, int* start, int* dst, int W, hipStream_t st, int* dup_flag, int* sorted = nullptr) {
+                  int* count, int* start, int* dst, int W, Room room, hipStream_t st, int* dup_flag, int* sorted = nullptr) {
   const int Wk = (Skv + 31) / 32;
   const size_t lds = (size_t)Wk * 4 * (sorted ? 2 : 1) + (sorted ? (size_t)K * 4 : 0);
   if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)qmap_kernel, lds);
-  qmap_kernel<<<dim3(cnt), dim3(256), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag);
+  unsigned* qmap = qmap_place(room, prefix, cnt, Wk);
+  qmap_kernel<<<dim3(cnt), dim3(256), lds, st>>>(ids, q0, cnt, K, Skv, q_start, qmap, Wk, sorted, dup_flag);
   // with `sorted` (rows of the block's queries, [cnt][K]) the ranks are those of the sorted slots
-  build_ranks(sorted ? sorted : ids, sorted ? 0 : q0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, nullptr, 1, st);
+  build_ranks(sorted ? sorted : ids, sorted ? 0 : q0, q0, cnt, K, Skv, q_start, qmap, bitmap, prefix, count, start, dst, W, WorkList{nullptr, cnt, 1, nullptr}, st);
 }
 // LDS of qmap_unit_kernel
 inline size_t unit_lists_lds(int G, int Skv, int K) { return (size_t)unit_words((Skv + 31) / 32) * 4 * (G + G / 2) + (size_t)G * K * 4; }
 // build with the sorted lists, for groups of G (2 or 4) queries that may be units; 16 bytes of `marks` for every row (cnt K at most) are
 // cleared if there are any.  work: cnt + 2 ints
 inline void build_units(const int* ids, int q0, int cnt, int K, int Skv, int q_start, unsigned* bitmap, unsigned* prefix, int* count, int* start,
-                        int* dst, int W, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
+                        int* dst, int W, Room room, hipStream_t st, int* dup_flag, int* sorted, int G, const unsigned* bad, int* units, int max_slots,
                         UnitCost cost, uint4* marks, int* work) {
   const int Wk = (Skv + 31) / 32;
   const size_t lds = unit_lists_lds(G, Skv, K);
   const bool small = G * K <= 2048 && Wk <= 1024;      // (one round of ids for 256 threads, and then twice the workgroups on a compute unit)
   auto kernel = G == 2 ? (small ? qmap_unit_kernel<2, 256> : qmap_unit_kernel<2, 512>) : small ? qmap_unit_kernel<4, 256> : qmap_unit_kernel<4, 512>;
   if (lds > 48 * 1024) (void)dsa_reserve_lds((const void*)kernel, lds);
-  kernel<<<dim3((cnt + G - 1) / G), dim3(small ? 256 : 512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, prefix, Wk, sorted, dup_flag, bad, units, max_slots, cost);
-  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, bitmap, prefix, count, start, dst, W, units, G, st, dup_flag, marks, (size_t)cnt * K, work);
+  unsigned* qmap = qmap_place(room, prefix, cnt, Wk);
+  kernel<<<dim3((cnt + G - 1) / G), dim3(small ? 256 : 512), lds, st>>>(ids, q0, cnt, K, Skv, q_start, qmap, Wk, sorted, dup_flag, bad, units, max_slots, cost);
+  build_ranks(sorted, 0, q0, cnt, K, Skv, q_start, qmap, bitmap, prefix, count, start, dst, W, WorkList{units, cnt, G, work}, st, dup_flag, marks, (size_t)cnt * K);
 }
 
 }  // namespace order
