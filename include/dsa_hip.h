@@ -375,8 +375,8 @@ int dsa_sparse_mla_bwd_groups(int S, int H, int Skv, int K, size_t workspace_byt
  */
 int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S,
                         int K, float eps, float* row_loss, float* grad, void* stream);
-/* The same with every gradient times factor, rounded once more: what dsa_indexer_kl_scale makes of it with *g = 1. */
-int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S,
+/* The same with every gradient times factor, rounded once more: what dsa_indexer_kl_scale makes of it with *g = 1; target_bf16: target [S, K] bf16. */
+int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const void* target, int target_bf16, int64_t ld_t, int S,
                                int K, float eps, float factor, float* row_loss, float* grad, void* stream);
 /* *out = factor * the sum of row_loss [S]; and out = grad * (*g * factor), n elements: the two ways through the scaled sum of the rows. */
 int dsa_indexer_kl_total(const float* row_loss, int S, float factor, float* out, void* stream);
@@ -391,6 +391,9 @@ int dsa_indexer_kl_scale(const float* grad, const float* g, float factor, float*
  */
 int dsa_attn_dist(const void* p_out, int p_out_f32, int S, int H, int K, int64_t ld_s,
                   int64_t ld_h, float sm_scale, float* target, void* stream);
+/* The same; target_bf16: target [S, K] bf16, rounded from the means. */
+int dsa_attn_dist_as(const void* p_out, int p_out_f32, int S, int H, int K, int64_t ld_s,
+                     int64_t ld_h, float sm_scale, void* target, int target_bf16, void* stream);
 
 /*
  * The same distribution without materialised logits: recomputed from q, kv, ids and the forward's

@@ -59,10 +59,11 @@ SIGNATURES = {
     "dsa_sparse_mla_bwd_groups": (_i, [_i, _i, _i, _i, _sz, _vp]),
     "dsa_indexer_kl_total": (_i, [_vp, _i, _f, _vp, _vp]),
     "dsa_indexer_kl_scale": (_i, [_vp, _vp, _f, _vp, _i64, _vp]),
-    "dsa_indexer_kl_loss_scaled": (_i, [_vp, _i64, _vp, _i64, _i, _i, _f, _f, _vp, _vp, _vp]),
+    "dsa_indexer_kl_loss_scaled": (_i, [_vp, _i64, _vp, _i, _i64, _i, _i, _f, _f, _vp, _vp, _vp]),
     "dsa_indexer_kl_loss": (_i, [_vp, _i64, _vp, _i64, _i, _i, _f, _vp, _vp, _vp]),
     "dsa_sparse_mla_fwd_dist": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _sz, _vp]),
     "dsa_attn_dist": (_i, [_vp, _i, _i, _i, _i, _i64, _i64, _f, _vp, _vp]),
+    "dsa_attn_dist_as": (_i, [_vp, _i, _i, _i, _i, _i64, _i64, _f, _vp, _i, _vp]),
     "dsa_attn_dist_qk": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]),
     "dsa_mla_absorb": (_i, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _i, _i, _i, _i, _vp]),
     "dsa_absorb_rope_query": (_i, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp]),

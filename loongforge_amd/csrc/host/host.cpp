@@ -668,28 +668,38 @@ py::object mla_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& out_, cons
   return py::make_tuple(dq, dkv);
 }
 
-py::object attn_dist(const Tensor& p_, double sm_scale, bool force) {
-  PLAIN_OR_NONE(p_);
+// `as_input`: in the logits' type, rounded by the kernel
+Tensor attn_dist_of(const Tensor& p_, double sm_scale, bool as_input) {
   need_gpus(p_);
   REQUIRE(p_.dim() == 3 && (p_.scalar_type() == at::kBFloat16 || p_.scalar_type() == at::kFloat), "attn_dist expects p_out [S,H,K] in bf16 or fp32");
   const Tensor p = p_.stride(2) == 1 ? p_ : p_.contiguous();
   const int64_t S = p.size(0), H = p.size(1), K = p.size(2);
   Call call(p);
-  Tensor target = make({S, K}, at::kFloat, p);
-  run("dsa_attn_dist", dsa_attn_dist, p.const_data_ptr(), p.scalar_type() == at::kFloat, (int)S, (int)H, (int)K, S > 0 ? p.stride(0) : H * K, p.stride(1), (float)sm_scale, (float*)target.data_ptr(), call.stream);
-  return py::cast(target);
+  const auto type = as_input ? p.scalar_type() : at::kFloat;
+  Tensor target = make({S, K}, type, p);
+  run("dsa_attn_dist", dsa_attn_dist_as, p.const_data_ptr(), p.scalar_type() == at::kFloat, (int)S, (int)H, (int)K, S > 0 ? p.stride(0) : H * K, p.stride(1), (float)sm_scale, target.data_ptr(), type == at::kBFloat16, call.stream);
+  return target;
+}
+
+py::object attn_dist(const Tensor& p, double sm_scale, bool force) {
+  PLAIN_OR_NONE(p);
+  return py::cast(attn_dist_of(p, sm_scale, false));
+}
+py::object attn_dist_as_input(const Tensor& p, double sm_scale, bool force) {
+  PLAIN_OR_NONE(p);
+  return py::cast(attn_dist_of(p, sm_scale, true));
 }
 
 std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, double eps, double factor) {
   need_gpus(scores_, target_);
   REQUIRE(scores_.dim() == 2 && target_.sizes() == scores_.sizes(), "indexer_kl_loss expects scores and target of one shape [S, K]");
   const int64_t S = scores_.size(0), K = scores_.size(1);
-  Tensor scores = scores_.to(at::kFloat), target = target_.to(at::kFloat);
+  Tensor scores = scores_.to(at::kFloat), target = target_.scalar_type() == at::kBFloat16 ? target_ : target_.to(at::kFloat);
   if (scores.stride(1) != 1) scores = scores.contiguous();
   if (target.stride(1) != 1) target = target.contiguous();
   Call call(scores);
   Tensor row_loss = make({S}, at::kFloat, scores), grad = make({S, K}, at::kFloat, scores);
-  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss_scaled, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, (const float*)target.const_data_ptr(), S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float)factor, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
+  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss_scaled, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, target.const_data_ptr(), target.scalar_type() == at::kBFloat16, S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float)factor, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
   return {row_loss, grad};
 }
 
@@ -881,6 +891,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   DEF(pad_heads);
   DEF(mla_bwd);
   DEF(attn_dist);
+  DEF(attn_dist_as_input);
   DEF(kl_loss);
   DEF(kl_total);
   DEF(kl_loss_total);

@@ -7,7 +7,8 @@
 // One workgroup per row; the row's scores and targets stay in registers between the three reductions
 // (maximum, normaliser, loss and sum_j w_j pred_j), so each array crosses HBM once and the gradient is
 // written once.  A padded slot (score -inf, target 0) has pred = 0, contributes eps (log eps - log eps) = 0
-// to the loss and gets gradient 0.  HBM-bound: 12 bytes per slot.
+// to the loss and gets gradient 0.  HBM-bound: 12 bytes per slot, 10 with targets in bf16, which are read as they are (3072 x 512: 7.8 us
+// behind a pass of 6.1 that makes them 32 bits wide, 8.3 us by itself).
 #include "dsa_common.h"
 
 namespace {
@@ -60,20 +61,31 @@ __device__ __forceinline__ float pairs_sum(const float (&v)[N]) {
   return a;
 }
 
+// a target slot as it is or from bf16
+__device__ __forceinline__ float slot(float x) { return x; }
+__device__ __forceinline__ float slot(unsigned short x) { return bf16_bits_to_f32(x); }
+
 // thread tid of the NT that share a row has its slots tid, tid + NT, ..: K <= NE * NT
-template <int NE, int NT, class Row>
+template <int NE, int NT, class T, class Row>
 __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, const float* __restrict__ scores, int64_t ld_s,
-                                       const float* __restrict__ target, int64_t ld_t, int K, float eps, float factor, float* __restrict__ row_loss,
+                                       const T* __restrict__ target, int64_t ld_t, int K, float eps, float factor, float* __restrict__ row_loss,
                                        float* __restrict__ grad) {
   const float* sp = scores + row * ld_s;
-  const float* tp = target + row * ld_t;
+  const T* tp = target + row * ld_t;
   float s[NE], u[NE];
+  T raw[NE];
   float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NE; i++) {             // (no branch between the loads, and nothing that waits for one of them)
+    const int t = min(tid + NT * i, K - 1);
+    s[i] = sp[t];
+    raw[i] = tp[t];
+  }
 #pragma unroll
   for (int i = 0; i < NE; i++) {
     const int t = tid + NT * i;
-    s[i] = t < K ? sp[t] : -INFINITY;
-    u[i] = (t < K ? tp[t] : 0.f) + eps;
+    s[i] = t < K ? s[i] : -INFINITY;
+    u[i] = (t < K ? slot(raw[i]) : 0.f) + eps;
     mx = fmaxf(mx, s[i]);
   }
   mx = over.max(mx);
@@ -116,9 +128,9 @@ __device__ __forceinline__ void kl_row(const Row& over, int tid, int64_t row, co
   if (tid == 0) row_loss[row] = loss;
 }
 
-template <int NE>
+template <int NE, class T>
 __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict__ scores, int64_t ld_s,
-                                                        const float* __restrict__ target, int64_t ld_t, int K, float eps, float factor,
+                                                        const T* __restrict__ target, int64_t ld_t, int K, float eps, float factor,
                                                         float* __restrict__ row_loss, float* __restrict__ grad) {
   __shared__ float scratch[8];
   kl_row<NE, BLOCK>(BlockRow{scratch}, threadIdx.x, blockIdx.x, scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
@@ -127,8 +139,8 @@ __global__ __launch_bounds__(BLOCK) void kl_loss_kernel(const float* __restrict_
 // Up to 512 slots: a row to a wave.  A workgroup to a row spent its time in three reductions with barriers and on eight slots a thread of
 // which one or two were there (7951 x 256 slots 30.4 us and 7.6 so, 2077 x 512 11.3 and 6.1, 300 x 256 4.8 and 3.3; beyond, four
 // slots a thread where that is enough: 4000 x 1024 18.8 and 13.8).
-template <int NE>
-__global__ __launch_bounds__(BLOCK) void kl_loss_wave_kernel(const float* __restrict__ scores, int64_t ld_s, const float* __restrict__ target,
+template <int NE, class T>
+__global__ __launch_bounds__(BLOCK) void kl_loss_wave_kernel(const float* __restrict__ scores, int64_t ld_s, const T* __restrict__ target,
                                                              int64_t ld_t, int S, int K, float eps, float factor, float* __restrict__ row_loss,
                                                              float* __restrict__ grad) {
   const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6));
@@ -174,6 +186,17 @@ __global__ __launch_bounds__(256) void kl_scale_kernel(const f32x4* __restrict__
   if (blockIdx.x == 0 && (int64_t)threadIdx.x < n % 4) ((float*)y)[4 * n4 + threadIdx.x] = ((const float*)x)[4 * n4 + threadIdx.x] * f;
 }
 
+template <class T>
+void launch_rows(const float* scores, int64_t ld_s, const T* target, int64_t ld_t, int S, int K, float eps, float factor, float* row_loss, float* grad,
+                 hipStream_t st) {
+  const dim3 waves(dsa_cdiv(S, BLOCK / 64));
+  if (K <= 256) kl_loss_wave_kernel<4, T><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
+  else if (K <= 512) kl_loss_wave_kernel<8, T><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
+  else if (K <= 4 * BLOCK) kl_loss_kernel<4, T><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+  else if (K <= 8 * BLOCK) kl_loss_kernel<8, T><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+  else kl_loss_kernel<32, T><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+}
+
 }  // namespace
 
 extern "C" int dsa_indexer_kl_total(const float* row_loss, int S, float factor, float* out, void* stream) {
@@ -196,22 +219,17 @@ extern "C" int dsa_indexer_kl_scale(const float* grad, const float* g, float fac
 
 extern "C" int dsa_indexer_kl_loss(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S, int K,
                                    float eps, float* row_loss, float* grad, void* stream) {
-  return dsa_indexer_kl_loss_scaled(scores, ld_s, target, ld_t, S, K, eps, 1.0f, row_loss, grad, stream);
+  return dsa_indexer_kl_loss_scaled(scores, ld_s, target, 0, ld_t, S, K, eps, 1.0f, row_loss, grad, stream);
 }
 
-extern "C" int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const float* target, int64_t ld_t, int S, int K,
+extern "C" int dsa_indexer_kl_loss_scaled(const float* scores, int64_t ld_s, const void* target, int target_bf16, int64_t ld_t, int S, int K,
                                           float eps, float factor, float* row_loss, float* grad, void* stream) {
   DSA_REQUIRE(S >= 0 && K > 0 && K <= 32 * BLOCK, "dsa_indexer_kl_loss: K must lie in [1, %d], got %d", 32 * BLOCK, K);
   DSA_REQUIRE(ld_s >= K && ld_t >= K, "dsa_indexer_kl_loss: row strides %lld / %lld below K = %d", (long long)ld_s,
               (long long)ld_t, K);
   if (S == 0) return DSA_OK;
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 waves(dsa_cdiv(S, BLOCK / 64));
-  if (K <= 256) kl_loss_wave_kernel<4><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
-  else if (K <= 512) kl_loss_wave_kernel<8><<<waves, dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, S, K, eps, factor, row_loss, grad);
-  else if (K <= 4 * BLOCK) kl_loss_kernel<4><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
-  else if (K <= 8 * BLOCK) kl_loss_kernel<8><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
-  else kl_loss_kernel<32><<<dim3(S), dim3(BLOCK), 0, st>>>(scores, ld_s, target, ld_t, K, eps, factor, row_loss, grad);
+  if (target_bf16) launch_rows(scores, ld_s, (const unsigned short*)target, ld_t, S, K, eps, factor, row_loss, grad, (hipStream_t)stream);
+  else launch_rows(scores, ld_s, (const float*)target, ld_t, S, K, eps, factor, row_loss, grad, (hipStream_t)stream);
   DSA_CHECK_LAUNCH("dsa_indexer_kl_loss");
   return DSA_OK;
 }

@@ -636,7 +636,8 @@ __global__ __launch_bounds__(256, 1) void mla_fwd_kernel(FwdArgs a) {
       }
       return;
     }
-  } else if (head_ok && !again) {    const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
+  } else if (head_ok && !again) {
+    const Final fin = finish_head(m_ref, l_tot, a.sink ? a.sink + h : nullptr);
     if (stats) a.lse[(size_t)qi * H + h] = fin.lse;
     unsigned short* op = (unsigned short*)a.out + ((size_t)qi * H + h) * DV + 32 * dt0 + 8 * g;
     finish_mine([&](const f32x16& t, int dt) { store_out(t, fin.inv, op + 32 * dt); });

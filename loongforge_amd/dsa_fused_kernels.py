@@ -27,7 +27,7 @@ def triton_attn_dist(p_out: torch.Tensor, sm_scale) -> torch.Tensor:
     """
     if p_out.ndim != 3:
         raise ValueError("p_out must be (s_q, h_q, topk)")
-    return ops.attn_dist(p_out, float(sm_scale)).to(p_out.dtype)
+    return ops.attn_dist_as_input(p_out, float(sm_scale))
 
 
 def padded_flashinfer_topk(logits, topk, sk, *, sorted=True):

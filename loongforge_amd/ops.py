@@ -614,6 +614,11 @@ def attn_dist(p_out, sm_scale: float):
     return _direct("attn_dist", _attn_dist_op, p_out, float(sm_scale))
 
 
+def attn_dist_as_input(p_out, sm_scale: float):
+    """:func:`attn_dist` in ``p_out.dtype``."""
+    return _direct("attn_dist_as_input", lambda *a: _attn_dist_op(*a).to(p_out.dtype), p_out, float(sm_scale))
+
+
 @torch.library.custom_op("dsa::attn_dist_qk", mutates_args=())
 def _attn_dist_qk_op(q: torch.Tensor, kv: torch.Tensor, ids: torch.Tensor, lse: torch.Tensor, q_start: int,
                      sm_scale: float, heads_in_mean: int) -> torch.Tensor:

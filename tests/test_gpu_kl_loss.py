@@ -107,3 +107,24 @@ def test_sum_of_the_rows_losses_is_rounded_once(gpu, S, step):
         want = x.double().sum()
         got = ops._native().kl_total(x.to(gpu), 1.0).cpu()
         assert got == want.float() or abs(got.double() - want) <= (2.0 ** -24 + S * 2.0 ** -52) * want
+
+
+@pytest.mark.parametrize("S,H,K", [(1, 4, 1), (5, 3, 200), (9, 16, 256), (7, 16, 264), (33, 64, 512), (6, 8, 1000), (5, 32, 2048), (3, 2, 2500)])
+def test_distribution_and_targets_in_bf16(gpu, S, H, K):
+    """The kernels that round the distribution to the logits' bf16 and that read bf16 targets have the bits of the conversions beside
+    them, with rows at a stride too."""
+    from loongforge_amd import ops
+    from loongforge_amd.dsa_fused_kernels import triton_attn_dist
+
+    gen = torch.Generator().manual_seed(K)
+    p = torch.randn(S, H, K, generator=gen).to(torch.bfloat16)
+    p[:, :, K // 2:][torch.rand(S, H, K - K // 2, generator=gen) < 0.1] = float("-inf")
+    p = p.to(gpu)
+    target = triton_attn_dist(p, 0.3)
+    assert target.dtype == torch.bfloat16 and torch.equal(target, ops.attn_dist(p, 0.3).to(torch.bfloat16))
+    assert triton_attn_dist(p.float(), 0.3).dtype == torch.float32
+    scores = torch.randn(S, K, generator=gen).to(gpu)
+    wide = torch.nn.functional.pad(target, (0, 3))
+    for t in (target, wide[:, :K]):
+        got, want = ops._kl_loss_op(scores, t, 1e-10), ops._kl_loss_op(scores, t.float(), 1e-10)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
