@@ -288,7 +288,8 @@ int dsa_sparse_mla_fwd_ex(const void* q, const void* kv, const int32_t* ids, int
 /*
  * The same with a workspace (16-byte aligned), which lets a call with few queries spread the slots of a query over
  * several workgroups: dsa_sparse_mla_fwd_workspace_bytes is what the call can use (0: it would not spread them).
- * With less, every query's slots stay in one workgroup.
+ * With less, every query's slots stay in one workgroup.  What the workspace holds before the call does not matter; two calls
+ * that may run at the same time need one each.
  */
 size_t dsa_sparse_mla_fwd_workspace_bytes(int S, int H, int Skv, int K);
 int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* ids, int S, int H, int Skv,
