@@ -84,6 +84,11 @@ __device__ __forceinline__ uint4 weighted_query(unsigned q_lds, const float* w_s
 }
 // The mask [r > 0] of an accumulator of scores (times 2^20: at least 4 where positive, r is a multiple of 2^-18) as the bf16 operand of
 // the next product, each entry 0 or 2^-7: the half-precision 1.0 read as bf16, a conversion and a packed clamp for two.
+__device__ __forceinline__ unsigned mask_pair(float lo, float hi) {
+  unsigned pk = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+  asm("v_pk_max_f16 %0, %0, %0 clamp" : "+v"(pk));
+  return pk;
+}
 template <int NHT>
 __device__ __forceinline__ void score_masks(const f32x16 (&acc)[NHT], bf16x8 (&mk)[2 * NHT]) {
 #pragma unroll
@@ -92,10 +97,7 @@ __device__ __forceinline__ void score_masks(const f32x16 (&acc)[NHT], bf16x8 (&m
     for (int s = 0; s < 2; s++) {
       unsigned pk[4];
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        pk[e] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(acc[t][8 * s + 2 * e], acc[t][8 * s + 2 * e + 1]));
-        asm("v_pk_max_f16 %0, %0, %0 clamp" : "+v"(pk[e]));
-      }
+      for (int e = 0; e < 4; e++) pk[e] = mask_pair(acc[t][8 * s + 2 * e], acc[t][8 * s + 2 * e + 1]);
       mk[2 * t + s] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
     }
 }
@@ -842,9 +844,11 @@ __device__ __forceinline__ void dma4(unsigned lds_base, unsigned goff, const voi
                :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
 }
 
-// 0.81 ms at 8192 queries x 2048 slots x 64 heads (34 M pairs of query and key in the tiles): by the counters the matrix pipe is 50 % busy
-// and LDS 26 %.  With the sums behind all products of a query instead of between them, and a branch per sum for operands that are not
-// finite, 0.877; without a query's scores under the products of the one before, 0.965.
+// 1.57 M cycles at 8192 queries x 2048 slots x 64 heads (34 M pairs of query and key in the tiles; 0.81 - 0.85 ms): by the counters the matrix
+// pipe is 52 % busy and LDS 27 %.  A wave waits for operands that it asks for one d-tile ahead, and there are no registers for two.  With the
+// masks and a query's last sums by themselves instead of under products 1.65 M (inside the training pass 890 us and 849, 3072 x 512 of 768 keys
+// 66.5 and 64.2, 32 heads the same); with the sums behind all products of a query and a branch per sum for operands that are not finite 8 % more
+// than that, without a query's scores under the products of the one before another 10 %.
 // One workgroup of eight waves, 32 keys a wave: scores of the query's heads with the wave's keys on the columns, their masks, the rows
 // of the keys, times the pairs' factors into the sums.  Two queries a step; their operands and factors come into a ring of three steps
 // by transfers that the waves share out.
@@ -924,7 +928,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   look_up(2);
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16 sum[4], acc[NHT], racc[2];
-  bf16x8 mk[2 * NHT], qt[2][2 * NHT];
+  bf16x8 qt[2][2 * NHT];
+  unsigned __attribute__((ext_vector_type(4))) mk[2][2 * NHT];       // of the query in hand and of the next one, in turn
 #pragma unroll
   for (int dt = 0; dt < 4; dt++) sum[dt] = zero;
   auto read_query = [&](int t, unsigned ob, i32x8 (&aq)[2]) {
@@ -951,10 +956,16 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     read_query(t, ob, aq);
     scores(t, aq);
   }
-  score_masks<NHT>(acc, mk);
+#pragma unroll
+  for (int t = 0; t < NHT; t++)
+#pragma unroll
+    for (int j = 0; j < 8; j++) mk[0][2 * t + (j >> 2)][j & 3] = mask_pair(acc[t][2 * j], acc[t][2 * j + 1]);
   read_weighted(0, ob);
+  float before = __builtin_bit_cast(float, UNSELECTED);        // factor of the query whose last d-tile is still to be added
+  racc[1] = zero;
   // Scores and masks of the query behind the one in hand are made under the products of the latter (behind the last one: of what lies
-  // in the ring, unused).  FINITE: every operand of the chunk is; otherwise infinities and NaN stay with the keys that the query selected.
+  // in the ring, unused), and a query's last sums under the next one's first products.  FINITE: every operand of the chunk is; otherwise
+  // infinities and NaN stay with the keys that the query selected.
   auto sweep = [&](auto finite) {
     constexpr bool FINITE = decltype(finite)::value;
     int slot = 0;
@@ -972,35 +983,47 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
         const unsigned on = x == 0 ? ob + OPS : lds0 + (unsigned)(next_slot * STAGE + lane * 16);
         const float a = lds_read<float>(lds0 + (unsigned)(slot * STAGE + 2 * OPS + wave * 256 + x * 128 + r * 4));
-        const float a128 = a * 128.f;               // (the masks' entries are 2^-7)
+        // the products of a d-tile run while the one before it is added (the masks' entries are 2^-7)
+        auto add = [&](int dt, int e, float f) {
+          float v = racc[dt & 1][e];
+          if (!FINITE) v = __builtin_bit_cast(unsigned, f) == UNSELECTED ? 0.f : v;
+          sum[dt][e] = fmaf(f * 128.f, v, sum[dt][e]);
+        };
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int dt = 0; dt < 5; dt++) {            // the products of a d-tile run while the one before it is added
+        for (int dt = 0; dt < 4; dt++) {
           constexpr int STEP = 16 / (2 * NHT);
           i32x8 aq[2];
-          if (dt < 4) read_weighted((dt + 1) & 3, dt < 3 ? ob : on);
+          read_weighted((dt + 1) & 3, dt < 3 ? ob : on);
           if (dt < NHT) read_query(dt, on, aq);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int kk = 0; kk < 2 * NHT; kk++) {
-            if (dt < 4) racc[dt & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt[dt & 1][kk], mk[kk], kk ? racc[dt & 1] : zero, 0, 0, 0);
-            if (dt > 0) {
+            racc[dt & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt[dt & 1][kk], __builtin_bit_cast(bf16x8, mk[x][kk]), kk ? racc[dt & 1] : zero, 0, 0, 0);
 #pragma unroll
-              for (int e = STEP * kk; e < STEP * (kk + 1); e++) {
-                float v = racc[(dt - 1) & 1][e];
-                if (!FINITE) v = __builtin_bit_cast(unsigned, a) == UNSELECTED ? 0.f : v;
-                sum[dt - 1][e] = fmaf(a128, v, sum[dt - 1][e]);
+            for (int e = STEP * kk; e < STEP * (kk + 1); e++) add(dt > 0 ? dt - 1 : 3, e, dt > 0 ? a : before);
+            if (dt >= 2) {                          // (the scores were made by then)
+#pragma unroll
+              for (int i = 0; i < 2; i++) {
+                const int j = 4 * NHT * (dt - 2) + 2 * kk + i, t = j >> 3;
+                mk[x ^ 1][j >> 2][j & 3] = mask_pair(acc[t][2 * (j & 7)], acc[t][2 * (j & 7) + 1]);
               }
             }
             __builtin_amdgcn_sched_barrier(0);
           }
           if (dt < NHT) scores(dt, aq);
-          if (dt == 3) score_masks<NHT>(acc, mk);   // (the masks in hand have had their last use)
           __builtin_amdgcn_sched_barrier(0);
         }
+        before = a;
         ob = on;
       }
       slot = next_slot;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      float v = racc[1][e];
+      if (!FINITE) v = __builtin_bit_cast(unsigned, before) == UNSELECTED ? 0.f : v;
+      sum[3][e] = fmaf(before * 128.f, v, sum[3][e]);
     }
   };
   if (bad) sweep(std::false_type()); else sweep(std::true_type());
