@@ -99,6 +99,21 @@ __device__ __forceinline__ int spread_start(int i, int n, int round, int ramp) {
   if (j >= round * (step - 1)) return n - tail + round + j;
   return n - tail + j + j / (step - 1) + 1;
 }
+// Transfers from memory to LDS: each lane fetches 16 bytes at gbase + goff; the wave's 64 chunks land at lds_base + 16 * lane.
+// (m0 carries the LDS base; nothing else in these kernels uses m0.)  The transfer is counted by the vector-memory counter but invisible to
+// the compiler, which therefore never waits for it: callers wait with DSA_WAIT_VMCNT before a barrier.
+// gbase may come straight out of v_readfirstlane, and a memory instruction may read what a vector one wrote into scalar registers only five
+// wait states later, which the compiler sees to for its own loads alone.  A scalar move waits for the write by itself, and is also the wait
+// state between m0 and the transfer.
+#define DSA_LDS_TRANSFER(instruction, hint)                                                                                            \
+  unsigned long long base;                                                                                                             \
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\t" instruction " %2, %0" hint : "=&s"(base) : "s"(lds_base), "v"(goff), "s"(gbase) : "memory")
+__device__ __forceinline__ void dma16(unsigned lds_base, unsigned goff, const void* gbase) { DSA_LDS_TRANSFER("global_load_lds_dwordx4", ""); }
+// With the non-temporal hint, for what is read once: it then leaves the L2 to the key rows that neighbouring workgroups share.
+// Whole 128-byte lines by eight neighbouring lanes: a line that comes in by parts would be fetched for each.
+__device__ __forceinline__ void dma16_once(unsigned lds_base, unsigned goff, const void* gbase) { DSA_LDS_TRANSFER("global_load_lds_dwordx4", " nt"); }
+__device__ __forceinline__ void dma4(unsigned lds_base, unsigned goff, const void* gbase) { DSA_LDS_TRANSFER("global_load_lds_dword", ""); }
+#undef DSA_LDS_TRANSFER
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding).
 #define DSA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 0xf) | (((n) >> 4) << 14)) | (0x7 << 4) | (0xf << 8))
 

@@ -36,15 +36,6 @@ constexpr unsigned NOWHERE = 0x40000000u;   // a store offset behind any row, al
 
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-__device__ __forceinline__ void dma16(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
-}
-__device__ __forceinline__ void dma4(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
-}
-
 // max(x, 0) as one instruction, on the bit pattern (a negative float is a negative integer):
 // fmaxf would first quiet a possible signalling NaN with a second v_max, which doubles the cost
 // of the epilogue.

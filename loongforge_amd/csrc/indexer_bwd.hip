@@ -40,10 +40,6 @@ constexpr int WAVE_BYTES = 32 * D;      // fp8 key rows of a wave's share of a t
 constexpr int THREADS = 512;
 constexpr int RED_STRIDE = 132;         // floats per head row of the cross-wave reduction buffers
 
-__device__ __forceinline__ void dma16(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
-}
 // The 16-byte chunk c of a 128-byte row r sits in slot c ^ slot_xor(r): eight rows of one parity of any 16 consecutive ones
 // use eight different slots (row reads), and the eight rows of a transposing read four different pairs of slots per
 // parity: neither kind of read has a bank conflict.
@@ -837,11 +833,6 @@ __global__ __launch_bounds__(256) void indexer_scatter_kernel(const DenseArgs A)
   if (bad || dup) atomicOr(&flags_s, (bad ? QUERY_BAD : 0) | (dup ? QUERY_DUP : 0));
   __syncthreads();
   if (tid == 0) A.state[ql] = flags_s;
-}
-
-__device__ __forceinline__ void dma4(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
 }
 
 // 1.57 M cycles at 8192 queries x 2048 slots x 64 heads (34 M pairs of query and key in the tiles; 0.81 - 0.85 ms): by the counters the matrix

@@ -24,21 +24,6 @@ __device__ __forceinline__ int swz(int r) {
   return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r ^ (r >> 3)) & 1);
 }
 
-// Each lane fetches 16 bytes at gbase + goff; the wave's 64 chunks land at lds_base + 16*lane.
-// (m0 carries the LDS base; nothing else in these kernels uses m0.)  The transfer is counted by
-// the vector-memory counter but invisible to the compiler, which therefore never waits for it:
-// callers wait with DSA_WAIT_VMCNT before a barrier.
-__device__ __forceinline__ void dma16(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
-}
-// The same with the non-temporal hint, for what is read once: it then leaves the L2 to the key rows that neighbouring workgroups share.
-// Whole 128-byte lines by eight neighbouring lanes: a line that comes in by parts would be fetched for each.
-__device__ __forceinline__ void dma16_once(unsigned lds_base, unsigned goff, const void* gbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-               :: "s"(lds_base), "v"(goff), "s"(gbase) : "memory");
-}
-
 // A pointer that is the same for every lane, forced into scalar registers.
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* p) {
