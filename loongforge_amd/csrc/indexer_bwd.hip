@@ -56,6 +56,8 @@ __device__ __forceinline__ bf16x8 fp8_to_bf16(const i32x2& w) {
   }
   return o;
 }
+typedef _Float16 __attribute__((ext_vector_type(2))) f16x2;
+typedef unsigned short __attribute__((ext_vector_type(2))) u16x2;
 // LDS by 32-bit address: sums of a lane's offset, a tile's and a constant then stay in the read's own offset field
 template <typename T>
 __device__ __forceinline__ T lds_read(unsigned addr) { return *(__attribute__((address_space(3))) const T*)(uintptr_t)addr; }
@@ -80,10 +82,13 @@ __device__ __forceinline__ uint4 weighted_query(unsigned q_lds, const float* w_s
 }
 // The mask [r > 0] of an accumulator of scores (times 2^20: at least 4 where positive, r is a multiple of 2^-18) as the bf16 operand of
 // the next product, each entry 0 or 2^-7: the half-precision 1.0 read as bf16, a conversion and a packed clamp for two.
+// The clamp is written in C, so that the compiler knows a vector instruction in front of the product and keeps the wait states between.  Of a
+// conversion without another use it would become the conversion's own clamp, which does nothing.
 __device__ __forceinline__ unsigned mask_pair(float lo, float hi) {
-  unsigned pk = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(lo, hi));
-  asm("v_pk_max_f16 %0, %0, %0 clamp" : "+v"(pk));
-  return pk;
+  const auto pk = __builtin_amdgcn_cvt_pkrtz(lo, hi);
+  asm volatile("" :: "v"(pk));
+  const f16x2 none = {0.f, 0.f}, one = {1.f, 1.f};
+  return __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(f16x2, pk), none), one));
 }
 template <int NHT>
 __device__ __forceinline__ void score_masks(const f32x16 (&acc)[NHT], bf16x8 (&mk)[2 * NHT]) {
@@ -550,8 +555,9 @@ __global__ __launch_bounds__(ROWS ? THREADS : THREADS / 2) __attribute__((amdgpu
         dw[t] = fmaf(a4[b][2 * x + 1], __builtin_bit_cast(float, p1), dw[t]);
         unsigned m = __builtin_amdgcn_perm((unsigned)p1, (unsigned)p0, 0x07060302u);
         asm("v_pk_min_u16 %0, %0, %1" : "+v"(m) : "s"(0x00010001u));
-        asm("v_pk_mul_lo_u16 %0, %1, %2" : "=v"(ph[t][2 * b + x]) : "v"(m), "v"((int)hl[b][x]));     // (as C: two selects each)
-        asm("v_pk_mul_lo_u16 %0, %1, %2" : "=v"(pl[t][2 * b + x]) : "v"(m), "v"((int)hl[b][2 + x]));
+        // (the products in C, so that the compiler keeps their wait states; of a mask that it knew it would make two selects each)
+        ph[t][2 * b + x] = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, m) * __builtin_bit_cast(u16x2, (int)hl[b][x]));
+        pl[t][2 * b + x] = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, m) * __builtin_bit_cast(u16x2, (int)hl[b][2 + x]));
       }
     };
     if (ntile > 0) {

@@ -83,10 +83,16 @@ def _memory(i):
     return i.op.startswith(("global_", "flat_", "buffer_", "scratch_"))
 
 
+def _vector(i):
+    return i.op.startswith("v_") and not i.op.startswith(("v_mfma", "v_smfma"))
+
+
 # wait states, the second instruction, the first, and the registers that they share
 RULES = {
+    "a matrix instruction reads what a vector instruction wrote":
+        (2, lambda i: i.op.startswith("v_mfma"), _vector, lambda first, second: first.written & second.read),
     "a memory instruction reads a scalar register that a vector instruction wrote":
-        (5, _memory, lambda i: i.op.startswith("v_"), lambda first, second: {r for r in first.written if r[0] == "s"} & second.read),
+        (5, _memory, _vector, lambda first, second: {r for r in first.written if r[0] == "s"} & second.read),
     "a vector instruction writes the data of a store of more than 8 bytes":
         (2, lambda i: i.op.startswith("v_"), lambda i: re.match(r"(global|flat|scratch)_store_dwordx[34]", i.op),
          lambda first, second: _regs(first.operands[1]) & second.written),
