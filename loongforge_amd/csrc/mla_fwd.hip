@@ -142,13 +142,15 @@ __device__ __forceinline__ void store_partial(const f32x16& t, f32x4* p) {
     p[j * 64] = v;
   }
 }
-// The same in device scope: written through, for a workgroup on another XCD to read
+// The same in device scope: written through, for a workgroup on another XCD to read.  (Of assembly the compiler does not know that the data of
+// such a store may be written again two wait states later: they are part of it.)
 __device__ __forceinline__ void store_partial_through(const f32x16& t, f32x4* p) {
+  f32x4 v[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const f32x4 v = {t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]};
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p + j * 64), "v"(v) : "memory");
-  }
+  for (int j = 0; j < 4; j++) v[j] = f32x4{t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]};
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\tglobal_store_dwordx4 %0, %2, off offset:1024 sc1\n\t"
+               "global_store_dwordx4 %0, %3, off offset:2048 sc1\n\tglobal_store_dwordx4 %0, %4, off offset:3072 sc1\n\ts_nop 1"
+               :: "v"(p), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]) : "memory");
 }
 __device__ __forceinline__ void store_out(const f32x16& t, float scale, unsigned short* p) {   // all lanes of the wave
   uint4 o[2];

@@ -1,6 +1,7 @@
 """Wait states that gfx950 leaves to software, in the library as it was compiled.  The compiler keeps them for the instructions that it
 knows; what is written as inline assembly it takes for neither a vector nor a memory instruction, so the waits have to be in the text."""
 import collections
+import glob
 import os
 import re
 import shutil
@@ -117,3 +118,16 @@ def test_wait_states(functions, rule):
                     short.append("%s: %s | %d | %s" % (name, ins[j].text, waits, second.text))
                 ways += [(p, waits + ins[j].waits) for p in before[j]]
     assert not short, "\n".join(short)
+
+
+def test_wide_stores_in_assembly_bring_their_wait():
+    """Whatever the compiler puts behind them today."""
+    from loongforge_amd.csrc import build
+
+    found = 0
+    for path in sorted(glob.glob(os.path.join(build.HERE, "**", "*.h*"), recursive=True)):
+        for text in re.findall(r'\basm\b[^;"]*((?:"(?:[^"\\]|\\.)*"\s*)+)', open(path).read()):
+            behind = re.split(r"_store_dwordx[34]\b", text)
+            found += len(behind) - 1
+            assert len(behind) == 1 or re.search(r"s_nop [1-9]", behind[-1]), (path, text)
+    assert found
