@@ -690,7 +690,7 @@ py::object attn_dist_as_input(const Tensor& p, double sm_scale, bool force) {
   return py::cast(attn_dist_of(p, sm_scale, true));
 }
 
-std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, double eps, double factor) {
+std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, double eps) {
   need_gpus(scores_, target_);
   REQUIRE(scores_.dim() == 2 && target_.sizes() == scores_.sizes(), "indexer_kl_loss expects scores and target of one shape [S, K]");
   const int64_t S = scores_.size(0), K = scores_.size(1);
@@ -699,13 +699,13 @@ std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, 
   if (target.stride(1) != 1) target = target.contiguous();
   Call call(scores);
   Tensor row_loss = make({S}, at::kFloat, scores), grad = make({S, K}, at::kFloat, scores);
-  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss_scaled, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, target.const_data_ptr(), target.scalar_type() == at::kBFloat16, S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, (float)factor, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
+  run("dsa_indexer_kl_loss", dsa_indexer_kl_loss_scaled, (const float*)scores.const_data_ptr(), S > 1 ? scores.stride(0) : K, target.const_data_ptr(), target.scalar_type() == at::kBFloat16, S > 1 ? target.stride(0) : K, (int)S, (int)K, (float)eps, 1.0f, (float*)row_loss.data_ptr(), (float*)grad.data_ptr(), call.stream);
   return {row_loss, grad};
 }
 
 py::object kl_loss(const Tensor& scores, const Tensor& target, double eps, bool force) {
   PLAIN_OR_NONE(scores, target);
-  const auto [row_loss, grad] = kl_rows(scores, target, eps, 1.0);
+  const auto [row_loss, grad] = kl_rows(scores, target, eps);
   return py::make_tuple(row_loss, grad);
 }
 
@@ -720,9 +720,9 @@ py::object kl_total(const Tensor& row_loss, double factor) {
   if (!plain(row_loss) || !row_loss.is_cuda() || row_loss.scalar_type() != at::kFloat || row_loss.dim() != 1 || !row_loss.is_contiguous()) return py::none();
   return py::cast(rows_total(row_loss, factor));
 }
-// Both, the gradient times factor: (loss of all rows times factor, its gradient).
+// Both: (loss of all rows times factor, gradient of the loss without it).
 py::object kl_loss_total(const Tensor& scores, const Tensor& target, double eps, double factor) {
-  const auto [row_loss, grad] = kl_rows(scores, target, eps, factor);
+  const auto [row_loss, grad] = kl_rows(scores, target, eps);
   return py::make_tuple(rows_total(row_loss, factor), grad);
 }
 

@@ -686,6 +686,15 @@ def _(scores, target, eps):
     return scores.new_empty(scores.shape[0], dtype=torch.float32), scores.new_empty(scores.shape, dtype=torch.float32)
 
 
+def _scaled_kl_gradient(grad, g, factor: float):
+    """``grad * (g * factor)``, one launch where nothing records or traces it; never ``grad`` itself, which a hook may write to."""
+    if not torch.is_grad_enabled() and not torch.compiler.is_compiling() and ordinary(grad, g):
+        scaled = _native().kl_scale(grad, g, factor)
+        if scaled is not None:
+            return scaled
+    return grad * (g * factor)
+
+
 class _IndexerKLLoss(torch.autograd.Function):
     """The loss and its gradient come out of the same kernel; backward only scales what forward kept."""
 
@@ -700,10 +709,7 @@ class _IndexerKLLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         (grad,) = ctx.saved_tensors
-        scaled = None
-        if not torch.is_grad_enabled() and not torch.compiler.is_compiling() and ordinary(grad, g):
-            scaled = _native().kl_scale(grad, g, ctx.factor)
-        return (grad * (g * ctx.factor) if scaled is None else scaled).to(ctx.in_dtype), None, None, None
+        return _scaled_kl_gradient(grad, g, ctx.factor).to(ctx.in_dtype), None, None, None
 
 
 def indexer_kl_loss(scores: torch.Tensor, target: torch.Tensor, eps: float = 1e-10, factor: float = 1.0) -> torch.Tensor:
@@ -713,15 +719,13 @@ def indexer_kl_loss(scores: torch.Tensor, target: torch.Tensor, eps: float = 1e-
 
 
 class _AttachedKLLoss(torch.autograd.Function):
-    """:class:`_IndexerKLLoss` and the auto-scaler that feeds its backward, in one node: the gradient of the scores is made, times
-    ``factor``, with the loss, and goes out as it is while no loss scale is set (two nodes, a fill and a pass over the scores' gradient
-    less)."""
+    """:class:`_IndexerKLLoss` and the auto-scaler that feeds its backward, in one node (a node and a fill less)."""
 
     @staticmethod
     def forward(ctx, output, scores, target, eps, factor, scaler):
         loss, grad = _native().kl_loss_total(scores.detach(), target.detach(), eps, factor)
         ctx.save_for_backward(grad)
-        ctx.in_dtype, ctx.scaler = scores.dtype, scaler
+        ctx.in_dtype, ctx.factor, ctx.scaler = scores.dtype, factor, scaler
         ctx.mark_non_differentiable(loss)
         ctx.set_materialize_grads(False)
         return output, loss
@@ -730,12 +734,12 @@ class _AttachedKLLoss(torch.autograd.Function):
     def backward(ctx, grad_output, _):
         d_scores, scale = None, ctx.scaler.main_loss_backward_scale
         if ctx.needs_input_grad[1]:
-            (d_scores,) = ctx.saved_tensors
-            if scale is not None:
-                g, scaled = scale.to(d_scores.device).to(torch.float32), None
-                if not torch.is_grad_enabled() and not torch.compiler.is_compiling() and ordinary(d_scores, g):
-                    scaled = _native().kl_scale(d_scores, g, 1.0)
-                d_scores = d_scores * g.reshape(()) if scaled is None else scaled
+            (grad,) = ctx.saved_tensors
+            if scale is None:
+                d_scores = grad * ctx.factor
+            else:
+                g = scale.to(grad.device).to(torch.float32)
+                d_scores = _scaled_kl_gradient(grad, g.reshape(()) if g.numel() == 1 else g.sum(), ctx.factor)
             d_scores = d_scores.to(ctx.in_dtype)
         return grad_output, d_scores, None, None, None, None
 

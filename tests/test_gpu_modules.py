@@ -483,11 +483,43 @@ def test_heads_are_padded_inside_the_attention(gpu, heads, S, packed):
         assert torch.equal(ops.pad_heads(x, total), torch.nn.functional.pad(x, (0, 0, 0, total - heads)))
 
 
-@pytest.mark.parametrize("scale", [None, 4.0, "one element"])
+def _loss_scale(scale, gpu):
+    return torch.tensor([3.7], device=gpu) if scale == "one element" else torch.tensor(3.7) if scale == "on the host" else torch.tensor(scale, device=gpu)
+
+
+@pytest.mark.parametrize("scale", [None, 3.7, 2.0 ** 70, "one element", "on the host"])
+def test_gradient_of_the_attached_loss_belongs_to_its_receiver(gpu, scale, monkeypatch):
+    """A hook that writes into the gradient of the scores changes what this pass hands on and nothing else: a second pass over a kept graph
+    has the bits of the first, and those of the loss function and the auto-scaler by themselves (for a scale that makes up for a factor
+    below what 32 bits hold of the gradients, too)."""
+    from loongforge_amd import megatron_compat, ops
+
+    S, K, factor = 40, 256, 1.5e-38 if scale == 2.0 ** 70 else 1.5 / 40
+    g = torch.Generator(device=gpu).manual_seed(3)
+    x, start = torch.randn(S, 8, generator=g, device=gpu), torch.randn(S, K, generator=g, device=gpu)
+    target, scaler = torch.softmax(torch.randn(S, K, generator=g, device=gpu), -1), megatron_compat.DSAIndexerLossAutoScaler
+    monkeypatch.setattr(scaler, "main_loss_backward_scale", None if scale is None else _loss_scale(scale, gpu))
+    results = []
+    for one in (True, False):
+        leaf = start.clone().requires_grad_(True)
+        scores = leaf * 1.0
+        scores.register_hook(lambda grad: grad.mul_(3.0))
+        if one:
+            out, loss = ops.attached_indexer_kl_loss(x, scores, target, 1e-10, factor, scaler)
+        else:
+            loss = ops.indexer_kl_loss(scores, target, 1e-10, factor)
+            out = scaler.apply(x, loss)
+        for _ in range(2):
+            results.append((loss.detach(), torch.autograd.grad(out, leaf, torch.ones_like(out), retain_graph=True)[0]))
+    assert results[0][1].abs().max().item() > 0
+    for loss, grad in results[1:]:
+        assert torch.equal(loss, results[0][0]) and torch.equal(grad, results[0][1])
+
+
+@pytest.mark.parametrize("scale", [None, 4.0, 3.7, "one element", "on the host"])
 def test_loss_attached_in_one_node_is_that_of_the_two(gpu, scale, monkeypatch):
     """The indexer's loss with its attachment in one node: the bits of the loss function and the auto-scaler by themselves, for no loss scale
-    and for one (a power of two: it is applied behind the loss's factor there and before it here), in a second backward pass, with
-    saved tensors on their way through a hook and where the indexer needs no gradient."""
+    and for one, in a second backward pass, with saved tensors on their way through a hook and where the indexer needs no gradient."""
     from loongforge_amd import dsa_fused, megatron_compat, ops
     from loongforge_amd.megatron_compat import AttnMaskType, ModuleSpec
 
@@ -507,7 +539,7 @@ def test_loss_attached_in_one_node_is_that_of_the_two(gpu, scale, monkeypatch):
     g = torch.Generator(device=gpu).manual_seed(0)
     rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=torch.bfloat16)      # noqa: E731
     query, key, x, qr, dout = rnd(S, 1, H, 576).requires_grad_(True), rnd(S, 1, 576).requires_grad_(True), rnd(S, 1, hid), rnd(S, 1, qlr), rnd(1, S, H, 512)
-    value = None if scale is None else torch.tensor(4.0, device=gpu) if scale == 4.0 else torch.tensor(4.0)
+    value = None if scale is None else _loss_scale(scale, gpu)
 
     class Subclass(megatron_compat.DSAIndexerLossAutoScaler):        # no longer the class itself: the two nodes
         pass
