@@ -694,7 +694,9 @@ std::pair<Tensor, Tensor> kl_rows(const Tensor& scores_, const Tensor& target_, 
   need_gpus(scores_, target_);
   REQUIRE(scores_.dim() == 2 && target_.sizes() == scores_.sizes(), "indexer_kl_loss expects scores and target of one shape [S, K]");
   const int64_t S = scores_.size(0), K = scores_.size(1);
-  Tensor scores = scores_.to(at::kFloat), target = target_.scalar_type() == at::kBFloat16 ? target_ : target_.to(at::kFloat);
+  // bf16 targets are read as they are, but for rows that overlap (one row for all of them): those become fp32 rows of their own
+  const bool as_is = target_.scalar_type() == at::kBFloat16 && (S < 2 || target_.stride(0) >= K);
+  Tensor scores = scores_.to(at::kFloat), target = as_is ? target_ : target_.to(at::kFloat);
   if (scores.stride(1) != 1) scores = scores.contiguous();
   if (target.stride(1) != 1) target = target.contiguous();
   Call call(scores);

@@ -128,3 +128,41 @@ def test_distribution_and_targets_in_bf16(gpu, S, H, K):
     for t in (target, wide[:, :K]):
         got, want = ops._kl_loss_op(scores, t, 1e-10), ops._kl_loss_op(scores, t.float(), 1e-10)
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("S,K", [(1, 3), (7, 1), (9, 256), (5, 700)])
+def test_targets_in_bf16_of_any_strides(gpu, S, K):
+    """One row for all queries, rows that overlap, columns of a wider tensor and a transposed one: what their copies give."""
+    from loongforge_amd import ops
+
+    gen = torch.Generator().manual_seed(S + K)
+    scores = torch.randn(S, K, generator=gen).to(gpu)
+    base = torch.softmax(torch.randn(S * (K + 2), generator=gen), 0).to(torch.bfloat16).to(gpu)
+    for target in (base[:K].expand(S, K), base.as_strided((S, K), (1, 1)), base.view(S, K + 2)[:, 1:K + 1], base[:S * K].view(K, S).t(),
+                   base.as_strided((S, K), (2, 2)) if S * 2 + K * 2 < base.numel() else base[:K].expand(S, K)):
+        got, want = ops._kl_loss_op(scores, target, 1e-10), ops._kl_loss_op(scores, target.contiguous(), 1e-10)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    if S > 1 and K > 1:                                             # in fp32 such rows are refused, as ever
+        with pytest.raises((RuntimeError, ValueError)):
+            ops._kl_loss_op(scores, base.float()[:K].expand(S, K), 1e-10)
+
+
+@pytest.mark.parametrize("factor", [1.0, 1.5 / 40, -3.7])
+def test_scaled_gradient_through_the_c_abi(gpu, factor):
+    """The gradients of the plain call times the factor, rounded once more; the rows' losses without it."""
+    from loongforge_amd import _lib
+
+    lib, S, K = _lib.load(), 33, 300
+    gen = torch.Generator().manual_seed(5)
+    scores, target = torch.randn(S, K, generator=gen).to(gpu), torch.softmax(torch.randn(S, K, generator=gen), -1).to(gpu)
+    results = []
+    for scaled in (False, True):
+        loss, grad = torch.full((S,), 7.0, device=gpu), torch.full((S, K), 7.0, device=gpu)
+        out, stream = (loss.data_ptr(), grad.data_ptr()), torch.cuda.current_stream().cuda_stream
+        if scaled:
+            rc = lib.dsa_indexer_kl_loss_scaled(scores.data_ptr(), K, target.data_ptr(), 0, K, S, K, 1e-10, factor, *out, stream)
+        else:
+            rc = lib.dsa_indexer_kl_loss(scores.data_ptr(), K, target.data_ptr(), K, S, K, 1e-10, *out, stream)
+        assert rc == 0, lib.dsa_last_error()
+        results.append((loss, grad))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1] * factor, results[1][1])
