@@ -390,6 +390,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   if (!(span > 0.f) || !(span < INFINITY)) return 0;
   const int keff = min(K, m - off);
   const float scale = ((float)BINS - 0.5f) / span;
+  if (!(scale < INFINITY)) return 0;         // (a span below 1.2e-35: there would be no bin for any value but the largest)
   auto bin_of = [&](float x) { return (int)((mx - x) * scale); };
 #pragma unroll
   for (int i = 0; i < NV; i++) {

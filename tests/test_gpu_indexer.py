@@ -235,6 +235,27 @@ def test_topk_segments_of_equal_values(gpu, copies, n, K):
     assert (ids.cpu()[:, kk:] == -1).all()
 
 
+@pytest.mark.parametrize("span", [2.0 ** -149, 1e-44, 1e-40, 1e-38, 2e-36, 1.1e-35, 1.3e-35, 1e-34])
+@pytest.mark.parametrize("copies,n,K", [(1, 300, 64), (1, 6000, 2048), (300, 300, 512), (300, 2000, 64), (300, 8000, 512)])
+def test_topk_of_values_close_to_one_another(gpu, copies, n, K, span):
+    """Rows whose bins would be narrower than what 32 bits hold, on both sides of the line (4095.5 / span), of either sign and with one
+    value beside equal ones; the general path takes them."""
+    from loongforge_amd import ops
+
+    g = torch.Generator().manual_seed(n + K)
+    a = torch.rand(n, generator=g, dtype=torch.float64)
+    x = torch.stack([((a + 1) * span).float(), (-(a + 1) * span).float(), torch.zeros(n), torch.full((n,), -0.0), ((a + 1) * span).float()])
+    x[2, n // 3], x[3, n // 2] = span, -span
+    x[4, n // 4] = -torch.inf                            # (the form for values that are not finite)
+    assert x[0].max() > x[0].min()
+    sc, ids = ops.topk(x.repeat(copies, 1).to(gpu), K)
+    ref = torch.sort(-x, stable=True, dim=-1).indices[:, :K]
+    kk = min(n - 1, K)
+    for row in (slice(0, 5), slice(5 * copies - 5, None)):
+        assert torch.equal(ids[row, :kk].cpu().long(), ref[:, :kk])
+        assert torch.equal(sc[row, :kk].cpu(), torch.gather(x, 1, ref)[:, :kk])
+
+
 def test_fused_rotation_and_quantiser(gpu):
     """rotate_quant_e4m3 against the unfused sequence rotate_activation -> quantiser: the rotated bf16
     values agree to one bf16 step (the fp32 sums are taken in a different order), payload and scale
