@@ -10,6 +10,8 @@
 // of up to 8192 columns are held in registers for it, which leaves room for four workgroups per
 // compute unit.  HBM-bound by design (4 bytes read per candidate, 8 bytes written per output slot);
 // in practice the LDS atomics of the histogram and the scatter set the pace.
+#include <type_traits>
+
 #include "dsa_common.h"
 
 namespace {
@@ -194,10 +196,10 @@ constexpr int LIN_MAX_BIN = 256;             // largest segment ranked by pairwi
 
 // Threshold bin of a filled histogram (thread t owns bins [PER t, PER t + PER)), then the segment
 // starts written over the counts.  False when a bin is too crowded for the ranking step.
-template <int BL, int BINS>
+template <int BL>
 __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff, int& tbin, int& above, int& c) {
   const int tid = threadIdx.x;
-  constexpr int PER = BINS / BL;
+  constexpr int PER = HBINS / BL;
   static_assert(PER % 4 == 0, "a thread's bins go by 16 bytes");
   int* found = scratch + 3 * NWAVES<BL>;
   int cnt[PER], local = 0;
@@ -238,19 +240,20 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
 
 // Final position of every scattered element: hist[b] is the end of segment b by now.  The elements of later segments come behind it
 // and so do the LIN_PAD entries behind the last one, so that counting may run past the end of its segment: four entries at a time for
-// two elements of a thread together, as often as the longest segment of the wave asks for.  (One entry at a time in a loop of every
-// lane's own length is a chain of LDS trips.  us, then / now, with the number of bins by the row's length below: top-k 2048, 8192 causal
-// rows 102 / 95, 1500 rows of 7500 33.0 / 30.5, 8192 of 2048 84 / 76; top-k 512, 4000 rows of 1000 29.0 / 21.8, 2077 of up to 692
-// 15.6 / 12.6; up to 256 rows the same.)
+// two elements of a thread together (of 1024, one where none of a wave has a second), as often as the longest segment of the wave asks for.
+// (One entry at a time in a loop of every lane's own length is a chain of LDS trips.  us, then / now: top-k 2048, 8192 causal rows 103 / 97,
+// 1500 rows of 7500 33.2 / 30.4, 8192 of 2048 83 / 77; top-k 512, 4000 rows of 1000 28.9 / 27.2, 2077 of up to 692 15.6 / 14.9; 200 rows of
+// 1000, top-k 256, with all but one in a segment 51 / 36.  Fewer bins for short rows, which a row's clearing and scanning of 4096 is a
+// quarter of, were 22 at 4000 x 1000, but 106 and not 37 where half of the values are close to zero, and 63 and not 41 with an outlier.)
 template <int BL, class BinOf>
 __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const int* hist, int filled, int keff, int K,
                                          int base_id, BinOf bin_of, float* sv, int* si) {
   const int tid = threadIdx.x;
-  constexpr int PAIR = 2;
-  for (int p0 = tid; p0 < filled; p0 += PAIR * BL) {
+  auto rank_at = [&](int p0, auto pair) {
+    constexpr int PAIR = decltype(pair)::value;
     unsigned long long key[PAIR];
     float v[PAIR];
-    int start[PAIR], end[PAIR], rank[PAIR];
+    int start[PAIR], rank[PAIR], longest = 0;
 #pragma unroll
     for (int u = 0; u < PAIR; u++) key[u] = obuf[min(p0 + u * BL, filled)];
 #pragma unroll
@@ -259,10 +262,9 @@ __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const i
       const bool in = p0 + u * BL < filled;
       const int b = in ? bin_of(v[u]) : 0;
       start[u] = in ? (b > 0 ? hist[b - 1] : 0) : filled;
-      end[u] = in ? hist[b] : filled;
+      longest = max(longest, (in ? hist[b] : filled) - start[u]);
       rank[u] = 0;
     }
-    int longest = max(end[0] - start[0], end[1] - start[1]);
     for (int j = 0; __any(j < longest); j += LIN_PAD) {
 #pragma unroll
       for (int u = 0; u < PAIR; u++) {
@@ -275,6 +277,16 @@ __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const i
     for (int u = 0; u < PAIR; u++) {
       const int pos = start[u] + rank[u];
       if (pos < keff && p0 + u * BL < filled) { sv[pos] = v[u]; si[pos] = base_id + (int)(unsigned)key[u]; }
+    }
+  };
+  const std::integral_constant<int, 1> one;
+  const std::integral_constant<int, 2> two;
+  if constexpr (BL < 1024) {
+    for (int p = tid; p < filled; p += 2 * BL) rank_at(p, two);
+  } else {                                   // (a row of up to 1024 selected elements has no second ones, and might lie in one segment)
+    for (int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63); wave0 < filled; wave0 += 2 * BL) {
+      if (wave0 + BL < filled) rank_at(wave0 + (tid & 63), two);
+      else rank_at(wave0 + (tid & 63), one);
     }
   }
   for (int t = keff + tid; t < K; t += BL) { sv[t] = -INFINITY; si[t] = -1; }
@@ -351,14 +363,14 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
 // x in [mn, mx]), and chunks wholly inside the row need no position tests.  Returns 1 when the row is
 // done, 0 when it is unsuitable (no spread, a crowded bin), -1 when it holds a non-finite value (the
 // caller then runs the tolerant form below on the same registers).
-template <int BL, int NV, int BINS>
+template <int BL, int NV>
 __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int off, int m, int K, int base_id, int* hist,
                                                   int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr int CH = 4 * BL;
   const int nch = (m + CH - 1) / CH;                        // chunks that hold any of the row
   auto chunk_full = [&](int i) { return (i > 0 || off == 0) && CH * (i + 1) <= m; };   // the same for all threads
-  for (int b = tid; b < BINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
+  for (int b = tid; b < HBINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
   float mn = INFINITY, mx = -INFINITY;
   bool nan = false;
 #pragma unroll
@@ -389,7 +401,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   const float span = mx - mn;
   if (!(span > 0.f) || !(span < INFINITY)) return 0;
   const int keff = min(K, m - off);
-  const float scale = ((float)BINS - 0.5f) / span;
+  const float scale = ((float)HBINS - 0.5f) / span;
   if (!(scale < INFINITY)) return 0;         // (a span below 1.2e-35: there would be no bin for any value but the largest)
   auto bin_of = [&](float x) { return (int)((mx - x) * scale); };
 #pragma unroll
@@ -407,7 +419,7 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
   }
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold<BL, BINS>(hist, scratch, keff, tbin, above, c)) return 0;
+  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return 0;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     if (i >= nch) continue;
@@ -428,11 +440,11 @@ __device__ __forceinline__ int select_regs_finite(const float (&v)[NV][4], int o
 
 // The tolerant form: values that are not finite (-inf marks a column that cannot be selected) are skipped
 // one by one.
-template <int BL, int NV, int BINS>
+template <int BL, int NV>
 __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], int off, int K, int base_id, int* hist,
                                                      int* scratch, unsigned long long* obuf, float* sv, int* si) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int b = tid; b < BINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
+  for (int b = tid; b < HBINS / 4; b += BL) ((int4*)hist)[b] = make_int4(0, 0, 0, 0);
   float mn = INFINITY, mx = -INFINITY;
   int nfin = 0;
 #pragma unroll
@@ -450,8 +462,8 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
   const float span = mx - mn;
   if (!(span > 0.f) || !(span < INFINITY)) return false;
   const int keff = min(K, nfin);
-  const float scale = ((float)BINS - 0.5f) / span;
-  auto bin_of = [&](float x) { return min(BINS - 1, (int)((mx - x) * scale)); };
+  const float scale = ((float)HBINS - 0.5f) / span;
+  auto bin_of = [&](float x) { return min(HBINS - 1, (int)((mx - x) * scale)); };
 #pragma unroll
   for (int i = 0; i < NV; i++)
 #pragma unroll
@@ -459,7 +471,7 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
       if (fabsf(v[i][j]) < INFINITY) atomicAdd(&hist[bin_of(v[i][j])], 1);
   __syncthreads();
   int tbin, above, c;
-  if (!lin_threshold<BL, BINS>(hist, scratch, keff, tbin, above, c)) return false;
+  if (!lin_threshold<BL>(hist, scratch, keff, tbin, above, c)) return false;
 #pragma unroll
   for (int i = 0; i < NV; i++)
 #pragma unroll
@@ -474,18 +486,16 @@ __device__ __forceinline__ bool select_regs_tolerant(const float (&v)[NV][4], in
   return true;
 }
 
-// BINS: as many as the registers have elements, up to HBINS: clearing and scanning 4096 of them is most of the work of a short row.
 template <int BL, int NV>
 __device__ __forceinline__ bool linear_select_sort_regs(const float* __restrict__ src, int n, int K, int base_id,
                                                         int* hist, int* scratch, unsigned long long* obuf, float* sv, int* si) {
-  constexpr int BINS = 4 * NV * BL < HBINS ? 4 * NV * BL : HBINS;
   float v[NV][4];
   int off, m;
   load_row_regs<BL, NV>(src, n, v, off, m);
-  const int r = select_regs_finite<BL, NV, BINS>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
+  const int r = select_regs_finite<BL, NV>(v, off, m, K, base_id, hist, scratch, obuf, sv, si);
   if (r >= 0) return r == 1;
   __syncthreads();
-  return select_regs_tolerant<BL, NV, BINS>(v, off, K, base_id, hist, scratch, obuf, sv, si);
+  return select_regs_tolerant<BL, NV>(v, off, K, base_id, hist, scratch, obuf, sv, si);
 }
 
 // LEAN 0: unsorted output, the row staged in LDS where it fits.  1, 2, 3: sorted output, rows held in registers.  1: rows of up

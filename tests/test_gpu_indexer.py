@@ -212,7 +212,7 @@ def test_topk_on_full_width_rows_at_every_alignment(gpu):
 @pytest.mark.parametrize("n,K", [(1021, 64), (1022, 1000), (2045, 64), (2046, 2048), (4090, 2048), (8189, 512)])
 def test_topk_segments_of_equal_values(gpu, copies, n, K):
     """Bins that hold 1 .. 256 elements, and a bin at the K-th place with as many as the buffer has room for and one more: each
-    element's place among its bin's, on both sides of the lengths at which the number of bins changes."""
+    element's place among its bin's, on both sides of the lengths at which a row takes more registers."""
     from loongforge_amd import ops
 
     g = torch.Generator().manual_seed(n + K)
