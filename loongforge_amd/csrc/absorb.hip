@@ -53,10 +53,13 @@ __device__ __forceinline__ void store_rotated(const AbsorbArgs& p, const rope::Q
   else rope::store_quad<rope::SPLIT>(rope::rotate<false>(x, t), dst, q, EMB);
 }
 
-// Rows read and written from which the latter are stored with the non-temporal hint (whole 128-byte lines each): 8192 tokens x 128 heads
-// 340 -> 326 us on the query side, 256 -> 236 on the output side.  Below, the attention behind it finds rows in the memory-side cache:
-// 1500 x 128 73 -> 62 us for the kernel and 1067 -> 1075 with all that follows up to the output's projection, 900 x 128 706 -> 717,
-// 4000 x 64 909 -> 916; above, 2600 x 128 1271 -> 1260, 3000 x 128 1142 -> 1127, 6000 x 64 the same, 8192 x 128 2605 -> 2589.
+// Bytes of a side's rows, read and written, from which the latter are stored with the non-temporal hint (whole 128-byte lines each): 8192
+// tokens x 128 heads 340 -> 326 us on the query side, 256 -> 236 on the output side.  Below, the attention behind it finds rows in the
+// memory-side cache: 1500 x 128 73 -> 62 us for the kernel and 1067 -> 1075 with all that follows up to the output's projection, 900 x 128
+// 706 -> 717.  A prompt with all that follows, us, neither side / both sides so stored, in MB the query side and the output side: 4000 x 64
+// (393, 328) 874 / 875, 5000 x 64 (492, 410) 1041 / 1030, 2600 x 128 (511, 426) 1225 / 1230, 2800 x 128 (551, 459) 1263 / 1249, 3000 x 128 (590, 492) 1315 / 1314,
+// 6000 x 64 (590, 492) 1217 / 1195, 3400 x 128 (668, 557) 1718 / 1702, 6800 x 64 (668, 557) 1382 / 1359, 8192 x 128 (1611, 1342) 2574 / 2504.  The line
+// is where it began to pay with 128 heads; with 64 it would from 490 MB on, and the output side of the sizes in between stays plain.
 constexpr long STREAMED_BYTES = 512l << 20;
 // WAVES * 32 rows per step.  ROPE: the rotary part of the same rows, read one step ahead like the rows themselves.
 template <int K, int N, int WAVES, bool ROPE, bool STREAMED>

@@ -1376,11 +1376,14 @@ order::UnitCost unit_cost(int HG, int S) {       // (HG 1 or 2)
 constexpr size_t DEFAULT_BUDGET = (size_t)160 << 30;
 // What is read or written once passes by the L2, whose key rows the workgroups of an XCD share: Q (with up to 64 heads dO too: the other
 // loads of the set-up take lines by parts) and, with 128 heads, dS both ways.  Up to 64 heads dS is read so up to this size (of queries by
-// themselves); beyond, where it no longer lies in the memory-side cache, that is the slower way.  Whole backward, us, plain / Q (and dO) / dS read
-// so besides: 64 heads 10000 x 512 slots 4021 / 3864 / 3842 (655 MB), 1000 x 2048 1479 / 1473 / 1388 (262 MB), 6000 x 1024 3929 / 3900 / 3913 (786 MB),
-// 3000 x 2048 4227 / 4216 / 4267 beside plain Q (786 MB), 2077 x 512 741 / 726 / 707; 32 heads 3000 x 2048 3912 / 3895 / 3833 (393 MB), 6000 x 1024
-// 2902 / 2863 / 2894 (393 MB).  128 heads, plain / Q / dS written so / read so: 8192 x 2048 12 968 / 12 883 / 12 835 / 13 002 against 13 028, 400 x
-// 2048 833 / 828 / 822 / 809, 1500 x 1024 1501 / 1490 / 1491 / 1465; units write dS as before (1024 x 256 x 32 heads 175 and 180).
+// themselves).  Whole backward, us, dS read plain / so: 64 heads 262 MB (2000 x 1024 slots) 1451 / 1424, 367 MB (1400 x 2048, 2800 x 1024, 5600 x 512)
+// 1901 / 1860, 1926 / 1896, 2081 / 2051, above the line 445 MB (1700 x 2048, 3400 x 1024, 6800 x 512) 2286 / 2255, 2230 / 2202, 2523 / 2500, 655 MB
+// (2500 x 2048, 5000 x 1024, 10000 x 512) 2938 / 2914, 3041 / 3048, 3790 / 3771, 1049 MB (4000 x 2048) 5214 / 5254; 32 heads 393 MB (3000 x 2048,
+// 6000 x 1024, 12000 x 512) 1147 / 1140, 2832 / 2869, 3747 / 3717, 590 MB (4500 x 2048, 9000 x 1024) 2975 / 3012, 4970 / 5020.  So the bytes alone do not
+// tell: the line costs 1.3 % at one of the sizes below it and leaves up to 1.4 % of 64 heads above it.  Q and dO: 64 heads 10000 x 512
+// 4021 -> 3864, 1000 x 2048 1479 -> 1473, 2077 x 512 741 -> 726, 32 heads 6000 x 1024 2902 -> 2863.  128 heads, plain / Q / dS written so / read
+// so: 8192 x 2048 12 968 / 12 883 / 12 835 / 13 002 against 13 028, 400 x 2048 833 / 828 / 822 / 809, 1500 x 1024 1501 / 1490 / 1491 / 1465; units
+// write dS as before (1024 x 256 x 32 heads 175 and 180).
 constexpr size_t DS_ONCE_BYTES = (size_t)384 << 20;
 
 }  // namespace
