@@ -240,10 +240,10 @@ __device__ __forceinline__ bool lin_threshold(int* hist, int* scratch, int keff,
 
 // Final position of every scattered element: hist[b] is the end of segment b by now.  The elements of later segments come behind it
 // and so do the LIN_PAD entries behind the last one, so that counting may run past the end of its segment: four entries at a time for
-// two elements of a thread together (of 1024, one where none of a wave has a second), as often as the longest segment of the wave asks for.
+// two elements of a thread together (of 1024, one where few have a second), as often as the longest segment of the wave asks for.
 // (One entry at a time in a loop of every lane's own length is a chain of LDS trips.  us, then / now: top-k 2048, 8192 causal rows 103 / 97,
 // 1500 rows of 7500 33.2 / 30.4, 8192 of 2048 83 / 77; top-k 512, 4000 rows of 1000 28.9 / 27.2, 2077 of up to 692 15.6 / 14.9; 200 rows of
-// 1000, top-k 256, with all but one in a segment 51 / 36.  Fewer bins for short rows, which a row's clearing and scanning of 4096 is a
+// 1000, top-k 256, with all but one in a segment 51 / 35, 62 in pairs.  Fewer bins for short rows, which a row's clearing and scanning of 4096 is a
 // quarter of, were 22 at 4000 x 1000, but 106 and not 37 where half of the values are close to zero, and 63 and not 41 with an outlier.)
 template <int BL, class BinOf>
 __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const int* hist, int filled, int keff, int K,
@@ -281,13 +281,10 @@ __device__ __forceinline__ void lin_rank(const unsigned long long* obuf, const i
   };
   const std::integral_constant<int, 1> one;
   const std::integral_constant<int, 2> two;
-  if constexpr (BL < 1024) {
+  if (BL == 1024 && filled <= BL + BL / 2) {
+    for (int p = tid; p < filled; p += BL) rank_at(p, one);
+  } else {
     for (int p = tid; p < filled; p += 2 * BL) rank_at(p, two);
-  } else {                                   // (a row of up to 1024 selected elements has no second ones, and might lie in one segment)
-    for (int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63); wave0 < filled; wave0 += 2 * BL) {
-      if (wave0 + BL < filled) rank_at(wave0 + (tid & 63), two);
-      else rank_at(wave0 + (tid & 63), one);
-    }
   }
   for (int t = keff + tid; t < K; t += BL) { sv[t] = -INFINITY; si[t] = -1; }
 }
